@@ -41,6 +41,8 @@ const uint16_t* cbfp(const c10::optional<Tensor>& t) {
   return t.has_value() ? reinterpret_cast<const uint16_t*>(t->data_ptr()) : nullptr;
 }
 
+void post_launch(const char* name);
+
 // ------------------------------------------------------------------ norms / activations
 void rmsnorm(Tensor out, Tensor x, Tensor w, double eps) {
   CHECK_BF16(out); CHECK_BF16(x); CHECK_BF16(w);
@@ -803,6 +805,139 @@ void ivf_plan(Tensor probes, int64_t nlist, Tensor qtab, Tensor slot_rows) {
   if (nq == 0) return;
   nga::launch_ivf_plan(probes.data_ptr<int64_t>(), (int)nq, (int)nprobe, (int)nlist, qtab.data_ptr<int32_t>(),
                        slot_rows.data_ptr<int32_t>(), cur_stream(probes));
+}
+
+// What flat and list searches share: room for candidates and results.
+struct Search {
+  Tensor cand_v, cand_r, out_v, out_id;
+  nga::ScanArgs a{};
+  hipStream_t st;
+};
+
+Search search_begin(const Tensor& q, const Tensor& X, const Tensor& bias, double dot_scale, int64_t metric, int64_t k,
+                    int64_t cap) {
+  const int64_t nq = q.size(0);
+  Search s;
+  s.st = cur_stream(X);
+  const auto f = X.options().dtype(at::kFloat), i32 = X.options().dtype(at::kInt), i64 = X.options().dtype(at::kLong);
+  TORCH_CHECK(cap < (int64_t(1) << 31), "search: too many candidates");
+  s.cand_v = at::empty({nq, cap}, f);
+  s.cand_r = at::empty({nq, cap}, i32);
+  s.out_v = at::empty({nq, k}, f);
+  s.out_id = at::empty({nq, k}, i64);
+  s.a.q_stride = q.stride(0);
+  s.a.metric = (int)metric;
+  s.a.nq = (int)nq;
+  s.a.X = bfp(X);
+  s.a.N = X.size(0);
+  s.a.D = (int)X.size(1);
+  s.a.bias = bias.data_ptr<float>();
+  s.a.dot_scale = (float)dot_scale;
+  s.a.k = (int)k;
+  s.a.cap = (int32_t)cap;
+  s.a.cand_v = s.cand_v.data_ptr<float>();
+  s.a.cand_r = s.cand_r.data_ptr<int32_t>();
+  return s;
+}
+
+std::vector<Tensor> search_end(Search& s, const Tensor& q, const Tensor& ids, int32_t n_fixed, const char* name) {
+  nga::launch_search_finish(s.a.cand_v, s.a.cand_r, s.a.cnt, n_fixed, s.a.cap, s.a.nq, s.a.k,
+                            s.a.metric == nga::SEARCH_L2 ? q.data_ptr<float>() : nullptr, s.a.q_stride, s.a.D,
+                            ids.data_ptr<int64_t>(), s.out_v.data_ptr<float>(), s.out_id.data_ptr<int64_t>(), s.st);
+  post_launch(name);
+  return {s.out_v, s.out_id};
+}
+
+void search_check(const Tensor& q, const Tensor& X, const Tensor& bias, const Tensor& ids, int64_t metric, int64_t k) {
+  CHECK_DEV(q); CHECK_DT(q, at::kFloat);
+  CHECK_BF16(X); CHECK_CONTIG(X);
+  CHECK_DEV(bias); CHECK_DT(bias, at::kFloat); CHECK_CONTIG(bias);
+  CHECK_DEV(ids); CHECK_DT(ids, at::kLong); CHECK_CONTIG(ids);
+  TORCH_CHECK(q.dim() == 2 && X.dim() == 2 && q.size(1) == X.size(1) && q.stride(1) == 1, "search: q [nq, D] and X [N, D]");
+  TORCH_CHECK(nga::scan_chunk((int)X.size(1), 1) > 0, "search: D must be a multiple of 128 up to 1,024");
+  TORCH_CHECK(X.size(0) >= 1 && X.size(0) < (int64_t(1) << 31), "search: 1 .. 2^31 - 1 rows");
+  TORCH_CHECK(bias.numel() == X.size(0) && ids.numel() == X.size(0), "search: one bias and one id per row");
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(X.data_ptr()) % 16 == 0, "search: X must be 16-byte aligned");
+  TORCH_CHECK(k >= 1 && k <= 256 && k <= X.size(0), "search: k must be in [1, min(256, rows)]");
+  TORCH_CHECK(metric >= 0 && metric <= 2, "search: unknown metric");
+  TORCH_CHECK(q.size(0) >= 1 && q.size(0) <= 65535, "search: 1 .. 65,535 queries");
+}
+
+// scores [nq, k] and external ids [nq, k] (-inf / -1 where fewer than k rows are live)
+std::vector<Tensor> flat_search(Tensor q, Tensor X, Tensor bias, Tensor ids, double dot_scale, int64_t metric, int64_t k,
+                                int64_t cus) {
+  search_check(q, X, bias, ids, metric, k);
+  TORCH_CHECK(cus >= 1 && cus <= 4096, "flat_search: compute units");
+  const int64_t nq = q.size(0), N = X.size(0);
+  const int D = (int)X.size(1), ng = nq <= 16 ? 1 : nq <= 32 ? 2 : nq <= 48 ? 3 : 4;
+  const int items = (int)((nq + 16 * ng - 1) / (16 * ng)), K = nga::scan_list((int)k, ng, false);
+  const int blocks = nga::scan_blocks(D, ng, (int)cus);
+  const int64_t tiles = (N + 127) / 128;
+  const int parts = (int)std::min<int64_t>(std::max(1, blocks / items), tiles);
+  constexpr int64_t SEG = 8192;
+  const int64_t nseg = (N + SEG - 1) / SEG, cap = (K ? parts : nseg) * k;
+  Search s = search_begin(q, X, bias, dot_scale, metric, k, cap);
+  s.a.parts = parts;
+  Tensor qb, S;
+  if (ng == 1) {   // up to 16 queries are prepared by every workgroup, while its first vectors come in
+    s.a.qf = q.data_ptr<float>();
+  } else {
+    qb = at::empty({nq, D}, X.options());
+    s.a.Q = bfp(qb);
+    nga::launch_search_prep(q.data_ptr<float>(), q.stride(0), (int)nq, D, (int)metric, bfp(qb), s.st);
+  }
+  if (K == 0) {
+    s.a.s_stride = (N + 3) / 4 * 4;
+    S = at::empty({nq, s.a.s_stride}, X.options().dtype(at::kFloat));
+    s.a.S = S.data_ptr<float>();
+  }
+  nga::launch_scan(s.a, ng, K, items * parts, s.st);
+  if (K == 0)
+    nga::launch_select_segments(s.a.S, s.a.s_stride, (int)nq, N, SEG, (int)k, s.a.cap, s.a.cand_v, s.a.cand_r, s.st);
+  return search_end(s, q, ids, (int32_t)cap, "flat_search");
+}
+
+// the same over the nprobe lists whose centroids score highest; X, bias, ids in list order
+std::vector<Tensor> ivf_search(Tensor q, Tensor X, Tensor bias, Tensor ids, Tensor centroids, Tensor list_beg, Tensor list_end,
+                               double dot_scale, int64_t metric, int64_t nprobe, int64_t k, int64_t cus) {
+  search_check(q, X, bias, ids, metric, k);
+  const int64_t nq = q.size(0), nlist = centroids.size(0);
+  const int D = (int)X.size(1);
+  CHECK_DEV(centroids); CHECK_DT(centroids, at::kFloat); CHECK_CONTIG(centroids);
+  CHECK_DEV(list_beg); CHECK_DT(list_beg, at::kLong); CHECK_CONTIG(list_beg);
+  CHECK_DEV(list_end); CHECK_DT(list_end, at::kLong); CHECK_CONTIG(list_end);
+  TORCH_CHECK(centroids.dim() == 2 && centroids.size(1) == D && nlist >= 1 && nlist <= nga::IVF_SCAN_MAX_LISTS,
+              "ivf_search: 1 .. 1,024 centroids of dimension D");
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(centroids.data_ptr()) % 16 == 0, "ivf_search: centroids must be 16-byte aligned");
+  TORCH_CHECK(list_beg.numel() == nlist && list_end.numel() == nlist, "ivf_search: one row range per list");
+  TORCH_CHECK(nprobe >= 1 && nprobe <= nlist, "ivf_search: nprobe must be in [1, lists]");
+  TORCH_CHECK(k <= 32 && cus >= 1 && cus <= 4096, "ivf_search: k must be at most 32");
+  int ng = nq <= 16 ? 1 : nq <= 32 ? 2 : nq <= 48 ? 3 : 4;
+  if (ng > 2 && k > 8) ng = 2;   // longer register lists leave room for 32 queries
+  const int sl = 16 * ng, K = nga::scan_list((int)k, ng, true), blocks = nga::scan_blocks(D, ng, (int)cus);
+  const int64_t npairs = nq * nprobe, chunks = (nq + sl - 1) / sl;
+  const int64_t max_items = std::min(npairs, nlist * chunks);
+  TORCH_CHECK(chunks * ((X.size(0) + 127) / 128 + nlist) < (int64_t(1) << 31), "ivf_search: too many queries for one call");
+  // the lists of a query lie in at most blocks + 2 nprobe runs
+  Search s = search_begin(q, X, bias, dot_scale, metric, k, (blocks + 2 * nprobe) * k);
+  const auto i32 = X.options().dtype(at::kInt);
+  static_assert(sizeof(nga::ScanItem) == 32, "ScanItem");
+  Tensor qb = at::empty({nq, D}, X.options());
+  Tensor tab = at::empty({8 * max_items + nq + npairs + (blocks + 1) + max_items * sl}, i32);
+  auto* items = reinterpret_cast<nga::ScanItem*>(tab.data_ptr<int32_t>());
+  int32_t *cnt = tab.data_ptr<int32_t>() + 8 * max_items, *probes = cnt + nq, *run_item = probes + npairs,
+          *qtab = run_item + blocks + 1;
+  nga::launch_ivf_probe(q.data_ptr<float>(), q.stride(0), (int)nq, D, (int)metric, centroids.data_ptr<float>(), (int)nlist,
+                        (int)nprobe, bfp(qb), cnt, probes, s.st);
+  nga::launch_ivf_items(probes, (int)npairs, (int)nprobe, (int)nlist, sl, (int)max_items, blocks, list_beg.data_ptr<int64_t>(),
+                        list_end.data_ptr<int64_t>(), items, run_item, qtab, s.st);
+  s.a.Q = bfp(qb);
+  s.a.cnt = cnt;
+  s.a.items = items;
+  s.a.run_item = run_item;
+  s.a.qtab = qtab;
+  nga::launch_scan(s.a, ng, K, blocks, s.st);
+  return search_end(s, q, ids, -1, "ivf_search");
 }
 
 void topk(Tensor in, c10::optional<Tensor> in_idx, int64_t seg_len, int64_t k, Tensor out_v,
@@ -2094,6 +2229,9 @@ PYBIND11_MODULE(_C, m) {
   m.def("embedding", checked("embedding", &embedding));
   m.def("score", checked("score", &score));
   m.def("topk", checked("topk", &topk));
+  m.def("flat_search", &flat_search);
+  m.def("ivf_search", &ivf_search);
+  m.def("search_covers", [](int64_t d) { return d <= 1024 && nga::scan_chunk((int)d, 1) > 0; });
   m.def("score_topk", checked("score_topk", &score_topk));
   m.def("ivf_plan", checked("ivf_plan", &ivf_plan));
   m.def("score_topk_kmax", [](int64_t q) { return (int64_t)nga::score_topk_kmax((int)q); });

@@ -131,6 +131,53 @@ void launch_ivf_plan(const int64_t* probes, int nq, int nprobe, int nlist, int32
 void launch_topk(const float* in, const int64_t* in_idx, int64_t rows, int64_t row_len,
                  int64_t seg_len, int k, float* out_v, int64_t* out_i, hipStream_t stream);
 
+// search_scan.hip: whole searches of bf16 vectors with D a multiple of 128 up to 1,024
+enum SearchMetric { SEARCH_IP = 0, SEARCH_COSINE = 1, SEARCH_L2 = 2 };
+constexpr int IVF_SCAN_MAX_LISTS = 1024;
+struct ScanItem {               // a list with the queries that probe it
+  int32_t tile0, tile1;         // its tiles in the sequence of all items' tiles
+  int32_t nq, unused;
+  int64_t beg, end;             // its rows
+};
+struct ScanArgs {
+  const uint16_t* Q;            // [nq, D] prepared queries, or
+  const float* qf;              // fp32 queries (flat search of at most 16)
+  int64_t q_stride;
+  int metric;
+  int nq;
+  const uint16_t* X;            // [N, D]
+  int64_t N;
+  int D;
+  const float* bias;            // [N]
+  float dot_scale;
+  // lists: items, the first item of each workgroup (and behind them the count of tiles), query of each slot
+  const ScanItem* items;
+  const int32_t *run_item, *qtab;
+  int parts;                    // flat (items null): workgroups of a query group
+  int k;
+  int32_t cap;                  // candidates of a query
+  int32_t* cnt;                 // lists: [nq]
+  float* cand_v;                // [nq, cap]
+  int32_t* cand_r;
+  float* S;                     // [nq, s_stride] where no list is kept
+  int64_t s_stride;
+};
+int scan_chunk(int D, int ng);                  // dims of a unit of work, 0: not covered
+int scan_blocks(int D, int ng, int cus);        // workgroups that fill the chip
+int scan_list(int k, int ng, bool ivf);         // length of the register lists, 0: scores to S
+void launch_scan(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream);
+void launch_search_prep(const float* q, int64_t q_stride, int nq, int D, int metric, uint16_t* qb, hipStream_t stream);
+void launch_ivf_probe(const float* q, int64_t q_stride, int nq, int D, int metric, const float* cent, int nlist, int nprobe,
+                      uint16_t* qb, int32_t* cnt, int32_t* probes, hipStream_t stream);
+void launch_ivf_items(const int32_t* probes, int npairs, int nprobe, int nlist, int sl, int max_items, int blocks,
+                      const int64_t* lbeg, const int64_t* lend, ScanItem* items, int32_t* run_item, int32_t* qtab,
+                      hipStream_t stream);
+void launch_select_segments(const float* S, int64_t s_stride, int nq, int64_t N, int64_t seg, int k, int32_t cap, float* cand_v,
+                            int32_t* cand_r, hipStream_t stream);
+void launch_search_finish(const float* cand_v, const int32_t* cand_r, const int32_t* cnt, int32_t n_fixed, int32_t cap, int nq,
+                          int k, const float* qf, int64_t q_stride, int D, const int64_t* ids, float* out_v, int64_t* out_id,
+                          hipStream_t stream);
+
 // embedding.hip: rows of this rank's vocabulary shard [vocab_lo, vocab_lo + rows), zeros
 // for ids outside it; H % 8 == 0
 void launch_embedding(uint16_t* out, const uint16_t* table, const int32_t* ids, int T, int H, int64_t vocab_lo,

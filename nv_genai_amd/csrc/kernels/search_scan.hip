@@ -1,0 +1,740 @@
+// Whole vector searches in few launches: query preparation, list probing and planning (IVF), one scan of the
+// vectors with the top-k folded in, and the merge that already gives external ids.
+//
+// The work of a scan is one sequence of 128-row tiles over all (list, query group) items, cut into equal runs, one
+// run per workgroup. A run that crosses from one item into the next ends its top-k there and starts again, so lists
+// of any sizes load the chip evenly: with a fixed count of workgroups per list the longest list decided (1M x 1024
+// in 64 lists of unequal size, 16 probed, one query: scan 143 us, now 102; the whole search 189 us, now 113).
+#include "common.h"
+#include "kernels.h"
+
+namespace nga {
+
+namespace {
+constexpr int SS_W = 4;               // waves of a scan workgroup
+constexpr int SS_ROWS = 32 * SS_W;    // rows of a tile
+constexpr int SS_LDS = 160 * 1024;
+constexpr int SEL_CAP = 1024;         // candidates that the selection sorts in LDS
+
+__device__ __forceinline__ uint32_t ss_key(float f) {
+  const uint32_t u = __float_as_uint(f);
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+constexpr uint32_t KEY_NEG_INF = 0x007fffffu;
+
+template <int K>
+__device__ __forceinline__ void ss_insert(float (&v)[K], int (&r)[K], float x, int row) {
+  float cv = x;
+  int cr = row;
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    const bool sw = cv > v[j];
+    const float tv = v[j];
+    const int tr = r[j];
+    v[j] = sw ? cv : tv;
+    r[j] = sw ? cr : tr;
+    cv = sw ? tv : cv;
+    cr = sw ? tr : cr;
+  }
+}
+
+// (v, r) := top K of itself and of the list held by lane ^ mask (both sorted, descending)
+template <int K>
+__device__ __forceinline__ void ss_merge_xor(float (&v)[K], int (&r)[K], int mask) {
+  float ov[K];
+  int orr[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    ov[j] = __shfl_xor(v[j], mask, 64);
+    orr[j] = __shfl_xor(r[j], mask, 64);
+  }
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    const bool tb = ov[K - 1 - j] > v[j];
+    v[j] = tb ? ov[K - 1 - j] : v[j];
+    r[j] = tb ? orr[K - 1 - j] : r[j];
+  }
+#pragma unroll
+  for (int st = K / 2; st > 0; st >>= 1) {
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      if ((j & st) == 0) {
+        const bool sw = v[j + st] > v[j];
+        const float a = v[j], b = v[j + st];
+        const int ra = r[j], rb = r[j + st];
+        v[j] = sw ? b : a;
+        v[j + st] = sw ? a : b;
+        r[j] = sw ? rb : ra;
+        r[j + st] = sw ? ra : rb;
+      }
+    }
+  }
+}
+}  // namespace
+
+// ---------------------------------------------------------------- queries
+// The bf16 form of one query as the stored vectors have it, divided by its norm for cosine; by one wave. Lane l holds
+// elements 4 l + 256 j (D a multiple of 128 up to 1,024).
+namespace {
+struct WaveQuery {
+  f32x4 v[4];
+  __device__ __forceinline__ void load(const float* __restrict__ x, int D, int metric, int lane) {
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i = 4 * lane + 256 * j;
+      v[j] = (f32x4)(0.f);
+      if (i < D) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[j][e] = x[i + e];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ss += v[j][e] * v[j][e];
+    }
+    if (metric == SEARCH_COSINE) {
+      const float nrm = fmaxf(sqrtf(wave_sum(ss)), 1e-12f);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[j][e] /= nrm;
+    }
+  }
+  __device__ __forceinline__ u16x4 bf(int j) const {
+    return (u16x4){f2bf(v[j][0]), f2bf(v[j][1]), f2bf(v[j][2]), f2bf(v[j][3])};
+  }
+};
+}  // namespace
+
+// One wave per query: its bf16 form. Replaces four elementwise and reduction launches of 4 to 5 us each.
+__global__ void __launch_bounds__(256) search_prep_kernel(const float* __restrict__ q, int64_t q_stride, int nq, int D, int metric,
+                                                          uint16_t* __restrict__ qb) {
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (row >= nq) return;
+  WaveQuery wq;
+  wq.load(q + row * q_stride, D, metric, lane);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (4 * lane + 256 * j < D) *reinterpret_cast<u16x4*>(qb + row * D + 4 * lane + 256 * j) = wq.bf(j);
+}
+
+// One workgroup per query: its bf16 form, its products with every centroid (rounded to bf16 as the stored vectors are,
+// sums in fp32; a wave takes four centroids at once, all their loads in flight), each centroid's rank by counting, the
+// nprobe first ones. Takes the place of the preparation, a cast, a score launch over one row tile (11 us) and a radix
+// selection (9 us).
+__global__ void __launch_bounds__(1024) ivf_probe_kernel(const float* __restrict__ q, int64_t q_stride, int D, int metric,
+                                                         const float* __restrict__ cent, int nlist, int nprobe,
+                                                         uint16_t* __restrict__ qb, int32_t* __restrict__ cnt,
+                                                         int32_t* __restrict__ probes) {
+  __shared__ uint32_t sk[IVF_SCAN_MAX_LISTS];
+  const int64_t row = blockIdx.x;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  WaveQuery wq;
+  wq.load(q + row * q_stride, D, metric, lane);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const u16x4 b = wq.bf(j);
+    if (w == 0 && 4 * lane + 256 * j < D) *reinterpret_cast<u16x4*>(qb + row * D + 4 * lane + 256 * j) = b;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wq.v[j][e] = bf2f(b[e]);
+  }
+  if (threadIdx.x == 0) cnt[row] = 0;
+  for (int c0 = 4 * w; c0 < nlist; c0 += 64) {
+    f32x4 v[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = 4 * lane + 256 * j;
+        v[u][j] = (f32x4)(0.f);
+        if (i < D && c0 + u < nlist) v[u][j] = *reinterpret_cast<const f32x4*>(cent + (int64_t)(c0 + u) * D + i);
+      }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      float s = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s += wq.v[j][e] * bf2f(f2bf(v[u][j][e]));
+      s = wave_sum(s);
+      if (lane == 0 && c0 + u < nlist) sk[c0 + u] = ss_key(s);
+    }
+  }
+  __syncthreads();
+  const int c = threadIdx.x;
+  if (c < nlist) {
+    const uint32_t mine = sk[c];
+    int rank = 0;
+    for (int o = 0; o < nlist; ++o) rank += sk[o] > mine || (sk[o] == mine && o < c);
+    if (rank < nprobe) probes[row * nprobe + rank] = c;
+  }
+}
+
+// One workgroup groups the (query, probe) pairs by list: list l with n probing queries becomes ceil(n / sl) items of sl
+// query slots (-1: empty), items in list order. run_item[b] is the item with which workgroup b of the scan begins, so
+// that a scan workgroup is two dependent loads away from its first vectors.
+__global__ void __launch_bounds__(1024) ivf_items_kernel(const int32_t* __restrict__ probes, int npairs, int nprobe, int nlist,
+                                                         int sl, int max_items, int blocks, const int64_t* __restrict__ lbeg,
+                                                         const int64_t* __restrict__ lend, ScanItem* __restrict__ items,
+                                                         int32_t* __restrict__ run_item, int32_t* __restrict__ qtab) {
+  __shared__ int cnt[IVF_SCAN_MAX_LISTS], base[IVF_SCAN_MAX_LISTS], sm[1024], st[1024];
+  const int t = threadIdx.x;
+  cnt[t] = 0;
+  for (int i = t; i < max_items * sl; i += 1024) qtab[i] = -1;
+  __syncthreads();
+  for (int i = t; i < npairs; i += 1024) atomicAdd(&cnt[probes[i]], 1);
+  __syncthreads();
+  int m = 0, tl = 0, mine = cnt[t];
+  int64_t lb = 0, le = 0;
+  if (t < nlist) {
+    m = (mine + sl - 1) / sl;
+    lb = lbeg[t];
+    le = lend[t];
+    tl = le > lb ? (int)((le - lb + SS_ROWS - 1) / SS_ROWS) : 0;
+  }
+  sm[t] = m;
+  st[t] = m * tl;
+  __syncthreads();
+  for (int o = 1; o < 1024; o <<= 1) {
+    const int a = t >= o ? sm[t - o] : 0, b = t >= o ? st[t - o] : 0;
+    __syncthreads();
+    sm[t] += a;
+    st[t] += b;
+    __syncthreads();
+  }
+  const int ib = sm[t] - m, tb = st[t] - m * tl;
+  const int64_t total = st[1023];
+  for (int j = 0; j < m; ++j) {
+    const int t0 = tb + j * tl, t1 = t0 + tl;
+    ScanItem it;
+    it.tile0 = t0;
+    it.tile1 = t1;
+    it.nq = mine - j * sl < sl ? mine - j * sl : sl;
+    it.unused = 0;
+    it.beg = lb;
+    it.end = le;
+    items[ib + j] = it;
+    // the workgroups whose first tile lies in [t0, t1): total * b / blocks >= t0 from b = ceil(t0 * blocks / total)
+    if (t1 > t0)
+      for (int64_t b = ((int64_t)t0 * blocks + total - 1) / total; b < blocks && total * b / blocks < t1; ++b) run_item[b] = ib + j;
+  }
+  if (t == 0) run_item[blocks] = (int)total;
+  base[t] = ib;
+  cnt[t] = 0;
+  __syncthreads();
+  for (int i = t; i < npairs; i += 1024) {
+    const int p = probes[i], rank = atomicAdd(&cnt[p], 1);
+    qtab[(base[p] + rank / sl) * sl + rank % sl] = i / nprobe;
+  }
+}
+
+// ---------------------------------------------------------------- scan
+// Per wave a 32-row x CH-dim LDS slot, filled by lane-linear LDS-DMA (1 KiB per instruction, non-temporal) and read
+// into registers as MFMA fragments; the next unit's DMA goes out before the MFMAs of this one. NG groups of 16 queries
+// lie in LDS beside the slots: one workgroup fills a CU at D 1,024. Bound by the stream of vectors: 6.6 TB/s at one
+// query (1M x 1024; whole search 312 us, 340 with the launches around it that are now in it). With 33 queries and k 25
+// (250k x 1024) 115 us, 4.5 TB/s, half the LDS being queries; reading MFMA fragments from HBM directly, 16 rows x 64 B an
+// instruction, took 187 us.
+// K > 0: a register list of K per lane and group, merged over lanes and waves at the end of a run, and appended to the
+// query's candidates. K = 0 (more than 16 results of up to 32 queries, or 8 of up to 64): scores to S, since inserting
+// into longer lists costs more than the 4 bytes a score.
+template <int NG, int K, int CH>
+__global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
+  constexpr int SL = 16 * NG;
+  constexpr int SLOT = 32 * CH;     // elements of a wave's slot
+  constexpr int NC = CH / 8;        // 16-B positions of a row chunk
+  constexpr int NI = NC / 2;        // DMA instructions of a unit: 32 rows x NC positions / 64 lanes
+  constexpr int NS = CH / 32;       // MFMA k-steps of a unit
+  constexpr int KR = K > 0 ? K : 1;
+  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+  uint16_t* const q_s = smem + SS_W * SLOT;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int col = lane & 15, h = lane >> 4;
+  const int D = p.D, nch = D / 8, nchx = D / CH;
+  const bool flat = p.items == nullptr;
+  uint16_t* const slot = smem + w * SLOT;
+  // flat: workgroup b takes tiles part, part + parts, ... of query group `item` (neighbouring workgroups read
+  // neighbouring tiles: 309 us for 1M x 1024 with the preparation of the query, 311 with one stretch of rows each and
+  // without it). Lists: tiles [g0, g1) of the sequence of all items' tiles
+  int item = 0, part = 0;
+  int64_t g0 = 0, g1 = 1, stride = 1;
+  if (flat) {
+    item = blockIdx.x / p.parts;
+    part = blockIdx.x % p.parts;
+    stride = p.parts;
+  } else {
+    const int64_t total = p.run_item[gridDim.x];
+    g0 = total * blockIdx.x / gridDim.x;
+    g1 = total * (blockIdx.x + 1) / gridDim.x;
+    if (g0 >= g1) return;
+    item = p.run_item[blockIdx.x];
+  }
+  for (; g0 < g1; ++item) {
+    int64_t beg = 0, end = p.N, t0 = part, t1 = (p.N + SS_ROWS - 1) / SS_ROWS;
+    int nql;
+    if (flat) {
+      nql = p.nq - item * SL < SL ? p.nq - item * SL : SL;
+      g0 = g1;
+    } else {
+      const ScanItem it = p.items[item];
+      if (it.tile1 <= g0) continue;   // an empty list
+      beg = it.beg;
+      end = it.end;
+      nql = it.nq;
+      t0 = g0 - it.tile0;
+      t1 = (g1 < it.tile1 ? g1 : it.tile1) - it.tile0;
+      g0 = it.tile0 + t1;
+    }
+    auto slot_q = [&](int s) -> int { return flat ? item * SL + s : p.qtab[(int64_t)item * SL + s]; };
+    const int ngrp = (nql + 15) / 16;
+
+    float bnext[2][4], bcur[2][4];
+    auto issue = [&](int64_t tile, int c) {
+      const int64_t rbase = beg + tile * SS_ROWS + w * 32;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const unsigned li = i * 64 + lane, row = li / NC, pos = li % NC;
+        int64_t gr = rbase + row;
+        if (gr >= end) gr = end - 1;
+        const uint16_t* src = p.X + gr * D + c * CH + ((pos ^ (row & 15)) << 3);
+        __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)(slot + i * 512), 16, 0, 2);
+      }
+      if (c == 0) {   // the tile's biases arrive with its first unit
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr) {
+            const int64_t r = rbase + 16 * i + 4 * h + rr;
+            bnext[i][rr] = (p.bias && r < end) ? p.bias[r] : 0.f;
+          }
+      }
+    };
+    if (t0 < t1) issue(t0, 0);
+    if (NG == 1 && p.qf) {   // unprepared queries: a wave makes the bf16 form of four of them
+      for (int r = w; r < SL; r += SS_W) {
+        WaveQuery wq;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) wq.v[j] = (f32x4)(0.f);
+        if (r < nql) wq.load(p.qf + (int64_t)slot_q(r) * p.q_stride, D, p.metric, lane);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int i = 4 * lane + 256 * j;
+          if (i < D) *reinterpret_cast<u16x4*>(&q_s[r * D + (((i >> 3) ^ (r & 15)) << 3) + (i & 7)]) = wq.bf(j);
+        }
+      }
+    } else {
+      for (int i = tid; i < SL * nch; i += 256) {
+        const int r = i / nch, ch = i % nch;
+        u16x8 v = (u16x8)(0);
+        if (r < nql) v = load8(p.Q + (int64_t)slot_q(r) * D + ch * 8);
+        *reinterpret_cast<u16x8*>(&q_s[r * D + ((ch ^ (r & 15)) * 8)]) = v;
+      }
+    }
+    __syncthreads();
+
+    float tv[NG][KR];
+    int tr[NG][KR];
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int j = 0; j < KR; ++j) {
+        tv[g][j] = -INFINITY;
+        tr[g][j] = -1;
+      }
+    f32x4 acc[2][NG];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int g = 0; g < NG; ++g) acc[i][g] = (f32x4)(0.f);
+    int64_t t = t0;
+    int c = 0;
+    while (t < t1) {
+      int c2 = c + 1;
+      int64_t t2 = t;
+      if (c2 == nchx) {
+        c2 = 0;
+        t2 = t + stride;
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (c == 0) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr) bcur[i][rr] = bnext[i][rr];
+      }
+      u16x8 a[2][NS];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+          a[i][s] = *reinterpret_cast<const u16x8*>(slot + (16 * i + col) * CH + (((4 * s + h) ^ col) << 3));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slot is free
+      if (t2 < t1) issue(t2, c2);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const int ch = c * NC + 4 * s + h;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+          if (g < ngrp) {
+            const bf16x8 bq = as_bf16x8(*reinterpret_cast<const u16x8*>(&q_s[(16 * g + col) * D + ((ch ^ col) << 3)]));
+            acc[0][g] = mfma16(as_bf16x8(a[0][s]), bq, acc[0][g]);
+            acc[1][g] = mfma16(as_bf16x8(a[1][s]), bq, acc[1][g]);
+          }
+        }
+      }
+      if (c == nchx - 1) {
+        // acc[i][g][rr]: row tile + 16 i + 4 h + rr, query slot 16 g + col
+        const int64_t rbase = beg + t * SS_ROWS + w * 32;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int64_t rb = rbase + 16 * i + 4 * h;
+#pragma unroll
+          for (int g = 0; g < NG; ++g) {
+            if constexpr (K > 0) {
+              if (g < ngrp) {
+#pragma unroll
+                for (int rr = 0; rr < 4; ++rr) {
+                  const float sc = acc[i][g][rr] * p.dot_scale + bcur[i][rr];
+                  if (rb + rr < end && sc > tv[g][K - 1]) ss_insert<KR>(tv[g], tr[g], sc, (int)(rb + rr));
+                }
+              }
+            } else {
+              const int q = item * SL + 16 * g + col;   // flat only
+              if (q < p.nq) {
+                float* dst = p.S + (int64_t)q * p.s_stride + rb;   // s_stride % 4 == 0
+                f32x4 v;
+#pragma unroll
+                for (int rr = 0; rr < 4; ++rr) v[rr] = acc[i][g][rr] * p.dot_scale + bcur[i][rr];
+                if (rb + 3 < end) {
+                  *reinterpret_cast<f32x4*>(dst) = v;
+                } else {
+#pragma unroll
+                  for (int rr = 0; rr < 4; ++rr)
+                    if (rb + rr < end) dst[rr] = v[rr];
+                }
+              }
+            }
+            acc[i][g] = (f32x4)(0.f);
+          }
+        }
+      }
+      t = t2;
+      c = c2;
+    }
+    if constexpr (K > 0) {
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        if (g < ngrp) {
+          ss_merge_xor<KR>(tv[g], tr[g], 16);
+          ss_merge_xor<KR>(tv[g], tr[g], 32);
+        }
+      }
+      __syncthreads();   // every wave is past its last DMA wait and done with the query tile
+      float* mv = reinterpret_cast<float*>(smem);   // [SL][4][K]
+      int* mr = reinterpret_cast<int*>(mv + SL * SS_W * K);
+      if (h == 0) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+#pragma unroll
+          for (int j = 0; j < K; ++j) {
+            mv[((16 * g + col) * SS_W + w) * K + j] = tv[g][j];
+            mr[((16 * g + col) * SS_W + w) * K + j] = tr[g][j];
+          }
+        }
+      }
+      __syncthreads();
+      if (tid < nql) {
+        const int q = slot_q(tid);
+        const float* lv = mv + tid * SS_W * K;
+        const int* lr = mr + tid * SS_W * K;
+        int n = 0;
+        for (int j = 0; j < SS_W * K; ++j) n += lr[j] >= 0;
+        n = n < p.k ? n : p.k;
+        // flat: the workgroup's own k places; lists: behind what other runs have appended
+        const int pos = flat ? part * p.k : atomicAdd(&p.cnt[q], n);
+        if (flat)
+          for (int j = n; j < p.k; ++j) {
+            p.cand_v[(int64_t)q * p.cap + pos + j] = -INFINITY;
+            p.cand_r[(int64_t)q * p.cap + pos + j] = -1;
+          }
+        int head[SS_W] = {0, 0, 0, 0};
+        for (int j = 0; j < n && pos + j < p.cap; ++j) {
+          float best = -INFINITY;
+          int bu = 0;
+#pragma unroll
+          for (int u = 0; u < SS_W; ++u) {
+            const float x = head[u] < K ? lv[u * K + head[u]] : -INFINITY;
+            if (x > best) {
+              best = x;
+              bu = u;
+            }
+          }
+          int row = -1;
+#pragma unroll
+          for (int u = 0; u < SS_W; ++u)
+            if (u == bu) {
+              row = lr[u * K + head[u]];
+              ++head[u];
+            }
+          p.cand_v[(int64_t)q * p.cap + pos + j] = best;
+          p.cand_r[(int64_t)q * p.cap + pos + j] = row;
+        }
+      }
+    }
+    __syncthreads();   // the slots and the query tile are free for the next item
+  }
+}
+
+// ---------------------------------------------------------------- selection
+// The k <= 256 largest of n values, sorted, by one workgroup. The k-th largest of the 256 threads' maxima (of 64 groups'
+// maxima where k is at most 32) is a lower bound of the k-th largest value, so a first pass takes maxima, their ranks (by
+// counting) give the bound, and a second pass collects what reaches it: a few more than k values, which are ranked by
+// counting again. Eight loads are in flight per thread. Values of -inf (removed rows) are left out. Should more than
+// 1,024 values reach the bound (equal scores), the k-th key is found bit by bit. Three passes over 2,048 LDS counters,
+// most of them on the same few exponents, took 82 us for both levels of 33 x 250k scores, k 25; these take 30.
+// Order: value, then row (the lower first).
+namespace {
+struct SelShared {
+  uint32_t key[SEL_CAP];
+  int32_t row[SEL_CAP];
+  uint32_t tmax[256];
+  uint32_t bound, n_got;
+  int red[4];
+};
+
+__device__ __forceinline__ int sel_block_count(int c, int* red) {
+  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = c;
+  __syncthreads();
+  return red[0] + red[1] + red[2] + red[3];
+}
+
+// returns how many of the first k places are filled; emit(place, value, row) is called for each of them
+template <typename Emit>
+__device__ __forceinline__ int sel_topk(const float* __restrict__ v, const int32_t* __restrict__ r, int64_t row0, int64_t n, int k,
+                                        SelShared& s, Emit emit) {
+  const int t = threadIdx.x;
+  uint32_t mx = 0;
+  for (int64_t i0 = t; i0 < n; i0 += 8 * 256) {
+    float x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = i0 + 256 * u < n ? v[i0 + 256 * u] : -INFINITY;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const uint32_t key = ss_key(x[u]);
+      mx = key > mx ? key : mx;
+    }
+  }
+  const int ngr = k <= 32 ? 64 : 256;   // groups of four threads, or threads
+  if (ngr == 64) {
+    uint32_t o = __shfl_xor(mx, 1, 64);
+    mx = o > mx ? o : mx;
+    o = __shfl_xor(mx, 2, 64);
+    mx = o > mx ? o : mx;
+    if ((t & 3) == 0) s.tmax[t >> 2] = mx;
+  } else {
+    s.tmax[t] = mx;
+  }
+  if (t == 0) s.n_got = 0;
+  __syncthreads();
+  if (t < ngr) {
+    const uint32_t own = s.tmax[t];
+    int rank = 0;
+#pragma unroll 16
+    for (int o = 0; o < ngr; ++o) {
+      const uint32_t m = s.tmax[o];
+      rank += m > own || (m == own && o < t);
+    }
+    if (rank == k - 1) s.bound = own > KEY_NEG_INF ? own : KEY_NEG_INF + 1;
+  }
+  __syncthreads();
+  const uint32_t bound = s.bound;
+  for (int64_t i0 = t; i0 < n; i0 += 8 * 256) {
+    float x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = i0 + 256 * u < n ? v[i0 + 256 * u] : -INFINITY;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const uint32_t key = ss_key(x[u]);
+      if (key >= bound) {
+        const uint32_t pos = atomicAdd(&s.n_got, 1u);
+        if (pos < SEL_CAP) {
+          const int64_t i = i0 + 256 * u;
+          s.key[pos] = key;
+          s.row[pos] = r ? r[i] : (int32_t)(row0 + i);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  int got = (int)s.n_got;
+  if (got > SEL_CAP) {   // the k-th largest key, its bits from the highest down
+    uint32_t kth = 0;
+    for (int b = 31; b >= 0; --b) {
+      const uint32_t cand = kth | (1u << b);
+      int c = 0;
+      for (int64_t i = t; i < n; i += 256) c += ss_key(v[i]) >= cand;
+      if (sel_block_count(c, s.red) >= k) kth = cand;
+    }
+    __syncthreads();
+    if (t == 0) s.n_got = 0;
+    __syncthreads();
+    for (int pass = 0; pass < 2; ++pass) {   // above it (fewer than k), then equal ones until k are there
+      for (int64_t i = t; i < n; i += 256) {
+        const uint32_t key = ss_key(v[i]);
+        if (pass == 0 ? key > kth : key == kth) {
+          const uint32_t pos = atomicAdd(&s.n_got, 1u);
+          if (pos < (uint32_t)k) {
+            s.key[pos] = key;
+            s.row[pos] = r ? r[i] : (int32_t)(row0 + i);
+          }
+        }
+      }
+      __syncthreads();
+    }
+    got = (int)s.n_got < k ? (int)s.n_got : k;
+  }
+  for (int i = t; i < got; i += 256) {
+    const uint32_t key = s.key[i];
+    const int32_t row = s.row[i];
+    int place = 0;
+    for (int o = 0; o < got; ++o) place += s.key[o] > key || (s.key[o] == key && (s.row[o] < row || (s.row[o] == row && o < i)));
+    if (place < k) emit(place, __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key), row);
+  }
+  return got < k ? got : k;
+}
+}  // namespace
+
+// the k best of each segment of a row of scores, as candidates
+__global__ void __launch_bounds__(256) select_segments_kernel(const float* __restrict__ S, int64_t s_stride, int64_t N,
+                                                              int64_t seg, int k, int32_t cap, float* __restrict__ cand_v,
+                                                              int32_t* __restrict__ cand_r) {
+  __shared__ SelShared s;
+  const int64_t q = blockIdx.y, beg = blockIdx.x * seg;
+  const int64_t n = N - beg < seg ? N - beg : seg;
+  float* ov = cand_v + q * cap + (int64_t)blockIdx.x * k;
+  int32_t* orow = cand_r + q * cap + (int64_t)blockIdx.x * k;
+  const int got = sel_topk(S + q * s_stride + beg, (const int32_t*)nullptr, beg, n, k, s, [&](int place, float v, int32_t r) {
+    ov[place] = v;
+    orow[place] = r;
+  });
+  for (int i = got + threadIdx.x; i < k; i += 256) {
+    ov[i] = -INFINITY;
+    orow[i] = -1;
+  }
+}
+
+// a query's result from its candidates: the k best, less |q|^2 (l2), with the external ids of finite scores
+__global__ void __launch_bounds__(256) search_finish_kernel(const float* __restrict__ cand_v, const int32_t* __restrict__ cand_r,
+                                                            const int32_t* __restrict__ cnt, int32_t n_fixed, int32_t cap,
+                                                            int k, const float* __restrict__ qf, int64_t q_stride, int D,
+                                                            const int64_t* __restrict__ ids, float* __restrict__ out_v,
+                                                            int64_t* __restrict__ out_id) {
+  __shared__ SelShared s;
+  __shared__ float red[4];
+  const int64_t q = blockIdx.x;
+  int n = n_fixed >= 0 ? n_fixed : cnt[q];
+  n = n < cap ? n : cap;
+  float less = 0.f;
+  if (qf) {   // l2
+    for (int i = threadIdx.x; i < D; i += 256) less += qf[q * q_stride + i] * qf[q * q_stride + i];
+    less = block_sum(less, red);
+  }
+  const int got = sel_topk(cand_v + q * cap, cand_r + q * cap, 0, n, k, s, [&](int place, float v, int32_t r) {
+    const float x = v - less;
+    out_v[q * k + place] = x;
+    out_id[q * k + place] = r >= 0 && isfinite(x) ? ids[r] : -1;
+  });
+  for (int i = got + threadIdx.x; i < k; i += 256) {
+    out_v[q * k + i] = -INFINITY;
+    out_id[q * k + i] = -1;
+  }
+}
+
+// ---------------------------------------------------------------- launches
+// dims of a unit: the largest of 512, 384, 256, 128 that divides D and fits beside the queries (more bytes in flight)
+int scan_chunk(int D, int ng) {
+  if (D % 128 != 0 || D < 128 || D > 1024 || ng < 1 || ng > 4) return 0;
+  for (int ch : {512, 384, 256, 128})
+    if (D % ch == 0 && (ng == 1 || ch < 512) && SS_W * 32 * ch * 2 + 16 * ng * D * 2 <= SS_LDS) return ch;
+  return 0;
+}
+
+static size_t scan_lds(int D, int ng, int ch, int K) {
+  const size_t tiles = (size_t)(SS_W * 32 * ch + 16 * ng * D) * 2, merge = (size_t)16 * ng * SS_W * K * 8;
+  return tiles > merge ? tiles : merge;
+}
+
+int scan_blocks(int D, int ng, int cus) {
+  const int ch = scan_chunk(D, ng);
+  const int per_cu = (int)(SS_LDS / scan_lds(D, ng, ch, 32));
+  return cus * (per_cu < 1 ? 1 : per_cu > 4 ? 4 : per_cu);
+}
+
+template <int NG, int K, int CH>
+static void scan_go(const ScanArgs& a, int blocks, hipStream_t stream) {
+  static const bool attr = [] {
+    (void)hipFuncSetAttribute((const void*)scan_kernel<NG, K, CH>, hipFuncAttributeMaxDynamicSharedMemorySize, SS_LDS);
+    (void)hipGetLastError();
+    return true;
+  }();
+  (void)attr;
+  scan_kernel<NG, K, CH><<<blocks, 256, scan_lds(a.D, NG, CH, K), stream>>>(a);
+}
+
+template <int NG, int K>
+static void scan_ch(const ScanArgs& a, int blocks, hipStream_t stream) {
+  switch (scan_chunk(a.D, NG)) {
+    case 512: if constexpr (NG == 1) scan_go<NG, K, 512>(a, blocks, stream); break;
+    case 384: scan_go<NG, K, 384>(a, blocks, stream); break;
+    case 256: scan_go<NG, K, 256>(a, blocks, stream); break;
+    case 128: scan_go<NG, K, 128>(a, blocks, stream); break;
+    default: break;
+  }
+}
+
+// lists: 4, 8, 16, 32 results with up to 32 queries of an item, 4, 8 with up to 64; K = 0: scores
+int scan_list(int k, int ng, bool ivf) {
+  const int most = ng <= 2 ? (ivf ? 32 : 16) : 8;
+  return k > most ? 0 : k <= 4 ? 4 : k <= 8 ? 8 : k <= 16 ? 16 : 32;
+}
+
+void launch_scan(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream) {
+#define NGA_SCAN(NG_, K_) if (ng == NG_ && K == K_) return scan_ch<NG_, K_>(a, blocks, stream)
+  NGA_SCAN(1, 0); NGA_SCAN(1, 4); NGA_SCAN(1, 8); NGA_SCAN(1, 16); NGA_SCAN(1, 32);
+  NGA_SCAN(2, 0); NGA_SCAN(2, 4); NGA_SCAN(2, 8); NGA_SCAN(2, 16); NGA_SCAN(2, 32);
+  NGA_SCAN(3, 0); NGA_SCAN(3, 4); NGA_SCAN(3, 8);
+  NGA_SCAN(4, 0); NGA_SCAN(4, 4); NGA_SCAN(4, 8);
+#undef NGA_SCAN
+}
+
+void launch_search_prep(const float* q, int64_t q_stride, int nq, int D, int metric, uint16_t* qb, hipStream_t stream) {
+  search_prep_kernel<<<(nq + 3) / 4, 256, 0, stream>>>(q, q_stride, nq, D, metric, qb);
+}
+
+void launch_ivf_probe(const float* q, int64_t q_stride, int nq, int D, int metric, const float* cent, int nlist, int nprobe,
+                      uint16_t* qb, int32_t* cnt, int32_t* probes, hipStream_t stream) {
+  ivf_probe_kernel<<<nq, 1024, 0, stream>>>(q, q_stride, D, metric, cent, nlist, nprobe, qb, cnt, probes);
+}
+
+void launch_ivf_items(const int32_t* probes, int npairs, int nprobe, int nlist, int sl, int max_items, int blocks,
+                      const int64_t* lbeg, const int64_t* lend, ScanItem* items, int32_t* run_item, int32_t* qtab,
+                      hipStream_t stream) {
+  ivf_items_kernel<<<1, 1024, 0, stream>>>(probes, npairs, nprobe, nlist, sl, max_items, blocks, lbeg, lend, items, run_item,
+                                           qtab);
+}
+
+void launch_select_segments(const float* S, int64_t s_stride, int nq, int64_t N, int64_t seg, int k, int32_t cap, float* cand_v,
+                            int32_t* cand_r, hipStream_t stream) {
+  dim3 grid((unsigned)((N + seg - 1) / seg), (unsigned)nq);
+  select_segments_kernel<<<grid, 256, 0, stream>>>(S, s_stride, N, seg, k, cap, cand_v, cand_r);
+}
+
+void launch_search_finish(const float* cand_v, const int32_t* cand_r, const int32_t* cnt, int32_t n_fixed, int32_t cap, int nq,
+                          int k, const float* qf, int64_t q_stride, int D, const int64_t* ids, float* out_v, int64_t* out_id,
+                          hipStream_t stream) {
+  search_finish_kernel<<<nq, 256, 0, stream>>>(cand_v, cand_r, cnt, n_fixed, cap, k, qf, q_stride, D, ids, out_v, out_id);
+}
+
+}  // namespace nga

@@ -13,8 +13,9 @@ Bookkeeping is batched: the id -> row map is the native runtime's ``IdMap`` (an 
 addressing table fed numpy batches), and tombstones are one device scatter per call, so
 ingesting or deleting millions of chunks never loops over ids in Python or syncs per row.
 
-Search is one fused kernel (``ops.search_topk``): the MFMA scoring stream keeps a per-lane
-register top-k, so only [queries, blocks, k] candidates reach HBM before the final k-merge.
+Search is one native call (``ops.flat_search``): the MFMA scoring stream keeps a per-lane register top-k, so only
+candidates reach HBM before the final merge, which gives external ids. Dimensions that it does not cover take
+``ops.search_topk``.
 
 Metrics: ``ip`` (inner product), ``cosine`` (vectors/queries pre-normalised, then ip),
 ``l2``. Search returns (scores [nq, k], ids [nq, k]) with external int64 ids.
@@ -144,11 +145,17 @@ class FlatIndex:
     def search(self, q: torch.Tensor, k: int) -> Tuple[torch.Tensor, torch.Tensor]:
         if q.dim() == 1:
             q = q.unsqueeze(0)
+        nq = q.shape[0]
+        if self.n and 0 < nq <= 65535 and ops.search_covers(self.X, min(k, self.n)):
+            with gpu_range(f"search q={nq} n={self.n}"):
+                q = q.to(self.device, torch.float32)
+                n = self.n
+                return ops.flat_search(q if q.stride(1) == 1 else q.contiguous(), self.X[:n], self.bias[:n], self.ids[:n],
+                                       self.metric, min(k, n))
         q = self._prep(q)
         if self.n == 0:
-            nq = q.shape[0]
             return (torch.empty(nq, 0, device=self.device), torch.empty(nq, 0, dtype=torch.int64, device=self.device))
-        with gpu_range(f"search q={q.shape[0]} n={self.n}"):
+        with gpu_range(f"search q={nq} n={self.n}"):
             return self._search(q, k)
 
     def _search(self, q: torch.Tensor, k: int) -> Tuple[torch.Tensor, torch.Tensor]:

@@ -142,9 +142,16 @@ class IVFFlatIndex:
     def search(self, q: torch.Tensor, k: int, nprobe: Optional[int] = None) -> Tuple[torch.Tensor, torch.Tensor]:
         if q.dim() == 1:
             q = q.unsqueeze(0)
-        q = self._prep(q)
         nq = q.shape[0]
         self._ensure_trained()
+        np_ = min(nprobe or self.nprobe, self.nlist)
+        if (self.is_trained and 0 < nq <= 4096 and 1 <= np_ and self.nlist <= ops.IVF_SCAN_MAX_LISTS
+                and self.centroids.shape[0] == self.nlist and ops.search_covers(self.X, k, 32) and k <= self.X.shape[0]):
+            beg, end, _ = self._list_ranges()
+            q = q.to(self.device, torch.float32)
+            return ops.ivf_search(q if q.stride(1) == 1 else q.contiguous(), self.X, self.bias, self.ids,
+                                  self.centroids.float().contiguous(), beg, end, self.metric, np_, k)
+        q = self._prep(q)
         if not self.is_trained:
             return (torch.empty(nq, 0, device=self.device), torch.empty(nq, 0, dtype=torch.int64, device=self.device))
         nprobe = min(nprobe or self.nprobe, self.nlist)

@@ -1718,6 +1718,37 @@ def search_topk(Q: torch.Tensor, X: torch.Tensor, row_bias=None, dot_scale: floa
     return v, r
 
 
+_METRIC = {"ip": 0, "cosine": 1, "l2": 2}
+
+
+def search_covers(X: torch.Tensor, k: int, most: int = 256) -> bool:
+    """Whether a whole search of X [N, D] runs in the native pipeline (``flat_search``, ``ivf_search``): bf16 vectors on
+    the GPU, D a multiple of 128 up to 1,024 (queries and a wave's rows lie in LDS together), at most ``most`` results
+    (256 for flat: the selection's bound is one of 256 threads' maxima; 32 for lists: the register lists). Others take
+    the kernels one by one."""
+    return (_gpu(X) and X.dtype == torch.bfloat16 and X.is_contiguous() and X.data_ptr() % 16 == 0
+            and 1 <= k <= most and 0 < X.shape[0] < 2 ** 31 and bool(kernels().search_covers(X.shape[1])))
+
+
+def flat_search(q: torch.Tensor, X: torch.Tensor, row_bias: torch.Tensor, ids: torch.Tensor, metric: str,
+                k: int) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Top-k of every row of X [N, D] for fp32 queries q [nq, D]: query preparation (normalised for cosine), scan, merge
+    and id lookup in three launches, four where k is large. Returns (scores [nq, k], external ids [nq, k]; -1 where the
+    score is not finite)."""
+    return tuple(kernels().flat_search(q, X, row_bias, ids, 2.0 if metric == "l2" else 1.0, _METRIC[metric], int(k),
+                                       _cu_count(X.device)))
+
+
+def ivf_search(q: torch.Tensor, X: torch.Tensor, row_bias: torch.Tensor, ids: torch.Tensor, centroids: torch.Tensor,
+               list_beg: torch.Tensor, list_end: torch.Tensor, metric: str, nprobe: int,
+               k: int) -> Tuple[torch.Tensor, torch.Tensor]:
+    """``flat_search`` over the rows of the nprobe lists (X in list order) whose centroids have the largest products with
+    the query: five launches, no host synchronisation."""
+    return tuple(kernels().ivf_search(q, X, row_bias, ids, centroids, list_beg, list_end, 2.0 if metric == "l2" else 1.0,
+                                      _METRIC[metric], int(nprobe), int(k), _cu_count(X.device)))
+
+
+IVF_SCAN_MAX_LISTS = 1024   # the planning workgroup's lists, one per thread
 IVF_MAX_ITEMS = 65535   # score_topk's work-item limit (grid dimension)
 
 

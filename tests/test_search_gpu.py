@@ -135,3 +135,94 @@ def test_ivf_index_recall_vs_flat_nlist64_nprobe16(gpu):
     assert len(ivf) == 200_000 - len(set(ii[:, 0].tolist()))
     _, ii2 = ivf.search(Q, 10)
     assert not set(ii[:, 0].tolist()) & set(ii2.reshape(-1).tolist())
+
+
+def _check_found(v, i, S, k):
+    """Scores sorted and those of the returned ids (row = id); none outside the result is larger. Sums of at most 1,024
+    products of bf16 values in fp32: 1,024 * 2^-24 of the summed magnitudes, which are at most 4 here."""
+    S = S.double()
+    rv = torch.topk(S, k, dim=1).values
+    fin = torch.isfinite(rv)
+    assert torch.equal(torch.isfinite(v), fin) and torch.equal(i >= 0, fin)
+    assert bool((v[fin].double() - rv[fin]).abs().max() <= 2.5e-4) if fin.any() else True
+    assert bool((torch.gather(S, 1, i.clamp_min(0))[fin] - v[fin].double()).abs().max() <= 2.5e-4) if fin.any() else True
+    for row in i.tolist():
+        live = [x for x in row if x >= 0]
+        assert len(set(live)) == len(live)
+
+
+# one tile and less, tile and run edges, each unit width (512, 384, 256, 128 dims), each query group count, lists and
+# scores (k above 16, or above 8 with more than 32 queries), several query groups
+@pytest.mark.parametrize("N,D,nq,k,metric", [(1, 128, 1, 1, "ip"), (127, 1024, 3, 25, "cosine"), (129, 384, 16, 4, "l2"),
+                                             (33_000, 1024, 17, 16, "cosine"), (32_769, 768, 33, 8, "l2"), (40_001, 768, 64, 9, "ip"),
+                                             (20_003, 512, 31, 17, "cosine"), (9_001, 640, 65, 4, "cosine"), (8_193, 896, 5, 256, "l2"),
+                                             (70_000, 1024, 48, 25, "l2"), (50_001, 384, 100, 16, "cosine")])
+def test_flat_search_against_fp64(gpu, N, D, nq, k, metric):
+    from nv_genai_amd.index.flat import FlatIndex
+
+    g = torch.Generator().manual_seed(N + D + nq)
+    idx = FlatIndex(D, metric, gpu, capacity=N)
+    x = torch.randn(N, D, generator=g) / D ** 0.5
+    idx.add(x)
+    if N > 200:
+        idx.remove(list(range(0, N, 9)))
+    q = torch.randn(nq, D, generator=g).to(gpu) / D ** 0.5
+    assert ops.search_covers(idx.X, k)
+    v, i = idx.search(q, k)
+    k = min(k, N)
+    assert v.shape == i.shape == (nq, k)
+    qb = idx._prep(q).to(torch.bfloat16).double()
+    S = qb @ idx.X[:N].double().t()
+    if metric == "l2":
+        S = 2 * S - idx.X[:N].double().pow(2).sum(1) - q.double().pow(2).sum(1, keepdim=True)
+    _check_found(v, i, S.masked_fill(idx.bias[:N] == float("-inf"), float("-inf")), k)
+
+
+def test_flat_search_equal_scores_and_strided_queries(gpu):
+    """More equal scores than the selection sorts at once (one vector many times), with lists and with scores; queries
+    that are every second row of a wider matrix."""
+    from nv_genai_amd.index.flat import FlatIndex
+
+    idx = FlatIndex(256, "ip", gpu, capacity=20_000)
+    one = torch.randn(1, 256) / 16
+    x = one.repeat(20_000, 1)
+    x[5] = 0
+    idx.add(x)
+    big = torch.randn(12, 300, device=gpu) / 16
+    q = big[::2, 7:263]
+    S = q.to(torch.bfloat16).double() @ idx.X[: idx.n].double().t()
+    for k in (4, 40, 256):
+        v, i = idx.search(q, k)
+        _check_found(v, i, S, k)
+    idx.remove(list(range(19_998)))                     # fewer live rows than asked for
+    v, i = idx.search(q, 16)
+    assert bool((i[:, 2:] == -1).all()) and bool(torch.isinf(v[:, 2:]).all()) and bool((i[:, :2] >= 0).all())
+
+
+# queries per list of each group count, register lists of each length, more than 64 probing queries of one list
+@pytest.mark.parametrize("D,nq,nprobe,k,metric", [(1024, 1, 16, 4, "cosine"), (256, 1, 1, 32, "l2"), (384, 16, 16, 25, "cosine"),
+                                                  (768, 33, 7, 8, "ip"), (128, 150, 50, 4, "l2"), (256, 70, 50, 32, "cosine")])
+def test_ivf_search_against_fp64(gpu, D, nq, nprobe, k, metric):
+    from nv_genai_amd.index.ivf import IVFFlatIndex
+
+    N, nlist = 21_011, 50
+    g = torch.Generator().manual_seed(D + nq)
+    idx = IVFFlatIndex(D, nlist, nprobe, metric, gpu)
+    c = torch.randn(5, D, generator=g)
+    x = (torch.randn(N, D, generator=g) + c[torch.randint(0, 5, (N,), generator=g)]) / (2 * D) ** 0.5   # uneven lists
+    idx.train(x[:4000].to(gpu))
+    idx.add(x.to(gpu), torch.arange(N))
+    idx.remove(list(range(0, N, 11)))
+    q = (x[:nq] + 0.02 * torch.randn(nq, D, generator=g)).to(gpu)
+    v, i = idx.search(q, k)
+    qb = idx._prep(q).to(torch.bfloat16)
+    probes = torch.topk(qb.double() @ idx.centroids.to(torch.bfloat16).double().t(), nprobe, dim=1).indices
+    lists = torch.repeat_interleave(torch.arange(nlist), idx.offsets[1:] - idx.offsets[:-1]).to(gpu)
+    S = qb.double() @ idx.X.double().t()
+    if metric == "l2":
+        S = 2 * S - idx.X.double().pow(2).sum(1) - q.double().pow(2).sum(1, keepdim=True)
+    seen = (lists[None, :, None] == probes[:, None, :]).any(-1) if nq <= 40 else torch.stack([torch.isin(lists, p) for p in probes])
+    S = S.masked_fill(~seen | (idx.bias == float("-inf"))[None], float("-inf"))
+    by_id = torch.full((nq, N), float("-inf"), dtype=torch.float64, device=gpu)
+    by_id[:, idx.ids] = S
+    _check_found(v, i, by_id, k)
