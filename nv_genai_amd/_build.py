@@ -88,6 +88,7 @@ def _run(cmd):
 # linear scan scales its state with VALU ops once per block of rows.
 PER_FILE_FLAGS = {
     "attention_prefill": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "attention_varlen": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "linear_scan": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 

@@ -670,12 +670,24 @@ void prefill_attention(Tensor out, Tensor q, c10::optional<Tensor> k, c10::optio
     CHECK_BF16(*k); CHECK_BF16(*v);
     TORCH_CHECK(k->dim() == 2 && k->stride(1) == 1 && k->stride(0) == v->stride(0) && k->size(0) == q.size(0));
     TORCH_CHECK(k->stride(0) % 8 == 0 && k->size(1) >= Hkv * D && v->size(1) >= Hkv * D);
-    p.k = bfp(*k);
-    p.v = bfp(*v);
-    p.kv_stride = k->stride(0);
+    if (B == 0 || max_q_len == 0) return;
+    // the kernel's LDS-DMA moves aligned 16-byte pieces: rows of other origins are copied once
+    auto rows = [&](const Tensor& t) {
+      return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.narrow(1, 0, Hkv * D).clone(at::MemoryFormat::Contiguous);
+    };
+    Tensor kr = rows(*k), vr = rows(*v);
+    if (kr.stride(0) != vr.stride(0)) {
+      kr = k->narrow(1, 0, Hkv * D).clone(at::MemoryFormat::Contiguous);
+      vr = v->narrow(1, 0, Hkv * D).clone(at::MemoryFormat::Contiguous);
+    }
+    p.k = bfp(kr);
+    p.v = bfp(vr);
+    p.kv_stride = kr.stride(0);
+    nga::launch_varlen_attention(p, (int)B, (int)max_q_len, (int)D, causal, cur_stream(q));
+    return;
   }
   p.impl = (int)impl;
-  nga::launch_prefill_attention(p, (int)B, (int)max_q_len, (int)D, paged, causal, cur_stream(q));
+  nga::launch_prefill_attention(p, (int)B, (int)max_q_len, (int)D, causal, cur_stream(q));
 }
 
 // ------------------------------------------------------------------ sampling

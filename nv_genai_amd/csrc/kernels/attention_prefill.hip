@@ -1,5 +1,4 @@
-// Flash-style prefill / encoder attention on MFMA (K1 causal-GQA over the paged KV cache,
-// K10 bidirectional encoder attention over packed variable-length sequences).
+// Flash-style prefill attention on MFMA (K1 causal-GQA over the paged KV cache).
 //
 // Workgroup = 4 waves = a 64-row query tile of one query head; each wave owns 16 query
 // rows, which are the 16 columns of its mfma_f32_16x16x32_bf16 tiles. Per 64-key tile the
@@ -12,12 +11,9 @@
 // The next tile's K/V are loaded into registers before the current tile's MFMAs and written
 // to LDS after the barrier (issue-early / write-late, guide §5.5 T14).
 //
-// PAGED: K from the [blocks, Hkv, 64, D] cache, V^T from the [blocks, Hkv, D, 64] cache,
-//        queries are the last q_len positions of a ctx_len context (chunked prefill and
-//        prefix-cache hits work unchanged).  Otherwise: K and V rows come from packed
-//        [T, H, D] tensors with per-sequence offsets (cu_q), V is transposed while staging.
-// D is 64 or 128 (either mode), 256 (paged: Gemma) or 32 (packed mode only: the
-// all-MiniLM-L6-v2 encoder). Paged caches may be fp8 e4m3fn (P.kv_fp8): widened to bf16 in
+// K from the [blocks, Hkv, 64, D] cache, V^T from the [blocks, Hkv, D, 64] cache, queries are
+// the last q_len positions of a ctx_len context (chunked prefill and prefix-cache hits work
+// unchanged). D is 64, 128 or 256 (Gemma). Caches may be fp8 e4m3fn (P.kv_fp8): widened to bf16 in
 // registers before staging; P.scale carries the K scale, P.v_scale the V scale. P.window > 0: sliding-window causal attention (query i sees keys
 // (i - window, i]); key tiles wholly before every query's window are skipped.
 #include <cstdlib>
@@ -36,7 +32,7 @@ __device__ __forceinline__ int row_swz(int row) {  // 4-bit key: distinct over a
 }
 }  // namespace
 
-template <int D, bool PAGED, bool CAUSAL, int NCG>
+template <int D, bool CAUSAL, int NCG>
 __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, uint16_t* v_s, int b, int hq,
                                         int tile) {
   // NCG query column-groups (16 rows each) per wave: the K and V^T fragments read from LDS
@@ -55,7 +51,7 @@ __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, u
   constexpr int SWS = NCH_K >= 16 ? 0 : NCH_K == 8 ? 1 : 2;
   const int q0 = P.cu_q[b], qlen = P.cu_q[b + 1] - q0;
   if (tile * QT >= qlen) return;
-  const int ctx = PAGED ? P.ctx_lens[b] : qlen;
+  const int ctx = P.ctx_lens[b];
   const int G = P.Hq / P.Hkv;
   const int kvh = hq / G;
   const int lane = threadIdx.x & 63;
@@ -95,41 +91,25 @@ __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, u
   // and costs 32 VGPRs that the accumulators need)
   u16x8 kA[PER_T], vA[PER_T];
   auto load_tile = [&](int t, u16x8 (&kreg)[PER_T], u16x8 (&vreg)[PER_T]) {
-    if (PAGED) {
-      const int64_t blk = P.block_tables[(int64_t)b * P.max_blocks + t];
-      const int64_t pg = (blk * P.Hkv + kvh) * (int64_t)(KT * D);   // elements (= bytes for fp8)
-      if (P.kv_fp8) {   // 8-byte fp8 chunks widened to bf16 before they are staged
-        const uint8_t* kp = reinterpret_cast<const uint8_t*>(P.kc) + pg;
-        const uint8_t* vp = reinterpret_cast<const uint8_t*>(P.vc) + pg;
-#pragma unroll
-        for (int i = 0; i < PER_T; ++i) {
-          const int c = tid + 256 * i;
-          kreg[i] = load8_fp8(kp + (int64_t)c * 8);
-          vreg[i] = load8_fp8(vp + (int64_t)c * 8);
-        }
-      } else {
-        const uint16_t* kp = P.kc + pg;
-        const uint16_t* vp = P.vc + pg;
-#pragma unroll
-        for (int i = 0; i < PER_T; ++i) {
-          const int c = tid + 256 * i;
-          kreg[i] = load8(kp + (int64_t)c * 8);
-          vreg[i] = load8(vp + (int64_t)c * 8);
-        }
-      }
-    } else {
+    const int64_t blk = P.block_tables[(int64_t)b * P.max_blocks + t];
+    const int64_t pg = (blk * P.Hkv + kvh) * (int64_t)(KT * D);   // elements (= bytes for fp8)
+    if (P.kv_fp8) {   // 8-byte fp8 chunks widened to bf16 before they are staged
+      const uint8_t* kp = reinterpret_cast<const uint8_t*>(P.kc) + pg;
+      const uint8_t* vp = reinterpret_cast<const uint8_t*>(P.vc) + pg;
 #pragma unroll
       for (int i = 0; i < PER_T; ++i) {
         const int c = tid + 256 * i;
-        const int key = t * KT + c / NCH_K, ch = c % NCH_K;
-        if (key < ctx) {
-          const int64_t off = (int64_t)(q0 + key) * P.kv_stride + (int64_t)kvh * D + ch * 8;
-          kreg[i] = load8(P.k + off);
-          vreg[i] = load8(P.v + off);
-        } else {
-          kreg[i] = (u16x8)(0);
-          vreg[i] = (u16x8)(0);
-        }
+        kreg[i] = load8_fp8(kp + (int64_t)c * 8);
+        vreg[i] = load8_fp8(vp + (int64_t)c * 8);
+      }
+    } else {
+      const uint16_t* kp = P.kc + pg;
+      const uint16_t* vp = P.vc + pg;
+#pragma unroll
+      for (int i = 0; i < PER_T; ++i) {
+        const int c = tid + 256 * i;
+        kreg[i] = load8(kp + (int64_t)c * 8);
+        vreg[i] = load8(vp + (int64_t)c * 8);
       }
     }
   };
@@ -142,17 +122,9 @@ __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, u
         const int sw = row_swz(row) >> SWS;
         *reinterpret_cast<u16x8*>(&k_s[row * D + ((ch ^ sw) * 8)]) = kreg[i];
       }
-      if (PAGED) {  // Vt page is already [d][key]: row = d, chunk = key/8
+      {  // Vt page is already [d][key]: row = d, chunk = key/8
         const int row = c / 8, ch = c % 8;
         *reinterpret_cast<u16x8*>(&v_s[row * KT + ((ch ^ ((row >> 1) & 7)) * 8)]) = vreg[i];
-      } else {  // transpose: vreg holds V[key][d0..d0+7]
-        const int key = c / NCH_K, d0 = (c % NCH_K) * 8;
-        const int ch = key / 8, kin = key % 8;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int row = d0 + j;
-          v_s[row * KT + ((ch ^ ((row >> 1) & 7)) * 8) + kin] = vreg[i][j];
-        }
       }
     }
   };
@@ -279,7 +251,7 @@ __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, u
     ll += __shfl_xor(ll, 16, 64);
     ll += __shfl_xor(ll, 32, 64);
     if (row_ok[cg]) {
-      const float inv = (ll > 0.f ? 1.f / ll : 0.f) * (PAGED && P.kv_fp8 ? P.v_scale : 1.f);
+      const float inv = (ll > 0.f ? 1.f / ll : 0.f) * (P.kv_fp8 ? P.v_scale : 1.f);
       uint16_t* op = P.out + (int64_t)(q0 + qr[cg]) * P.out_stride + (int64_t)hq * D;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
@@ -298,7 +270,7 @@ __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, u
 // query heads sharing a KV head read its pages through the same L2; longest causal tiles
 // first) — or a host-planned work list of (sequence, 64-row tile) pairs walked by a fixed
 // grid with q head it % Hq (graph-captured steps with fp8 KV pages or head_dim != 128).
-template <int D, bool PAGED, bool CAUSAL, int NCG>
+template <int D, bool CAUSAL, int NCG>
 __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams P) {
   constexpr int KT = 64;
   __shared__ __attribute__((aligned(16))) uint16_t k_s[KT * D];
@@ -308,7 +280,7 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams P) {
     for (int it = blockIdx.x; it < total; it += gridDim.x) {
       __syncthreads();
       const int k = it / P.Hq;
-      v1_tile<D, PAGED, CAUSAL, NCG>(P, k_s, v_s, P.items[2 * k], it % P.Hq, P.items[2 * k + 1]);
+      v1_tile<D, CAUSAL, NCG>(P, k_s, v_s, P.items[2 * k], it % P.Hq, P.items[2 * k + 1]);
     }
     return;
   }
@@ -318,62 +290,47 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams P) {
   const int tile = P.ntiles - 1 - L % P.ntiles;
   const int hq = (L / P.ntiles) % P.Hq;
   const int b = L / (P.ntiles * P.Hq);
-  v1_tile<D, PAGED, CAUSAL, NCG>(P, k_s, v_s, b, hq, tile);
+  v1_tile<D, CAUSAL, NCG>(P, k_s, v_s, b, hq, tile);
 }
 
 void launch_prefill_attention_v1_worklist(const PrefillParams& p, int grid, int D, bool causal,
                                           hipStream_t stream) {
   dim3 g(grid);
   if (D == 256) {
-    if (causal) prefill_attn_kernel<256, true, true, 1><<<g, 256, 0, stream>>>(p);
-    else prefill_attn_kernel<256, true, false, 1><<<g, 256, 0, stream>>>(p);
+    if (causal) prefill_attn_kernel<256, true, 1><<<g, 256, 0, stream>>>(p);
+    else prefill_attn_kernel<256, false, 1><<<g, 256, 0, stream>>>(p);
   } else if (D == 128) {
-    if (causal) prefill_attn_kernel<128, true, true, 1><<<g, 256, 0, stream>>>(p);
-    else prefill_attn_kernel<128, true, false, 1><<<g, 256, 0, stream>>>(p);
+    if (causal) prefill_attn_kernel<128, true, 1><<<g, 256, 0, stream>>>(p);
+    else prefill_attn_kernel<128, false, 1><<<g, 256, 0, stream>>>(p);
   } else {
-    if (causal) prefill_attn_kernel<64, true, true, 1><<<g, 256, 0, stream>>>(p);
-    else prefill_attn_kernel<64, true, false, 1><<<g, 256, 0, stream>>>(p);
+    if (causal) prefill_attn_kernel<64, true, 1><<<g, 256, 0, stream>>>(p);
+    else prefill_attn_kernel<64, false, 1><<<g, 256, 0, stream>>>(p);
   }
 }
 
 void launch_prefill_attention(const PrefillParams& p, int num_seqs, int max_q_len, int D,
-                              bool paged, bool causal, hipStream_t stream) {
+                              bool causal, hipStream_t stream) {
   if (num_seqs == 0 || max_q_len == 0) return;
-  // large paged head_dim-128 prefills run the 32x32-MFMA kernel (attention_prefill_v2.hip)
-  if (launch_prefill_attention_v2(p, num_seqs, max_q_len, D, paged, causal, stream)) return;
+  // large head_dim-128 prefills run the 32x32-MFMA kernel (attention_prefill_v2.hip)
+  if (launch_prefill_attention_v2(p, num_seqs, max_q_len, D, causal, stream)) return;
   // 64-row query tiles (a 128-row variant with two column groups per wave halved the LDS
   // fragment traffic per MFMA but needed ~300 VGPR+AGPR — one wave per SIMD — and measured
   // 1.4-1.5x slower on MI355X; removed)
-  const int ncg = 1;
   PrefillParams pp = p;
-  pp.ntiles = (max_q_len + 64 * ncg - 1) / (64 * ncg);
+  pp.ntiles = (max_q_len + 63) / 64;
   const int64_t total = (int64_t)pp.ntiles * p.Hq * num_seqs;
   pp.total = (int)total;
   pp.per_xcd = (int)((total + 7) / 8);
   // 1-D grid of 8 * per_xcd workgroups (see the XCD mapping in the kernel)
   dim3 grid(8 * pp.per_xcd);
-#define NGA_PF(DD, PG, CS)                                                    \
+#define NGA_PF(DD)                                                            \
   do {                                                                        \
-    if (ncg == 2) prefill_attn_kernel<DD, PG, CS, 2><<<grid, 256, 0, stream>>>(pp); \
-    else prefill_attn_kernel<DD, PG, CS, 1><<<grid, 256, 0, stream>>>(pp);          \
+    if (causal) prefill_attn_kernel<DD, true, 1><<<grid, 256, 0, stream>>>(pp); \
+    else prefill_attn_kernel<DD, false, 1><<<grid, 256, 0, stream>>>(pp);       \
   } while (0)
-  if (D == 256 && paged) {   // Gemma (head_dim 256): paged causal prefill
-    if (causal) NGA_PF(256, true, true); else NGA_PF(256, true, false);
-  } else if (D == 128) {
-    if (paged) {
-      if (causal) NGA_PF(128, true, true); else NGA_PF(128, true, false);
-    } else {
-      if (causal) NGA_PF(128, false, true); else NGA_PF(128, false, false);
-    }
-  } else if (D == 64) {
-    if (paged) {
-      if (causal) NGA_PF(64, true, true); else NGA_PF(64, true, false);
-    } else {
-      if (causal) NGA_PF(64, false, true); else NGA_PF(64, false, false);
-    }
-  } else if (D == 32 && !paged) {  // small encoders (MiniLM: 12 heads x 32); one MFMA d-step
-    if (causal) NGA_PF(32, false, true); else NGA_PF(32, false, false);
-  }
+  if (D == 256) NGA_PF(256);   // Gemma
+  else if (D == 128) NGA_PF(128);
+  else if (D == 64) NGA_PF(64);
 #undef NGA_PF
 }
 

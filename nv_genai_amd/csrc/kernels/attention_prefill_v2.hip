@@ -413,9 +413,9 @@ __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) prefill_attn_v2_ker
 }
 
 bool launch_prefill_attention_v2(const PrefillParams& p, int num_seqs, int max_q_len, int D,
-                                 bool paged, bool causal, hipStream_t stream) {
+                                 bool causal, hipStream_t stream) {
   const bool disabled = kernel_form(KF_PREFILL_V1) != 0;
-  if (p.impl == 1 || ((p.impl == 0 || p.impl == 4) && disabled) || D != 128 || !paged || p.kv_fp8 ||
+  if (p.impl == 1 || ((p.impl == 0 || p.impl == 4) && disabled) || D != 128 || p.kv_fp8 ||
       p.max_blocks > V2_MAX_TILES)
     return false;
   const int ks_env = kernel_form(KF_PREFILL_KS);   // 1 | 2 forces the wave-group count (A/B)

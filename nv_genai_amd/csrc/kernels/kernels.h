@@ -94,10 +94,12 @@ struct PrefillParams {
   const int32_t* n_items;
 };
 void launch_prefill_attention(const PrefillParams& p, int num_seqs, int max_q_len, int D,
-                              bool paged, bool causal, hipStream_t stream);
+                              bool causal, hipStream_t stream);
+// packed K / V rows (p.k, p.v; 16-byte aligned), head_dim 32, 64 or 128
+void launch_varlen_attention(const PrefillParams& p, int num_seqs, int max_q_len, int D, bool causal, hipStream_t stream);
 // 32x32-MFMA prefill (paged, head_dim 128); returns false when it does not take the call
 bool launch_prefill_attention_v2(const PrefillParams& p, int num_seqs, int max_q_len, int D,
-                                 bool paged, bool causal, hipStream_t stream);
+                                 bool causal, hipStream_t stream);
 // work-list launch (p.items / p.n_items set): a fixed grid of `grid` workgroups; ks = wave
 // groups (1 or 2). Rows per row block: 32 * 4 / hpw with hpw = 4, 2, 1 for Hq/Hkv % 4, % 2, else.
 void launch_prefill_attention_v2_worklist(const PrefillParams& p, int grid, int ks, bool causal,

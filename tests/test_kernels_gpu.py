@@ -898,3 +898,23 @@ def test_packed_upload_scatters_segments(gpu):
     torch.cuda.synchronize()
     for i in range(3):
         assert torch.equal(ds[i][:5].cpu(), want[i]), i
+
+
+# lengths at the edges of a wave's 32 rows, a workgroup's 128, a 64-key tile; both head layouts (four row blocks of one
+# head; four heads of one KV head), rows that are a view of a wider matrix, K and V at addresses that are not 16-byte ones
+@pytest.mark.parametrize("D,Hq,Hkv", [(32, 3, 3), (64, 4, 4), (64, 8, 2), (128, 4, 1), (128, 6, 3)])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("shift", [0, 2])
+def test_varlen_attention_edges(gpu, D, Hq, Hkv, causal, shift):
+    torch.manual_seed(D + Hq)
+    lens = [1, 31, 32, 33, 63, 64, 65, 96, 127, 128, 129, 257, 300]
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0).tolist()), dtype=torch.int32, device=gpu)
+    T = sum(lens)
+    w = (Hq + 2 * Hkv) * D
+    qkv = _bf(T, w + 8, dev=gpu)[:, : w + shift]
+    q, k, v = qkv[:, : Hq * D], qkv[:, Hq * D + shift: (Hq + Hkv) * D + shift], qkv[:, (Hq + Hkv) * D + shift: w + shift]
+    # a few large scores, so that the running maximum moves between tiles
+    q[::17] *= 6
+    out = ops.varlen_attention(q, k, v, cu, Hq, Hkv, D, max(lens), D ** -0.5, causal)
+    o_ref = ref.varlen_attention(q.float(), k, v, cu, Hq, Hkv, D, D ** -0.5, causal)
+    _close_rows(out, o_ref, width=D)
