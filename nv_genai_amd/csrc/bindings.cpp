@@ -729,6 +729,110 @@ void embedding(Tensor out, Tensor table, Tensor ids, int64_t vocab_lo, double sc
                         vocab_lo, table.size(0), (float)scale, cur_stream(ids));
 }
 
+// ------------------------------------------------------------------ encoder
+// K slices of a projection whose norm sums the slabs: 256-deep ones up to 32 rows (eight waves share a slice), at most 8;
+// with LDS tiles 4 slices while the tiles leave CUs idle (512 rows of 1,024 features: 128 tiles)
+int encoder_split(int64_t M, int64_t K) {
+  if (M <= 32) return (int)std::min<int64_t>(8, std::max<int64_t>(1, K / 256));
+  return M <= 512 ? (int)std::min<int64_t>(4, K / 64) : K > 1024 ? 4 : 2;
+}
+
+// Post-norm encoder stack (BERT): embedding sum + norm, then per layer q/k/v, packed attention, output + norm, up + GELU,
+// down + norm. Layer tensors: wqkv, bqkv, wo, bo, ln1_g, ln1_b, wi, bi, wo2, bo2, ln2_g, ln2_b. All launches go out from
+// here: from Python the 200 of a BERT-large forward took longer than they ran (2.3 ms for one query).
+Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tensor cu, int64_t max_len, Tensor word,
+                       Tensor ptab, Tensor ttab, Tensor emb_g, Tensor emb_b, std::vector<Tensor> L, int64_t heads, double eps,
+                       double scale) {
+  at::NoGradGuard no_grad;
+  CHECK_DEV(ids); CHECK_DT(ids, at::kInt); CHECK_CONTIG(ids);
+  CHECK_DEV(pos); CHECK_DT(pos, at::kInt); CHECK_CONTIG(pos);
+  CHECK_DEV(cu); CHECK_DT(cu, at::kInt); CHECK_CONTIG(cu);
+  const int64_t T = ids.numel(), H = word.size(1), D = heads > 0 ? H / heads : 0;
+  TORCH_CHECK(pos.numel() == T && (!types.has_value() || types->numel() == T), "encoder: one position and type per token");
+  if (types.has_value()) { CHECK_DEV(*types); CHECK_DT(*types, at::kInt); CHECK_CONTIG(*types); }
+  auto weight = [&](const Tensor& t, at::IntArrayRef sizes) {
+    CHECK_BF16(t); CHECK_CONTIG(t);
+    TORCH_CHECK(t.sizes() == sizes && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, "encoder: weight of another shape");
+  };
+  weight(word, {word.size(0), H}); weight(ptab, {ptab.size(0), H}); weight(ttab, {ttab.size(0), H});
+  weight(emb_g, {H}); weight(emb_b, {H});
+  TORCH_CHECK(H % 64 == 0 && H <= 8192 && heads * D == H && (D == 32 || D == 64 || D == 128), "encoder: head size 32, 64 or 128");
+  TORCH_CHECK(L.size() % 12 == 0 && T < (int64_t(1) << 31) && cu.numel() >= 1 && max_len >= 0, "encoder: layers / tokens");
+  const int64_t F = L.empty() ? H : L[6].size(0);
+  TORCH_CHECK(F % 64 == 0, "encoder: feed-forward size must be a multiple of 64");
+  const int64_t B = cu.numel() - 1;
+  const hipStream_t st = cur_stream(ids);
+  const auto opt = word.options();
+  Tensor x = at::empty({T, H}, opt);
+  if (T == 0) return x;
+  nga::launch_embed_layernorm(ids.data_ptr<int32_t>(), pos.data_ptr<int32_t>(), types.has_value() ? types->data_ptr<int32_t>() : nullptr,
+                              bfp(word), (int)word.size(0), bfp(ptab), (int)ptab.size(0), bfp(ttab), (int)ttab.size(0),
+                              bfp(emb_g), bfp(emb_b), (float)eps, T, (int)H, bfp(x), st);
+  Tensor qkv = at::empty({T, 3 * H}, opt), a = at::empty({T, H}, opt), y = at::empty({T, H}, opt), h = at::empty({T, F}, opt);
+  const bool rows = T <= 32, tiles = !rows && T <= 1024;
+  Tensor slabs;
+  if (rows || tiles) slabs = at::empty({std::max(encoder_split(T, H), encoder_split(T, F)), T, H}, opt.dtype(at::kFloat));
+  // out = x w^T + bias (GELU)
+  auto project = [&](const Tensor& in, const Tensor& w, const Tensor& bias, Tensor& out, bool gelu) {
+    const int64_t N = w.size(0), K = w.size(1);
+    if (rows) {
+      nga::launch_row_gemm({bfp(in), K, bfp(w), bfp(bias), out.data_ptr(), N, (int)T, (int)N, (int)K, 1}, gelu ? 2 : 0, st);
+    } else if (tiles) {
+      nga::SkinnyGemmParams p{};
+      p.x = bfp(in); p.ldx = K; p.w = bfp(w); p.M = (int)T; p.N = (int)N; p.K = (int)K;
+      p.out = out.data_ptr(); p.ldo = N; p.bias = bfp(bias);
+      nga::launch_skinny_bias(p, gelu, st);
+    } else if (gelu) {
+      at::mm_out(out, in, w.t());
+      nga::launch_bias_gelu(bfp(out), bfp(bias), T, (int)N, 0, st);
+    } else {
+      at::addmm_out(out, bias, in, w.t());
+    }
+  };
+  // out = LN(in w^T + bias + resid)
+  auto project_norm = [&](const Tensor& in, const Tensor& w, const Tensor& bias, const Tensor& resid, const Tensor& g,
+                          const Tensor& b, Tensor& out) {
+    const int64_t K = w.size(1);
+    const int split = encoder_split(T, K);
+    if (rows) {
+      nga::launch_row_gemm({bfp(in), K, bfp(w), nullptr, slabs.data_ptr(), H, (int)T, (int)H, (int)K, split}, 1, st);
+    } else if (tiles) {
+      nga::SkinnyGemmParams p{};
+      p.x = bfp(in); p.ldx = K; p.w = bfp(w); p.M = (int)T; p.N = (int)H; p.K = (int)K; p.split = split;
+      p.out = slabs.data_ptr(); p.ldo = H;
+      nga::launch_skinny_slabs(p, st);
+    } else {
+      at::addmm_out(y, bias, in, w.t());
+      nga::launch_layernorm(bfp(out), bfp(y), bfp(resid), bfp(g), bfp(b), (float)eps, T, (int)H, st);
+      return;
+    }
+    nga::launch_splitk_layernorm(slabs.data_ptr<float>(), split, (int)T, bfp(bias), bfp(resid), bfp(g), bfp(b), (float)eps, (int)H,
+                                 bfp(out), st);
+  };
+  nga::PrefillParams p{};
+  p.out = bfp(a);
+  p.out_stride = H;
+  p.q = bfp(qkv);
+  p.k = bfp(qkv) + H;
+  p.v = bfp(qkv) + 2 * H;
+  p.q_stride = p.kv_stride = 3 * H;
+  p.cu_q = cu.data_ptr<int32_t>();
+  p.Hq = p.Hkv = (int)heads;
+  p.scale = (float)scale;
+  for (size_t i = 0; i < L.size(); i += 12) {
+    weight(L[i], {3 * H, H}); weight(L[i + 1], {3 * H}); weight(L[i + 2], {H, H}); weight(L[i + 3], {H});
+    weight(L[i + 4], {H}); weight(L[i + 5], {H}); weight(L[i + 6], {F, H}); weight(L[i + 7], {F});
+    weight(L[i + 8], {H, F}); weight(L[i + 9], {H}); weight(L[i + 10], {H}); weight(L[i + 11], {H});
+    project(x, L[i], L[i + 1], qkv, false);
+    if (B > 0 && max_len > 0) nga::launch_varlen_attention(p, (int)B, (int)max_len, (int)D, false, st);
+    project_norm(a, L[i + 2], L[i + 3], x, L[i + 4], L[i + 5], x);
+    project(x, L[i + 6], L[i + 7], h, true);
+    project_norm(h, L[i + 8], L[i + 9], x, L[i + 10], L[i + 11], x);
+  }
+  post_launch("encoder_forward");
+  return x;
+}
+
 // ------------------------------------------------------------------ vector search
 void score(Tensor Q, Tensor X, c10::optional<Tensor> row_bias, Tensor S, double dot_scale) {
   CHECK_BF16(Q); CHECK_BF16(X); CHECK_CONTIG(Q); CHECK_CONTIG(X);
@@ -2241,6 +2345,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("embedding", checked("embedding", &embedding));
   m.def("score", checked("score", &score));
   m.def("topk", checked("topk", &topk));
+  m.def("encoder_forward", &encoder_forward);
   m.def("flat_search", &flat_search);
   m.def("ivf_search", &ivf_search);
   m.def("search_covers", [](int64_t d) { return d <= 1024 && nga::scan_chunk((int)d, 1) > 0; });

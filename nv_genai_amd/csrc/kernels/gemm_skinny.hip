@@ -33,7 +33,7 @@
 //
 // Epilogues: 0 = bf16 out, 1 = fp32 partial slab [split, M, N] (summed by splitk_reduce /
 // splitk_add_rmsnorm / the consumer), 2 = SwiGLU bf16 out [M, F] (N = F, gate rows [0, F),
-// up rows [F, 2F)).
+// up rows [F, 2F)), 3 = bf16 out + bias, 4 = bf16 out, GELU (erf form) of . + bias.
 #include <cstdlib>
 
 #include "common.h"
@@ -62,6 +62,8 @@ __device__ __forceinline__ void sk_wait_vm() {
   static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
+
+__device__ __forceinline__ float sk_gelu(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
 
 __device__ __forceinline__ float sk_silu(float x) { return x / (1.f + __expf(-x)); }
 
@@ -226,7 +228,7 @@ __global__ void __launch_bounds__(64 * WN * WM) skinny_gemm_kernel(SkinnyGemmPar
   for (int mt = 0; mt < MTW; ++mt) {
     const int t = t_base + mt * 16 + col;
     if (t >= P.M) continue;
-    if constexpr (EPI == 0) {
+    if constexpr (EPI == 0 || EPI == 3 || EPI == 4) {
       uint16_t* op = reinterpret_cast<uint16_t*>(P.out) + (int64_t)t * P.ldo;
 #pragma unroll
       for (int nt = 0; nt < NTW; ++nt) {
@@ -234,7 +236,12 @@ __global__ void __launch_bounds__(64 * WN * WM) skinny_gemm_kernel(SkinnyGemmPar
         if (n >= P.N) continue;
         u16x4 v;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = f2bf(acc[nt][mt][r]);
+        for (int r = 0; r < 4; ++r) {
+          float y = acc[nt][mt][r];
+          if constexpr (EPI >= 3) y += bf2f(P.bias[n + r]);
+          if constexpr (EPI == 4) y = sk_gelu(y);
+          v[r] = f2bf(y);
+        }
         *reinterpret_cast<u16x4*>(op + n) = v;
       }
     } else if constexpr (EPI == 1) {
@@ -434,6 +441,37 @@ void launch_skinny_gemm(const SkinnyGemmParams& p, int cfg, int epi, hipStream_t
   }
   NGA_SKINNY_CFGS(NGA_LAUNCH)
 #undef NGA_LAUNCH
+}
+
+// Encoder projections (K 384 to 4,096): 64 x 64 tiles up to 512 rows, 64 x 128 above. BERT-large, weights from HBM (us,
+// library / here): 64 rows q/k/v 11.4 / 7.6, output 8.4 / 4.1, up 11.6 / 7.7, down 14.8 / 7.5; 512 rows 10.8 / 10.3, 8.5 / 5.6,
+// 10.6 / 10.2, 13.8 / 11.6; 1,024 rows 14.1 / 13.8, 9.5 / 7.9, 13.6 / 14.1 (and its GELU launch of 4.6 saved), 18.9 / 17.3; at
+// 1,536 rows the library's larger tiles win everywhere.
+static int skinny_tile(SkinnyGemmParams& p) {
+  const bool small = p.M <= 512;
+  p.nN = (p.N + 63) / 64;
+  p.nM = (p.M + (small ? 63 : 127)) / (small ? 64 : 128);
+  return p.nN * p.nM * p.split;
+}
+
+void launch_skinny_bias(SkinnyGemmParams p, bool gelu, hipStream_t stream) {
+  p.split = 1;
+  const int nblk = skinny_tile(p);
+  if (nblk == 0) return;
+  if (p.M <= 512) {
+    if (gelu) skinny_gemm_kernel<64, 64, 2, 2, 4, 4, 64><<<nblk, 256, 0, stream>>>(p);
+    else skinny_gemm_kernel<64, 64, 2, 2, 4, 3, 64><<<nblk, 256, 0, stream>>>(p);
+  } else {
+    if (gelu) skinny_gemm_kernel<64, 128, 1, 4, 3, 4, 64><<<nblk, 256, 0, stream>>>(p);
+    else skinny_gemm_kernel<64, 128, 1, 4, 3, 3, 64><<<nblk, 256, 0, stream>>>(p);
+  }
+}
+
+void launch_skinny_slabs(SkinnyGemmParams p, hipStream_t stream) {
+  const int nblk = skinny_tile(p);
+  if (nblk == 0) return;
+  if (p.M <= 512) skinny_gemm_kernel<64, 64, 2, 2, 4, 1, 64><<<nblk, 256, 0, stream>>>(p);
+  else skinny_gemm_kernel<64, 128, 1, 4, 3, 1, 64><<<nblk, 256, 0, stream>>>(p);
 }
 
 void launch_splitk_reduce(const float* P, int S, int M, int N, uint16_t* out, int64_t ldo,

@@ -180,6 +180,23 @@ void launch_search_finish(const float* cand_v, const int32_t* cand_r, const int3
                           int k, const float* qf, int64_t q_stride, int D, const int64_t* ids, float* out_v, int64_t* out_id,
                           hipStream_t stream);
 
+// gemm_rows.hip: projections of few rows with the steps around them
+struct RowGemmParams {
+  const uint16_t* x;   // [M, K], row stride ldx
+  int64_t ldx;
+  const uint16_t* w;   // [N, K]; N % 16 == 0, K % 32 == 0; M <= 32
+  const uint16_t* bias;
+  void* out;
+  int64_t ldo;
+  int M, N, K, split;
+};
+void launch_row_gemm(const RowGemmParams& p, int epi, hipStream_t stream);
+void launch_splitk_layernorm(const float* P, int S, int M, const uint16_t* bias, const uint16_t* resid, const uint16_t* g,
+                             const uint16_t* b, float eps, int H, uint16_t* out, hipStream_t stream);
+void launch_embed_layernorm(const int32_t* ids, const int32_t* pos, const int32_t* types, const uint16_t* word, int n_word,
+                            const uint16_t* ptab, int n_pos, const uint16_t* ttab, int n_type, const uint16_t* g,
+                            const uint16_t* b, float eps, int64_t rows, int H, uint16_t* out, hipStream_t stream);
+
 // embedding.hip: rows of this rank's vocabulary shard [vocab_lo, vocab_lo + rows), zeros
 // for ids outside it; H % 8 == 0
 void launch_embedding(uint16_t* out, const uint16_t* table, const int32_t* ids, int T, int H, int64_t vocab_lo,
@@ -281,6 +298,7 @@ struct SkinnyGemmParams {
   int krot;            // 1: each block starts its K walk at a block-dependent step
   int wpack;           // 1: w is tile-packed [nN][K/64][BN][64] for this cfg's BN (pack_weight)
   int xpack;           // 1: x is tile-packed [nM][K/64][BM][64] for this cfg's BM (pack_rows)
+  const uint16_t* bias;  // [N], launch_skinny_bias
 };
 // scatter of packed step inputs (staging.hip): segment s = bytes [off, off + bytes) of the
 // device staging buffer -> dst (16-B aligned offsets / destinations, bytes % 4 == 0)
@@ -297,6 +315,10 @@ int skinny_gemm_cfg_count();
 void launch_region_marker(int end, int* sink, hipStream_t stream);
 void skinny_gemm_cfg_info(int cfg, int* info);   // {BN, BM, WN, WM, NSTAGE, BK}
 void launch_skinny_gemm(const SkinnyGemmParams& p, int cfg, int epi, hipStream_t stream);
+// encoder projections of up to 1,024 rows: bf16 out, + p.bias, and GELU (erf form) with `gelu`; fills in the tiling
+void launch_skinny_bias(SkinnyGemmParams p, bool gelu, hipStream_t stream);
+// fp32 slabs [p.split, M, N] with the same tiles
+void launch_skinny_slabs(SkinnyGemmParams p, hipStream_t stream);
 void launch_splitk_swiglu(const float* P, int S, int M, int F, uint16_t* out, int64_t ldo,
                           hipStream_t stream);
 void launch_splitk_reduce(const float* P, int S, int M, int N, uint16_t* out, int64_t ldo,

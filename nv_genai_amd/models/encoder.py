@@ -12,6 +12,9 @@ Per layer (post-LN BERT):
     h   = gelu(x @ Wi^T + bi)                 K11 (bias+GELU kernel)
     x   = LN(h @ Wo2^T + bo2 + x)
 then CLS / masked-mean pooling + L2 normalisation in one kernel (K12).
+
+On the GPU the stack is one native call (``ops.encoder_forward``), which takes kernels of its own where rows are few;
+the steps below in Python are for the CPU and for weights that it does not cover.
 """
 from __future__ import annotations
 
@@ -131,6 +134,10 @@ class EncoderModel:
         for a reranker (num_labels > 0) returns [B, num_labels] fp32 logits."""
         cfg = self.cfg
         H, nh, hd = cfg.hidden, cfg.heads, cfg.head_dim
+        if ids.is_cuda and ops.encoder_covers(self.word, self.layers, nh):
+            x = ops.encoder_forward(ids, pos, type_ids, cu, max_len, self.word, self.pos, self.type, self.emb_ln, self.layers,
+                                    nh, cfg.eps, self.scale)
+            return self._pool(x, cu)
         tt = self.type[0] if type_ids is None else None
         e = torch.nn.functional.embedding(ids.long(), self.word)
         e = e + torch.nn.functional.embedding(pos.long(), self.pos)
@@ -149,6 +156,10 @@ class EncoderModel:
             ops.bias_gelu_(h, L["bi"])
             o2 = torch.addmm(L["bo2"], h, L["wo2"].t())
             x = ops.layernorm(o2, L["ln2_g"], L["ln2_b"], cfg.eps, resid=x)
+        return self._pool(x, cu)
+
+    def _pool(self, x: torch.Tensor, cu: torch.Tensor) -> torch.Tensor:
+        cfg = self.cfg
         mode = 0 if cfg.pooling == "cls" else 1
         if cfg.num_labels:
             pooled = ops.pool_l2norm(x, cu, mode, False)

@@ -918,3 +918,57 @@ def test_varlen_attention_edges(gpu, D, Hq, Hkv, causal, shift):
     out = ops.varlen_attention(q, k, v, cu, Hq, Hkv, D, max(lens), D ** -0.5, causal)
     o_ref = ref.varlen_attention(q.float(), k, v, cu, Hq, Hkv, D, D ** -0.5, causal)
     _close_rows(out, o_ref, width=D)
+
+
+# token counts at the edges of the three forms of the projections (32, 512 and 1,024 rows) and of their tiles, hidden sizes
+# that split K unevenly, head sizes 32 and 64, with and without token types
+@pytest.mark.parametrize("H,heads,F", [(384, 12, 1536), (1024, 16, 4096), (320, 5, 704)])
+@pytest.mark.parametrize("lens", [[1], [16], [17], [5, 27], [33], [60, 5], [511], [200, 313], [1000, 24], [700, 325, 60]])
+def test_encoder_forward(gpu, H, heads, F, lens):
+    from dataclasses import replace
+
+    from nv_genai_amd.models.config import encoder_config
+    from nv_genai_amd.models.encoder import EncoderModel
+
+    cfg = replace(encoder_config("arctic-embed-l"), hidden=H, heads=heads, ffn=F, layers=2, vocab_size=500, max_position=1024,
+                  pooling="mean")
+    m = EncoderModel(cfg, gpu)
+    g = torch.Generator().manual_seed(H + sum(lens))
+    for L in m.layers:                       # biases and norms that matter
+        for n in ("bqkv", "bo", "bi", "bo2", "ln1_b", "ln2_b"):
+            L[n].copy_((0.1 * torch.randn(L[n].shape, generator=g)).to(torch.bfloat16))
+    ref_m = EncoderModel(cfg, "cpu", dtype=torch.float32, weights={k: v.cpu().float() for k, v in m.state_dict().items()})
+    T = sum(lens)
+    ids = torch.randint(0, 500, (T,), generator=g, dtype=torch.int32)
+    pos = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens])
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0).tolist()), dtype=torch.int32)
+    types = torch.randint(0, 2, (T,), generator=g, dtype=torch.int32) if T % 2 else None
+    assert ops.encoder_covers(m.word, m.layers, heads)
+    x = ops.encoder_forward(ids.to(gpu), pos.to(gpu), None if types is None else types.to(gpu), cu.to(gpu), max(lens), m.word, m.pos,
+                            m.type, m.emb_ln, m.layers, heads, cfg.eps, m.scale)
+    H_, nh, hd = H, heads, H // heads
+    e = ref_m.word[ids.long()] + ref_m.pos[pos.long()] + ref_m.type[types.long() if types is not None else torch.zeros(T, dtype=torch.long)]
+    y = ref.layernorm(e, *ref_m.emb_ln, cfg.eps)
+    for L in ref_m.layers:
+        qkv = torch.addmm(L["bqkv"], y, L["wqkv"].t())
+        a = ref.varlen_attention(qkv[:, :H_], qkv[:, H_:2 * H_], qkv[:, 2 * H_:], cu, nh, nh, hd, m.scale, False)
+        y = ref.layernorm(torch.addmm(L["bo"], a, L["wo"].t()), L["ln1_g"], L["ln1_b"], cfg.eps, resid=y)
+        h = torch.nn.functional.gelu(y @ L["wi"].t() + L["bi"])
+        y = ref.layernorm(torch.addmm(L["bo2"], h, L["wo2"].t()), L["ln2_g"], L["ln2_b"], cfg.eps, resid=y)
+    # two layers of bf16 activations: about 2^-8 relative each, five roundings a layer
+    err = ((x.float().cpu() - y).norm(dim=1) / y.norm(dim=1)).max().item()
+    assert err < 1.5e-2, err
+
+
+def test_encoder_forward_marks_indices_outside_the_tables(gpu):
+    from nv_genai_amd.models.config import encoder_config
+    from nv_genai_amd.models.encoder import EncoderModel
+
+    m = EncoderModel(encoder_config("encoder-tiny"), gpu)
+    ids = torch.tensor([1, 2, 3], dtype=torch.int32, device=gpu)
+    cu = torch.tensor([0, 3], dtype=torch.int32, device=gpu)
+    for bad_ids, bad_pos in ((m.word.shape[0], 0), (-1, 0), (0, m.pos.shape[0])):
+        i, p = ids.clone(), torch.arange(3, dtype=torch.int32, device=gpu)
+        i[1], p[1] = bad_ids, bad_pos
+        x = ops.encoder_forward(i, p, None, cu, 3, m.word, m.pos, m.type, m.emb_ln, [], m.cfg.heads, m.cfg.eps, m.scale)
+        assert x[1].isnan().all() and x[0].isfinite().all() and x[2].isfinite().all()
