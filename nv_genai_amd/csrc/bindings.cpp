@@ -5,6 +5,7 @@
 #include <atomic>
 #include <torch/extension.h>
 
+#include <cmath>
 #include <cstdlib>
 #include <functional>
 #include <c10/hip/HIPStream.h>
@@ -26,6 +27,15 @@ hipStream_t cur_stream(const Tensor& t) {
 #define CHECK_BF16(x) \
   CHECK_DEV(x);       \
   CHECK_DT(x, at::kBFloat16)
+
+#define CHECK_F32(x) \
+  CHECK_DEV(x);      \
+  CHECK_DT(x, at::kFloat); \
+  CHECK_CONTIG(x)
+#define CHECK_I32(x) \
+  CHECK_DEV(x);      \
+  CHECK_DT(x, at::kInt); \
+  CHECK_CONTIG(x)
 
 uint16_t* bfp(const Tensor& t) { return reinterpret_cast<uint16_t*>(t.data_ptr()); }
 
@@ -690,6 +700,79 @@ void prefill_attention(Tensor out, Tensor q, c10::optional<Tensor> k, c10::optio
   nga::launch_prefill_attention(p, (int)B, (int)max_q_len, (int)D, causal, cur_stream(q));
 }
 
+// tables of at most OPT_TENSORS tensors each; fn(table) for every one
+template <typename F>
+int64_t opt_tables(const std::vector<Tensor>& p, const std::vector<Tensor>& g, const std::vector<Tensor>& m,
+                   const std::vector<Tensor>& v, F fn) {
+  nga::OptTable t;
+  t.n = 0;
+  t.first[0] = 0;
+  int64_t all = 0;
+  auto out = [&] {
+    if (t.n == 0) return;
+    fn(t, all);
+    all += t.first[t.n];
+    t.n = 0;
+  };
+  for (size_t i = 0; i < g.size(); ++i) {
+    const int64_t n = g[i].numel(), chunks = (n + nga::OPT_CHUNK - 1) / nga::OPT_CHUNK;
+    if (n == 0) continue;
+    if (t.n == nga::OPT_TENSORS || (t.n && t.first[t.n] + chunks > (1 << 30))) out();
+    TORCH_CHECK(chunks < (1 << 30), "optimiser: tensor too large");
+    t.len[t.n] = n;
+    t.g[t.n] = g[i].data_ptr<float>();
+    t.p[t.n] = p.empty() ? nullptr : p[i].data_ptr<float>();
+    t.m[t.n] = m.empty() ? nullptr : m[i].data_ptr<float>();
+    t.v[t.n] = v.empty() ? nullptr : v[i].data_ptr<float>();
+    t.first[t.n + 1] = t.first[t.n] + (int)chunks;
+    ++t.n;
+  }
+  out();
+  return all;
+}
+
+void opt_check(const std::vector<Tensor>& ts, const std::vector<Tensor>& like) {
+  TORCH_CHECK(ts.size() == like.size(), "optimiser: as many tensors");
+  for (size_t i = 0; i < ts.size(); ++i) {
+    CHECK_F32(ts[i]);
+    TORCH_CHECK(ts[i].numel() == like[i].numel() && ts[i].device() == like[0].device(), "optimiser: tensors of one size and device");
+  }
+}
+
+// [norm, clip factor] of fp32 gradients
+Tensor grad_norm(std::vector<Tensor> g, double max_norm) {
+  TORCH_CHECK(!g.empty(), "grad_norm: no gradients");
+  opt_check(g, g);
+  const hipStream_t st = cur_stream(g[0]);
+  int64_t chunks = 0;
+  for (const Tensor& t : g) chunks += (t.numel() + nga::OPT_CHUNK - 1) / nga::OPT_CHUNK;
+  TORCH_CHECK(chunks < (int64_t(1) << 31), "grad_norm: too many elements");
+  Tensor part = at::empty({std::max<int64_t>(chunks, 1)}, g[0].options()), out = at::empty({2}, g[0].options());
+  opt_tables({}, g, {}, {}, [&](const nga::OptTable& t, int64_t at) { nga::launch_opt_sumsq(t, part.data_ptr<float>() + at, st); });
+  nga::launch_opt_norm(part.data_ptr<float>(), (int)chunks, (float)max_norm, out.data_ptr<float>(), st);
+  post_launch("grad_norm");
+  return out;
+}
+
+// one step of a parameter group; clip: grad_norm's result (gradients are scaled by its factor) or none
+void adamw(std::vector<Tensor> p, std::vector<Tensor> g, std::vector<Tensor> m, std::vector<Tensor> v, c10::optional<Tensor> clip,
+           double lr, double wd, double b1, double b2, double eps, int64_t step) {
+  if (p.empty()) return;
+  opt_check(p, p); opt_check(g, p); opt_check(m, p); opt_check(v, p);
+  TORCH_CHECK(step >= 1, "adamw: steps count from 1");
+  const float* cp = nullptr;
+  if (clip.has_value()) {
+    CHECK_F32(*clip);
+    TORCH_CHECK(clip->numel() == 2, "adamw: clip of grad_norm");
+    cp = clip->data_ptr<float>();
+  }
+  const nga::AdamWArgs a{(float)(1.0 - lr * wd), (float)(1.0 - b1), (float)b2, (float)(1.0 - b2),
+                         (float)(lr / (1.0 - std::pow(b1, (double)step))), (float)std::sqrt(1.0 - std::pow(b2, (double)step)), (float)eps};
+  const hipStream_t st = cur_stream(p[0]);
+  opt_tables(p, g, m, v, [&](const nga::OptTable& t, int64_t) { nga::launch_opt_adamw(t, a, cp, st); });
+  post_launch("adamw");
+}
+
 // ------------------------------------------------------------------ sampling
 void sample(Tensor logits, Tensor temperature, Tensor top_k, Tensor top_p,
             c10::optional<Tensor> rep_penalty, c10::optional<Tensor> history, Tensor seeds,
@@ -1311,15 +1394,6 @@ bool act_f32(const Tensor& t) {
   TORCH_CHECK(t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat, "activations must be bfloat16 or float32");
   return t.scalar_type() == at::kFloat;
 }
-#define CHECK_F32(x) \
-  CHECK_DEV(x);      \
-  CHECK_DT(x, at::kFloat); \
-  CHECK_CONTIG(x)
-#define CHECK_I32(x) \
-  CHECK_DEV(x);      \
-  CHECK_DT(x, at::kInt); \
-  CHECK_CONTIG(x)
-
 void embed_pos(Tensor x, Tensor ids, Tensor pos, Tensor embed, Tensor ptab) {
   CHECK_F32(x); CHECK_I32(ids); CHECK_I32(pos);
   const bool f32 = act_f32(embed);
@@ -2346,6 +2420,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("score", checked("score", &score));
   m.def("topk", checked("topk", &topk));
   m.def("encoder_forward", &encoder_forward);
+  m.def("grad_norm", &grad_norm);
+  m.def("adamw", &adamw);
   m.def("flat_search", &flat_search);
   m.def("ivf_search", &ivf_search);
   m.def("search_covers", [](int64_t d) { return d <= 1024 && nga::scan_chunk((int)d, 1) > 0; });

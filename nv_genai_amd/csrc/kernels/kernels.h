@@ -197,6 +197,22 @@ void launch_embed_layernorm(const int32_t* ids, const int32_t* pos, const int32_
                             const uint16_t* ptab, int n_pos, const uint16_t* ttab, int n_type, const uint16_t* g,
                             const uint16_t* b, float eps, int64_t rows, int H, uint16_t* out, hipStream_t stream);
 
+// adamw.hip
+constexpr int OPT_TENSORS = 48;
+constexpr int OPT_CHUNK = 32768;
+struct OptTable {
+  int n;
+  int first[OPT_TENSORS + 1];   // first chunk of each tensor; [n]: their count
+  int64_t len[OPT_TENSORS];
+  float *p[OPT_TENSORS], *g[OPT_TENSORS], *m[OPT_TENSORS], *v[OPT_TENSORS];
+};
+struct AdamWArgs {
+  float decay, one_b1, b2, one_b2, step, sqrt_c2, eps;   // 1 - lr wd, 1 - b1, b2, 1 - b2, lr / (1 - b1^t), sqrt(1 - b2^t)
+};
+void launch_opt_sumsq(const OptTable& t, float* part, hipStream_t st);
+void launch_opt_norm(const float* part, int n, float max_norm, float* out, hipStream_t st);
+void launch_opt_adamw(const OptTable& t, const AdamWArgs& a, const float* clip, hipStream_t st);
+
 // embedding.hip: rows of this rank's vocabulary shard [vocab_lo, vocab_lo + rows), zeros
 // for ids outside it; H % 8 == 0
 void launch_embedding(uint16_t* out, const uint16_t* table, const int32_t* ids, int T, int H, int64_t vocab_lo,

@@ -32,6 +32,7 @@ import torch
 
 from . import functional as Fn
 from .lora import LoRA, LoRAConfig
+from .optim import AdamW
 
 
 @dataclass
@@ -104,9 +105,10 @@ class Trainer:
         self.sync = GradBucketer(self.params, group=group, bucket_mb=cfg.bucket_mb)
         decay = [p for n, p in named.items() if p.ndim >= 2]
         nodecay = [p for n, p in named.items() if p.ndim < 2]
-        self.opt = torch.optim.AdamW([{"params": decay, "weight_decay": cfg.weight_decay},
-                                      {"params": nodecay, "weight_decay": 0.0}], lr=cfg.lr, betas=cfg.betas,
-                                     **({"fused": True} if fused else {}))
+        # fp32 masters on the GPU step in the native kernel whatever ``fused`` says, which others of torch's then use
+        self.opt = AdamW([{"params": decay, "weight_decay": cfg.weight_decay},
+                          {"params": nodecay, "weight_decay": 0.0}], lr=cfg.lr, betas=cfg.betas,
+                         **({"fused": True} if fused else {}))
         self.step = 0
         self.cursor = 0
         self.ckpt_dir = ckpt_dir
@@ -143,9 +145,7 @@ class Trainer:
             loss.backward()
             total += float(loss.detach())
         self.sync.finish()
-        if cfg.grad_clip:
-            torch.nn.utils.clip_grad_norm_(self.params, cfg.grad_clip)
-        self.opt.step()
+        self.opt.step(max_norm=cfg.grad_clip)
         self.step += 1
         if self.world > 1:
             t = torch.tensor([total], dtype=torch.float64, device=self.params[0].device)

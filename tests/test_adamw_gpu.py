@@ -1,0 +1,44 @@
+"""The native AdamW step on the GPU against torch's in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, b):
+    return ((a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-30)).item()
+
+
+@pytest.mark.parametrize("max_norm", [None, 0.5, 1e9])
+def test_adamw_matches_torch(gpu, max_norm):
+    from nv_genai_amd.training.optim import AdamW
+
+    sizes = [(1,), (7, 5), (33_000,), (128, 300), (65_537,)] + [(3, 4)] * 60    # ragged ends, several chunks, two tables
+    g = torch.Generator(device="cuda").manual_seed(1)
+    ps = [torch.randn(s, device="cuda", generator=g) for s in sizes]
+    # the last is a view at an odd address
+    ps[-1] = torch.randn(13, device="cuda", generator=g)[1:]
+    a, b = [p.clone().requires_grad_() for p in ps], [p.double().requires_grad_() for p in ps]
+    a[-1] = torch.nn.Parameter(ps[-1])
+    kw = dict(lr=1e-2, betas=(0.9, 0.98))
+    oa = AdamW([{"params": a[:3], "weight_decay": 0.1}, {"params": a[3:], "weight_decay": 0.0}], **kw)
+    ob = torch.optim.AdamW([{"params": b[:3], "weight_decay": 0.1}, {"params": b[3:], "weight_decay": 0.0}], **kw)
+    for step in range(4):
+        for i, (p, q) in enumerate(zip(a, b)):
+            d = torch.randn(p.shape, device="cuda", generator=g)
+            p.grad, q.grad = (None, None) if i == 4 and step == 1 else (d.clone(), d.double())
+        assert oa._covers()
+        oa.step(max_norm=max_norm)
+        if max_norm:
+            torch.nn.utils.clip_grad_norm_(b, max_norm)
+        ob.step()
+        for p, q in zip(a, b):
+            assert _rel(p.detach(), q.detach()) < 2e-6
+            if p.grad is not None:
+                assert _rel(p.grad, q.grad) < 2e-6
+    sa, sb = oa.state_dict(), ob.state_dict()
+    assert sa["param_groups"][0].keys() == sb["param_groups"][0].keys()
+    assert all(float(sa["state"][i]["step"]) == float(sb["state"][i]["step"]) for i in sb["state"])
+    again = AdamW([{"params": a[:3], "weight_decay": 0.1}, {"params": a[3:], "weight_decay": 0.0}], **kw)
+    again.load_state_dict(sa)
+    again.step(max_norm=max_norm)
