@@ -700,6 +700,223 @@ void prefill_attention(Tensor out, Tensor q, c10::optional<Tensor> k, c10::optio
   nga::launch_prefill_attention(p, (int)B, (int)max_q_len, (int)D, causal, cur_stream(q));
 }
 
+// ------------------------------------------------------------------ training steps (train.hip)
+// weights and biases of a step: all fp32 or all bf16, [n], contiguous, 16-byte aligned
+const void* train_weight(const Tensor& t, int64_t n, bool& w32, bool first) {
+  CHECK_DEV(t); CHECK_CONTIG(t);
+  const bool f = t.scalar_type() == at::kFloat;
+  TORCH_CHECK((f || t.scalar_type() == at::kBFloat16) && t.numel() == n && (first || f == w32) &&
+                  reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, "train: weight [", n, "], fp32 or bf16");
+  w32 = f;
+  return t.data_ptr();
+}
+
+void train_rows(const Tensor& t, int64_t R, int64_t C) {
+  CHECK_BF16(t); CHECK_CONTIG(t);
+  TORCH_CHECK(t.numel() == R * C && C % 8 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, "train: rows [", R, ", ", C, "]");
+}
+
+// (xn, its squares in fp32); o none: (x, squares)
+std::vector<Tensor> rms_sq(Tensor x, c10::optional<Tensor> o) {
+  const int64_t H = x.size(-1), R = H ? x.numel() / H : 0;
+  train_rows(x, R, H);
+  Tensor xn = x, sq = at::empty(x.sizes(), x.options().dtype(at::kFloat));
+  if (o.has_value()) {
+    train_rows(*o, R, H);
+    xn = at::empty_like(x);
+  }
+  nga::launch_rms_sq(bfp(x), cbfp(o), x.numel(), bfp(xn), sq.data_ptr<float>(), cur_stream(x));
+  post_launch("rms_sq");
+  return {xn, sq};
+}
+
+// (y, rstd [R]) from the rows' mean squares ms
+std::vector<Tensor> rms_apply(Tensor xn, Tensor ms, Tensor w, double eps) {
+  const int64_t H = xn.size(-1), R = H ? xn.numel() / H : 0;
+  train_rows(xn, R, H);
+  CHECK_F32(ms);
+  TORCH_CHECK(ms.numel() == R && H >= 8 && H <= 8192, "rms_apply");
+  bool w32 = false;
+  const void* wp = train_weight(w, H, w32, true);
+  Tensor y = at::empty_like(xn), rstd = at::empty({R}, ms.options());
+  nga::launch_rms_apply(bfp(xn), ms.data_ptr<float>(), wp, w32, (float)eps, R, (int)H, bfp(y), rstd.data_ptr<float>(), cur_stream(xn));
+  post_launch("rms_apply");
+  return {y, rstd};
+}
+
+// ((dy w) xn in fp32, dw fp32 or an empty tensor)
+std::vector<Tensor> rms_prod(Tensor dy, Tensor xn, Tensor w, Tensor rstd, bool want_dw) {
+  const int64_t H = xn.size(-1), R = H ? xn.numel() / H : 0;
+  train_rows(xn, R, H); train_rows(dy, R, H);
+  CHECK_F32(rstd);
+  TORCH_CHECK(rstd.numel() == R && H >= 8 && H <= 8192, "rms_prod");
+  bool w32 = false;
+  const void* wp = train_weight(w, H, w32, true);
+  const auto f = xn.options().dtype(at::kFloat);
+  Tensor prod = at::empty(xn.sizes(), f), dw = at::empty({0}, f), part;
+  if (want_dw) {
+    dw = R ? at::empty({H}, f) : at::zeros({H}, f);
+    part = at::empty({nga::train_parts(R), H}, f);
+  }
+  nga::launch_rms_prod(bfp(dy), bfp(xn), wp, w32, rstd.data_ptr<float>(), R, (int)H, prod.data_ptr<float>(),
+                       want_dw ? part.data_ptr<float>() : nullptr, want_dw ? dw.data_ptr<float>() : nullptr, cur_stream(xn));
+  post_launch("rms_prod");
+  return {prod, dw};
+}
+
+Tensor rms_dx(Tensor dy, Tensor xn, Tensor w, Tensor rstd, Tensor dr, c10::optional<Tensor> dxn) {
+  const int64_t H = xn.size(-1), R = H ? xn.numel() / H : 0;
+  train_rows(xn, R, H); train_rows(dy, R, H);
+  if (dxn.has_value()) train_rows(*dxn, R, H);
+  CHECK_F32(rstd); CHECK_F32(dr);
+  TORCH_CHECK(rstd.numel() == R && dr.numel() == R && H >= 8 && H <= 8192, "rms_dx");
+  bool w32 = false;
+  const void* wp = train_weight(w, H, w32, true);
+  Tensor dx = at::empty_like(xn);
+  nga::launch_rms_dx(bfp(dy), bfp(xn), wp, w32, rstd.data_ptr<float>(), dr.data_ptr<float>(), cbfp(dxn), R, (int)H, bfp(dx),
+                     cur_stream(xn));
+  post_launch("rms_dx");
+  return dx;
+}
+
+// (dx, dw fp32 or an empty tensor)
+std::vector<Tensor> rms_bwd(Tensor xn, Tensor rstd, Tensor w, Tensor dy, c10::optional<Tensor> dxn, bool want_dw) {
+  const int64_t H = xn.size(-1), R = H ? xn.numel() / H : 0;
+  train_rows(xn, R, H); train_rows(dy, R, H);
+  if (dxn.has_value()) train_rows(*dxn, R, H);
+  CHECK_F32(rstd);
+  TORCH_CHECK(H >= 8 && H <= 8192 && rstd.numel() == R, "rms_bwd");
+  bool w32 = false;
+  const void* wp = train_weight(w, H, w32, true);
+  const auto f = xn.options().dtype(at::kFloat);
+  Tensor dx = at::empty_like(xn), dw, part;
+  if (want_dw) {
+    dw = R ? at::empty({H}, f) : at::zeros({H}, f);
+    part = at::empty({nga::train_parts(R), H}, f);
+  }
+  nga::launch_rms_bwd(bfp(xn), rstd.data_ptr<float>(), wp, w32, bfp(dy), cbfp(dxn), R, (int)H, bfp(dx),
+                      want_dw ? part.data_ptr<float>() : nullptr, want_dw ? dw.data_ptr<float>() : nullptr, cur_stream(xn));
+  post_launch("rms_bwd");
+  return {dx, want_dw ? dw : at::empty({0}, f)};
+}
+
+// x + o in fp32
+Tensor add_f32(Tensor x, Tensor o) {
+  const int64_t H = x.size(-1), R = H ? x.numel() / H : 0;
+  train_rows(x, R, H); train_rows(o, R, H);
+  Tensor s = at::empty(x.sizes(), x.options().dtype(at::kFloat));
+  nga::launch_add_f32(bfp(x), bfp(o), x.numel(), s.data_ptr<float>(), cur_stream(x));
+  post_launch("add_f32");
+  return s;
+}
+
+// gradients [2, H] of a layer norm's weight and bias
+Tensor ln_sums(Tensor s, Tensor mean, Tensor rstd, Tensor dy) {
+  const int64_t H = s.size(-1), R = H ? s.numel() / H : 0;
+  train_rows(dy, R, H);
+  CHECK_F32(s); CHECK_F32(mean); CHECK_F32(rstd);
+  TORCH_CHECK(mean.numel() == R && rstd.numel() == R && H >= 8 && H <= 8192 && reinterpret_cast<uintptr_t>(s.data_ptr()) % 16 == 0,
+              "ln_sums");
+  Tensor part = at::empty({nga::train_parts(R), 2, H}, s.options()), out = R ? at::empty({2, H}, s.options()) : at::zeros({2, H}, s.options());
+  nga::launch_ln_sums(s.data_ptr<float>(), mean.data_ptr<float>(), rstd.data_ptr<float>(), bfp(dy), R, (int)H, part.data_ptr<float>(),
+                      out.data_ptr<float>(), cur_stream(s));
+  post_launch("ln_sums");
+  return out;
+}
+
+// GELU of z, or its gradient for dh
+Tensor gelu_rows(Tensor z, c10::optional<Tensor> dh) {
+  const int64_t F = z.size(-1), R = F ? z.numel() / F : 0;
+  train_rows(z, R, F);
+  if (dh.has_value()) train_rows(*dh, R, F);
+  Tensor out = at::empty_like(z);
+  nga::launch_gelu(bfp(z), cbfp(dh), z.numel(), bfp(out), cur_stream(z));
+  post_launch("gelu_rows");
+  return out;
+}
+
+// column sums of bf16 rows in fp32
+Tensor col_sums(Tensor x) {
+  CHECK_BF16(x);
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.size(1) % 8 == 0 &&
+                  reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0, "col_sums: rows at 16-byte addresses");
+  const int64_t R = x.size(0), F = x.size(1);
+  const auto f = x.options().dtype(at::kFloat);
+  if (R == 0 || F == 0) return at::zeros({F}, f);
+  Tensor part = at::empty({nga::train_col_parts(R, (int)F), F}, f), out = at::empty({F}, f);
+  nga::launch_col_sums(bfp(x), x.stride(0), R, (int)F, part.data_ptr<float>(), out.data_ptr<float>(), cur_stream(x));
+  post_launch("col_sums");
+  return out;
+}
+
+// silu(gate) up of [gate | up] rows, or the gradient of those for dh
+Tensor swiglu_rows(Tensor gu, c10::optional<Tensor> dh) {
+  const int64_t F = gu.size(-1) / 2, R = F ? gu.numel() / (2 * F) : 0;
+  train_rows(gu, R, 2 * F);
+  TORCH_CHECK(F % 8 == 0, "swiglu_rows");
+  if (dh.has_value()) train_rows(*dh, R, F);
+  auto sizes = gu.sizes().vec();
+  if (!dh.has_value()) sizes.back() = F;
+  Tensor out = at::empty(sizes, gu.options());
+  nga::launch_swiglu(bfp(gu), cbfp(dh), R, (int)F, bfp(out), cur_stream(gu));
+  post_launch("swiglu_rows");
+  return out;
+}
+
+// y += scale d (as bf16), in place
+void add_scaled(Tensor y, Tensor d, double scale) {
+  const int64_t H = y.size(-1), R = H ? y.numel() / H : 0;
+  train_rows(y, R, H); train_rows(d, R, H);
+  nga::launch_add_scaled(bfp(d), (float)scale, y.numel(), bfp(y), cur_stream(y));
+  post_launch("add_scaled");
+}
+
+// rows [T, nh D], first nr heads rotated by cs [P, D] (row t % P); inplace or a new tensor
+Tensor rope_rows(Tensor x, Tensor cs, int64_t nr, int64_t nh, int64_t D, bool back, bool inplace) {
+  TORCH_CHECK(D % 16 == 0 && D >= 16 && nr >= 0 && nr <= nh && nh >= 1, "rope_rows: head size a multiple of 16");
+  const int64_t T = x.numel() / (nh * D);
+  train_rows(x, T, nh * D);
+  CHECK_F32(cs);
+  TORCH_CHECK(cs.dim() == 2 && cs.size(1) == D && (T == 0 || cs.size(0) >= 1) && reinterpret_cast<uintptr_t>(cs.data_ptr()) % 16 == 0,
+              "rope_rows: cs [P, D]");
+  Tensor out = inplace ? x : at::empty_like(x);
+  nga::launch_rope_rows(bfp(x), cs.data_ptr<float>(), T, cs.size(0), (int)nr, (int)nh, (int)D, back ? -1.f : 1.f, bfp(out), cur_stream(x));
+  post_launch("rope_rows");
+  return out;
+}
+
+// (loss [R], lse [R]) of bf16 logits [R, V]
+std::vector<Tensor> ce_fwd(Tensor lg, Tensor y) {
+  const int64_t R = lg.size(0), V = lg.size(1);
+  train_rows(lg, R, V);
+  CHECK_DEV(y); CHECK_DT(y, at::kLong); CHECK_CONTIG(y);
+  TORCH_CHECK(y.numel() == R, "ce_fwd: one label a row");
+  const auto f = lg.options().dtype(at::kFloat);
+  Tensor loss = at::empty({R}, f), lse = at::empty({R}, f);
+  nga::launch_ce_fwd(bfp(lg), y.data_ptr<int64_t>(), R, V, lse.data_ptr<float>(), loss.data_ptr<float>(), cur_stream(lg));
+  post_launch("ce_fwd");
+  return {loss, lse};
+}
+
+// gradient in bf16 from bf16 logits and their lse, or (lse none) from fp32 log softmax rows
+Tensor ce_bwd(Tensor x, Tensor y, c10::optional<Tensor> lse, Tensor scale) {
+  const int64_t R = x.size(0), V = x.size(1);
+  CHECK_DEV(x); CHECK_DT(x, lse.has_value() ? at::kBFloat16 : at::kFloat); CHECK_CONTIG(x);
+  TORCH_CHECK(V % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0, "ce_bwd: rows");
+  CHECK_DEV(y); CHECK_DT(y, at::kLong); CHECK_CONTIG(y);
+  CHECK_F32(scale);
+  TORCH_CHECK(y.numel() == R && scale.numel() == 1, "ce_bwd");
+  if (lse.has_value()) {
+    CHECK_F32(*lse);
+    TORCH_CHECK(lse->numel() == R, "ce_bwd");
+  }
+  Tensor d = at::empty(x.sizes(), x.options().dtype(at::kBFloat16));
+  nga::launch_ce_bwd(x.data_ptr(), y.data_ptr<int64_t>(), lse.has_value() ? lse->data_ptr<float>() : nullptr, scale.data_ptr<float>(), R, V,
+                     bfp(d), cur_stream(x));
+  post_launch("ce_bwd");
+  return d;
+}
+
 // tables of at most OPT_TENSORS tensors each; fn(table) for every one
 template <typename F>
 int64_t opt_tables(const std::vector<Tensor>& p, const std::vector<Tensor>& g, const std::vector<Tensor>& m,
@@ -2420,6 +2637,20 @@ PYBIND11_MODULE(_C, m) {
   m.def("score", checked("score", &score));
   m.def("topk", checked("topk", &topk));
   m.def("encoder_forward", &encoder_forward);
+  m.def("rms_sq", &rms_sq);
+  m.def("rms_apply", &rms_apply);
+  m.def("rms_prod", &rms_prod);
+  m.def("rms_dx", &rms_dx);
+  m.def("rms_bwd", &rms_bwd);
+  m.def("add_f32", &add_f32);
+  m.def("ln_sums", &ln_sums);
+  m.def("gelu_rows", &gelu_rows);
+  m.def("col_sums", &col_sums);
+  m.def("swiglu_rows", &swiglu_rows);
+  m.def("add_scaled", &add_scaled);
+  m.def("rope_rows", &rope_rows);
+  m.def("ce_fwd", &ce_fwd);
+  m.def("ce_bwd", &ce_bwd);
   m.def("grad_norm", &grad_norm);
   m.def("adamw", &adamw);
   m.def("flat_search", &flat_search);

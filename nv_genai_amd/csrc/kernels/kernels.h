@@ -197,6 +197,30 @@ void launch_embed_layernorm(const int32_t* ids, const int32_t* pos, const int32_
                             const uint16_t* ptab, int n_pos, const uint16_t* ttab, int n_type, const uint16_t* g,
                             const uint16_t* b, float eps, int64_t rows, int H, uint16_t* out, hipStream_t stream);
 
+// train.hip: w32: weights and biases are fp32 (else bf16)
+int train_parts(int64_t R);                  // rows of `part` of the norms' backward
+int train_col_parts(int64_t R, int F);       // of launch_col_sums
+void launch_rms_sq(const uint16_t* x, const uint16_t* o, int64_t n, uint16_t* xn, float* sq, hipStream_t st);
+void launch_rms_apply(const uint16_t* xn, const float* ms, const void* w, bool w32, float eps, int64_t R, int H, uint16_t* y,
+                      float* rstd, hipStream_t st);
+void launch_rms_prod(const uint16_t* dy, const uint16_t* xn, const void* w, bool w32, const float* rstd, int64_t R, int H,
+                     float* prod, float* part, float* dw, hipStream_t st);
+void launch_rms_dx(const uint16_t* dy, const uint16_t* xn, const void* w, bool w32, const float* rstd, const float* dr,
+                   const uint16_t* dxn, int64_t R, int H, uint16_t* dx, hipStream_t st);
+void launch_rms_bwd(const uint16_t* xn, const float* rstd, const void* w, bool w32, const uint16_t* dy, const uint16_t* dxn,
+                    int64_t R, int H, uint16_t* dx, float* part, float* dw, hipStream_t st);
+void launch_add_f32(const uint16_t* x, const uint16_t* o, int64_t n, float* s, hipStream_t st);
+void launch_ln_sums(const float* s, const float* mean, const float* rstd, const uint16_t* dy, int64_t R, int H, float* part,
+                    float* sums, hipStream_t st);
+void launch_gelu(const uint16_t* z, const uint16_t* dh, int64_t n, uint16_t* out, hipStream_t st);
+void launch_col_sums(const uint16_t* x, int64_t ld, int64_t R, int F, float* part, float* out, hipStream_t st);
+void launch_swiglu(const uint16_t* gu, const uint16_t* dh, int64_t R, int F, uint16_t* out, hipStream_t st);
+void launch_add_scaled(const uint16_t* d, float scale, int64_t n, uint16_t* y, hipStream_t st);
+void launch_rope_rows(const uint16_t* in, const float* cs, int64_t T, int64_t P, int nr, int nh, int D, float sign, uint16_t* out,
+                      hipStream_t st);
+void launch_ce_fwd(const uint16_t* lg, const int64_t* y, int64_t R, int64_t V, float* lse, float* loss, hipStream_t st);
+void launch_ce_bwd(const void* x, const int64_t* y, const float* lse, const float* scale, int64_t R, int64_t V, uint16_t* d,
+                   hipStream_t st);
 // adamw.hip
 constexpr int OPT_TENSORS = 48;
 constexpr int OPT_CHUNK = 32768;

@@ -2,11 +2,15 @@
 
 The serving forwards (models/llama.py, models/encoder.py) run packed tokens through the
 hand-written gfx950 kernels, which have no backward. Training runs the same weights through
-autograd-capable PyTorch-ROCm ops on padded ``[B, S]`` batches:
+autograd on padded ``[B, S]`` batches:
 
 * matmuls in bf16 (``torch.autocast``) on MFMA via hipBLASLt, fp32 accumulation;
 * attention through ``F.scaled_dot_product_attention`` (the flash/memory-efficient backends
   of PyTorch-ROCm), causal for the LLM, key-padding-masked for the encoder;
+* on the GPU norms with their residual, activations, rotation and cross entropy through the functions of
+  :mod:`.fused`, elsewhere and for what those do not take through torch operations. All weights trained, they
+  keep every bit of the torch operations' activations and gradients (full fine-tuning goes on as it did), with
+  adapters those of the activations, and the gradients take the forms that are a single pass;
 * RMSNorm / LayerNorm / softmax statistics in fp32.
 
 Parameters are taken from the serving model objects by reference (no copy), so a LoRA
@@ -24,6 +28,8 @@ from typing import Callable, Dict, Optional
 import torch
 import torch.nn.functional as F
 from torch.utils.checkpoint import checkpoint as _ckpt
+
+from . import fused
 
 LinearFn = Callable[[torch.Tensor, int, str], torch.Tensor]
 
@@ -71,7 +77,9 @@ def llama_hidden(model, ids: torch.Tensor, linear: Optional[LinearFn] = None,
     cos, sin = cs[..., : D // 2].unsqueeze(2), cs[..., D // 2:].unsqueeze(2)
     dt = torch.bfloat16
     layer_norm = cfg.norm == "layer"
-    amask = _window_mask(S, cfg.sliding_window, ids.device) if cfg.sliding_window and S > cfg.sliding_window else None
+    window = cfg.sliding_window if cfg.sliding_window and S > cfg.sliding_window else 0
+    amask = None   # made where it is needed
+    once = linear is not None
 
     def W(li, name):
         return P.get((li, name), model.layers[li].get(name) if li >= 0 else None)
@@ -111,6 +119,8 @@ def llama_hidden(model, ids: torch.Tensor, linear: Optional[LinearFn] = None,
             return out.to(h.dtype).view_as(h)
         gu = lin(h, li, "wgu", "bgu")
         if cfg.gated_mlp:
+            if cfg.act == "silu" and fused.swiglu_usable(gu):
+                return lin(fused.swiglu(gu), li, "wd", "bd")
             g, u = gu.chunk(2, dim=-1)
             return lin(act(g) * u, li, "wd", "bd")
         return lin(act(gu), li, "wd", "bd")
@@ -120,26 +130,48 @@ def llama_hidden(model, ids: torch.Tensor, linear: Optional[LinearFn] = None,
     if cfg.embed_scale != 1.0:
         x = x * torch.tensor(cfg.embed_scale, dtype=dt)
 
-    def layer(x, li):
-        h = norm(x, li, "attn_norm")
-        qkv = lin(h, li, "wqkv", "bqkv")
+    # rotation rows
+    rows = cs.reshape(B * S, D).float().contiguous() if fused.rope_usable(x, D) else None
+
+    def attend(qkv):
+        nonlocal amask
+        fits = rows is not None and fused.rope_usable(qkv, D)
+        if fits:
+            qkv = fused.rope(qkv, rows, hq + hkv, hq + 2 * hkv, D)
         q, k, v = qkv.split([hq * D, hkv * D, hkv * D], dim=-1)
-        q = apply_rope(q.view(B, S, hq, D), cos, sin).transpose(1, 2)
-        k = apply_rope(k.view(B, S, hkv, D), cos, sin).transpose(1, 2)
-        v = v.view(B, S, hkv, D).transpose(1, 2)
-        if amask is None:
-            a = F.scaled_dot_product_attention(q, k, v, is_causal=True, scale=model.scale, enable_gqa=hq != hkv)
-        else:
-            a = F.scaled_dot_product_attention(q, k, v, attn_mask=amask, scale=model.scale, enable_gqa=hq != hkv)
-        a = a.transpose(1, 2).reshape(B, S, hq * D)
-        x = x + lin(a, li, "wo", "bo")
+        q, k, v = q.view(B, S, hq, D), k.view(B, S, hkv, D), v.view(B, S, hkv, D).transpose(1, 2)
+        if not fits:
+            q, k = apply_rope(q, cos, sin), apply_rope(k, cos, sin)
+        q, k = q.transpose(1, 2), k.transpose(1, 2)
+        if window and amask is None:
+            amask = _window_mask(S, window, ids.device)
+        a = F.scaled_dot_product_attention(q, k, v, attn_mask=amask, is_causal=not window, scale=model.scale, enable_gqa=hq != hkv)
+        return a.transpose(1, 2).reshape(B, S, hq * D)
+
+    def layer(x, li):
+        x = x + lin(attend(lin(norm(x, li, "attn_norm"), li, "wqkv", "bqkv")), li, "wo", "bo")
         return x + mlp(norm(x, li, "mlp_norm"), li)
 
-    for li in range(len(model.layers)):
-        if grad_ckpt and torch.is_grad_enabled():
-            x = _ckpt(layer, x, li, use_reentrant=False)
-        else:
-            x = layer(x, li)
+    def joined(x, d, li, name):
+        """(x + d, its norm); d is what the last step leaves to be added."""
+        w = W(li, name) if li >= 0 else P.get(name, getattr(model, name))
+        return (x, fused.rms_norm(x, w, cfg.eps, once)) if d is None else fused.add_rms_norm(x, d, w, cfg.eps, once)
+
+    def layer_joined(x, d, li):
+        x, h = joined(x, d, li, "attn_norm")
+        x, h = joined(x, lin(attend(lin(h, li, "wqkv", "bqkv")), li, "wo", "bo"), li, "mlp_norm")
+        return x, mlp(h, li)
+
+    ckpt = grad_ckpt and torch.is_grad_enabled()
+    n = len(model.layers)
+    if not layer_norm and x.numel() and fused.usable(
+            x, P.get("final_norm", model.final_norm), *(W(li, w) for li in range(n) for w in ("attn_norm", "mlp_norm"))):
+        d = None
+        for li in range(n):
+            x, d = _ckpt(layer_joined, x, d, li, use_reentrant=False) if ckpt else layer_joined(x, d, li)
+        return joined(x, d, -1, "final_norm")[1]
+    for li in range(n):
+        x = _ckpt(layer, x, li, use_reentrant=False) if ckpt else layer(x, li)
     return norm(x, -1, "final_norm")
 
 
@@ -157,8 +189,11 @@ def lm_loss(model, hidden: torch.Tensor, labels: torch.Tensor, params: Optional[
     h, y = h.index_select(0, keep), y.index_select(0, keep)
     total = h.new_zeros((), dtype=torch.float32)
     for s in range(0, h.shape[0], chunk):
-        lg = (h[s:s + chunk] @ head.t()).float()
-        total = total + F.cross_entropy(lg, y[s:s + chunk], reduction="sum")
+        lg = h[s:s + chunk] @ head.t()
+        if fused.cross_entropy_usable(lg):
+            total = total + fused.cross_entropy_sum(lg, y[s:s + chunk], params is None)
+        else:
+            total = total + F.cross_entropy(lg.float(), y[s:s + chunk], reduction="sum")
     return total / max(1, y.numel())
 
 
@@ -181,17 +216,25 @@ def encoder_embed(model, ids: torch.Tensor, mask: torch.Tensor, params: Optional
                      cfg.eps).to(dt)
     amask = mask.bool()[:, None, None, :]
 
+    def lin(x, li, w, b):
+        w, b = g(li, w), g(li, b)
+        if fused.usable(x, w, b) and w.shape[0] % 8 == 0:
+            return fused.linear(x, w, b)
+        return F.linear(x, w.to(dt), b.to(dt))
+
+    def add_norm(x, o, li, n):
+        w, b = g(li, n + "_g"), g(li, n + "_b")
+        if fused.usable(x, w, b):
+            return fused.residual_layer_norm(x, o, w, b, cfg.eps)
+        return F.layer_norm((x.float() + o.float()), (H,), w.float(), b.float(), cfg.eps).to(dt)
+
     def layer(x, li):
-        qkv = F.linear(x, g(li, "wqkv").to(dt), g(li, "bqkv").to(dt))
-        q, k, v = (t.view(B, S, nh, hd).transpose(1, 2) for t in qkv.split(H, dim=-1))
+        q, k, v = (t.view(B, S, nh, hd).transpose(1, 2) for t in lin(x, li, "wqkv", "bqkv").split(H, dim=-1))
         a = F.scaled_dot_product_attention(q, k, v, attn_mask=amask, scale=model.scale)
-        a = a.transpose(1, 2).reshape(B, S, H)
-        o = F.linear(a, g(li, "wo").to(dt), g(li, "bo").to(dt))
-        x = F.layer_norm((x.float() + o.float()), (H,), g(li, "ln1_g").float(), g(li, "ln1_b").float(), cfg.eps).to(dt)
-        h = F.gelu(F.linear(x, g(li, "wi").to(dt), g(li, "bi").to(dt)).float()).to(dt)
-        o2 = F.linear(h, g(li, "wo2").to(dt), g(li, "bo2").to(dt))
-        return F.layer_norm((x.float() + o2.float()), (H,), g(li, "ln2_g").float(), g(li, "ln2_b").float(),
-                            cfg.eps).to(dt)
+        x = add_norm(x, lin(a.transpose(1, 2).reshape(B, S, H), li, "wo", "bo"), li, "ln1")
+        z = lin(x, li, "wi", "bi")
+        h = fused.gelu(z) if fused.usable(z) else F.gelu(z.float()).to(dt)
+        return add_norm(x, lin(h, li, "wo2", "bo2"), li, "ln2")
 
     for li in range(len(model.layers)):
         x = _ckpt(layer, x, li, use_reentrant=False) if grad_ckpt and torch.is_grad_enabled() else layer(x, li)

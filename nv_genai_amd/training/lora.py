@@ -17,6 +17,8 @@ from typing import Dict, Sequence, Tuple
 
 import torch
 
+from . import fused
+
 TARGETS = {"qkv": "wqkv", "o": "wo", "gate_up": "wgu", "down": "wd"}
 
 
@@ -59,8 +61,11 @@ class LoRA:
             yield f"layers.{k[0]}.{k[1]}.lora_B", self.B[k]
 
     def linear(self, x: torch.Tensor, li: int, name: str) -> torch.Tensor:
-        y = x @ self.model.layers[li][name].t()
-        a = self.A.get((li, name))
+        w, a = self.model.layers[li][name], self.A.get((li, name))
+        if (a is not None and not w.requires_grad and w.dtype == torch.bfloat16 and w.shape[0] % 8 == 0
+                and fused.usable(x, w, a, self.B[(li, name)]) and not (self.cfg.dropout and torch.is_grad_enabled())):
+            return fused.lora_linear(x, w, a, self.B[(li, name)], self.cfg.scale)
+        y = x @ w.t()
         if a is None:
             return y
         h = x
