@@ -89,6 +89,7 @@ def _run(cmd):
 PER_FILE_FLAGS = {
     "attention_prefill": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "attention_varlen": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "attention_backward": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "linear_scan": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 

@@ -700,6 +700,42 @@ void prefill_attention(Tensor out, Tensor q, c10::optional<Tensor> k, c10::optio
   nga::launch_prefill_attention(p, (int)B, (int)max_q_len, (int)D, causal, cur_stream(q));
 }
 
+// ------------------------------------------------------------------ attention with gradients (packed rows)
+void train_attn_check(const Tensor& t, int64_t T, int64_t cols) {
+  CHECK_BF16(t);
+  TORCH_CHECK(t.dim() == 2 && t.size(0) == T && t.size(1) == cols && t.stride(1) == 1 && t.stride(0) % 8 == 0 &&
+                  reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0,
+              "attention: rows of ", cols, " bf16 values at 16-byte addresses");
+}
+
+// gradients of causal attention of q [T, Hq D], k and v [T, Hkv D] over the sequences of cu, the longest of max_len; out [T, Hq D];
+// lse [Hq, T]: log2 of each row's sum of exponentials
+void train_attention_backward(Tensor dq, Tensor dk, Tensor dv, Tensor dout, Tensor q, Tensor k, Tensor v, Tensor out, Tensor lse,
+                              Tensor cu, int64_t Hq, int64_t Hkv, int64_t D, int64_t max_len, double scale) {
+  const int64_t T = q.size(0), B = cu.numel() - 1;
+  TORCH_CHECK((D == 32 || D == 64 || D == 128) && Hkv >= 1 && Hq % Hkv == 0, "attention");
+  for (const Tensor& t : {q, out, dout, dq}) train_attn_check(t, T, Hq * D);
+  for (const Tensor& t : {k, v, dk, dv}) train_attn_check(t, T, Hkv * D);
+  TORCH_CHECK(k.stride(0) == v.stride(0) && dk.stride(0) == dv.stride(0), "attention: k and v rows at one stride");
+  CHECK_F32(lse);
+  TORCH_CHECK(lse.numel() == Hq * T && scale > 0, "attention: lse [Hq, T]");
+  CHECK_I32(cu);
+  if (B < 1 || T == 0 || max_len <= 0) return;
+  Tensor delta = at::empty_like(lse), part;
+  nga::AttnBwdParams p{};
+  p.parts = nga::attn_bwd_parts((int)B, (int)max_len, (int)Hq, (int)Hkv);
+  if (p.parts > 1) {
+    part = at::empty({p.parts, 2, T, Hkv * D}, lse.options());
+    p.part = part.data_ptr<float>();
+  }
+  p.q = bfp(q); p.k = bfp(k); p.v = bfp(v); p.out = bfp(out); p.dout = bfp(dout);
+  p.q_stride = q.stride(0); p.kv_stride = k.stride(0); p.out_stride = out.stride(0); p.dout_stride = dout.stride(0);
+  p.lse = lse.data_ptr<float>(); p.delta = delta.data_ptr<float>();
+  p.dq = bfp(dq); p.dk = bfp(dk); p.dv = bfp(dv); p.dq_stride = dq.stride(0); p.dkv_stride = dk.stride(0);
+  p.cu = cu.data_ptr<int32_t>(); p.T = T; p.Hq = (int)Hq; p.Hkv = (int)Hkv; p.scale = (float)scale;
+  nga::launch_varlen_attention_backward(p, (int)B, (int)max_len, (int)D, cur_stream(q));
+}
+
 // ------------------------------------------------------------------ training steps (train.hip)
 // weights and biases of a step: all fp32 or all bf16, [n], contiguous, 16-byte aligned
 const void* train_weight(const Tensor& t, int64_t n, bool& w32, bool first) {
@@ -2653,6 +2689,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("ce_bwd", &ce_bwd);
   m.def("grad_norm", &grad_norm);
   m.def("adamw", &adamw);
+  m.def("train_attention_backward", checked("train_attention_backward", &train_attention_backward));
   m.def("flat_search", &flat_search);
   m.def("ivf_search", &ivf_search);
   m.def("search_covers", [](int64_t d) { return d <= 1024 && nga::scan_chunk((int)d, 1) > 0; });

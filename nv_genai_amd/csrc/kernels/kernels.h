@@ -93,6 +93,24 @@ struct PrefillParams {
   const int32_t* items;
   const int32_t* n_items;
 };
+// attention_backward.hip: gradients of causal attention over packed sequences
+struct AttnBwdParams {
+  const uint16_t *q, *k, *v, *out, *dout;
+  int64_t q_stride, kv_stride, out_stride, dout_stride;
+  const float* lse;    // [Hq, T], log2 of each row's sum of exponentials
+  float* delta;        // [Hq, T] scratch
+  uint16_t *dq, *dk, *dv;
+  int64_t dq_stride, dkv_stride;
+  const int32_t* cu;
+  int64_t T;
+  int Hq, Hkv;
+  float scale;
+  int parts;           // attn_bwd_parts: parts of a KV head's query heads; above 1 through part [parts, 2, T, Hkv D]
+  float* part;
+  int ntiles, per_xcd, total;   // set by the launcher
+};
+int attn_bwd_parts(int num_seqs, int max_len, int Hq, int Hkv);
+void launch_varlen_attention_backward(const AttnBwdParams& p, int num_seqs, int max_len, int D, hipStream_t stream);
 void launch_prefill_attention(const PrefillParams& p, int num_seqs, int max_q_len, int D,
                               bool causal, hipStream_t stream);
 // packed K / V rows (p.k, p.v; 16-byte aligned), head_dim 32, 64 or 128

@@ -6,7 +6,8 @@ autograd on padded ``[B, S]`` batches:
 
 * matmuls in bf16 (``torch.autocast``) on MFMA via hipBLASLt, fp32 accumulation;
 * attention through ``F.scaled_dot_product_attention`` (the flash/memory-efficient backends
-  of PyTorch-ROCm), causal for the LLM, key-padding-masked for the encoder;
+  of PyTorch-ROCm), causal for the LLM, key-padding-masked for the encoder; with adapters
+  the framework's own kernel gives the flash attention's gradients on the GPU;
 * on the GPU norms with their residual, activations, rotation and cross entropy through the functions of
   :mod:`.fused`, elsewhere and for what those do not take through torch operations. All weights trained, they
   keep every bit of the torch operations' activations and gradients (full fine-tuning goes on as it did), with
@@ -130,12 +131,15 @@ def llama_hidden(model, ids: torch.Tensor, linear: Optional[LinearFn] = None,
     if cfg.embed_scale != 1.0:
         x = x * torch.tensor(cfg.embed_scale, dtype=dt)
 
-    # rotation rows
+    # rotation rows, and the sequences' starts for the attention whose gradients are the framework's own
     rows = cs.reshape(B * S, D).float().contiguous() if fused.rope_usable(x, D) else None
+    cu = torch.arange(0, B * S + 1, S, dtype=torch.int32, device=ids.device) if once and rows is not None else None
 
     def attend(qkv):
         nonlocal amask
         fits = rows is not None and fused.rope_usable(qkv, D)
+        if fits and once and not window and fused.attention_usable(qkv, D, hq, hkv, model.scale):
+            return fused.attention(qkv, rows, cu, hq, hkv, D, model.scale)
         if fits:
             qkv = fused.rope(qkv, rows, hq + hkv, hq + 2 * hkv, D)
         q, k, v = qkv.split([hq * D, hkv * D, hkv * D], dim=-1)

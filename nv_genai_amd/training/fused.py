@@ -1,14 +1,15 @@
-"""Autograd functions over the training kernels (csrc/kernels/train.hip).
+"""Autograd functions over the training kernels (csrc/kernels/train.hip, attention_backward.hip).
 
 Each takes the place of a chain of single torch operations in :mod:`.functional` (forward and backward): activations bf16,
 statistics, sums and the gradients of weights fp32, weights either fp32 masters or bf16. Activations are bit for bit those of
-the chain. So are, all weights trained, their gradients; ``lora_linear`` and the ``once`` forms, for adapters,
+the chain. So are, all weights trained, their gradients; ``attention``, ``lora_linear`` and the ``once`` forms, for adapters,
 form them in the kernels' own order. Callers ask ``usable`` first; the torch operations stay for the CPU, other types and
 sizes, and under transforms that pass functions of this kind by (tracing, functorch, forward-mode). Like the flash attention
 that they stand beside they have a first derivative only.
 """
 from __future__ import annotations
 
+import math
 from typing import Optional, Tuple
 
 import torch
@@ -187,6 +188,49 @@ def rope(qkv: torch.Tensor, cs: torch.Tensor, nr: int, nh: int, D: int) -> torch
 
 def rope_usable(x: torch.Tensor, D: int) -> bool:
     return x.is_cuda and x.dtype is BF16 and D % 16 == 0 and x.numel() > 0 and _plain(x)
+
+
+class _Attention(Function):
+    @staticmethod
+    def forward(ctx, qkv, cs, cu, B, hq, hkv, D, scale):
+        r = ops.kernels().rope_rows(_rows(qkv.reshape(-1, (hq + 2 * hkv) * D)), cs, hq + hkv, hq + 2 * hkv, D, False, False)
+        q, k, v = _heads(r.view(B, -1, r.shape[1]), hq, hkv, D)
+        out, lse = torch.ops.aten._scaled_dot_product_flash_attention(q, k, v, 0.0, True, scale=scale)[:2]
+        out = out.transpose(1, 2).reshape(-1, hq * D)
+        ctx.save_for_backward(r, out, lse, cs, cu)
+        ctx.how = (qkv.shape, hq, hkv, D, scale)
+        return out.view(*qkv.shape[:-1], hq * D)
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dout):
+        r, out, lse, cs, cu = ctx.saved_tensors
+        shape, hq, hkv, D, scale = ctx.how
+        C = ops.kernels()
+        d = torch.empty_like(r)
+        w = [hq * D, hkv * D, hkv * D]
+        l2 = (lse.transpose(0, 1) * math.log2(math.e)).reshape(hq, -1).contiguous()
+        C.train_attention_backward(*d.split(w, 1), _rows(dout.reshape(-1, hq * D)), *r.split(w, 1), out, l2, cu, hq, hkv, D, lse.shape[2],
+                                   scale)
+        C.rope_rows(d, cs, hq + hkv, hq + 2 * hkv, D, True, True)
+        return (d.view(shape),) + (None,) * 7
+
+
+def _heads(qkv, hq, hkv, D):
+    return (t.unflatten(-1, (-1, D)).transpose(1, 2) for t in qkv.split([hq * D, hkv * D, hkv * D], -1))
+
+
+def attention(qkv: torch.Tensor, cs: torch.Tensor, cu: torch.Tensor, hq: int, hkv: int, D: int, scale: float) -> torch.Tensor:
+    """Causal attention of qkv [B, S, (hq + 2 hkv) D], q and k rotated as ``rope`` does, whose gradients come from the framework's
+    kernel; cu: the sequences' starts [B + 1], int32."""
+    return _Attention.apply(qkv, cs, cu, qkv.shape[0], hq, hkv, D, float(scale))
+
+
+def attention_usable(qkv: torch.Tensor, D: int, hq: int, hkv: int, scale: float) -> bool:
+    """Whether ``attention`` takes qkv, and torch would take its flash attention for it (1), whose output that gives."""
+    if not (rope_usable(qkv, D) and D in (32, 64, 128) and hkv >= 1 and hq % hkv == 0 and scale > 0):
+        return False
+    return torch._fused_sdp_choice(*_heads(qkv.detach(), hq, hkv, D), None, 0.0, True, scale=scale, enable_gqa=hq != hkv) == 1
 
 
 class _CrossEntropySum(Function):

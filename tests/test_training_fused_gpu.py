@@ -4,6 +4,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from nv_genai_amd import ops
 from nv_genai_amd.training import functional as Fn
 from nv_genai_amd.training import fused
 
@@ -115,6 +116,47 @@ def test_rope(gpu, T, P, hq, hkv, D):
         return torch.cat([Fn.apply_rope(h[:, :, : hq + hkv], c, s), h[:, :, hq + hkv:]], 2).reshape(T, -1)
 
     _bits(lambda x: fused.rope(x, cs, hq + hkv, hq + 2 * hkv, D), ref, [_bf(T, (hq + 2 * hkv) * D)])
+
+
+def _causal(q, k, v, n):
+    """[n, heads, D] in 64 bits; also the rows' log-sums."""
+    k, v = (t.repeat_interleave(q.shape[1] // t.shape[1], 1).transpose(0, 1) for t in (k, v))
+    s = q.transpose(0, 1) @ k.transpose(1, 2) * q.shape[2] ** -0.5
+    s = s.masked_fill(torch.ones(n, n, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+    return (torch.softmax(s, -1) @ v).transpose(0, 1).flatten(1), torch.logsumexp(s, -1)
+
+
+@pytest.mark.parametrize("lens", [[1], [64, 65], [128, 129, 31], [300, 1, 257]])
+@pytest.mark.parametrize("D,hq,hkv", [(32, 3, 3), (64, 4, 1), (128, 8, 2)])
+def test_attention_backward(gpu, lens, D, hq, hkv):
+    T, w = sum(lens), [hq * D, hkv * D, hkv * D]
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0).tolist()), dtype=torch.int32, device="cuda")
+    qkv, dout = _bf(T, sum(w)), _bf(T, hq * D, seed=4)
+    x = qkv.double().requires_grad_()
+    parts = [_causal(*(t[a:a + n].unflatten(1, (-1, D)) for t in x.split(w, 1)), n) for a, n in zip(cu.tolist(), lens)]
+    ref = torch.cat([p[0] for p in parts])
+    want = torch.autograd.grad(ref, x, dout.double())[0].split(w, 1)
+    lse = torch.cat([p[1] for p in parts], 1).detach().float() * 1.4426950408889634
+    d = torch.empty_like(qkv)
+    ops.kernels().train_attention_backward(*d.split(w, 1), dout, *qkv.split(w, 1), ref.detach().to(BF), lse, cu, hq, hkv, D, max(lens), D ** -0.5)
+    # probabilities, their gradient and the result round to bf16, 2^-9 each: 6e-3; a lone key's p (dp - delta) cancels in full
+    for p, q in zip(d.split(w, 1), want):
+        assert _rel(p, q) < 6e-3 or (T == 1 and (p.double() - q).abs().max() < 0.1), _rel(p, q)
+
+
+@pytest.mark.parametrize("B,S,D,hq,hkv", [(1, 1, 64, 2, 2), (2, 130, 64, 4, 1), (3, 77, 128, 8, 2)])
+def test_attention_matches_torch_operations(gpu, B, S, D, hq, hkv):
+    a = torch.arange(B * S, device="cuda")[:, None] % S * 10000.0 ** (-torch.arange(D // 2, device="cuda") / (D // 2))
+    cs = torch.cat([a.cos(), a.sin()], 1).float()
+    cu = torch.arange(0, B * S + 1, S, dtype=torch.int32, device="cuda")
+    x = _bf(B, S, (hq + 2 * hkv) * D).requires_grad_()
+    assert fused.attention_usable(x, D, hq, hkv, D ** -0.5)
+    ya = fused.attention(x, cs, cu, hq, hkv, D, D ** -0.5)
+    q, k, v = fused._heads(fused.rope(x, cs, hq + hkv, hq + 2 * hkv, D), hq, hkv, D)
+    yb = F.scaled_dot_product_attention(q, k, v, is_causal=True, scale=D ** -0.5, enable_gqa=hq != hkv).transpose(1, 2).reshape(ya.shape)
+    dy = _bf(*ya.shape, seed=6)
+    assert torch.equal(ya, yb)
+    assert _rel(*(torch.autograd.grad(y, x, dy)[0] for y in (ya, yb))) < 1e-2
 
 
 @pytest.mark.parametrize("R,V", [(1, 8), (3, 32768), (65, 50264)])
