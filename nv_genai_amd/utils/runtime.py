@@ -29,8 +29,16 @@ GPU_CAPTURE_LOCK = threading.RLock()
 
 @contextlib.contextmanager
 def capture_guard():
+    """The lock above, and no cyclic collection: one that starts inside a capture destroys whatever unreachable graphs, streams
+    and events an earlier engine left, calls that are not permitted there and invalidate the capture."""
     with GPU_CAPTURE_LOCK:
-        yield
+        on = gc.isenabled()
+        gc.disable()
+        try:
+            yield
+        finally:
+            if on:
+                gc.enable()
 
 
 def quiet_gc(gen0_threshold: int = 50_000) -> None:
