@@ -492,6 +492,24 @@ void gemv(Tensor out, Tensor x, Tensor w, int64_t epi) {
   TORCH_CHECK(nga::launch_gemv(p, (int)epi, cur_stream(x)), "gemv: shape out of range");
 }
 
+void stream_gemm(Tensor out, Tensor x, Tensor w, int64_t epi) {
+  CHECK_DEV(x); CHECK_BF16(x); CHECK_BF16(w);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2, "stream_gemm: 2-D x / w / out");
+  TORCH_CHECK(x.device() == w.device() && x.device() == out.device(), "stream_gemm: one device");
+  const int64_t M = x.size(0), K = x.size(1);
+  TORCH_CHECK(epi >= 0 && epi <= 2 && (epi != 2 || w.size(0) % 2 == 0), "stream_gemm: epi 0 (bf16), 1 (fp32), 2 (SwiGLU)");
+  const int64_t N = epi == 2 ? w.size(0) / 2 : w.size(0);
+  TORCH_CHECK(M <= 16 && K % 256 == 0 && N % 16 == 0 && w.size(1) == K && N < (int64_t(1) << 30), "stream_gemm: M <= 16, K % 256 == 0, N % 16 == 0");
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 8 == 0 && w.is_contiguous() &&
+                  (reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) % 16 == 0,
+              "stream_gemm: 16-byte aligned rows");
+  TORCH_CHECK(out.size(0) == M && out.size(1) == N && out.stride(1) == 1 && out.stride(0) % 4 == 0 &&
+                  reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0 &&
+                  out.scalar_type() == (epi == 1 ? at::kFloat : at::kBFloat16),
+              "stream_gemm: out [M, N]");
+  nga::launch_stream_gemm({bfp(x), x.stride(0), bfp(w), (int)M, (int)N, (int)K, out.data_ptr(), out.stride(0)}, (int)epi, cur_stream(x));
+}
+
 void splitk_swiglu(Tensor out, Tensor P, int64_t S) {
   CHECK_DEV(P); CHECK_BF16(out);
   TORCH_CHECK(out.device() == P.device(), "splitk_swiglu: out and P on one device");
@@ -2666,6 +2684,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("skinny_gemm", checked("skinny_gemm", &skinny_gemm));
   m.def("splitk_reduce", checked("splitk_reduce", &splitk_reduce));
   m.def("splitk_swiglu", checked("splitk_swiglu", &splitk_swiglu));
+  m.def("stream_gemm", checked("stream_gemm", &stream_gemm));
+  m.def("stream_gemm_covers", &nga::stream_gemm_covers);
   m.def("gemv", checked("gemv", &gemv));
   m.def("splitk_add_rmsnorm", checked("splitk_add_rmsnorm", &splitk_add_rmsnorm));
   m.def("sample", checked("sample", &sample));

@@ -1,0 +1,183 @@
+// Decode projections of up to 16 rows: out[M, N] = x[M, K] . W[N, K]^T as one stream of the weights.
+//
+// Nothing but the weights' bytes counts here, and HBM gives them at full rate only in long pieces with much in flight. A wave
+// therefore has a stream of its own: 16 or 32 weight rows (NT), 512 or 256 bytes of each at a time, by LDS-DMA into two private
+// 8-KiB buffers, eight waves a CU, and no barrier before the end. The weight rows are the A operand of 16x16x32 MFMA, the token
+// rows the B operand, from L2 straight into registers one stage ahead. The four waves of a workgroup share the rows and split K;
+// they meet once in LDS, so no partial sums go through memory.
+//
+// Weights from HBM, us at 1 / 4 / 8 / 16 rows, the kernel that did it before and here (before: gemv.hip, then gemm_skinny.hip's
+// table, the K split's sums not counted; its 128 weight rows come in pieces of 128 bytes):
+//   4,096 x 4,096    9.1  8.8  9.2  9.6    7.8  7.9  8.2  9.5
+//   6,144 x 4,096   10.9 11.1 11.5 12.1   10.4 10.6 10.9 12.1
+//   4,096 x 14,336  25.3 22.3 22.7 23.6   21.3 21.5 22.4 26.6
+//   SwiGLU 2 x 14,336 x 4,096   39.4 45.3 48.8 49.1   39.5 39.7 40.6 44.7   (235 MB: 5.3 to 5.9 TB/s)
+// One wave a tile and eight waves were slower everywhere (28,672 rows: 44.8 and 44.4 us for 38.7), and so are 17 to 32 rows,
+// whose tokens cost as much L2 traffic as the weights (SwiGLU above at 32 rows: 55.6, table 49.6).
+#include "common.h"
+#include "kernels.h"
+
+namespace nga {
+
+namespace {
+template <int N>
+__device__ __forceinline__ void st_wait_vm() {
+  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+__device__ __forceinline__ float st_silu(float x) { return x / (1.f + __expf(-x)); }
+}  // namespace
+
+// EPI 0: bf16 out; 1: fp32 out; 2: bf16 silu(gate) up of W = [gate | up] rows, N = F (8 NT features a tile)
+template <int NT, int EPI>
+__global__ void __launch_bounds__(256) stream_gemm_kernel(StreamGemmParams P) {
+  constexpr int NW = 4;
+  constexpr int KS = 256 / NT, CPR = KS / 8, KSTEPS = KS / 32;   // k of a stage, its 16-byte chunks a row, its MFMA steps
+  __shared__ __attribute__((aligned(16))) uint16_t ring[NW * 2 * 4096];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, h = lane >> 4;
+  const int tile = blockIdx.x;
+  const int stages = P.K / KS;
+  const int s0 = stages * wv / NW, s1 = stages * (wv + 1) / NW;
+
+  // chunk c of row r lies at c ^ r (mod 16); with SwiGLU the second half of the rows are up's
+  const uint16_t* wsrc[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int r = 2 * NT * i + lane / CPR, hr = 8 * NT;
+    const int64_t row = EPI == 2 ? (r < hr ? (int64_t)tile * hr + r : (int64_t)P.N + tile * hr + r - hr) : (int64_t)tile * 16 * NT + r;
+    wsrc[i] = P.w + row * P.K + ((lane % CPR ^ (r & 15)) << 3);
+  }
+  const uint16_t* xp = P.x + (int64_t)min(col, P.M - 1) * P.ldx + 8 * h;
+  uint16_t* buf = ring + wv * (2 * 4096);
+
+  auto issue = [&](int s) {
+    uint16_t* b = buf + (s & 1) * 4096;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) glds16(wsrc[i] + (int64_t)s * KS, b + i * 512);
+  };
+  auto load_x = [&](int s, u16x8 (&x)[KSTEPS]) {
+#pragma unroll
+    for (int k = 0; k < KSTEPS; ++k) x[k] = load8(xp + (int64_t)s * KS + 32 * k);
+  };
+  f32x4 acc[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) acc[i] = (f32x4)(0.f);
+  auto multiply = [&](int s, u16x8 (&x)[KSTEPS]) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    const uint16_t* b = buf + (s & 1) * 4096 + col * KS;
+    u16x8 a[NT][KSTEPS];
+#pragma unroll
+    for (int k = 0; k < KSTEPS; ++k)
+#pragma unroll
+      for (int i = 0; i < NT; ++i) a[i][k] = *reinterpret_cast<const u16x8*>(b + i * 16 * KS + (((4 * k + h) ^ col) << 3));
+#pragma unroll
+    for (int k = 0; k < KSTEPS; ++k)
+#pragma unroll
+      for (int i = 0; i < NT; ++i) acc[i] = mfma16(as_bf16x8(a[i][k]), as_bf16x8(x[k]), acc[i]);
+    __builtin_amdgcn_sched_barrier(0);   // the buffer is read before it is filled again
+    asm volatile("" ::: "memory");
+  };
+  // ask for stage s + 1 and its rows y, wait for what was asked for before them, multiply stage s
+  auto step = [&](int s, u16x8 (&x)[KSTEPS], u16x8 (&y)[KSTEPS]) {
+    load_x(s + 1, y);
+    __builtin_amdgcn_sched_barrier(0);
+    issue(s + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    st_wait_vm<8 + KSTEPS>();
+    multiply(s, x);
+  };
+  u16x8 xa[KSTEPS], xb[KSTEPS];
+  if (s0 < s1) {
+    load_x(s0, xa);
+    __builtin_amdgcn_sched_barrier(0);
+    issue(s0);
+    __builtin_amdgcn_sched_barrier(0);
+    int s = s0;   // the last steps apart: a branch around the loads would make the compiler wait for all of them
+    for (; s + 2 < s1; s += 2) {
+      step(s, xa, xb);
+      step(s + 1, xb, xa);
+    }
+    if (s + 1 < s1) {
+      step(s, xa, xb);
+      st_wait_vm<0>();
+      multiply(s + 1, xb);
+    } else {
+      st_wait_vm<0>();
+      multiply(s, xa);
+    }
+  }
+
+  // lane: features 4 h .. 4 h + 3 of each 16, token col; the first wave adds the four up
+  float* part = reinterpret_cast<float*>(ring);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NT; ++i) *reinterpret_cast<f32x4*>(part + ((wv * NT + i) * 64 + lane) * 4) = acc[i];
+  __syncthreads();
+  if (wv) return;
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    f32x4 v = (f32x4)(0.f);
+#pragma unroll
+    for (int u = 0; u < NW; ++u) v += *reinterpret_cast<const f32x4*>(part + ((u * NT + i) * 64 + lane) * 4);
+    acc[i] = v;
+  }
+  if constexpr (EPI == 2) {
+    float up[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) up[r] = NT == 2 ? acc[NT - 1][r] : __shfl_xor(acc[0][r], 32, 64);
+    if (col >= P.M || (NT == 1 && h >= 2)) return;
+    u16x4 o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = f2bf(st_silu(acc[0][r]) * up[r]);
+    *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + (int64_t)col * P.ldo + 8 * NT * tile + 4 * h) = o;
+  } else {
+    if (col >= P.M) return;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int64_t at = (int64_t)col * P.ldo + 16 * (NT * tile + i) + 4 * h;
+      if constexpr (EPI == 1) {
+        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(P.out) + at) = acc[i];
+      } else {
+        u16x4 o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = f2bf(acc[i][r]);
+        *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + at) = o;
+      }
+    }
+  }
+}
+
+// tiles of 16 weight rows
+static int64_t st_tiles(int64_t N, bool swiglu) { return swiglu ? N / 8 : N / 16; }
+
+// Whether this kernel is the fastest of those here for a projection (N = F with SwiGLU). Up to K = 4,096 it is for 2 to 16 rows;
+// for one row from 512 tiles on gemv.hip is as fast or faster (32,768 x 768: 10.0 and 10.8 us). Longer rows of 16 tokens at once
+// keep the L2 busier than HBM: up to 256 tiles 8 rows still gain (above), beyond the others are level (8,192 x 8,192 at 4 rows:
+// table 25.6, here 27.8; 10,240 x 8,192: library 35.5, here 36.7).
+bool stream_gemm_covers(int64_t M, int64_t N, int64_t K, bool swiglu) {
+  if (M < 1 || M > 16 || K < 256 || K % 256 || N < 16 || N % 16 || N >= (int64_t(1) << 30)) return false;
+  const int64_t t = st_tiles(N, swiglu);
+  if (K > 4096) return t <= 256 && M <= 8;
+  return M > 1 || t <= 512;
+}
+
+// 32 rows a workgroup (half the token traffic) where 16 would give some CUs two workgroups and others one, or from 9 tokens on.
+// 4,096 x 4,096 at 8 rows: 16 rows 8.2 us, 32 rows 9.5; 6,144 x 4,096: 12.5, 10.9; SwiGLU 14,336 x 4,096: 40.6, 42.3, at 16
+// rows 49.6, 44.7
+void launch_stream_gemm(const StreamGemmParams& p, int epi, hipStream_t stream) {
+  const int t = (int)st_tiles(p.N, epi == 2);
+  if (p.M == 0 || t == 0) return;
+  const bool two = t > 256 && (t < 1024 || p.M > 8) && p.N % 32 == 0;
+#define NGA_ST(EPI)                                                                      \
+  if (two) stream_gemm_kernel<2, EPI><<<t / 2, 256, 0, stream>>>(p);                     \
+  else stream_gemm_kernel<1, EPI><<<t, 256, 0, stream>>>(p)
+  if (epi == 0) { NGA_ST(0); }
+  else if (epi == 1) { NGA_ST(1); }
+  else { NGA_ST(2); }
+#undef NGA_ST
+}
+
+}  // namespace nga

@@ -344,6 +344,17 @@ struct GemvParams {
 // out = x . W^T for M <= 4 rows (gemv.hip); false if the shape is out of range
 bool launch_gemv(const GemvParams& p, int epi, hipStream_t stream);
 
+struct StreamGemmParams {
+  const uint16_t* x;   // [M, K], row stride ldx; M <= 16
+  int64_t ldx;
+  const uint16_t* w;   // [N, K] (epi 2: [2N, K] = [gate | up]); K % 256 == 0, N % 16 == 0
+  int M, N, K;
+  void* out;           // epi 0 / 2: bf16 [M, ldo]; 1: fp32 [M, ldo]
+  int64_t ldo;
+};
+bool stream_gemm_covers(int64_t M, int64_t N, int64_t K, bool swiglu);
+void launch_stream_gemm(const StreamGemmParams& p, int epi, hipStream_t stream);
+
 struct SkinnyGemmParams {
   const uint16_t* x;   // [M, K] rows, stride ldx (16-B aligned)
   int64_t ldx;

@@ -194,6 +194,11 @@ class LlamaModel:
             a = ops.silu_mul(x) if swiglu else x
             w = L[name]
             M = a.shape[0]
+            if self.skinny and ops.stream_covers(a, w):
+                # up to 16 rows: one stream of the weights; its fp32 sums go to the norm or the rotation as one slab
+                if partial_ok and self.p.tp_size == 1:
+                    return ops.PartialSum(ops.stream_gemm(a, w, 1).unsqueeze(0))
+                return ops.stream_gemm(a, w, 0)
             if M == 1 and self.skinny and self._gemv_ok(a, w):
                 # one row (batch-1 decode): the weight-streaming GEMV (profiles/r4_gemv/)
                 return ops.gemv(a, w, 0)
@@ -516,6 +521,8 @@ class LlamaModel:
                                expert0=self.expert0, act=cfg.act, ws=self.moe_ws)
         if cfg.gated_mlp:
             if cfg.act == "silu":
+                if self.skinny and "wgu" in L and ops.stream_covers(x, L["wgu"], True):
+                    return self._lin(ops.stream_gemm(x, L["wgu"], 2), L, "wd", partial_ok=partial_ok)
                 if self.skinny and "wgu" in L and x.shape[0] <= ops.GEMV_MAX_M and self._gemv_ok(x, L["wgu"]):
                     # 1-4 rows: weight-streaming GEMV with the SwiGLU epilogue (5.0-5.8 TB/s)
                     return self._lin(ops.gemv(x, L["wgu"], 2), L, "wd", partial_ok=partial_ok)
@@ -850,7 +857,9 @@ class LlamaModel:
         ok = (self.skinny and h.is_cuda and h.dtype == torch.bfloat16 and self.lm_head.dtype == torch.bfloat16
               and h.stride(1) == 1 and h.stride(0) % 8 == 0)
         pk = self._pick(self.lm_head, h.shape[0]) if ok else None
-        if ok and h.shape[0] <= ops.GEMV_MAX_M and self.lm_head.is_contiguous():
+        if ok and ops.stream_covers(h, self.lm_head):
+            lg = ops.stream_gemm(h, self.lm_head, 1)
+        elif ok and h.shape[0] <= ops.GEMV_MAX_M and self.lm_head.is_contiguous():
             # 1-4 rows (batch-1..4 decode): the weight-streaming GEMV (6.4 TB/s vs 5.9 library)
             lg = ops.gemv(h, self.lm_head, 1)
         elif pk is not None and pk[1] == 1:

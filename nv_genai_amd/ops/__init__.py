@@ -228,6 +228,20 @@ def gemv(x: torch.Tensor, w: torch.Tensor, epi: int = 0, out: Optional[torch.Ten
     return out
 
 
+def stream_covers(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:
+    """Whether :func:`stream_gemm` is the kernel for x [M, K] @ w^T (bf16 on the GPU, w contiguous)."""
+    return (_gpu(x) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.is_contiguous() and x.stride(1) == 1
+            and x.stride(0) % 8 == 0 and kernels().stream_gemm_covers(x.shape[0], w.shape[0] // (2 if swiglu else 1), x.shape[1], swiglu))
+
+
+def stream_gemm(x: torch.Tensor, w: torch.Tensor, epi: int = 0) -> torch.Tensor:
+    """x @ w^T of up to 16 token rows as one stream of the weights (gemm_stream.hip); ``epi`` as of :func:`gemv`."""
+    N = w.shape[0] // 2 if epi == 2 else w.shape[0]
+    out = torch.empty(x.shape[0], N, dtype=torch.float32 if epi == 1 else x.dtype, device=x.device)
+    kernels().stream_gemm(out, x, w, int(epi))
+    return out
+
+
 def splitk_reduce(P: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """bf16 sum of the K-split partial slabs P [S, M, N]."""
     S, M, N = P.shape

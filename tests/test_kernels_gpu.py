@@ -972,3 +972,22 @@ def test_encoder_forward_marks_indices_outside_the_tables(gpu):
         i[1], p[1] = bad_ids, bad_pos
         x = ops.encoder_forward(i, p, None, cu, 3, m.word, m.pos, m.type, m.emb_ln, [], m.cfg.heads, m.cfg.eps, m.scale)
         assert x[1].isnan().all() and x[0].isfinite().all() and x[2].isfinite().all()
+
+
+# one stage for four waves, an odd count, a long row; tiles on either side of the change from 16 to 32 rows a workgroup
+@pytest.mark.parametrize("N,K", [(16, 256), (48, 1280), (4096, 512), (4112, 768), (6144, 256), (16416, 256), (64, 14336)])
+@pytest.mark.parametrize("M", [1, 7, 16])
+@pytest.mark.parametrize("epi", [0, 1, 2])
+def test_stream_gemm(gpu, N, K, M, epi):
+    g = torch.Generator(device="cuda").manual_seed(N + K + M)
+    x = torch.randn(M + 1, K + 8, device="cuda", generator=g).to(torch.bfloat16)[1:, :K]
+    w = (0.05 * torch.randn(N * (2 if epi == 2 else 1), K, device="cuda", generator=g)).to(torch.bfloat16)
+    y = x.double() @ w.double().t().contiguous()
+    if epi == 2:
+        y = torch.nn.functional.silu(y[:, :N]) * y[:, N:]
+    out = ops.stream_gemm(x, w, epi)
+    assert out.shape == (M, N) and out.dtype == (torch.float32 if epi == 1 else torch.bfloat16)
+    # fp32 sums of K products: sqrt(K) 2^-24; else the result's rounding to bf16, 2^-9
+    assert ((out.double() - y).norm() / y.norm()).item() < (1e-5 if epi == 1 else 4e-3)
+    assert not ops.stream_covers(torch.zeros(17, K, dtype=torch.bfloat16, device="cuda"), w, epi == 2)
+    assert not ops.stream_covers(x[:, : K - 8], w[:, : K - 8].contiguous(), epi == 2)
