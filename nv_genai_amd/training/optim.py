@@ -3,6 +3,7 @@ of csrc/kernels/adamw.hip) instead of a dozen passes of foreach operations. Stat
 ``torch.optim.AdamW``; tensors that the kernels do not take go through its step."""
 from __future__ import annotations
 
+import inspect
 from collections import defaultdict
 from typing import Optional
 
@@ -47,7 +48,8 @@ class AdamW(torch.optim.AdamW):
                     st = self.state.get(p)
                     if st and (g["fused"] or g["capturable"]) and st["step"].device != p.device:
                         st["step"] = st["step"].to(p.device)
-            super().step()
+            # without the hooks that torch wraps around the base's step: those around this one run already
+            inspect.unwrap(torch.optim.AdamW.step, stop=lambda f: not getattr(f, "hooked", False))(self)
             return loss
         C = ops.kernels()
         clip = None
