@@ -71,6 +71,9 @@ class AdamW(torch.optim.AdamW):
             for p in ps:
                 at[int(self.state[p]["step"].item())].append(p)
             for step, q in at.items():
-                C.adamw(q, [p.grad for p in q], [self.state[p]["exp_avg"] for p in q], [self.state[p]["exp_avg_sq"] for p in q], clip,
-                        float(g["lr"]), float(g["weight_decay"]), float(g["betas"][0]), float(g["betas"][1]), float(g["eps"]), step)
+                gr, m, v = [p.grad for p in q], [self.state[p]["exp_avg"] for p in q], [self.state[p]["exp_avg_sq"] for p in q]
+                C.adamw(q, gr, m, v, clip, float(g["lr"]), float(g["weight_decay"]), float(g["betas"][0]), float(g["betas"][1]),
+                        float(g["eps"]), step)
+                # the kernel writes through addresses: a graph that saved one of these must see that it changed
+                torch.autograd.graph.increment_version(q + m + v + (gr if max_norm else []))
         return loss

@@ -42,3 +42,20 @@ def test_adamw_matches_torch(gpu, max_norm):
     again = AdamW([{"params": a[:3], "weight_decay": 0.1}, {"params": a[3:], "weight_decay": 0.0}], **kw)
     again.load_state_dict(sa)
     again.step(max_norm=max_norm)
+
+
+@pytest.mark.parametrize("max_norm", [None, 1.0])
+def test_a_kept_graph_sees_the_step(gpu, max_norm):
+    """A backward through a graph that saved the weights raises after the step, as behind torch's."""
+    from nv_genai_amd.training.optim import AdamW
+
+    p = torch.nn.Parameter(torch.randn(64, device=gpu))
+    opt = AdamW([p], lr=0.1)
+    loss = p.pow(3).sum()
+    loss.backward(retain_graph=True)
+    seen = p.grad._version
+    assert opt._covers()
+    opt.step(max_norm=max_norm)
+    assert (p.grad._version > seen) == (max_norm is not None)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        loss.backward()
