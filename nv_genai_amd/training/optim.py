@@ -18,6 +18,8 @@ def _native(t: torch.Tensor) -> bool:
 
 class AdamW(torch.optim.AdamW):
     def _covers(self) -> bool:
+        if getattr(self, "grad_scale", None) is not None or getattr(self, "found_inf", None) is not None:
+            return False   # a GradScaler leaves scaling and skipping to torch's fused step
         dev = None
         for g in self.param_groups:
             if g["amsgrad"] or g["maximize"] or g["capturable"] or g["differentiable"] or isinstance(g["lr"], torch.Tensor):

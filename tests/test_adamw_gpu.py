@@ -59,3 +59,22 @@ def test_a_kept_graph_sees_the_step(gpu, max_norm):
     assert (p.grad._version > seen) == (max_norm is not None)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         loss.backward()
+
+
+@pytest.mark.parametrize("factor", [1.0, float("inf")])
+def test_grad_scaler_with_the_fused_form(gpu, factor):
+    """A GradScaler hands the scale and the found infinities to a fused optimiser's step."""
+    from nv_genai_amd.training.optim import AdamW
+
+    start, got = torch.randn(64, device=gpu), []
+    for cls in (AdamW, torch.optim.AdamW):
+        p = torch.nn.Parameter(start.clone())
+        opt, scaler = cls([p], lr=0.1, fused=True), torch.amp.GradScaler("cuda", init_scale=1024.0)
+        for _ in range(2):
+            opt.zero_grad()
+            scaler.scale((p * torch.linspace(0.0, 1.0, 64, device=gpu)).sum() * factor).backward()
+            scaler.step(opt)
+            scaler.update()
+        got.append((p.detach(), scaler.get_scale()))
+    assert torch.equal(got[0][0], got[1][0]) and got[0][1] == got[1][1]
+    assert torch.equal(got[0][0], start) == (factor > 1)
