@@ -132,7 +132,9 @@ def llama_hidden(model, ids: torch.Tensor, linear: Optional[LinearFn] = None,
         x = x * torch.tensor(cfg.embed_scale, dtype=dt)
 
     # rotation rows, and the sequences' starts for the attention whose gradients are the framework's own
-    rows = cs.reshape(B * S, D).float().contiguous() if fused.rope_usable(x, D) else None
+    rows = None
+    if pos.dim() == 2 and fused.rope_usable(x, D):   # one table for all sequences, or one a token
+        rows = cs.expand(len(cs) if cs.shape[1] == S else B, S, D).reshape(-1, D).float().contiguous()
     cu = torch.arange(0, B * S + 1, S, dtype=torch.int32, device=ids.device) if once and rows is not None else None
 
     def attend(qkv):

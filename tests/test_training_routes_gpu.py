@@ -1,0 +1,52 @@
+"""Calls that the fused training functions take or leave to the torch operations: every form that those accept gives their
+results."""
+import pytest
+import torch
+
+from nv_genai_amd.training import functional as Fn
+from nv_genai_amd.training import fused
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+def _rel(a, b):
+    return ((a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-30)).item()
+
+
+def _rows(*shape, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed + sum(shape))
+    return torch.randn(*shape, device="cuda", generator=g).to(BF)
+
+
+def _without(monkeypatch):
+    """The torch operations in place of the functions."""
+    for n in ("usable", "swiglu_usable", "rope_usable", "cross_entropy_usable"):
+        monkeypatch.setattr(fused, n, lambda *a, **k: False)
+
+
+def _llama(dev, name="llama-tiny"):
+    from nv_genai_amd.models.config import llama_config
+    from nv_genai_amd.models.llama import LlamaModel
+
+    return LlamaModel(llama_config(name), dev, seed=3)
+
+
+@pytest.mark.parametrize("shape", [(1, 40), (2, 1), (1, 1), (2, 40), (40,)])
+def test_positions_of_any_shape(gpu, monkeypatch, shape):
+    """Positions broadcast over the ids [2, 40]; a bare [40] raises, as it does without the functions."""
+    m = _llama(gpu)
+    ids = torch.randint(0, 1000, (2, 40), device=gpu)
+    pos = torch.randint(0, 60, shape, device=gpu)
+
+    def hidden():
+        with torch.no_grad(), torch.autocast("cuda", dtype=BF):
+            return Fn.llama_hidden(m, ids, pos=pos)
+
+    if len(shape) == 1:
+        with pytest.raises(RuntimeError):
+            hidden()
+        return
+    a = hidden()
+    _without(monkeypatch)
+    assert torch.equal(a, hidden())
