@@ -161,7 +161,11 @@ def llama_hidden(model, ids: torch.Tensor, linear: Optional[LinearFn] = None,
     def joined(x, d, li, name):
         """(x + d, its norm); d is what the last step leaves to be added."""
         w = W(li, name) if li >= 0 else P.get(name, getattr(model, name))
-        return (x, fused.rms_norm(x, w, cfg.eps, once)) if d is None else fused.add_rms_norm(x, d, w, cfg.eps, once)
+        if d is not None:
+            if fused.usable(x, w) and fused.usable(d) and d.shape == x.shape:
+                return fused.add_rms_norm(x, d, w, cfg.eps, once)
+            x = x + d   # a projection of another type; the rows from here on may have it too
+        return x, fused.rms_norm(x, w, cfg.eps, once) if fused.usable(x, w) else rms_norm(x, w, cfg.eps)
 
     def layer_joined(x, d, li):
         x, h = joined(x, d, li, "attn_norm")

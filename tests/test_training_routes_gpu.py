@@ -50,3 +50,20 @@ def test_positions_of_any_shape(gpu, monkeypatch, shape):
     a = hidden()
     _without(monkeypatch)
     assert torch.equal(a, hidden())
+
+
+@pytest.mark.parametrize("name", ["wo", "wd", "all"])
+def test_projections_of_another_type(gpu, monkeypatch, name):
+    """A caller's projections may return fp32 rows."""
+    m = _llama(gpu)
+    ids = torch.randint(0, 1000, (2, 40), device=gpu)
+
+    def linear(x, li, n):
+        w = m.layers[li][n]
+        return x.float() @ w.float().t() if name in (n, "all") else x.to(BF) @ w.t()
+
+    with torch.no_grad():
+        a = Fn.llama_hidden(m, ids, linear=linear)
+        _without(monkeypatch)
+        b = Fn.llama_hidden(m, ids, linear=linear)
+    assert a.dtype == b.dtype and torch.equal(a, b)
