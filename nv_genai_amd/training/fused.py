@@ -24,13 +24,20 @@ BF16 = torch.bfloat16
 def usable(x: torch.Tensor, *weights: Optional[torch.Tensor]) -> bool:
     """Whether these functions take bf16 rows x (last dimension 8 to 8,192, a multiple of 8) with fp32 or bf16 weights."""
     H = x.shape[-1] if x.dim() else 0
-    return (x.is_cuda and x.dtype is BF16 and H % 8 == 0 and 8 <= H <= 8192 and x.numel() > 0 and _plain(x)
+    return (_takes(x) and H % 8 == 0 and 8 <= H <= 8192
             and all(w is None or (w.is_cuda and w.is_contiguous() and w.dtype in (torch.float32, BF16) and _plain(w)) for w in weights))
 
 
 def _plain(t: torch.Tensor) -> bool:
-    return (type(t) in (torch.Tensor, torch.nn.Parameter) and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
-            and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0)
+    return type(t) in (torch.Tensor, torch.nn.Parameter)
+
+
+def _takes(x: torch.Tensor) -> bool:
+    """bf16 rows on the GPU, nothing active that these functions would pass by, and no autocast to another type: the torch
+    operations between them would change the rows' type."""
+    return (x.is_cuda and x.dtype is BF16 and x.numel() > 0 and _plain(x) and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+            and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+            and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") is BF16))
 
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
@@ -165,7 +172,7 @@ def swiglu(gu: torch.Tensor) -> torch.Tensor:
 
 
 def swiglu_usable(gu: torch.Tensor) -> bool:
-    return gu.is_cuda and gu.dtype is BF16 and gu.shape[-1] % 16 == 0 and gu.numel() > 0 and _plain(gu)
+    return _takes(gu) and gu.shape[-1] % 16 == 0
 
 
 class _Rope(Function):
@@ -187,7 +194,7 @@ def rope(qkv: torch.Tensor, cs: torch.Tensor, nr: int, nh: int, D: int) -> torch
 
 
 def rope_usable(x: torch.Tensor, D: int) -> bool:
-    return x.is_cuda and x.dtype is BF16 and D % 16 == 0 and x.numel() > 0 and _plain(x)
+    return _takes(x) and D % 16 == 0
 
 
 class _Attention(Function):
@@ -260,7 +267,7 @@ def cross_entropy_sum(logits: torch.Tensor, y: torch.Tensor, once: bool = False)
 
 
 def cross_entropy_usable(logits: torch.Tensor) -> bool:
-    return logits.is_cuda and logits.dtype is BF16 and logits.shape[-1] % 8 == 0 and logits.shape[0] > 0 and _plain(logits)
+    return _takes(logits) and logits.shape[-1] % 8 == 0
 
 
 class _LoraLinear(Function):

@@ -67,3 +67,37 @@ def test_projections_of_another_type(gpu, monkeypatch, name):
         _without(monkeypatch)
         b = Fn.llama_hidden(m, ids, linear=linear)
     assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("how", ["params", "lora", "encoder"])
+def test_autocast_to_half(gpu, monkeypatch, how):
+    from nv_genai_amd.models.config import encoder_config
+    from nv_genai_amd.models.encoder import EncoderModel
+    from nv_genai_amd.training.lora import LoRA, LoRAConfig
+
+    m = _llama(gpu) if how != "encoder" else EncoderModel(encoder_config("encoder-tiny"), gpu, seed=2)
+    ids = torch.randint(0, 1000, (2, 40), device=gpu)
+
+    def loss_and_grads():
+        if how == "lora":
+            ad = LoRA(m, LoRAConfig(r=8, alpha=16), seed=1)
+            for t in ad.B.values():
+                t.data.normal_(0, 0.02, generator=torch.Generator(device="cuda").manual_seed(4))
+            ps, kw = list(ad.parameters()), {"linear": ad.linear}
+        else:
+            P = Fn.trainable_params(m, "llama" if how == "params" else how)
+            ps, kw = [P[k] for k in sorted(P, key=str)], {"params": P}
+        with torch.autocast("cuda", dtype=torch.float16):
+            if how == "encoder":
+                loss = Fn.encoder_embed(m, ids, torch.ones_like(ids), **kw).pow(3).sum()
+            else:
+                loss = Fn.lm_loss(m, Fn.llama_hidden(m, ids, **kw), ids, params=kw.get("params"))
+        return loss.detach(), torch.autograd.grad(loss, ps, allow_unused=True)
+
+    la, ga = loss_and_grads()
+    _without(monkeypatch)
+    lb, gb = loss_and_grads()
+    assert torch.equal(la, lb)
+    for p, q in zip(ga, gb):   # the same operations; torch adds the embeddings' gradient in no fixed order
+        assert (p is None) == (q is None)
+        assert p is None or _rel(p, q) < 1e-3, (p.shape, _rel(p, q))
