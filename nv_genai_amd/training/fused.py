@@ -37,6 +37,7 @@ def _takes(x: torch.Tensor) -> bool:
     operations between them would change the rows' type."""
     return (x.is_cuda and x.dtype is BF16 and x.numel() > 0 and _plain(x) and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
             and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+            and not torch._C._len_torch_dispatch_stack()   # make_fx and other modes that watch the operations
             and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") is BF16))
 
 

@@ -101,3 +101,21 @@ def test_autocast_to_half(gpu, monkeypatch, how):
     for p, q in zip(ga, gb):   # the same operations; torch adds the embeddings' gradient in no fixed order
         assert (p is None) == (q is None)
         assert p is None or _rel(p, q) < 1e-3, (p.shape, _rel(p, q))
+
+
+def test_make_fx_records_the_operations(gpu):
+    """A graph recorded from real tensors computes from its inputs."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    m = _llama(gpu)
+    ids = torch.randint(0, 1000, (2, 40), device=gpu)
+
+    def loss(h, w):
+        with torch.autocast("cuda", dtype=BF):
+            x = Fn.llama_hidden(m, ids, params={"final_norm": w}) + h
+        return Fn.lm_loss(m, x, ids)
+
+    with torch.no_grad():
+        g = make_fx(loss)(_rows(2, 40, m.cfg.hidden), _rows(m.cfg.hidden))
+        h, w = _rows(2, 40, m.cfg.hidden, seed=9), _rows(m.cfg.hidden, seed=9)
+        assert abs(g(h, w) - loss(h, w)) < 1e-5 * abs(loss(h, w))
