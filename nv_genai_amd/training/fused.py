@@ -22,10 +22,12 @@ BF16 = torch.bfloat16
 
 
 def usable(x: torch.Tensor, *weights: Optional[torch.Tensor]) -> bool:
-    """Whether these functions take bf16 rows x (last dimension 8 to 8,192, a multiple of 8) with fp32 or bf16 weights."""
+    """Whether these functions take bf16 rows x (last dimension 8 to 8,192, a multiple of 8) with fp32 or bf16 weights, which
+    the kernels read 16 bytes at a time (rows at other addresses are copied, see _rows)."""
     H = x.shape[-1] if x.dim() else 0
     return (_takes(x) and H % 8 == 0 and 8 <= H <= 8192
-            and all(w is None or (w.is_cuda and w.is_contiguous() and w.dtype in (torch.float32, BF16) and _plain(w)) for w in weights))
+            and all(w is None or (w.is_cuda and w.is_contiguous() and w.dtype in (torch.float32, BF16) and _plain(w)
+                                  and w.data_ptr() % 16 == 0) for w in weights))
 
 
 def _plain(t: torch.Tensor) -> bool:

@@ -119,3 +119,17 @@ def test_make_fx_records_the_operations(gpu):
         g = make_fx(loss)(_rows(2, 40, m.cfg.hidden), _rows(m.cfg.hidden))
         h, w = _rows(2, 40, m.cfg.hidden, seed=9), _rows(m.cfg.hidden, seed=9)
         assert abs(g(h, w) - loss(h, w)) < 1e-5 * abs(loss(h, w))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, BF])
+def test_norm_weights_at_any_address(gpu, monkeypatch, dtype):
+    """Norms' weights may be views that do not begin at 16 bytes."""
+    m = _llama(gpu)
+    ids = torch.randint(0, 1000, (2, 40), device=gpu)
+    P = {k: v.detach().to(dtype) for k, v in Fn.trainable_params(m, "llama").items()}
+    for k in [k for k in P if P[k].ndim == 1]:
+        P[k] = torch.empty(P[k].numel() + 1, dtype=dtype, device=gpu)[1:].copy_(P[k])
+    with torch.no_grad(), torch.autocast("cuda", dtype=BF):
+        a = Fn.llama_hidden(m, ids, params=P)
+        _without(monkeypatch)
+        assert torch.equal(a, Fn.llama_hidden(m, ids, params=P))
