@@ -4,8 +4,9 @@ Each takes the place of a chain of single torch operations in :mod:`.functional`
 statistics, sums and the gradients of weights fp32, weights either fp32 masters or bf16. Activations are bit for bit those of
 the chain. So are, all weights trained, their gradients; ``attention``, ``lora_linear`` and the ``once`` forms, for adapters,
 form them in the kernels' own order. Callers ask ``usable`` first; the torch operations stay for the CPU, other types and
-sizes, and under transforms that pass functions of this kind by (tracing, functorch, forward-mode). Like the flash attention
-that they stand beside they have a first derivative only.
+sizes, and under transforms that pass functions of this kind by (tracing, functorch, forward-mode). Where a graph of the
+backward is asked for (create_graph) the gradients come from torch operations; ``attention``, like the flash attention that it
+stands for, has a first derivative only.
 """
 from __future__ import annotations
 
@@ -49,29 +50,35 @@ def _rows(t: torch.Tensor) -> torch.Tensor:
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
+def _again(chain, inputs, dy):
+    """The inputs' gradients (None where they need none) through torch operations, from tensors that carry the graph of the
+    forward: to be differentiated in turn."""
+    ins = [t.view_as(t) for t in inputs]
+    got = iter(torch.autograd.grad(chain(*ins), [t for t in ins if t.requires_grad], dy, create_graph=True))
+    return [next(got) if t.requires_grad else None for t in ins]
+
+
 class _Linear(Function):
     @staticmethod
     def forward(ctx, x, w, b):
-        x2, wb = x.reshape(-1, x.shape[-1]), w.to(BF16)
-        ctx.save_for_backward(x2, wb)
-        ctx.how = (x.shape, w.dtype, b.dtype)
-        return torch.addmm(b.to(BF16), x2, wb.t()).view(*x.shape[:-1], w.shape[0])
+        ctx.save_for_backward(x, w, b)
+        return torch.addmm(b, x.reshape(-1, x.shape[-1]), w.t()).view(*x.shape[:-1], w.shape[0])
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, dy):
-        x2, wb = ctx.saved_tensors
-        shape, wd, bd = ctx.how
+        x, w, b = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return tuple(_again(torch.nn.functional.linear, (x, w, b), dy))
         dy2 = _rows(dy.reshape(-1, dy.shape[-1]))
-        dx = (dy2 @ wb).view(shape) if ctx.needs_input_grad[0] else None
-        dw = (dy2.t() @ x2).to(wd) if ctx.needs_input_grad[1] else None
-        db = ops.kernels().col_sums(dy2).to(BF16).to(bd) if ctx.needs_input_grad[2] else None   # a bf16 bias's gradient
+        dx = (dy2 @ w).view(x.shape) if ctx.needs_input_grad[0] else None
+        dw = dy2.t() @ x.reshape(-1, x.shape[-1]) if ctx.needs_input_grad[1] else None
+        db = ops.kernels().col_sums(dy2).to(BF16) if ctx.needs_input_grad[2] else None
         return dx, dw, db
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """x w^T + b in bf16, w's and b's gradients in their own type (w.shape[0] % 8 == 0)."""
-    return _Linear.apply(x, w, b)
+    return _Linear.apply(x, w.to(BF16), b.to(BF16))
 
 
 class _AddRmsNorm(Function):
@@ -81,20 +88,28 @@ class _AddRmsNorm(Function):
         C = ops.kernels()
         xn, sq = C.rms_sq(_rows(x), None if o is None else _rows(o))
         y, rstd = C.rms_apply(xn, sq.mean(-1), w, eps)
-        ctx.save_for_backward(xn, rstd, w)
-        ctx.once = once
+        ctx.save_for_backward(x if o is None else xn, rstd, w)
+        ctx.how = (eps, once)
         return (xn, y) if o is not None else y
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, *grads):
         xn, rstd, w = ctx.saved_tensors
         C, both, dy, want = ops.kernels(), len(grads) == 2, grads[-1], ctx.needs_input_grad[2]
+        eps, once = ctx.how
         dxn = grads[0] if both else None
         if dy is None:
             return dxn, dxn, None, None, None
-        dy, dxn = _rows(dy), None if dxn is None else _rows(dxn)
-        if ctx.once:
+        if torch.is_grad_enabled():
+            def chain(x, w):
+                x = x.float()
+                return (x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + eps) * w.float()).to(BF16)
+
+            dx, dw = _again(chain, (xn, w), dy)
+            dx = dx if dxn is None else dx + dxn
+            return dx, dx if both else None, dw, None, None
+        xn, dy, dxn = _rows(xn), _rows(dy), None if dxn is None else _rows(dxn)
+        if once:
             dx, dw = C.rms_bwd(xn, rstd, w, dy, dxn, want)
         else:
             prod, dw = C.rms_prod(dy, xn, w, rstd, want)
@@ -114,41 +129,48 @@ def add_rms_norm(x: torch.Tensor, o: torch.Tensor, w: torch.Tensor, eps: float, 
 class _ResidualLayerNorm(Function):
     @staticmethod
     def forward(ctx, x, o, g, b, eps):
-        s, gf, bf = ops.kernels().add_f32(_rows(x), _rows(o)), g.float(), b.float()
-        y, mean, rstd = torch.native_layer_norm(s, s.shape[-1:], gf, bf, eps)
-        ctx.save_for_backward(s, mean, rstd, gf, bf)
-        ctx.kinds = (g.dtype, b.dtype)
-        return y.to(BF16)
+        ctx.set_materialize_grads(False)
+        s = ops.kernels().add_f32(_rows(x), _rows(o))
+        y, mean, rstd = torch.native_layer_norm(s, s.shape[-1:], g, b, eps)
+        ctx.save_for_backward(s, mean, rstd, g, b)
+        ctx.eps = eps
+        return y.to(BF16), s   # an output carries the graph to x and o, for a derivative of the backward
 
     @staticmethod
-    @once_differentiable
-    def backward(ctx, dy):
-        s, mean, rstd, gf, bf = ctx.saved_tensors
-        dy = _rows(dy)
-        ds = torch.ops.aten.native_layer_norm_backward(dy.float(), s, s.shape[-1:], mean, rstd, gf, bf, [True, False, False])[0].to(BF16)
+    def backward(ctx, dy, more):
+        s, mean, rstd, g, b = ctx.saved_tensors
         dg = db = None
-        if ctx.needs_input_grad[2] or ctx.needs_input_grad[3]:
-            dg, db = ops.kernels().ln_sums(s, mean, rstd, dy).unbind(0)
-            dg, db = dg.to(ctx.kinds[0]), db.to(ctx.kinds[1])
+        if dy is None:
+            ds = more
+        elif torch.is_grad_enabled():
+            ds, dg, db = _again(lambda s, g, b: torch.nn.functional.layer_norm(s, s.shape[-1:], g, b, ctx.eps).to(BF16), (s, g, b), dy)
+            ds = ds if more is None else ds + more
+        else:
+            dy = _rows(dy)
+            ds = torch.ops.aten.native_layer_norm_backward(dy.float(), s, s.shape[-1:], mean, rstd, g, b, [True, False, False])[0]
+            ds = ds if more is None else ds + more
+            if ctx.needs_input_grad[2] or ctx.needs_input_grad[3]:
+                dg, db = ops.kernels().ln_sums(s, mean, rstd, dy).unbind(0)
+        ds = None if ds is None else ds.to(BF16)
         return ds, ds, dg, db, None
 
 
 def residual_layer_norm(x, o, g, b, eps: float) -> torch.Tensor:
     """LN(x + o) g + b, the sum in fp32."""
-    return _ResidualLayerNorm.apply(x, o, g, b, eps)
+    return _ResidualLayerNorm.apply(x, o, g.float(), b.float(), eps)[0]
 
 
 class _Gelu(Function):
     @staticmethod
     def forward(ctx, z):
-        zr = _rows(z)
-        ctx.save_for_backward(zr)
-        return ops.kernels().gelu_rows(zr, None)
+        ctx.save_for_backward(z)
+        return ops.kernels().gelu_rows(_rows(z), None)
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, dh):
-        return ops.kernels().gelu_rows(ctx.saved_tensors[0], _rows(dh))
+        if torch.is_grad_enabled():
+            return _again(lambda z: torch.nn.functional.gelu(z.float()).to(BF16), ctx.saved_tensors, dh)[0]
+        return ops.kernels().gelu_rows(_rows(ctx.saved_tensors[0]), _rows(dh))
 
 
 def gelu(z: torch.Tensor) -> torch.Tensor:
@@ -159,14 +181,14 @@ def gelu(z: torch.Tensor) -> torch.Tensor:
 class _SwiGlu(Function):
     @staticmethod
     def forward(ctx, gu):
-        g = _rows(gu)
-        ctx.save_for_backward(g)
-        return ops.kernels().swiglu_rows(g, None)
+        ctx.save_for_backward(gu)
+        return ops.kernels().swiglu_rows(_rows(gu), None)
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, dh):
-        return ops.kernels().swiglu_rows(ctx.saved_tensors[0], _rows(dh))
+        if torch.is_grad_enabled():
+            return _again(lambda t: torch.nn.functional.silu(t.chunk(2, -1)[0]) * t.chunk(2, -1)[1], ctx.saved_tensors, dh)[0]
+        return ops.kernels().swiglu_rows(_rows(ctx.saved_tensors[0]), _rows(dh))
 
 
 def swiglu(gu: torch.Tensor) -> torch.Tensor:
@@ -180,20 +202,19 @@ def swiglu_usable(gu: torch.Tensor) -> bool:
 
 class _Rope(Function):
     @staticmethod
-    def forward(ctx, qkv, cs, nr, nh, D):
+    def forward(ctx, qkv, cs, nr, nh, D, back):
         ctx.save_for_backward(cs)
-        ctx.how = (nr, nh, D)
-        return ops.kernels().rope_rows(_rows(qkv.reshape(-1, nh * D)), cs, nr, nh, D, False, False).view(qkv.shape)
+        ctx.how = (nr, nh, D, not back)
+        return ops.kernels().rope_rows(_rows(qkv.reshape(-1, nh * D)), cs, nr, nh, D, back, False).view(qkv.shape)
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, d):
-        return ops.kernels().rope_rows(_rows(d.reshape(-1, d.shape[-1])), ctx.saved_tensors[0], *ctx.how, True, False).view(d.shape), None, None, None, None
+        return (_Rope.apply(d, ctx.saved_tensors[0], *ctx.how),) + (None,) * 5
 
 
 def rope(qkv: torch.Tensor, cs: torch.Tensor, nr: int, nh: int, D: int) -> torch.Tensor:
     """Rows of nh heads, the first nr rotated (halves) by the [cos | sin] rows cs [P, D], row t by t % P."""
-    return _Rope.apply(qkv, cs, nr, nh, D)
+    return _Rope.apply(qkv, cs, nr, nh, D, False)
 
 
 def rope_usable(x: torch.Tensor, D: int) -> bool:
@@ -246,27 +267,34 @@ def attention_usable(qkv: torch.Tensor, D: int, hq: int, hkv: int, scale: float)
 class _CrossEntropySum(Function):
     @staticmethod
     def forward(ctx, logits, y, once):
-        lg = _rows(logits)
+        ctx.set_materialize_grads(False)
         ctx.once = once
         if once:
-            loss, lse = ops.kernels().ce_fwd(lg, y)
-            ctx.save_for_backward(lg, y, lse)
-            return loss.sum()
-        lp = torch.log_softmax(lg.float(), -1)
+            loss, lse = ops.kernels().ce_fwd(_rows(logits), y)
+            ctx.save_for_backward(logits, y, lse)
+            return loss.sum(), None
+        lp = torch.log_softmax(_rows(logits).float(), -1)
         ctx.save_for_backward(lp, y, None)
-        return torch.nn.functional.nll_loss(lp, y, reduction="sum")
+        return torch.nn.functional.nll_loss(lp, y, reduction="sum"), lp   # an output carries the graph to the logits
 
     @staticmethod
-    @once_differentiable
-    def backward(ctx, g):
+    def backward(ctx, g, more):
         t, y, lse = ctx.saved_tensors
-        return ops.kernels().ce_bwd(t, y, lse, g.float().reshape(1).contiguous()), None, None
+        if g is not None and more is None and not torch.is_grad_enabled():
+            return ops.kernels().ce_bwd(_rows(t) if ctx.once else t, y, lse, g.float().reshape(1).contiguous()), None, None
+        p, d = torch.softmax(t.float(), -1) if ctx.once else t.exp(), None
+        if g is not None:
+            d = g * (p - torch.nn.functional.one_hot(y, t.shape[-1]))
+        if more is not None:
+            more = more - p * more.sum(-1, keepdim=True)
+            d = more if d is None else d + more
+        return None if d is None else d.to(BF16), None, None
 
 
 def cross_entropy_sum(logits: torch.Tensor, y: torch.Tensor, once: bool = False) -> torch.Tensor:
     """Sum over the rows of the cross entropy of bf16 logits [n, V] (V % 8 == 0) with labels y in [0, V); fp32. once: one pass
     over the logits, kept in bf16, for the probabilities' fp32 logarithms of the other form."""
-    return _CrossEntropySum.apply(logits, y, once)
+    return _CrossEntropySum.apply(logits, y, once)[0]
 
 
 def cross_entropy_usable(logits: torch.Tensor) -> bool:
@@ -275,30 +303,31 @@ def cross_entropy_usable(logits: torch.Tensor) -> bool:
 
 class _LoraLinear(Function):
     @staticmethod
-    def forward(ctx, x, w, a, b, scale):
+    def forward(ctx, x, w, a, b, ab, bb, scale):
         x2 = x.reshape(-1, x.shape[-1])
-        ab, bb = a.to(BF16), b.to(BF16)
         h = x2 @ ab.t()
         y = x2 @ w.t()
         ops.kernels().add_scaled(y, h @ bb.t(), scale)
-        ctx.save_for_backward(x2, w, ab, bb, h)
-        ctx.how = (x.shape, scale, a.dtype, b.dtype)
+        ctx.save_for_backward(x, w, ab, bb, h)
+        ctx.how = (scale, a.dtype, b.dtype)
         return y.view(*x.shape[:-1], w.shape[0])
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, dy):
-        x2, w, ab, bb, h = ctx.saved_tensors
-        shape, scale, ad, bd = ctx.how
+        x, w, ab, bb, h = ctx.saved_tensors
+        scale, ad, bd = ctx.how
+        if torch.is_grad_enabled():   # the adapter's gradients through its bf16 copies
+            dx, da, db = _again(lambda x, a, b: x @ w.t() + ((x @ a.t()) @ b.t()) * scale, (x, ab, bb), dy)
+            return dx, None, None, None, da, db, None
         dy2 = dy.reshape(-1, dy.shape[-1])
         dh = (dy2 @ bb).mul_(scale)
-        dx = torch.addmm(dy2 @ w, dh, ab).view(shape) if ctx.needs_input_grad[0] else None
-        da = (dh.t() @ x2).to(ad) if ctx.needs_input_grad[2] else None
-        db = (dy2.t() @ h).to(bd).mul_(scale) if ctx.needs_input_grad[3] else None
-        return dx, None, da, db, None
+        dx = torch.addmm(dy2 @ w, dh, ab).view(x.shape) if ctx.needs_input_grad[0] else None
+        da = (dh.t() @ x.reshape(-1, x.shape[-1])).to(ad) if ctx.needs_input_grad[2] else None
+        db = (dy2.t() @ h).to(bd).mul_(scale) if ctx.needs_input_grad[3] else None   # scaled in its own type
+        return dx, None, da, db, None, None, None
 
 
 def lora_linear(x: torch.Tensor, w: torch.Tensor, a: torch.Tensor, b: torch.Tensor, scale: float) -> torch.Tensor:
     """x w^T + scale (x a^T) b^T with a frozen bf16 w (w.shape[0] % 8 == 0); the adapter's part of x's gradient joins in the
     accumulator of its second product."""
-    return _LoraLinear.apply(x, w, a, b, scale)
+    return _LoraLinear.apply(x, w, a, b, a.to(BF16), b.to(BF16), scale)

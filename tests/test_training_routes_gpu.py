@@ -133,3 +133,58 @@ def test_norm_weights_at_any_address(gpu, monkeypatch, dtype):
         a = Fn.llama_hidden(m, ids, params=P)
         _without(monkeypatch)
         assert torch.equal(a, Fn.llama_hidden(m, ids, params=P))
+
+
+def _twice(monkeypatch, f, xs, tol):
+    """Gradients of f and of a function of those, with the fused functions and without."""
+    got = []
+    for fused_too in (True, False):
+        if not fused_too:
+            _without(monkeypatch)
+        a = [x.detach().clone().requires_grad_() for x in xs]
+        g = torch.autograd.grad(f(*a), a, create_graph=True)
+        s = sum((t.float() * torch.linspace(-1, 1, t.numel(), device="cuda").view(t.shape)).sum() for t in g)
+        got.append(g + torch.autograd.grad(s, a, allow_unused=True))
+    for i, (p, q) in enumerate(zip(*got)):
+        assert (p is None) == (q is None), i
+        assert p is None or (p.dtype == q.dtype and _rel(p, q) < tol), (i, p.shape, _rel(p, q))
+
+
+@pytest.mark.parametrize("kind", ["llama", "encoder", "lora", "loss", "loss of adapters"])
+def test_second_derivatives(gpu, monkeypatch, kind):
+    """Under create_graph the gradients can be differentiated again (attention through torch's plain form, its fast ones cannot).
+    Both sides compute in bf16, and the second pass carries the rounding of the first: a few times 1e-2 at most."""
+    from torch.nn.attention import SDPBackend, sdpa_kernel
+
+    from nv_genai_amd.models.config import encoder_config
+    from nv_genai_amd.models.encoder import EncoderModel
+    from nv_genai_amd.training.lora import LoRA, LoRAConfig
+
+    m = EncoderModel(encoder_config("encoder-tiny"), gpu, seed=2) if kind == "encoder" else _llama(gpu)
+    ids = torch.randint(0, 1000, (2, 24), device=gpu)
+    if kind.startswith("loss"):
+        P = {"lm_head": m.lm_head.float()} if kind == "loss" else None
+        _twice(monkeypatch, lambda h: Fn.lm_loss(m, h, ids, params=P), [_rows(2, 24, m.cfg.hidden)], 1e-2)
+        return
+    if kind == "lora":
+        ad = LoRA(m, LoRAConfig(r=8, alpha=24, targets=("qkv", "o")), seed=1)
+        for t in ad.B.values():
+            t.data.normal_(0, 0.02, generator=torch.Generator(device="cuda").manual_seed(4))
+        ks, xs = [(d, k) for d in ("A", "B") for k in sorted(ad.A)], [*(ad.A[k] for k in sorted(ad.A)), *(ad.B[k] for k in sorted(ad.A))]
+    else:
+        P = Fn.trainable_params(m, kind)
+        ks = sorted(P, key=str)
+        xs = [P[k] for k in ks]
+
+    def f(*ps):
+        with torch.autocast("cuda", dtype=BF), sdpa_kernel(SDPBackend.MATH):
+            if kind == "lora":
+                for (d, k), p in zip(ks, ps):
+                    getattr(ad, d)[k] = p
+                return Fn.lm_loss(m, Fn.llama_hidden(m, ids, linear=ad.linear), ids)
+            Q = dict(zip(ks, ps))
+            if kind == "llama":
+                return Fn.lm_loss(m, Fn.llama_hidden(m, ids, params=Q), ids, params=Q)
+            return Fn.encoder_embed(m, ids, torch.ones_like(ids), Q).pow(3).sum()
+
+    _twice(monkeypatch, f, xs, 5e-2)
