@@ -1091,6 +1091,28 @@ int encoder_split(int64_t M, int64_t K) {
   return M <= 512 ? (int)std::min<int64_t>(4, K / 64) : K > 1024 ? 4 : 2;
 }
 
+// nullptr, or why encoder_forward does not take these weights; tables: positions, types, the embedding norm's weight and bias
+const char* encoder_refuses(const Tensor& word, const std::vector<Tensor>& tables, const std::vector<Tensor>& L, int64_t heads) {
+  if (word.dim() != 2 || heads <= 0) return "encoder: word table [words, hidden]";
+  const int64_t H = word.size(1), D = H / heads, F = L.size() > 6 && L[6].dim() == 2 ? L[6].size(0) : H;
+  if (H % 64 != 0 || H > 8192 || heads * D != H || !(D == 32 || D == 64 || D == 128)) return "encoder: head size 32, 64 or 128";
+  if (F % 64 != 0) return "encoder: feed-forward size must be a multiple of 64";
+  if (L.size() % 12 != 0) return "encoder: 12 tensors a layer";
+  auto takes = [&](const Tensor& t) {
+    return t.is_cuda() && t.device() == word.device() && t.scalar_type() == at::kBFloat16 && t.is_contiguous() &&
+           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  bool ok = takes(word);
+  for (size_t i = 0; ok && i < tables.size(); ++i)
+    ok = takes(tables[i]) && (i < 2 ? tables[i].dim() == 2 && tables[i].size(1) == H : tables[i].sizes() == at::IntArrayRef{H});
+  const int64_t rows[12] = {3 * H, 3 * H, H, H, H, H, F, F, H, H, H, H}, cols[12] = {H, 0, H, 0, 0, 0, H, 0, F, 0, 0, 0};
+  for (size_t i = 0; ok && i < L.size(); ++i) {
+    const int j = (int)(i % 12);
+    ok = takes(L[i]) && L[i].dim() == (cols[j] ? 2 : 1) && L[i].size(0) == rows[j] && (!cols[j] || L[i].size(1) == cols[j]);
+  }
+  return ok ? nullptr : "encoder: weights must be contiguous bf16 of their shapes, at 16-byte addresses on one GPU";
+}
+
 // Post-norm encoder stack (BERT): embedding sum + norm, then per layer q/k/v, packed attention, output + norm, up + GELU,
 // down + norm. Layer tensors: wqkv, bqkv, wo, bo, ln1_g, ln1_b, wi, bi, wo2, bo2, ln2_g, ln2_b. All launches go out from
 // here: from Python the 200 of a BERT-large forward took longer than they ran (2.3 ms for one query).
@@ -1101,19 +1123,13 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
   CHECK_DEV(ids); CHECK_DT(ids, at::kInt); CHECK_CONTIG(ids);
   CHECK_DEV(pos); CHECK_DT(pos, at::kInt); CHECK_CONTIG(pos);
   CHECK_DEV(cu); CHECK_DT(cu, at::kInt); CHECK_CONTIG(cu);
-  const int64_t T = ids.numel(), H = word.size(1), D = heads > 0 ? H / heads : 0;
+  const int64_t T = ids.numel(), H = word.size(-1), D = heads > 0 ? H / heads : 0;
   TORCH_CHECK(pos.numel() == T && (!types.has_value() || types->numel() == T), "encoder: one position and type per token");
   if (types.has_value()) { CHECK_DEV(*types); CHECK_DT(*types, at::kInt); CHECK_CONTIG(*types); }
-  auto weight = [&](const Tensor& t, at::IntArrayRef sizes) {
-    CHECK_BF16(t); CHECK_CONTIG(t);
-    TORCH_CHECK(t.sizes() == sizes && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, "encoder: weight of another shape");
-  };
-  weight(word, {word.size(0), H}); weight(ptab, {ptab.size(0), H}); weight(ttab, {ttab.size(0), H});
-  weight(emb_g, {H}); weight(emb_b, {H});
-  TORCH_CHECK(H % 64 == 0 && H <= 8192 && heads * D == H && (D == 32 || D == 64 || D == 128), "encoder: head size 32, 64 or 128");
-  TORCH_CHECK(L.size() % 12 == 0 && T < (int64_t(1) << 31) && cu.numel() >= 1 && max_len >= 0, "encoder: layers / tokens");
+  const char* why = encoder_refuses(word, {ptab, ttab, emb_g, emb_b}, L, heads);
+  TORCH_CHECK(why == nullptr, why);
+  TORCH_CHECK(ids.device() == word.device() && T < (int64_t(1) << 31) && cu.numel() >= 1 && max_len >= 0, "encoder: tokens");
   const int64_t F = L.empty() ? H : L[6].size(0);
-  TORCH_CHECK(F % 64 == 0, "encoder: feed-forward size must be a multiple of 64");
   const int64_t B = cu.numel() - 1;
   const hipStream_t st = cur_stream(ids);
   const auto opt = word.options();
@@ -1174,9 +1190,6 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
   p.Hq = p.Hkv = (int)heads;
   p.scale = (float)scale;
   for (size_t i = 0; i < L.size(); i += 12) {
-    weight(L[i], {3 * H, H}); weight(L[i + 1], {3 * H}); weight(L[i + 2], {H, H}); weight(L[i + 3], {H});
-    weight(L[i + 4], {H}); weight(L[i + 5], {H}); weight(L[i + 6], {F, H}); weight(L[i + 7], {F});
-    weight(L[i + 8], {H, F}); weight(L[i + 9], {H}); weight(L[i + 10], {H}); weight(L[i + 11], {H});
     project(x, L[i], L[i + 1], qkv, false);
     if (B > 0 && max_len > 0) nga::launch_varlen_attention(p, (int)B, (int)max_len, (int)D, false, st);
     project_norm(a, L[i + 2], L[i + 3], x, L[i + 4], L[i + 5], x);
@@ -2693,6 +2706,9 @@ PYBIND11_MODULE(_C, m) {
   m.def("score", checked("score", &score));
   m.def("topk", checked("topk", &topk));
   m.def("encoder_forward", &encoder_forward);
+  m.def("encoder_covers", [](const Tensor& word, const std::vector<Tensor>& tables, const std::vector<Tensor>& L, int64_t heads) {
+    return encoder_refuses(word, tables, L, heads) == nullptr;
+  });
   m.def("rms_sq", &rms_sq);
   m.def("rms_apply", &rms_apply);
   m.def("rms_prod", &rms_prod);

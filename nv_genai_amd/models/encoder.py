@@ -134,7 +134,8 @@ class EncoderModel:
         for a reranker (num_labels > 0) returns [B, num_labels] fp32 logits."""
         cfg = self.cfg
         H, nh, hd = cfg.hidden, cfg.heads, cfg.head_dim
-        if ids.is_cuda and ops.encoder_covers(self.word, self.layers, nh):
+        if (ids.is_cuda and ids.dim() == 1 and pos.shape == ids.shape and (type_ids is None or type_ids.shape == ids.shape)
+                and ops.encoder_covers(self.word, self.layers, nh, (self.pos, self.type, *self.emb_ln))):
             x = ops.encoder_forward(ids, pos, type_ids, cu, max_len, self.word, self.pos, self.type, self.emb_ln, self.layers,
                                     nh, cfg.eps, self.scale)
             return self._pool(x, cu)

@@ -1287,15 +1287,15 @@ def varlen_attention(q, k, v, cu, Hq, Hkv, D, max_len, scale, causal=False, out=
 ENCODER_LAYER = ("wqkv", "bqkv", "wo", "bo", "ln1_g", "ln1_b", "wi", "bi", "wo2", "bo2", "ln2_g", "ln2_b")
 
 
-def encoder_covers(word: torch.Tensor, layers, heads: int) -> bool:
-    """Whether ``encoder_forward`` takes these weights: contiguous bf16 ones on the GPU, hidden and feed-forward sizes
-    multiples of 64 (the projections' K steps), head size 32, 64 or 128."""
-    H = word.shape[1]
-    if not _gpu(word) or word.dtype != torch.bfloat16 or heads <= 0 or H % 64 or H // heads not in (32, 64, 128) or H % heads or H > 8192:
-        return False
-    F = layers[0]["wi"].shape[0] if layers else 64
-    return F % 64 == 0 and all(L["wi"].shape[0] == F and all(L[n].dtype == torch.bfloat16 and L[n].is_contiguous() for n in ENCODER_LAYER)
-                               for L in layers)
+def _encoder_weights(layers):
+    return [L[n] for L in layers for n in ENCODER_LAYER]
+
+
+def encoder_covers(word: torch.Tensor, layers, heads: int, tables=()) -> bool:
+    """Whether ``encoder_forward`` takes these weights: contiguous bf16 ones of their shapes at 16-byte addresses of one GPU,
+    hidden and feed-forward sizes multiples of 64 (the projections' K steps), head size 32, 64 or 128. ``tables``: positions,
+    types, the embedding norm's weight and bias."""
+    return _gpu(word) and kernels().encoder_covers(word, list(tables), _encoder_weights(layers), int(heads))
 
 
 def encoder_forward(ids, pos, types, cu, max_len: int, word, ptab, ttab, emb_ln, layers, heads: int, eps: float,
@@ -1306,7 +1306,7 @@ def encoder_forward(ids, pos, types, cu, max_len: int, word, ptab, ttab, emb_ln,
     def i32(t):
         return None if t is None else t.to(torch.int32).contiguous()
     return kernels().encoder_forward(i32(ids), i32(pos), i32(types), i32(cu), int(max_len), word, ptab, ttab, emb_ln[0], emb_ln[1],
-                                     [L[n] for L in layers for n in ENCODER_LAYER], int(heads), float(eps), float(scale))
+                                     _encoder_weights(layers), int(heads), float(eps), float(scale))
 
 
 # ------------------------------------------------------------------------- MoE

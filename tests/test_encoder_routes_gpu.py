@@ -1,0 +1,67 @@
+"""Encoder forwards that the native call takes or leaves to the steps in Python."""
+import pytest
+import torch
+
+from nv_genai_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(dev):
+    from nv_genai_amd.models.config import encoder_config
+    from nv_genai_amd.models.encoder import EncoderModel
+
+    return EncoderModel(encoder_config("encoder-tiny"), dev, seed=2)
+
+
+def _tokens(dev, n):
+    """n tokens in sequences of up to 60."""
+    g = torch.Generator().manual_seed(n)
+    ids = torch.randint(0, 1000, (n,), generator=g, dtype=torch.int32)
+    cu = torch.tensor([*range(0, n, 60), n], dtype=torch.int32)
+    return ids.to(dev), (torch.arange(n) % 60).int().to(dev), cu.to(dev), 60
+
+
+def _close(a, b):
+    """Two forms that round to bf16 at different places, some 2^-9 of a value each, through a few layers."""
+    assert a.shape == b.shape and ((a - b).norm() / b.norm()).item() < 2e-2
+
+
+def _odd(t):
+    return torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape).copy_(t)
+
+
+def _apart(t):
+    return torch.stack([t, t], -1)[..., 0]
+
+
+@pytest.mark.parametrize("n", [30, 1200])
+@pytest.mark.parametrize("what,how", [(w, _odd) for w in ("word", "pos", "type", "emb_ln", "wqkv", "bqkv", "bi", "ln1_g", "wo2")]
+                         + [(w, _apart) for w in ("word", "pos", "type", "wqkv")])
+def test_weights_of_any_layout(gpu, n, what, how):
+    """Views that do not begin at 16 bytes, and tables and projections whose elements lie apart."""
+    m, t = _model(gpu), _tokens(gpu, n)
+    want = m.forward(*t)
+    if what in m.layers[0]:
+        m.layers[0][what] = how(m.layers[0][what])
+    else:
+        setattr(m, what, tuple(how(w) for w in m.emb_ln) if what == "emb_ln" else how(getattr(m, what)))
+    assert not ops.encoder_covers(m.word, m.layers, m.cfg.heads, (m.pos, m.type, *m.emb_ln))
+    _close(m.forward(*t), want)
+
+
+@pytest.mark.parametrize("name,size", [("wi", (192, 64)), ("bi", (64,))])
+def test_weights_of_other_shapes_are_not_covered(gpu, name, size):
+    m = _model(gpu)
+    tables = (m.pos, m.type, *m.emb_ln)
+    assert ops.encoder_covers(m.word, m.layers, m.cfg.heads, tables)
+    m.layers[1][name] = torch.zeros(size, dtype=torch.bfloat16, device=gpu)
+    assert not ops.encoder_covers(m.word, m.layers, m.cfg.heads, tables)
+    with pytest.raises(RuntimeError):
+        m.forward(*_tokens(gpu, 30))
+
+
+def test_one_type_for_all_tokens(gpu):
+    m, t = _model(gpu), _tokens(gpu, 30)
+    one = torch.ones(1, device=gpu, dtype=torch.int32)
+    _close(m.forward(*t, one), m.forward(*t, one.expand(30).contiguous()))
