@@ -229,9 +229,10 @@ def gemv(x: torch.Tensor, w: torch.Tensor, epi: int = 0, out: Optional[torch.Ten
 
 
 def stream_covers(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:
-    """Whether :func:`stream_gemm` is the kernel for x [M, K] @ w^T (bf16 on the GPU, w contiguous)."""
+    """Whether :func:`stream_gemm` is the kernel for x [M, K] @ w^T (bf16 on the GPU, w contiguous, rows at 16-byte addresses)."""
     return (_gpu(x) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.is_contiguous() and x.stride(1) == 1
-            and x.stride(0) % 8 == 0 and kernels().stream_gemm_covers(x.shape[0], w.shape[0] // (2 if swiglu else 1), x.shape[1], swiglu))
+            and x.stride(0) % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0
+            and kernels().stream_gemm_covers(x.shape[0], w.shape[0] // (2 if swiglu else 1), x.shape[1], swiglu))
 
 
 def stream_gemm(x: torch.Tensor, w: torch.Tensor, epi: int = 0) -> torch.Tensor:
