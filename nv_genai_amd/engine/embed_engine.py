@@ -125,11 +125,14 @@ class EmbeddingEngine:
                     cu.append(cu[-1] + len(seqs[b]))
                 cu_t = torch.tensor(cu, dtype=torch.int32)
                 rows = torch.tensor(batch, dtype=torch.int64)
-                if pin:
-                    ids, pos, cu_t, rows = (t.pin_memory() for t in (ids, pos, cu_t, rows))
                 tt = None
                 if type_ids is not None:
                     tt = torch.tensor([t for b in batch for t in type_ids[b]], dtype=torch.int32)
+                if isinstance(self.model, EncoderModel):
+                    self.model.check_tokens(ids, max(len(seqs[b]) for b in batch), tt)
+                if pin:
+                    ids, pos, cu_t, rows = (t.pin_memory() for t in (ids, pos, cu_t, rows))
+                if tt is not None:
                     tt = (tt.pin_memory() if pin else tt).to(self.device, non_blocking=True)
                 with gpu_range(f"embed n={len(batch)} tok={tok}"):
                     res = self.model.forward(ids.to(self.device, non_blocking=True),

@@ -128,6 +128,16 @@ class EncoderModel:
             out["classifier.bias"] = self.cls_b
         return out
 
+    def check_tokens(self, ids: torch.Tensor, longest: int, type_ids: Optional[torch.Tensor] = None) -> None:
+        """Raises IndexError where host tokens do not lie in the tables (the forward on the GPU gives their sequences NaN)."""
+        for what, t, table in (("token", ids, self.word), ("type", type_ids, self.type)):
+            if t is not None and t.numel():
+                lo, hi = (int(v) for v in torch.aminmax(t))
+                if lo < 0 or hi >= table.shape[0]:
+                    raise IndexError(f"{what} {lo if lo < 0 else hi} outside the table of {table.shape[0]}")
+        if longest > self.pos.shape[0]:
+            raise IndexError(f"{longest} tokens, the table has {self.pos.shape[0]} positions")
+
     def forward(self, ids: torch.Tensor, pos: torch.Tensor, cu: torch.Tensor, max_len: int,
                 type_ids: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Packed tokens -> pooled [B, H] fp32 (L2-normalised unless configured otherwise);
