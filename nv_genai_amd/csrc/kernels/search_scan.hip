@@ -22,13 +22,17 @@ __device__ __forceinline__ uint32_t ss_key(float f) {
 }
 constexpr uint32_t KEY_NEG_INF = 0x007fffffu;
 
+// order of results: the higher value, of equal ones the lower row
+__device__ __forceinline__ bool ss_first(float av, int ar, float bv, int br) { return (av > bv) | ((av == bv) & (ar < br)); }
+
+// a lane sees its rows in ascending order: one of equal value goes behind, and what it pushes down keeps its order
 template <int K>
 __device__ __forceinline__ void ss_insert(float (&v)[K], int (&r)[K], float x, int row) {
   float cv = x;
   int cr = row;
 #pragma unroll
   for (int j = 0; j < K; ++j) {
-    const bool sw = cv > v[j];
+    const bool sw = x > v[j];   // from the place of x on
     const float tv = v[j];
     const int tr = r[j];
     v[j] = sw ? cv : tv;
@@ -50,7 +54,7 @@ __device__ __forceinline__ void ss_merge_xor(float (&v)[K], int (&r)[K], int mas
   }
 #pragma unroll
   for (int j = 0; j < K; ++j) {
-    const bool tb = ov[K - 1 - j] > v[j];
+    const bool tb = ss_first(ov[K - 1 - j], orr[K - 1 - j], v[j], r[j]);
     v[j] = tb ? ov[K - 1 - j] : v[j];
     r[j] = tb ? orr[K - 1 - j] : r[j];
   }
@@ -59,7 +63,7 @@ __device__ __forceinline__ void ss_merge_xor(float (&v)[K], int (&r)[K], int mas
 #pragma unroll
     for (int j = 0; j < K; ++j) {
       if ((j & st) == 0) {
-        const bool sw = v[j + st] > v[j];
+        const bool sw = ss_first(v[j + st], r[j + st], v[j], r[j]);
         const float a = v[j], b = v[j + st];
         const int ra = r[j], rb = r[j + st];
         v[j] = sw ? b : a;
@@ -459,23 +463,24 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
           }
         int head[SS_W] = {0, 0, 0, 0};
         for (int j = 0; j < n && pos + j < p.cap; ++j) {
-          float best = -INFINITY;
-          int bu = 0;
+          float x[SS_W], best = -INFINITY;
+          int xr[SS_W], bu = 0, row = -1;
 #pragma unroll
           for (int u = 0; u < SS_W; ++u) {
-            const float x = head[u] < K ? lv[u * K + head[u]] : -INFINITY;
-            if (x > best) {
-              best = x;
-              bu = u;
-            }
+            const int at = u * K + (head[u] < K ? head[u] : K - 1);
+            x[u] = head[u] < K ? lv[at] : -INFINITY;
+            xr[u] = lr[at];
           }
-          int row = -1;
+#pragma unroll
+          for (int u = 0; u < SS_W; ++u) {
+            const bool first = ss_first(x[u], xr[u], best, row);
+            best = first ? x[u] : best;
+            bu = first ? u : bu;
+            row = first ? xr[u] : row;
+          }
 #pragma unroll
           for (int u = 0; u < SS_W; ++u)
-            if (u == bu) {
-              row = lr[u * K + head[u]];
-              ++head[u];
-            }
+            if (u == bu) ++head[u];
           p.cand_v[(int64_t)q * p.cap + pos + j] = best;
           p.cand_r[(int64_t)q * p.cap + pos + j] = row;
         }
@@ -490,7 +495,8 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
 // maxima where k is at most 32) is a lower bound of the k-th largest value, so a first pass takes maxima, their ranks (by
 // counting) give the bound, and a second pass collects what reaches it: a few more than k values, which are ranked by
 // counting again. Eight loads are in flight per thread. Values of -inf (removed rows) are left out. Should more than
-// 1,024 values reach the bound (equal scores), the k-th key is found bit by bit. Three passes over 2,048 LDS counters,
+// 1,024 values reach the bound (equal scores), the k-th key is found bit by bit, and the last row that is taken of those with
+// that key in the same way. Three passes over 2,048 LDS counters,
 // most of them on the same few exponents, took 82 us for both levels of 33 x 250k scores, k 25; these take 30.
 // Order: value, then row (the lower first).
 namespace {
@@ -577,22 +583,31 @@ __device__ __forceinline__ int sel_topk(const float* __restrict__ v, const int32
       for (int64_t i = t; i < n; i += 256) c += ss_key(v[i]) >= cand;
       if (sel_block_count(c, s.red) >= k) kth = cand;
     }
+    int above = 0;
+    for (int64_t i = t; i < n; i += 256) above += ss_key(v[i]) > kth;
+    const int left = k - sel_block_count(above, s.red);   // at least one of those that are equal
+    uint32_t last = 0;   // the largest row such that fewer than `left` of them lie below it; rows are not negative
+    for (int b = 30; b >= 0; --b) {
+      const uint32_t cand = last | (1u << b);
+      int c = 0;
+      for (int64_t i = t; i < n; i += 256) c += ss_key(v[i]) == kth && (uint32_t)(r ? r[i] : (int32_t)(row0 + i)) < cand;
+      if (sel_block_count(c, s.red) < left) last = cand;
+    }
     __syncthreads();
     if (t == 0) s.n_got = 0;
     __syncthreads();
-    for (int pass = 0; pass < 2; ++pass) {   // above it (fewer than k), then equal ones until k are there
-      for (int64_t i = t; i < n; i += 256) {
-        const uint32_t key = ss_key(v[i]);
-        if (pass == 0 ? key > kth : key == kth) {
-          const uint32_t pos = atomicAdd(&s.n_got, 1u);
-          if (pos < (uint32_t)k) {
-            s.key[pos] = key;
-            s.row[pos] = r ? r[i] : (int32_t)(row0 + i);
-          }
+    for (int64_t i = t; i < n; i += 256) {
+      const uint32_t key = ss_key(v[i]);
+      const int32_t row = r ? r[i] : (int32_t)(row0 + i);
+      if (key > kth || (key == kth && (uint32_t)row <= last)) {
+        const uint32_t pos = atomicAdd(&s.n_got, 1u);
+        if (pos < (uint32_t)k) {
+          s.key[pos] = key;
+          s.row[pos] = row;
         }
       }
-      __syncthreads();
     }
+    __syncthreads();
     got = (int)s.n_got < k ? (int)s.n_got : k;
   }
   for (int i = t; i < got; i += 256) {
