@@ -14,8 +14,8 @@ addressing table fed numpy batches), and tombstones are one device scatter per c
 ingesting or deleting millions of chunks never loops over ids in Python or syncs per row.
 
 Search is one native call (``ops.flat_search``): the MFMA scoring stream keeps a per-lane register top-k, so only
-candidates reach HBM before the final merge, which gives external ids. Dimensions that it does not cover take
-``ops.search_topk``.
+candidates reach HBM before the final merge, which gives external ids. Dimensions that it does not cover, and hundreds
+of queries over many rows (``ops.search_many``), take ``ops.search_topk``.
 
 Metrics: ``ip`` (inner product), ``cosine`` (vectors/queries pre-normalised, then ip),
 ``l2``. Search returns (scores [nq, k], ids [nq, k]) with external int64 ids.
@@ -146,7 +146,8 @@ class FlatIndex:
         if q.dim() == 1:
             q = q.unsqueeze(0)
         nq = q.shape[0]
-        if self.n and 0 < nq <= 65535 and ops.search_covers(self.X, min(k, self.n)):
+        if (self.n and 0 < nq <= 65535 and ops.search_covers(self.X, min(k, self.n))
+                and not ops.search_many(nq, self.n, self.dim, min(k, self.n))):
             with gpu_range(f"search q={nq} n={self.n}"):
                 q = q.to(self.device, torch.float32)
                 n = self.n

@@ -1770,6 +1770,16 @@ def search_covers(X: torch.Tensor, k: int, most: int = 256) -> bool:
             and 1 <= k <= most and 0 < X.shape[0] < 2 ** 31 and bool(kernels().search_covers(X.shape[1])))
 
 
+def search_many(nq: int, rows: int, D: int, k: int) -> bool:
+    """Whether many queries over all rows are faster through ``search_topk``, whose kernel (vector_search.hip) holds 64 queries
+    in registers' reach and reads the vectors straight into fragments: then the products bound the scan and not the stream of
+    vectors, of which the other has half the LDS full of queries. The line lies at 4.5e10 products of whole groups of 64
+    queries, vectors below 512 dimensions counted as such, for what its register lists hold (k 8). k 4, us, this / that:
+    1M x 1,024, 65 queries 791 / 899, 512: 2,290 / 3,266; 100k x 1,024, 256: 249 / 224, 512: 380 / 386, 4,096: 1,781 / 2,614;
+    300k x 256, 256: 241 / 243, 1,000: 616 / 762; 1M x 128, 1,000: 1,206 / 987."""
+    return nq > 64 and k <= kernels().score_topk_kmax(64) and D >= 256 and -(-nq // 64) * 64 * rows * max(D, 512) >= 4.5e10
+
+
 def flat_search(q: torch.Tensor, X: torch.Tensor, row_bias: torch.Tensor, ids: torch.Tensor, metric: str,
                 k: int) -> Tuple[torch.Tensor, torch.Tensor]:
     """Top-k of every row of X [N, D] for fp32 queries q [nq, D]: query preparation (normalised for cosine), scan, merge

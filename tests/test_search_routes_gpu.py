@@ -1,0 +1,42 @@
+"""Searches of many queries: which kernels take them, and that both give the same."""
+import pytest
+import torch
+
+from nv_genai_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _spy(monkeypatch, name):
+    calls, f = [], getattr(ops, name)
+    monkeypatch.setattr(ops, name, lambda *a: calls.append(1) or f(*a))
+    return calls
+
+
+def _same(a, b):
+    """Scores to the order of their fp32 sums, and for cosine to one element of a query that the norm's last bit rounds to the
+    other bf16 neighbour: 2^-8 of a product of two elements of unit vectors, which stay below 0.16 at 1,024 dimensions. Ids
+    but for neighbours whose scores that turns round."""
+    assert torch.allclose(a[0], b[0], rtol=1e-5, atol=1e-4) and (a[1] == b[1]).float().mean() > 0.999
+
+
+@pytest.mark.parametrize("nq,rows,k,here", [(4096, 10_728, 4, True), (4096, 10_730, 4, False), (4096, 10_730, 9, True),
+                                            (4096, 10_730, 8, False), (4033, 10_730, 1, False), (4032, 10_730, 1, True)])
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+def test_flat_of_many_queries(gpu, monkeypatch, nq, rows, k, here, metric):
+    from nv_genai_amd.index.flat import FlatIndex
+
+    g = torch.Generator(device="cuda").manual_seed(rows + k)
+    idx = FlatIndex(1024, metric, "cuda", capacity=rows)
+    idx.add(torch.randn(rows, 1024, device=gpu, generator=g), torch.arange(rows) + 7)
+    idx.remove([9, 11])
+    q = torch.randn(nq, 1024, device=gpu, generator=g)
+    calls = _spy(monkeypatch, "flat_search")
+    a = idx.search(q, k)
+    assert bool(calls) == here
+    monkeypatch.setattr(ops, "search_many", lambda *a: here)   # the other route
+    _same(idx.search(q, k), a)
+
+
+def test_flat_of_many_short_vectors_or_few_queries(gpu):
+    assert not ops.search_many(10_000, 10 ** 7, 128, 4) and not ops.search_many(64, 10 ** 8, 1024, 4)
