@@ -146,7 +146,8 @@ class IVFFlatIndex:
         self._ensure_trained()
         np_ = min(nprobe or self.nprobe, self.nlist)
         if (self.is_trained and 0 < nq <= 4096 and 1 <= np_ and self.nlist <= ops.IVF_SCAN_MAX_LISTS
-                and self.centroids.shape[0] == self.nlist and ops.search_covers(self.X, k, 32) and k <= self.X.shape[0]):
+                and self.centroids.shape[0] == self.nlist and ops.search_covers(self.X, k, 32) and k <= self.X.shape[0]
+                and not ops.search_many_lists(nq, self.X.shape[0], self.dim, k, self.nlist, np_)):
             beg, end, _ = self._list_ranges()
             q = q.to(self.device, torch.float32)
             return ops.ivf_search(q if q.stride(1) == 1 else q.contiguous(), self.X, self.bias, self.ids,

@@ -40,3 +40,29 @@ def test_flat_of_many_queries(gpu, monkeypatch, nq, rows, k, here, metric):
 
 def test_flat_of_many_short_vectors_or_few_queries(gpu):
     assert not ops.search_many(10_000, 10 ** 7, 128, 4) and not ops.search_many(64, 10 ** 8, 1024, 4)
+
+
+@pytest.mark.parametrize("nq,nprobe,k,here", [(1024, 2, 4, False), (1024, 2, 9, True), (700, 2, 4, True)])
+def test_lists_of_many_queries(gpu, monkeypatch, nq, nprobe, k, here):
+    """Two lists of 100,000 x 1,024 rows, both probed."""
+    from nv_genai_amd.index.ivf import IVFFlatIndex
+
+    g = torch.Generator(device="cuda").manual_seed(nq + k)
+    X = torch.randn(200_000, 1024, device=gpu, generator=g)
+    idx = IVFFlatIndex(1024, 2, nprobe, "l2", "cuda")
+    idx.train(X[:2000], iters=1, seed=1)
+    idx.add(X, torch.arange(200_000) + 7)
+    q = torch.randn(nq, 1024, device=gpu, generator=g)
+    calls = _spy(monkeypatch, "ivf_search")
+    a = idx.search(q, k)
+    assert bool(calls) == here
+    if k <= 8:   # the other route; above, it goes query by query
+        monkeypatch.setattr(ops, "search_many_lists", lambda *a: here)
+        _same(idx.search(q, k), a)
+
+
+def test_lists_that_stay(gpu):
+    """Short lists, short vectors, few probes."""
+    for rows, D, nlist, nprobe in ((300_000, 1024, 64, 64), (1_000_000, 512, 64, 64), (1_000_000, 1024, 64, 4)):
+        assert not ops.search_many_lists(4096, rows, D, 4, nlist, nprobe)
+    assert ops.search_many_lists(4096, 1_000_000, 1024, 4, 64, 8) and ops.search_many_lists(256, 1_000_000, 1024, 8, 64, 64)
