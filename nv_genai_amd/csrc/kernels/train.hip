@@ -390,10 +390,13 @@ __global__ void __launch_bounds__(512) ce_fwd_kernel(const uint16_t* __restrict_
     if (m > -INFINITY) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) s += __expf(v[j] - m);
+    } else {   // -inf throughout, or NaN, which the maximum leaves out
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += v[j] == v[j] ? 0.f : v[j];
     }
   }
   const float M = block_max(m, red);
-  s = m > -INFINITY ? s * __expf(m - M) : 0.f;
+  if (m > -INFINITY) s *= __expf(m - M);
   s = block_sum(s, red);
   if (threadIdx.x == 0) {
     const float l = M + logf(s);

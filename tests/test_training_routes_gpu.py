@@ -188,3 +188,20 @@ def test_second_derivatives(gpu, monkeypatch, kind):
             return Fn.encoder_embed(m, ids, torch.ones_like(ids), Q).pow(3).sum()
 
     _twice(monkeypatch, f, xs, 5e-2)
+
+
+@pytest.mark.parametrize("once", [False, True])
+@pytest.mark.parametrize("at,n", [(0, 8), (0, 4104), (8, 1), (4088, 8), (4096, 8), (0, 0)])
+def test_logits_that_are_not_numbers(gpu, once, at, n):
+    """A NaN anywhere in a row, also where a thread of the one-pass form sees nothing else, makes its loss and gradient NaN;
+    -inf does not."""
+    lg = _rows(2, 4104)
+    lg[:, 16:24] = float("-inf")
+    lg[1, at:at + n] = float("nan")
+    lg.requires_grad_()
+    y = torch.tensor([5, 100], device=gpu)
+    loss = fused.cross_entropy_sum(lg, y, once)
+    want = torch.nn.functional.cross_entropy(lg.double(), y, reduction="sum")
+    assert loss.isnan() == want.isnan() == (n > 0) and (n or abs(loss - want) < 1e-4)
+    g = torch.autograd.grad(loss, lg)[0]
+    assert not g[0].isnan().any() and g[1].isnan().all() == (n > 0)
