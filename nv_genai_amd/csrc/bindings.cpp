@@ -2705,7 +2705,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("embedding", checked("embedding", &embedding));
   m.def("score", checked("score", &score));
   m.def("topk", checked("topk", &topk));
-  m.def("encoder_forward", &encoder_forward);
+  m.def("encoder_forward", &encoder_forward, py::call_guard<py::gil_scoped_release>());   // some 200 launches
   m.def("encoder_covers", [](const Tensor& word, const std::vector<Tensor>& tables, const std::vector<Tensor>& L, int64_t heads) {
     return encoder_refuses(word, tables, L, heads) == nullptr;
   });

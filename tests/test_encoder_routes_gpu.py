@@ -65,3 +65,27 @@ def test_one_type_for_all_tokens(gpu):
     m, t = _model(gpu), _tokens(gpu, 30)
     one = torch.ones(1, device=gpu, dtype=torch.int32)
     _close(m.forward(*t, one), m.forward(*t, one.expand(30).contiguous()))
+
+
+def test_other_threads_run_during_the_launches(gpu):
+    """The native call gives up the interpreter lock: with switching by time off, a waiting thread can only run while it does."""
+    import sys
+    import threading
+
+    m, (ids, pos, cu, longest) = _model(gpu), _tokens(gpu, 30)
+    w = [L[n] for L in m.layers for n in ops.ENCODER_LAYER] * 40   # as long as a large model's
+    go, ran = threading.Event(), []
+    t = threading.Thread(target=lambda: (go.wait(), ran.append(1)))
+    t.start()
+    was = sys.getswitchinterval()
+    sys.setswitchinterval(1000.0)
+    try:
+        f = ops.kernels().encoder_forward
+        go.set()
+        for _ in range(20):
+            f(ids, pos, None, cu, longest, m.word, m.pos, m.type, m.emb_ln[0], m.emb_ln[1], w, m.cfg.heads, m.cfg.eps, m.scale)
+        seen = bool(ran)
+    finally:
+        sys.setswitchinterval(was)
+    t.join()
+    assert seen
