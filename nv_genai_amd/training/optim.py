@@ -5,7 +5,7 @@ from __future__ import annotations
 
 import inspect
 from collections import defaultdict
-from typing import Optional
+from typing import Optional, Sequence
 
 import torch
 
@@ -36,15 +36,16 @@ class AdamW(torch.optim.AdamW):
         return dev is not None and not (dev.type == "cuda" and torch.cuda.is_current_stream_capturing())
 
     @torch.no_grad()
-    def step(self, closure=None, max_norm: Optional[float] = None):
-        """One step; ``max_norm``: first scale all gradients (in place) to that norm, as ``clip_grad_norm_`` does."""
+    def step(self, closure=None, max_norm: Optional[float] = None, among: Optional[Sequence[torch.Tensor]] = None):
+        """One step; ``max_norm``: first scale all gradients (in place) to that norm, as ``clip_grad_norm_`` does, which where it
+        does the work itself adds up the norms in the order of ``among`` (the groups' order otherwise)."""
         loss = None
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
         if not self._covers():
             if max_norm:
-                torch.nn.utils.clip_grad_norm_([p for g in self.param_groups for p in g["params"]], max_norm)
+                torch.nn.utils.clip_grad_norm_(among or [p for g in self.param_groups for p in g["params"]], max_norm)
             for g in self.param_groups:   # torch's fused step keeps the count beside the weights
                 for p in g["params"]:
                     st = self.state.get(p)

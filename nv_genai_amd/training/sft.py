@@ -145,7 +145,7 @@ class Trainer:
             loss.backward()
             total += float(loss.detach())
         self.sync.finish()
-        self.opt.step(max_norm=cfg.grad_clip)
+        self.opt.step(max_norm=cfg.grad_clip, among=self.params)
         self.step += 1
         if self.world > 1:
             t = torch.tensor([total], dtype=torch.float64, device=self.params[0].device)
