@@ -201,6 +201,8 @@ def lm_loss(model, hidden: torch.Tensor, labels: torch.Tensor, params: Optional[
     for s in range(0, h.shape[0], chunk):
         lg = h[s:s + chunk] @ head.t()
         if fused.cross_entropy_usable(lg):
+            if s == 0 and params is None and int(y.max()) >= lg.shape[1]:   # the one-pass form would give NaN
+                raise IndexError(f"label {int(y.max())} outside the vocabulary of {lg.shape[1]}")
             total = total + fused.cross_entropy_sum(lg, y[s:s + chunk], params is None)
         else:
             total = total + F.cross_entropy(lg.float(), y[s:s + chunk], reduction="sum")

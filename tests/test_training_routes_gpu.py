@@ -205,3 +205,14 @@ def test_logits_that_are_not_numbers(gpu, once, at, n):
     assert loss.isnan() == want.isnan() == (n > 0) and (n or abs(loss - want) < 1e-4)
     g = torch.autograd.grad(loss, lg)[0]
     assert not g[0].isnan().any() and g[1].isnan().all() == (n > 0)
+
+
+def test_labels_outside_the_vocabulary_raise(gpu):
+    m = _llama(gpu)
+    V = m.lm_head.shape[0]
+    h, lab = _rows(1, 6, m.cfg.hidden), torch.tensor([[-100, 3, V - 1, -1, 0, 5]], device=gpu)
+    assert torch.isfinite(Fn.lm_loss(m, h, lab))
+    assert float(Fn.lm_loss(m, h, torch.full_like(lab, -100))) == 0.0
+    lab[0, 4] = V
+    with pytest.raises(IndexError):
+        Fn.lm_loss(m, h, lab)
