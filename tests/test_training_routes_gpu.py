@@ -216,3 +216,39 @@ def test_labels_outside_the_vocabulary_raise(gpu):
     lab[0, 4] = V
     with pytest.raises(IndexError):
         Fn.lm_loss(m, h, lab)
+
+
+@pytest.mark.parametrize("how,reached", [
+    ("params", {"rms_norm", "add_rms_norm", "rope", "swiglu", "cross_entropy_sum"}),
+    ("checkpointed", {"rms_norm", "add_rms_norm", "rope", "swiglu", "cross_entropy_sum"}),
+    ("lora", {"rms_norm", "add_rms_norm", "attention", "lora_linear", "swiglu", "cross_entropy_sum"}),
+    ("encoder", {"linear", "residual_layer_norm", "gelu"})])
+def test_models_reach_the_functions(gpu, monkeypatch, how, reached):
+    """Comparisons of the models with and without the functions compare something: these are called, and without them none is."""
+    from nv_genai_amd.models.config import encoder_config
+    from nv_genai_amd.models.encoder import EncoderModel
+    from nv_genai_amd.training.lora import LoRA, LoRAConfig
+
+    called = set()
+    names = {"rms_norm", "add_rms_norm", "rope", "swiglu", "cross_entropy_sum", "attention", "lora_linear", "linear",
+             "residual_layer_norm", "gelu"}
+    for n in names:
+        monkeypatch.setattr(fused, n, lambda *a, n=n, f=getattr(fused, n): called.add(n) or f(*a))
+    m = EncoderModel(encoder_config("encoder-tiny"), gpu, seed=2) if how == "encoder" else _llama(gpu)
+    ids = torch.randint(0, 1000, (2, 40), device=gpu)
+
+    def run():
+        with torch.autocast("cuda", dtype=BF):
+            if how == "encoder":
+                return Fn.encoder_embed(m, ids, torch.ones_like(ids), Fn.trainable_params(m, "encoder")).sum()
+            if how == "lora":
+                return Fn.lm_loss(m, Fn.llama_hidden(m, ids, linear=LoRA(m, LoRAConfig(r=8, alpha=16), seed=1).linear), ids)
+            P = Fn.trainable_params(m, "llama")
+            return Fn.lm_loss(m, Fn.llama_hidden(m, ids, params=P, grad_ckpt=how == "checkpointed"), ids, params=P)
+
+    run().backward()
+    assert called == reached
+    called.clear()
+    _without(monkeypatch)
+    run().backward()
+    assert not called
