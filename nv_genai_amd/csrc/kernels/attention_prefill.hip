@@ -9,7 +9,7 @@
 //   O^T += V^T . P^T (the S accumulator is the P^T B operand with no lane movement — same
 //   key<->row mapping as attention_decode.hip).
 // The next tile's K/V are loaded into registers before the current tile's MFMAs and written
-// to LDS after the barrier (issue-early / write-late, guide §5.5 T14).
+// to LDS after the barrier (issued early, written late).
 //
 // K from the [blocks, Hkv, 64, D] cache, V^T from the [blocks, Hkv, D, 64] cache, queries are
 // the last q_len positions of a ctx_len context (chunked prefill and prefix-cache hits work
@@ -32,19 +32,16 @@ __device__ __forceinline__ int row_swz(int row) {  // 4-bit key: distinct over a
 }
 }  // namespace
 
-template <int D, bool CAUSAL, int NCG>
+template <int D, bool CAUSAL>
 __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, uint16_t* v_s, int b, int hq,
                                         int tile) {
-  // NCG query column-groups (16 rows each) per wave: the K and V^T fragments read from LDS
-  // for one key tile feed NCG MFMAs each, and the tile's staging + barriers are amortised
-  // over a 64*NCG-row query tile.
-  constexpr int KT = 64;          // keys per tile (= KV page size when PAGED)
+  constexpr int KT = 64;          // keys per tile (= KV page size)
   constexpr int NCH_K = D / 8;    // 16-B chunks per K row
   constexpr int DS = D / 32;      // d-steps of the QK^T MFMA
   constexpr int DT = D / 16;      // d-tiles of the PV MFMA
   constexpr int K_CHUNKS = KT * NCH_K;   // = V chunks too
   constexpr int PER_T = K_CHUNKS / 256;  // chunks per thread per operand
-  constexpr int QT = 64 * NCG;           // query rows per workgroup
+  constexpr int QT = 64;                 // query rows per workgroup
 
   // K-row swizzle: XOR the 16-B chunk index with up to 4 bits of the row (fewer for short
   // rows: the XOR value must stay below the chunk count)
@@ -59,24 +56,18 @@ __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, u
   const int col = lane & 15, h = lane >> 4;
   const int tid = threadIdx.x;
 
-  // this lane's query rows (one per column group)
-  int qr[NCG], qpos[NCG];
-  bool row_ok[NCG];
-  bf16x8 qf[NCG][DS];
+  // this lane's query row
+  int qr = tile * QT + w * 16 + col;
+  const bool row_ok = qr < qlen;
+  if (!row_ok) qr = qlen - 1;
+  const int qpos = ctx - qlen + qr;  // absolute key index of this query
+  bf16x8 qf[DS];
+  const uint16_t* qp = P.q + (int64_t)(q0 + qr) * P.q_stride + (int64_t)hq * D;
 #pragma unroll
-  for (int cg = 0; cg < NCG; ++cg) {
-    int r = tile * QT + w * 16 * NCG + cg * 16 + col;
-    row_ok[cg] = r < qlen;
-    if (!row_ok[cg]) r = qlen - 1;
-    qr[cg] = r;
-    qpos[cg] = ctx - qlen + r;  // absolute key index of this query
-    const uint16_t* qp = P.q + (int64_t)(q0 + r) * P.q_stride + (int64_t)hq * D;
-#pragma unroll
-    for (int s2 = 0; s2 < DS; ++s2) qf[cg][s2] = as_bf16x8(load8(qp + 32 * s2 + 8 * h));
-  }
+  for (int s2 = 0; s2 < DS; ++s2) qf[s2] = as_bf16x8(load8(qp + 32 * s2 + 8 * h));
 
-  const int qpos_w0 = ctx - qlen + tile * QT + w * 16 * NCG;  // smallest query position of this wave
-  const int qpos_w1 = qpos_w0 + 16 * NCG - 1;                  // largest (may exceed ctx: masked rows)
+  const int qpos_w0 = ctx - qlen + tile * QT + w * 16;  // smallest query position of this wave
+  const int qpos_w1 = qpos_w0 + 15;                     // largest (may exceed ctx: masked rows)
   const int W = CAUSAL ? P.window : 0;
   int last_key = ctx - 1;
   if (CAUSAL) {
@@ -130,34 +121,27 @@ __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, u
   };
 
   const float sl2 = P.scale * LOG2E_P;
-  float m[NCG], l[NCG];
-  f32x4 o[NCG][DT];
+  float m = -INFINITY, l = 0.f;
+  f32x4 o[DT];
 #pragma unroll
-  for (int cg = 0; cg < NCG; ++cg) {
-    m[cg] = -INFINITY;
-    l[cg] = 0.f;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) o[cg][dt] = (f32x4)(0.f);
-  }
+  for (int dt = 0; dt < DT; ++dt) o[dt] = (f32x4)(0.f);
 
   // (Tried: separate masked/unmasked instantiations of this body behind a wave-uniform
   // branch to drop the ~60 if-converted mask selects per tile. 39.3 -> 34.5 us at 1 x 1,196
   // but 658 -> 672 us at 27 x 1,200: the two bodies need 252 VGPRs, 3 -> 2 waves/SIMD, and
   // forcing 3 waves spills.)
   auto compute_tile = [&](int t) {
-      f32x4 sacc[NCG][4];
+      f32x4 sacc[4];
 #pragma unroll
       for (int tau = 0; tau < 4; ++tau) {
         const int row = 32 * (tau >> 1) + 8 * (col >> 2) + 4 * (tau & 1) + (col & 3);
         const int sw = row_swz(row) >> SWS;
-#pragma unroll
-        for (int cg = 0; cg < NCG; ++cg) sacc[cg][tau] = (f32x4)(0.f);
+        sacc[tau] = (f32x4)(0.f);
 #pragma unroll
         for (int s2 = 0; s2 < DS; ++s2) {
           const int ch = 4 * s2 + h;
           bf16x8 a = as_bf16x8(*reinterpret_cast<const u16x8*>(&k_s[row * D + ((ch ^ sw) * 8)]));
-#pragma unroll
-          for (int cg = 0; cg < NCG; ++cg) sacc[cg][tau] = mfma16(a, qf[cg][s2], sacc[cg][tau]);
+          sacc[tau] = mfma16(a, qf[s2], sacc[tau]);
         }
       }
       const int kbase = t * KT;
@@ -165,64 +149,58 @@ __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, u
       // of the context); the test is wave-uniform
       const bool need_mask = CAUSAL ? (kbase + KT - 1 > qpos_w0 || (W > 0 && kbase <= qpos_w1 - W))
                                     : (kbase + KT > ctx);
-      bf16x8 pf[NCG][2];
+      bf16x8 pf[2];
+      float mloc = -INFINITY;
 #pragma unroll
-      for (int cg = 0; cg < NCG; ++cg) {
-        float mloc = -INFINITY;
+      for (int tau = 0; tau < 4; ++tau)
 #pragma unroll
-        for (int tau = 0; tau < 4; ++tau)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float sv = sacc[cg][tau][r];  // raw score; the scale is folded into the exp
-            if (need_mask) {
-              const int key = kbase + 32 * (tau >> 1) + 8 * h + 4 * (tau & 1) + r;
-              const bool ok = CAUSAL ? (key <= qpos[cg] && (W == 0 || key > qpos[cg] - W)) : (key < ctx);
-              sv = ok ? sv : -INFINITY;
-            }
-            sacc[cg][tau][r] = sv;
-            mloc = fmaxf(mloc, sv);
+        for (int r = 0; r < 4; ++r) {
+          float sv = sacc[tau][r];  // raw score; the scale is folded into the exp
+          if (need_mask) {
+            const int key = kbase + 32 * (tau >> 1) + 8 * h + 4 * (tau & 1) + r;
+            const bool ok = CAUSAL ? (key <= qpos && (W == 0 || key > qpos - W)) : (key < ctx);
+            sv = ok ? sv : -INFINITY;
           }
-        mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
-        mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
-        mloc *= sl2;  // scale > 0: max commutes with it
-        // Lazy rescaling: the running max only moves (and O / l are only rescaled) when a
-        // row's tile max exceeds it by more than 2^RESCALE_LOG2; until then P = 2^(s - m)
-        // stays <= 2^8, harmless in fp32 accumulators and bf16 P. Keeps O in the MFMA
-        // accumulators instead of a VALU round trip every tile. m starts at -inf, so the
-        // first tile always rescales (alpha = 2^-inf = 0 on an all-zero O).
-        const bool grow = mloc > m[cg] + RESCALE_LOG2;
-        if (__ballot(grow)) {
-          const float m_new = grow ? mloc : m[cg];
-          // non-growing lanes keep their scale (and a still -inf m must not meet -inf - -inf)
-          const float alpha = grow ? __builtin_amdgcn_exp2f(m[cg] - m_new) : 1.f;
-          m[cg] = m_new;
-          l[cg] *= alpha;
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt) o[cg][dt] *= alpha;
+          sacc[tau][r] = sv;
+          mloc = fmaxf(mloc, sv);
         }
-        // exponent argument and row-sum in packed fp32 (v_pk_fma_f32 / v_pk_add_f32: two
-        // scores per VALU op, two independent add chains instead of one 16-long chain).
-        // Loop VALU 141 -> 128 instructions per tile at the same 148 VGPRs; kernel time within
-        // run-to-run noise (633 us at 27 x 1,200, profiles/r1_prefill_valu).
-        // a tile can be fully masked for a row (sliding window): m may still be -inf then,
-        // and the offset must not become +inf (2^(-inf + inf) = NaN)
-        const float mo = m[cg] == -INFINITY ? 0.f : -m[cg];
-        const f32x2 sl2v = {sl2, sl2}, nmc = {mo, mo};
-        f32x2 lsum = {0.f, 0.f};
+      mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
+      mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+      mloc *= sl2;  // scale > 0: max commutes with it
+      // Lazy rescaling: the running max only moves (and O / l are only rescaled) when a
+      // row's tile max exceeds it by more than 2^RESCALE_LOG2; until then P = 2^(s - m)
+      // stays <= 2^8, harmless in fp32 accumulators and bf16 P. Keeps O in the MFMA
+      // accumulators instead of a VALU round trip every tile. m starts at -inf, so the
+      // first tile always rescales (alpha = 2^-inf = 0 on an all-zero O).
+      const bool grow = mloc > m + RESCALE_LOG2;
+      if (__ballot(grow)) {
+        const float m_new = grow ? mloc : m;
+        // non-growing lanes keep their scale (and a still -inf m must not meet -inf - -inf)
+        const float alpha = grow ? __builtin_amdgcn_exp2f(m - m_new) : 1.f;
+        m = m_new;
+        l *= alpha;
 #pragma unroll
-        for (int g = 0; g < 2; ++g)
-#pragma unroll
-          for (int j = 0; j < 8; j += 2) {
-            const f32x4& sv = sacc[cg][2 * g + (j >> 2)];
-            f32x2 e = __builtin_elementwise_fma((f32x2){sv[j & 3], sv[(j & 3) + 1]}, sl2v, nmc);
-            e[0] = __builtin_amdgcn_exp2f(e[0]);  // 2^-inf = 0
-            e[1] = __builtin_amdgcn_exp2f(e[1]);
-            lsum += e;
-            pf[cg][g][j] = (__bf16)e[0];
-            pf[cg][g][j + 1] = (__bf16)e[1];
-          }
-        l[cg] += lsum[0] + lsum[1];
+        for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
       }
+      // two independent add chains instead of one 16-long chain
+      // a tile can be fully masked for a row (sliding window): m may still be -inf then,
+      // and the offset must not become +inf (2^(-inf + inf) = NaN)
+      const float mo = m == -INFINITY ? 0.f : -m;
+      const f32x2 sl2v = {sl2, sl2}, nmc = {mo, mo};
+      f32x2 lsum = {0.f, 0.f};
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+          const f32x4& sv = sacc[2 * g + (j >> 2)];
+          f32x2 e = __builtin_elementwise_fma((f32x2){sv[j & 3], sv[(j & 3) + 1]}, sl2v, nmc);
+          e[0] = __builtin_amdgcn_exp2f(e[0]);  // 2^-inf = 0
+          e[1] = __builtin_amdgcn_exp2f(e[1]);
+          lsum += e;
+          pf[g][j] = (__bf16)e[0];
+          pf[g][j + 1] = (__bf16)e[1];
+        }
+      l += lsum[0] + lsum[1];
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
         const int ch = 4 * g + h;
@@ -231,8 +209,7 @@ __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, u
           const int row = 16 * dt + col;
           bf16x8 a = as_bf16x8(
               *reinterpret_cast<const u16x8*>(&v_s[row * KT + ((ch ^ ((row >> 1) & 7)) * 8)]));
-#pragma unroll
-          for (int cg = 0; cg < NCG; ++cg) o[cg][dt] = mfma16(a, pf[cg][g], o[cg][dt]);
+          o[dt] = mfma16(a, pf[g], o[dt]);
         }
       }
   };
@@ -245,21 +222,17 @@ __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, u
     if (t + 1 < n_tiles) load_tile(t + 1, kA, vA);
     compute_tile(t);
   }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (row_ok) {
+    const float inv = (l > 0.f ? 1.f / l : 0.f) * (P.kv_fp8 ? P.v_scale : 1.f);
+    uint16_t* op = P.out + (int64_t)(q0 + qr) * P.out_stride + (int64_t)hq * D;
 #pragma unroll
-  for (int cg = 0; cg < NCG; ++cg) {
-    float ll = l[cg];
-    ll += __shfl_xor(ll, 16, 64);
-    ll += __shfl_xor(ll, 32, 64);
-    if (row_ok[cg]) {
-      const float inv = (ll > 0.f ? 1.f / ll : 0.f) * (P.kv_fp8 ? P.v_scale : 1.f);
-      uint16_t* op = P.out + (int64_t)(q0 + qr[cg]) * P.out_stride + (int64_t)hq * D;
+    for (int dt = 0; dt < DT; ++dt) {
+      u16x4 v;
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        u16x4 v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = f2bf(o[cg][dt][r] * inv);
-        *reinterpret_cast<u16x4*>(op + 16 * dt + 4 * h) = v;
-      }
+      for (int r = 0; r < 4; ++r) v[r] = f2bf(o[dt][r] * inv);
+      *reinterpret_cast<u16x4*>(op + 16 * dt + 4 * h) = v;
     }
   }
 }
@@ -270,7 +243,7 @@ __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, u
 // query heads sharing a KV head read its pages through the same L2; longest causal tiles
 // first) — or a host-planned work list of (sequence, 64-row tile) pairs walked by a fixed
 // grid with q head it % Hq (graph-captured steps with fp8 KV pages or head_dim != 128).
-template <int D, bool CAUSAL, int NCG>
+template <int D, bool CAUSAL>
 __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams P) {
   constexpr int KT = 64;
   __shared__ __attribute__((aligned(16))) uint16_t k_s[KT * D];
@@ -280,7 +253,7 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams P) {
     for (int it = blockIdx.x; it < total; it += gridDim.x) {
       __syncthreads();
       const int k = it / P.Hq;
-      v1_tile<D, CAUSAL, NCG>(P, k_s, v_s, P.items[2 * k], it % P.Hq, P.items[2 * k + 1]);
+      v1_tile<D, CAUSAL>(P, k_s, v_s, P.items[2 * k], it % P.Hq, P.items[2 * k + 1]);
     }
     return;
   }
@@ -290,21 +263,21 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams P) {
   const int tile = P.ntiles - 1 - L % P.ntiles;
   const int hq = (L / P.ntiles) % P.Hq;
   const int b = L / (P.ntiles * P.Hq);
-  v1_tile<D, CAUSAL, NCG>(P, k_s, v_s, b, hq, tile);
+  v1_tile<D, CAUSAL>(P, k_s, v_s, b, hq, tile);
 }
 
 void launch_prefill_attention_v1_worklist(const PrefillParams& p, int grid, int D, bool causal,
                                           hipStream_t stream) {
   dim3 g(grid);
   if (D == 256) {
-    if (causal) prefill_attn_kernel<256, true, 1><<<g, 256, 0, stream>>>(p);
-    else prefill_attn_kernel<256, false, 1><<<g, 256, 0, stream>>>(p);
+    if (causal) prefill_attn_kernel<256, true><<<g, 256, 0, stream>>>(p);
+    else prefill_attn_kernel<256, false><<<g, 256, 0, stream>>>(p);
   } else if (D == 128) {
-    if (causal) prefill_attn_kernel<128, true, 1><<<g, 256, 0, stream>>>(p);
-    else prefill_attn_kernel<128, false, 1><<<g, 256, 0, stream>>>(p);
+    if (causal) prefill_attn_kernel<128, true><<<g, 256, 0, stream>>>(p);
+    else prefill_attn_kernel<128, false><<<g, 256, 0, stream>>>(p);
   } else {
-    if (causal) prefill_attn_kernel<64, true, 1><<<g, 256, 0, stream>>>(p);
-    else prefill_attn_kernel<64, false, 1><<<g, 256, 0, stream>>>(p);
+    if (causal) prefill_attn_kernel<64, true><<<g, 256, 0, stream>>>(p);
+    else prefill_attn_kernel<64, false><<<g, 256, 0, stream>>>(p);
   }
 }
 
@@ -325,8 +298,8 @@ void launch_prefill_attention(const PrefillParams& p, int num_seqs, int max_q_le
   dim3 grid(8 * pp.per_xcd);
 #define NGA_PF(DD)                                                            \
   do {                                                                        \
-    if (causal) prefill_attn_kernel<DD, true, 1><<<grid, 256, 0, stream>>>(pp); \
-    else prefill_attn_kernel<DD, false, 1><<<grid, 256, 0, stream>>>(pp);       \
+    if (causal) prefill_attn_kernel<DD, true><<<grid, 256, 0, stream>>>(pp); \
+    else prefill_attn_kernel<DD, false><<<grid, 256, 0, stream>>>(pp);       \
   } while (0)
   if (D == 256) NGA_PF(256);   // Gemma
   else if (D == 128) NGA_PF(128);

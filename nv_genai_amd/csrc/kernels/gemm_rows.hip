@@ -22,31 +22,26 @@ __device__ __forceinline__ float gr_gelu(float x) { return 0.5f * x * (1.f + erf
 // EPI 0: bf16 out, + bias; 1: fp32 slab [split, M, N]; 2: bf16 out, GELU(. + bias)
 template <int MT, int EPI>
 __global__ void __launch_bounds__(512) row_gemm_kernel(RowGemmParams P) {
-  constexpr int NT = 1, PD = 4, NW = 8;
-  __shared__ __attribute__((aligned(16))) float part[NW * MT * NT * 256];
+  constexpr int PD = 4, NW = 8;
+  __shared__ __attribute__((aligned(16))) float part[NW * MT * 256];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, h = lane >> 4;
-  const int f0 = blockIdx.x * 16 * NT, t0 = blockIdx.y * 16 * MT, ks = blockIdx.z;
+  const int f0 = blockIdx.x * 16, t0 = blockIdx.y * 16 * MT, ks = blockIdx.z;
   const int steps = P.K / 32, slices = NW * P.split, sl = ks * NW + w;
   const int s0 = steps * sl / slices, s1 = steps * (sl + 1) / slices;
-  const uint16_t *wp[NT], *xp[MT];
-#pragma unroll
-  for (int i = 0; i < NT; ++i) wp[i] = P.w + (int64_t)(f0 + 16 * i + col) * P.K + 8 * h;
+  const uint16_t *wp = P.w + (int64_t)(f0 + col) * P.K + 8 * h, *xp[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) xp[i] = P.x + (int64_t)min(t0 + 16 * i + col, P.M - 1) * P.ldx + 8 * h;
-  f32x4 acc[NT][MT];
+  f32x4 acc[MT];
 #pragma unroll
-  for (int i = 0; i < NT; ++i)
-#pragma unroll
-    for (int j = 0; j < MT; ++j) acc[i][j] = (f32x4)(0.f);
-  u16x8 a[PD][NT], b[PD][MT], an[PD][NT], bn[PD][MT];
-  auto load = [&](int s, u16x8 (&av)[PD][NT], u16x8 (&bv)[PD][MT]) {
+  for (int j = 0; j < MT; ++j) acc[j] = (f32x4)(0.f);
+  u16x8 a[PD], b[PD][MT], an[PD], bn[PD][MT];
+  auto load = [&](int s, u16x8 (&av)[PD], u16x8 (&bv)[PD][MT]) {
 #pragma unroll
     for (int d = 0; d < PD; ++d)
       if (s + d < s1) {
-#pragma unroll
-        for (int i = 0; i < NT; ++i) av[d][i] = load8(wp[i] + 32 * (s + d));
+        av[d] = load8(wp + 32 * (s + d));
 #pragma unroll
         for (int i = 0; i < MT; ++i) bv[d][i] = load8(xp[i] + 32 * (s + d));
       }
@@ -58,35 +53,28 @@ __global__ void __launch_bounds__(512) row_gemm_kernel(RowGemmParams P) {
     for (int d = 0; d < PD; ++d)
       if (s + d < s1) {
 #pragma unroll
-        for (int i = 0; i < NT; ++i)
-#pragma unroll
-          for (int j = 0; j < MT; ++j) acc[i][j] = mfma16(as_bf16x8(a[d][i]), as_bf16x8(b[d][j]), acc[i][j]);
+        for (int j = 0; j < MT; ++j) acc[j] = mfma16(as_bf16x8(a[d]), as_bf16x8(b[d][j]), acc[j]);
       }
     if (s + PD < s1) {
 #pragma unroll
       for (int d = 0; d < PD; ++d) {
-#pragma unroll
-        for (int i = 0; i < NT; ++i) a[d][i] = an[d][i];
+        a[d] = an[d];
 #pragma unroll
         for (int i = 0; i < MT; ++i) b[d][i] = bn[d][i];
       }
     }
   }
 #pragma unroll
-  for (int i = 0; i < NT; ++i)
-#pragma unroll
-    for (int j = 0; j < MT; ++j)
-      *reinterpret_cast<f32x4*>(&part[(((w * NT + i) * MT + j) * 64 + lane) * 4]) = acc[i][j];
+  for (int j = 0; j < MT; ++j) *reinterpret_cast<f32x4*>(&part[((w * MT + j) * 64 + lane) * 4]) = acc[j];
   __syncthreads();
-  // tile (i, j): features f0 + 16 i + 4 h + 0..3 of token t0 + 16 j + col; the waves take the tiles in turn
+  // tile j: features f0 + 4 h + 0..3 of token t0 + 16 j + col; one wave each
 #pragma unroll
-  for (int tile = 0; tile < NT * MT; ++tile) {
-    if (tile % NW != w) continue;
-    const int i = tile / MT, j = tile % MT;
+  for (int j = 0; j < MT; ++j) {
+    if (j != w) continue;
     f32x4 v = (f32x4)(0.f);
 #pragma unroll
-    for (int u = 0; u < NW; ++u) v += *reinterpret_cast<const f32x4*>(&part[((u * NT * MT + tile) * 64 + lane) * 4]);
-    const int t = t0 + 16 * j + col, n = f0 + 16 * i + 4 * h;
+    for (int u = 0; u < NW; ++u) v += *reinterpret_cast<const f32x4*>(&part[((u * MT + j) * 64 + lane) * 4]);
+    const int t = t0 + 16 * j + col, n = f0 + 4 * h;
     if (t >= P.M) continue;
     if constexpr (EPI == 1) {
       *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(P.out) + ((int64_t)ks * P.M + t) * P.N + n) = v;
@@ -94,7 +82,7 @@ __global__ void __launch_bounds__(512) row_gemm_kernel(RowGemmParams P) {
       u16x4 o;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float y = v[r] + (P.bias ? bf2f(P.bias[n + r]) : 0.f);
+        const float y = v[r] + bf2f(P.bias[n + r]);
         o[r] = f2bf(EPI == 2 ? gr_gelu(y) : y);
       }
       *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + (int64_t)t * P.ldo + n) = o;
