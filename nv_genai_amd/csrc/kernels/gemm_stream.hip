@@ -156,8 +156,9 @@ static int64_t st_tiles(int64_t N, bool swiglu) { return swiglu ? N / 8 : N / 16
 // Whether this kernel is the fastest of those here for a projection (N = F with SwiGLU). Up to K = 4,096 it is for 2 to 16 rows,
 // measured against what took them before over all projections of the presets with 1 to 8 ranks. gemv.hip, which splits rows of
 // any count evenly over the CUs, is faster where the tiles do not come out even: for one row between 256 and 512 tiles and above
-// (6,144 rows of 1,536 / 3,072: 5.5 / 8.8 us, here 5.8 / 9.5; with the rotation behind it 6,144 x 4,096 13.6, here 14.6; at 256 and
-// 512 tiles this one: 4,096 x 4,096 9.3 and 7.9, 8,192 x 4,096 14.0 and 13.3), and for two rows of SwiGLU between 512 and 768
+// (6,144 rows of 1,536 / 3,072: 5.5 / 8.8 us, here 5.8 / 9.5; at 256 and 512 tiles this one: 4,096 x 4,096 9.3 and 7.9, 8,192 x
+// 4,096 14.0 and 13.3; up to 448 tiles of 4,096 values too: 6,144 x 4,096 10.8 and 10.7, in a decode step 10.8 and 9.9; 7,680 12.8
+// and 13.2), and for two rows of SwiGLU between 512 and 768
 // tiles of long rows (2 x 4,608 x 4,096: 16.9, here 18.5; of 2,048: 10.8, 10.9; 2 x 6,656 x 4,096: 22.9, 20.5). Longer rows of 16
 // tokens at once keep the L2 busier than HBM: up to 256 tiles 8 rows still gain (above, and 1,280 x 8,192 at 1 / 4 / 8 rows with
 // the rotation 14.8 17.9 18.1 from the table's slabs, here 13.1 14.2 15.8), beyond the others are level (8,192 x 8,192 at 4 rows:
@@ -168,7 +169,7 @@ bool stream_gemm_covers(int64_t M, int64_t N, int64_t K, bool swiglu) {
   const int64_t t = st_tiles(N, swiglu);
   if (K > 4096) return t <= 256 && M <= 8;
   if (swiglu && M == 2 && K > 2048 && t > 512 && t < 768) return false;
-  return M > 1 || t <= 256 || t == 512;
+  return M > 1 || t <= 256 || t == 512 || (!swiglu && K > 3072 && t <= 448);
 }
 
 // 32 rows a workgroup (half the token traffic) where 16 would give some CUs two workgroups and others one, or from 9 tokens on.
