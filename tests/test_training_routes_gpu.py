@@ -252,3 +252,42 @@ def test_models_reach_the_functions(gpu, monkeypatch, how, reached):
     _without(monkeypatch)
     run().backward()
     assert not called
+
+
+@pytest.mark.parametrize("how", ["llama", "checkpointed", "encoder"])
+def test_all_weight_gradients_keep_their_bits(gpu, monkeypatch, how):
+    """All weights trained, one step's loss and the gradients of matrices and embeddings are those of the torch operations to the
+    bit; those of norms' weights and of biases are sums over the rows in another order: in fp32 1e-5 for some hundred rows, and
+    biases, which round that sum to bf16, one step of it, 2^-8."""
+    from nv_genai_amd.models.config import encoder_config
+    from nv_genai_amd.models.encoder import EncoderModel
+
+    kind = "encoder" if how == "encoder" else "llama"
+    m = EncoderModel(encoder_config("encoder-tiny"), gpu, seed=2) if kind == "encoder" else _llama(gpu, "llama-small")
+    ids = torch.randint(0, 1000, (2, 129), device=gpu)
+    got = []
+    for fused_too in (True, False):
+        if not fused_too:
+            _without(monkeypatch)
+        P = Fn.trainable_params(m, kind)
+        with torch.autocast("cuda", dtype=BF):
+            if kind == "encoder":
+                loss = Fn.encoder_embed(m, ids, torch.ones_like(ids), P).pow(3).sum()
+            else:
+                loss = Fn.lm_loss(m, Fn.llama_hidden(m, ids, params=P, grad_ckpt=how == "checkpointed"), ids, params=P)
+        ks = sorted(P, key=str)
+        got.append((loss.detach(), dict(zip(ks, torch.autograd.grad(loss, [P[k] for k in ks], allow_unused=True)))))
+    (la, ga), (lb, gb) = got
+    assert torch.equal(la, lb)
+    for k, q in gb.items():
+        p, name = ga[k], k if isinstance(k, str) else k[1]
+        if q is None:
+            assert p is None
+        elif name.startswith("b"):   # the keys' bias has no gradient but rounding
+            H = m.cfg.hidden
+            p, q = (torch.cat([t[:H], t[2 * H:]]) if name == "bqkv" else t for t in (p, q))
+            assert _rel(p, q) < 4e-3, (k, _rel(p, q))
+        elif p.ndim == 1:
+            assert _rel(p, q) < 1e-5, (k, _rel(p, q))
+        else:
+            assert torch.equal(p, q), (k, _rel(p, q))
