@@ -1,6 +1,6 @@
 """Micro-benchmarks of the hand-written hot kernels at serving shapes (Llama-3-8B):
 prefill attention (paged, causal, GQA 32/8, D=128), decode attention, sampling, and the
-1M x 1024 flat-index search (MFMA scoring + radix top-k)."""
+1M x 1024 searches: an index's whole search (flat, lists), and the scoring, selection and fused kernels by themselves."""
 import json
 import os
 import sys
@@ -125,15 +125,21 @@ def main():
         N, Dx = 1_000_000, 1024
         X = torch.nn.functional.normalize(torch.randn(N, Dx, device=dev), dim=1).to(torch.bfloat16)
         bias = torch.zeros(N, device=dev)
-        for nq in (1, 8, 64):
-            Q = torch.nn.functional.normalize(torch.randn(nq, Dx, device=dev), dim=1).to(torch.bfloat16)
+        ids = torch.arange(N, device=dev)
+        for nq in (1, 8, 64, 512):
+            q32 = torch.randn(nq, Dx, device=dev)
+            Q = torch.nn.functional.normalize(q32, dim=1).to(torch.bfloat16)
+            us_w = timeit(lambda: ops.flat_search(q32, X, bias, ids, "cosine", 4))   # an index's whole search,
+            many = ops.search_many(nq, N, Dx, 4)                                     # unless it leaves it to search_topk
             us = timeit(lambda: ops.score(Q, X, None, 1.0))
             us_all = timeit(lambda: ops.topk(ops.score(Q, X, None, 1.0), 4))
             us_f = timeit(lambda: ops.search_topk(Q, X, bias, 1.0, 4))
             ops.kernels().set_kernel_form("search_dma", 0)    # the register-load form
             us_reg = timeit(lambda: ops.search_topk(Q, X, bias, 1.0, 4))
             ops.kernels().set_kernel_form("search_dma", 1)
-            out[f"search_1Mx1024_q{nq}"] = {"reg_us": round(us_reg, 1),
+            out[f"search_1Mx1024_q{nq}"] = {"index_us": round(us_w, 1), "index_TBps": round(N * Dx * 2 / us_w / 1e6, 2),
+                                             "index_takes_search_topk": many,
+                                             "reg_us": round(us_reg, 1),
                                              "reg_TBps": round(N * Dx * 2 / us_reg / 1e6, 2),
                                              "score_us": round(us, 1), "score_TBps": round(N * Dx * 2 / us / 1e6, 2),
                                              "score_topk_us": round(us_all, 1),
@@ -146,11 +152,13 @@ def main():
         bs = torch.zeros(Xs.shape[0], device=dev)
         for nq in (8, 64):
             Q = torch.nn.functional.normalize(torch.randn(nq, Dx, device=dev), dim=1).to(torch.bfloat16)
+            q32, xid = Q.float(), torch.arange(Xs.shape[0], device=dev)
+            us_w = timeit(lambda: ops.flat_search(q32, Xs, bs, xid, "cosine", 4))
             us_f = timeit(lambda: ops.search_topk(Q, Xs, bs, 1.0, 4))
             ops.kernels().set_kernel_form("search_dma", 0)
             us_reg = timeit(lambda: ops.search_topk(Q, Xs, bs, 1.0, 4))
             ops.kernels().set_kernel_form("search_dma", 1)
-            out[f"search_shard1.25Mx1024_q{nq}"] = {"reg_us": round(us_reg, 1), "fused_us": round(us_f, 1),
+            out[f"search_shard1.25Mx1024_q{nq}"] = {"index_us": round(us_w, 1), "reg_us": round(us_reg, 1), "fused_us": round(us_f, 1),
                                                     "fused_TBps": round(Xs.numel() * 2 / us_f / 1e6, 2)}
         del Xs, bs
         # IVF-Flat, the reference's GPU_IVF_FLAT nlist 64 / nprobe 16 over 1M vectors
@@ -162,10 +170,7 @@ def main():
         for nq in (1, 8, 64):
             Q = torch.nn.functional.normalize(torch.randn(nq, Dx, device=dev), dim=1)
             us_i = timeit(lambda: ivf.search(Q, 4))
-            ops.kernels().set_kernel_form("search_dma", 0)
-            us_ir = timeit(lambda: ivf.search(Q, 4))
-            ops.kernels().set_kernel_form("search_dma", 1)
-            out[f"ivf_1Mx1024_nlist64_nprobe16_q{nq}"] = {"us": round(us_i, 1), "reg_us": round(us_ir, 1)}
+            out[f"ivf_1Mx1024_nlist64_nprobe16_q{nq}"] = {"us": round(us_i, 1)}
         del ivf
         del X
         if args.only == "search":

@@ -2,10 +2,10 @@
 // sums. Activations bf16, statistics, sums and weights' gradients fp32. Each takes the place of a chain of single
 // torch operations (a norm and its residual: 10 launches forward, 14 backward; a rotation: 14 each way).
 //
-// Steps marked "as written" round where that chain rounds, in its order, without contraction: their results are its bits, so
-// training goes on as it did (bf16 rounding decides on, and one other bit in an activation is an independent rounding error of
-// the whole gradient a few layers later). The means and sums over a row that such a step needs are left to
-// torch, whose order of summation is its own.
+// Steps marked "as written" round where that chain rounds, in its order, without contraction: their results are its bits (one
+// other bit in an activation is an independent rounding error of the whole gradient a few layers later). The means and sums
+// over a row that such a step needs are left to torch, whose order of summation is its own. Column sums, the gradients of
+// norms' weights and biases, are in this file's order, and so within fp32 rounding of torch's.
 #include "common.h"
 #include "kernels.h"
 

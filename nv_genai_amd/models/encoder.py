@@ -7,7 +7,7 @@ Triton MiniLM config of the reference pads every batch to 512
 (experimental/streaming_ingest_rag/docker/extras/all-MiniLM-L6-v2_config.pbtxt:1-45).
 Per layer (post-LN BERT):
     qkv = x @ Wqkv^T + b                      hipBLASLt (bias fused in addmm)
-    a   = varlen MFMA attention, no mask      K10 (attention_prefill.hip, non-paged)
+    a   = varlen MFMA attention, no mask      K10 (attention_varlen.hip)
     x   = LN(a @ Wo^T + bo + x)               K11 (residual fused into the LN kernel)
     h   = gelu(x @ Wi^T + bi)                 K11 (bias+GELU kernel)
     x   = LN(h @ Wo2^T + bo2 + x)

@@ -9,9 +9,11 @@ autograd on padded ``[B, S]`` batches:
   of PyTorch-ROCm), causal for the LLM, key-padding-masked for the encoder; with adapters
   the framework's own kernel gives the flash attention's gradients on the GPU;
 * on the GPU norms with their residual, activations, rotation and cross entropy through the functions of
-  :mod:`.fused`, elsewhere and for what those do not take through torch operations. All weights trained, they
-  keep every bit of the torch operations' activations and gradients (full fine-tuning goes on as it did), with
-  adapters those of the activations, and the gradients take the forms that are a single pass;
+  :mod:`.fused`, elsewhere and for what those do not take through torch operations. All weights trained, a
+  step's loss and its gradients of matrices and embeddings are the torch operations' to the bit; the gradients of
+  norms' weights and biases, the clipping norm and AdamW's update are fp32 sums in another order, so that weights
+  differ by their last bits from the first step on. With adapters the activations keep their bits, and the
+  gradients take the forms that are a single pass;
 * RMSNorm / LayerNorm / softmax statistics in fp32.
 
 Parameters are taken from the serving model objects by reference (no copy), so a LoRA

@@ -2,8 +2,9 @@
 
 Each takes the place of a chain of single torch operations in :mod:`.functional` (forward and backward): activations bf16,
 statistics, sums and the gradients of weights fp32, weights either fp32 masters or bf16. Activations are bit for bit those of
-the chain. So are, all weights trained, their gradients; ``attention``, ``lora_linear`` and the ``once`` forms, for adapters,
-form them in the kernels' own order. Callers ask ``usable`` first; the torch operations stay for the CPU, other types and
+the chain. So are, all weights trained, their gradients and those of matrices; the gradients of norms' weights and of biases
+are fp32 sums over the rows in the kernels' own order. ``attention``, ``lora_linear`` and the ``once`` forms, for adapters, form
+the activations' gradients in that too. Callers ask ``usable`` first; the torch operations stay for the CPU, other types and
 sizes, and under transforms that pass functions of this kind by (tracing, functorch, forward-mode). Where a graph of the
 backward is asked for (create_graph) the gradients come from torch operations; ``attention``, like the flash attention that it
 stands for, has a first derivative only.

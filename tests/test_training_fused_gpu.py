@@ -222,7 +222,8 @@ def test_llama_hidden_matches_torch_operations(gpu, monkeypatch, name, S, how):
         # equal activations; the loss sums in another order, the gradients carry bf16 rounding through two to four layers
         ltol, tol = 1e-6, 3e-2
     else:
-        # equal bits, but for the fp32 sums of norms' weights and what torch adds up in no fixed order (attention's, embeddings')
+        # equal bits but for the fp32 sums of norms' weights (test_training_routes_gpu.py compares them); experts' rows are added
+        # up in no fixed order
         ltol, tol = 0.0, 4e-3
     assert abs(la.item() - lb.item()) <= ltol * abs(lb.item())
     for p, q in zip(ga, gb):
