@@ -752,6 +752,7 @@ void train_attention_backward(Tensor dq, Tensor dk, Tensor dv, Tensor dout, Tens
   p.dq = bfp(dq); p.dk = bfp(dk); p.dv = bfp(dv); p.dq_stride = dq.stride(0); p.dkv_stride = dk.stride(0);
   p.cu = cu.data_ptr<int32_t>(); p.T = T; p.Hq = (int)Hq; p.Hkv = (int)Hkv; p.scale = (float)scale;
   nga::launch_varlen_attention_backward(p, (int)B, (int)max_len, (int)D, cur_stream(q));
+  post_launch("train_attention_backward");
 }
 
 // ------------------------------------------------------------------ training steps (train.hip)
@@ -1673,6 +1674,17 @@ std::function<void(A...)> checked(const char* name, void (*f)(A...)) {
   };
 }
 
+// A training step stands between torch operations, which run on their tensors' GPU whichever is the current one: so does f
+inline c10::Device first_device(const Tensor& t) { return t.device(); }
+inline c10::Device first_device(const std::vector<Tensor>& t) { return t.empty() ? c10::Device(at::kCPU) : t[0].device(); }
+
+template <typename R, typename T, typename... A>
+std::function<R(T, A...)> on_device(R (*f)(T, A...)) {
+  return [f](T t, A... a) -> R {
+    const c10::DeviceGuard guard(first_device(t));
+    return f(std::forward<T>(t), std::forward<A>(a)...);
+  };
+}
 
 // ------------------------------------------------------------------ post-norm fp32 residual / sigmoid attention
 // activations are bf16 or fp32 (one type per call); residual, norm weights and state are fp32
@@ -2712,23 +2724,23 @@ PYBIND11_MODULE(_C, m) {
   m.def("encoder_covers", [](const Tensor& word, const std::vector<Tensor>& tables, const std::vector<Tensor>& L, int64_t heads) {
     return encoder_refuses(word, tables, L, heads) == nullptr;
   });
-  m.def("rms_sq", &rms_sq);
-  m.def("rms_apply", &rms_apply);
-  m.def("rms_prod", &rms_prod);
-  m.def("rms_dx", &rms_dx);
-  m.def("rms_bwd", &rms_bwd);
-  m.def("add_f32", &add_f32);
-  m.def("ln_sums", &ln_sums);
-  m.def("gelu_rows", &gelu_rows);
-  m.def("col_sums", &col_sums);
-  m.def("swiglu_rows", &swiglu_rows);
-  m.def("add_scaled", &add_scaled);
-  m.def("rope_rows", &rope_rows);
-  m.def("ce_fwd", &ce_fwd);
-  m.def("ce_bwd", &ce_bwd);
-  m.def("grad_norm", &grad_norm);
-  m.def("adamw", &adamw);
-  m.def("train_attention_backward", checked("train_attention_backward", &train_attention_backward));
+  m.def("rms_sq", on_device(&rms_sq));
+  m.def("rms_apply", on_device(&rms_apply));
+  m.def("rms_prod", on_device(&rms_prod));
+  m.def("rms_dx", on_device(&rms_dx));
+  m.def("rms_bwd", on_device(&rms_bwd));
+  m.def("add_f32", on_device(&add_f32));
+  m.def("ln_sums", on_device(&ln_sums));
+  m.def("gelu_rows", on_device(&gelu_rows));
+  m.def("col_sums", on_device(&col_sums));
+  m.def("swiglu_rows", on_device(&swiglu_rows));
+  m.def("add_scaled", on_device(&add_scaled));
+  m.def("rope_rows", on_device(&rope_rows));
+  m.def("ce_fwd", on_device(&ce_fwd));
+  m.def("ce_bwd", on_device(&ce_bwd));
+  m.def("grad_norm", on_device(&grad_norm));
+  m.def("adamw", on_device(&adamw));
+  m.def("train_attention_backward", on_device(&train_attention_backward));
   m.def("flat_search", &flat_search);
   m.def("ivf_search", &ivf_search);
   m.def("search_covers", [](int64_t d) { return d <= 1024 && nga::scan_chunk((int)d, 1) > 0; });

@@ -291,3 +291,22 @@ def test_all_weight_gradients_keep_their_bits(gpu, monkeypatch, how):
             assert _rel(p, q) < 1e-5, (k, _rel(p, q))
         else:
             assert torch.equal(p, q), (k, _rel(p, q))
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="two GPUs")
+def test_a_gpu_that_is_not_the_current_one(gpu):
+    """Weights, rows and optimiser on the second GPU, the first the current one: as torch's operations run there."""
+    from nv_genai_amd.training.optim import AdamW
+
+    got = []
+    for dev in (gpu, torch.device("cuda:1")):
+        torch.manual_seed(0)
+        w = {n: (0.1 * torch.randn(s)).to(dev).requires_grad_() for n, s in dict(n=(256,), i=(1024, 256), b=(1024,), o=(256, 512)).items()}
+        x, y = torch.randn(48, 256).to(BF).to(dev), torch.randint(0, 256, (48,)).to(dev)
+        opt = AdamW(list(w.values()), lr=0.1)
+        h = fused.swiglu(fused.linear(fused.rms_norm(x, w["n"], 1e-5), w["i"], w["b"]))
+        fused.cross_entropy_sum(h @ w["o"].to(BF).t(), y, True).backward()
+        assert opt._covers() and torch.cuda.current_device() == 0
+        opt.step(max_norm=1.0)
+        got.append([t.detach().cpu() for t in w.values()])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
