@@ -586,6 +586,56 @@ void decode_attention(Tensor out, Tensor q, Tensor kc, Tensor vc, Tensor block_t
                                (float)k_scale, (float)v_scale, cur_stream(q), skip_empty);
 }
 
+// Attention of a decode step: q | k | v of one new token a row (bf16 [B, (Hq + 2 Hkv) 128], or fp32 K-split slabs [S, B, ..])
+// are rotated, written to the cache at `slots` (the slots of places ctx - 1; -1: not written) and attended to. `done` int32
+// zeros [>= B Hkv], given back as zeros.
+void decode_step(Tensor out, Tensor qkv, Tensor pos, Tensor cos_sin, Tensor slots, Tensor kc, Tensor vc, Tensor block_tables,
+                 Tensor ctx_lens, int64_t Hq, int64_t Hkv, int64_t max_ctx, double scale, int64_t pages_per_part,
+                 Tensor part_ml, Tensor part_o, Tensor done, int64_t window) {
+  CHECK_BF16(out); CHECK_BF16(kc); CHECK_BF16(vc);
+  CHECK_DEV(qkv); CHECK_CONTIG(qkv); CHECK_CONTIG(kc); CHECK_CONTIG(vc);
+  CHECK_DEV(pos); CHECK_DT(pos, at::kInt); CHECK_CONTIG(pos);
+  CHECK_DEV(slots); CHECK_DT(slots, at::kInt); CHECK_CONTIG(slots);
+  CHECK_DEV(cos_sin); CHECK_DT(cos_sin, at::kFloat); CHECK_CONTIG(cos_sin);
+  CHECK_DEV(block_tables); CHECK_DT(block_tables, at::kInt); CHECK_CONTIG(block_tables);
+  CHECK_DEV(ctx_lens); CHECK_DT(ctx_lens, at::kInt); CHECK_CONTIG(ctx_lens);
+  CHECK_DEV(done); CHECK_DT(done, at::kInt); CHECK_CONTIG(done);
+  const int64_t B = ctx_lens.numel(), D = 128, row = (Hq + 2 * Hkv) * D;
+  const bool slabs = qkv.dim() == 3;
+  TORCH_CHECK(Hkv > 0 && Hq % Hkv == 0 && Hq / Hkv >= 1 && Hq / Hkv <= 16, "decode_step: G = Hq/Hkv must be 1 to 16");
+  TORCH_CHECK(kc.dim() == 4 && kc.size(1) == Hkv && kc.size(2) == 64 && kc.size(3) == D, "decode_step: k cache must be [nb, Hkv, 64, 128]");
+  TORCH_CHECK(vc.sizes() == at::IntArrayRef({kc.size(0), Hkv, D, 64}), "decode_step: v cache must be [nb, Hkv, 128, 64]");
+  TORCH_CHECK(slabs ? qkv.scalar_type() == at::kFloat && qkv.size(0) >= 1 : qkv.dim() == 2 && qkv.scalar_type() == at::kBFloat16,
+              "decode_step: qkv bf16 [B, row] or fp32 slabs [S, B, row]");
+  TORCH_CHECK(qkv.size(-2) == B && qkv.size(-1) == row && reinterpret_cast<uintptr_t>(qkv.data_ptr()) % 16 == 0,
+              "decode_step: qkv must hold (Hq + 2 Hkv) x 128 values a row at 16-byte addresses");
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(cos_sin.data_ptr()) % 16 == 0 && cos_sin.dim() == 2 && cos_sin.size(1) == D,
+              "decode_step: cos_sin must be [positions, 128]");
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == B && out.size(1) == Hq * D && out.stride(1) == 1, "decode_step: out [B, Hq * 128]");
+  TORCH_CHECK(pos.numel() == B && slots.numel() == B && done.numel() >= B * Hkv, "decode_step: a position, a slot and Hkv counters a row");
+  TORCH_CHECK(block_tables.dim() == 2 && block_tables.size(0) >= B && block_tables.size(1) * 64 >= max_ctx,
+              "decode_step: block table too narrow for max_ctx");
+  TORCH_CHECK(window >= 0 && pages_per_part >= 1 && nga::decode_step_covers((int)B, (int)max_ctx, (int)pages_per_part, (int)window),
+              "decode_step: not covered");
+  const int64_t nparts = ((max_ctx + 63) / 64 + pages_per_part - 1) / pages_per_part;
+  if (nparts > 1) {
+    CHECK_DEV(part_ml); CHECK_DEV(part_o);
+    TORCH_CHECK(part_ml.numel() >= B * Hq * nparts * 2 && part_o.numel() >= B * Hq * nparts * D, "decode_step: partition workspace too small");
+  }
+  nga::DecodeStep st{};
+  if (slabs) { st.part = qkv.data_ptr<float>(); st.S = (int)qkv.size(0); st.slab = B * row; }
+  st.pos = pos.data_ptr<int32_t>();
+  st.cos_sin = cos_sin.data_ptr<float>();
+  st.slots = slots.data_ptr<int32_t>();
+  st.kc = bfp(kc);
+  st.vc = bfp(vc);
+  st.done = done.data_ptr<int32_t>();
+  nga::launch_decode_step(bfp(out), out.stride(0), slabs ? nullptr : bfp(qkv), st, block_tables.data_ptr<int32_t>(),
+                          (int)block_tables.size(1), ctx_lens.data_ptr<int32_t>(), (int)B, (int)Hq, (int)Hkv, (int)max_ctx,
+                          (float)scale, (int)pages_per_part, nparts > 1 ? part_ml.data_ptr<float>() : nullptr,
+                          nparts > 1 ? part_o.data_ptr<float>() : nullptr, (int)window, cur_stream(qkv));
+}
+
 // Work-list prefill (32x32 kernel): q / out rows are absolute token rows of the step (the
 // cu_q offsets of ALL its sequences); items [n, 2] int32 (sequence, row block) pairs, n_items
 // a 1-element device int32 (read by the kernel, so a captured graph replays any step's list)
@@ -2696,6 +2746,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("bias_gelu", checked("bias_gelu", &bias_gelu));
   m.def("rope_cache", checked("rope_cache", &rope_cache));
   m.def("decode_pages_per_part", &decode_pages_per_part);
+  m.def("decode_step", checked("decode_step", &decode_step));
+  m.def("decode_step_covers", &nga::decode_step_covers);
   m.def("decode_attention", checked("decode_attention", &decode_attention));
   m.def("prefill_attention", checked("prefill_attention", &prefill_attention));
   m.def("prefill_attention_worklist", checked("prefill_attention_worklist", &prefill_attention_worklist));

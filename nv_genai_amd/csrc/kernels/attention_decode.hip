@@ -306,31 +306,56 @@ __device__ __forceinline__ int dvswz(int row) { return (row >> 1) & 7; }
 // 64-B halves and ran at 4.7 TB/s against 6.7.)
 // AUX: cache policy of the KV-page DMA loads (form decode_dma_aux): 2 = nt (each page is read
 // once per step), 0 = default policy
-template <bool RING, int AUX>
+// Values that workgroups of one launch hand over
+__device__ __forceinline__ void put_agent(float* p, float v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float get_agent(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// STEP = true: the whole attention of a decode step in this one launch. The workgroup takes its
+// query rows from the projection's output (bf16, or its fp32 K-split slabs) and rotates them; the
+// one whose partition ends the sequence rotates the new key too, lays the new key and value over
+// their places in the page it has just read (the page's DMA does not wait for them) and writes
+// them to the cache at the end; and the partition that finishes last adds all of a sequence's
+// partitions up. Each of the three kernels that this replaces cost 4.6 us a layer in a captured
+// step, nearly all of it launch, first-byte latency and drain (8B, one sequence of 227 tokens:
+// rotation 4.6, attention 7.2, sum of the partitions 4.6; here 8.6. 16 sequences of some 800: 5.1, 14.3, 4.6; here 18.4).
+template <bool RING, int AUX, bool STEP>
 __global__ void __launch_bounds__(256, 1) decode_attn_dma_kernel(
     uint16_t* __restrict__ out, int64_t out_stride, const uint16_t* __restrict__ q,
     int64_t q_stride, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const int32_t* __restrict__ block_tables, int max_blocks,
     const int32_t* __restrict__ ctx_lens, int Hq, int Hkv, float scale,
-    float* __restrict__ part_ml, float* __restrict__ part_o, int window, int skip_empty) {
+    float* __restrict__ part_ml, float* __restrict__ part_o, int window, int skip_empty, DecodeStep st) {
+  static_assert(RING || !STEP, "a step runs the ring");
   constexpr int D = 128, DS = 4, DT = 8;
   // ONE LDS object (a second one makes the compiler drain the DMA before fragment reads):
-  // the waves' page slots, reused by the wave combine after the loop
-  __shared__ __attribute__((aligned(16))) uint16_t smem[NW * DSLOT + 2 * DMA_MAX_PAGES];
+  // the waves' page slots, reused by the wave combine after the loop; a step's query rows, its
+  // new key and value
+  constexpr int QS = NW * DSLOT + 2 * DMA_MAX_PAGES;
+  __shared__ __attribute__((aligned(16))) uint16_t smem[QS + (STEP ? 18 * D : 0)];
   const int b = blockIdx.x, kvh = blockIdx.y, part = blockIdx.z, nparts = gridDim.z;
   const int G = Hq / Hkv;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int col = lane & 15, h = lane >> 4;
   const int ctx = ctx_lens[b];
+  const int step_pos = STEP ? st.pos[b] : 0, slot = STEP ? st.slots[b] : -1;
   const int n_pages = (ctx + BS - 1) / BS;
   const int key_lo = window > 0 ? max(0, ctx - window) : 0;
   const int p_lo = key_lo / BS;
   const int ppp = max(NW, (n_pages - p_lo + nparts - 1) / nparts);
   const int p_begin = p_lo + part * ppp;
   const int p_end = min(n_pages, p_begin + ppp);
+  const int active = STEP ? (n_pages - p_lo + ppp - 1) / ppp : nparts;   // partitions with pages
   if (p_begin >= p_end) {   // as decode_attn_kernel
     if (skip_empty && ctx == 0) return;
-    if (nparts == 1) {
+    if constexpr (STEP) {   // nobody adds an empty partition up; a row without a context is zero
+      if (active == 0 && part == 0)
+        for (int i = threadIdx.x; i < G * D; i += blockDim.x)
+          out[(int64_t)b * out_stride + (int64_t)(kvh * G) * D + i] = 0;
+    } else if (nparts == 1) {
       for (int i = threadIdx.x; i < G * D; i += blockDim.x)
         out[(int64_t)b * out_stride + (int64_t)(kvh * G) * D + i] = 0;
     } else {
@@ -375,7 +400,53 @@ __global__ void __launch_bounds__(256, 1) decode_attn_dma_kernel(
   // the partition's block ids in LDS: a VMEM block-id load in the loop would be sunk past the
   // page wait by the compiler and then waited for on its own before every next-page DMA
   int32_t* const sbt = reinterpret_cast<int32_t*>(smem + NW * DSLOT);
-  for (int i = threadIdx.x; i < p_end - p_begin; i += blockDim.x) sbt[i] = bt[p_begin + i];
+  const bool last = STEP && p_end == n_pages && slot >= 0;
+  if constexpr (STEP) {
+    // rows to rotate: 0 .. G - 1 query heads, G the new key, G + 1 the new value (as it is), eight values of each half a
+    // thread. All loads are asked for before any is used: one latency, and the pages' DMA behind it
+    const int n = p_end - p_begin, r = threadIdx.x >> 3, at = (threadIdx.x & 7) * 8;
+    const int32_t id = bt[p_begin + min((int)threadIdx.x, n - 1)];
+    const int row = min(r, G + 1), head = row < G ? kvh * G + row : row == G ? Hq + kvh : Hq + Hkv + kvh;
+    const int64_t xi = ((int64_t)b * (Hq + 2 * Hkv) + head) * D + at;
+    const float* cs = st.cos_sin + (int64_t)step_pos * D + at;
+    f32x4 v[4], c[4];   // the first slab's values, or bf16 ones in v[0] and v[2]
+    if (st.part != nullptr) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const f32x4*>(st.part + xi + (j >> 1) * (D / 2) + (j & 1) * 4);
+    } else {
+      v[0] = *reinterpret_cast<const f32x4*>(q + xi);
+      v[2] = *reinterpret_cast<const f32x4*>(q + xi + D / 2);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c[j] = *reinterpret_cast<const f32x4*>(cs + (j >> 1) * (D / 2) + (j & 1) * 4);
+    if ((int)threadIdx.x < n) sbt[threadIdx.x] = id;
+    for (int i = threadIdx.x + 256; i < n; i += 256) sbt[i] = bt[p_begin + i];
+    u16x8 x[2];
+    if (st.part != nullptr) {
+      for (int s = 1; s < st.S; ++s)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] += *reinterpret_cast<const f32x4*>(st.part + s * st.slab + xi + (j >> 1) * (D / 2) + (j & 1) * 4);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) x[j >> 3][j & 7] = f2bf(v[j >> 2][j & 3]);
+    } else {
+      x[0] = __builtin_bit_cast(u16x8, v[0]);
+      x[1] = __builtin_bit_cast(u16x8, v[2]);
+    }
+    if (row <= G)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float x1 = bf2f(x[0][j]), x2 = bf2f(x[1][j]), co = c[j >> 2][j & 3], si = c[2 + (j >> 2)][j & 3];
+        x[0][j] = f2bf(x1 * co - x2 * si);
+        x[1][j] = f2bf(x2 * co + x1 * si);
+      }
+    if (r < G + 2) {
+      uint16_t* to = smem + QS + (r < G ? r : 16 + r - G) * D + at;
+      store8(to, x[0]);
+      store8(to + D / 2, x[1]);
+    }
+  } else {
+    for (int i = threadIdx.x; i < p_end - p_begin; i += blockDim.x) sbt[i] = bt[p_begin + i];
+  }
   __syncthreads();
   if constexpr (RING) {
     // the slot as a ring of two 16-KiB DMA units, the wave's page k's K (buffer ks) and V^T
@@ -401,21 +472,24 @@ __global__ void __launch_bounds__(256, 1) decode_attn_dma_kernel(
                                          (lptr_t)(vs + i * 512), 16, 0, AUX);
       }
     };
-    if (my_pages > 0) {
-      issue_k(blk_of(0));
-      issue_v(blk_of(0));
-    }
     bf16x8 qf[DS];
-    {
+    auto load_q = [&] {
       const bool qv = col < G;
-      const uint16_t* qp = q + (int64_t)b * q_stride + (int64_t)(kvh * G + (qv ? col : 0)) * D;
+      const uint16_t* qp = STEP ? smem + QS + (qv ? col : 0) * D
+                                : q + (int64_t)b * q_stride + (int64_t)(kvh * G + (qv ? col : 0)) * D;
 #pragma unroll
       for (int s = 0; s < DS; ++s) {
         u16x8 v = load8(qp + 32 * s + 8 * h);
         if (!qv) v = (u16x8)(0);
         qf[s] = as_bf16x8(v);
       }
+    };
+    if constexpr (STEP) load_q();   // from LDS: after the DMAs' start they would wait for those
+    if (my_pages > 0) {
+      issue_k(blk_of(0));
+      issue_v(blk_of(0));
     }
+    if constexpr (!STEP) load_q();
     // Q is consumed here, so the compiler's wait for it (a full vmcnt drain beside the DMAs)
     // lands before the loop and not inside it
 #pragma unroll
@@ -423,6 +497,10 @@ __global__ void __launch_bounds__(256, 1) decode_attn_dma_kernel(
     for (int k = 0; k < my_pages; ++k) {
       const bool more = k + 1 < my_pages;
       asm volatile("s_waitcnt vmcnt(16)" ::: "memory");   // K(k) landed (V(k) may not have)
+      const bool fresh = STEP && last && p_begin + w + NW * k == n_pages - 1;   // the page of the new token
+      const int new_key = (ctx - 1) % BS;
+      if (fresh && lane < 16)   // a wave's LDS accesses keep their order
+        store8(ks + new_key * D + ((lane ^ dkswz(new_key)) << 3), load8(smem + QS + 16 * D + 8 * lane));
       u16x8 kf[4][DS];
 #pragma unroll
       for (int ti = 0; ti < 4; ++ti) {
@@ -483,6 +561,12 @@ __global__ void __launch_bounds__(256, 1) decode_attn_dma_kernel(
       // V(k) landed: K(k+1), if issued, is the only younger DMA
       if (more) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (fresh)
+#pragma unroll
+        for (int i = 0; i < D; i += 64) {
+          const int d = i + lane;
+          vs[d * BS + (((new_key >> 3) ^ dvswz(d)) << 3) + (new_key & 7)] = smem[QS + 17 * D + d];
+        }
       u16x8 vf[2][DT];
 #pragma unroll
       for (int g = 0; g < 2; ++g)
@@ -617,15 +701,67 @@ __global__ void __launch_bounds__(256, 1) decode_attn_dma_kernel(
       acc += f * o_s[(ww * 16 + qi) * (D + 4) + d];
     }
     const int hq = kvh * G + qi;
-    if (nparts == 1) {
+    if (active == 1) {
       out[(int64_t)b * out_stride + (int64_t)hq * D + d] = f2bf(L > 0.f ? acc / L : 0.f);
     } else {
       const int64_t idx = ((int64_t)b * Hq + hq) * nparts + part;
-      part_o[idx * D + d] = acc;
-      if (d == 0) {
-        part_ml[2 * idx] = M;
-        part_ml[2 * idx + 1] = L;
+      if constexpr (STEP) {   // read by a workgroup of this launch, maybe of another die
+        put_agent(part_o + idx * D + d, acc);
+        if (d == 0) {
+          put_agent(part_ml + 2 * idx, M);
+          put_agent(part_ml + 2 * idx + 1, L);
+        }
+      } else {
+        part_o[idx * D + d] = acc;
+        if (d == 0) {
+          part_ml[2 * idx] = M;
+          part_ml[2 * idx + 1] = L;
+        }
       }
+    }
+  }
+  if constexpr (STEP) {
+    if (last && threadIdx.x < D) {
+      const int64_t page = ((int64_t)(slot / BS) * Hkv + kvh) * (BS * D);
+      const int off = slot % BS, d = threadIdx.x;
+      st.kc[page + (int64_t)off * D + d] = smem[QS + 16 * D + d];
+      __builtin_nontemporal_store(smem[QS + 17 * D + d], st.vc + page + (int64_t)d * BS + off);
+    }
+    if (active == 1) return;
+    // Every wave waits until its sums have reached memory, then its workgroup is counted. Nobody waits for another: whoever
+    // counts last does the rest. Sums and counter are accessed past the dies' L2s; with ordinary stores and fences, each
+    // workgroup wrote its die's whole L2 back and emptied it (16 rows of 800 tokens in two partitions: 28.7 us, so 19.6)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int32_t* const done = reinterpret_cast<int32_t*>(smem);
+    int32_t* const count = st.done + b * Hkv + kvh;
+    if (threadIdx.x == 0) *done = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == active - 1;
+    __syncthreads();
+    if (!*done) return;
+    if (threadIdx.x == 0) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = threadIdx.x; i < G * D; i += blockDim.x) {
+      const int64_t idx = ((int64_t)b * Hq + kvh * G + i / D) * nparts;
+      const int d = i % D;
+      float M = -INFINITY, L = 0.f, acc = 0.f;
+      for (int p0 = 0; p0 < active; p0 += 4) {   // four partitions' loads in flight
+        float m4[4], l4[4], v4[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int64_t at = idx + min(p0 + j, active - 1);
+          m4[j] = get_agent(part_ml + 2 * at);
+          l4[j] = get_agent(part_ml + 2 * at + 1);
+          v4[j] = get_agent(part_o + at * D + d);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (p0 + j >= active || m4[j] == -INFINITY) continue;   // nothing seen: its sums are 0
+          const float m = fmaxf(M, m4[j]), f = exp2f(M - m), g = exp2f(m4[j] - m);   // 2^-inf = 0
+          L = f * L + g * l4[j];
+          acc = f * acc + g * v4[j];
+          M = m;
+        }
+      }
+      out[(int64_t)b * out_stride + (int64_t)(kvh * G) * D + i] = f2bf(L > 0.f ? acc / L : 0.f);
     }
   }
 }
@@ -734,9 +870,9 @@ void launch_decode_attention(uint16_t* out, int64_t out_stride, const uint16_t* 
     if (kv_fp8) NGA_DEC(128, uint8_t);
     else if (dma && (pages + nparts - 1) / nparts <= DMA_MAX_PAGES) {
 #define NGA_DMA(RING, AUX)                                                                                   \
-  decode_attn_dma_kernel<RING, AUX><<<grid, 256, 0, stream>>>(                                              \
+  decode_attn_dma_kernel<RING, AUX, false><<<grid, 256, 0, stream>>>(                                       \
       out, out_stride, q, q_stride, static_cast<const uint16_t*>(kc), static_cast<const uint16_t*>(vc), \
-      block_tables, max_blocks, ctx_lens, Hq, Hkv, sc, part_ml, part_o, window, skip_empty ? 1 : 0)
+      block_tables, max_blocks, ctx_lens, Hq, Hkv, sc, part_ml, part_o, window, skip_empty ? 1 : 0, DecodeStep{})
       const bool cached = kernel_form(KF_DECODE_DMA_AUX) == 0;
       if (dma == 2) {
         if (cached) NGA_DMA(true, 0); else NGA_DMA(true, 2);
@@ -750,6 +886,29 @@ void launch_decode_attention(uint16_t* out, int64_t out_stride, const uint16_t* 
                                                              ctx_lens, skip_empty ? 1 : 0);
   }
 #undef NGA_DEC
+}
+
+// The page DMA's form for bf16 pages of head_dim 128 (`decode_dma` 2), up to 1,024 pages a partition.
+bool decode_step_covers(int num_seqs, int max_ctx, int pages_per_part, int window) {
+  int pages = (max_ctx + BS - 1) / BS;
+  if (window > 0) pages = min(pages, (window + BS - 1) / BS + 1);
+  const int nparts = (pages + pages_per_part - 1) / pages_per_part;
+  return num_seqs > 0 && kernel_form(KF_DECODE_DMA) == 2 && (pages + nparts - 1) / nparts <= DMA_MAX_PAGES;
+}
+
+void launch_decode_step(uint16_t* out, int64_t out_stride, const uint16_t* qkv, const DecodeStep& st,
+                        const int32_t* block_tables, int max_blocks, const int32_t* ctx_lens, int num_seqs, int Hq,
+                        int Hkv, int max_ctx, float scale, int pages_per_part, float* part_ml, float* part_o,
+                        int window, hipStream_t stream) {
+  int pages = (max_ctx + BS - 1) / BS;
+  if (window > 0) pages = min(pages, (window + BS - 1) / BS + 1);
+  const dim3 grid(num_seqs, Hkv, (pages + pages_per_part - 1) / pages_per_part);
+#define NGA_STEP(AUX)                                                                                          \
+  decode_attn_dma_kernel<true, AUX, true><<<grid, 256, 0, stream>>>(                                          \
+      out, out_stride, qkv, 0, st.kc, st.vc, block_tables, max_blocks, ctx_lens, Hq, Hkv, scale, part_ml, part_o, \
+      window, 0, st)
+  if (kernel_form(KF_DECODE_DMA_AUX) == 0) NGA_STEP(0); else NGA_STEP(2);
+#undef NGA_STEP
 }
 
 }  // namespace nga

@@ -63,6 +63,24 @@ void launch_decode_attention(uint16_t* out, int64_t out_stride, const uint16_t* 
                              bool kv_fp8, float k_scale, float v_scale, hipStream_t stream,
                              bool skip_empty = false);
 
+// Attention of a decode step, rotation and cache write included (bf16 pages of head_dim 128)
+struct DecodeStep {
+  const float* part;       // fp32 K-split slabs of q | k | v [S, rows, (Hq + 2 Hkv) 128], or null: they are bf16
+  int S;
+  int64_t slab;            // elements of a slab
+  const int32_t* pos;      // position of each row's token
+  const float* cos_sin;    // [positions, 128]: cosines | sines
+  const int32_t* slots;    // cache slot of each row's token, the one of place ctx - 1, or -1: not written
+  uint16_t* kc;
+  uint16_t* vc;
+  int32_t* done;           // [rows, Hkv] partitions that have finished; zero before and after every launch
+};
+bool decode_step_covers(int num_seqs, int max_ctx, int pages_per_part, int window);
+void launch_decode_step(uint16_t* out, int64_t out_stride, const uint16_t* qkv, const DecodeStep& st,
+                        const int32_t* block_tables, int max_blocks, const int32_t* ctx_lens, int num_seqs, int Hq,
+                        int Hkv, int max_ctx, float scale, int pages_per_part, float* part_ml, float* part_o,
+                        int window, hipStream_t stream);
+
 // attention_prefill.hip
 struct PrefillParams {
   uint16_t* out;

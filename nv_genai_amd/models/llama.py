@@ -647,6 +647,13 @@ class LlamaModel:
         ``ops.PartialSum`` when ``partial_ok`` and the o GEMM split K)."""
         L = self.layers[li]
         qkv = self._qkv(x, L, partial_ok=True)
+        if meta.kind == "decode" and ops.decode_step_covers(qkv, self.k_cache[li], meta.ctx_lens, meta.slots, meta.max_ctx,
+                                                            meta.decode_ws, self.window):
+            attn = ops.decode_step(qkv, pos, self.cos_sin, meta.slots, self.k_cache[li], self.v_cache[li], meta.block_tables,
+                                   meta.ctx_lens, self.hq, self.hkv, meta.max_ctx, self.scale, meta.decode_ws, self.window)
+            if "bo" in L:
+                return self._bias_rank0(self._lin(attn, L, "wo"), L.get("bo"))
+            return self._lin(attn, L, "wo", partial_ok=partial_ok)
         part = None
         if isinstance(qkv, ops.PartialSum):   # K-split projection: the RoPE kernel sums the slabs
             part = qkv

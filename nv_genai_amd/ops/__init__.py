@@ -1103,6 +1103,7 @@ class DecodeWorkspace:
         need = max(b * self.nparts(b) for b in range(1, max_seqs + 1))
         self.ml = torch.empty(need * Hq * 2, dtype=torch.float32, device=device)
         self.o = torch.empty(need * Hq * D, dtype=torch.float32, device=device)
+        self.done = torch.zeros(max_seqs * Hkv, dtype=torch.int32, device=device)   # decode_step: partitions that have finished
         self.D = D
 
     def nparts(self, B: int) -> int:
@@ -1177,6 +1178,28 @@ def decode_attention(q, kc, vc, block_tables, ctx_lens, Hq, Hkv, max_ctx, scale,
     kernels().decode_attention(out, q, kc, vc, block_tables, ctx_lens, Hq, Hkv, int(max_ctx),
                                float(scale), ws.pages_per_part(B, max_ctx), ws.ml, ws.o,
                                int(window), float(kv_scales[0]), float(kv_scales[1]), bool(skip_empty))
+    return out
+
+
+def decode_step_covers(qkv, kc, ctx_lens, slots, max_ctx, ws: Optional[DecodeWorkspace], window: int = 0) -> bool:
+    """Whether :func:`decode_step` runs this step: bf16 pages of head_dim 128 on the GPU, one new token a row."""
+    t = qkv.slabs if isinstance(qkv, PartialSum) else qkv
+    B = ctx_lens.numel()
+    return (_gpu(t) and kc.dtype == torch.bfloat16 and kc.shape[3] == 128 and ws is not None and ws.D == 128 and max_ctx <= ws.max_ctx
+            and t.is_contiguous() and t.dtype == (torch.float32 if t.dim() == 3 else torch.bfloat16) and t.data_ptr() % 16 == 0
+            and slots is not None and t.shape[-2] == B == slots.numel() and B * kc.shape[1] <= ws.done.numel()
+            and kernels().decode_step_covers(B, int(max_ctx), ws.pages_per_part(B, max_ctx), int(window)))
+
+
+def decode_step(qkv, pos, cos_sin, slots, kc, vc, block_tables, ctx_lens, Hq, Hkv, max_ctx, scale, ws: DecodeWorkspace,
+                window: int = 0):
+    """:func:`rope_cache_` and :func:`decode_attention` of one new token a row in one launch. ``qkv``: the projection's bf16
+    rows or its :class:`PartialSum`; ``slots``: the cache slots of places ``ctx_lens - 1`` (-1: not written)."""
+    t = qkv.slabs if isinstance(qkv, PartialSum) else qkv
+    B = ctx_lens.numel()
+    out = torch.empty(B, Hq * 128, dtype=kc.dtype, device=kc.device)
+    kernels().decode_step(out, t, pos, cos_sin, slots, kc, vc, block_tables, ctx_lens, Hq, Hkv, int(max_ctx), float(scale),
+                          ws.pages_per_part(B, max_ctx), ws.ml, ws.o, ws.done, int(window))
     return out
 
 

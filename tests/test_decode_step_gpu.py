@@ -1,0 +1,63 @@
+"""The fused kernels of a decode step against the launches that they stand for."""
+import math
+
+import pytest
+import torch
+
+from nv_genai_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _pages(ctxs, Hkv, dev):
+    pages = [(c + 63) // 64 for c in ctxs]
+    nb = sum(pages) + 3
+    kc = torch.randn(nb, Hkv, 64, 128, device=dev).to(torch.bfloat16)
+    vc = torch.randn(nb, Hkv, 128, 64, device=dev).to(torch.bfloat16)
+    perm = torch.randperm(nb).tolist()
+    bt = torch.zeros(len(ctxs), max(pages), dtype=torch.int32)
+    slots, k = [], 0
+    for i, (c, p) in enumerate(zip(ctxs, pages)):
+        for j in range(p):
+            bt[i, j], k = perm[k], k + 1
+        slots.append(int(bt[i, (c - 1) // 64]) * 64 + (c - 1) % 64 if c else -1)
+    return kc, vc, bt.to(dev), torch.tensor(slots, dtype=torch.int32, device=dev)
+
+
+@pytest.mark.parametrize("G,Hkv", [(4, 8), (1, 8), (5, 2), (16, 1)])
+@pytest.mark.parametrize("ppp,window", [(None, 0), (1, 0), (3, 0), (2, 200), (None, 64)])
+@pytest.mark.parametrize("slabs", [0, 1, 3])
+def test_decode_step_is_rotation_and_attention(gpu, G, Hkv, ppp, window, slabs):
+    """Contexts around the ends of pages and of partitions, rows without a context and rows whose key is not written. The
+    cache is the same to the bit. The outputs are bf16 of the same products; only the sum over the partitions has another
+    form (two fp32 sums over up to 16 parts, then one rounding): one bf16 step, 2^-8 of the value, and of the largest where
+    values cancel."""
+    torch.manual_seed(G * 100 + slabs)
+    Hq, D, dev = Hkv * G, 128, gpu
+    part = 64 * 4 * (ppp or 1)
+    ctxs = [1, 0, 63, 64, 65, 700, 128, part - 1, part, part + 1, 3 * part + 1, 2500]
+    kc, vc, bt, slots = _pages(ctxs, Hkv, dev)
+    slots[6] = -1
+    B, row = len(ctxs), (Hq + 2 * Hkv) * D
+    if slabs:
+        qkv = ops.PartialSum(torch.randn(slabs, B, row, device=dev))
+        flat = ops.splitk_reduce(qkv.slabs)
+    else:
+        flat = torch.randn(B, row, device=dev).to(torch.bfloat16)
+        qkv = flat.clone()
+    ctx = torch.tensor(ctxs, dtype=torch.int32, device=dev)
+    pos = (ctx - 1).clamp(min=0)
+    cs = ops.rope_cos_sin(4096, D).to(dev)
+    most, scale = max(ctxs), 1 / math.sqrt(D)
+    ws = ops.DecodeWorkspace(B, Hq, Hkv, most, dev, ppp)
+    k1, v1, k2, v2 = kc.clone(), vc.clone(), kc.clone(), vc.clone()
+    ops.rope_cache_(flat, pos, cs, slots, k1, v1, Hq, Hkv, D)
+    want = ops.decode_attention(flat[:, : Hq * D], k1, v1, bt, ctx, Hq, Hkv, most, scale, ws=ws, window=window)
+    assert ops.decode_step_covers(qkv, k2, ctx, slots, most, ws, window)
+    for _ in range(2):   # the counters are zero again after a launch
+        got = ops.decode_step(qkv, pos, cs, slots, k2, v2, bt, ctx, Hq, Hkv, most, scale, ws, window)
+        assert torch.equal(k1, k2) and torch.equal(v1, v2)
+        assert not ws.done.any()
+        w, g = want.float(), got.float()
+        assert (g[1] == 0).all()
+        assert ((g - w).abs() <= 2 ** -8 * w.abs() + 2 ** -8 * w.abs().amax(1, keepdim=True)).all()
