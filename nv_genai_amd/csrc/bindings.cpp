@@ -465,7 +465,17 @@ void skinny_gemm(Tensor out, Tensor x, Tensor w, int64_t epi, int64_t split, int
   nga::launch_skinny_gemm(p, (int)cfg, (int)epi, cur_stream(x));
 }
 
-void gemv(Tensor out, Tensor x, Tensor w, int64_t epi) {
+// the RMSNorm weight that a decode projection applies to its rows first
+const uint16_t* norm_weight(const c10::optional<Tensor>& nw, const Tensor& x, int64_t epi, const char* what) {
+  if (!nw.has_value()) return nullptr;
+  CHECK_BF16((*nw)); CHECK_CONTIG((*nw));
+  TORCH_CHECK(nw->device() == x.device() && nw->numel() == x.size(1) && reinterpret_cast<uintptr_t>(nw->data_ptr()) % 16 == 0, what,
+              ": norm weight of K values at a 16-byte address");
+  TORCH_CHECK((epi == 1 || epi == 2) && x.size(0) == 1 && x.numel() <= 8192, what, ": norm for epi 1 or 2, one row, K <= 8192");
+  return bfp(*nw);
+}
+
+void gemv(Tensor out, Tensor x, Tensor w, int64_t epi, c10::optional<Tensor> norm_w, double eps) {
   CHECK_DEV(x); CHECK_BF16(x); CHECK_BF16(w);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2, "gemv: 2-D x / w / out");
   TORCH_CHECK(x.device() == w.device() && x.device() == out.device(), "gemv: one device");
@@ -489,15 +499,17 @@ void gemv(Tensor out, Tensor x, Tensor w, int64_t epi) {
   p.K = (int)K;
   p.out = out.data_ptr();
   p.ldo = out.stride(0);
+  p.norm_w = norm_weight(norm_w, x, epi, "gemv");
+  p.eps = (float)eps;
   TORCH_CHECK(nga::launch_gemv(p, (int)epi, cur_stream(x)), "gemv: shape out of range");
 }
 
-void stream_gemm(Tensor out, Tensor x, Tensor w, int64_t epi) {
+void stream_gemm(Tensor out, Tensor x, Tensor w, int64_t epi, c10::optional<Tensor> norm_w, double eps) {
   CHECK_DEV(x); CHECK_BF16(x); CHECK_BF16(w);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2, "stream_gemm: 2-D x / w / out");
   TORCH_CHECK(x.device() == w.device() && x.device() == out.device(), "stream_gemm: one device");
   const int64_t M = x.size(0), K = x.size(1);
-  TORCH_CHECK(epi >= 0 && epi <= 2 && (epi != 2 || w.size(0) % 2 == 0), "stream_gemm: epi 0 (bf16), 1 (fp32), 2 (SwiGLU)");
+  TORCH_CHECK(epi >= 0 && epi <= 3 && (epi != 2 || w.size(0) % 2 == 0), "stream_gemm: epi 0 (bf16), 1 (fp32), 2 (SwiGLU), 3 (bf16, added)");
   const int64_t N = epi == 2 ? w.size(0) / 2 : w.size(0);
   TORCH_CHECK(M <= 16 && K % 256 == 0 && N % 16 == 0 && w.size(1) == K && N < (int64_t(1) << 30), "stream_gemm: M <= 16, K % 256 == 0, N % 16 == 0");
   TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 8 == 0 && w.is_contiguous() &&
@@ -507,7 +519,8 @@ void stream_gemm(Tensor out, Tensor x, Tensor w, int64_t epi) {
                   reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0 &&
                   out.scalar_type() == (epi == 1 ? at::kFloat : at::kBFloat16),
               "stream_gemm: out [M, N]");
-  nga::launch_stream_gemm({bfp(x), x.stride(0), bfp(w), (int)M, (int)N, (int)K, out.data_ptr(), out.stride(0)}, (int)epi, cur_stream(x));
+  nga::launch_stream_gemm({bfp(x), x.stride(0), bfp(w), (int)M, (int)N, (int)K, out.data_ptr(), out.stride(0),
+                           norm_weight(norm_w, x, epi, "stream_gemm"), (float)eps}, (int)epi, cur_stream(x));
 }
 
 void splitk_swiglu(Tensor out, Tensor P, int64_t S) {

@@ -101,6 +101,38 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// A bf16 row of K <= 512 NJ values in one wave's registers (16-byte rows, K % 8 == 0), and 1 / rms of it
+template <int NJ>
+__device__ __forceinline__ void wave_row_load(u16x8 (&v)[NJ], const uint16_t* row, int K, int lane) {
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) v[j] = 512 * j + 8 * lane < K ? load8(row + 512 * j + 8 * lane) : (u16x8)(0);
+}
+
+template <int NJ>
+__device__ __forceinline__ float wave_row_rstd(const u16x8 (&v)[NJ], int K, float eps) {
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss = __builtin_fmaf(bf2f(v[j][i]), bf2f(v[j][i]), ss);
+  return rsqrtf(wave_sum(ss) / (float)K + eps);
+}
+
+// 16 bytes to LDS while LDS-DMAs are under way: the compiler makes an ordinary store wait for all of them. Followed by
+// lds_stored() before it is read.
+__device__ __forceinline__ void lds_store8(uint16_t* p, u16x8 v) {
+  asm volatile("ds_write_b128 %0, %1" ::"v"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)p), "v"(v) : "memory");
+}
+__device__ __forceinline__ void lds_stored() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// rounded as the RMSNorm kernel rounds
+__device__ __forceinline__ u16x8 rms_apply8(u16x8 x, float r, u16x8 w) {
+  u16x8 o;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[i] = f2bf(bf2f(x[i]) * r * bf2f(w[i]));
+  return o;
+}
+
 // Block-wide sum; `red` must hold >= blockDim.x/64 floats. All threads get the result.
 __device__ __forceinline__ float block_sum(float v, float* red) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;

@@ -29,12 +29,17 @@ __device__ __forceinline__ void st_wait_vm() {
 __device__ __forceinline__ float st_silu(float x) { return x / (1.f + __expf(-x)); }
 }  // namespace
 
-// EPI 0: bf16 out; 1: fp32 out; 2: bf16 silu(gate) up of W = [gate | up] rows, N = F (8 NT features a tile)
-template <int NT, int EPI>
+// EPI 0: bf16 out; 1: fp32 out; 2: bf16 silu(gate) up of W = [gate | up] rows, N = F (8 NT features a tile); 3: bf16 out += product
+// NJ > 0: the one row is normed first (RMSNorm, K <= 512 NJ), while the first two stages are under way. Each wave sums the row's
+// squares by itself and lays the K range that it multiplies in its own part of LDS, so that none waits for another. It takes the
+// place of a launch of 4.6 us (6,144 x 4,096: 10.0 us, with the norm 12.1); for two rows it costs what it saves (SwiGLU 2 x 14,336 x
+// 4,096: 38.3, with the norm 43.0), since every workgroup reads them whole.
+template <int NT, int EPI, int NJ>
 __global__ void __launch_bounds__(256) stream_gemm_kernel(StreamGemmParams P) {
   constexpr int NW = 4;
   constexpr int KS = 256 / NT, CPR = KS / 8, KSTEPS = KS / 32;   // k of a stage, its 16-byte chunks a row, its MFMA steps
-  __shared__ __attribute__((aligned(16))) uint16_t ring[NW * 2 * 4096];
+  constexpr int XS = NW * 2 * 4096;                              // the normed row
+  __shared__ __attribute__((aligned(16))) uint16_t ring[XS + 512 * NJ];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, h = lane >> 4;
   const int tile = blockIdx.x;
@@ -57,10 +62,12 @@ __global__ void __launch_bounds__(256) stream_gemm_kernel(StreamGemmParams P) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) glds16(wsrc[i] + (int64_t)s * KS, b + i * 512);
   };
+  const uint16_t* xl = ring + XS + 8 * h;
   auto load_x = [&](int s, u16x8 (&x)[KSTEPS]) {
 #pragma unroll
-    for (int k = 0; k < KSTEPS; ++k) x[k] = load8(xp + (int64_t)s * KS + 32 * k);
+    for (int k = 0; k < KSTEPS; ++k) x[k] = NJ ? *reinterpret_cast<const u16x8*>(xl + s * KS + 32 * k) : load8(xp + (int64_t)s * KS + 32 * k);
   };
+  constexpr int XV = NJ ? 0 : KSTEPS;   // loads of token rows in flight
   f32x4 acc[NT];
 #pragma unroll
   for (int i = 0; i < NT; ++i) acc[i] = (f32x4)(0.f);
@@ -86,16 +93,48 @@ __global__ void __launch_bounds__(256) stream_gemm_kernel(StreamGemmParams P) {
     __builtin_amdgcn_sched_barrier(0);
     issue(s + 1);
     __builtin_amdgcn_sched_barrier(0);
-    st_wait_vm<8 + KSTEPS>();
+    st_wait_vm<8 + XV>();
     multiply(s, x);
   };
   u16x8 xa[KSTEPS], xb[KSTEPS];
   if (s0 < s1) {
-    load_x(s0, xa);
-    __builtin_amdgcn_sched_barrier(0);
-    issue(s0);
-    __builtin_amdgcn_sched_barrier(0);
-    int s = s0;   // the last steps apart: a branch around the loads would make the compiler wait for all of them
+    int s = s0;
+    if constexpr (NJ > 0) {
+      constexpr int SJ = NJ / NW + 1;   // 512-value pieces of a wave's K range, at most
+      const int k0 = s0 * KS, k1 = s1 * KS;
+      u16x8 nw[SJ], xr[SJ], v[NJ];
+      wave_row_load(v, P.x, P.K, lane);
+#pragma unroll
+      for (int j = 0; j < SJ; ++j) {
+        const int k = min(k0 + 512 * j + 8 * lane, k1 - 8);
+        nw[j] = load8(P.norm_w + k);
+        xr[j] = load8(P.x + k);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      issue(s0);
+      if (s0 + 1 < s1) issue(s0 + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      const float r = wave_row_rstd(v, P.K, P.eps);
+#pragma unroll
+      for (int j = 0; j < SJ; ++j) {
+        const int k = k0 + 512 * j + 8 * lane;
+        if (k < k1) lds_store8(ring + XS + k, rms_apply8(xr[j], r, nw[j]));
+      }
+      lds_stored();
+      if (s0 + 1 < s1) {
+        load_x(s0, xb);
+        st_wait_vm<8>();
+        multiply(s0, xb);
+        s = s0 + 1;
+      }
+      load_x(s, xa);
+    } else {
+      load_x(s0, xa);
+      __builtin_amdgcn_sched_barrier(0);
+      issue(s0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the last steps apart: a branch around the loads would make the compiler wait for all of them
     for (; s + 2 < s1; s += 2) {
       step(s, xa, xb);
       step(s + 1, xb, xa);
@@ -141,10 +180,12 @@ __global__ void __launch_bounds__(256) stream_gemm_kernel(StreamGemmParams P) {
       if constexpr (EPI == 1) {
         *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(P.out) + at) = acc[i];
       } else {
+        u16x4* to = reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + at);
         u16x4 o;
+        if constexpr (EPI == 3) o = *to;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = f2bf(acc[i][r]);
-        *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + at) = o;
+        for (int r = 0; r < 4; ++r) o[r] = f2bf(EPI == 3 ? bf2f(o[r]) + acc[i][r] : acc[i][r]);
+        *to = o;
       }
     }
   }
@@ -179,12 +220,19 @@ void launch_stream_gemm(const StreamGemmParams& p, int epi, hipStream_t stream) 
   const int t = (int)st_tiles(p.N, epi == 2);
   if (p.M == 0 || t == 0) return;
   const bool two = t > 256 && (t < 1024 || p.M > 8) && p.N % 32 == 0;
-#define NGA_ST(EPI)                                                                      \
-  if (two) stream_gemm_kernel<2, EPI><<<t / 2, 256, 0, stream>>>(p);                     \
-  else stream_gemm_kernel<1, EPI><<<t, 256, 0, stream>>>(p)
-  if (epi == 0) { NGA_ST(0); }
-  else if (epi == 1) { NGA_ST(1); }
-  else { NGA_ST(2); }
+#define NGA_ST(EPI, NJ)                                                                  \
+  if (two) stream_gemm_kernel<2, EPI, NJ><<<t / 2, 256, 0, stream>>>(p);                 \
+  else stream_gemm_kernel<1, EPI, NJ><<<t, 256, 0, stream>>>(p)
+  if (p.norm_w != nullptr && p.K <= 4096) {
+    if (epi == 1) { NGA_ST(1, 8); }
+    else { NGA_ST(2, 8); }
+  } else if (p.norm_w != nullptr) {
+    if (epi == 1) { NGA_ST(1, 16); }
+    else { NGA_ST(2, 16); }
+  } else if (epi == 0) { NGA_ST(0, 0); }
+  else if (epi == 1) { NGA_ST(1, 0); }
+  else if (epi == 2) { NGA_ST(2, 0); }
+  else { NGA_ST(3, 0); }
 #undef NGA_ST
 }
 

@@ -358,6 +358,8 @@ struct GemvParams {
   int M, N, K;         // M <= 4; K % 8 == 0, M * K * 2 <= 160 KiB
   void* out;           // epi 0 / 2: bf16 [M, ldo]; epi 1: fp32 [M, ldo]
   int64_t ldo;
+  const uint16_t* norm_w;   // epi 1 / 2: x goes through an RMSNorm of this weight first (M 1, K <= 8,192), or null
+  float eps;
 };
 // out = x . W^T for M <= 4 rows (gemv.hip); false if the shape is out of range
 bool launch_gemv(const GemvParams& p, int epi, hipStream_t stream);
@@ -367,8 +369,10 @@ struct StreamGemmParams {
   int64_t ldx;
   const uint16_t* w;   // [N, K] (epi 2: [2N, K] = [gate | up]); K % 256 == 0, N % 16 == 0
   int M, N, K;
-  void* out;           // epi 0 / 2: bf16 [M, ldo]; 1: fp32 [M, ldo]
+  void* out;           // epi 0 / 2: bf16 [M, ldo]; 1: fp32 [M, ldo]; 3: bf16 [M, ldo], added to
   int64_t ldo;
+  const uint16_t* norm_w;   // epi 1 / 2: x goes through an RMSNorm of this weight first (M 1, K <= 8,192), or null
+  float eps;
 };
 bool stream_gemm_covers(int64_t M, int64_t N, int64_t K, bool swiglu);
 void launch_stream_gemm(const StreamGemmParams& p, int epi, hipStream_t stream);

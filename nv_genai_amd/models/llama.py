@@ -646,24 +646,24 @@ class LlamaModel:
         """qkv projection + RoPE/KV write + attention + o projection (TP partial; an
         ``ops.PartialSum`` when ``partial_ok`` and the o GEMM split K)."""
         L = self.layers[li]
-        qkv = self._qkv(x, L, partial_ok=True)
-        if meta.kind == "decode" and ops.decode_step_covers(qkv, self.k_cache[li], meta.ctx_lens, meta.slots, meta.max_ctx,
-                                                            meta.decode_ws, self.window):
-            attn = ops.decode_step(qkv, pos, self.cos_sin, meta.slots, self.k_cache[li], self.v_cache[li], meta.block_tables,
-                                   meta.ctx_lens, self.hq, self.hkv, meta.max_ctx, self.scale, meta.decode_ws, self.window)
-            if "bo" in L:
-                return self._bias_rank0(self._lin(attn, L, "wo"), L.get("bo"))
-            return self._lin(attn, L, "wo", partial_ok=partial_ok)
-        part = None
-        if isinstance(qkv, ops.PartialSum):   # K-split projection: the RoPE kernel sums the slabs
-            part = qkv
-            qkv = torch.empty(part.shape, dtype=x.dtype, device=x.device)
-        ops.rope_cache_(qkv, pos, self.cos_sin, meta.slots, self.k_cache[li],
-                        self.v_cache[li], self.hq, self.hkv, self.D, kv_scales=self.kv_scales, partial=part)
-        attn = self._attention(qkv[:, :self.hq * self.D], qkv, li, meta, T)
+        attn = self._rotate_attend(li, self._qkv(x, L, partial_ok=True), pos, meta, T)
         if "bo" in L:
             return self._bias_rank0(self._lin(attn, L, "wo"), L.get("bo"))
         return self._lin(attn, L, "wo", partial_ok=partial_ok)
+
+    def _rotate_attend(self, li: int, qkv, pos, meta: AttnMeta, T: int):
+        """RoPE, KV write and attention of a projection's rows (or its ``ops.PartialSum``)."""
+        if meta.kind == "decode" and ops.decode_step_covers(qkv, self.k_cache[li], meta.ctx_lens, meta.slots, meta.max_ctx,
+                                                            meta.decode_ws, self.window):
+            return ops.decode_step(qkv, pos, self.cos_sin, meta.slots, self.k_cache[li], self.v_cache[li], meta.block_tables,
+                                   meta.ctx_lens, self.hq, self.hkv, meta.max_ctx, self.scale, meta.decode_ws, self.window)
+        part = None
+        if isinstance(qkv, ops.PartialSum):   # K-split projection: the RoPE kernel sums the slabs
+            part = qkv
+            qkv = torch.empty(part.shape, dtype=self.dtype, device=part.slabs.device)
+        ops.rope_cache_(qkv, pos, self.cos_sin, meta.slots, self.k_cache[li],
+                        self.v_cache[li], self.hq, self.hkv, self.D, kv_scales=self.kv_scales, partial=part)
+        return self._attention(qkv[:, :self.hq * self.D], qkv, li, meta, T)
 
     def _layer(self, li: int, x, resid, pos, meta: AttnMeta):
         """One decoder layer on rows (x = norm(resid)); returns the MLP output d — still
@@ -681,7 +681,33 @@ class LlamaModel:
             return self._norm(rows.contiguous(), self.final_norm, self.final_norm_b)
         return self._add_norm(resid, d, self.final_norm, self.final_norm_b)
 
+    def _fused_decode(self, resid, meta: AttnMeta) -> bool:
+        """Whether a decode step runs as :meth:`_decode_layers`: one row of a dense gated RMSNorm model in bf16 on one rank,
+        whose projections the kernels with norm and residual cover in every layer. From two rows on, a norm in every workgroup
+        of the next projection costs what its launch does (gemm_stream.hip)."""
+        c, M = self.cfg, resid.shape[0]
+        if (meta.kind != "decode" or M != 1 or not self.skinny or self.fp8 or self.p.tp_size > 1 or c.is_moe
+                or not c.gated_mlp or c.act != "silu" or c.norm == "layer" or not resid.is_contiguous()):
+            return False
+        return all("bqkv" not in L and "bo" not in L and "bd" not in L
+                   and ops.norm_linear_covers(resid, L["attn_norm"], L["wqkv"]) and ops.linear_add_covers(M, L["wo"])
+                   and ops.norm_linear_covers(resid, L["mlp_norm"], L["wgu"], True) and ops.linear_add_covers(M, L["wd"])
+                   for L in self.layers)
+
+    def _decode_layers(self, resid, pos, meta: AttnMeta) -> None:
+        """All layers of a decode step of one row, in five launches each: the norms are part of the projections behind
+        them and the residual of those before (8B: 91 us a layer, with the norms and
+        residuals in launches of their own 95)."""
+        for li, L in enumerate(self.layers):
+            qkv = ops.PartialSum(ops.norm_linear(resid, L["attn_norm"], self.cfg.eps, L["wqkv"], 1).unsqueeze(0))
+            ops.linear_add_(resid, self._rotate_attend(li, qkv, pos, meta, resid.shape[0]), L["wo"])
+            ops.linear_add_(resid, ops.norm_linear(resid, L["mlp_norm"], self.cfg.eps, L["wgu"], 2), L["wd"])
+
     def _stack(self, resid, pos, meta: AttnMeta, sample_idx: Optional[torch.Tensor]):
+        if self._fused_decode(resid, meta):
+            self._decode_layers(resid, pos, meta)
+            rows = resid if sample_idx is None else resid.index_select(0, sample_idx)
+            return self._norm(rows, self.final_norm, self.final_norm_b)
         L0 = self.layers[0]
         x = self._norm(resid, L0["attn_norm"], L0.get("attn_norm_b"))
         n = len(self.layers)

@@ -224,7 +224,7 @@ def gemv(x: torch.Tensor, w: torch.Tensor, epi: int = 0, out: Optional[torch.Ten
     N = w.shape[0] // 2 if epi == 2 else w.shape[0]
     if out is None:
         out = torch.empty(M, N, dtype=torch.float32 if epi == 1 else x.dtype, device=x.device)
-    kernels().gemv(out, x, w, int(epi))
+    kernels().gemv(out, x, w, int(epi), None, 0.0)
     return out
 
 
@@ -239,8 +239,37 @@ def stream_gemm(x: torch.Tensor, w: torch.Tensor, epi: int = 0) -> torch.Tensor:
     """x @ w^T of up to 16 token rows as one stream of the weights (gemm_stream.hip); ``epi`` as of :func:`gemv`."""
     N = w.shape[0] // 2 if epi == 2 else w.shape[0]
     out = torch.empty(x.shape[0], N, dtype=torch.float32 if epi == 1 else x.dtype, device=x.device)
-    kernels().stream_gemm(out, x, w, int(epi))
+    kernels().stream_gemm(out, x, w, int(epi), None, 0.0)
     return out
+
+
+def norm_linear_covers(x: torch.Tensor, norm_w: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:
+    """Whether :func:`norm_linear` runs rmsnorm(x [1, K]) @ w^T: one row (K <= 8,192) of bf16 on the GPU at 16-byte addresses."""
+    return (_gpu(x) and x.dim() == 2 and x.shape[0] == 1 and x.numel() <= 8192 and x.shape[1] % 8 == 0 and w.shape[0] > 0
+            and all(t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0 for t in (x, norm_w, w)) and w.is_contiguous()
+            and norm_w.is_contiguous() and x.stride(1) == 1 and x.stride(0) % 8 == 0)
+
+
+def norm_linear(x: torch.Tensor, norm_w: torch.Tensor, eps: float, w: torch.Tensor, epi: int) -> torch.Tensor:
+    """rmsnorm(x) @ w^T of one row with the norm in the projection's kernel; ``epi`` 1 -> fp32, 2 -> SwiGLU in bf16.
+    The stream kernel where it is the projection's (:func:`stream_covers`), else the GEMV."""
+    N = w.shape[0] // 2 if epi == 2 else w.shape[0]
+    out = torch.empty(x.shape[0], N, dtype=torch.float32 if epi == 1 else x.dtype, device=x.device)
+    run = kernels().stream_gemm if stream_covers(x, w, epi == 2) else kernels().gemv
+    run(out, x, w, int(epi), norm_w, float(eps))
+    return out
+
+
+def linear_add_covers(M: int, w: torch.Tensor) -> bool:
+    """Whether :func:`linear_add_` takes M contiguous rows against ``w``."""
+    return (_gpu(w) and w.dtype == torch.bfloat16 and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and kernels().stream_gemm_covers(M, w.shape[0], w.shape[1], False))
+
+
+def linear_add_(resid: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """resid += x @ w^T of up to 16 rows (fp32 sums, one bf16 rounding of the residual)."""
+    kernels().stream_gemm(resid, x, w, 3, None, 0.0)
+    return resid
 
 
 def splitk_reduce(P: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -61,3 +61,38 @@ def test_decode_step_is_rotation_and_attention(gpu, G, Hkv, ppp, window, slabs):
         w, g = want.float(), got.float()
         assert (g[1] == 0).all()
         assert ((g - w).abs() <= 2 ** -8 * w.abs() + 2 ** -8 * w.abs().amax(1, keepdim=True)).all()
+
+
+@pytest.mark.parametrize("N,K", [(4096, 4096), (6144, 4096), (16, 256), (48, 768), (1008, 2304), (14336, 4096), (512, 8192), (384, 5120),
+                                 (101, 520), (33, 1032), (7, 8), (2064, 8184)])
+@pytest.mark.parametrize("epi", [1, 2])
+def test_norm_linear(gpu, N, K, epi, M=1):
+    """Stages that do not split evenly over the waves, K below and at the kernels' ends, the GEMV for odd shapes. The norm's
+    sum of squares has another order, so a normed value may fall on the next bf16 (2^-8 of it): at most 2^-8 of a row of
+    products, and with SwiGLU, a product of two of them rounded to bf16, three times that."""
+    torch.manual_seed(N + K)
+    x = (2 * torch.randn(M, K, device=gpu)).to(torch.bfloat16)
+    nw = (1 + 0.3 * torch.randn(K, device=gpu)).to(torch.bfloat16)
+    w = (torch.randn((2 if epi == 2 else 1) * N, K, device=gpu) / math.sqrt(K)).to(torch.bfloat16)
+    assert ops.norm_linear_covers(x, nw, w, epi == 2)
+    got = ops.norm_linear(x, nw, 1e-5, w, epi).float()
+    y = ops.rmsnorm(x, nw, 1e-5).double() @ w.double().t()
+    want = torch.nn.functional.silu(y[:, :N]) * y[:, N:] if epi == 2 else y
+    assert got.shape == want.shape
+    err = (got.double() - want).norm(dim=1) / want.norm(dim=1)
+    assert (err <= 2 ** -8 * (3 if epi == 2 else 1)).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 4096), (2, 4096, 14336), (1, 16, 256), (7, 48, 768), (16, 4096, 4096), (8, 1024, 8192)])
+def test_linear_add(gpu, M, N, K):
+    """One rounding of the sum: half a bf16 step of it, and the products' fp32 sums in another order (K values, 2^-24 each)."""
+    torch.manual_seed(N + K)
+    x = torch.randn(M, K, device=gpu).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=gpu) / math.sqrt(K)).to(torch.bfloat16)
+    resid = torch.randn(M, N, device=gpu).to(torch.bfloat16)
+    assert ops.linear_add_covers(M, w)
+    want = resid.double() + x.double() @ w.double().t()
+    got = ops.linear_add_(resid, x, w)
+    assert got.data_ptr() == resid.data_ptr()
+    slack = 2 ** -24 * math.sqrt(K) * (x.double().abs() @ w.double().abs().t())
+    assert ((got.double() - want).abs() <= 2 ** -8 * want.abs() + slack + 1e-6).all()
