@@ -1208,7 +1208,9 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
   Tensor qkv = at::empty({T, 3 * H}, opt), a = at::empty({T, H}, opt), y = at::empty({T, H}, opt), h = at::empty({T, F}, opt);
   const bool rows = T <= 32, tiles = !rows && T <= 1024;
   Tensor slabs;
-  if (rows || tiles) slabs = at::empty({std::max(encoder_split(T, H), encoder_split(T, F)), T, H}, opt.dtype(at::kFloat));
+  const bool one = rows && B == 1 && max_len >= T;   // a single query; where several lie is known on the GPU alone
+  const int att_split = one ? nga::row_attn_split((int)heads) : 0;
+  if (rows || tiles) slabs = at::empty({std::max({encoder_split(T, H), encoder_split(T, F), att_split}), T, H}, opt.dtype(at::kFloat));
   // out = x w^T + bias (GELU)
   auto project = [&](const Tensor& in, const Tensor& w, const Tensor& bias, Tensor& out, bool gelu) {
     const int64_t N = w.size(0), K = w.size(1);
@@ -1258,8 +1260,15 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
   p.scale = (float)scale;
   for (size_t i = 0; i < L.size(); i += 12) {
     project(x, L[i], L[i + 1], qkv, false);
-    if (B > 0 && max_len > 0) nga::launch_varlen_attention(p, (int)B, (int)max_len, (int)D, false, st);
-    project_norm(a, L[i + 2], L[i + 3], x, L[i + 4], L[i + 5], x);
+    if (one) {
+      nga::launch_row_attn_gemm({bfp(qkv), 3 * H, bfp(L[i + 2]), nullptr, slabs.data_ptr(), H, (int)T, (int)H, (int)H, att_split,
+                                 p.cu_q, p.scale}, (int)D, st);
+      nga::launch_splitk_layernorm(slabs.data_ptr<float>(), att_split, (int)T, bfp(L[i + 3]), bfp(x), bfp(L[i + 4]), bfp(L[i + 5]),
+                                   (float)eps, (int)H, bfp(x), st);
+    } else {
+      if (B > 0 && max_len > 0) nga::launch_varlen_attention(p, (int)B, (int)max_len, (int)D, false, st);
+      project_norm(a, L[i + 2], L[i + 3], x, L[i + 4], L[i + 5], x);
+    }
     project(x, L[i + 6], L[i + 7], h, true);
     project_norm(h, L[i + 8], L[i + 9], x, L[i + 10], L[i + 11], x);
   }

@@ -14,6 +14,9 @@
 namespace nga {
 
 namespace {
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4* ltr_t;
+
 // 0.5 x (1 + erf(x / sqrt 2))
 __device__ __forceinline__ float gr_gelu(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
 }  // namespace
@@ -33,6 +36,8 @@ __global__ void __launch_bounds__(512) row_gemm_kernel(RowGemmParams P) {
   const uint16_t *wp = P.w + (int64_t)(f0 + col) * P.K + 8 * h, *xp[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) xp[i] = P.x + (int64_t)min(t0 + 16 * i + col, P.M - 1) * P.ldx + 8 * h;
+  u16x4 bias = (u16x4)(0);   // asked for with the rest: at the end it would be a latency of its own
+  if (EPI != 1 && w < MT) bias = *reinterpret_cast<const u16x4*>(P.bias + f0 + 4 * h);
   f32x4 acc[MT];
 #pragma unroll
   for (int j = 0; j < MT; ++j) acc[j] = (f32x4)(0.f);
@@ -82,7 +87,7 @@ __global__ void __launch_bounds__(512) row_gemm_kernel(RowGemmParams P) {
       u16x4 o;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float y = v[r] + bf2f(P.bias[n + r]);
+        const float y = v[r] + bf2f(bias[r]);
         o[r] = f2bf(EPI == 2 ? gr_gelu(y) : y);
       }
       *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + (int64_t)t * P.ldo + n) = o;
@@ -90,7 +95,126 @@ __global__ void __launch_bounds__(512) row_gemm_kernel(RowGemmParams P) {
   }
 }
 
-// out = LN(sum_s P[s] + bias + resid): the norm behind a K-split projection (P [S, M, H] fp32)
+// The attention of one sequence of up to 32 rows and the output projection behind it, as slabs [split, M, N]: x = q | k | v, a
+// K slice is a few heads, and each of its N / 16 workgroups computes those heads by itself, a head's 16 queries a wave. As in
+// attention_decode.hip the key order of S^T makes P^T the next operand; V comes transposed from LDS (ds_read_b64_tr_b16).
+// (BERT-large, 19 rows: attention 4.5 and output 3.6 us in two launches, 5.4 in one.)
+template <int MT, int D>
+__global__ void __launch_bounds__(512) row_attn_gemm_kernel(RowGemmParams P) {
+  constexpr int NW = 8, PD = 4, VL = D + 8, DS = D / 32, DT = D / 16;
+  extern __shared__ __attribute__((aligned(16))) uint16_t sm[];   // [16 MT][columns + 8] rows, then V of each wave; partial sums
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, h = lane >> 4;
+  const int f0 = blockIdx.x * 16, ks = blockIdx.z, heads = P.K / D;
+  const int h0 = heads * ks / P.split, h1 = heads * (ks + 1) / P.split, cols = (h1 - h0) * D, ld = cols + 8;
+  const int steps = cols / 32, s0 = steps * w / NW, s1 = steps * (w + 1) / NW;
+  const uint16_t* wp = P.w + (int64_t)(f0 + col) * P.K + h0 * D + 8 * h;
+  u16x8 a[PD];
+#pragma unroll
+  for (int d = 0; d < PD; ++d) a[d] = s0 + d < s1 ? load8(wp + 32 * (s0 + d)) : (u16x8)(0);
+  // rows beside the sequence are clamped into it: whatever those hold, it would be multiplied by 0
+  const int lo = max(0, P.cu[0]), hi = min(P.M, P.cu[1]);
+  auto row = [&](int r) { return (int64_t)max(lo, min(r, hi - 1)) * P.ldx; };
+  uint16_t* const vh = sm + 16 * MT * ld + w * (16 * MT * VL);
+  for (int u = w; u < (h1 - h0) * MT; u += NW) {
+    const int hd = u / MT, i = u % MT;   // queries 16 i .. of head h0 + hd
+    const uint16_t* base = P.x + (h0 + hd) * D;
+    u16x8 vr[MT * D / 32], kf[MT][DS], qf[DS];
+#pragma unroll
+    for (int s = 0; s < DS; ++s) {
+      qf[s] = load8(base + row(16 * i + col) + 32 * s + 8 * h);
+#pragma unroll
+      for (int t = 0; t < MT; ++t)   // row `col` of key tile t: key 8 (col / 4) + 4 t + col % 4 (of 16 keys: their order)
+        kf[t][s] = load8(base + P.K + row(MT == 2 ? 8 * (col >> 2) + 4 * t + (col & 3) : col) + 32 * s + 8 * h);
+    }
+#pragma unroll
+    for (int j = 0; j < MT * D / 32; ++j) {
+      const int c = 64 * j + lane;
+      vr[j] = load8(base + 2 * P.K + row(c / (D / 8)) + 8 * (c % (D / 8)));
+    }
+#pragma unroll
+    for (int j = 0; j < MT * D / 32; ++j) {
+      const int c = 64 * j + lane;
+      store8(vh + c / (D / 8) * VL + 8 * (c % (D / 8)), vr[j]);
+    }
+    f32x4 S[MT];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      S[t] = (f32x4)(0.f);
+#pragma unroll
+      for (int s = 0; s < DS; ++s) S[t] = mfma16(as_bf16x8(kf[t][s]), as_bf16x8(qf[s]), S[t]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int key = MT == 2 ? 8 * h + 4 * t + r : 4 * h + r;
+        S[t][r] = key >= lo && key < hi ? S[t][r] * (P.scale * 1.4426950408889634f) : -INFINITY;
+        mx = fmaxf(mx, S[t][r]);
+      }
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    float l = 0.f;
+    u16x8 pf = (u16x8)(0);
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float e = __builtin_amdgcn_exp2f(S[t][r] - mx);
+        l += e;
+        pf[4 * t + r] = f2bf(e);
+      }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      // lane: dim 16 dt + col; keys 8 h .. 8 h + 7, of 16 keys 4 h .. 4 h + 3 and zeros
+      uint16_t* const at = vh + ((MT == 2 ? 8 : 4) * h + (col >> 2)) * VL + 16 * dt + 4 * (col & 3);
+      const s16x4 va = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ltr_t)at);
+      const s16x4 vb = MT == 2 ? __builtin_amdgcn_ds_read_tr16_b64_v4i16((ltr_t)(at + 4 * VL)) : (s16x4)(0);
+      const auto v8 = __builtin_shufflevector(va, vb, 0, 1, 2, 3, 4, 5, 6, 7);
+      const f32x4 o = mfma16(__builtin_bit_cast(bf16x8, v8), as_bf16x8(pf), (f32x4)(0.f));
+      u16x4 ob;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ob[r] = f2bf(o[r] * inv);
+      *reinterpret_cast<u16x4*>(sm + (16 * i + col) * ld + hd * D + 16 * dt + 4 * h) = ob;
+    }
+  }
+  f32x4 acc[MT];
+#pragma unroll
+  for (int j = 0; j < MT; ++j) acc[j] = (f32x4)(0.f);
+  __syncthreads();
+  for (int s = s0; s < s1; s += PD) {
+    if (s > s0)
+#pragma unroll
+      for (int d = 0; d < PD; ++d)
+        if (s + d < s1) a[d] = load8(wp + 32 * (s + d));
+#pragma unroll
+    for (int d = 0; d < PD; ++d)
+      if (s + d < s1)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[j] = mfma16(as_bf16x8(a[d]), as_bf16x8(load8(sm + (16 * j + col) * ld + 32 * (s + d) + 8 * h)), acc[j]);
+  }
+  float* const part = reinterpret_cast<float*>(sm + 16 * MT * ld);   // V is read
+#pragma unroll
+  for (int j = 0; j < MT; ++j) *reinterpret_cast<f32x4*>(&part[((w * MT + j) * 64 + lane) * 4]) = acc[j];
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < MT; ++j) {
+    const int t = 16 * j + col;
+    if (j != w || t >= P.M) continue;
+    f32x4 v = (f32x4)(0.f);
+#pragma unroll
+    for (int u = 0; u < NW; ++u) v += *reinterpret_cast<const f32x4*>(&part[((u * MT + j) * 64 + lane) * 4]);
+    *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(P.out) + ((int64_t)ks * P.M + t) * P.N + f0 + 4 * h) = v;
+  }
+}
+
+// out = LN(sum_s P[s] + bias + resid): the norm behind a K-split projection (P [S, M, H] fp32). NS: S, with all slabs' loads
+// in flight at once, or 0 (a loop waits for
+// each: 19 rows of 8 slabs 4.6 us, here 3.7)
+template <int NS>
 __global__ void __launch_bounds__(1024) splitk_layernorm_kernel(const float* __restrict__ P, int S, int M,
                                                                 const uint16_t* __restrict__ bias,
                                                                 const uint16_t* __restrict__ resid,
@@ -105,14 +229,32 @@ __global__ void __launch_bounds__(1024) splitk_layernorm_kernel(const float* __r
   u16x8 gv, bv;
   if (active) {
     const float* p = P + row * H + c;
-    f32x4 a0 = *reinterpret_cast<const f32x4*>(p), a1 = *reinterpret_cast<const f32x4*>(p + 4);
-    for (int k = 1; k < S; ++k) {
-      a0 += *reinterpret_cast<const f32x4*>(p + k * slab);
-      a1 += *reinterpret_cast<const f32x4*>(p + k * slab + 4);
-    }
+    f32x4 a0, a1;
     const u16x8 r = load8(resid + row * H + c), bi = load8(bias + c);
     gv = load8(g + c);
     bv = load8(b + c);
+    if constexpr (NS > 0) {
+      f32x4 v[NS][2];
+#pragma unroll
+      for (int k = 0; k < NS; ++k) {
+        v[k][0] = *reinterpret_cast<const f32x4*>(p + k * slab);
+        v[k][1] = *reinterpret_cast<const f32x4*>(p + k * slab + 4);
+      }
+      a0 = v[0][0];
+      a1 = v[0][1];
+#pragma unroll
+      for (int k = 1; k < NS; ++k) {
+        a0 += v[k][0];
+        a1 += v[k][1];
+      }
+    } else {
+      a0 = *reinterpret_cast<const f32x4*>(p);
+      a1 = *reinterpret_cast<const f32x4*>(p + 4);
+      for (int k = 1; k < S; ++k) {
+        a0 += *reinterpret_cast<const f32x4*>(p + k * slab);
+        a1 += *reinterpret_cast<const f32x4*>(p + k * slab + 4);
+      }
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       x[i] = (i < 4 ? a0[i] : a1[i - 4]) + bf2f(bi[i]) + bf2f(r[i]);
@@ -190,12 +332,40 @@ void launch_row_gemm(const RowGemmParams& p, int epi, hipStream_t stream) {
 #undef NGA_RG
 }
 
+// K slices of it: four heads each, eight at most
+int row_attn_split(int heads) { return heads <= 4 ? 1 : heads <= 32 ? (heads + 3) / 4 : 8; }
+
+void launch_row_attn_gemm(const RowGemmParams& p, int D, hipStream_t stream) {
+  if (p.M == 0 || p.N == 0) return;
+  const int mt = p.M <= 16 ? 1 : 2, heads = p.K / D;
+  const size_t cols = (size_t)((heads + p.split - 1) / p.split) * D, sums = (size_t)8 * mt * 1024, v = (size_t)8 * 16 * mt * (D + 8) * 2;
+  const size_t lds = 16 * mt * (cols + 8) * 2 + (v > sums ? v : sums);
+#define NGA_RA(MT_, DD)                                                                                    \
+  {                                                                                                        \
+    static const hipError_t attr = hipFuncSetAttribute((const void*)row_attn_gemm_kernel<MT_, DD>,         \
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
+    (void)attr;                                                                                            \
+    row_attn_gemm_kernel<MT_, DD><<<dim3(p.N / 16, 1, p.split), 512, lds, stream>>>(p);                    \
+  }
+#define NGA_RD(MT_) if (D == 32) NGA_RA(MT_, 32) else if (D == 64) NGA_RA(MT_, 64) else NGA_RA(MT_, 128)
+  if (mt == 1) { NGA_RD(1) } else { NGA_RD(2) }
+#undef NGA_RD
+#undef NGA_RA
+}
+
 static int rows_threads(int H) { return (H / 8 + 63) / 64 * 64; }
 
 void launch_splitk_layernorm(const float* P, int S, int M, const uint16_t* bias, const uint16_t* resid, const uint16_t* g,
                              const uint16_t* b, float eps, int H, uint16_t* out, hipStream_t stream) {
   if (M == 0) return;
-  splitk_layernorm_kernel<<<M, rows_threads(H), 0, stream>>>(P, S, M, bias, resid, g, b, eps, H, out);
+#define NGA_SL(NS) splitk_layernorm_kernel<NS><<<M, rows_threads(H), 0, stream>>>(P, S, M, bias, resid, g, b, eps, H, out)
+  if (S == 1) NGA_SL(1);
+  else if (S == 2) NGA_SL(2);
+  else if (S == 3) NGA_SL(3);
+  else if (S == 4) NGA_SL(4);
+  else if (S == 8) NGA_SL(8);
+  else NGA_SL(0);
+#undef NGA_SL
 }
 
 void launch_embed_layernorm(const int32_t* ids, const int32_t* pos, const int32_t* types, const uint16_t* word, int n_word,

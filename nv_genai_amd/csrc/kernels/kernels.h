@@ -225,8 +225,12 @@ struct RowGemmParams {
   void* out;
   int64_t ldo;
   int M, N, K, split;
+  const int32_t* cu;   // row_attn_gemm: the rows' one sequence, cu[0] .. cu[1]; x = q | k | v, K the values of one of them
+  float scale;
 };
 void launch_row_gemm(const RowGemmParams& p, int epi, hipStream_t stream);
+int row_attn_split(int heads);
+void launch_row_attn_gemm(const RowGemmParams& p, int D, hipStream_t stream);
 void launch_splitk_layernorm(const float* P, int S, int M, const uint16_t* bias, const uint16_t* resid, const uint16_t* g,
                              const uint16_t* b, float eps, int H, uint16_t* out, hipStream_t stream);
 void launch_embed_layernorm(const int32_t* ids, const int32_t* pos, const int32_t* types, const uint16_t* word, int n_word,
