@@ -73,9 +73,11 @@ __device__ __forceinline__ float sk_silu(float x) { return x / (1.f + __expf(-x)
 __device__ __forceinline__ f32x4 sk_ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 }  // namespace
 
-template <int BN, int BM, int WN, int WM, int NSTAGE, int EPI, int SBK>
-__global__ void __launch_bounds__(64 * WN * WM) skinny_gemm_kernel(SkinnyGemmParams P) {
-  constexpr int NW = WN * WM;   // waves per workgroup (4 or 8)
+// KG > 1: so many groups of WN x WM waves share the tile's K range, each with stages of its own, and meet once in LDS; each then
+// finishes some of the token tiles. For grids of at most a workgroup a CU, where one wave a SIMD waits out every latency.
+template <int BN, int BM, int WN, int WM, int NSTAGE, int EPI, int SBK, int KG = 1>
+__global__ void __launch_bounds__(64 * WN * WM * KG) skinny_gemm_kernel(SkinnyGemmParams P) {
+  constexpr int NW = WN * WM;   // waves per group (4 or 8)
   constexpr int RW = BN / WN;   // weight rows per wave
   constexpr int CW = BM / WM;   // token rows per wave
   constexpr int NTW = RW / 16, MTW = CW / 16;
@@ -90,7 +92,8 @@ __global__ void __launch_bounds__(64 * WN * WM) skinny_gemm_kernel(SkinnyGemmPar
   constexpr int W_GL = BN / (RPI * NW), X_GL = BM / (RPI * NW);   // DMA instructions per wave per stage
   constexpr int NPS = W_GL + X_GL;
   constexpr int STAGE = (BN + BM) * SBK;          // uint16 elements per stage
-  __shared__ __attribute__((aligned(16))) uint16_t smem[NSTAGE * STAGE];
+  static_assert(KG == 1 || (EPI != 2 && MTW % KG == 0), "groups finish whole token tiles");
+  __shared__ __attribute__((aligned(16))) uint16_t smem[KG * NSTAGE * STAGE];
 
   const int nblk = P.nN * P.nM * P.split;
   const int pb = blockIdx.x;
@@ -100,10 +103,11 @@ __global__ void __launch_bounds__(64 * WN * WM) skinny_gemm_kernel(SkinnyGemmPar
   const int ks = (L / P.nM) % P.split;
   const int nb = L / (P.nM * P.split);
   const int nk_all = P.K / SBK;
-  const int kb = ks * nk_all / P.split;
-  const int nk = (ks + 1) * nk_all / P.split - kb;
-
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, kg = KG > 1 ? tid / (64 * NW) : 0, wv = (tid >> 6) - kg * NW;
+  const int parts = P.split * KG, part = ks * KG + kg;
+  const int kb = part * nk_all / parts;
+  const int nk = (part + 1) * nk_all / parts - kb, turns = (nk_all + parts - 1) / parts;
+  uint16_t* const stages = smem + kg * (NSTAGE * STAGE);
   const int wn = wv % WN, wm = wv / WN;
   const int col = lane & 15, h = lane >> 4;
 
@@ -147,7 +151,7 @@ __global__ void __launch_bounds__(64 * WN * WM) skinny_gemm_kernel(SkinnyGemmPar
   // same 128-B column of it at the same moment
   const int rot = P.krot ? (int)((unsigned)(nb * 7 + mi * 3) % (unsigned)nk) : 0;
   auto issue = [&](int kt, int buf) {
-    uint16_t* base = smem + buf * STAGE;
+    uint16_t* base = stages + buf * STAGE;
     int ke = kt + rot;
     if (ke >= nk) ke -= nk;
     const int k0 = ke * SBK;
@@ -189,7 +193,18 @@ __global__ void __launch_bounds__(64 * WN * WM) skinny_gemm_kernel(SkinnyGemmPar
 #pragma unroll
   for (int st = 0; st < NSTAGE - 1; ++st)
     if (st < nk) issue(st, st);
-  for (int kt = 0; kt < nk; ++kt) {
+  u16x4 bias[EPI >= 3 ? NTW : 1];   // asked for now: behind the products it would be a latency of its own
+  if constexpr (EPI >= 3) {
+#pragma unroll
+    for (int nt = 0; nt < NTW; ++nt) bias[nt] = *reinterpret_cast<const u16x4*>(P.bias + min(nb * BN + wn * RW + nt * 16 + 4 * h, P.N - 4));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  for (int kt = 0; kt < (KG > 1 ? turns : nk); ++kt) {
+    if (KG > 1 && kt >= nk) {   // a shorter share than the other groups'
+      sk_wait_vm<0>();
+      __builtin_amdgcn_s_barrier();
+      continue;
+    }
     // retire stage kt (this wave's DMA); later stages stay in flight. The count is the DMA of
     // the stages issued after kt: NSTAGE - 2 of them in the steady state, fewer at the tail.
     const int after = min(nk - 1 - kt, NSTAGE - 2);
@@ -197,7 +212,7 @@ __global__ void __launch_bounds__(64 * WN * WM) skinny_gemm_kernel(SkinnyGemmPar
     else if (after == 1) sk_wait_vm<NPS>();
     else sk_wait_vm<0>();
     __builtin_amdgcn_s_barrier();
-    const uint16_t* ws = smem + (kt % NSTAGE) * STAGE;
+    const uint16_t* ws = stages + (kt % NSTAGE) * STAGE;
     if (kt + NSTAGE - 1 < nk) issue(kt + NSTAGE - 1, (kt + NSTAGE - 1) % NSTAGE);
     if constexpr (KSS == 2) {
       // k-step 0's fragments first; then its MFMAs with k-step 1's reads interleaved
@@ -221,13 +236,36 @@ __global__ void __launch_bounds__(64 * WN * WM) skinny_gemm_kernel(SkinnyGemmPar
   }
   sk_wait_vm<0>();   // no DMA may still target this CU's LDS when the workgroup ends
 
+  if constexpr (KG > 1) {
+    // group g finishes token tiles [g MTW / KG, (g + 1) MTW / KG): the others lay theirs down for it
+    __builtin_amdgcn_s_barrier();   // every stage is read, no DMA is under way
+    constexpr int MO = MTW / KG;
+    f32x4* const sums = reinterpret_cast<f32x4*>(smem);   // [KG][MTW][NTW][NW][64]
+    static_assert(KG * MTW * NTW * NW * 64 * 16 <= KG * NSTAGE * STAGE * 2, "sums fit the stages");
+#pragma unroll
+    for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NTW; ++nt)
+        if (mt / MO != kg) sums[(((kg * MTW + mt) * NTW + nt) * NW + wv) * 64 + lane] = acc[nt][mt];
+    __syncthreads();
+#pragma unroll
+    for (int mt = 0; mt < MTW; ++mt) {
+      if (mt / MO != kg) continue;
+#pragma unroll
+      for (int nt = 0; nt < NTW; ++nt)
+#pragma unroll
+        for (int g = 0; g < KG; ++g)
+          if (g != kg) acc[nt][mt] += sums[(((g * MTW + mt) * NTW + nt) * NW + wv) * 64 + lane];
+    }
+  }
+
   // epilogue: acc[nt][mt][r] = out[token (16-tile mt, col)][feature (16-tile nt, 4h + r)]
   const int t_base = mi * BM + wm * CW;
   const int n_base = nb * BN + wn * RW;
 #pragma unroll
   for (int mt = 0; mt < MTW; ++mt) {
     const int t = t_base + mt * 16 + col;
-    if (t >= P.M) continue;
+    if (t >= P.M || (KG > 1 && mt / (MTW / KG) != kg)) continue;
     if constexpr (EPI == 0 || EPI == 3 || EPI == 4) {
       uint16_t* op = reinterpret_cast<uint16_t*>(P.out) + (int64_t)t * P.ldo;
 #pragma unroll
@@ -238,7 +276,7 @@ __global__ void __launch_bounds__(64 * WN * WM) skinny_gemm_kernel(SkinnyGemmPar
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           float y = acc[nt][mt][r];
-          if constexpr (EPI >= 3) y += bf2f(P.bias[n + r]);
+          if constexpr (EPI >= 3) y += bf2f(bias[nt][r]);
           if constexpr (EPI == 4) y = sk_gelu(y);
           v[r] = f2bf(y);
         }
@@ -443,35 +481,43 @@ void launch_skinny_gemm(const SkinnyGemmParams& p, int cfg, int epi, hipStream_t
 #undef NGA_LAUNCH
 }
 
-// Encoder projections (K 384 to 4,096): 64 x 64 tiles up to 512 rows, 64 x 128 above. BERT-large, weights from HBM (us,
-// library / here): 64 rows q/k/v 11.4 / 7.6, output 8.4 / 4.1, up 11.6 / 7.7, down 14.8 / 7.5; 512 rows 10.8 / 10.3, 8.5 / 5.6,
-// 10.6 / 10.2, 13.8 / 11.6; 1,024 rows 14.1 / 13.8, 9.5 / 7.9, 13.6 / 14.1 (and its GELU launch of 4.6 saved), 18.9 / 17.3; at
+// Encoder projections (K 384 to 4,096): 64 x 64 tiles up to 512 rows, 64 x 128 above; 32 features a tile where 64 would take half
+// the CUs or fewer, since a CU draws some 47 bytes a nanosecond from its L2 and these are bound by that (BERT-large, 64 rows: the
+// forward 1,100 us with 64, 990 with 32; 128 rows 1,124 and 1,010). Two groups of waves where each workgroup has a CU of its own
+// (208 rows: up 12.1 us with one, 10.2 with two; q/k/v 9.8 and 9.0); not for the slabs, whose K range is short (6.9 and 7.3).
+// A rotated walk over K (krot) lost 5 %: tiles that share rows no longer read them together. With 64-feature tiles and one group,
+// weights from HBM (us, library / here): 64 rows q/k/v 11.4 / 7.6, output 8.4 / 4.1, up 11.6 / 7.7, down 14.8 / 7.5; 512 rows
+// 10.8 / 10.3, 8.5 / 5.6, 10.6 / 10.2, 13.8 / 11.6; 1,024 rows 14.1 / 13.8, 9.5 / 7.9, 13.6 / 14.1 (and its GELU launch of 4.6 saved), 18.9 / 17.3; at
 // 1,536 rows the library's larger tiles win everywhere.
-static int skinny_tile(SkinnyGemmParams& p) {
-  const bool small = p.M <= 512;
-  p.nN = (p.N + 63) / 64;
-  p.nM = (p.M + (small ? 63 : 127)) / (small ? 64 : 128);
+static int skinny_tile(SkinnyGemmParams& p, int* bn) {
+  const int bm = p.M <= 512 ? 64 : 128;
+  p.nM = (p.M + bm - 1) / bm;
+  *bn = p.M <= 512 && (p.N + 63) / 64 * p.nM * p.split <= 128 ? 32 : 64;
+  p.nN = (p.N + *bn - 1) / *bn;
   return p.nN * p.nM * p.split;
 }
 
 void launch_skinny_bias(SkinnyGemmParams p, bool gelu, hipStream_t stream) {
   p.split = 1;
-  const int nblk = skinny_tile(p);
+  int bn;
+  const int nblk = skinny_tile(p, &bn);
   if (nblk == 0) return;
-  if (p.M <= 512) {
-    if (gelu) skinny_gemm_kernel<64, 64, 2, 2, 4, 4, 64><<<nblk, 256, 0, stream>>>(p);
-    else skinny_gemm_kernel<64, 64, 2, 2, 4, 3, 64><<<nblk, 256, 0, stream>>>(p);
-  } else {
-    if (gelu) skinny_gemm_kernel<64, 128, 1, 4, 3, 4, 64><<<nblk, 256, 0, stream>>>(p);
-    else skinny_gemm_kernel<64, 128, 1, 4, 3, 3, 64><<<nblk, 256, 0, stream>>>(p);
-  }
+#define NGA_SB(EPI)                                                                                        \
+  if (p.M > 512) skinny_gemm_kernel<64, 128, 1, 4, 3, EPI, 64><<<nblk, 256, 0, stream>>>(p);               \
+  else if (bn == 32) skinny_gemm_kernel<32, 64, 2, 2, 4, EPI, 64, 2><<<nblk, 512, 0, stream>>>(p);         \
+  else if (nblk <= 256) skinny_gemm_kernel<64, 64, 2, 2, 4, EPI, 64, 2><<<nblk, 512, 0, stream>>>(p);      \
+  else skinny_gemm_kernel<64, 64, 2, 2, 4, EPI, 64><<<nblk, 256, 0, stream>>>(p)
+  if (gelu) { NGA_SB(4); } else { NGA_SB(3); }
+#undef NGA_SB
 }
 
 void launch_skinny_slabs(SkinnyGemmParams p, hipStream_t stream) {
-  const int nblk = skinny_tile(p);
+  int bn;
+  const int nblk = skinny_tile(p, &bn);
   if (nblk == 0) return;
-  if (p.M <= 512) skinny_gemm_kernel<64, 64, 2, 2, 4, 1, 64><<<nblk, 256, 0, stream>>>(p);
-  else skinny_gemm_kernel<64, 128, 1, 4, 3, 1, 64><<<nblk, 256, 0, stream>>>(p);
+  if (p.M > 512) skinny_gemm_kernel<64, 128, 1, 4, 3, 1, 64><<<nblk, 256, 0, stream>>>(p);
+  else if (bn == 32) skinny_gemm_kernel<32, 64, 2, 2, 4, 1, 64><<<nblk, 256, 0, stream>>>(p);
+  else skinny_gemm_kernel<64, 64, 2, 2, 4, 1, 64><<<nblk, 256, 0, stream>>>(p);
 }
 
 void launch_splitk_reduce(const float* P, int S, int M, int N, uint16_t* out, int64_t ldo,

@@ -1,4 +1,5 @@
-"""Encoder forwards of up to 32 rows, whose norms and attention lie inside the projections."""
+"""Encoder forwards of few rows: up to 32 with the attention of one sequence inside a projection, above them LDS tiles of 32 and 64
+features, with one group of waves and two."""
 import pytest
 import torch
 
@@ -28,7 +29,8 @@ def _exact(m, ids, cu):
 
 
 @pytest.mark.parametrize("H,heads,F", [(128, 2, 256), (192, 6, 448), (384, 12, 1536), (768, 12, 3072), (1024, 16, 4096), (1024, 8, 8192)])
-@pytest.mark.parametrize("lens", [[1], [5], [16], [17], [19], [32], [3, 1, 20], [32, 0]])
+@pytest.mark.parametrize("lens", [[1], [5], [16], [17], [19], [32], [3, 1, 20], [32, 0], [33], [64, 1],
+                                  [60, 64, 9], [50] * 5, [64] * 5])
 def test_rows_forward(gpu, H, heads, F, lens):
     """Head sizes 32, 64 and 128, K ranges that the waves share unevenly, one tile of rows and two, one sequence and several.
     Against 64 bits, beside the same layers step by step: their roundings to bf16 are the same but for the sums before the
