@@ -953,18 +953,82 @@ Tensor gelu_rows(Tensor z, c10::optional<Tensor> dh) {
   return out;
 }
 
-// column sums of bf16 rows in fp32
+// column sums of bf16 rows, added up in fp32
 Tensor col_sums(Tensor x) {
   CHECK_BF16(x);
   TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.size(1) % 8 == 0 &&
                   reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0, "col_sums: rows at 16-byte addresses");
   const int64_t R = x.size(0), F = x.size(1);
   const auto f = x.options().dtype(at::kFloat);
-  if (R == 0 || F == 0) return at::zeros({F}, f);
-  Tensor part = at::empty({nga::train_col_parts(R, (int)F), F}, f), out = at::empty({F}, f);
-  nga::launch_col_sums(bfp(x), x.stride(0), R, (int)F, part.data_ptr<float>(), out.data_ptr<float>(), cur_stream(x));
+  if (R == 0 || F == 0) return at::zeros({F}, x.options());
+  Tensor part = at::empty({nga::train_col_parts(R, (int)F), F}, f), out = at::empty({F}, x.options());
+  nga::launch_col_sums(bfp(x), x.stride(0), R, (int)F, part.data_ptr<float>(), bfp(out), cur_stream(x));
   post_launch("col_sums");
   return out;
+}
+
+template <typename F>
+void cast_tables(const std::vector<Tensor>& f, const std::vector<Tensor>& a, const std::vector<c10::optional<Tensor>>& b, F fn) {
+  nga::CastTable t;
+  t.n = 0;
+  t.first[0] = 0;
+  auto out = [&] {
+    if (t.n) fn(t);
+    t.n = 0;
+  };
+  for (size_t i = 0; i < f.size(); ++i) {
+    const int64_t n = f[i].numel(), chunks = (n + nga::CAST_CHUNK - 1) / nga::CAST_CHUNK;
+    if (n == 0) continue;
+    TORCH_CHECK(chunks < (1 << 30), "half copies: tensor too large");
+    if (t.n == nga::CAST_TENSORS || (t.n && t.first[t.n] + chunks > (1 << 30))) out();
+    t.len[t.n] = n;
+    t.f[t.n] = f[i].data_ptr<float>();
+    t.a[t.n] = bfp(a[i]);
+    t.b[t.n] = i < b.size() && b[i].has_value() ? bfp(*b[i]) : nullptr;
+    t.first[t.n + 1] = t.first[t.n] + (int)chunks;
+    ++t.n;
+  }
+  out();
+}
+
+// bf16 copies of fp32 tensors
+std::vector<Tensor> half_copies(std::vector<Tensor> f) {
+  std::vector<Tensor> a;
+  for (const Tensor& x : f) {
+    CHECK_F32(x); CHECK_CONTIG(x);
+    TORCH_CHECK(x.device() == f[0].device() && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0, "half_copies: one device, 16-byte addresses");
+    a.push_back(at::empty(x.sizes(), x.options().dtype(at::kBFloat16)));
+  }
+  if (f.empty()) return a;
+  const hipStream_t st = cur_stream(f[0]);
+  cast_tables(f, a, {}, [&](const nga::CastTable& t) { nga::launch_half_copies(t, st); });
+  post_launch("half_copies");
+  return a;
+}
+
+// a + b of bf16 tensors in fp32, b[i] none: a[i]
+std::vector<Tensor> half_grads(std::vector<Tensor> a, std::vector<c10::optional<Tensor>> b) {
+  TORCH_CHECK(a.size() == b.size(), "half_grads: as many tensors");
+  std::vector<Tensor> f;
+  auto plain = [&](Tensor& x) {
+    CHECK_BF16(x);
+    TORCH_CHECK(x.device() == a[0].device(), "half_grads: one device");
+    x = x.contiguous();
+    if (reinterpret_cast<uintptr_t>(x.data_ptr()) % 16) x = x.clone();
+  };
+  for (size_t i = 0; i < a.size(); ++i) {
+    plain(a[i]);
+    if (b[i].has_value()) {
+      TORCH_CHECK(b[i]->sizes() == a[i].sizes(), "half_grads: one shape");
+      plain(*b[i]);
+    }
+    f.push_back(at::empty(a[i].sizes(), a[i].options().dtype(at::kFloat)));
+  }
+  if (a.empty()) return f;
+  const hipStream_t st = cur_stream(a[0]);
+  cast_tables(f, a, b, [&](const nga::CastTable& t) { nga::launch_half_grads(t, st); });
+  post_launch("half_grads");
+  return f;
 }
 
 // silu(gate) up of [gate | up] rows, or the gradient of those for dh
@@ -2807,6 +2871,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("ln_sums", on_device(&ln_sums));
   m.def("gelu_rows", on_device(&gelu_rows));
   m.def("col_sums", on_device(&col_sums));
+  m.def("half_copies", on_device(&half_copies));
+  m.def("half_grads", on_device(&half_grads));
   m.def("swiglu_rows", on_device(&swiglu_rows));
   m.def("add_scaled", on_device(&add_scaled));
   m.def("rope_rows", on_device(&rope_rows));

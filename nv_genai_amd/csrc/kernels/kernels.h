@@ -253,7 +253,19 @@ void launch_add_f32(const uint16_t* x, const uint16_t* o, int64_t n, float* s, h
 void launch_ln_sums(const float* s, const float* mean, const float* rstd, const uint16_t* dy, int64_t R, int H, float* part,
                     float* sums, hipStream_t st);
 void launch_gelu(const uint16_t* z, const uint16_t* dh, int64_t n, uint16_t* out, hipStream_t st);
-void launch_col_sums(const uint16_t* x, int64_t ld, int64_t R, int F, float* part, float* out, hipStream_t st);
+void launch_col_sums(const uint16_t* x, int64_t ld, int64_t R, int F, float* part, uint16_t* out, hipStream_t st);
+// tensors of one launch by value, a workgroup takes CAST_CHUNK elements of one; all at 16-byte addresses
+constexpr int CAST_TENSORS = 64;
+constexpr int CAST_CHUNK = 8192;
+struct CastTable {
+  int n;
+  int first[CAST_TENSORS + 1];   // first chunk of each tensor; [n]: their count
+  int64_t len[CAST_TENSORS];
+  float* f[CAST_TENSORS];
+  uint16_t *a[CAST_TENSORS], *b[CAST_TENSORS];
+};
+void launch_half_copies(const CastTable& t, hipStream_t st);   // a = bf16(f)
+void launch_half_grads(const CastTable& t, hipStream_t st);    // f = a + b (b may be null)
 void launch_swiglu(const uint16_t* gu, const uint16_t* dh, int64_t R, int F, uint16_t* out, hipStream_t st);
 void launch_add_scaled(const uint16_t* d, float scale, int64_t n, uint16_t* y, hipStream_t st);
 void launch_rope_rows(const uint16_t* in, const float* cs, int64_t T, int64_t P, int nr, int nh, int D, float sign, uint16_t* out,

@@ -83,8 +83,9 @@ def embed_trainer(engine, records: Sequence[dict], cfg: TrainConfig, hard_negati
     def loss_fn(mb):
         qi, qm, pi, pm = (t.to(dev) for t in mb)
         with torch.autocast(dev.type, dtype=torch.bfloat16):
-            q = Fn.encoder_embed(model, qi, qm, params, cfg.grad_ckpt)
-            p = Fn.encoder_embed(model, pi, pm, params, cfg.grad_ckpt)
+            for_q, for_p = Fn.half_params(params)
+            q = Fn.encoder_embed(model, qi, qm, for_q, cfg.grad_ckpt)
+            p = Fn.encoder_embed(model, pi, pm, for_p, cfg.grad_ckpt)
         return contrastive_loss(q, p, 1 + hard_negatives, scale)
 
     return Trainer(named, loss_fn, batches, cfg, group, ckpt_dir), params

@@ -26,7 +26,7 @@ Reference behaviour: NeMo Megatron GPT SFT/LoRA (models/Gemma/lora.ipynb, sft.ip
 """
 from __future__ import annotations
 
-from typing import Callable, Dict, Optional
+from typing import Callable, Dict, List, Optional
 
 import torch
 import torch.nn.functional as F
@@ -281,6 +281,25 @@ def trainable_params(model, kind: str = "llama") -> Dict:
             for n, t in L.items():
                 out[(li, n)] = t
     return {k: v.detach().float().clone().requires_grad_(True) for k, v in out.items()}
+
+
+# what the encoder's forward takes in bf16 and no other type
+_HALF = ("wqkv", "bqkv", "wo", "bo", "wi", "bi", "wo2", "bo2")
+
+
+def half_params(params: Dict) -> List[Dict]:
+    """An encoder's ``params`` for each of the two passes of a step (questions and passages), with the layers' projections in
+    bf16, cast once for both and a layer at a time, so that a layer's gradients are there when its backward is done. Where the
+    kernel does not take them, or under a mode that watches the operations, they are ``params``, which the passes cast
+    themselves. One pass alone has nothing to share: a small decoder's step took 19.0 ms with and without."""
+    out = [dict(params), dict(params)]
+    for li in sorted({k[0] for k in params if isinstance(k, tuple)}):
+        keys = [(li, n) for n in _HALF if (li, n) in params]
+        masters = [params[k] for k in keys]
+        if fused.half_copies_usable(masters):
+            for p, got in zip(out, fused.half_copies(masters)):
+                p.update(zip(keys, got))
+    return out
 
 
 def write_back(model, params: Dict, kind: str = "llama") -> None:

@@ -12,7 +12,7 @@ stands for, has a first derivative only.
 from __future__ import annotations
 
 import math
-from typing import Optional, Tuple
+from typing import Optional, Sequence, Tuple
 
 import torch
 from torch.autograd import Function
@@ -39,7 +39,11 @@ def _plain(t: torch.Tensor) -> bool:
 def _takes(x: torch.Tensor) -> bool:
     """bf16 rows on the GPU, nothing active that these functions would pass by, and no autocast to another type: the torch
     operations between them would change the rows' type."""
-    return (x.is_cuda and x.dtype is BF16 and x.numel() > 0 and _plain(x) and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+    return x.is_cuda and x.dtype is BF16 and x.numel() > 0 and _plain(x) and _undisturbed()
+
+
+def _undisturbed() -> bool:
+    return (not torch.jit.is_tracing() and not torch.compiler.is_compiling()
             and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
             and not torch._C._len_torch_dispatch_stack()   # make_fx and other modes that watch the operations
             and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") is BF16))
@@ -73,13 +77,44 @@ class _Linear(Function):
         dy2 = _rows(dy.reshape(-1, dy.shape[-1]))
         dx = (dy2 @ w).view(x.shape) if ctx.needs_input_grad[0] else None
         dw = dy2.t() @ x.reshape(-1, x.shape[-1]) if ctx.needs_input_grad[1] else None
-        db = ops.kernels().col_sums(dy2).to(BF16) if ctx.needs_input_grad[2] else None
+        db = ops.kernels().col_sums(dy2) if ctx.needs_input_grad[2] else None
         return dx, dw, db
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """x w^T + b in bf16, w's and b's gradients in their own type (w.shape[0] % 8 == 0)."""
     return _Linear.apply(x, w.to(BF16), b.to(BF16))
+
+
+class _HalfCopies(Function):
+    @staticmethod
+    def forward(ctx, *masters):
+        ctx.set_materialize_grads(False)
+        out = ops.kernels().half_copies(masters)
+        return (*out, *(t.detach() for t in out))
+
+    @staticmethod
+    def backward(ctx, *grads):
+        n = len(ctx.needs_input_grad)
+        two = [[g for g in grads[i::n] if g is not None] if ctx.needs_input_grad[i] else [] for i in range(n)]
+        if torch.is_grad_enabled():
+            return tuple(sum(g.float() for g in gs) if gs else None for gs in two)
+        live = [gs for gs in two if gs]
+        got = iter(ops.kernels().half_grads([gs[0] for gs in live], [gs[1] if len(gs) > 1 else None for gs in live]) if live else ())
+        return tuple(next(got) if gs else None for gs in two)
+
+
+def half_copies(masters: Sequence[torch.Tensor]) -> Tuple[Tuple[torch.Tensor, ...], Tuple[torch.Tensor, ...]]:
+    """bf16 copies of fp32 masters for two forward passes, a tuple for each: the same values, whose gradients (bf16 each) are
+    added up in fp32."""
+    out = _HalfCopies.apply(*masters)
+    return out[:len(masters)], out[len(masters):]
+
+
+def half_copies_usable(masters: Sequence[torch.Tensor]) -> bool:
+    return len(masters) > 0 and _undisturbed() and all(
+        t.is_cuda and t.dtype is torch.float32 and t.device == masters[0].device and t.is_contiguous() and t.data_ptr() % 16 == 0
+        and _plain(t) for t in masters)
 
 
 class _AddRmsNorm(Function):

@@ -261,3 +261,43 @@ def test_encoder_embed_matches_torch_operations(gpu, monkeypatch, pooling, ckpt)
         # the key bias has no gradient in exact arithmetic: what either side has of it is rounding
         p, q = (t[k] if k[1] != "bqkv" else torch.cat([t[k][: m.cfg.hidden], t[k][2 * m.cfg.hidden:]]) for t in (ga, gb))
         assert _rel(p, q) < 4e-3, (k, _rel(p, q))
+
+
+# one element, tails of a chunk and of eight, more tensors than a launch takes; both passes use all of them, or one leaves one out
+@pytest.mark.parametrize("skip", [None, 1])
+def test_half_copies_keep_every_bit(gpu, skip):
+    shapes = [(1,), (7, 3), (8192,), (8193,), (3, 8190)] + [(5,)] * 70
+    m = [torch.randn(s, device=gpu).mul_(3).requires_grad_() for s in shapes]
+    assert fused.half_copies_usable(m)
+    got, ref = fused.half_copies(m), [[t.to(BF) for t in m] for _ in range(2)]
+    dy = [[torch.randn(s, device=gpu).to(BF) for s in shapes] for _ in range(2)]
+    sums = []
+    for use in (got, ref):
+        sums.append(sum((y * d).float().sum() for u in range(2) for i, (y, d) in enumerate(zip(use[u], dy[u])) if not (u == 1 and i == skip)))
+    for a, b in zip(got, ref):
+        assert all(torch.equal(p, q) for p, q in zip(a, b))
+    for create in (False, True):
+        ga, gb = (torch.autograd.grad(s, m, retain_graph=True, create_graph=create) for s in sums)
+        assert all(p.dtype == torch.float32 and torch.equal(p, q) for p, q in zip(ga, gb))
+
+
+def test_half_params_keep_the_gradients(gpu):
+    """A step of both passes over shared copies against each pass casting for itself."""
+    from nv_genai_amd.models.config import encoder_config
+    from nv_genai_amd.models.encoder import EncoderModel
+
+    m = EncoderModel(encoder_config("encoder-tiny"), gpu, seed=2)
+    ids = torch.randint(0, 1000, (3, 40), device=gpu)
+    got = []
+    for shared in (True, False):
+        P = Fn.trainable_params(m, "encoder")
+        with torch.autocast("cuda", dtype=BF):
+            a, b = Fn.half_params(P) if shared else (P, P)
+            assert (a[(0, "wo")].dtype is BF) == shared
+            y = (Fn.encoder_embed(m, ids, torch.ones_like(ids), a) * Fn.encoder_embed(m, ids[:, :9], torch.ones_like(ids[:, :9]), b)).pow(3).sum()
+        y.backward()
+        got.append((y.detach(), {k: v.grad for k, v in P.items()}))
+    (ya, ga), (yb, gb) = got
+    assert torch.equal(ya, yb)
+    for k in gb:
+        assert torch.equal(ga[k], gb[k]), k
