@@ -601,10 +601,10 @@ void decode_attention(Tensor out, Tensor q, Tensor kc, Tensor vc, Tensor block_t
 
 // Attention of a decode step: q | k | v of one new token a row (bf16 [B, (Hq + 2 Hkv) 128], or fp32 K-split slabs [S, B, ..])
 // are rotated, written to the cache at `slots` (the slots of places ctx - 1; -1: not written) and attended to. `done` int32
-// zeros [>= B Hkv], given back as zeros.
+// zeros [>= B Hkv], given back as zeros. next: the weights of the projection behind it, which CUs without keys read ahead.
 void decode_step(Tensor out, Tensor qkv, Tensor pos, Tensor cos_sin, Tensor slots, Tensor kc, Tensor vc, Tensor block_tables,
                  Tensor ctx_lens, int64_t Hq, int64_t Hkv, int64_t max_ctx, double scale, int64_t pages_per_part,
-                 Tensor part_ml, Tensor part_o, Tensor done, int64_t window) {
+                 Tensor part_ml, Tensor part_o, Tensor done, int64_t window, c10::optional<Tensor> next) {
   CHECK_BF16(out); CHECK_BF16(kc); CHECK_BF16(vc);
   CHECK_DEV(qkv); CHECK_CONTIG(qkv); CHECK_CONTIG(kc); CHECK_CONTIG(vc);
   CHECK_DEV(pos); CHECK_DT(pos, at::kInt); CHECK_CONTIG(pos);
@@ -643,6 +643,14 @@ void decode_step(Tensor out, Tensor qkv, Tensor pos, Tensor cos_sin, Tensor slot
   st.kc = bfp(kc);
   st.vc = bfp(vc);
   st.done = done.data_ptr<int32_t>();
+  // a hint only: weights in another form are not read ahead
+  if (next.has_value() && next->device() == qkv.device() && next->scalar_type() == at::kBFloat16 && next->dim() == 2 && next->is_contiguous() &&
+      next->size(1) % 128 == 0 && next->size(1) < (1 << 20) && next->size(0) % 16 == 0 && next->numel() <= (int64_t(1) << 26) &&
+      reinterpret_cast<uintptr_t>(next->data_ptr()) % 16 == 0) {
+    st.next = bfp(*next);
+    st.next_pieces = (int)(next->size(0) / 16);
+    st.next_kb = (int)(next->size(1) / 128);
+  }
   nga::launch_decode_step(bfp(out), out.stride(0), slabs ? nullptr : bfp(qkv), st, block_tables.data_ptr<int32_t>(),
                           (int)block_tables.size(1), ctx_lens.data_ptr<int32_t>(), (int)B, (int)Hq, (int)Hkv, (int)max_ctx,
                           (float)scale, (int)pages_per_part, nparts > 1 ? part_ml.data_ptr<float>() : nullptr,

@@ -314,6 +314,21 @@ __device__ __forceinline__ float get_agent(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A workgroup without keys reads its share of the weights that the next launch streams, so that these come from the caches:
+// for short contexts most CUs have no keys (one sequence of 227 tokens: 8 of 128 workgroups) and HBM would lie idle while the
+// others wait for their first bytes. Piece t, the rows of the next kernel's workgroup t, goes to the die that will run that.
+// What the loads bring into LDS is never looked at. 8B, one sequence of 227 tokens: output projection (33.5 MB) 7.9 -> 5.4 us, attention
+// 8.5 -> 9.2; where all partitions have keys nothing is read ahead.
+__device__ __forceinline__ void warm_next(const DecodeStep& st, uint16_t* lds, int w, int lane) {
+  const int total = gridDim.x * gridDim.y * gridDim.z, id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+  const int die = id & 7, n = (total - die + 7) >> 3, blocks = ((st.next_pieces - die + 7) >> 3) * st.next_kb;
+  for (int k = id >> 3; k < blocks; k += n) {
+    const int piece = die + 8 * (k / st.next_kb);
+    glds16(st.next + ((int64_t)piece * st.next_kb + k % st.next_kb) * 2048 + w * 512 + lane * 8, lds);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the LDS is another workgroup's after this one's end
+}
+
 // STEP = true: the whole attention of a decode step in this one launch. The workgroup takes its
 // query rows from the projection's output (bf16, or its fp32 K-split slabs) and rotates them; the
 // one whose partition ends the sequence rotates the new key too, lays the new key and value over
@@ -355,6 +370,7 @@ __global__ void __launch_bounds__(256, 1) decode_attn_dma_kernel(
       if (active == 0 && part == 0)
         for (int i = threadIdx.x; i < G * D; i += blockDim.x)
           out[(int64_t)b * out_stride + (int64_t)(kvh * G) * D + i] = 0;
+      if (st.next != nullptr) warm_next(st, smem + w * 512, w, lane);
     } else if (nparts == 1) {
       for (int i = threadIdx.x; i < G * D; i += blockDim.x)
         out[(int64_t)b * out_stride + (int64_t)(kvh * G) * D + i] = 0;

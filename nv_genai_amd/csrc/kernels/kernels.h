@@ -74,6 +74,8 @@ struct DecodeStep {
   uint16_t* kc;
   uint16_t* vc;
   int32_t* done;           // [rows, Hkv] partitions that have finished; zero before and after every launch
+  const uint16_t* next;    // weights that the next launch reads, in pieces of next_kb 4-KiB blocks, or null
+  int next_pieces, next_kb;
 };
 bool decode_step_covers(int num_seqs, int max_ctx, int pages_per_part, int window);
 void launch_decode_step(uint16_t* out, int64_t out_stride, const uint16_t* qkv, const DecodeStep& st,

@@ -656,7 +656,7 @@ class LlamaModel:
         if meta.kind == "decode" and ops.decode_step_covers(qkv, self.k_cache[li], meta.ctx_lens, meta.slots, meta.max_ctx,
                                                             meta.decode_ws, self.window):
             return ops.decode_step(qkv, pos, self.cos_sin, meta.slots, self.k_cache[li], self.v_cache[li], meta.block_tables,
-                                   meta.ctx_lens, self.hq, self.hkv, meta.max_ctx, self.scale, meta.decode_ws, self.window)
+                                   meta.ctx_lens, self.hq, self.hkv, meta.max_ctx, self.scale, meta.decode_ws, self.window, self.layers[li].get("wo"))
         part = None
         if isinstance(qkv, ops.PartialSum):   # K-split projection: the RoPE kernel sums the slabs
             part = qkv

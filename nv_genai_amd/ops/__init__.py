@@ -1221,14 +1221,15 @@ def decode_step_covers(qkv, kc, ctx_lens, slots, max_ctx, ws: Optional[DecodeWor
 
 
 def decode_step(qkv, pos, cos_sin, slots, kc, vc, block_tables, ctx_lens, Hq, Hkv, max_ctx, scale, ws: DecodeWorkspace,
-                window: int = 0):
+                window: int = 0, next_w: Optional[torch.Tensor] = None):
     """:func:`rope_cache_` and :func:`decode_attention` of one new token a row in one launch. ``qkv``: the projection's bf16
-    rows or its :class:`PartialSum`; ``slots``: the cache slots of places ``ctx_lens - 1`` (-1: not written)."""
+    rows or its :class:`PartialSum`; ``slots``: the cache slots of places ``ctx_lens - 1`` (-1: not written); ``next_w``: the
+    weights that the next launch reads, for CUs without keys to bring into the caches."""
     t = qkv.slabs if isinstance(qkv, PartialSum) else qkv
     B = ctx_lens.numel()
     out = torch.empty(B, Hq * 128, dtype=kc.dtype, device=kc.device)
     kernels().decode_step(out, t, pos, cos_sin, slots, kc, vc, block_tables, ctx_lens, Hq, Hkv, int(max_ctx), float(scale),
-                          ws.pages_per_part(B, max_ctx), ws.ml, ws.o, ws.done, int(window))
+                          ws.pages_per_part(B, max_ctx), ws.ml, ws.o, ws.done, int(window), next_w)
     return out
 
 

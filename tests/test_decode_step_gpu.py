@@ -54,8 +54,9 @@ def test_decode_step_is_rotation_and_attention(gpu, G, Hkv, ppp, window, slabs):
     ops.rope_cache_(flat, pos, cs, slots, k1, v1, Hq, Hkv, D)
     want = ops.decode_attention(flat[:, : Hq * D], k1, v1, bt, ctx, Hq, Hkv, most, scale, ws=ws, window=window)
     assert ops.decode_step_covers(qkv, k2, ctx, slots, most, ws, window)
-    for _ in range(2):   # the counters are zero again after a launch
-        got = ops.decode_step(qkv, pos, cs, slots, k2, v2, bt, ctx, Hq, Hkv, most, scale, ws, window)
+    for k in (128, 4096):   # the counters are zero again after a launch; weights to read ahead of one and of many blocks a piece
+        nxt = torch.empty(16 * 37, k, dtype=torch.bfloat16, device=dev)
+        got = ops.decode_step(qkv, pos, cs, slots, k2, v2, bt, ctx, Hq, Hkv, most, scale, ws, window, nxt)
         assert torch.equal(k1, k2) and torch.equal(v1, v2)
         assert not ws.done.any()
         w, g = want.float(), got.float()
