@@ -1502,8 +1502,9 @@ std::vector<Tensor> flat_search(Tensor q, Tensor X, Tensor bias, Tensor ids, dou
   const int64_t nq = q.size(0), N = X.size(0);
   const int D = (int)X.size(1), ng = nq <= 16 ? 1 : nq <= 32 ? 2 : nq <= 48 ? 3 : 4;
   const int items = (int)((nq + 16 * ng - 1) / (16 * ng)), K = nga::scan_list((int)k, ng, false);
-  const int blocks = nga::scan_blocks(D, ng, (int)cus);
-  const int64_t tiles = (N + 127) / 128;
+  const bool wide = nga::scan_wide_covers(D, ng);
+  const int blocks = wide ? (int)cus : nga::scan_blocks(D, ng, (int)cus);
+  const int64_t tiles = wide ? (N + 31) / 32 : (N + 127) / 128;
   const int parts = (int)std::min<int64_t>(std::max(1, blocks / items), tiles);
   constexpr int64_t SEG = 8192;
   const int64_t nseg = (N + SEG - 1) / SEG, cap = (K ? parts : nseg) * k;
@@ -1522,7 +1523,8 @@ std::vector<Tensor> flat_search(Tensor q, Tensor X, Tensor bias, Tensor ids, dou
     S = at::empty({nq, s.a.s_stride}, X.options().dtype(at::kFloat));
     s.a.S = S.data_ptr<float>();
   }
-  nga::launch_scan(s.a, ng, K, items * parts, s.st);
+  if (wide) nga::launch_scan_wide(s.a, ng, K, items * parts, s.st);
+  else nga::launch_scan(s.a, ng, K, items * parts, s.st);
   if (K == 0)
     nga::launch_select_segments(s.a.S, s.a.s_stride, (int)nq, N, SEG, (int)k, s.a.cap, s.a.cand_v, s.a.cand_r, s.st);
   return search_end(s, q, ids, (int32_t)cap, "flat_search");

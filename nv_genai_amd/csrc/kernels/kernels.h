@@ -206,6 +206,8 @@ int scan_chunk(int D, int ng);                  // dims of a unit of work, 0: no
 int scan_blocks(int D, int ng, int cus);        // workgroups that fill the chip
 int scan_list(int k, int ng, bool ivf);         // length of the register lists, 0: scores to S
 void launch_scan(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream);
+bool scan_wide_covers(int D, int ng);           // flat scans of more than 16 queries
+void launch_scan_wide(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream);
 void launch_search_prep(const float* q, int64_t q_stride, int nq, int D, int metric, uint16_t* qb, hipStream_t stream);
 void launch_ivf_probe(const float* q, int64_t q_stride, int nq, int D, int metric, const float* cent, int nlist, int nprobe,
                       uint16_t* qb, int32_t* cnt, int32_t* probes, hipStream_t stream);

@@ -236,9 +236,9 @@ __global__ void __launch_bounds__(1024) ivf_items_kernel(const int32_t* __restri
 // Per wave a 32-row x CH-dim LDS slot, filled by lane-linear LDS-DMA (1 KiB per instruction, non-temporal) and read
 // into registers as MFMA fragments; the next unit's DMA goes out before the MFMAs of this one. NG groups of 16 queries
 // lie in LDS beside the slots: one workgroup fills a CU at D 1,024. Bound by the stream of vectors: 6.6 TB/s at one
-// query (1M x 1024; whole search 312 us, 340 with the launches around it that are now in it). With 33 queries and k 25
-// (250k x 1024) 115 us, 4.5 TB/s, half the LDS being queries; reading MFMA fragments from HBM directly, 16 rows x 64 B an
-// instruction, took 187 us.
+// query (1M x 1024; whole search 312 us, 340 with the launches around it that are now in it). More queries of lists, or of
+// vectors that scan_wide_kernel below does not take, halve what is left of LDS for the stream (33 of them, 250k x 1,024: 4.5 TB/s);
+// reading MFMA fragments from HBM directly, 16 rows x 64 B an instruction, took 187 us.
 // K > 0: a register list of K per lane and group, merged over lanes and waves at the end of a run, and appended to the
 // query's candidates. K = 0 (more than 16 results of up to 32 queries, or 8 of up to 64): scores to S, since inserting
 // into longer lists costs more than the 4 bytes a score.
@@ -490,6 +490,203 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
   }
 }
 
+// Flat scan for 17 to 64 queries. Held in LDS they leave a wave half of it to stream through; here a wave holds a quarter of every
+// query in registers (NG x KS fragments), reads that quarter of every row, and the four waves add up in LDS, 32 rows at a time.
+// LDS is then a ring of NSL units (16 rows) a wave, which all stay under way. The sums are handed over in the accumulators'
+// layout, so that a lane ends with four rows of one query as in the other kernel; wave w takes rows 16 (w & 1) .. and every
+// second group of queries.
+namespace {
+constexpr int wide_slots(int KS, int NG) { return KS == 8 ? (NG == 4 ? 3 : 4) : KS == 6 ? 5 : 10; }   // of 4 KS KiB for all waves
+constexpr int wide_swizzle(int KS) { return KS % 4 == 0 ? 15 : KS % 2 == 0 ? 7 : 3; }
+constexpr int WIDE_BIAS = 8;   // tiles whose biases have a place, more than are under way
+template <int N>
+__device__ __forceinline__ void wide_wait() {
+  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// an accumulator to LDS while DMAs are under way (an ordinary store would wait for them); the compiler does not see that the
+// instruction reads an MFMA's result, which is there after 19 cycles
+__device__ __forceinline__ void wide_store(float* p, f32x4 v) {
+  asm volatile("s_nop 15\n\ts_nop 7\n\tds_write_b128 %0, %1" ::"v"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)p), "v"(v)
+               : "memory");
+}
+__device__ __forceinline__ void wide_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+}  // namespace
+
+static size_t wide_lds(int NG, int KS) { return (size_t)SS_W * wide_slots(KS, NG) * KS * 1024 + 8192 * NG + WIDE_BIAS * SS_W * 64; }
+
+template <int NG, int K, int KS>
+__global__ void __launch_bounds__(256, 1) scan_wide_kernel(ScanArgs p) {
+  constexpr int SL = 16 * NG, NSL = wide_slots(KS, NG), UNIT = 512 * KS, NC = 4 * KS, SW = wide_swizzle(KS), GW = (NG + 1) / 2;
+  constexpr int KR = K > 0 ? K : 1;
+  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+  float* const xch = reinterpret_cast<float*>(smem + SS_W * NSL * UNIT);
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, h = lane >> 4;
+  const int D = 128 * KS;
+  uint16_t* const ring = smem + w * NSL * UNIT;
+  float* const bias_s = xch + 2048 * NG + w * 16;   // [WIDE_BIAS][SS_W][16]
+  const int item = blockIdx.x / p.parts, part = blockIdx.x % p.parts;
+  const int nql = p.nq - item * SL < SL ? p.nq - item * SL : SL, ngrp = (nql + 15) / 16;
+  const int tiles = (int)((p.N + 31) / 32), nt = part < tiles ? (tiles - 1 - part) / p.parts + 1 : 0, units = 2 * nt;
+
+  bf16x8 bq[NG][KS];
+#pragma unroll
+  for (int g = 0; g < NG; ++g)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      u16x8 v = load8(p.Q + (int64_t)(item * SL + min(16 * g + col, nql - 1)) * D + w * (D / 4) + 32 * s + 8 * h);
+      bq[g][s] = as_bf16x8(16 * g + col < nql ? v : (u16x8)(0));
+    }
+  int off[KS], row[KS];   // of this lane's 16 bytes of instruction i: chunk c of row r lies at c ^ (r & SW)
+#pragma unroll
+  for (int i = 0; i < KS; ++i) {
+    const int li = 64 * i + lane;
+    row[i] = li / NC;
+    off[i] = w * (D / 4) + (((li % NC) ^ (row[i] & SW)) << 3);
+  }
+  auto issue = [&](int u, bool first) {   // first: of a tile, whose biases come before it
+    const int64_t rbase = (part + (int64_t)(u >> 1) * p.parts) * 32 + (u & 1) * 16;
+    if (first && lane < 16) {
+      const int64_t r = rbase + 16 * (w & 1) + lane;
+      __builtin_amdgcn_global_load_lds((gptr_t)(p.bias + (r < p.N ? r : p.N - 1)), (lptr_t)(bias_s + ((u >> 1) % WIDE_BIAS) * (SS_W * 16)), 4, 0, 0);
+    }
+    uint16_t* to = ring + (u % NSL) * UNIT;
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+      const int64_t r = rbase + row[i];
+      __builtin_amdgcn_global_load_lds((gptr_t)(p.X + (r < p.N ? r : p.N - 1) * D + off[i]), (lptr_t)(to + i * 512), 16, 0, 2);
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < NSL; ++u) issue(u, u % 2 == 0);
+  // the queries are used here, so that the compiler's wait for them lies before the loop
+#pragma unroll
+  for (int g = 0; g < NG; ++g)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(bq[g][s]));
+
+  float tv[GW][KR];
+  int tr[GW][KR];
+#pragma unroll
+  for (int g = 0; g < GW; ++g)
+#pragma unroll
+    for (int j = 0; j < KR; ++j) {
+      tv[g][j] = -INFINITY;
+      tr[g][j] = -1;
+    }
+  f32x4 acc[2][NG];
+  auto multiply = [&](int u, int i) {
+    const uint16_t* from = ring + (u % NSL) * UNIT + col * (NC * 8);
+    u16x8 a[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) a[s] = *reinterpret_cast<const u16x8*>(from + (((4 * s + h) ^ (col & SW)) << 3));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the unit's place is free
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) acc[i][g] = (f32x4)(0.f);
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int g = 0; g < NG; ++g) acc[i][g] = mfma16(as_bf16x8(a[s]), bq[g][s], acc[i][g]);
+  };
+  auto finish = [&](int n) {   // tile n of this workgroup
+    wide_barrier();   // the sums of the tile before have been read
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int g = 0; g < NG; ++g) wide_store(xch + (((w * 2 + i) * NG + g) * 64 + lane) * 4, acc[i][g]);
+    wide_barrier();
+    const int64_t rb = (part + (int64_t)n * p.parts) * 32 + 16 * (w & 1) + 4 * h;
+    const f32x4 b = *reinterpret_cast<const f32x4*>(bias_s + (n % WIDE_BIAS) * (SS_W * 16) + 4 * h);
+#pragma unroll
+    for (int gg = 0; gg < GW; ++gg) {
+      const int g = 2 * gg + (w >> 1);
+      if (g >= ngrp) continue;
+      f32x4 v = (f32x4)(0.f);
+#pragma unroll
+      for (int o = 0; o < SS_W; ++o) v += *reinterpret_cast<const f32x4*>(xch + (((o * 2 + (w & 1)) * NG + g) * 64 + lane) * 4);
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) v[rr] = v[rr] * p.dot_scale + b[rr];
+      if constexpr (K > 0) {
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr)
+          if (rb + rr < p.N && v[rr] > tv[gg][K - 1]) ss_insert<KR>(tv[gg], tr[gg], v[rr], (int)(rb + rr));
+      } else if (16 * g + col < nql) {
+        float* dst = p.S + (int64_t)(item * SL + 16 * g + col) * p.s_stride + rb;   // s_stride % 4 == 0
+        if (rb + 3 < p.N) {
+          *reinterpret_cast<f32x4*>(dst) = v;
+        } else {
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr)
+            if (rb + rr < p.N) dst[rr] = v[rr];
+        }
+      }
+    }
+  };
+  // younger than unit u when its turn comes: the NSL - 1 units behind it, a bias before each even one. Stores of scores are not
+  // counted: they may be done before older loads
+  constexpr int Y0 = (NSL - 1) * KS + (NSL - 1) / 2, Y1 = (NSL - 1) * KS + NSL / 2;
+  int n = 0;
+  for (; 2 * n + 1 + NSL < units; ++n) {
+    wide_wait<Y0>();
+    multiply(2 * n, 0);
+    issue(2 * n + NSL, NSL % 2 == 0);
+    wide_wait<Y1>();
+    multiply(2 * n + 1, 1);
+    issue(2 * n + 1 + NSL, NSL % 2 == 1);
+    finish(n);
+  }
+  for (; n < nt; ++n) {   // the last units: nothing more to ask for, but one unit if it is the ring's first place that is missing
+    wide_wait<0>();
+    multiply(2 * n, 0);
+    if (2 * n + NSL < units) issue(2 * n + NSL, NSL % 2 == 0);
+    multiply(2 * n + 1, 1);
+    finish(n);
+  }
+
+  if constexpr (K > 0) {
+#pragma unroll
+    for (int g = 0; g < GW; ++g) {
+      ss_merge_xor<KR>(tv[g], tr[g], 16);
+      ss_merge_xor<KR>(tv[g], tr[g], 32);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    float* mv = reinterpret_cast<float*>(smem);   // [SL][2][K]
+    int* mr = reinterpret_cast<int*>(mv + SL * 2 * K);
+    if (h == 0) {
+#pragma unroll
+      for (int gg = 0; gg < GW; ++gg) {
+        const int g = 2 * gg + (w >> 1);
+        if (g < NG) {
+#pragma unroll
+          for (int j = 0; j < K; ++j) {
+            mv[((16 * g + col) * 2 + (w & 1)) * K + j] = tv[gg][j];
+            mr[((16 * g + col) * 2 + (w & 1)) * K + j] = tr[gg][j];
+          }
+        }
+      }
+    }
+    __syncthreads();
+    if (tid < nql) {
+      const float* lv = mv + tid * 2 * K;
+      const int* lr = mr + tid * 2 * K;
+      int a = 0, b = 0;
+      const int64_t at = (int64_t)(item * SL + tid) * p.cap + part * p.k;
+      for (int j = 0; j < p.k; ++j) {   // k <= K; empty places are -inf, row -1
+        const float av = a < K ? lv[a] : -INFINITY, bv = b < K ? lv[K + b] : -INFINITY;
+        const int ar = a < K ? lr[a] : -1, br = b < K ? lr[K + b] : -1;
+        const bool first = br < 0 || (ar >= 0 && ss_first(av, ar, bv, br));
+        p.cand_v[at + j] = first ? av : bv;
+        p.cand_r[at + j] = first ? ar : br;
+        a += first;
+        b += !first;
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------- selection
 // The k <= 256 largest of n values, sorted, by one workgroup. The k-th largest of the 256 threads' maxima (of 64 groups'
 // maxima where k is at most 32) is a lower bound of the k-th largest value, so a first pass takes maxima, their ranks (by
@@ -722,6 +919,33 @@ void launch_scan(const ScanArgs& a, int ng, int K, int blocks, hipStream_t strea
   NGA_SCAN(3, 0); NGA_SCAN(3, 4); NGA_SCAN(3, 8);
   NGA_SCAN(4, 0); NGA_SCAN(4, 4); NGA_SCAN(4, 8);
 #undef NGA_SCAN
+}
+
+// 17 to 64 queries of all rows, prepared
+bool scan_wide_covers(int D, int ng) { return ng >= 2 && ng <= 4 && (D == 384 || D == 768 || D == 1024); }
+
+template <int NG, int K, int KS>
+static void wide_go(const ScanArgs& a, int blocks, hipStream_t stream) {
+  static const bool attr = [] {
+    (void)hipFuncSetAttribute((const void*)scan_wide_kernel<NG, K, KS>, hipFuncAttributeMaxDynamicSharedMemorySize, SS_LDS);
+    (void)hipGetLastError();
+    return true;
+  }();
+  (void)attr;
+  scan_wide_kernel<NG, K, KS><<<blocks, 256, wide_lds(NG, KS), stream>>>(a);
+}
+
+void launch_scan_wide(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream) {
+#define NGA_WIDE(NG_, K_)                                              \
+  if (ng == NG_ && K == K_) {                                          \
+    if (a.D == 1024) return wide_go<NG_, K_, 8>(a, blocks, stream);    \
+    if (a.D == 768) return wide_go<NG_, K_, 6>(a, blocks, stream);     \
+    return wide_go<NG_, K_, 3>(a, blocks, stream);                     \
+  }
+  NGA_WIDE(2, 0); NGA_WIDE(2, 4); NGA_WIDE(2, 8); NGA_WIDE(2, 16);
+  NGA_WIDE(3, 0); NGA_WIDE(3, 4); NGA_WIDE(3, 8);
+  NGA_WIDE(4, 0); NGA_WIDE(4, 4); NGA_WIDE(4, 8);
+#undef NGA_WIDE
 }
 
 void launch_search_prep(const float* q, int64_t q_stride, int nq, int D, int metric, uint16_t* qb, hipStream_t stream) {

@@ -1826,11 +1826,13 @@ def search_covers(X: torch.Tensor, k: int, most: int = 256) -> bool:
 def search_many(nq: int, rows: int, D: int, k: int) -> bool:
     """Whether many queries over all rows are faster through ``search_topk``, whose kernel (vector_search.hip) holds 64 queries
     in registers' reach and reads the vectors straight into fragments: then the products bound the scan and not the stream of
-    vectors, of which the other has half the LDS full of queries. The line lies at 4.5e10 products of whole groups of 64
-    queries, vectors below 512 dimensions counted as such, for what its register lists hold (k 8). k 4, us, this / that:
-    1M x 1,024, 65 queries 791 / 899, 512: 2,290 / 3,266; 100k x 1,024, 256: 249 / 224, 512: 380 / 386, 4,096: 1,781 / 2,614;
-    300k x 256, 256: 241 / 243, 1,000: 616 / 762; 1M x 128, 1,000: 1,206 / 987."""
-    return nq > 64 and k <= kernels().score_topk_kmax(64) and D >= 256 and -(-nq // 64) * 64 * rows * max(D, 512) >= 4.5e10
+    vectors. The line lies at 4.5e10 products of whole groups of 64 queries, vectors below 512 dimensions counted as such, for
+    what its register lists hold (k 8); of 1,024 dimensions on at 512 queries besides, where the flat scan's groups of 64 in
+    registers keep up. k 4, us, this / that: 1M x 1,024, 65 queries 748 / 657, 512: 2,232 / 2,144; 100k x 1,024, 512: 314 / 270,
+    4,096: 1,737 / 1,714; 300k x 768, 256: 376 / 356, 1,024: 1,098 / 1,229; 1M x 384, 128: 422 / 463, 1,024: 2,089 / 3,041; 300k x
+    256, 256: 241 / 243, 1,000: 616 / 762; 1M x 128, 1,000: 1,206 / 987."""
+    return (nq > 64 and k <= kernels().score_topk_kmax(64) and D >= 256 and not (D >= 1024 and nq <= 512)
+            and -(-nq // 64) * 64 * rows * max(D, 512) >= 4.5e10)
 
 
 def search_many_lists(nq: int, rows: int, D: int, k: int, nlist: int, nprobe: int) -> bool:

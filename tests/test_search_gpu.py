@@ -178,6 +178,15 @@ def test_flat_search_against_fp64(gpu, N, D, nq, k, metric):
     _check_found(v, i, S.masked_fill(idx.bias[:N] == float("-inf"), float("-inf")), k)
 
 
+# rows around the ends of units, tiles and one tile a workgroup; groups of queries that are full, have one query, or fill a second item;
+# register lists of each length, and scores
+@pytest.mark.parametrize("D", [384, 768, 1024])
+@pytest.mark.parametrize("N,nq,k", [(1, 17, 1), (16, 33, 4), (33, 64, 8), (8191, 49, 9), (8193, 32, 16), (24_577, 48, 17), (100_001, 17, 4),
+                                    (100_001, 65, 25), (70_000, 129, 8), (300, 64, 256)])
+def test_flat_search_of_many_against_fp64(gpu, D, N, nq, k):
+    test_flat_search_against_fp64(gpu, N, D, nq, k, ("ip", "cosine", "l2")[N % 3])
+
+
 def test_flat_search_equal_scores_and_strided_queries(gpu):
     """More equal scores than the selection sorts at once (one vector many times), with lists and with scores; queries
     that are every second row of a wider matrix."""
