@@ -494,7 +494,9 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
 // query in registers (NG x KS fragments), reads that quarter of every row, and the four waves add up in LDS, 32 rows at a time.
 // LDS is then a ring of NSL units (16 rows) a wave, which all stay under way. The sums are handed over in the accumulators'
 // layout, so that a lane ends with four rows of one query as in the other kernel; wave w takes rows 16 (w & 1) .. and every
-// second group of queries.
+// second group of queries. Bound by the stream: 1M x 1,024, k 4, whole search, before and here, 17 / 33 / 64 queries: 322 372
+// 493 us, 307 299 336; k 25 (scores) 434 473 568, 412 445 504; 250k x 768, k 4: 88 100 126, 69 81 96; 10k x 384: 20 23 27, 17 19 20.
+// Dimensions are those that come in earnest (384, 768, 1,024); each takes its own registers.
 namespace {
 constexpr int wide_slots(int KS, int NG) { return KS == 8 ? (NG == 4 ? 3 : 4) : KS == 6 ? 5 : 10; }   // of 4 KS KiB for all waves
 constexpr int wide_swizzle(int KS) { return KS % 4 == 0 ? 15 : KS % 2 == 0 ? 7 : 3; }
@@ -691,15 +693,16 @@ __global__ void __launch_bounds__(256, 1) scan_wide_kernel(ScanArgs p) {
 // The k <= 256 largest of n values, sorted, by one workgroup. The k-th largest of the 256 threads' maxima (of 64 groups'
 // maxima where k is at most 32) is a lower bound of the k-th largest value, so a first pass takes maxima, their ranks (by
 // counting) give the bound, and a second pass collects what reaches it: a few more than k values, which are ranked by
-// counting again. Eight loads are in flight per thread. Values of -inf (removed rows) are left out. Should more than
+// counting again, as keys of 64 bits, sixteen comparisons' reads in flight. Up to 256 RV values stay in registers between the
+// passes. Values of -inf (removed rows) are left out. Should more than
 // 1,024 values reach the bound (equal scores), the k-th key is found bit by bit, and the last row that is taken of those with
 // that key in the same way. Three passes over 2,048 LDS counters,
-// most of them on the same few exponents, took 82 us for both levels of 33 x 250k scores, k 25; these take 30.
+// most of them on the same few exponents, took 82 us for both levels of 33 x 250k scores, k 25; two reads of the scores, and ranks
+// from one LDS read after another, 30; these take 23.
 // Order: value, then row (the lower first).
 namespace {
 struct SelShared {
-  uint32_t key[SEL_CAP];
-  int32_t row[SEL_CAP];
+  uint64_t kr[SEL_CAP];   // key, then the row's complement: their order is that of results
   uint32_t tmax[256];
   uint32_t bound, n_got;
   int red[4];
@@ -713,18 +716,24 @@ __device__ __forceinline__ int sel_block_count(int c, int* red) {
   return red[0] + red[1] + red[2] + red[3];
 }
 
-// returns how many of the first k places are filled; emit(place, value, row) is called for each of them
-template <typename Emit>
+// returns how many of the first k places are filled; emit(place, value, row) is called for each of them. More than 256 RV values are
+// read twice.
+template <int RV, typename Emit>
 __device__ __forceinline__ int sel_topk(const float* __restrict__ v, const int32_t* __restrict__ r, int64_t row0, int64_t n, int k,
                                         SelShared& s, Emit emit) {
   const int t = threadIdx.x;
+  const bool kept = n <= 256 * RV;
   uint32_t mx = 0;
-  for (int64_t i0 = t; i0 < n; i0 += 8 * 256) {
-    float x[8];
+  float x[RV];
+  int32_t xr[RV];
+  for (int64_t i0 = t; i0 < (kept ? t + 1 : n); i0 += RV * 256) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = i0 + 256 * u < n ? v[i0 + 256 * u] : -INFINITY;
+    for (int u = 0; u < RV; ++u) x[u] = i0 + 256 * u < n ? v[i0 + 256 * u] : -INFINITY;
+    if (r && kept)
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < RV; ++u) xr[u] = i0 + 256 * u < n ? r[i0 + 256 * u] : -1;
+#pragma unroll
+    for (int u = 0; u < RV; ++u) {
       const uint32_t key = ss_key(x[u]);
       mx = key > mx ? key : mx;
     }
@@ -753,19 +762,19 @@ __device__ __forceinline__ int sel_topk(const float* __restrict__ v, const int32
   }
   __syncthreads();
   const uint32_t bound = s.bound;
-  for (int64_t i0 = t; i0 < n; i0 += 8 * 256) {
-    float x[8];
+  for (int64_t i0 = t; i0 < (kept ? t + 1 : n); i0 += RV * 256) {
+    if (!kept)
 #pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = i0 + 256 * u < n ? v[i0 + 256 * u] : -INFINITY;
+      for (int u = 0; u < RV; ++u) x[u] = i0 + 256 * u < n ? v[i0 + 256 * u] : -INFINITY;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < RV; ++u) {
       const uint32_t key = ss_key(x[u]);
       if (key >= bound) {
         const uint32_t pos = atomicAdd(&s.n_got, 1u);
         if (pos < SEL_CAP) {
           const int64_t i = i0 + 256 * u;
-          s.key[pos] = key;
-          s.row[pos] = r ? r[i] : (int32_t)(row0 + i);
+          const int32_t row = r ? (kept ? xr[u] : r[i]) : (int32_t)(row0 + i);
+          s.kr[pos] = (uint64_t)key << 32 | (uint32_t)~row;
         }
       }
     }
@@ -798,21 +807,22 @@ __device__ __forceinline__ int sel_topk(const float* __restrict__ v, const int32
       const int32_t row = r ? r[i] : (int32_t)(row0 + i);
       if (key > kth || (key == kth && (uint32_t)row <= last)) {
         const uint32_t pos = atomicAdd(&s.n_got, 1u);
-        if (pos < (uint32_t)k) {
-          s.key[pos] = key;
-          s.row[pos] = row;
-        }
+        if (pos < (uint32_t)k) s.kr[pos] = (uint64_t)key << 32 | (uint32_t)~row;
       }
     }
     __syncthreads();
     got = (int)s.n_got < k ? (int)s.n_got : k;
   }
   for (int i = t; i < got; i += 256) {
-    const uint32_t key = s.key[i];
-    const int32_t row = s.row[i];
+    const uint64_t own = s.kr[i];
     int place = 0;
-    for (int o = 0; o < got; ++o) place += s.key[o] > key || (s.key[o] == key && (s.row[o] < row || (s.row[o] == row && o < i)));
-    if (place < k) emit(place, __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key), row);
+#pragma unroll 16
+    for (int o = 0; o < got; ++o) {
+      const uint64_t x = s.kr[o];
+      place += x > own || (x == own && o < i);
+    }
+    const uint32_t key = (uint32_t)(own >> 32);
+    if (place < k) emit(place, __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key), (int32_t)~(uint32_t)own);
   }
   return got < k ? got : k;
 }
@@ -827,7 +837,7 @@ __global__ void __launch_bounds__(256) select_segments_kernel(const float* __res
   const int64_t n = N - beg < seg ? N - beg : seg;
   float* ov = cand_v + q * cap + (int64_t)blockIdx.x * k;
   int32_t* orow = cand_r + q * cap + (int64_t)blockIdx.x * k;
-  const int got = sel_topk(S + q * s_stride + beg, (const int32_t*)nullptr, beg, n, k, s, [&](int place, float v, int32_t r) {
+  const int got = sel_topk<32>(S + q * s_stride + beg, (const int32_t*)nullptr, beg, n, k, s, [&](int place, float v, int32_t r) {
     ov[place] = v;
     orow[place] = r;
   });
@@ -853,7 +863,7 @@ __global__ void __launch_bounds__(256) search_finish_kernel(const float* __restr
     for (int i = threadIdx.x; i < D; i += 256) less += qf[q * q_stride + i] * qf[q * q_stride + i];
     less = block_sum(less, red);
   }
-  const int got = sel_topk(cand_v + q * cap, cand_r + q * cap, 0, n, k, s, [&](int place, float v, int32_t r) {
+  const int got = sel_topk<16>(cand_v + q * cap, cand_r + q * cap, 0, n, k, s, [&](int place, float v, int32_t r) {
     const float x = v - less;
     out_v[q * k + place] = x;
     out_id[q * k + place] = r >= 0 && isfinite(x) ? ids[r] : -1;
