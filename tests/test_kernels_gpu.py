@@ -397,6 +397,21 @@ def test_score_topk(gpu, nq, N, D):
         assert torch.equal(torch.gather(S.cpu(), 1, i.cpu()), v.cpu())
 
 
+@pytest.mark.parametrize("H", [8, 384, 1000, 1024, 8192])
+def test_pool_of_many_rows(gpu, H):
+    """Rows around what the threads take at once (eight each, threads / (H / 8) groups); sums of at most 700 bf16 values in fp32,
+    of unit rows: 700 * 2^-24 of a value, and the norm's."""
+    lens = [1, 7, 8, 9, 0, 57, 168, 169, 700]
+    cu = torch.tensor([0] + lens, device=gpu).cumsum(0).int()
+    h = torch.randn(sum(lens), H, device=gpu).to(torch.bfloat16)
+    for norm in (False, True):
+        got = ops.pool_l2norm(h, cu, 1, norm).double()
+        want = torch.stack([h[a:b].double().mean(0) if b > a else torch.zeros(H, device=gpu, dtype=torch.float64)
+                            for a, b in zip(cu[:-1].tolist(), cu[1:].tolist())])
+        want = want / want.norm(dim=1, keepdim=True).clamp_min(1e-12) if norm else want
+        assert (got - want).abs().max() <= 1e-4 * want.abs().max()
+
+
 def test_pool(gpu):
     torch.manual_seed(7)
     lens = [3, 1, 77]
