@@ -1221,14 +1221,24 @@ void embedding(Tensor out, Tensor table, Tensor ids, int64_t vocab_lo, double sc
 
 // ------------------------------------------------------------------ encoder
 // K slices of a projection whose norm sums the slabs: 256-deep ones up to 32 rows (eight waves share a slice), at most 8;
-// with LDS tiles 4 slices while the tiles leave CUs idle (512 rows of 1,024 features: 128 tiles). Chosen at hidden size 1,024;
+// with LDS tiles 4 slices while the tiles leave CUs idle (512 rows of 1,024 features: 128 tiles), above 1,024 rows no more than two
+// tiles a CU (19,200 x 384: 49 us a projection in 2 and 4 slices, and their norms 14 and 22). Chosen at hidden size 1,024;
 // the whole forward beside the same steps with the library's products, us at 16 / 64 / 256 / 512 / 1,024 rows: 1,024 x 12 layers
 // 633 742 725 870 1,036, here 389 538 564 759 1,030; 768 x 12 493 554 561 665 793, here 354 470 515 630 810; 384 x 6 214 252 266
 // 304 334, here 148 194 210 265 324
-int encoder_split(int64_t M, int64_t K) {
+int encoder_split(int64_t M, int64_t N, int64_t K) {
   if (M <= 32) return (int)std::min<int64_t>(8, std::max<int64_t>(1, K / 256));
-  return M <= 512 ? (int)std::min<int64_t>(4, K / 64) : K > 1024 ? 4 : 2;
+  if (M <= 512) return (int)std::min<int64_t>(4, K / 64);
+  const int64_t most = K > 1024 ? 4 : 2, tiles = (M + 127) / 128 * ((N + 63) / 64);
+  return M <= 1024 ? (int)most : (int)std::max<int64_t>(1, std::min(most, 512 / tiles));
 }
+
+// Most rows that the LDS tiles take: beyond, the library's larger tiles are faster than these without their launches' cost on the
+// host. Where they meet lies at 1.2e9 rows x hidden^2: a forward, library / here, us: 1,024 x 24 layers at 1,152 rows 2,391 2,314,
+// 1,280 2,378 2,397; 768 x 12 at 1,536 rows 1,130 948, 2,048 1,122 1,125, 3,072 1,383 1,481; 512 x 8 at 4,096 756 771. Small models
+// are bound by the host's launches there: embedding token lists with 384 x 6 layers, 1,152 rows 723 329, 4,096 873 518, 9,600
+// 1,215 945, 19,200 1,828 1,636 (the forward alone over and over: 9,600 rows of 12 layers 1,370 1,625).
+int64_t encoder_tile_rows(int64_t H) { return H <= 384 ? 20480 : std::max<int64_t>(1024, 1200000000 / (H * H)); }
 
 // nullptr, or why encoder_forward does not take these weights; tables: positions, types, the embedding norm's weight and bias
 const char* encoder_refuses(const Tensor& word, const std::vector<Tensor>& tables, const std::vector<Tensor>& L, int64_t heads) {
@@ -1278,11 +1288,11 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
                               bfp(word), (int)word.size(0), bfp(ptab), (int)ptab.size(0), bfp(ttab), (int)ttab.size(0),
                               bfp(emb_g), bfp(emb_b), (float)eps, T, (int)H, bfp(x), st);
   Tensor qkv = at::empty({T, 3 * H}, opt), a = at::empty({T, H}, opt), y = at::empty({T, H}, opt), h = at::empty({T, F}, opt);
-  const bool rows = T <= 32, tiles = !rows && T <= 1024;
+  const bool rows = T <= 32, tiles = !rows && T <= encoder_tile_rows(H);
   Tensor slabs;
   const bool one = rows && B == 1 && max_len >= T;   // a single query; where several lie is known on the GPU alone
   const int att_split = one ? nga::row_attn_split((int)heads) : 0;
-  if (rows || tiles) slabs = at::empty({std::max({encoder_split(T, H), encoder_split(T, F), att_split}), T, H}, opt.dtype(at::kFloat));
+  if (rows || tiles) slabs = at::empty({std::max({encoder_split(T, H, H), encoder_split(T, H, F), att_split}), T, H}, opt.dtype(at::kFloat));
   // out = x w^T + bias (GELU)
   auto project = [&](const Tensor& in, const Tensor& w, const Tensor& bias, Tensor& out, bool gelu) {
     const int64_t N = w.size(0), K = w.size(1);
@@ -1304,7 +1314,7 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
   auto project_norm = [&](const Tensor& in, const Tensor& w, const Tensor& bias, const Tensor& resid, const Tensor& g,
                           const Tensor& b, Tensor& out) {
     const int64_t K = w.size(1);
-    const int split = encoder_split(T, K);
+    const int split = encoder_split(T, H, K);
     if (rows) {
       nga::launch_row_gemm({bfp(in), K, bfp(w), nullptr, slabs.data_ptr(), H, (int)T, (int)H, (int)K, split}, 1, st);
     } else if (tiles) {

@@ -71,6 +71,13 @@ def test_rows_forward(gpu, H, heads, F, lens):
     assert torch.equal(got, hidden())
 
 
+# above 1,024 rows: the smallest, the last of hidden 1,024 and of 768 with LDS tiles, K slices of each count
+@pytest.mark.parametrize("H,heads,F,T", [(384, 12, 1536, 1025), (384, 12, 1536, 2047), (128, 2, 256, 4100), (768, 12, 3072, 2034),
+                                         (1024, 16, 4096, 1144), (1024, 16, 4096, 1145), (384, 12, 1536, 9001)])
+def test_many_rows_forward(gpu, H, heads, F, T):
+    test_rows_forward(gpu, H, heads, F, [64] * (T // 64) + [T % 64])
+
+
 def test_rows_of_another_sequence_do_not_mix(gpu):
     """A token outside the table gives its own sequence NaN and no other; infinities in one stay there."""
     from nv_genai_amd.models.config import encoder_config
