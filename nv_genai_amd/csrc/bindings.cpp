@@ -523,6 +523,26 @@ void stream_gemm(Tensor out, Tensor x, Tensor w, int64_t epi, c10::optional<Tens
                            norm_weight(norm_w, x, epi, "stream_gemm"), (float)eps}, (int)epi, cur_stream(x));
 }
 
+// x [M, K] . w [K, N], rows of x at any multiple of 8 values
+Tensor gemm_kn(Tensor x, Tensor w) {
+  CHECK_DEV(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_CONTIG(w);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.device() == w.device() && x.size(1) == w.size(0), "gemm_kn: x [M, K] and w [K, N]");
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(1);
+  TORCH_CHECK(M >= 1 && M < (1 << 24) && N % 256 == 0 && N >= 256 && N < (1 << 20) && K % 32 == 0 && K >= 256 && K < (1 << 24),
+              "gemm_kn: N % 256 == 0, K % 32 == 0, K >= 256");
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.stride(0) >= K && x.stride(0) < (1 << 22) &&
+                  reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
+              "gemm_kn: rows at 16-byte addresses");
+  const int S = nga::gemm_kn_split(M, N, K);
+  Tensor out = at::empty({M, N}, x.options());
+  Tensor slabs = S > 1 ? at::empty({S, M, N}, x.options().dtype(at::kFloat)) : out;
+  const hipStream_t st = cur_stream(x);
+  nga::launch_gemm_kn({bfp(x), bfp(w), x.stride(0), slabs.data_ptr(), (int)M, (int)N, (int)K, S}, st);
+  if (S > 1) nga::launch_splitk_reduce(slabs.data_ptr<float>(), S, (int)M, (int)N, bfp(out), N, st);
+  post_launch("gemm_kn");
+  return out;
+}
+
 void splitk_swiglu(Tensor out, Tensor P, int64_t S) {
   CHECK_DEV(P); CHECK_BF16(out);
   TORCH_CHECK(out.device() == P.device(), "splitk_swiglu: out and P on one device");
@@ -2890,6 +2910,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("add_f32", on_device(&add_f32));
   m.def("ln_sums", on_device(&ln_sums));
   m.def("gelu_rows", on_device(&gelu_rows));
+  m.def("gemm_kn", on_device(&gemm_kn));
   m.def("col_sums", on_device(&col_sums));
   m.def("half_copies", on_device(&half_copies));
   m.def("half_grads", on_device(&half_grads));

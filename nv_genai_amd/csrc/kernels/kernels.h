@@ -241,6 +241,16 @@ void launch_embed_layernorm(const int32_t* ids, const int32_t* pos, const int32_
                             const uint16_t* ptab, int n_pos, const uint16_t* ttab, int n_type, const uint16_t* g,
                             const uint16_t* b, float eps, int64_t rows, int H, uint16_t* out, hipStream_t stream);
 
+// gemm_kn.hip: out[M, N] = x[M, K] . w[K, N], bf16, or fp32 slabs [split, M, N]; K % 32 == 0, N % 256 == 0, K / 32 >= 8 split
+struct GemmKnParams {
+  const uint16_t *x, *w;
+  int64_t ldx;
+  void* out;
+  int M, N, K, split;
+};
+int gemm_kn_split(int64_t M, int64_t N, int64_t K);
+void launch_gemm_kn(const GemmKnParams& p, hipStream_t stream);
+
 // train.hip: w32: weights and biases are fp32 (else bf16)
 int train_parts(int64_t R);                  // rows of `part` of the norms' backward
 int train_col_parts(int64_t R, int F);       // of launch_col_sums

@@ -243,6 +243,15 @@ def stream_gemm(x: torch.Tensor, w: torch.Tensor, epi: int = 0) -> torch.Tensor:
     return out
 
 
+def gemm_kn_covers(M: int, N: int, K: int) -> bool:
+    """Whether x [M, K] . w [K, N] (a frozen projection's gradient, w as it lies) is faster through gemm_kn.hip than the library's
+    product: contractions so long that splitting them fills the chip, and few rows. us, library / here: K 28,672, N 4,096, M 64 / 512 /
+    1,024 / 2,048: 166 87, 284 117, 348 192, 382 352; K 128,256: 471 308, 855 427, 1,442 785, 1,587 1,521; K 6,144, M 128 / 512 / 1,024:
+    46 30, 47 44, 57 60; K 4,096, M 128 / 200: 32 23, 23 27; N 14,336, M 128 / 1,024: 42 41, 98 101."""
+    return (M >= 1 and N % 256 == 0 and N >= 256 and K % 32 == 0 and N < 1 << 20 and K < 1 << 22
+            and (K >= 16384 and M <= 2048 and N <= 8192 or M <= 128 and N <= 4096 and K >= 4096))
+
+
 def norm_linear_covers(x: torch.Tensor, norm_w: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:
     """Whether :func:`norm_linear` runs rmsnorm(x [1, K]) @ w^T: one row (K <= 8,192) of bf16 on the GPU at 16-byte addresses."""
     return (_gpu(x) and x.dim() == 2 and x.shape[0] == 1 and x.numel() <= 8192 and x.shape[1] % 8 == 0 and w.shape[0] > 0

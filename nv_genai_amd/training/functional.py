@@ -201,7 +201,8 @@ def lm_loss(model, hidden: torch.Tensor, labels: torch.Tensor, params: Optional[
     h, y = h.index_select(0, keep), y.index_select(0, keep)
     total = h.new_zeros((), dtype=torch.float32)
     for s in range(0, h.shape[0], chunk):
-        lg = h[s:s + chunk] @ head.t()
+        hs = h[s:s + chunk]
+        lg = fused.frozen_linear(hs, head) if fused.frozen_linear_usable(hs, head) else hs @ head.t()
         if fused.cross_entropy_usable(lg):
             if s == 0 and params is None and int(y.max()) >= lg.shape[1]:   # the one-pass form would give NaN
                 raise IndexError(f"label {int(y.max())} outside the vocabulary of {lg.shape[1]}")

@@ -337,6 +337,37 @@ def cross_entropy_usable(logits: torch.Tensor) -> bool:
     return _takes(logits) and logits.shape[-1] % 8 == 0
 
 
+class _FrozenLinear(Function):
+    @staticmethod
+    def forward(ctx, x, w):
+        ctx.save_for_backward(w)
+        return x @ w.t()
+
+    @staticmethod
+    def backward(ctx, dy):
+        w, = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return dy @ w, None
+        return _input_grad(dy.reshape(-1, w.shape[0]), w).view(*dy.shape[:-1], w.shape[1]), None
+
+
+def _input_grad(dy2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    if ops.gemm_kn_covers(dy2.shape[0], w.shape[1], w.shape[0]) and w.is_contiguous() and w.data_ptr() % 16 == 0 and dy2.dtype is BF16:
+        return ops.kernels().gemm_kn(_rows(dy2), w)
+    return dy2 @ w
+
+
+def frozen_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x w^T with a frozen bf16 w; x's gradient from the framework's own product where that is the faster one."""
+    return _FrozenLinear.apply(x, w)
+
+
+def frozen_linear_usable(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (_takes(x) and x.requires_grad and torch.is_grad_enabled() and w.dim() == 2 and w.device == x.device and w.dtype is BF16
+            and not w.requires_grad and _plain(w) and w.is_contiguous() and w.data_ptr() % 16 == 0 and x.shape[-1] == w.shape[1]
+            and ops.gemm_kn_covers(x.numel() // w.shape[1], w.shape[1], w.shape[0]))
+
+
 class _LoraLinear(Function):
     @staticmethod
     def forward(ctx, x, w, a, b, ab, bb, scale):
@@ -357,7 +388,7 @@ class _LoraLinear(Function):
             return dx, None, None, None, da, db, None
         dy2 = dy.reshape(-1, dy.shape[-1])
         dh = (dy2 @ bb).mul_(scale)
-        dx = torch.addmm(dy2 @ w, dh, ab).view(x.shape) if ctx.needs_input_grad[0] else None
+        dx = torch.addmm(_input_grad(dy2, w), dh, ab).view(x.shape) if ctx.needs_input_grad[0] else None
         da = (dh.t() @ x.reshape(-1, x.shape[-1])).to(ad) if ctx.needs_input_grad[2] else None
         db = (dy2.t() @ h).to(bd).mul_(scale) if ctx.needs_input_grad[3] else None   # scaled in its own type
         return dx, None, da, db, None, None, None

@@ -65,9 +65,9 @@ class LoRA:
         if (a is not None and not w.requires_grad and w.dtype == torch.bfloat16 and w.shape[0] % 8 == 0
                 and fused.usable(x, w, a, self.B[(li, name)]) and not (self.cfg.dropout and torch.is_grad_enabled())):
             return fused.lora_linear(x, w, a, self.B[(li, name)], self.cfg.scale)
-        y = x @ w.t()
         if a is None:
-            return y
+            return fused.frozen_linear(x, w) if fused.frozen_linear_usable(x, w) else x @ w.t()
+        y = x @ w.t()
         h = x
         if self.cfg.dropout and torch.is_grad_enabled():
             h = torch.nn.functional.dropout(h, self.cfg.dropout)
