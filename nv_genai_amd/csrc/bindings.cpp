@@ -543,6 +543,23 @@ Tensor gemm_kn(Tensor x, Tensor w) {
   return out;
 }
 
+// GELU(x [M, K] . w [N, K]^T + bias), rows of x at any multiple of 8 values
+Tensor gemm_nt_gelu(Tensor x, Tensor w, Tensor bias) {
+  CHECK_DEV(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_CONTIG(w); CHECK_BF16(bias); CHECK_CONTIG(bias);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.device() == w.device() && x.device() == bias.device() && x.size(1) == w.size(1) &&
+                  bias.numel() == w.size(0), "gemm_nt_gelu: x [M, K], w [N, K] and bias [N]");
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(M >= 1 && M < (1 << 24) && N % 256 == 0 && N >= 256 && N < (1 << 20) && K % 32 == 0 && K >= 256 && K < (1 << 20),
+              "gemm_nt_gelu: N % 256 == 0, K % 32 == 0, K >= 256");
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.stride(0) >= K && x.stride(0) < (1 << 22) &&
+                  reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(bias.data_ptr()) % 8 == 0, "gemm_nt_gelu: rows at 16-byte addresses");
+  Tensor out = at::empty({M, N}, x.options());
+  nga::launch_gemm_nt_gelu({bfp(x), bfp(w), bfp(bias), x.stride(0), bfp(out), (int)M, (int)N, (int)K}, cur_stream(x));
+  post_launch("gemm_nt_gelu");
+  return out;
+}
+
 void splitk_swiglu(Tensor out, Tensor P, int64_t S) {
   CHECK_DEV(P); CHECK_BF16(out);
   TORCH_CHECK(out.device() == P.device(), "splitk_swiglu: out and P on one device");
@@ -1323,6 +1340,8 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
       p.x = bfp(in); p.ldx = K; p.w = bfp(w); p.M = (int)T; p.N = (int)N; p.K = (int)K;
       p.out = out.data_ptr(); p.ldo = N; p.bias = bfp(bias);
       nga::launch_skinny_bias(p, gelu, st);
+    } else if (gelu && nga::gemm_nt_gelu_covers(T, N, K)) {
+      nga::launch_gemm_nt_gelu({bfp(in), bfp(w), bfp(bias), K, bfp(out), (int)T, (int)N, (int)K}, st);
     } else if (gelu) {
       at::mm_out(out, in, w.t());
       nga::launch_bias_gelu(bfp(out), bfp(bias), T, (int)N, 0, st);
@@ -2911,6 +2930,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("ln_sums", on_device(&ln_sums));
   m.def("gelu_rows", on_device(&gelu_rows));
   m.def("gemm_kn", on_device(&gemm_kn));
+  m.def("gemm_nt_gelu", on_device(&gemm_nt_gelu));
   m.def("col_sums", on_device(&col_sums));
   m.def("half_copies", on_device(&half_copies));
   m.def("half_grads", on_device(&half_grads));

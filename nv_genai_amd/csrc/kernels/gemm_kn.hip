@@ -8,11 +8,7 @@
 // transpose read (a group of 16 lanes reads 4 k x 16 n and each lane receives 4 k of one n); it is the A operand, so that a lane
 // ends with four neighbouring columns of one row. M 1,024, N 4,096, K 28,672: 192 us, 1,250 TFLOP/s with the sum of the slabs (library
 // 348); K 128,256: 785 us, 1,370 (1,442). More in ops.gemm_kn_covers.
-//
-// The DMAs are inline asm without outputs: behind the builtin the compiler waits for all that are under way before each
-// transpose read, and they are counted here. So are the products, whose sums it moved between register files (1,030 TFLOP/s, all
-// reads of a stage before its products; 1,250 with them between).
-#include "common.h"
+#include "gemm_tile.h"
 #include "kernels.h"
 
 namespace nga {
@@ -22,16 +18,6 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4* ltr_t;
 constexpr int KN_T = 256, KN_K = 32, KN_STAGE = 2 * KN_T * KN_K, KN_NST = 4;   // tile, depth, elements and count of stages
 
-// 16 bytes a lane from base + off to lds + 16 lane; m0 needs one cycle
-__device__ __forceinline__ void kn_dma(const uint16_t* base, uint32_t off, uint16_t* lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"((uint32_t)(uintptr_t)(lptr_t)lds), "v"(off), "s"(base)
-               : "memory", "m0");
-}
-// acc += a b, the sums in accumulation registers throughout: with the builtin the compiler moves a good part of the 256 to and fro in
-// every round. The wait covers operands that an instruction before it has written.
-__device__ __forceinline__ void kn_mfma(f32x4& acc, bf16x8 a, bf16x8 b) {
-  asm("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-}
 // w's stage: 16-column unit u of row k lies at u ^ kn_swz(k): the eight rows that are read together lie in different banks
 __device__ __forceinline__ int kn_swz(int k) { return (k & 3) | (((k >> 3) & 1) << 2); }
 }  // namespace
@@ -60,8 +46,8 @@ __global__ void __launch_bounds__(256, 1) gemm_kn_kernel(GemmKnParams p) {
   const uint16_t* const wb = p.w + (int64_t)i0 * KN_K * p.N + n0;
   auto issue_one = [&](int i, int j) {   // j-th of eight
     uint16_t* const s = smem + (i % KN_NST) * KN_STAGE;
-    if (j < 4) kn_dma(xb + (int64_t)i * KN_K, xo[j & 3], s + (w * 64 + 16 * j) * KN_K);
-    else kn_dma(wb + (int64_t)i * KN_K * p.N, wo[j & 3], s + KN_T * KN_K + (w * 8 + 2 * (j - 4)) * KN_T);
+    if (j < 4) tile_dma(xb + (int64_t)i * KN_K, xo[j & 3], s + (w * 64 + 16 * j) * KN_K);
+    else tile_dma(wb + (int64_t)i * KN_K * p.N, wo[j & 3], s + KN_T * KN_K + (w * 8 + 2 * (j - 4)) * KN_T);
   };
   auto issue = [&](int i) {
 #pragma unroll
@@ -93,7 +79,7 @@ __global__ void __launch_bounds__(256, 1) gemm_kn_kernel(GemmKnParams p) {
 #pragma unroll
     for (int t = 0; t < 8; ++t)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) kn_mfma(acc[t][j], y[t], x[j]);
+      for (int j = 0; j < 8; ++j) tile_mfma(acc[t][j], y[t], x[j]);
   };
 
   bf16x8 xa[8], ya[8], xc[8], yc[8];
@@ -112,13 +98,13 @@ __global__ void __launch_bounds__(256, 1) gemm_kn_kernel(GemmKnParams p) {
 #pragma unroll
     for (int t = 0; t < 8; ++t) {   // between two products there is time for another instruction
 #pragma unroll
-      for (int j = 0; j < 4; ++j) kn_mfma(acc[t][j], y[t], x[j]);
+      for (int j = 0; j < 4; ++j) tile_mfma(acc[t][j], y[t], x[j]);
       __builtin_amdgcn_sched_barrier(0);
       issue_one(i + 4, t);
       read_one(i + 1, t, nx[t], ny[t]);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 4; j < 8; ++j) kn_mfma(acc[t][j], y[t], x[j]);
+      for (int j = 4; j < 8; ++j) tile_mfma(acc[t][j], y[t], x[j]);
       __builtin_amdgcn_sched_barrier(0);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -143,11 +129,7 @@ __global__ void __launch_bounds__(256, 1) gemm_kn_kernel(GemmKnParams p) {
     last(i + 2 * j + 1, xc, yc, xa, ya);
   }
 
-  asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");   // the last products' results
-#pragma unroll
-  for (int t = 0; t < 8; ++t)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[t][j]));   // not read before
+  tile_settle(acc);
   const int64_t at = (int64_t)sl * p.M * p.N + n0 + wn * 128 + 4 * h;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {

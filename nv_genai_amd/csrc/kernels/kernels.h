@@ -251,6 +251,17 @@ struct GemmKnParams {
 int gemm_kn_split(int64_t M, int64_t N, int64_t K);
 void launch_gemm_kn(const GemmKnParams& p, hipStream_t stream);
 
+// gemm_nt.hip: out[M, N] = GELU(x[M, K] . w[N, K]^T + bias); N % 256 == 0, K % 32 == 0, K >= 256. covers: and faster than the library's
+// product and a launch of bias and GELU
+struct GemmNtParams {
+  const uint16_t *x, *w, *bias;
+  int64_t ldx;
+  uint16_t* out;
+  int M, N, K;
+};
+bool gemm_nt_gelu_covers(int64_t M, int64_t N, int64_t K);
+void launch_gemm_nt_gelu(const GemmNtParams& p, hipStream_t stream);
+
 // train.hip: w32: weights and biases are fp32 (else bf16)
 int train_parts(int64_t R);                  // rows of `part` of the norms' backward
 int train_col_parts(int64_t R, int F);       // of launch_col_sums

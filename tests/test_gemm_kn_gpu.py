@@ -1,4 +1,5 @@
-"""Gradient of a projection's inputs, x [M, K] . w [K, N] (gemm_kn.hip), against 64 bits."""
+"""The 256 x 256 tiles: a projection's input gradient, x [M, K] . w [K, N] (gemm_kn.hip), and an
+encoder's GELU(x . w [N, K]^T + bias) (gemm_nt.hip), against 64 bits."""
 import pytest
 import torch
 
@@ -47,3 +48,35 @@ def test_frozen_linear(gpu, shape, N):
     assert torch.autograd.grad(got.float().pow(2).sum(), dy)[0].isfinite().all()
     for v, u in ((x.detach(), w), (x, w.clone().requires_grad_()), (x, w.float()), (x.float(), w), (x, w.t().contiguous().t())):
         assert not fused.frozen_linear_usable(v, u)
+
+
+# one tile, tiles of rows that are not full, blocks of eight of them and one more, more tiles than CUs (a workgroup's second and third),
+# stages that end anywhere in the ring's round
+@pytest.mark.parametrize("M,N,K,apart", [(1, 256, 256, 0), (256, 768, 288, 8), (257, 256, 320, 0), (2100, 512, 352, 0), (2305, 1024, 1024, 0),
+                                         (4200, 4096, 1024, 24), (9000, 3072, 768, 0), (3000, 1024, 4096, 0)])
+def test_gemm_nt_gelu(gpu, M, N, K, apart):
+    """The fp32 sum's error grows with the root of the terms (2^-24 of their magnitudes each); GELU's slope is at most 1.13, and its form
+    here is within 3e-7 of the exact one; then one rounding to bf16."""
+    g = torch.Generator(gpu).manual_seed(M + K)
+    x = torch.randn(M, K + apart, device=gpu, generator=g).to(BF)[:, :K]
+    w = torch.randn(N, K, device=gpu, generator=g).mul_(2 / K ** 0.5).to(BF)
+    b = torch.randn(N, device=gpu, generator=g).to(BF)
+    sums, mag = x.double() @ w.double().t() + b.double(), x.double().abs() @ w.double().abs().t() + b.double().abs()
+    want = torch.nn.functional.gelu(sums)
+    got = ops.kernels().gemm_nt_gelu(x, w, b)
+    assert ((got.double() - want).abs() <= 2 ** -8 * want.abs() + 1.13 * 2 ** -24 * K ** 0.5 * mag + 3e-7 * sums.abs()).all()
+
+
+def test_gemm_nt_gelu_at_the_ends(gpu):
+    """Sums of every size, infinities and NaN: K values of which one counts."""
+    v = torch.cat([torch.linspace(-12, 12, 4001), torch.tensor([0.0, -0.0, 1e-30, -1e-30, 3e38, -3e38, float("inf"), float("-inf"), float("nan")])])
+    x = torch.zeros(v.numel(), 256, device=gpu, dtype=BF)
+    x[:, 0] = v.to(gpu)
+    w = torch.zeros(256, 256, device=gpu, dtype=BF)
+    w[:, 0] = 1
+    got = ops.kernels().gemm_nt_gelu(x, w, torch.zeros(256, device=gpu, dtype=BF))
+    a = x[:, 0].double()
+    want = torch.where(a == 0, a, a * 0.5 * torch.erfc(-a * 0.5 ** 0.5))   # torch's own loses the digits of a small 1 + erf
+    fin = want.isfinite()
+    assert torch.equal(got.isnan(), want.isnan()[:, None].expand_as(got)) and (got[want == float("inf")] == float("inf")).all()
+    assert ((got[fin].double() - want[fin, None]).abs() <= 2 ** -8 * want[fin, None].abs() + 3e-7).all()
