@@ -237,11 +237,8 @@ __device__ __forceinline__ void v1_tile(const PrefillParams& P, uint16_t* k_s, u
   }
 }
 
-// Grid modes (as attention_prefill_v2.hip): enumerated — workgroups dealt round-robin over
-// the 8 XCDs, physical block p runs on XCD p % 8 and logical item L = (p % 8) * per_xcd + p / 8
-// gives every XCD one contiguous range of the (sequence, kv head, q head, tile) order (the G
-// query heads sharing a KV head read its pages through the same L2; longest causal tiles
-// first) — or a host-planned work list of (sequence, 64-row tile) pairs walked by a fixed
+// Grid modes (as attention_prefill_v2.hip): enumerated — the (sequence, kv head, q head, tile)
+// order of deal_xcds, longest causal tiles first — or a host-planned work list of (sequence, 64-row tile) pairs walked by a fixed
 // grid with q head it % Hq (graph-captured steps with fp8 KV pages or head_dim != 128).
 template <int D, bool CAUSAL>
 __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams P) {
@@ -257,8 +254,7 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams P) {
     }
     return;
   }
-  const int pblk = blockIdx.x;
-  const int L = (pblk & 7) * P.per_xcd + (pblk >> 3);
+  const int L = xcd_item(P);
   if (L >= P.total) return;
   const int tile = P.ntiles - 1 - L % P.ntiles;
   const int hq = (L / P.ntiles) % P.Hq;
@@ -291,11 +287,7 @@ void launch_prefill_attention(const PrefillParams& p, int num_seqs, int max_q_le
   // 1.4-1.5x slower on MI355X; removed)
   PrefillParams pp = p;
   pp.ntiles = (max_q_len + 63) / 64;
-  const int64_t total = (int64_t)pp.ntiles * p.Hq * num_seqs;
-  pp.total = (int)total;
-  pp.per_xcd = (int)((total + 7) / 8);
-  // 1-D grid of 8 * per_xcd workgroups (see the XCD mapping in the kernel)
-  dim3 grid(8 * pp.per_xcd);
+  const dim3 grid(deal_xcds(pp, num_seqs, pp.ntiles * (p.Hq / p.Hkv)));
 #define NGA_PF(DD)                                                            \
   do {                                                                        \
     if (causal) prefill_attn_kernel<DD, true><<<grid, 256, 0, stream>>>(pp); \

@@ -401,10 +401,8 @@ __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) prefill_attn_v2_ker
     }
     return;
   }
-  // XCD-aware order (as the 16x16 kernel): each XCD gets a contiguous range of
-  // (sequence, kv head, head group, query block), longest causal blocks first.
-  const int pblk = blockIdx.x;
-  const int L = (pblk & 7) * P.per_xcd + (pblk >> 3);
+  // order (sequence, kv head, head group, query block), longest causal blocks first
+  const int L = xcd_item(P);
   if (L >= P.total) return;
   const int qb = P.ntiles - 1 - L % P.ntiles;
   const int hg = (L / P.ntiles) % NG;
@@ -439,9 +437,7 @@ bool launch_prefill_attention_v2(const PrefillParams& p, int num_seqs, int max_q
   int ks = p.impl == 3 ? 2 : p.impl == 2 ? 1 : (total <= 320 ? 2 : 1);
   if (ks_env == 1 || ks_env == 2) ks = ks_env;
   if (p.impl == 0 && ks == 1 && total < 2 * 256 * 2) return false;
-  pp.total = (int)total;
-  pp.per_xcd = (int)((total + 7) / 8);
-  dim3 grid(8 * pp.per_xcd);
+  const dim3 grid(deal_xcds(pp, num_seqs, pp.ntiles * (p.Hq / hpw / p.Hkv)));
 #define NGA_PF2(CS, HP)                                                                   \
   do {                                                                                      \
     if (ks == 2) prefill_attn_v2_kernel<CS, HP, 0, 2><<<grid, 512, 0, stream>>>(pp);        \

@@ -14,7 +14,7 @@
 // Bound by the softmax: 32 exponentials and about 100 other vector operations per lane and tile against 16 MFMAs of 32
 // cycles at head_dim 64, and by rounding up short sequences: 670 to 770 TFLOP/s at 512 and 2,048 tokens, 390 for 90 to 512
 // tokens. The 16x16 form before it wrote V transposed into LDS two bytes at a time. Layers as measured: 64 sequences of 90
-// to 512 tokens, 16 heads of 64: 170 -> 96 us; 20 sequences, 32 / 8 heads of 128: 298 -> 124 us. (The transpose read as
+// to 512 tokens, 16 heads of 64: 170 -> 96 us, with deal_xcds 77; 20 sequences, 32 / 8 heads of 128: 298 -> 124 us. (The transpose read as
 // an asm block that waits for its own reads alone, where the compiler waits for the next tile's DMA too: equal.)
 #include "common.h"
 #include "kernels.h"
@@ -51,9 +51,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) varlen_attn_kernel(Pref
   uint16_t* const kbuf = smem;
   uint16_t* const vbuf = smem + 2 * TILE;
 
-  // each XCD takes one stretch of the (sequence, head, row block) order: heads of one KV head share its rows in L2
-  const int pblk = blockIdx.x;
-  const int L = (pblk & 7) * P.per_xcd + (pblk >> 3);
+  const int L = xcd_item(P);
   if (L >= P.total) return;
   const int G = P.Hq / P.Hkv, ngrp = P.Hq / HPW;
   const int qb = P.ntiles - 1 - L % P.ntiles;
@@ -213,10 +211,7 @@ void launch_varlen_attention(const PrefillParams& p, int num_seqs, int max_q_len
   const int rw = 128 / hpw;
   PrefillParams pp = p;
   pp.ntiles = (max_q_len + rw - 1) / rw;
-  const int64_t total = (int64_t)pp.ntiles * (p.Hq / hpw) * num_seqs;
-  pp.total = (int)total;
-  pp.per_xcd = (int)((total + 7) / 8);
-  const dim3 grid(8 * pp.per_xcd);
+  const dim3 grid(deal_xcds(pp, num_seqs, pp.ntiles * (p.Hq / hpw / p.Hkv)));
 #define NGA_VL(DD)                                                                                         \
   do {                                                                                                     \
     if (hpw == 4) {                                                                                        \
