@@ -523,21 +523,22 @@ void stream_gemm(Tensor out, Tensor x, Tensor w, int64_t epi, c10::optional<Tens
                            norm_weight(norm_w, x, epi, "stream_gemm"), (float)eps}, (int)epi, cur_stream(x));
 }
 
-// x [M, K] . w [K, N], rows of x at any multiple of 8 values
-Tensor gemm_kn(Tensor x, Tensor w) {
-  CHECK_DEV(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_CONTIG(w);
-  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.device() == w.device() && x.size(1) == w.size(0), "gemm_kn: x [M, K] and w [K, N]");
-  const int64_t M = x.size(0), K = x.size(1), N = w.size(1);
-  TORCH_CHECK(M >= 1 && M < (1 << 24) && N % 256 == 0 && N >= 256 && N < (1 << 20) && K % 32 == 0 && K >= 256 && K < (1 << 24),
-              "gemm_kn: N % 256 == 0, K % 32 == 0, K >= 256");
-  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.stride(0) >= K && x.stride(0) < (1 << 22) &&
+// x [M, K] . w [K, N], rows of x at any multiple of 8 values; xt: x^T . w of x [K, M], both operands' rows so, any K
+Tensor gemm_kn(Tensor x, Tensor w, bool xt) {
+  CHECK_DEV(x); CHECK_BF16(x); CHECK_BF16(w);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.device() == w.device() && x.size(xt ? 0 : 1) == w.size(0), "gemm_kn: x [M, K] (xt: [K, M]) and w [K, N]");
+  CHECK_CONTIG(w);
+  const int64_t M = x.size(xt ? 1 : 0), K = w.size(0), N = w.size(1);
+  TORCH_CHECK(M >= 1 && M < (1 << 24) && N % 256 == 0 && N >= 256 && N < (1 << 20) && K >= 256 && K < (1 << 24) &&
+                  (xt ? M % 256 == 0 : K % 32 == 0), "gemm_kn: N (xt: and M) % 256 == 0, K >= 256, without xt K % 32 == 0");
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.stride(0) >= x.size(1) && x.stride(0) < (1 << 22) &&
                   reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
               "gemm_kn: rows at 16-byte addresses");
   const int S = nga::gemm_kn_split(M, N, K);
   Tensor out = at::empty({M, N}, x.options());
   Tensor slabs = S > 1 ? at::empty({S, M, N}, x.options().dtype(at::kFloat)) : out;
   const hipStream_t st = cur_stream(x);
-  nga::launch_gemm_kn({bfp(x), bfp(w), x.stride(0), slabs.data_ptr(), (int)M, (int)N, (int)K, S}, st);
+  nga::launch_gemm_kn({bfp(x), bfp(w), x.stride(0), slabs.data_ptr(), (int)M, (int)N, (int)K, S}, xt, st);
   if (S > 1) nga::launch_splitk_reduce(slabs.data_ptr<float>(), S, (int)M, (int)N, bfp(out), N, st);
   post_launch("gemm_kn");
   return out;

@@ -8,6 +8,12 @@
 // transpose read (a group of 16 lanes reads 4 k x 16 n and each lane receives 4 k of one n); it is the A operand, so that a lane
 // ends with four neighbouring columns of one row. M 1,024, N 4,096, K 28,672: 192 us, 1,250 TFLOP/s with the sum of the slabs (library
 // 348); K 128,256: 785 us, 1,370 (1,442). More in ops.gemm_kn_covers.
+//
+// XT: x lies as [K, M], for the gradient of a weight, dy^T . x: rows of the micro-batch are the long K then, both operands are read
+// transposed. K of any size from 256 on: the last stage is the last 32 rows, of which the ones that were there before count as zero. 10,240 rows:
+// 4,096 x 1,024 84 us (library 105), 1,024 x 1,024 39 (66). More in ops.weight_grad_covers.
+#include <algorithm>
+
 #include "gemm_tile.h"
 #include "kernels.h"
 
@@ -22,7 +28,7 @@ constexpr int KN_T = 256, KN_K = 32, KN_STAGE = 2 * KN_T * KN_K, KN_NST = 4;   /
 __device__ __forceinline__ int kn_swz(int k) { return (k & 3) | (((k >> 3) & 1) << 2); }
 }  // namespace
 
-template <bool SLABS>
+template <bool SLABS, bool XT>
 __global__ void __launch_bounds__(256, 1) gemm_kn_kernel(GemmKnParams p) {
   __shared__ __attribute__((aligned(16))) uint16_t smem[KN_NST * KN_STAGE];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -31,23 +37,24 @@ __global__ void __launch_bounds__(256, 1) gemm_kn_kernel(GemmKnParams p) {
   const int nb = gridDim.x, id = nb % 8 == 0 ? (blockIdx.x & 7) * (nb >> 3) + (blockIdx.x >> 3) : blockIdx.x;
   const int tm = (p.M + KN_T - 1) / KN_T, per = tm * (p.N / KN_T), sl = id / per, r = id - sl * per;
   const int m0 = (r % tm) * KN_T, n0 = (r / tm) * KN_T;
-  const int all = p.K / KN_K, i0 = (int)((int64_t)all * sl / p.split), steps = (int)((int64_t)all * (sl + 1) / p.split) - i0;   // >= 4
+  const int all = (p.K + KN_K - 1) / KN_K, i0 = (int)((int64_t)all * sl / p.split), steps = (int)((int64_t)all * (sl + 1) / p.split) - i0;   // >= 8
 
   // this wave's part of a stage: 64 rows of x, 4 chunks of 8 each (chunk c of row r at c ^ (r >> 2 & 3)); 8 rows of w
   uint32_t xo[4], wo[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int row = w * 64 + 16 * i + (lane >> 2), c = (lane & 3) ^ ((row >> 2) & 3);
-    xo[i] = 2 * (uint32_t)(min(row, p.M - 1 - m0) * (int)p.ldx + 8 * c);
-    const int k = w * 8 + 2 * i + (lane >> 5), pos = lane & 31;
-    wo[i] = 2 * (uint32_t)(k * p.N + (((pos >> 1) ^ kn_swz(k)) << 4) + ((pos & 1) << 3));
+    const int k = w * 8 + 2 * i + (lane >> 5), pos = lane & 31, at = (((pos >> 1) ^ kn_swz(k)) << 4) + ((pos & 1) << 3);
+    xo[i] = 2 * (uint32_t)(XT ? k * (int)p.ldx + at : min(row, p.M - 1 - m0) * (int)p.ldx + 8 * c);
+    wo[i] = 2 * (uint32_t)(k * p.N + at);
   }
-  const uint16_t* const xb = p.x + (int64_t)m0 * p.ldx + (int64_t)i0 * KN_K;
-  const uint16_t* const wb = p.w + (int64_t)i0 * KN_K * p.N + n0;
+  const uint16_t* const xb = p.x + (XT ? m0 : (int64_t)m0 * p.ldx);
+  const uint16_t* const wb = p.w + n0;
   auto issue_one = [&](int i, int j) {   // j-th of eight
     uint16_t* const s = smem + (i % KN_NST) * KN_STAGE;
-    if (j < 4) tile_dma(xb + (int64_t)i * KN_K, xo[j & 3], s + (w * 64 + 16 * j) * KN_K);
-    else tile_dma(wb + (int64_t)i * KN_K * p.N, wo[j & 3], s + KN_T * KN_K + (w * 8 + 2 * (j - 4)) * KN_T);
+    const int k = min((i0 + i) * KN_K, p.K - KN_K);
+    if (j < 4) tile_dma(xb + (XT ? k * p.ldx : k), xo[j & 3], s + (XT ? (w * 8 + 2 * j) * KN_T : (w * 64 + 16 * j) * KN_K));
+    else tile_dma(wb + (int64_t)k * p.N, wo[j & 3], s + KN_T * KN_K + (w * 8 + 2 * (j - 4)) * KN_T);
   };
   auto issue = [&](int i) {
 #pragma unroll
@@ -56,20 +63,28 @@ __global__ void __launch_bounds__(256, 1) gemm_kn_kernel(GemmKnParams p) {
   // a lane's fragments in a stage: 8 k of a row of x (16 j rows on for the j-th), of a column of w
   const int fx0 = (wm * 128 + col) * KN_K + ((h ^ ((col >> 2) & 3)) << 3);
   const int kr = 8 * h + (col >> 2);
-  int fw0[8];
+  int fw0[8], fxt[8];
 #pragma unroll
-  for (int t = 0; t < 8; ++t) fw0[t] = KN_T * KN_K + kr * KN_T + (((wn * 8 + t) ^ kn_swz(kr)) << 4) + 4 * (col & 3);
+  for (int t = 0; t < 8; ++t) {
+    fw0[t] = KN_T * KN_K + kr * KN_T + (((wn * 8 + t) ^ kn_swz(kr)) << 4) + 4 * (col & 3);
+    fxt[t] = kr * KN_T + (((wm * 8 + t) ^ kn_swz(kr)) << 4) + 4 * (col & 3);
+  }
+  auto transposed = [&](uint16_t* s) {   // four rows on the swizzle is the same
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ltr_t)s);
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ltr_t)(s + 4 * KN_T));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
   auto read_one = [&](int i, int t, bf16x8& x, bf16x8& y) {   // t-th of eight of each
     uint16_t* const s = smem + (i % KN_NST) * KN_STAGE;
-    x = as_bf16x8(*reinterpret_cast<const u16x8*>(s + fx0 + 16 * KN_K * t));
-    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ltr_t)(s + fw0[t]));
-    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ltr_t)(s + fw0[t] + 4 * KN_T));   // four rows on the swizzle is the same
-    y = __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+    if constexpr (XT) x = transposed(s + fxt[t]);
+    else x = as_bf16x8(*reinterpret_cast<const u16x8*>(s + fx0 + 16 * KN_K * t));
+    y = transposed(s + fw0[t]);
   };
   auto read = [&](int i, bf16x8 (&x)[8], bf16x8 (&y)[8]) {
 #pragma unroll
     for (int t = 0; t < 8; ++t) read_one(i, t, x[t], y[t]);
   };
+  const int again = all * KN_K - p.K;   // rows of the last stage that the one before it has
   f32x4 acc[8][8];   // [columns][rows]
 #pragma unroll
   for (int t = 0; t < 8; ++t)
@@ -113,7 +128,18 @@ __global__ void __launch_bounds__(256, 1) gemm_kn_kernel(GemmKnParams p) {
     if (i >= steps) return;
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (i + 4 < steps) issue(i + 4);
-    if (i + 1 < steps) read(i + 1, nx, ny);
+    if (i + 1 < steps) {
+      read(i + 1, nx, ny);
+      if (XT && again > 0 && i0 + i + 1 == all - 1) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            nx[t][e] = 8 * h + e >= again ? nx[t][e] : (__bf16)0.f;
+            ny[t][e] = 8 * h + e >= again ? ny[t][e] : (__bf16)0.f;
+          }
+      }
+    }
     multiply(x, y);
   };
   int i = 0;
@@ -150,19 +176,24 @@ __global__ void __launch_bounds__(256, 1) gemm_kn_kernel(GemmKnParams p) {
   }
 }
 
-// slices of K: as many as the tiles leave CUs for, of eight stages at least, at most 8
+// slices of K: as many as the tiles leave CUs for, of eight stages at least, at most 16
 int gemm_kn_split(int64_t M, int64_t N, int64_t K) {
   const int64_t tiles = (M + KN_T - 1) / KN_T * (N / KN_T);
   if (tiles < 1) return 1;
-  const int64_t s = 256 / tiles, most = K / KN_K / 8;
-  return (int)(s < 1 ? 1 : s > 8 ? (most < 8 ? most : 8) : s > most ? most : s);
+  const int64_t s = 256 / tiles, most = (K + KN_K - 1) / KN_K / 8;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(s, 16), most));
 }
 
-void launch_gemm_kn(const GemmKnParams& p, hipStream_t stream) {
+void launch_gemm_kn(const GemmKnParams& p, bool xt, hipStream_t stream) {
   const int blocks = (p.M + KN_T - 1) / KN_T * (p.N / KN_T) * p.split;
   if (blocks == 0) return;
-  if (p.split > 1) gemm_kn_kernel<true><<<blocks, 256, 0, stream>>>(p);
-  else gemm_kn_kernel<false><<<blocks, 256, 0, stream>>>(p);
+  if (xt) {
+    if (p.split > 1) gemm_kn_kernel<true, true><<<blocks, 256, 0, stream>>>(p);
+    else gemm_kn_kernel<false, true><<<blocks, 256, 0, stream>>>(p);
+  } else {
+    if (p.split > 1) gemm_kn_kernel<true, false><<<blocks, 256, 0, stream>>>(p);
+    else gemm_kn_kernel<false, false><<<blocks, 256, 0, stream>>>(p);
+  }
 }
 
 }  // namespace nga

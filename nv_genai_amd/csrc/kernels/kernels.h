@@ -262,7 +262,8 @@ void launch_embed_layernorm(const int32_t* ids, const int32_t* pos, const int32_
                             const uint16_t* ptab, int n_pos, const uint16_t* ttab, int n_type, const uint16_t* g,
                             const uint16_t* b, float eps, int64_t rows, int H, uint16_t* out, hipStream_t stream);
 
-// gemm_kn.hip: out[M, N] = x[M, K] . w[K, N], bf16, or fp32 slabs [split, M, N]; K % 32 == 0, N % 256 == 0, K / 32 >= 8 split
+// gemm_kn.hip: out[M, N] = x[M, K] . w[K, N], bf16, or fp32 slabs [split, M, N]; K % 32 == 0, N % 256 == 0, K >= 256 a slice. xt: x lies as
+// [K, M], M % 256 == 0, any K
 struct GemmKnParams {
   const uint16_t *x, *w;
   int64_t ldx;
@@ -270,7 +271,7 @@ struct GemmKnParams {
   int M, N, K, split;
 };
 int gemm_kn_split(int64_t M, int64_t N, int64_t K);
-void launch_gemm_kn(const GemmKnParams& p, hipStream_t stream);
+void launch_gemm_kn(const GemmKnParams& p, bool xt, hipStream_t stream);
 
 // gemm_nt.hip: out[M, N] = GELU(x[M, K] . w[N, K]^T + bias); N % 256 == 0, K % 32 == 0, K >= 256. covers: and faster than the library's
 // product and a launch of bias and GELU

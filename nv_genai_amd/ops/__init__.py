@@ -246,10 +246,17 @@ def stream_gemm(x: torch.Tensor, w: torch.Tensor, epi: int = 0) -> torch.Tensor:
 def gemm_kn_covers(M: int, N: int, K: int) -> bool:
     """Whether x [M, K] . w [K, N] (a frozen projection's gradient, w as it lies) is faster through gemm_kn.hip than the library's
     product: contractions so long that splitting them fills the chip, and few rows. us, library / here: K 28,672, N 4,096, M 64 / 512 /
-    1,024 / 2,048: 166 87, 284 117, 348 192, 382 352; K 128,256: 471 308, 855 427, 1,442 785, 1,587 1,521; K 6,144, M 128 / 512 / 1,024:
-    46 30, 47 44, 57 60; K 4,096, M 128 / 200: 32 23, 23 27; N 14,336, M 128 / 1,024: 42 41, 98 101."""
+    1,024 / 2,048: 165 69, 285 120, 348 192, 382 352; K 128,256: 474 241, 856 440, 1,442 785, 1,587 1,521; K 6,144, M 128 / 512 / 1,024:
+    46 27, 49 45, 57 60; K 4,096, M 128 / 200: 34 24, 26 29; N 14,336, M 128 / 1,024: 44 43, 98 101."""
     return (M >= 1 and N % 256 == 0 and N >= 256 and K % 32 == 0 and N < 1 << 20 and K < 1 << 22
             and (K >= 16384 and M <= 2048 and N <= 8192 or M <= 128 and N <= 4096 and K >= 4096))
+
+
+def weight_grad_covers(T: int, N: int, K: int) -> bool:
+    """Whether dy [T, N]^T . x [T, K], the gradient of a weight, is faster through gemm_kn.hip than the library's product, whose tiles do
+    not fill the chip and which does not split T enough. us, library / here, T 4,096 / 5,000 / 10,240: 3,072 x 1,024 45 56 96, 43 48 69;
+    1,024 x 1,024 29 37 66, 32 33 39; 4,096 x 1,024 47 59 105, 50 56 84; 768 x 768 29 37 60, 29 30 34."""
+    return T >= 5000 and T < 1 << 24 and all(d >= 256 and d % 256 == 0 and d < 1 << 20 for d in (N, K))
 
 
 def norm_linear_covers(x: torch.Tensor, norm_w: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:

@@ -3,7 +3,7 @@
 Each takes the place of a chain of single torch operations in :mod:`.functional` (forward and backward): activations bf16,
 statistics, sums and the gradients of weights fp32, weights either fp32 masters or bf16. Activations are bit for bit those of
 the chain. So are, all weights trained, their gradients and those of matrices; the gradients of norms' weights and of biases
-are fp32 sums over the rows in the kernels' own order. ``attention``, ``lora_linear`` and the ``once`` forms, for adapters, form
+are fp32 sums over the rows in the kernels' own order, and so are those of ``linear``'s matrices over some thousand rows. ``attention``, ``lora_linear`` and the ``once`` forms, for adapters, form
 the activations' gradients in that too. Callers ask ``usable`` first; the torch operations stay for the CPU, other types and
 sizes, and under transforms that pass functions of this kind by (tracing, functorch, forward-mode). Where a graph of the
 backward is asked for (create_graph) the gradients come from torch operations; ``attention``, like the flash attention that it
@@ -76,9 +76,15 @@ class _Linear(Function):
             return tuple(_again(torch.nn.functional.linear, (x, w, b), dy))
         dy2 = _rows(dy.reshape(-1, dy.shape[-1]))
         dx = (dy2 @ w).view(x.shape) if ctx.needs_input_grad[0] else None
-        dw = dy2.t() @ x.reshape(-1, x.shape[-1]) if ctx.needs_input_grad[1] else None
+        dw = _weight_grad(dy2, x.reshape(-1, x.shape[-1])) if ctx.needs_input_grad[1] else None
         db = ops.kernels().col_sums(dy2) if ctx.needs_input_grad[2] else None
         return dx, dw, db
+
+
+def _weight_grad(dy2: torch.Tensor, x2: torch.Tensor) -> torch.Tensor:
+    if dy2.dtype is BF16 and x2.dtype is BF16 and ops.weight_grad_covers(dy2.shape[0], dy2.shape[1], x2.shape[1]):
+        return ops.kernels().gemm_kn(_rows(dy2), _rows(x2), True)
+    return dy2.t() @ x2
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
@@ -353,7 +359,7 @@ class _FrozenLinear(Function):
 
 def _input_grad(dy2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if ops.gemm_kn_covers(dy2.shape[0], w.shape[1], w.shape[0]) and w.is_contiguous() and w.data_ptr() % 16 == 0 and dy2.dtype is BF16:
-        return ops.kernels().gemm_kn(_rows(dy2), w)
+        return ops.kernels().gemm_kn(_rows(dy2), w, False)
     return dy2 @ w
 
 

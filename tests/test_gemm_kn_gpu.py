@@ -19,10 +19,26 @@ def test_gemm_kn(gpu, M, N, K, apart):
     g = torch.Generator(gpu).manual_seed(M + K)
     x = torch.randn(M, K + apart, device=gpu, generator=g).to(BF)[:, :K]
     w = torch.randn(K, N, device=gpu, generator=g).to(BF)
-    got = ops.kernels().gemm_kn(x, w)
+    got = ops.kernels().gemm_kn(x, w, False)
     want, mag = x.double() @ w.double(), x.double().abs() @ w.double().abs()
     assert ((got.double() - want).abs() <= 2 ** -8 * want.abs() + 2 ** -24 * K ** 0.5 * mag).all()
-    assert torch.equal(got, ops.kernels().gemm_kn(x, w))
+    assert torch.equal(got, ops.kernels().gemm_kn(x, w, False))
+
+
+# last stages of each kind: whole, one row, all but one; slices of each count; columns of a wider matrix
+@pytest.mark.parametrize("K,M,N,apart", [(256, 256, 256, 0), (257, 256, 512, 8), (287, 512, 256, 0), (1000, 768, 1024, 0), (10_240, 1024, 4096, 0),
+                                         (8_743, 3072, 1024, 0), (4_096, 4096, 4096, 64), (300, 16384, 1024, 0)])
+def test_gemm_kn_of_transposed_rows(gpu, K, M, N, apart):
+    """The bound of test_gemm_kn; infinities in rows that the last stage has twice come once."""
+    g = torch.Generator(gpu).manual_seed(M + K)
+    x = torch.randn(K, M + apart, device=gpu, generator=g).to(BF)[:, :M]
+    w = torch.randn(K, N, device=gpu, generator=g).to(BF)
+    got = ops.kernels().gemm_kn(x, w, True)
+    want, mag = x.double().t() @ w.double(), x.double().abs().t() @ w.double().abs()
+    assert ((got.double() - want).abs() <= 2 ** -8 * want.abs() + 2 ** -24 * K ** 0.5 * mag).all()
+    x[K - 30, 3], w[K - 30] = float("inf"), w[K - 30].abs() + 1
+    got = ops.kernels().gemm_kn(x, w, True)
+    assert (got[3] == float("inf")).all() and got.isfinite().sum() == got.numel() - N
 
 
 @pytest.mark.parametrize("shape,N", [((2, 40), 16384), ((700,), 16384), ((3, 0), 16384), ((100,), 4096), ((100,), 4128)])
@@ -80,3 +96,18 @@ def test_gemm_nt_gelu_at_the_ends(gpu):
     fin = want.isfinite()
     assert torch.equal(got.isnan(), want.isnan()[:, None].expand_as(got)) and (got[want == float("inf")] == float("inf")).all()
     assert ((got[fin].double() - want[fin, None]).abs() <= 2 ** -8 * want[fin, None].abs() + 3e-7).all()
+
+
+@pytest.mark.parametrize("T", [4999, 5000, 6003])
+def test_weight_gradients(gpu, T):
+    """fused.linear's weight gradient on both sides of the line, of rows that lie apart in memory: the library's to one bf16 step."""
+    from nv_genai_amd.training import fused
+
+    x = torch.randn(T, 264, device=gpu).to(BF)[:, :256]
+    w = torch.randn(512, 256, device=gpu).requires_grad_()
+    b = torch.zeros(512, device=gpu, requires_grad=True)
+    assert ops.weight_grad_covers(T, 512, 256) == (T >= 5000)
+    dy = torch.randn(T, 512, device=gpu).to(BF)
+    got, = torch.autograd.grad(fused.linear(x, w, b), w, dy)
+    want, mag = dy.double().t() @ x.double(), dy.double().abs().t() @ x.double().abs()
+    assert got.dtype == torch.float32 and ((got.double() - want).abs() <= 2 ** -8 * want.abs() + 2 ** -24 * T ** 0.5 * mag).all()
