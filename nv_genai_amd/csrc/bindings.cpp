@@ -1610,9 +1610,12 @@ std::vector<Tensor> ivf_search(Tensor q, Tensor X, Tensor bias, Tensor ids, Tens
   auto* items = reinterpret_cast<nga::ScanItem*>(tab.data_ptr<int32_t>());
   int32_t *cnt = tab.data_ptr<int32_t>() + 8 * max_items, *probes = cnt + nq, *run_item = probes + npairs,
           *qtab = run_item + blocks + 1;
+  nga::IvfOne one{};
+  if (nq == 1) one = {sl, blocks, list_beg.data_ptr<int64_t>(), list_end.data_ptr<int64_t>(), items, run_item, qtab};
   nga::launch_ivf_probe(q.data_ptr<float>(), q.stride(0), (int)nq, D, (int)metric, centroids.data_ptr<float>(), (int)nlist,
-                        (int)nprobe, bfp(qb), cnt, probes, s.st);
-  nga::launch_ivf_items(probes, (int)npairs, (int)nprobe, (int)nlist, sl, (int)max_items, blocks, list_beg.data_ptr<int64_t>(),
+                        (int)nprobe, bfp(qb), cnt, probes, one, s.st);
+  if (nq > 1)
+    nga::launch_ivf_items(probes, (int)npairs, (int)nprobe, (int)nlist, sl, (int)max_items, blocks, list_beg.data_ptr<int64_t>(),
                         list_end.data_ptr<int64_t>(), items, run_item, qtab, s.st);
   s.a.Q = bfp(qb);
   s.a.cnt = cnt;

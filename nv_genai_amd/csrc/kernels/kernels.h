@@ -230,8 +230,14 @@ void launch_scan(const ScanArgs& a, int ng, int K, int blocks, hipStream_t strea
 bool scan_wide_covers(int D, int ng);           // flat scans of more than 16 queries
 void launch_scan_wide(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream);
 void launch_search_prep(const float* q, int64_t q_stride, int nq, int D, int metric, uint16_t* qb, hipStream_t stream);
+struct IvfOne {   // for a single query: what launch_ivf_items makes, in the same launch; items null: not
+  int sl, blocks;
+  const int64_t *lbeg, *lend;
+  ScanItem* items;
+  int32_t *run_item, *qtab;
+};
 void launch_ivf_probe(const float* q, int64_t q_stride, int nq, int D, int metric, const float* cent, int nlist, int nprobe,
-                      uint16_t* qb, int32_t* cnt, int32_t* probes, hipStream_t stream);
+                      uint16_t* qb, int32_t* cnt, int32_t* probes, const IvfOne& one, hipStream_t stream);
 void launch_ivf_items(const int32_t* probes, int npairs, int nprobe, int nlist, int sl, int max_items, int blocks,
                       const int64_t* lbeg, const int64_t* lend, ScanItem* items, int32_t* run_item, int32_t* qtab,
                       hipStream_t stream);

@@ -122,6 +122,73 @@ __global__ void __launch_bounds__(256) search_prep_kernel(const float* __restric
     if (4 * lane + 256 * j < D) *reinterpret_cast<u16x4*>(qb + row * D + 4 * lane + 256 * j) = wq.bf(j);
 }
 
+// Plans of the scan by one workgroup of 1,024 threads, thread t for list t with `mine` probing queries: items of sl query slots
+// in list order, and run_item[b], the item with which workgroup b of the scan begins, so that a scan workgroup is two dependent loads
+// away from its first vectors. Returns the first item of the thread's list.
+namespace {
+struct PlanShared {
+  int items[1024], tiles[1024], len[1024];   // of a list: its first item, its tiles and those before it, tiles of an item
+  int wave[2][16];
+};
+
+__device__ __forceinline__ int ivf_plan(PlanShared& s, int mine, int nlist, int sl, int blocks, const int64_t* __restrict__ lbeg,
+                                        const int64_t* __restrict__ lend, ScanItem* __restrict__ items, int32_t* __restrict__ run_item) {
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  int m = 0, tl = 0;
+  int64_t lb = 0, le = 0;
+  if (t < nlist) {
+    m = (mine + sl - 1) / sl;
+    lb = lbeg[t];
+    le = lend[t];
+    tl = le > lb ? (int)((le - lb + SS_ROWS - 1) / SS_ROWS) : 0;
+  }
+  int si = m, st = m * tl;   // sums up to this list
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int a = __shfl_up(si, o, 64), b = __shfl_up(st, o, 64);
+    si += lane >= o ? a : 0;
+    st += lane >= o ? b : 0;
+  }
+  if (lane == 63) {
+    s.wave[0][w] = si;
+    s.wave[1][w] = st;
+  }
+  __syncthreads();
+  int total = 0;
+#pragma unroll
+  for (int o = 0; o < 16; ++o) {
+    si += o < w ? s.wave[0][o] : 0;
+    st += o < w ? s.wave[1][o] : 0;
+    total += s.wave[1][o];
+  }
+  const int ib = si - m, tb = st - m * tl;
+  s.items[t] = ib;
+  s.tiles[t] = st;
+  s.len[t] = tl;
+  for (int j = 0; j < m; ++j) {
+    ScanItem it;
+    it.tile0 = tb + j * tl;
+    it.tile1 = it.tile0 + tl;
+    it.nq = mine - j * sl < sl ? mine - j * sl : sl;
+    it.unused = 0;
+    it.beg = lb;
+    it.end = le;
+    items[ib + j] = it;
+  }
+  __syncthreads();
+  for (int b = t; b < blocks; b += 1024) {
+    const int g = (int)((int64_t)total * b / blocks);
+    if (total == 0) break;
+    int l = 0;   // the first list whose tiles end behind g
+#pragma unroll
+    for (int o = 512; o > 0; o >>= 1) l += s.tiles[l + o - 1] <= g ? o : 0;
+    run_item[b] = s.items[l] + (g - (l ? s.tiles[l - 1] : 0)) / s.len[l];
+  }
+  if (t == 0) run_item[blocks] = total;
+  return ib;
+}
+}  // namespace
+
 // One workgroup per query: its bf16 form, its products with every centroid (rounded to bf16 as the stored vectors are,
 // sums in fp32; a wave takes four centroids at once, all their loads in flight), each centroid's rank by counting, the
 // nprobe first ones. Takes the place of the preparation, a cast, a score launch over one row tile (11 us) and a radix
@@ -129,8 +196,9 @@ __global__ void __launch_bounds__(256) search_prep_kernel(const float* __restric
 __global__ void __launch_bounds__(1024) ivf_probe_kernel(const float* __restrict__ q, int64_t q_stride, int D, int metric,
                                                          const float* __restrict__ cent, int nlist, int nprobe,
                                                          uint16_t* __restrict__ qb, int32_t* __restrict__ cnt,
-                                                         int32_t* __restrict__ probes) {
+                                                         int32_t* __restrict__ probes, IvfOne one) {
   __shared__ uint32_t sk[IVF_SCAN_MAX_LISTS];
+  __shared__ PlanShared ps;
   const int64_t row = blockIdx.x;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   WaveQuery wq;
@@ -166,65 +234,41 @@ __global__ void __launch_bounds__(1024) ivf_probe_kernel(const float* __restrict
   }
   __syncthreads();
   const int c = threadIdx.x;
+  bool first = false;
   if (c < nlist) {
     const uint32_t mine = sk[c];
     int rank = 0;
-    for (int o = 0; o < nlist; ++o) rank += sk[o] > mine || (sk[o] == mine && o < c);
-    if (rank < nprobe) probes[row * nprobe + rank] = c;
+#pragma unroll 16
+    for (int o = 0; o < nlist; ++o) {
+      const uint32_t x = sk[o];
+      rank += x > mine || (x == mine && o < c);
+    }
+    first = rank < nprobe;
+    if (first) probes[row * nprobe + rank] = c;
   }
+  if (one.items == nullptr) return;
+  // the only query: its items, one a list, here, instead of in a launch of 8 us
+  const int item = ivf_plan(ps, first, nlist, one.sl, one.blocks, one.lbeg, one.lend, one.items, one.run_item);
+  if (first)
+    for (int o = 0; o < one.sl; ++o) one.qtab[item * one.sl + o] = o ? -1 : 0;
 }
 
 // One workgroup groups the (query, probe) pairs by list: list l with n probing queries becomes ceil(n / sl) items of sl
-// query slots (-1: empty), items in list order. run_item[b] is the item with which workgroup b of the scan begins, so
-// that a scan workgroup is two dependent loads away from its first vectors.
+// query slots (-1: empty).
 __global__ void __launch_bounds__(1024) ivf_items_kernel(const int32_t* __restrict__ probes, int npairs, int nprobe, int nlist,
                                                          int sl, int max_items, int blocks, const int64_t* __restrict__ lbeg,
                                                          const int64_t* __restrict__ lend, ScanItem* __restrict__ items,
                                                          int32_t* __restrict__ run_item, int32_t* __restrict__ qtab) {
-  __shared__ int cnt[IVF_SCAN_MAX_LISTS], base[IVF_SCAN_MAX_LISTS], sm[1024], st[1024];
+  __shared__ int cnt[IVF_SCAN_MAX_LISTS], base[IVF_SCAN_MAX_LISTS];
+  __shared__ PlanShared ps;
   const int t = threadIdx.x;
   cnt[t] = 0;
   for (int i = t; i < max_items * sl; i += 1024) qtab[i] = -1;
   __syncthreads();
   for (int i = t; i < npairs; i += 1024) atomicAdd(&cnt[probes[i]], 1);
   __syncthreads();
-  int m = 0, tl = 0, mine = cnt[t];
-  int64_t lb = 0, le = 0;
-  if (t < nlist) {
-    m = (mine + sl - 1) / sl;
-    lb = lbeg[t];
-    le = lend[t];
-    tl = le > lb ? (int)((le - lb + SS_ROWS - 1) / SS_ROWS) : 0;
-  }
-  sm[t] = m;
-  st[t] = m * tl;
-  __syncthreads();
-  for (int o = 1; o < 1024; o <<= 1) {
-    const int a = t >= o ? sm[t - o] : 0, b = t >= o ? st[t - o] : 0;
-    __syncthreads();
-    sm[t] += a;
-    st[t] += b;
-    __syncthreads();
-  }
-  const int ib = sm[t] - m, tb = st[t] - m * tl;
-  const int64_t total = st[1023];
-  for (int j = 0; j < m; ++j) {
-    const int t0 = tb + j * tl, t1 = t0 + tl;
-    ScanItem it;
-    it.tile0 = t0;
-    it.tile1 = t1;
-    it.nq = mine - j * sl < sl ? mine - j * sl : sl;
-    it.unused = 0;
-    it.beg = lb;
-    it.end = le;
-    items[ib + j] = it;
-    // the workgroups whose first tile lies in [t0, t1): total * b / blocks >= t0 from b = ceil(t0 * blocks / total)
-    if (t1 > t0)
-      for (int64_t b = ((int64_t)t0 * blocks + total - 1) / total; b < blocks && total * b / blocks < t1; ++b) run_item[b] = ib + j;
-  }
-  if (t == 0) run_item[blocks] = (int)total;
-  base[t] = ib;
-  cnt[t] = 0;
+  base[t] = ivf_plan(ps, cnt[t], nlist, sl, blocks, lbeg, lend, items, run_item);
+  cnt[t] = 0;   // its own, read above
   __syncthreads();
   for (int i = t; i < npairs; i += 1024) {
     const int p = probes[i], rank = atomicAdd(&cnt[p], 1);
@@ -963,8 +1007,8 @@ void launch_search_prep(const float* q, int64_t q_stride, int nq, int D, int met
 }
 
 void launch_ivf_probe(const float* q, int64_t q_stride, int nq, int D, int metric, const float* cent, int nlist, int nprobe,
-                      uint16_t* qb, int32_t* cnt, int32_t* probes, hipStream_t stream) {
-  ivf_probe_kernel<<<nq, 1024, 0, stream>>>(q, q_stride, D, metric, cent, nlist, nprobe, qb, cnt, probes);
+                      uint16_t* qb, int32_t* cnt, int32_t* probes, const IvfOne& one, hipStream_t stream) {
+  ivf_probe_kernel<<<nq, 1024, 0, stream>>>(q, q_stride, D, metric, cent, nlist, nprobe, qb, cnt, probes, one);
 }
 
 void launch_ivf_items(const int32_t* probes, int npairs, int nprobe, int nlist, int sl, int max_items, int blocks,
