@@ -1272,11 +1272,13 @@ int encoder_split(int64_t M, int64_t N, int64_t K) {
 }
 
 // Most rows that the LDS tiles take: beyond, the library's larger tiles are faster than these without their launches' cost on the
-// host. Where they meet lies at 1.2e9 rows x hidden^2: a forward, library / here, us: 1,024 x 24 layers at 1,152 rows 2,391 2,314,
-// 1,280 2,378 2,397; 768 x 12 at 1,536 rows 1,130 948, 2,048 1,122 1,125, 3,072 1,383 1,481; 512 x 8 at 4,096 756 771. Small models
-// are bound by the host's launches there: embedding token lists with 384 x 6 layers, 1,152 rows 723 329, 4,096 873 518, 9,600
-// 1,215 945, 19,200 1,828 1,636 (the forward alone over and over: 9,600 rows of 12 layers 1,370 1,625).
-int64_t encoder_tile_rows(int64_t H) { return H <= 384 ? 20480 : std::max<int64_t>(1024, 1200000000 / (H * H)); }
+// host. Where they meet lies at 1.2e9 to 1.34e9 rows x hidden^2: a forward, library / here, us: 1,024 x 24 layers at 1,280 rows 2,378
+// 2,255, 1,536 2,438 2,711; 768 x 12 at 1,536 rows 1,130 950, 2,048 1,122 1,140, 3,072 1,383 1,481; 512 x 8 at 4,096 756 771, 6,400 854 1,076.
+// Small models are bound by the host's launches there: embedding token lists with 384 x 6 layers, 1,152 rows 723 329, 4,096 873
+// 518, 9,600 1,215 945, 19,200 1,828 1,636 (the forward alone over and over: 9,600 rows of 12 layers 1,370 1,625).
+int64_t encoder_tile_rows(int64_t H) {
+  return H <= 384 ? 20480 : std::max<int64_t>(1024, (H < 768 ? 1200000000 : 1343000000) / (H * H));
+}
 
 // nullptr, or why encoder_forward does not take these weights; tables: positions, types, the embedding norm's weight and bias
 const char* encoder_refuses(const Tensor& word, const std::vector<Tensor>& tables, const std::vector<Tensor>& L, int64_t heads) {

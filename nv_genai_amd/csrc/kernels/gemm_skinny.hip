@@ -36,6 +36,7 @@
 // up rows [F, 2F)), 3 = bf16 out + bias, 4 = bf16 out, GELU (erf form) of . + bias.
 #include <cstdlib>
 
+#include <cstdint>
 #include "common.h"
 #include "kernels.h"
 
@@ -481,42 +482,60 @@ void launch_skinny_gemm(const SkinnyGemmParams& p, int cfg, int epi, hipStream_t
 #undef NGA_LAUNCH
 }
 
-// Encoder projections (K 384 to 4,096): 64 x 64 tiles up to 512 rows, 64 x 128 above; 32 features a tile where 64 would take half
-// the CUs or fewer, since a CU draws some 47 bytes a nanosecond from its L2 and these are bound by that (BERT-large, 64 rows: the
-// forward 1,100 us with 64, 990 with 32; 128 rows 1,124 and 1,010). Two groups of waves where each workgroup has a CU of its own
-// (208 rows: up 12.1 us with one, 10.2 with two; q/k/v 9.8 and 9.0); not for the slabs, whose K range is short (6.9 and 7.3).
-// A rotated walk over K (krot) lost 5 %: tiles that share rows no longer read them together. With 64-feature tiles and one group,
-// weights from HBM (us, library / here): 64 rows q/k/v 11.4 / 7.6, output 8.4 / 4.1, up 11.6 / 7.7, down 14.8 / 7.5; 512 rows
-// 10.8 / 10.3, 8.5 / 5.6, 10.6 / 10.2, 13.8 / 11.6; 1,024 rows 14.1 / 13.8, 9.5 / 7.9, 13.6 / 14.1 (and its GELU launch of 4.6 saved), 18.9 / 17.3; at
-// 1,536 rows the library's larger tiles win everywhere.
-static int skinny_tile(SkinnyGemmParams& p, int* bn) {
-  const int bm = p.M <= 512 ? 64 : 128;
-  p.nM = (p.M + bm - 1) / bm;
-  *bn = p.M <= 512 && (p.N + 63) / 64 * p.nM * p.split <= 128 ? 32 : 64;
-  p.nN = (p.N + *bn - 1) / *bn;
-  return p.nN * p.nM * p.split;
+// Encoder projections (K 384 to 4,096). A CU draws some 47 bytes a nanosecond from its L2 and these are bound by that: what counts is
+// the longest time of a CU, its tiles times their rows and features. Of four tiles (features x rows) the one with the least is taken,
+// the smaller of equal ones. BERT-large, the forward, with 64 rows a tile up to 512 and 128 above, 64 features (32 where 64 filled half the
+// CUs or fewer), and so: 300 rows 1,328 us, 1,281; 512 1,490 1,405; 768 1,802 1,727; 1,024 1,959 1,772 (up 20.4 us a layer with 512 tiles
+// of 64 x 128). Slabs of a short K keep 64 rows up to 512: what they draw is little (768 x 12 layers, 512 rows 604 us, with 64 593).
+// Two groups of waves over K where each workgroup has a CU of its own (208 rows: up 12.1 us with one, 10.2 with two; 64 x 128 at 512 rows
+// the forward 1,470, 1,405), or eight waves (128 x 128 at 1,024 rows: 1,922 with four, 1,772); not for the slabs, whose K range is short
+// (6.9 and 7.3). A rotated walk over K (krot) lost 5 %: tiles that share rows no longer read them together.
+namespace {
+struct SkTile {
+  int bn, bm;
+};
+}  // namespace
+static SkTile skinny_tile(SkinnyGemmParams& p) {
+  constexpr SkTile all[4] = {{32, 64}, {64, 64}, {64, 128}, {128, 128}};
+  const bool short_slabs = p.split > 1 && p.K / p.split <= 256 && p.M <= 512;
+  SkTile best = all[1];
+  int64_t least = INT64_MAX;
+  for (const SkTile& t : all) {
+    if (short_slabs && t.bm > 64) break;
+    const int64_t n = (int64_t)((p.N + t.bn - 1) / t.bn) * ((p.M + t.bm - 1) / t.bm) * p.split, c = (n + 255) / 256 * (t.bn + t.bm);
+    if (c < least) {
+      least = c;
+      best = t;
+    }
+  }
+  p.nM = (p.M + best.bm - 1) / best.bm;
+  p.nN = (p.N + best.bn - 1) / best.bn;
+  return best;
 }
 
 void launch_skinny_bias(SkinnyGemmParams p, bool gelu, hipStream_t stream) {
   p.split = 1;
-  int bn;
-  const int nblk = skinny_tile(p, &bn);
+  const SkTile t = skinny_tile(p);
+  const int nblk = p.nN * p.nM;
   if (nblk == 0) return;
-#define NGA_SB(EPI)                                                                                        \
-  if (p.M > 512) skinny_gemm_kernel<64, 128, 1, 4, 3, EPI, 64><<<nblk, 256, 0, stream>>>(p);               \
-  else if (bn == 32) skinny_gemm_kernel<32, 64, 2, 2, 4, EPI, 64, 2><<<nblk, 512, 0, stream>>>(p);         \
-  else if (nblk <= 256) skinny_gemm_kernel<64, 64, 2, 2, 4, EPI, 64, 2><<<nblk, 512, 0, stream>>>(p);      \
+#define NGA_SB(EPI)                                                                                                                \
+  if (t.bn == 128) skinny_gemm_kernel<128, 128, 2, 4, 4, EPI, 64><<<nblk, 512, 0, stream>>>(p);                                    \
+  else if (t.bm == 128 && nblk <= 256) skinny_gemm_kernel<64, 128, 1, 4, 3, EPI, 64, 2><<<nblk, 512, 0, stream>>>(p);              \
+  else if (t.bm == 128) skinny_gemm_kernel<64, 128, 1, 4, 3, EPI, 64><<<nblk, 256, 0, stream>>>(p);                                \
+  else if (t.bn == 32) skinny_gemm_kernel<32, 64, 2, 2, 4, EPI, 64, 2><<<nblk, 512, 0, stream>>>(p);                               \
+  else if (nblk <= 256) skinny_gemm_kernel<64, 64, 2, 2, 4, EPI, 64, 2><<<nblk, 512, 0, stream>>>(p);                              \
   else skinny_gemm_kernel<64, 64, 2, 2, 4, EPI, 64><<<nblk, 256, 0, stream>>>(p)
   if (gelu) { NGA_SB(4); } else { NGA_SB(3); }
 #undef NGA_SB
 }
 
 void launch_skinny_slabs(SkinnyGemmParams p, hipStream_t stream) {
-  int bn;
-  const int nblk = skinny_tile(p, &bn);
+  const SkTile t = skinny_tile(p);
+  const int nblk = p.nN * p.nM * p.split;
   if (nblk == 0) return;
-  if (p.M > 512) skinny_gemm_kernel<64, 128, 1, 4, 3, 1, 64><<<nblk, 256, 0, stream>>>(p);
-  else if (bn == 32) skinny_gemm_kernel<32, 64, 2, 2, 4, 1, 64><<<nblk, 256, 0, stream>>>(p);
+  if (t.bn == 128) skinny_gemm_kernel<128, 128, 2, 4, 4, 1, 64><<<nblk, 512, 0, stream>>>(p);
+  else if (t.bm == 128) skinny_gemm_kernel<64, 128, 1, 4, 3, 1, 64><<<nblk, 256, 0, stream>>>(p);
+  else if (t.bn == 32) skinny_gemm_kernel<32, 64, 2, 2, 4, 1, 64><<<nblk, 256, 0, stream>>>(p);
   else skinny_gemm_kernel<64, 64, 2, 2, 4, 1, 64><<<nblk, 256, 0, stream>>>(p);
 }
 

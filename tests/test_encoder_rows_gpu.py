@@ -71,9 +71,11 @@ def test_rows_forward(gpu, H, heads, F, lens):
     assert torch.equal(got, hidden())
 
 
-# above 1,024 rows: the smallest, the last of hidden 1,024 and of 768 with LDS tiles, K slices of each count
-@pytest.mark.parametrize("H,heads,F,T", [(384, 12, 1536, 1025), (384, 12, 1536, 2047), (128, 2, 256, 4100), (768, 12, 3072, 2034),
-                                         (1024, 16, 4096, 1144), (1024, 16, 4096, 1145), (384, 12, 1536, 9001)])
+# each tile with rows and features that do not fill it; above 1,024 rows the smallest, the last of hidden 1,024 and of 768 with LDS
+# tiles, K slices of each count
+@pytest.mark.parametrize("H,heads,F,T", [(384, 12, 1536, 1025), (384, 12, 1536, 2047), (128, 2, 256, 4100), (768, 12, 3072, 2276),
+                                         (1024, 16, 4096, 1280), (1024, 16, 4096, 1281), (384, 12, 1536, 9001), (1024, 16, 4096, 301),
+                                         (1024, 16, 4096, 513), (1024, 16, 4096, 1001), (192, 6, 448, 700), (768, 12, 3072, 511)])
 def test_many_rows_forward(gpu, H, heads, F, T):
     test_rows_forward(gpu, H, heads, F, [64] * (T // 64) + [T % 64])
 
