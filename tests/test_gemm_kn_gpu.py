@@ -72,7 +72,7 @@ def test_frozen_linear(gpu, shape, N):
                                          (4200, 4096, 1024, 24), (9000, 3072, 768, 0), (3000, 1024, 4096, 0)])
 def test_gemm_nt_gelu(gpu, M, N, K, apart):
     """The fp32 sum's error grows with the root of the terms (2^-24 of their magnitudes each); GELU's slope is at most 1.13, and its form
-    here is within 3e-7 of the exact one; then one rounding to bf16."""
+    here is within 1e-7 of the exact one; then one rounding to bf16."""
     g = torch.Generator(gpu).manual_seed(M + K)
     x = torch.randn(M, K + apart, device=gpu, generator=g).to(BF)[:, :K]
     w = torch.randn(N, K, device=gpu, generator=g).mul_(2 / K ** 0.5).to(BF)
@@ -80,11 +80,13 @@ def test_gemm_nt_gelu(gpu, M, N, K, apart):
     sums, mag = x.double() @ w.double().t() + b.double(), x.double().abs() @ w.double().abs().t() + b.double().abs()
     want = torch.nn.functional.gelu(sums)
     got = ops.kernels().gemm_nt_gelu(x, w, b)
-    assert ((got.double() - want).abs() <= 2 ** -8 * want.abs() + 1.13 * 2 ** -24 * K ** 0.5 * mag + 3e-7 * sums.abs()).all()
+    assert ((got.double() - want).abs() <= 2 ** -8 * want.abs() + 1.13 * 2 ** -24 * K ** 0.5 * mag + 1e-7 * sums.abs()).all()
 
 
 def test_gemm_nt_gelu_at_the_ends(gpu):
-    """Sums of every size, infinities and NaN: K values of which one counts."""
+    """Sums of every size, infinities and NaN: K values of which one counts. Down to -7.5 a small result has its digits (relative 1.3e-4
+    before its rounding to bf16, where 1 + erf has none); below, GELU is at most 2.4e-13, and its form, which lacks the logarithm's last
+    change there, less than twice that."""
     v = torch.cat([torch.linspace(-12, 12, 4001), torch.tensor([0.0, -0.0, 1e-30, -1e-30, 3e38, -3e38, float("inf"), float("-inf"), float("nan")])])
     x = torch.zeros(v.numel(), 256, device=gpu, dtype=BF)
     x[:, 0] = v.to(gpu)
@@ -95,7 +97,8 @@ def test_gemm_nt_gelu_at_the_ends(gpu):
     want = torch.where(a == 0, a, a * 0.5 * torch.erfc(-a * 0.5 ** 0.5))   # torch's own loses the digits of a small 1 + erf
     fin = want.isfinite()
     assert torch.equal(got.isnan(), want.isnan()[:, None].expand_as(got)) and (got[want == float("inf")] == float("inf")).all()
-    assert ((got[fin].double() - want[fin, None]).abs() <= 2 ** -8 * want[fin, None].abs() + 3e-7).all()
+    rel = 2 ** -8 + torch.where(a < -7.5, 1.0, 1.4e-4)   # half a bf16 step, and GELU's own
+    assert ((got[fin].double() - want[fin, None]).abs() <= (rel * want.abs())[fin, None] + 2.0 ** -133).all()
 
 
 @pytest.mark.parametrize("T", [4999, 5000, 6003])
