@@ -1227,12 +1227,17 @@ def decode_attention(q, kc, vc, block_tables, ctx_lens, Hq, Hkv, max_ctx, scale,
 
 
 def decode_step_covers(qkv, kc, ctx_lens, slots, max_ctx, ws: Optional[DecodeWorkspace], window: int = 0) -> bool:
-    """Whether :func:`decode_step` runs this step: bf16 pages of head_dim 128 on the GPU, one new token a row."""
+    """Whether :func:`decode_step` runs this step: bf16 pages of head_dim 128 on the GPU, one new token a row, and at most two
+    workgroups a CU, one for each row and KV head. Each of them waits for its rows of q/k/v and the rotation before its first page, which
+    in further rounds costs more than the launches saved (how long the contexts are is known on the GPU alone). 8B (8 KV heads), a whole
+    layer with rows of 300 to 1,400 tokens, us, in launches of their own / in one: 1 row 96.7 91.1, 16 121.0 116.3, 32 139.4 133.7, 64 170.3
+    167.0, 72 191.5 191.0, 80 194.3 195.0, 96 209.4 213.5, 128 232.8 242.3, 256 356 381; of 32 to 200 tokens 64 141.1 132.6, 256 253.7 245.4;
+    32 KV heads, 12 rows 152.2 150.5, 16 165.7 165.4, 20 168.6 170.4, 48 245 263; 2 KV heads, 256 rows 248.3 245.3, 512 357.9 356.9."""
     t = qkv.slabs if isinstance(qkv, PartialSum) else qkv
     B = ctx_lens.numel()
     return (_gpu(t) and kc.dtype == torch.bfloat16 and kc.shape[3] == 128 and ws is not None and ws.D == 128 and max_ctx <= ws.max_ctx
             and t.is_contiguous() and t.dtype == (torch.float32 if t.dim() == 3 else torch.bfloat16) and t.data_ptr() % 16 == 0
-            and slots is not None and t.shape[-2] == B == slots.numel() and B * kc.shape[1] <= ws.done.numel()
+            and slots is not None and t.shape[-2] == B == slots.numel() and B * kc.shape[1] <= min(512, ws.done.numel())
             and kernels().decode_step_covers(B, int(max_ctx), ws.pages_per_part(B, max_ctx), int(window)))
 
 

@@ -64,6 +64,26 @@ def test_decode_step_is_rotation_and_attention(gpu, G, Hkv, ppp, window, slabs):
         assert ((g - w).abs() <= 2 ** -8 * w.abs() + 2 ** -8 * w.abs().amax(1, keepdim=True)).all()
 
 
+@pytest.mark.parametrize("rows,Hkv,one", [(64, 8, True), (65, 8, False), (16, 32, True), (17, 32, False), (256, 2, True), (512, 1, True), (513, 1, False)])
+def test_many_rows_take_launches_of_their_own(gpu, rows, Hkv, one):
+    """From more than two workgroups a CU on the rotation stands alone; at the line both give the same."""
+    D, dev = 128, gpu
+    ctxs = [1 + (37 * i) % 150 for i in range(rows)]
+    kc, vc, bt, slots = _pages(ctxs, Hkv, dev)
+    qkv = torch.randn(rows, 3 * Hkv * D, device=dev).to(torch.bfloat16)
+    ctx, cs = torch.tensor(ctxs, dtype=torch.int32, device=dev), ops.rope_cos_sin(256, D).to(dev)
+    ws = ops.DecodeWorkspace(rows, Hkv, Hkv, 192, dev)
+    assert ops.decode_step_covers(qkv, kc, ctx, slots, 192, ws) == one
+    if not one:
+        return
+    k1, v1, flat = kc.clone(), vc.clone(), qkv.clone()
+    got = ops.decode_step(qkv, ctx - 1, cs, slots, kc, vc, bt, ctx, Hkv, Hkv, 192, D ** -0.5, ws).float()
+    ops.rope_cache_(flat, ctx - 1, cs, slots, k1, v1, Hkv, Hkv, D)
+    want = ops.decode_attention(flat[:, : Hkv * D], k1, v1, bt, ctx, Hkv, Hkv, 192, D ** -0.5, ws=ws).float()
+    assert torch.equal(kc, k1) and torch.equal(vc, v1)
+    assert ((got - want).abs() <= 2 ** -8 * want.abs() + 2 ** -8 * want.abs().amax(1, keepdim=True)).all()   # as above
+
+
 @pytest.mark.parametrize("N,K", [(4096, 4096), (6144, 4096), (16, 256), (48, 768), (1008, 2304), (14336, 4096), (512, 8192), (384, 5120),
                                  (101, 520), (33, 1032), (7, 8), (2064, 8184)])
 @pytest.mark.parametrize("epi", [1, 2])
