@@ -681,10 +681,9 @@ void decode_step(Tensor out, Tensor qkv, Tensor pos, Tensor cos_sin, Tensor slot
   st.kc = bfp(kc);
   st.vc = bfp(vc);
   st.done = done.data_ptr<int32_t>();
-  // a hint only: weights in another form are not read ahead
+  // a hint only: weights in another form, or of another kernel, are not read ahead
   if (next.has_value() && next->device() == qkv.device() && next->scalar_type() == at::kBFloat16 && next->dim() == 2 && next->is_contiguous() &&
-      next->size(1) % 128 == 0 && next->size(1) < (1 << 20) && next->size(0) % 16 == 0 && next->numel() <= (int64_t(1) << 26) &&
-      reinterpret_cast<uintptr_t>(next->data_ptr()) % 16 == 0) {
+      nga::stream_gemm_reads_ahead(B, next->size(0), next->size(1)) && reinterpret_cast<uintptr_t>(next->data_ptr()) % 16 == 0) {
     st.next = bfp(*next);
     st.next_pieces = (int)(next->size(0) / 16);
     st.next_kb = (int)(next->size(1) / 128);
@@ -2916,6 +2915,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("splitk_reduce", checked("splitk_reduce", &splitk_reduce));
   m.def("splitk_swiglu", checked("splitk_swiglu", &splitk_swiglu));
   m.def("stream_gemm", checked("stream_gemm", &stream_gemm));
+  m.def("stream_gemm_reads_ahead", &nga::stream_gemm_reads_ahead);
   m.def("stream_gemm_covers", &nga::stream_gemm_covers);
   m.def("gemv", checked("gemv", &gemv));
   m.def("splitk_add_rmsnorm", checked("splitk_add_rmsnorm", &splitk_add_rmsnorm));

@@ -316,7 +316,8 @@ __device__ __forceinline__ float get_agent(const float* p) {
 
 // A workgroup without keys reads its share of the weights that the next launch streams, so that these come from the caches:
 // for short contexts most CUs have no keys (one sequence of 227 tokens: 8 of 128 workgroups) and HBM would lie idle while the
-// others wait for their first bytes. Piece t, the rows of the next kernel's workgroup t, goes to the die that will run that.
+// others wait for their first bytes. Piece t, the rows of the next kernel's workgroup t, goes to the die that will run that; only
+// weights of which this holds, and few enough of them, are given here (stream_gemm_reads_ahead).
 // What the loads bring into LDS is never looked at. 8B, one sequence of 227 tokens: output projection (33.5 MB) 7.9 -> 5.4 us, attention
 // 8.5 -> 9.2; where all partitions have keys nothing is read ahead.
 __device__ __forceinline__ void warm_next(const DecodeStep& st, uint16_t* lds, int w, int lane) {

@@ -216,10 +216,20 @@ bool stream_gemm_covers(int64_t M, int64_t N, int64_t K, bool swiglu) {
 // 32 rows a workgroup (half the token traffic) where 16 would give some CUs two workgroups and others one, or from 9 tokens on.
 // 4,096 x 4,096 at 8 rows: 16 rows 8.2 us, 32 rows 9.5; 6,144 x 4,096: 12.5, 10.9; SwiGLU 14,336 x 4,096: 40.6, 42.3, at 16
 // rows 49.6, 44.7
+static bool st_two(int64_t M, int64_t N, int64_t t) { return t > 256 && (t < 1024 || M > 8) && N % 32 == 0; }
+
+// The read-ahead warms the L2 of the die that runs a 16-row workgroup of this kernel; weights that others take, or that are cut into
+// other pieces, would come to the wrong dies, and what is read must be there before the slowest attention workgroup ends. One row of a
+// short context, a layer with / without, us: 4,096 x 4,096 (33.5 MB) 88.8 90.8, 3,072 x 3,072 55.2 56.1, 2,048 x 2,048 44.8 45.4; read ahead
+// all the same, 5,120 x 5,120 111.5 107.9, 6,144 x 6,144 161.9 155.5, 8,192 x 8,192 310.5 299.5. 2 to 16 rows of 4,096: 0.3 to 0.9 less.
+bool stream_gemm_reads_ahead(int64_t M, int64_t N, int64_t K) {
+  return stream_gemm_covers(M, N, K, false) && !st_two(M, N, st_tiles(N, false)) && N * K <= (int64_t(1) << 24);
+}
+
 void launch_stream_gemm(const StreamGemmParams& p, int epi, hipStream_t stream) {
   const int t = (int)st_tiles(p.N, epi == 2);
   if (p.M == 0 || t == 0) return;
-  const bool two = t > 256 && (t < 1024 || p.M > 8) && p.N % 32 == 0;
+  const bool two = st_two(p.M, p.N, t);
 #define NGA_ST(EPI, NJ)                                                                  \
   if (two) stream_gemm_kernel<2, EPI, NJ><<<t / 2, 256, 0, stream>>>(p);                 \
   else stream_gemm_kernel<1, EPI, NJ><<<t, 256, 0, stream>>>(p)

@@ -444,6 +444,7 @@ struct StreamGemmParams {
   float eps;
 };
 bool stream_gemm_covers(int64_t M, int64_t N, int64_t K, bool swiglu);
+bool stream_gemm_reads_ahead(int64_t M, int64_t N, int64_t K);   // whether a launch ahead of it does well to read its weights
 void launch_stream_gemm(const StreamGemmParams& p, int epi, hipStream_t stream);
 
 struct SkinnyGemmParams {

@@ -64,6 +64,14 @@ def test_decode_step_is_rotation_and_attention(gpu, G, Hkv, ppp, window, slabs):
         assert ((g - w).abs() <= 2 ** -8 * w.abs() + 2 ** -8 * w.abs().amax(1, keepdim=True)).all()
 
 
+@pytest.mark.parametrize("rows,N,K,ahead", [(1, 4096, 4096, True), (16, 4096, 4096, True), (1, 2048, 2048, True), (1, 5120, 5120, False), (1, 8192, 8192, False),
+                                           (4, 6144, 4096, False), (1, 8192, 4096, False), (1, 4096, 8192, False), (17, 4096, 4096, False),
+                                           (1, 4096, 4000, False)])
+def test_weights_are_read_ahead_for_the_kernel_that_takes_them(gpu, rows, N, K, ahead):
+    """The stream kernel with 16 weight rows a workgroup, and up to 33.5 MB."""
+    assert ops.kernels().stream_gemm_reads_ahead(rows, N, K) == ahead
+
+
 @pytest.mark.parametrize("rows,Hkv,one", [(64, 8, True), (65, 8, False), (16, 32, True), (17, 32, False), (256, 2, True), (512, 1, True), (513, 1, False)])
 def test_many_rows_take_launches_of_their_own(gpu, rows, Hkv, one):
     """From more than two workgroups a CU on the rotation stands alone; at the line both give the same."""
