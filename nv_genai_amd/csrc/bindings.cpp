@@ -1270,13 +1270,18 @@ int encoder_split(int64_t M, int64_t N, int64_t K) {
   return M <= 1024 ? (int)most : (int)std::max<int64_t>(1, std::min(most, 512 / tiles));
 }
 
-// Most rows that the LDS tiles take: beyond, the library's larger tiles are faster than these without their launches' cost on the
-// host. Where they meet lies at 1.2e9 to 1.34e9 rows x hidden^2: a forward, library / here, us: 1,024 x 24 layers at 1,280 rows 2,378
-// 2,255, 1,536 2,438 2,711; 768 x 12 at 1,536 rows 1,130 950, 2,048 1,122 1,140, 3,072 1,383 1,481; 512 x 8 at 4,096 756 771, 6,400 854 1,076.
-// Small models are bound by the host's launches there: embedding token lists with 384 x 6 layers, 1,152 rows 723 329, 4,096 873
-// 518, 9,600 1,215 945, 19,200 1,828 1,636 (the forward alone over and over: 9,600 rows of 12 layers 1,370 1,625).
+// Most rows that the LDS tiles take: beyond, the library's larger tiles are faster. A whole forward, us, of the GPU alone (a captured graph)
+// and of calls in a row, which the launches of the library's products bound on the host where models are small; library / here, each:
+// 1,024 x 24 layers at 1,200 rows 2,237 2,216, 2,337 2,228, 1,340 2,403 2,498, 2,413 2,512; 896 x 12 at 1,408 1,010 1,041, 1,083 1,072,
+// 1,700 1,080 1,232, 1,093 1,258; 768 x 12 at 1,280 786 779, 1,121 827, 1,700 925 961, 1,130 1,003, 2,000 1,039 1,136, 1,124 1,167; 640 x 12 at
+// 2,304 982 1,033, 1,126 1,053, 3,500 1,180 1,349, 1,206 1,378; 512 x 12 at 3,584 994 983, 1,062 1,009, 4,608 1,168 1,215, 1,199 1,245; 448 x
+// 12 at 6,144 1,217 1,215, 1,242 1,236; 384 x 6 at 5,500 513 536, 535 555, 6,500 560 552, 589 567, 7,168 531 569, 559 584, 9,600 638 704,
+// 658 718; 320 x 6 at 8,192 558 530, 587 551, 12,288 665 734, 689 754; 256 x 4 at 8,192 356 289, 408 307, 14,000 394 405, 422 431; 128 x 2
+// at 20,480 167 164, 274 188. The line is where calls meet: rows x hidden^2 of 9.4e8, above hidden 640 more, and for small models rows x
+// hidden of 2.6e6, since norms and slabs, and no products, bound those. Up to 1,024 rows stay as they were measured at 1,024 features.
 int64_t encoder_tile_rows(int64_t H) {
-  return H <= 384 ? 20480 : std::max<int64_t>(1024, (H < 768 ? 1200000000 : 1343000000) / (H * H));
+  const int64_t products = (940000000 + std::max<int64_t>(0, H - 640) * 800000) / (H * H);
+  return std::max<int64_t>(1024, std::min(products, 2600000 / H));
 }
 
 // nullptr, or why encoder_forward does not take these weights; tables: positions, types, the embedding norm's weight and bias
@@ -2923,6 +2928,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("embedding", checked("embedding", &embedding));
   m.def("score", checked("score", &score));
   m.def("topk", checked("topk", &topk));
+  m.def("encoder_tile_rows", &encoder_tile_rows);
   m.def("encoder_forward", &encoder_forward, py::call_guard<py::gil_scoped_release>());   // some 200 launches
   m.def("encoder_covers", [](const Tensor& word, const std::vector<Tensor>& tables, const std::vector<Tensor>& L, int64_t heads) {
     return encoder_refuses(word, tables, L, heads) == nullptr;

@@ -80,6 +80,27 @@ def test_many_rows_forward(gpu, H, heads, F, T):
     test_rows_forward(gpu, H, heads, F, [64] * (T // 64) + [T % 64])
 
 
+# rows at which both ways were timed: the last with the LDS tiles ahead, the first with the library's products ahead
+@pytest.mark.parametrize("H,tiles,library", [(128, 20_000, 36_000), (192, 12_288, 20_480), (256, 8_192, 14_000), (320, 8_000, 12_288),
+                                             (384, 6_144, 9_600), (448, 4_096, 7_000), (512, 3_500, 4_608), (576, 2_048, 3_584), (640, 2_048, 3_500),
+                                             (704, 1_792, 2_560), (768, 1_700, 1_900), (896, 1_408, 1_700), (1024, 1_100, 1_340), (1536, 1_024, 1_025)])
+def test_tiles_end_where_the_library_is_faster(gpu, H, tiles, library):
+    assert tiles <= ops.kernels().encoder_tile_rows(H) < library
+
+
+def test_no_hidden_size_jumps(gpu):
+    """Neighbouring sizes (64 apart) take the tiles up to neighbouring row counts: neither product nor quotient of rows and size jumps."""
+    rows = {H: ops.kernels().encoder_tile_rows(H) for H in range(64, 4097, 64)}
+    assert all(rows[H] >= rows[H + 64] >= rows[H] * (H / (H + 64)) ** 2 - 1 for H in range(64, 4096, 64) if H >= 128)
+
+
+@pytest.mark.parametrize("H,heads,F", [(1024, 16, 4096), (768, 12, 3072), (384, 12, 1536)])
+@pytest.mark.parametrize("more", [0, 1])
+def test_forward_on_both_sides_of_the_line(gpu, H, heads, F, more):
+    T = ops.kernels().encoder_tile_rows(H) + more
+    test_rows_forward(gpu, H, heads, F, [64] * (T // 64) + [T % 64])
+
+
 def test_rows_of_another_sequence_do_not_mix(gpu):
     """A token outside the table gives its own sequence NaN and no other; infinities in one stay there."""
     from nv_genai_amd.models.config import encoder_config
