@@ -255,8 +255,13 @@ def gemm_kn_covers(M: int, N: int, K: int) -> bool:
 def weight_grad_covers(T: int, N: int, K: int) -> bool:
     """Whether dy [T, N]^T . x [T, K], the gradient of a weight, is faster through gemm_kn.hip than the library's product, whose tiles do
     not fill the chip and which does not split T enough. us, library / here, T 4,096 / 5,000 / 10,240: 3,072 x 1,024 45 56 96, 43 48 69;
-    1,024 x 1,024 29 37 66, 32 33 39; 4,096 x 1,024 47 59 105, 50 56 84; 768 x 768 29 37 60, 29 30 34."""
-    return T >= 5000 and T < 1 << 24 and all(d >= 256 and d % 256 == 0 and d < 1 << 20 for d in (N, K))
+    1,024 x 1,024 29 37 66, 32 33 39; 4,096 x 1,024 47 59 105, 50 56 84; 768 x 768 29 37 60, 29 30 34. From 129 tiles of 256 x 256 on there
+    is one slice, and up to 159, and from 257 to 359, too few of them in the last round (T 8,192: 144 tiles 157 162, 165 174 163, 256 228 196,
+    272 304 347, 320 330 347, 360 358 349, 400 507 350, 576 541 539, 768 690 617, 1,024 912 816)."""
+    if T < 5000 or T >= 1 << 24 or not all(d >= 256 and d % 256 == 0 and d < 1 << 20 for d in (N, K)):
+        return False
+    tiles = N // 256 * (K // 256)
+    return not (128 < tiles < 160 or 256 < tiles < 360)
 
 
 def norm_linear_covers(x: torch.Tensor, norm_w: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:

@@ -114,3 +114,10 @@ def test_weight_gradients(gpu, T):
     got, = torch.autograd.grad(fused.linear(x, w, b), w, dy)
     want, mag = dy.double().t() @ x.double(), dy.double().abs().t() @ x.double().abs()
     assert got.dtype == torch.float32 and ((got.double() - want).abs() <= 2 ** -8 * want.abs() + 2 ** -24 * T ** 0.5 * mag).all()
+
+
+@pytest.mark.parametrize("N,K,here", [(2048, 4096, True), (6144, 1536, False), (7680, 1280, False), (5120, 2048, True), (4096, 4096, True), (4096, 4352, False),
+                                      (6144, 3072, False), (5120, 4608, True), (8192, 4096, True), (256, 256, True), (256, 128, False), (300, 256, False)])
+def test_weight_gradients_by_their_tiles(gpu, N, K, here):
+    """128 tiles, 144, 150, 160, 256, 272, 288, 360, 512, 1: the counts that leave CUs idle are the library's."""
+    assert ops.weight_grad_covers(8192, N, K) == here
