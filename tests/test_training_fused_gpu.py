@@ -301,3 +301,28 @@ def test_half_params_keep_the_gradients(gpu):
     assert torch.equal(ya, yb)
     for k in gb:
         assert torch.equal(ga[k], gb[k]), k
+
+
+def test_checkpointed_embedding_step_holds_no_copies(gpu):
+    """With checkpointing a step's loss holds the layers' inputs (two short texts) and no bf16 copy of the weights (21 MB); its loss and
+    gradients are those without."""
+    import gc
+
+    from nv_genai_amd.engine.embed_engine import EmbeddingEngine
+    from nv_genai_amd.training.embed_finetune import embed_trainer
+    from nv_genai_amd.training.sft import TrainConfig
+
+    eng, got = EmbeddingEngine("all-minilm-l6-v2", device=gpu), []
+    recs = [{"question": "one two", "pos_doc": ["three four"], "neg_doc": ["five six"]}] * 2
+    for ckpt in (True, False):
+        tr, P = embed_trainer(eng, recs, TrainConfig(micro_batch=2, global_batch=2, max_steps=2, log_every=0, grad_ckpt=ckpt), hard_negatives=1)
+        tr.loss_fn(tr.data[0]).backward()   # libraries' workspaces are there
+        for p in P.values():
+            p.grad = None
+        gc.collect()
+        before = torch.cuda.memory_allocated()
+        loss = tr.loss_fn(tr.data[0])
+        assert not ckpt or torch.cuda.memory_allocated() - before < 5e6
+        loss.backward()
+        got.append((loss.item(), {k: p.grad for k, p in P.items()}))
+    assert got[0][0] == got[1][0] and all(torch.equal(got[0][1][k], got[1][1][k]) for k in got[0][1])
