@@ -2954,6 +2954,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("grad_norm", on_device(&grad_norm));
   m.def("adamw", on_device(&adamw));
   m.def("train_attention_backward", on_device(&train_attention_backward));
+  m.def("scan_wide_covers", &nga::scan_wide_covers);
   m.def("flat_search", &flat_search);
   m.def("ivf_search", &ivf_search);
   m.def("search_covers", [](int64_t d) { return d <= 1024 && nga::scan_chunk((int)d, 1) > 0; });

@@ -539,12 +539,21 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
 // LDS is then a ring of NSL units (16 rows) a wave, which all stay under way. The sums are handed over in the accumulators'
 // layout, so that a lane ends with four rows of one query as in the other kernel; wave w takes rows 16 (w & 1) .. and every
 // second group of queries. Bound by the stream: 1M x 1,024, k 4, whole search, before and here, 17 / 33 / 64 queries: 322 372
-// 493 us, 307 299 336; k 25 (scores) 434 473 568, 412 445 504; 250k x 768, k 4: 88 100 126, 69 81 96; 10k x 384: 20 23 27, 17 19 20.
-// Dimensions are those that come in earnest (384, 768, 1,024); each takes its own registers.
+// 493 us, 307 299 336; k 25 (scores) 434 473 568, 412 445 504; 250k x 768, k 4: 88 100 126, 69 81 96; 10k x 384: 20 23 27, 17 19 20; 1M x 512,
+// k 4: 200 240 315, 183 218 272; x 640, 33 / 64: 287 371, 232 285; x 896, 17 / 33 / 64: 316 358 451, 267 283 343; x 256, 17 / 64: 153 245, 140 228.
+// Of 128 dimensions two barriers for 8 KB cost more than the smaller queries in LDS (1M, 17 / 33 / 64: 77 111 103, here 126 175 215); left there
+// too are 33 to 48 queries of 256 (1M 178, 189; 100k 41, 36) and 17 to 32 of 640 (1M 207, 214; 100k 39, 36). Each dimension takes its own registers.
 namespace {
-constexpr int wide_slots(int KS, int NG) { return KS == 8 ? (NG == 4 ? 3 : 4) : KS == 6 ? 5 : 10; }   // of 4 KS KiB for all waves
-constexpr int wide_swizzle(int KS) { return KS % 4 == 0 ? 15 : KS % 2 == 0 ? 7 : 3; }
 constexpr int WIDE_BIAS = 8;   // tiles whose biases have a place, more than are under way
+// which numbers of groups (NG) it takes of 128 KS dimensions
+constexpr bool wide_takes(int KS, int NG) { return NG >= 2 && NG <= 4 && KS >= 2 && KS <= 8 && !(KS == 2 && NG == 3) && !(KS == 5 && NG == 2); }
+// units of 4 KS KiB for all waves that fill the LDS beside the sums and the biases, ten at most (384 dimensions, 33 queries: 205 us with ten and
+// 213 with eleven)
+constexpr int wide_slots(int KS, int NG) {
+  const int n = (160 - 8 * NG - WIDE_BIAS / 4) / (4 * KS);
+  return n < 10 ? n : 10;
+}
+constexpr int wide_swizzle(int KS) { return KS % 4 == 0 ? 15 : KS % 2 == 0 ? 7 : 3; }
 template <int N>
 __device__ __forceinline__ void wide_wait() {
   static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
@@ -672,6 +681,7 @@ __global__ void __launch_bounds__(256, 1) scan_wide_kernel(ScanArgs p) {
   };
   // younger than unit u when its turn comes: the NSL - 1 units behind it, a bias before each even one. Stores of scores are not
   // counted: they may be done before older loads
+  static_assert(NSL / 2 + 2 <= WIDE_BIAS, "biases under way and of the tile in hand lie apart");
   constexpr int Y0 = (NSL - 1) * KS + (NSL - 1) / 2, Y1 = (NSL - 1) * KS + NSL / 2;
   int n = 0;
   for (; 2 * n + 1 + NSL < units; ++n) {
@@ -976,25 +986,33 @@ void launch_scan(const ScanArgs& a, int ng, int K, int blocks, hipStream_t strea
 }
 
 // 17 to 64 queries of all rows, prepared
-bool scan_wide_covers(int D, int ng) { return ng >= 2 && ng <= 4 && (D == 384 || D == 768 || D == 1024); }
+bool scan_wide_covers(int D, int ng) { return D % 128 == 0 && wide_takes(D / 128, ng); }
 
 template <int NG, int K, int KS>
 static void wide_go(const ScanArgs& a, int blocks, hipStream_t stream) {
-  static const bool attr = [] {
-    (void)hipFuncSetAttribute((const void*)scan_wide_kernel<NG, K, KS>, hipFuncAttributeMaxDynamicSharedMemorySize, SS_LDS);
-    (void)hipGetLastError();
-    return true;
-  }();
-  (void)attr;
-  scan_wide_kernel<NG, K, KS><<<blocks, 256, wide_lds(NG, KS), stream>>>(a);
+  if constexpr (wide_takes(KS, NG)) {
+    static const bool attr = [] {
+      (void)hipFuncSetAttribute((const void*)scan_wide_kernel<NG, K, KS>, hipFuncAttributeMaxDynamicSharedMemorySize, SS_LDS);
+      (void)hipGetLastError();
+      return true;
+    }();
+    (void)attr;
+    scan_wide_kernel<NG, K, KS><<<blocks, 256, wide_lds(NG, KS), stream>>>(a);
+  }
 }
 
 void launch_scan_wide(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream) {
 #define NGA_WIDE(NG_, K_)                                              \
   if (ng == NG_ && K == K_) {                                          \
-    if (a.D == 1024) return wide_go<NG_, K_, 8>(a, blocks, stream);    \
-    if (a.D == 768) return wide_go<NG_, K_, 6>(a, blocks, stream);     \
-    return wide_go<NG_, K_, 3>(a, blocks, stream);                     \
+    switch (a.D / 128) {                                               \
+      case 2: return wide_go<NG_, K_, 2>(a, blocks, stream);           \
+      case 3: return wide_go<NG_, K_, 3>(a, blocks, stream);           \
+      case 4: return wide_go<NG_, K_, 4>(a, blocks, stream);           \
+      case 5: return wide_go<NG_, K_, 5>(a, blocks, stream);           \
+      case 6: return wide_go<NG_, K_, 6>(a, blocks, stream);           \
+      case 7: return wide_go<NG_, K_, 7>(a, blocks, stream);           \
+      case 8: return wide_go<NG_, K_, 8>(a, blocks, stream);           \
+    }                                                                  \
   }
   NGA_WIDE(2, 0); NGA_WIDE(2, 4); NGA_WIDE(2, 8); NGA_WIDE(2, 16);
   NGA_WIDE(3, 0); NGA_WIDE(3, 4); NGA_WIDE(3, 8);

@@ -1852,13 +1852,19 @@ def search_covers(X: torch.Tensor, k: int, most: int = 256) -> bool:
 def search_many(nq: int, rows: int, D: int, k: int) -> bool:
     """Whether many queries over all rows are faster through ``search_topk``, whose kernel (vector_search.hip) holds 64 queries
     in registers' reach and reads the vectors straight into fragments: then the products bound the scan and not the stream of
-    vectors. The line lies at 4.5e10 products of whole groups of 64 queries, vectors below 512 dimensions counted as such, for
-    what its register lists hold (k 8); of 1,024 dimensions on at 512 queries besides, where the flat scan's groups of 64 in
-    registers keep up. k 4, us, this / that: 1M x 1,024, 65 queries 748 / 657, 512: 2,232 / 2,144; 100k x 1,024, 512: 314 / 270,
-    4,096: 1,737 / 1,714; 300k x 768, 256: 376 / 356, 1,024: 1,098 / 1,229; 1M x 384, 128: 422 / 463, 1,024: 2,089 / 3,041; 300k x
-    256, 256: 241 / 243, 1,000: 616 / 762; 1M x 128, 1,000: 1,206 / 987."""
-    return (nq > 64 and k <= kernels().score_topk_kmax(64) and D >= 256 and not (D >= 1024 and nq <= 512)
-            and -(-nq // 64) * 64 * rows * max(D, 512) >= 4.5e10)
+    vectors. Its cost of 64 queries more is the lower one the shorter the vectors are, the flat scan's of the first 64, so the line is one of
+    rows x groups of 64 queries: (D / 400)^1.5 million up to 4 results, 0.45 of that up to 8, which is what its register lists hold. k 4, us,
+    this / that, 128 / 256 / 512 / 1,024 queries: 300k x 256 161 222 348 566, 156 275 494 916; 300k x 384 190 283 460 775, 168 298 541 1,008;
+    300k x 512 235 326 529 879, 178 316 575 1,064; 1M x 512 521 814, 498 918; 300k x 640 283 384 607 1,026, 187 333 612 1,150; 1M x 768 691 1,048
+    1,835 3,385, 566 1,052 2,000 3,857; 300k x 896 322 454 748 1,300, 216 389 712 1,337; k 8: 300k x 384 245 362, 236 419; 300k x 768 345 489 789,
+    267 482 853; 1M x 896 857 1,405 2,488, 790 1,404 2,530. At 1,024 dimensions both are level from 512 queries on, and the line lies there and at
+    4.5e10 products (1M, 128 / 512 / 2,048: 814 2,291 8,132, 608 2,147 7,954; 100k, 4,096: 1,737 / 1,714). 1M x 128, 1,000: 1,206 / 987."""
+    groups = -(-nq // 64)
+    if nq <= 64 or D < 256 or k > kernels().score_topk_kmax(64):
+        return False
+    if D >= 1024:
+        return nq > 512 and groups * 64 * rows * D >= 4.5e10
+    return groups * rows > (D / 400) ** 1.5 * (1e6 if k <= 4 else 4.5e5)
 
 
 def search_many_lists(nq: int, rows: int, D: int, k: int, nlist: int, nprobe: int) -> bool:

@@ -187,6 +187,19 @@ def test_flat_search_of_many_against_fp64(gpu, D, N, nq, k):
     test_flat_search_against_fp64(gpu, N, D, nq, k, ("ip", "cosine", "l2")[N % 3])
 
 
+# the other dimensions, with the ring's length of each: the last rows of a workgroup's units, one workgroup's only tile
+@pytest.mark.parametrize("D", [128, 256, 512, 640, 896])
+@pytest.mark.parametrize("N,nq,k", [(1, 17, 1), (33, 64, 8), (8193, 32, 16), (24_577, 48, 17), (100_001, 33, 4), (100_001, 65, 25), (70_000, 129, 8)])
+def test_flat_search_of_many_of_other_dimensions_against_fp64(gpu, D, N, nq, k):
+    test_flat_search_against_fp64(gpu, N, D, nq, k, ("ip", "cosine", "l2")[N % 3])
+
+
+def test_flat_search_takes_what_it_was_measured_for(gpu):
+    """17 to 32, 33 to 48 and 49 to 64 queries of each dimension with the queries in registers, but where the other kernel is faster."""
+    took = {D: [ng for ng in (1, 2, 3, 4, 5) if ops.kernels().scan_wide_covers(D, ng)] for D in (64, *range(128, 1153, 128))}
+    assert took == {64: [], 128: [], 256: [2, 4], 640: [3, 4], 1152: [], **{D: [2, 3, 4] for D in (384, 512, 768, 896, 1024)}}
+
+
 def test_flat_search_equal_scores_and_strided_queries(gpu):
     """More equal scores than the selection sorts at once (one vector many times), with lists and with scores; queries
     that are every second row of a wider matrix."""

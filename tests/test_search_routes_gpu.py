@@ -42,6 +42,17 @@ def test_flat_of_many_short_vectors_or_few_queries(gpu):
     assert not ops.search_many(10_000, 10 ** 7, 128, 4) and not ops.search_many(64, 10 ** 8, 1024, 4)
 
 
+# points that were timed, the faster one by more than a twentieth each
+@pytest.mark.parametrize("D,rows,nq,k,topk", [(256, 300_000, 256, 4, True), (256, 100_000, 128, 4, False), (384, 300_000, 512, 4, True), (384, 100_000, 256, 4, False),
+                                              (512, 1_000_000, 256, 4, True), (512, 300_000, 128, 4, False), (640, 1_000_000, 512, 4, True),
+                                              (640, 1_000_000, 128, 4, False), (768, 1_000_000, 1024, 4, True), (768, 1_000_000, 128, 4, False),
+                                              (768, 300_000, 192, 4, False), (896, 300_000, 256, 4, False), (896, 1_000_000, 128, 4, False),
+                                              (384, 300_000, 256, 8, True), (640, 300_000, 256, 8, True), (768, 300_000, 192, 8, False),
+                                              (896, 100_000, 512, 8, False), (512, 100_000, 256, 9, False), (1024, 1_000_000, 512, 4, False)])
+def test_flat_line_agrees_with_the_measurements(gpu, D, rows, nq, k, topk):
+    assert ops.search_many(nq, rows, D, k) == topk
+
+
 @pytest.mark.parametrize("nq,nprobe,k,here", [(1024, 2, 4, False), (1024, 2, 9, True), (700, 2, 4, True)])
 def test_lists_of_many_queries(gpu, monkeypatch, nq, nprobe, k, here):
     """Two lists of 100,000 x 1,024 rows, both probed."""
