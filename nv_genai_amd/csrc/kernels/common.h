@@ -156,44 +156,6 @@ __device__ __forceinline__ float block_max(float v, float* red) {
   return t;
 }
 
-// Source of the qkv values: the bf16 projection output, or (part != nullptr) the S fp32 K-split
-// partial slabs of the skinny GEMM [S, T, row], summed here and rounded to bf16 exactly as the
-// materialised projection would be — the rotated / copied result is written to qkv either way,
-// so the projection output never makes a separate bf16 round trip.
-struct QkvSrc {
-  const float* part;
-  int S;
-  int64_t slab;   // T * row
-};
-
-__device__ __forceinline__ u16x8 qkv_ld8(const uint16_t* qkv, const QkvSrc& src, int64_t i) {
-  if (src.part == nullptr) return load8(qkv + i);
-  const float* p = src.part + i;
-  f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
-  for (int s = 1; s < src.S; ++s) {
-    a += *reinterpret_cast<const f32x4*>(p + s * src.slab);
-    b += *reinterpret_cast<const f32x4*>(p + s * src.slab + 4);
-  }
-  u16x8 r;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    r[j] = f2bf(a[j]);
-    r[4 + j] = f2bf(b[j]);
-  }
-  return r;
-}
-
-__device__ __forceinline__ u16x4 qkv_ld4(const uint16_t* qkv, const QkvSrc& src, int64_t i) {
-  if (src.part == nullptr) return *reinterpret_cast<const u16x4*>(qkv + i);
-  const float* p = src.part + i;
-  f32x4 a = *reinterpret_cast<const f32x4*>(p);
-  for (int s = 1; s < src.S; ++s) a += *reinterpret_cast<const f32x4*>(p + s * src.slab);
-  u16x4 r;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) r[j] = f2bf(a[j]);
-  return r;
-}
-
 // Counter-based RNG (splitmix64 finaliser) -> uniform in (0, 1].
 __device__ __forceinline__ float hash_uniform(uint64_t seed, uint64_t ctr) {
   uint64_t z = seed + 0x9E3779B97F4A7C15ull * (ctr + 1);

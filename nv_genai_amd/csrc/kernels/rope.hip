@@ -54,6 +54,44 @@ __device__ __forceinline__ void put1(CT* dst, uint16_t v, float inv_s) {
   }
 }
 
+// Source of the qkv values: the bf16 projection output, or (part != nullptr) the S fp32 K-split
+// partial slabs of the skinny GEMM [S, T, row], summed here and rounded to bf16 exactly as the
+// materialised projection would be — the rotated / copied result is written to qkv either way,
+// so the projection output never makes a separate bf16 round trip.
+struct QkvSrc {
+  const float* part;
+  int S;
+  int64_t slab;   // T * row
+};
+
+__device__ __forceinline__ u16x8 ld8(const uint16_t* qkv, const QkvSrc& src, int64_t i) {
+  if (src.part == nullptr) return load8(qkv + i);
+  const float* p = src.part + i;
+  f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
+  for (int s = 1; s < src.S; ++s) {
+    a += *reinterpret_cast<const f32x4*>(p + s * src.slab);
+    b += *reinterpret_cast<const f32x4*>(p + s * src.slab + 4);
+  }
+  u16x8 r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    r[j] = f2bf(a[j]);
+    r[4 + j] = f2bf(b[j]);
+  }
+  return r;
+}
+
+__device__ __forceinline__ u16x4 ld4(const uint16_t* qkv, const QkvSrc& src, int64_t i) {
+  if (src.part == nullptr) return *reinterpret_cast<const u16x4*>(qkv + i);
+  const float* p = src.part + i;
+  f32x4 a = *reinterpret_cast<const f32x4*>(p);
+  for (int s = 1; s < src.S; ++s) a += *reinterpret_cast<const f32x4*>(p + s * src.slab);
+  u16x4 r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) r[j] = f2bf(a[j]);
+  return r;
+}
+
 __device__ __forceinline__ uint32_t ld2(const uint16_t* qkv, const QkvSrc& src, int64_t i) {
   if (src.part == nullptr) return *reinterpret_cast<const uint32_t*>(qkv + i);
   const float* p = src.part + i;
@@ -87,8 +125,8 @@ __global__ void rope_cache_kernel(uint16_t* __restrict__ qkv, const int32_t* __r
       const int i0 = (w % G4) * 4;
       uint16_t* x = base + (int64_t)h * D;
       const int64_t xi = t * row + (int64_t)h * D;
-      u16x4 a = qkv_ld4(qkv, src, xi + i0);
-      u16x4 b = qkv_ld4(qkv, src, xi + HALF + i0);
+      u16x4 a = ld4(qkv, src, xi + i0);
+      u16x4 b = ld4(qkv, src, xi + HALF + i0);
       u16x4 oa, ob;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -110,7 +148,7 @@ __global__ void rope_cache_kernel(uint16_t* __restrict__ qkv, const int32_t* __r
       const int vh = r / (D / 8);
       const int d0 = (r % (D / 8)) * 8;
       const int64_t vi = (int64_t)(Hq + Hkv + vh) * D + d0;
-      u16x8 v = qkv_ld8(qkv, src, t * row + vi);
+      u16x8 v = ld8(qkv, src, t * row + vi);
       if (src.part != nullptr) store8(base + vi, v);
       if (slot >= 0) {
         CT* dst = vc + ((blk * Hkv + vh) * D + d0) * BS + off;
@@ -161,8 +199,8 @@ __global__ void __launch_bounds__(256) rope_cache_tiled_kernel(
 #pragma unroll
     for (int j = 0; j < HGMAX; ++j)
       if (h0 + j < h1) {
-        a[j] = qkv_ld8(qkv, src, xi + (int64_t)(h0 + j) * D);
-        b[j] = qkv_ld8(qkv, src, xi + (int64_t)(h0 + j) * D + HALF);
+        a[j] = ld8(qkv, src, xi + (int64_t)(h0 + j) * D);
+        b[j] = ld8(qkv, src, xi + (int64_t)(h0 + j) * D + HALF);
       }
     const float c[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
     const float sn[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
