@@ -267,6 +267,7 @@ def weight_grad_covers(T: int, N: int, K: int) -> bool:
 def norm_linear_covers(x: torch.Tensor, norm_w: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:
     """Whether :func:`norm_linear` runs rmsnorm(x [1, K]) @ w^T: one row (K <= 8,192) of bf16 on the GPU at 16-byte addresses."""
     return (_gpu(x) and x.dim() == 2 and x.shape[0] == 1 and x.numel() <= 8192 and x.shape[1] % 8 == 0 and w.shape[0] > 0
+            and not (swiglu and w.shape[0] % 2)
             and all(t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0 for t in (x, norm_w, w)) and w.is_contiguous()
             and norm_w.is_contiguous() and x.stride(1) == 1 and x.stride(0) % 8 == 0)
 

@@ -10,7 +10,8 @@ autograd on padded ``[B, S]`` batches:
   the framework's own kernel gives the flash attention's gradients on the GPU;
 * on the GPU norms with their residual, activations, rotation and cross entropy through the functions of
   :mod:`.fused`, elsewhere and for what those do not take through torch operations. All weights trained, a
-  step's loss and its gradients of matrices and embeddings are the torch operations' to the bit; the gradients of
+  step's loss and its gradients of matrices and embeddings are the torch operations' to the bit, but those of an
+  encoder's projections over 5,000 rows and more (``ops.weight_grad_covers``): these, the gradients of
   norms' weights and biases, the clipping norm and AdamW's update are fp32 sums in another order, so that weights
   differ by their last bits from the first step on. With adapters the activations keep their bits, and the
   gradients take the forms that are a single pass;
