@@ -2943,6 +2943,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("gelu_rows", on_device(&gelu_rows));
   m.def("gemm_kn", on_device(&gemm_kn));
   m.def("gemm_nt_gelu", on_device(&gemm_nt_gelu));
+  m.def("gemm_nt_gelu_covers", &nga::gemm_nt_gelu_covers);
   m.def("col_sums", on_device(&col_sums));
   m.def("half_copies", on_device(&half_copies));
   m.def("half_grads", on_device(&half_grads));

@@ -125,3 +125,68 @@ def test_linear_add(gpu, M, N, K):
     assert got.data_ptr() == resid.data_ptr()
     slack = 2 ** -24 * math.sqrt(K) * (x.double().abs() @ w.double().abs().t())
     assert ((got.double() - want).abs() <= 2 ** -8 * want.abs() + slack + 1e-6).all()
+
+
+def _step64(m, ids, pos, pages, bt, ctxs):
+    """Final-normed rows of one decode step in 64 bits; pages: K and V^T of every layer before it."""
+    c, D = m.cfg, m.D
+    d = lambda t: t.double()  # noqa: E731
+    rms = lambda x, w: x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + c.eps) * d(w)  # noqa: E731
+    x = d(m.embed)[ids.long()]
+    cos, sin = (t[:, None] for t in d(m.cos_sin[pos.long()]).split(D // 2, -1))
+    turn = lambda t: torch.cat([t[..., : D // 2] * cos - t[..., D // 2:] * sin, t[..., D // 2:] * cos + t[..., : D // 2] * sin], -1)  # noqa: E731
+    for li, L in enumerate(m.layers):
+        q, k, v = (t.unflatten(-1, (-1, D)) for t in (rms(x, L["attn_norm"]) @ d(L["wqkv"]).t()).split([m.hq * D, m.hkv * D, m.hkv * D], -1))
+        q, k, out = turn(q), turn(k), []
+        for b, n in enumerate(ctxs):
+            at = bt[b, : (n + 63) // 64].long()
+            K = d(pages[0][li, at].float()).transpose(1, 2).reshape(-1, m.hkv, D)[: n - 1]
+            V = d(pages[1][li, at].float()).permute(0, 3, 1, 2).reshape(-1, m.hkv, D)[: n - 1]
+            K, V = (torch.cat([a, t[b: b + 1]]).repeat_interleave(m.hq // m.hkv, 1) for a, t in ((K, k), (V, v)))
+            out.append(torch.einsum("hk,khd->hd", torch.softmax(torch.einsum("hd,khd->hk", q[b], K) * m.scale, -1), V).flatten())
+        x = x + torch.stack(out) @ d(L["wo"]).t()
+        g, u = (rms(x, L["mlp_norm"]) @ d(L["wgu"]).t()).chunk(2, -1)
+        x = x + (torch.nn.functional.silu(g) * u) @ d(L["wd"]).t()
+    return rms(x, m.final_norm)
+
+
+# one row with everything fused; pages of 256 dimensions and of fp8 behind the fused norms and residuals; a K that the GEMV takes; several rows
+@pytest.mark.parametrize("over,kv,ctxs,one", [({}, "auto", [300], True), ({}, "auto", [65], True), ({"heads": 2, "kv_heads": 1, "head_dim": 256}, "auto", [300], True),
+                                              ({}, "fp8", [300], True), ({"ffn": 1032}, "auto", [300], False), ({}, "auto", [300, 1, 64], False)])
+def test_a_models_decode_step(gpu, monkeypatch, over, kv, ctxs, one):
+    """Whether a step runs as _decode_layers, and its rows against 64 bits beside the same step in launches of their own: norms and
+    sums are rounded less often, so its error is theirs to within chance (a fifth at 512 values a row)."""
+    from nv_genai_amd.models.config import llama_config
+    from nv_genai_amd.models.llama import AttnMeta, LlamaModel
+
+    m = LlamaModel(llama_config("llama3-8b", **{**dict(layers=3, vocab_size=512, hidden=512, heads=4, kv_heads=2, head_dim=128, ffn=1024, max_position=512), **over}), gpu)
+    g = torch.Generator(gpu).manual_seed(11)
+    for L in m.layers:
+        for n in ("attn_norm", "mlp_norm"):
+            L[n].normal_(1, 0.1, generator=g)
+    m.embed.mul_(20)   # a residual stream of the size of what is added to it
+    pages = [(n + 63) // 64 for n in ctxs]
+    m.allocate_kv_cache(sum(pages) + 1, kv_dtype=kv)
+    for t in (m.k_cache, m.v_cache):
+        t.copy_(torch.randn(t.shape, device=gpu, generator=g).to(t.dtype))
+    before, bt, slots, at = [m.k_cache.clone(), m.v_cache.clone()], torch.zeros(len(ctxs), max(pages), dtype=torch.int32, device=gpu), [], 1
+    for b, n in enumerate(ctxs):
+        bt[b, : pages[b]] = torch.arange(at, at + pages[b])
+        at += pages[b]
+        slots.append(int(bt[b, (n - 1) // 64]) * 64 + (n - 1) % 64)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=gpu)  # noqa: E731
+    meta = AttnMeta(kind="decode", slots=i32(slots), cu_q=i32(list(range(len(ctxs) + 1))), ctx_lens=i32(ctxs), block_tables=bt, max_q_len=1,
+                    max_ctx=max(ctxs), decode_ws=ops.DecodeWorkspace(len(ctxs), m.hq, m.hkv, max(ctxs), gpu, D=m.D, kv_fp8=kv == "fp8"))
+    ids, pos = i32([7 + 3 * b for b in range(len(ctxs))]), i32([n - 1 for n in ctxs])
+    want, calls = _step64(m, ids, pos, before, bt, ctxs), []
+    monkeypatch.setattr(m, "_decode_layers", lambda *a, f=m._decode_layers: calls.append(1) or f(*a))
+    got = m.forward(ids, pos, meta)
+    assert bool(calls) == one
+    kept = m.k_cache.float()
+    rows = m.forward(ids, pos, meta, torch.tensor([0], device=gpu))
+    assert torch.equal(rows, got[:1]) and torch.equal(m.k_cache.float(), kept)
+    monkeypatch.setattr(m, "_fused_decode", lambda *a: False)
+    monkeypatch.setattr(ops, "decode_step_covers", lambda *a: False)
+    single = m.forward(ids, pos, meta)
+    err = lambda y: ((y.double() - want).norm() / want.norm()).item()  # noqa: E731
+    assert err(got) <= 1.2 * err(single) and err(single) < (0.1 if kv == "fp8" else 0.02), (err(got), err(single))

@@ -310,3 +310,30 @@ def test_a_gpu_that_is_not_the_current_one(gpu):
         opt.step(max_norm=1.0)
         got.append([t.detach().cpu() for t in w.values()])
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+def test_many_rows_change_only_the_matrices(gpu, monkeypatch):
+    """An encoder's step over 5,160 rows: its loss and its embeddings' gradients are the torch operations' to the bit, since a weight's
+    gradient moves nothing behind it; the projections' are fp32 sums in another order, rounded to bf16 (2^-8 at most, here of their norm)."""
+    from nv_genai_amd import ops
+    from nv_genai_amd.models.config import EncoderConfig
+    from nv_genai_amd.models.encoder import EncoderModel
+
+    m = EncoderModel(EncoderConfig(name="t", vocab_size=1000, hidden=256, layers=2, heads=4, ffn=512, max_position=136), gpu, seed=3)
+    ids, got, calls = torch.randint(0, 1000, (40, 129), device=gpu), [], []
+    monkeypatch.setattr(ops, "weight_grad_covers", lambda *a, f=ops.weight_grad_covers: f(*a) and not calls.append(a))
+    for fused_too in (True, False):
+        if not fused_too:
+            _without(monkeypatch)
+        P = Fn.trainable_params(m, "encoder")
+        with torch.autocast("cuda", dtype=BF):
+            loss = Fn.encoder_embed(m, ids, torch.ones_like(ids), P).pow(3).sum()
+        loss.backward()
+        got.append((loss.detach(), {k: p.grad for k, p in P.items()}))
+    (la, ga), (lb, gb) = got
+    assert len(calls) == 8 and torch.equal(la, lb)   # four projections a layer
+    for k in ga:
+        if not isinstance(k, tuple) and "emb_ln" not in k:
+            assert torch.equal(ga[k], gb[k]), k
+        elif ga[k].dim() == 2:
+            assert ((ga[k] - gb[k]).norm() <= 2 ** -8 * gb[k].norm()), k
