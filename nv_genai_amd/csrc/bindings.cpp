@@ -1601,6 +1601,14 @@ std::vector<Tensor> ivf_search(Tensor q, Tensor X, Tensor bias, Tensor ids, Tens
   TORCH_CHECK(list_beg.numel() == nlist && list_end.numel() == nlist, "ivf_search: one row range per list");
   TORCH_CHECK(nprobe >= 1 && nprobe <= nlist, "ivf_search: nprobe must be in [1, lists]");
   TORCH_CHECK(k <= 32 && cus >= 1 && cus <= 4096, "ivf_search: k must be at most 32");
+  if (nga::ivf_one_covers(nq, nlist, D, (int)k)) {
+    const int blocks = nga::scan_blocks(D, 1, (int)cus);
+    Search s = search_begin(q, X, bias, dot_scale, metric, k, blocks * k);
+    s.a.qf = q.data_ptr<float>();
+    nga::launch_ivf_one(s.a, {centroids.data_ptr<float>(), list_beg.data_ptr<int64_t>(), list_end.data_ptr<int64_t>(), (int)nlist,
+                              (int)nprobe}, blocks, s.st);
+    return search_end(s, q, ids, (int32_t)(blocks * k), "ivf_search");
+  }
   int ng = nq <= 16 ? 1 : nq <= 32 ? 2 : nq <= 48 ? 3 : 4;
   if (ng > 2 && k > 8) ng = 2;   // longer register lists leave room for 32 queries
   const int sl = 16 * ng, K = nga::scan_list((int)k, ng, true), blocks = nga::scan_blocks(D, ng, (int)cus);
@@ -2958,6 +2966,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("scan_wide_covers", &nga::scan_wide_covers);
   m.def("flat_search", &flat_search);
   m.def("ivf_search", &ivf_search);
+  m.def("ivf_one_covers", &nga::ivf_one_covers);
   m.def("search_covers", [](int64_t d) { return d <= 1024 && nga::scan_chunk((int)d, 1) > 0; });
   m.def("score_topk", checked("score_topk", &score_topk));
   m.def("ivf_plan", checked("ivf_plan", &ivf_plan));

@@ -230,6 +230,15 @@ void launch_scan(const ScanArgs& a, int ng, int K, int blocks, hipStream_t strea
 bool scan_wide_covers(int D, int ng);           // flat scans of more than 16 queries
 void launch_scan_wide(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream);
 void launch_search_prep(const float* q, int64_t q_stride, int nq, int D, int metric, uint16_t* qb, hipStream_t stream);
+// the whole search of one query but the merge: candidates of workgroup b in the k places from b k on; qf is the query
+constexpr int IVF_ONE_MAX_LISTS = 256;
+struct IvfLists {
+  const float* cent;            // [nlist, D]
+  const int64_t *beg, *end;     // [nlist]
+  int nlist, nprobe;
+};
+bool ivf_one_covers(int64_t nq, int64_t nlist, int D, int k);
+void launch_ivf_one(const ScanArgs& a, const IvfLists& l, int blocks, hipStream_t stream);
 struct IvfOne {   // for a single query: what launch_ivf_items makes, in the same launch; items null: not
   int sl, blocks;
   const int64_t *lbeg, *lend;

@@ -4,7 +4,8 @@
 // The work of a scan is one sequence of 128-row tiles over all (list, query group) items, cut into equal runs, one
 // run per workgroup. A run that crosses from one item into the next ends its top-k there and starts again, so lists
 // of any sizes load the chip evenly: with a fixed count of workgroups per list the longest list decided (1M x 1024
-// in 64 lists of unequal size, 16 probed, one query: scan 143 us, now 102; the whole search 189 us, now 113).
+// in 64 lists of unequal size, 16 probed, one query: scan 143 us, so 102; the whole search 189 us, so 113; in one launch with its
+// probing, further below, 103).
 #include "common.h"
 #include "kernels.h"
 
@@ -743,6 +744,268 @@ __global__ void __launch_bounds__(256, 1) scan_wide_kernel(ScanArgs p) {
   }
 }
 
+// ---------------------------------------------------------------- lists, one query
+// Probing, plan and scan of a single query in one launch. Every workgroup does the probing itself: of few centroids that is shorter (some 4 us
+// for 64) than a launch of one workgroup, the way from it to the next one and that one's tables (13). And one query's lists need no
+// restarts: the rows of all probed lists are one sequence of 32-row tiles, cut into equal runs, one a wave, which keeps its register list
+// and its DMA under way from one list to the next. Bound by the stream of vectors. Whole search, us, before (probing with the plan in a launch
+// of its own, runs that end with their list) and here: 1M x 1,024, 16 of 64 lists 88 75, 4 of 64 32.8 27.0; 500k x 768, 8 of 64 58 48; 200k x
+// 768, 8 of 64, k 10 39.7 33.1; 1M x 384, 16 of 64, k 25 122 108; 100k x 384, 8 of 16 32 25.
+template <int K, int CH>
+__global__ void __launch_bounds__(256, 1) ivf_one_kernel(ScanArgs p, IvfLists l) {
+  constexpr int SLOT = 32 * CH, NC = CH / 8, NI = NC / 2, NS = CH / 32, NB = 4;
+  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+  uint16_t* const q_s = smem + SS_W * SLOT;                       // the query, and a row of zeros
+  int64_t* const beg_s = reinterpret_cast<int64_t*>(q_s + 2 * p.D);         // of the probed lists
+  int64_t* const end_s = beg_s + IVF_ONE_MAX_LISTS;
+  int* const start_s = reinterpret_cast<int*>(end_s + IVF_ONE_MAX_LISTS);   // the first tile of each, and the count of tiles
+  uint32_t* const sk = reinterpret_cast<uint32_t*>(start_s + IVF_ONE_MAX_LISTS + 1);
+  int* const sum_s = reinterpret_cast<int*>(sk + IVF_ONE_MAX_LISTS);        // [2][SS_W]
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, h = lane >> 4;
+  const int D = p.D, nchx = D / CH;
+  uint16_t* const slot = smem + w * SLOT;
+
+  // probing, as in ivf_probe_kernel
+  int64_t lb = 0, le = 0;
+  if (tid < l.nlist) {
+    lb = l.beg[tid];
+    le = l.end[tid];
+  }
+  WaveQuery wq;
+  f32x4 va[NB][4], vb[NB][4];
+  auto ask = [&](f32x4 (&v)[NB][4], int c0) {   // a centroid beyond the last: the last one's again, not used
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (256 * j < D) {
+        const int i = 4 * lane + 256 * j;
+#pragma unroll
+        for (int u = 0; u < NB; ++u) v[u][j] = *reinterpret_cast<const f32x4*>(l.cent + (uint32_t)(min(c0 + u, l.nlist - 1) * D) + (uint32_t)(i < D ? i : 0));
+      }
+  };
+  auto products = [&](f32x4 (&v)[NB][4], int c0) {
+    float s[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) s[u] = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (256 * j < D) {
+        const bool in = 4 * lane + 256 * j < D;
+#pragma unroll
+        for (int u = 0; u < NB; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[u] += wq.v[j][e] * bf2f(f2bf(in ? v[u][j][e] : 0.f));
+      }
+    // wave_sum of all at once: one after another they would take 5 us
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int u = 0; u < NB; ++u) s[u] += __shfl_xor(s[u], o, 64);
+    float own = s[0];
+#pragma unroll
+    for (int u = 1; u < NB; ++u) own = lane == u ? s[u] : own;
+    if (lane < NB && c0 + lane < l.nlist) sk[c0 + lane] = ss_key(own);
+  };
+  constexpr int RB = NB * SS_W;   // centroids of a round
+  ask(va, NB * w);
+  ask(vb, NB * w + RB);
+  wq.load(p.qf, D, p.metric, lane);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const u16x4 b = wq.bf(j);
+    const int i = 4 * lane + 256 * j;
+    if (w == 0 && i < D) {
+      *reinterpret_cast<u16x4*>(&q_s[i]) = b;
+      *reinterpret_cast<u16x4*>(&q_s[D + i]) = (u16x4)(0);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wq.v[j][e] = bf2f(b[e]);
+  }
+  for (int c0 = NB * w; c0 - NB * w < l.nlist; c0 += 2 * RB) {
+    products(va, c0);
+    if (c0 + 2 * RB < l.nlist) ask(va, c0 + 2 * RB);
+    products(vb, c0 + RB);
+    if (c0 + 3 * RB < l.nlist) ask(vb, c0 + 3 * RB);
+  }
+  __syncthreads();
+  bool first = false;
+  if (tid < l.nlist) {
+    const uint32_t mine = sk[tid];
+    int rank = 0;
+#pragma unroll 16
+    for (int o = 0; o < l.nlist; ++o) {
+      const uint32_t x = sk[o];
+      rank += x > mine || (x == mine && o < tid);
+    }
+    first = rank < l.nprobe && le > lb;
+  }
+  // the probed lists that hold rows, in the order of their rows: that of the lists, or else found by counting
+  const int mine = first ? (int)((le - lb + 31) / 32) : 0;
+  const uint64_t who = __ballot(first);
+  int tiles = mine;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int a = __shfl_up(tiles, o, 64);
+    tiles += lane >= o ? a : 0;
+  }
+  if (lane == 63) {
+    sum_s[w] = tiles;
+    sum_s[SS_W + w] = __popcll(who);
+  }
+  __syncthreads();
+  int before = 0, place = __popcll(who & ((uint64_t(1) << lane) - 1)), total = 0, lists = 0;
+#pragma unroll
+  for (int u = 0; u < SS_W; ++u) {
+    before += u < w ? sum_s[u] : 0;
+    place += u < w ? sum_s[SS_W + u] : 0;
+    total += sum_s[u];
+    lists += sum_s[SS_W + u];
+  }
+  if (__syncthreads_or(tid + 1 < l.nlist && lb > l.beg[tid + 1])) {
+    if (tid < l.nlist) {
+      beg_s[tid] = lb;
+      start_s[tid] = mine;
+    }
+    __syncthreads();
+    place = before = 0;
+    for (int o = 0; o < l.nlist; ++o) {
+      const int to = start_s[o];   // 0: not of them
+      const int64_t bo = beg_s[o];
+      if (to > 0 && (bo < lb || (bo == lb && o < tid))) {
+        ++place;
+        before += to;
+      }
+    }
+    tiles = mine;
+    __syncthreads();
+  }
+  if (first) {
+    beg_s[place] = lb;
+    end_s[place] = le;
+    start_s[place] = before + tiles - mine;
+  }
+  if (tid == 0) start_s[lists] = total;
+  __syncthreads();
+
+  const int64_t runs = (int64_t)gridDim.x * SS_W, run = (int64_t)blockIdx.x * SS_W + w;
+  int t = __builtin_amdgcn_readfirstlane((int)(total * run / runs));
+  const int t1 = __builtin_amdgcn_readfirstlane((int)(total * (run + 1) / runs));
+  float tv[K];
+  int tr[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    tv[j] = -INFINITY;
+    tr[j] = -1;
+  }
+  if (t < t1) {
+    // the list of the tile that is asked for, and that tile's rows
+    int at = 0, next = 0;
+    int64_t nrow = 0, nend = 0, row = 0, end = 0;
+    for (int o = 0; o < lists; o += 64) at += __popcll(__ballot(o + lane < lists && start_s[o + lane] <= t));
+    at -= 1;
+    auto open = [&](int tile) {
+      while (tile >= start_s[at + 1]) ++at;   // start_s[lists] = total lies behind every tile
+      at = __builtin_amdgcn_readfirstlane(at);
+      next = tile;
+      nrow = beg_s[at] + (int64_t)(tile - start_s[at]) * 32;
+      nend = end_s[at];
+    };
+    float bnext[2][4], bcur[2][4];
+    auto issue = [&](int c) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const unsigned li = i * 64 + lane, r = li / NC, pos = li % NC;
+        int64_t gr = nrow + r;
+        if (gr >= nend) gr = nend - 1;
+        __builtin_amdgcn_global_load_lds((gptr_t)(p.X + gr * D + c * CH + ((pos ^ (r & 15)) << 3)), (lptr_t)(slot + i * 512), 16, 0, 2);
+      }
+      if (c == 0) {   // the tile's biases arrive with its first unit
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr) {
+            const int64_t r = nrow + 16 * i + 4 * h + rr;
+            bnext[i][rr] = r < nend ? p.bias[r] : 0.f;
+          }
+      }
+    };
+    f32x4 acc[2] = {(f32x4)(0.f), (f32x4)(0.f)};   // column 0 is the query's
+    open(t);
+    issue(0);
+    int c = 0;
+    while (t < t1) {
+      const int c2 = c + 1 == nchx ? 0 : c + 1, t2 = c2 == 0 ? t + 1 : t;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (c == 0) {
+        row = nrow;
+        end = nend;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr) bcur[i][rr] = bnext[i][rr];
+      }
+      u16x8 a[2][NS];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+          a[i][s] = *reinterpret_cast<const u16x8*>(slot + (16 * i + col) * CH + (((4 * s + h) ^ col) << 3));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slot is free
+      if (t2 < t1) {
+        if (t2 != next) open(t2);
+        issue(c2);
+      }
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const bf16x8 bq = as_bf16x8(*reinterpret_cast<const u16x8*>(&q_s[(col ? D : 0) + (c * NC + 4 * s + h) * 8]));
+        acc[0] = mfma16(as_bf16x8(a[0][s]), bq, acc[0]);
+        acc[1] = mfma16(as_bf16x8(a[1][s]), bq, acc[1]);
+      }
+      if (c == nchx - 1) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr) {
+            const int64_t r = row + 16 * i + 4 * h + rr;
+            const float sc = acc[i][rr] * p.dot_scale + bcur[i][rr];
+            if (r < end && sc > tv[K - 1]) ss_insert<K>(tv, tr, sc, (int)r);
+          }
+          acc[i] = (f32x4)(0.f);
+        }
+      }
+      t = t2;
+      c = c2;
+    }
+  }
+  ss_merge_xor<K>(tv, tr, 16);
+  ss_merge_xor<K>(tv, tr, 32);
+  __syncthreads();   // every wave is past its last DMA wait
+  float* const mv = reinterpret_cast<float*>(smem);   // [SS_W][K]
+  int* const mr = reinterpret_cast<int*>(mv + SS_W * K);
+  if (lane == 0) {   // the query's column
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      mv[w * K + j] = tv[j];
+      mr[w * K + j] = tr[j];
+    }
+  }
+  __syncthreads();
+  // each of the 4 K finds its place among all
+  if (tid < SS_W * K) {
+    const float x = mv[tid];
+    const int r = mr[tid];
+    int rank = 0;
+    for (int o = 0; o < SS_W * K; ++o) {
+      const int orow = mr[o];
+      rank += orow >= 0 ? (r < 0 || ss_first(mv[o], orow, x, r)) : (r < 0 && o < tid);
+    }
+    if (rank < p.k) {
+      p.cand_v[(int64_t)blockIdx.x * p.k + rank] = r >= 0 ? x : -INFINITY;
+      p.cand_r[(int64_t)blockIdx.x * p.k + rank] = r;
+    }
+  }
+}
+
 // ---------------------------------------------------------------- selection
 // The k <= 256 largest of n values, sorted, by one workgroup. The k-th largest of the 256 threads' maxima (of 64 groups'
 // maxima where k is at most 32) is a lower bound of the k-th largest value, so a first pass takes maxima, their ranks (by
@@ -983,6 +1246,43 @@ void launch_scan(const ScanArgs& a, int ng, int K, int blocks, hipStream_t strea
   NGA_SCAN(3, 0); NGA_SCAN(3, 4); NGA_SCAN(3, 8);
   NGA_SCAN(4, 0); NGA_SCAN(4, 4); NGA_SCAN(4, 8);
 #undef NGA_SCAN
+}
+
+// The dimensions whose slots fill a CU with one workgroup; with several (128, 256, 640, 896) all of them would probe: 100k x 640, 64 lists 30
+// us, here 54. And as many centroids as take no longer here than in a launch of their own; both, us, at 128 and 160 lists: 500k x 1,024
+// 50.4 43.9, 41.3 42.7; 100k x 1,024 35.6 32.9, 37.3 38.0; 100k x 768 33.9 29.2, 35.3 33.0; 100k x 384 30.9 25.1, 32.2 28.2 (256 lists, 200k:
+// 39.0 35.9; x 1,024 44.2 46.4).
+bool ivf_one_covers(int64_t nq, int64_t nlist, int D, int k) {
+  return nq == 1 && nlist <= IVF_ONE_MAX_LISTS && nlist * D <= 128 * 1024 && k >= 1 && k <= 32 && scan_chunk(D, 1) >= 384;
+}
+
+template <int K, int CH>
+static void one_go(const ScanArgs& a, const IvfLists& l, int blocks, hipStream_t stream) {
+  constexpr size_t lds = (size_t)SS_W * 32 * CH * 2 + 2 * 1024 * 2 + IVF_ONE_MAX_LISTS * 24 + 4 + 2 * SS_W * 4;
+  static_assert(lds <= SS_LDS, "LDS");
+  static const bool attr = [] {
+    (void)hipFuncSetAttribute((const void*)ivf_one_kernel<K, CH>, hipFuncAttributeMaxDynamicSharedMemorySize, SS_LDS);
+    (void)hipGetLastError();
+    return true;
+  }();
+  (void)attr;
+  ivf_one_kernel<K, CH><<<blocks, 256, lds, stream>>>(a, l);
+}
+
+template <int K>
+static void one_ch(const ScanArgs& a, const IvfLists& l, int blocks, hipStream_t stream) {
+  if (scan_chunk(a.D, 1) == 512) one_go<K, 512>(a, l, blocks, stream);
+  else one_go<K, 384>(a, l, blocks, stream);
+}
+
+void launch_ivf_one(const ScanArgs& a, const IvfLists& l, int blocks, hipStream_t stream) {
+  switch (scan_list(a.k, 1, true)) {
+    case 4: return one_ch<4>(a, l, blocks, stream);
+    case 8: return one_ch<8>(a, l, blocks, stream);
+    case 16: return one_ch<16>(a, l, blocks, stream);
+    case 32: return one_ch<32>(a, l, blocks, stream);
+    default: return;
+  }
 }
 
 // 17 to 64 queries of all rows, prepared

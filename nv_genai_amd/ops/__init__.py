@@ -1891,7 +1891,7 @@ def ivf_search(q: torch.Tensor, X: torch.Tensor, row_bias: torch.Tensor, ids: to
                list_beg: torch.Tensor, list_end: torch.Tensor, metric: str, nprobe: int,
                k: int) -> Tuple[torch.Tensor, torch.Tensor]:
     """``flat_search`` over the rows of the nprobe lists (X in list order) whose centroids have the largest products with
-    the query: four launches, no host synchronisation."""
+    the query: two to four launches, no host synchronisation."""
     return tuple(kernels().ivf_search(q, X, row_bias, ids, centroids, list_beg, list_end, 2.0 if metric == "l2" else 1.0,
                                       _METRIC[metric], int(nprobe), int(k), _cu_count(X.device)))
 
