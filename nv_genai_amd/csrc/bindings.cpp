@@ -1239,10 +1239,13 @@ void sample(Tensor logits, Tensor temperature, Tensor top_k, Tensor top_p,
     hp = history->data_ptr<int32_t>();
     hl = (int)history->size(1);
   }
+  const int64_t bytes = nga::sample_scratch((int)B, (int)logits.size(1));
+  Tensor scratch;
+  if (bytes > 0) scratch = at::empty({bytes}, logits.options().dtype(at::kByte));
   nga::launch_sample(logits.data_ptr<float>(), (int)B, (int)logits.size(1), temperature.data_ptr<float>(),
                      top_k.data_ptr<int32_t>(), top_p.data_ptr<float>(), rp, hp, hl,
-                     seeds.data_ptr<int64_t>(), steps.data_ptr<int64_t>(), out_tok.data_ptr<int32_t>(),
-                     out_logprob.data_ptr<float>(), cur_stream(logits));
+                     seeds.data_ptr<int64_t>(), steps.data_ptr<int64_t>(), bytes > 0 ? scratch.data_ptr() : nullptr,
+                     out_tok.data_ptr<int32_t>(), out_logprob.data_ptr<float>(), cur_stream(logits));
 }
 
 // ------------------------------------------------------------------ embedding gather

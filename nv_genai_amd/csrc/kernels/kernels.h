@@ -168,10 +168,11 @@ void launch_prefill_attention_v2_worklist(const PrefillParams& p, int grid, int 
 void launch_prefill_attention_v1_worklist(const PrefillParams& p, int grid, int D, bool causal,
                                           hipStream_t stream);
 
-// sampling.hip
+// sampling.hip; scratch: sample_scratch bytes (of 16-byte alignment), or null
+int64_t sample_scratch(int B, int V);
 void launch_sample(float* logits, int B, int V, const float* temperature, const int32_t* top_k,
                    const float* top_p, const float* rep_penalty, const int32_t* history,
-                   int hist_len, const int64_t* seeds, const int64_t* steps, int32_t* out_tok,
+                   int hist_len, const int64_t* seeds, const int64_t* steps, void* scratch, int32_t* out_tok,
                    float* out_logprob, hipStream_t stream);
 
 // vector_search.hip

@@ -15,6 +15,11 @@
 // Every pass over the row keeps eight 16-byte loads in flight per thread. Histogram weights are
 // 64-bit fixed point (2^-40 units of exp(v - M)) so the LDS atomics are ds_add_u64: LDS
 // ds_add_f32 measured ~8x slower on gfx950 (scripts/dev/lds_atomic_bench.hip).
+//   * rows of some thousand values first go through sample_slices_kernel, some 2,000 values a workgroup, which finds the largest value and
+//     the partition function's part of each slice and lists its values close to that maximum. One workgroup a row is bound by its
+//     own arithmetic: a pass over 128,256 values takes it 14 to 20 us. Where the lists reach far enough below the row's maximum (at the
+//     temperature of 0.2 that the servers use by default they do, with some 20 of 2,000 values) all passes of the fast path go over
+//     them, in registers, instead of the row. More in sample_slices.
 // Also returns the chosen token's log-probability under the temperature-scaled distribution.
 #include "common.h"
 #include "kernels.h"
@@ -42,6 +47,19 @@ struct ArgMax {
   float v;
   int i;
 };
+struct SampleEntry {   // a value that a slice lists, before the temperature
+  float v;
+  int i;
+};
+struct SampleSlice {
+  float m, z;   // the largest value, and the sum of exp(v - m)
+  int i, n;     // where it is; how many are listed
+  float range;  // those less than this below m
+};
+
+constexpr int SLICE = 2048;        // values of a slice: 8 a thread
+constexpr int MAX_SLICES = 128;    // of a row (262,144 values)
+constexpr int LISTED = 64;         // values that a slice can list
 
 constexpr double FIX = 1099511627776.0;  // 2^40: fixed-point unit of the mass histograms
 
@@ -146,11 +164,31 @@ __device__ __forceinline__ void for_row(const float* __restrict__ x, int V, F f)
   }
 }
 
+// A row as the fast path sees it: all its values, or those that the slices list, a thread's share of them in its registers
+constexpr int OWN = MAX_SLICES * LISTED / NT;
+struct Row {
+  const float* x;
+  int V;
+  bool listed;
+  SampleEntry own[OWN];   // i < 0: none
+};
+
+template <typename F>
+__device__ __forceinline__ void for_near(const Row& r, F f) {
+  if (!r.listed) {
+    for_row(r.x, r.V, f);
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < OWN; ++j)
+    if (r.own[j].i >= 0) f(r.own[j].i, r.own[j].v);
+}
+
 __device__ __forceinline__ ArgMax am_max(ArgMax a, ArgMax b) {
   return (b.v > a.v || (b.v == a.v && b.i < a.i)) ? b : a;
 }
 
-__device__ ArgMax block_argmax(ArgMax a, ArgMax* red) {
+__device__ __forceinline__ ArgMax wave_argmax(ArgMax a) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     ArgMax b;
@@ -158,6 +196,11 @@ __device__ ArgMax block_argmax(ArgMax a, ArgMax* red) {
     b.i = __shfl_xor(a.i, o, 64);
     a = am_max(a, b);
   }
+  return a;
+}
+
+__device__ ArgMax block_argmax(ArgMax a, ArgMax* red) {
+  a = wave_argmax(a);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = a;
   __syncthreads();
@@ -186,14 +229,14 @@ __device__ __forceinline__ float from_fixed(uint64_t q) {
 // the probability mass (relative to exp(M)) kept by that threshold. Returns false, uniformly
 // over the workgroup, when the caller must take the radix descent instead.
 template <bool MASS>
-__device__ __forceinline__ bool fast_select(const float* __restrict__ x, int V, float inv_t, float M,
+__device__ __forceinline__ bool fast_select(const Row& row, float inv_t, float M,
                             uint32_t floor_key, float target, Smem& sm, uint32_t* thr_out,
                             float* kept_out) {
   const int t = threadIdx.x, lane = t & 63;
   for (int i = t; i < NBINS; i += NT) sm.u.s.h.q[i] = 0ull;
   if (t == 0) sm.ncand = 0;
   __syncthreads();
-  for_row(x, V, [&](int, float raw) {
+  for_near(row, [&](int, float raw) {
     const float v = raw * inv_t;
     const float d = M - v;
     if (d < DRANGE && fkey(v) >= floor_key)
@@ -209,7 +252,7 @@ __device__ __forceinline__ bool fast_select(const float* __restrict__ x, int V, 
 
   // gather the crossing bin's keys (wave-aggregated slots), and the mass of the bins above it
   float m_above = 0.f;
-  for_row(x, V, [&](int, float raw) {
+  for_near(row, [&](int, float raw) {
     const float v = raw * inv_t;
     const float d = M - v;
     const uint32_t key = fkey(v);
@@ -304,11 +347,82 @@ __device__ __forceinline__ uint32_t radix_select(const float* __restrict__ x, in
 }
 }  // namespace
 
+// One slice of a row: its largest value and where, the sum of exp(v - it) over the slice, and unless the row is greedy its values near
+// the largest one: less than DRANGE below it, or a half, a quarter, an eighth of that if they are too many. (What counts is DRANGE below the
+// row's largest value; a slice of a smaller one need not reach as far.)
+__global__ void __launch_bounds__(256) sample_slices_kernel(const float* __restrict__ logits, int V, const float* __restrict__ temperature,
+                                                            const int32_t* __restrict__ top_k, const float* __restrict__ penalty,
+                                                            SampleSlice* __restrict__ slices, SampleEntry* __restrict__ list) {
+  __shared__ ArgMax ared[4];
+  __shared__ float red[4];
+  __shared__ int counts[4], count;
+  const int row = blockIdx.y, t = threadIdx.x;
+  if (penalty && penalty[row] != 1.f) return;   // sample_kernel changes the row first
+  const float* x = logits + (int64_t)row * V;
+  const float temp = temperature[row];
+  const bool greedy = !(temp > 0.f) || (top_k && top_k[row] == 1);
+  const float inv_t = greedy ? 1.f : 1.f / temp;
+  const int b = blockIdx.x * SLICE;
+  float raw[8];
+  const bool vec = (V & 3) == 0;   // rows at 16-byte addresses
+  auto at = [&](int j) { return vec ? b + 1024 * (j >> 2) + 4 * t + (j & 3) : b + 256 * j + t; };
+  if (vec) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const float4 v = at(4 * u) < V ? *reinterpret_cast<const float4*>(x + at(4 * u)) : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+      raw[4 * u] = v.x;
+      raw[4 * u + 1] = v.y;
+      raw[4 * u + 2] = v.z;
+      raw[4 * u + 3] = v.w;
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) raw[j] = at(j) < V ? x[at(j)] : -INFINITY;
+  }
+  ArgMax am{-INFINITY, 0x7fffffff};
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float v = raw[j] * inv_t;
+    if (v > am.v) am = ArgMax{v, at(j)};   // a thread's values in ascending order
+  }
+  am = wave_argmax(am);
+  if ((t & 63) == 0) ared[t >> 6] = am;
+  if (t < 4) counts[t] = 0;
+  if (t == 0) count = 0;
+  __syncthreads();
+  am = am_max(am_max(ared[0], ared[1]), am_max(ared[2], ared[3]));
+  SampleEntry* const own = list + ((int64_t)row * gridDim.x + blockIdx.x) * LISTED;
+  float z = 0.f, range = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float v = raw[j] * inv_t;
+    if (v > -INFINITY) z += v == am.v ? 1.f : __expf(v - am.v);
+  }
+  if (!greedy) {
+    int n[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) n[r] += __popcll(__ballot(am.v - raw[j] * inv_t < DRANGE / (1 << r)));
+    if ((t & 63) < 4) atomicAdd(&counts[t & 63], (t & 63) == 0 ? n[0] : (t & 63) == 1 ? n[1] : (t & 63) == 2 ? n[2] : n[3]);
+    __syncthreads();
+#pragma unroll
+    for (int r = 3; r >= 0; --r)
+      if (counts[r] <= LISTED) range = DRANGE / (1 << r);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (am.v - raw[j] * inv_t < range) own[atomicAdd(&count, 1)] = SampleEntry{raw[j], at(j)};   // at most LISTED
+  }
+  z = block_sum(z, red);   // with barriers: the count is complete
+  if (t == 0) slices[(int64_t)row * gridDim.x + blockIdx.x] = SampleSlice{am.v, z, am.i, count, range};
+}
+
 __global__ void __launch_bounds__(NT) sample_kernel(
     float* __restrict__ logits, int V, const float* __restrict__ temperature,
     const int32_t* __restrict__ top_k, const float* __restrict__ top_p,
     const float* __restrict__ rep_penalty, const int32_t* __restrict__ history, int hist_len,
     const int64_t* __restrict__ seeds, const int64_t* __restrict__ steps,
+    const SampleSlice* __restrict__ slices, const SampleEntry* __restrict__ list, int nslices,
     int32_t* __restrict__ out_tok, float* __restrict__ out_logprob) {
   __shared__ Smem sm;
 
@@ -316,7 +430,8 @@ __global__ void __launch_bounds__(NT) sample_kernel(
   float* x = logits + (int64_t)row * V;
   const float pen = rep_penalty ? rep_penalty[row] : 1.f;
 
-  if (pen != 1.f && history != nullptr) {
+  const bool changed = pen != 1.f && history != nullptr;
+  if (changed) {
     for (int i = t; i < 8192; i += NT) sm.u.bitmap[i] = 0;
     __syncthreads();
     const int32_t* hs = history + (int64_t)row * hist_len;
@@ -339,23 +454,47 @@ __global__ void __launch_bounds__(NT) sample_kernel(
   const bool greedy = !(temp > 0.f) || k == 1;
   const float inv_t = greedy ? 1.f : 1.f / temp;
 
-  // one pass: argmax and the partition function (online: per-thread running max + rescaled sum)
+  // argmax and the partition function: the slices', or in one pass (online: per-thread running max + rescaled sum)
   ArgMax am{-INFINITY, 0x7fffffff};
   float z = 0.f;
-  for_row(x, V, [&](int i, float raw) {
-    const float v = raw * inv_t;
-    if (v > am.v) {
-      z = z * __expf(am.v - v) + 1.f;
-      am = ArgMax{v, i};
-    } else if (v > -INFINITY) {
-      z += __expf(v - am.v);
-      if (v == am.v && i < am.i) am.i = i;
+  Row near;
+  near.x = x;
+  near.V = V;
+  near.listed = false;
+  float reach = -INFINITY;   // of this thread's slice all values above it are listed
+  if (nslices > 0 && !changed) {
+    const SampleSlice* const own = slices + (int64_t)row * nslices;
+#pragma unroll
+    for (int j = 0; j < OWN; ++j) {
+      const int e = t + j * NT;
+      near.own[j].i = -1;
+      if (e < nslices * LISTED && !greedy) {
+        const SampleEntry v = list[(int64_t)row * nslices * LISTED + e];
+        near.own[j] = SampleEntry{v.v, e % LISTED < own[e / LISTED].n ? v.i : -1};
+      }
     }
-  });
+    if (t < nslices) {
+      am = ArgMax{own[t].m, own[t].i};
+      z = own[t].z;
+      reach = am.v - own[t].range;
+    }
+  } else {
+    for_row(x, V, [&](int i, float raw) {
+      const float v = raw * inv_t;
+      if (v > am.v) {
+        z = z * __expf(am.v - v) + 1.f;
+        am = ArgMax{v, i};
+      } else if (v > -INFINITY) {
+        z += __expf(v - am.v);
+        if (v == am.v && i < am.i) am.i = i;
+      }
+    });
+  }
   const float m_thr = am.v;
   am = block_argmax(am, sm.ared);
   const float M = am.v;
-  const float Z = block_sum(m_thr == -INFINITY ? 0.f : z * __expf(m_thr - M), sm.red);
+  near.listed = __syncthreads_and(nslices > 0 && !changed && reach <= M - DRANGE);
+  const float Z = block_sum(m_thr == -INFINITY ? 0.f : m_thr == M ? z : z * __expf(m_thr - M), sm.red);
   const float logZ = __logf(Z);
 
   if (greedy) {
@@ -369,7 +508,7 @@ __global__ void __launch_bounds__(NT) sample_kernel(
   uint32_t thr = 0u;  // keep tokens with fkey(x * inv_t) >= thr
   float kept_mass = Z;
   if (k > 0 && k < V) {
-    if (!fast_select<false>(x, V, inv_t, M, 0u, (float)k, sm, &thr, &kept_mass)) {
+    if (!fast_select<false>(near, inv_t, M, 0u, (float)k, sm, &thr, &kept_mass)) {
       thr = radix_select<false>(x, V, inv_t, M, 0u, (float)k, sm);
       float km = 0.f;
       for_row(x, V, [&](int, float raw) {
@@ -382,7 +521,7 @@ __global__ void __launch_bounds__(NT) sample_kernel(
   if (p < 1.f) {
     uint32_t tp;
     float unused;
-    if (!fast_select<true>(x, V, inv_t, M, thr, p * kept_mass, sm, &tp, &unused))
+    if (!fast_select<true>(near, inv_t, M, thr, p * kept_mass, sm, &tp, &unused))
       tp = radix_select<true>(x, V, inv_t, M, thr, p * kept_mass, sm);
     thr = tp > thr ? tp : thr;
   }
@@ -391,7 +530,8 @@ __global__ void __launch_bounds__(NT) sample_kernel(
   const uint64_t seed = (uint64_t)seeds[row];
   const uint64_t base = (uint64_t)steps[row] * (uint64_t)V;
   ArgMax best{-INFINITY, 0x7fffffff};
-  for_row(x, V, [&](int i, float raw) {
+  if (!(M - fval(thr) < DRANGE)) near.listed = false;   // keeps values that the lists leave out (thr 0 is NaN's key: all)
+  for_near(near, [&](int i, float raw) {
     const float v = raw * inv_t;
     if (fkey(v) >= thr) {
       const float u = hash_uniform(seed, base + i);
@@ -407,13 +547,29 @@ __global__ void __launch_bounds__(NT) sample_kernel(
   }
 }
 
+// Slices of a row, 0: none. Their launch costs 3 us and up: short rows are through as soon, and many rows fill the chip by themselves. Both,
+// us, without / with: at the temperature 0.2 and top-p 0.7 that the servers use by default, and greedy, 1 row of 8,000 values (4 slices)
+// 15.3 16.9, 5.4 8.0; 1 of 32,000 24.8 17.3, 8.7 8.0; 1 of 128,256 53 19, 20.4 8.2; 64 of 128,256 60 29, 22.4 14.9; 256 of 128,256 87 58,
+// 27.3 34.6. Lists that are of no use (normal logits of deviation 3 at temperature 1, top-p 0.9): 1 of 32,000 38.4 39.6, 1 of 128,256 113
+// 103, 64 of 128,256 120 120, 256 128 153.
+int sample_slices(int B, int V) {
+  const int n = (V + SLICE - 1) / SLICE;
+  return n < 12 || n > MAX_SLICES || (int64_t)B * n > 4096 ? 0 : n;
+}
+int64_t sample_scratch(int B, int V) { return (int64_t)B * sample_slices(B, V) * (sizeof(SampleSlice) + LISTED * sizeof(SampleEntry)); }
+
 void launch_sample(float* logits, int B, int V, const float* temperature, const int32_t* top_k,
                    const float* top_p, const float* rep_penalty, const int32_t* history,
-                   int hist_len, const int64_t* seeds, const int64_t* steps, int32_t* out_tok,
+                   int hist_len, const int64_t* seeds, const int64_t* steps, void* scratch, int32_t* out_tok,
                    float* out_logprob, hipStream_t stream) {
   if (B == 0) return;
+  const int n = scratch ? sample_slices(B, V) : 0;
+  SampleEntry* const list = static_cast<SampleEntry*>(scratch);
+  SampleSlice* const slices = reinterpret_cast<SampleSlice*>(list + (int64_t)B * n * LISTED);
+  if (n > 0)
+    sample_slices_kernel<<<dim3(n, B), 256, 0, stream>>>(logits, V, temperature, top_k, history ? rep_penalty : nullptr, slices, list);
   sample_kernel<<<B, NT, 0, stream>>>(logits, V, temperature, top_k, top_p, rep_penalty, history,
-                                      hist_len, seeds, steps, out_tok, out_logprob);
+                                      hist_len, seeds, steps, slices, list, n, out_tok, out_logprob);
 }
 
 }  // namespace nga

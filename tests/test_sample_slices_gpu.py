@@ -1,0 +1,68 @@
+"""Sampling by slices of a row beside the passes over whole rows, which a batch too large for slices takes: the tokens are the same, the
+log-probabilities up to the order of their sums."""
+import pytest
+import torch
+
+from nv_genai_amd import ops
+
+pytestmark = pytest.mark.gpu
+# temperature, top_k, top_p
+HOW = [(0.0, 0, 1.0), (0.2, 0, 0.7), (0.2, 40, 0.95), (1.0, 0, 0.9), (1.0, 1, 1.0), (1.0, 0, 1.0), (0.7, 50, 1.0), (0.05, 3, 0.5), (0.2, 0, 0.9999999)]
+
+
+def _rows(V, g):
+    """Logits as a trained model has them, flat ones, a slice that lists too many, equal largest values, and rows with and of -inf."""
+    x = 2.5 * torch.randn(9, V, device="cuda", generator=g)
+    x[0, V // 3] += 12
+    x[1] *= 0.01
+    x[2, :2048] = x[2].max() - 0.1 * torch.rand(min(2048, V), device="cuda", generator=g)[: x[2, :2048].numel()]
+    x[3, [5, 2047, 2048, V - 1]] = x[3].max() + 1
+    x[4, V // 2:] = float("-inf")
+    x[5] = float("-inf")
+    x[6] = float("-inf")
+    x[6, V - 1] = 3.0
+    x[7, 100:] = x[7, :1].clone()
+    x[8, 7] = float("nan")
+    return x
+
+
+@pytest.mark.parametrize("V", [22_529, 24_576, 24_580, 50_257, 128_256, 262_144])
+@pytest.mark.parametrize("temp,k,p", HOW)
+def test_same_tokens(gpu, V, temp, k, p):
+    n = -(-V // 2048)
+    g = torch.Generator(device="cuda").manual_seed(V)
+    x = _rows(V, g)
+    B = 4096 // n + 1   # one row too many
+    assert B > len(x)
+    full = torch.cat([x, x[:1].expand(B - len(x), V)]) if B * V < 1 << 27 else None
+    if full is None:
+        pytest.skip("a batch of several GiB")
+
+    def run(lg, seed):
+        b = lg.shape[0]
+        arg = (torch.full((b,), temp, device=gpu), torch.full((b,), k, dtype=torch.int32, device=gpu), torch.full((b,), p, device=gpu))
+        return ops.sample(lg, *arg, seed + torch.arange(b, device=gpu), torch.arange(b, device=gpu))
+
+    for seed in (0, 1000):
+        (ta, la), (tb, lb) = run(x.clone(), seed), run(full.clone(), seed)
+        tb, lb = tb[: len(x)], lb[: len(x)]
+        assert torch.equal(ta, tb)
+        # sums of up to 262,144 terms in fp32, in two orders: about sqrt(V) 2^-24 of them
+        assert torch.allclose(la, lb, rtol=1e-5, atol=1e-5, equal_nan=True)
+
+
+def test_a_penalty_changes_the_row_first(gpu):
+    V = 32_000
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = 2.5 * torch.randn(3, V, device="cuda", generator=g)
+    hist = x.topk(3, 1).indices.int()
+    pen = torch.tensor([1.0, 5.0, 1.3], device=gpu)
+    arg = (torch.zeros(3, device=gpu), torch.zeros(3, dtype=torch.int32, device=gpu), torch.ones(3, device=gpu), torch.arange(3, device=gpu),
+           torch.arange(3, device=gpu))
+    want = x.clone()
+    for r in range(3):
+        v = want[r, hist[r].long()]
+        want[r, hist[r].long()] = torch.where(v > 0, v / pen[r], v * pen[r])
+    tok, lp = ops.sample(x.clone(), *arg, pen, hist)
+    assert torch.equal(tok.long(), want.argmax(1))
+    assert torch.allclose(lp, torch.log_softmax(want.double(), 1).max(1).values.float(), atol=1e-5)
