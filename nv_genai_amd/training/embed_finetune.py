@@ -85,8 +85,7 @@ def embed_trainer(engine, records: Sequence[dict], cfg: TrainConfig, hard_negati
         with torch.autocast(dev.type, dtype=torch.bfloat16):
             # checkpointed layers cast their own weights, and let them go: a copy of all would be held through the step (BERT-large 0.6 GB)
             for_q, for_p = (params, params) if cfg.grad_ckpt else Fn.half_params(params)
-            q = Fn.encoder_embed(model, qi, qm, for_q, cfg.grad_ckpt)
-            p = Fn.encoder_embed(model, pi, pm, for_p, cfg.grad_ckpt)
+            p, q = Fn.encoder_embed_pair(model, (pi, pm, for_p), (qi, qm, for_q), cfg.grad_ckpt)
         return contrastive_loss(q, p, 1 + hard_negatives, scale)
 
     return Trainer(named, loss_fn, batches, cfg, group, ckpt_dir), params
