@@ -1098,6 +1098,46 @@ void add_scaled(Tensor y, Tensor d, double scale) {
   post_launch("add_scaled");
 }
 
+// a low-rank adapter's gradients beside w's: (da, db) in fp32, each or an undefined tensor; dx, if given, is added to
+std::tuple<Tensor, Tensor> lora_grads(Tensor dy, Tensor x, Tensor h, Tensor a, Tensor b, c10::optional<Tensor> dx, double scale,
+                                      bool want_a, bool want_b) {
+  TORCH_CHECK(dy.dim() == 2 && x.dim() == 2 && a.dim() == 2 && b.dim() == 2, "lora_grads: matrices");
+  const int64_t T = x.size(0), K = x.size(1), N = dy.size(1), r = a.size(0);
+  TORCH_CHECK(r >= 8 && r <= 64 && r % 8 == 0 && N % 8 == 0 && K % 8 == 0 && N >= 8 && K >= 8 && N < (1 << 24) && K < (1 << 24) &&
+                  T < (1 << 24) && dy.size(0) == T && h.dim() == 2 && h.size(0) == T && h.size(1) == r && a.size(1) == K && b.size(0) == N &&
+                  b.size(1) == r, "lora_grads: dy [T, N], x [T, K], h [T, r], a [r, K], b [N, r], multiples of 8, r <= 64");
+  const int64_t W = r <= 16 ? 16 : r <= 32 ? 32 : 64;
+  train_rows(dy, T, N); train_rows(x, T, K); train_rows(h, T, r); train_rows(a, r, K); train_rows(b, N, r);
+  if (dx) train_rows(*dx, T, K);
+  const auto f32 = x.options().dtype(at::kFloat);
+  const bool back = (want_a || dx) && T > 0;
+  Tensor da, db, part, dh, sums;
+  if (want_a) da = T ? at::empty({r, K}, f32) : at::zeros({r, K}, f32);
+  if (want_b) db = T ? at::empty({N, r}, f32) : at::zeros({N, r}, f32);
+  if (T == 0) return {da, db};
+  nga::LoraGrads p{};
+  p.T = T; p.N = N; p.K = K; p.r = (int)r; p.scale = (float)scale;
+  nga::lora_plan(p);
+  p.dy = bfp(dy); p.x = bfp(x); p.h = bfp(h); p.a = bfp(a); p.b = bfp(b);
+  if (back) {
+    part = at::empty({p.parts, T, W}, f32);
+    dh = at::empty({T, std::max<int64_t>(W, 32)}, x.options());
+    p.part = part.data_ptr<float>();
+    p.dh = bfp(dh);
+  }
+  const int64_t room = std::max(want_b && p.slices_n > 1 ? p.slices_n * N * r : 0, want_a && p.slices_k > 1 ? p.slices_k * K * r : 0);
+  if (room) {
+    sums = at::empty({room}, f32);
+    p.sums = sums.data_ptr<float>();
+  }
+  if (want_a) p.da = da.data_ptr<float>();
+  if (want_b) p.db = db.data_ptr<float>();
+  if (dx) p.dx = bfp(*dx);
+  nga::launch_lora_grads(p, cur_stream(x));
+  post_launch("lora_grads");
+  return {da, db};
+}
+
 // rows [T, nh D], first nr heads rotated by cs [P, D] (row t % P); inplace or a new tensor
 Tensor rope_rows(Tensor x, Tensor cs, int64_t nr, int64_t nh, int64_t D, bool back, bool inplace) {
   TORCH_CHECK(D % 16 == 0 && D >= 16 && nr >= 0 && nr <= nh && nh >= 1, "rope_rows: head size a multiple of 16");
@@ -2960,6 +3000,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("half_grads", on_device(&half_grads));
   m.def("swiglu_rows", on_device(&swiglu_rows));
   m.def("add_scaled", on_device(&add_scaled));
+  m.def("lora_grads", on_device(&lora_grads));
   m.def("rope_rows", on_device(&rope_rows));
   m.def("ce_fwd", on_device(&ce_fwd));
   m.def("ce_bwd", on_device(&ce_bwd));

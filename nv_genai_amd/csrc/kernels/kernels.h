@@ -336,6 +336,23 @@ void launch_rope_rows(const uint16_t* in, const float* cs, int64_t T, int64_t P,
 void launch_ce_fwd(const uint16_t* lg, const int64_t* y, int64_t R, int64_t V, float* lse, float* loss, hipStream_t st);
 void launch_ce_bwd(const void* x, const int64_t* y, const float* lse, const float* scale, int64_t R, int64_t V, uint16_t* d,
                    hipStream_t st);
+// lora.hip: gradients of a low-rank adapter (r <= 64, r, N and K multiples of 8), all contiguous at 16-byte addresses; db, da and dx
+// may be null, and part and dh where neither da nor dx is asked for
+struct LoraGrads {
+  const uint16_t *dy, *x, *h, *a, *b;   // [T, N], [T, K], [T, r], [r, K], [N, r]
+  float *part;                          // [parts, T, 16, 32 or 64]: dh over each chunk of N's columns
+  uint16_t *dh;                         // [T, 32 or 64]
+  float *da, *db;                       // [r, K], [N, r]
+  uint16_t *dx;                         // [T, K], added to
+  float* sums;                          // [slices_n, N, r], then [slices_k, r, K], where those are more than one
+  int64_t T, N, K;
+  int r;
+  float scale;
+  int64_t chunk, slice_n, slice_k;      // lora_plan's
+  int parts, slices_n, slices_k;
+};
+void lora_plan(LoraGrads& p);
+void launch_lora_grads(const LoraGrads& p, hipStream_t st);
 // adamw.hip
 constexpr int OPT_TENSORS = 48;
 constexpr int OPT_CHUNK = 32768;

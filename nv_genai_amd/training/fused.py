@@ -393,10 +393,19 @@ class _LoraLinear(Function):
             dx, da, db = _again(lambda x, a, b: x @ w.t() + ((x @ a.t()) @ b.t()) * scale, (x, ab, bb), dy)
             return dx, None, None, None, da, db, None
         dy2 = dy.reshape(-1, dy.shape[-1])
+        need = ctx.needs_input_grad
+        if (bb.shape[1] <= 64 and all(n % 8 == 0 for n in (*bb.shape, x.shape[-1]))   # lora.hip; single operations under vmap too
+                and _takes(dy) and not torch._C._functorch.is_legacy_batchedtensor(dy)):
+            dy2 = _rows(dy2)
+            dx = _input_grad(dy2, w) if need[0] else None
+            da, db = ops.kernels().lora_grads(dy2, _rows(x.reshape(-1, x.shape[-1])), _rows(h), _rows(ab), _rows(bb), dx, scale,
+                                              need[2], need[3])
+            return (dx.view(x.shape) if need[0] else None, None, da.to(ad) if need[2] else None, db.to(bd) if need[3] else None,
+                    None, None, None)
         dh = (dy2 @ bb).mul_(scale)
-        dx = torch.addmm(_input_grad(dy2, w), dh, ab).view(x.shape) if ctx.needs_input_grad[0] else None
-        da = (dh.t() @ x.reshape(-1, x.shape[-1])).to(ad) if ctx.needs_input_grad[2] else None
-        db = (dy2.t() @ h).to(bd).mul_(scale) if ctx.needs_input_grad[3] else None   # scaled in its own type
+        dx = torch.addmm(_input_grad(dy2, w), dh, ab).view(x.shape) if need[0] else None
+        da = (dh.t() @ x.reshape(-1, x.shape[-1])).to(ad) if need[2] else None
+        db = (dy2.t() @ h).to(bd).mul_(scale) if need[3] else None   # scaled in its own type
         return dx, None, da, db, None, None, None
 
 
