@@ -843,6 +843,7 @@ void train_attention_backward(Tensor dq, Tensor dk, Tensor dv, Tensor dout, Tens
   for (const Tensor& t : {q, out, dout, dq}) train_attn_check(t, T, Hq * D);
   for (const Tensor& t : {k, v, dk, dv}) train_attn_check(t, T, Hkv * D);
   TORCH_CHECK(k.stride(0) == v.stride(0) && dk.stride(0) == dv.stride(0), "attention: k and v rows at one stride");
+  for (const Tensor& t : {q, k, dout}) TORCH_CHECK(t.stride(0) < (1 << 25), "attention: a tile's rows within 32 bits");
   CHECK_F32(lse);
   TORCH_CHECK(lse.numel() == Hq * T && scale > 0, "attention: lse [Hq, T]");
   CHECK_I32(cu);
