@@ -835,7 +835,7 @@ void train_attn_check(const Tensor& t, int64_t T, int64_t cols) {
 }
 
 // gradients of causal attention of q [T, Hq D], k and v [T, Hkv D] over the sequences of cu, the longest of max_len; out [T, Hq D];
-// lse [Hq, T]: log2 of each row's sum of exponentials
+// lse [Hq, T]: log2 of each row's sum of exponentials, or [B, Hq, S]: their natural logarithms, for B sequences of S tokens each
 void train_attention_backward(Tensor dq, Tensor dk, Tensor dv, Tensor dout, Tensor q, Tensor k, Tensor v, Tensor out, Tensor lse,
                               Tensor cu, int64_t Hq, int64_t Hkv, int64_t D, int64_t max_len, double scale) {
   const int64_t T = q.size(0), B = cu.numel() - 1;
@@ -845,10 +845,11 @@ void train_attention_backward(Tensor dq, Tensor dk, Tensor dv, Tensor dout, Tens
   TORCH_CHECK(k.stride(0) == v.stride(0) && dk.stride(0) == dv.stride(0), "attention: k and v rows at one stride");
   for (const Tensor& t : {q, k, dout}) TORCH_CHECK(t.stride(0) < (1 << 25), "attention: a tile's rows within 32 bits");
   CHECK_F32(lse);
-  TORCH_CHECK(lse.numel() == Hq * T && scale > 0, "attention: lse [Hq, T]");
+  TORCH_CHECK(lse.numel() == Hq * T && scale > 0 && (lse.dim() != 3 || (lse.size(0) == B && lse.size(1) == Hq)),
+              "attention: lse [Hq, T] or [B, Hq, S]");
   CHECK_I32(cu);
   if (B < 1 || T == 0 || max_len <= 0) return;
-  Tensor delta = at::empty_like(lse), part;
+  Tensor delta = at::empty({Hq, T}, lse.options()), l2 = lse.dim() == 3 ? at::empty_like(delta) : lse, part;
   nga::AttnBwdParams p{};
   p.parts = nga::attn_bwd_parts((int)B, (int)max_len, (int)Hq, (int)Hkv);
   if (p.parts > 1) {
@@ -857,7 +858,11 @@ void train_attention_backward(Tensor dq, Tensor dk, Tensor dv, Tensor dout, Tens
   }
   p.q = bfp(q); p.k = bfp(k); p.v = bfp(v); p.out = bfp(out); p.dout = bfp(dout);
   p.q_stride = q.stride(0); p.kv_stride = k.stride(0); p.out_stride = out.stride(0); p.dout_stride = dout.stride(0);
-  p.lse = lse.data_ptr<float>(); p.delta = delta.data_ptr<float>();
+  p.lse = l2.data_ptr<float>(); p.delta = delta.data_ptr<float>();
+  if (lse.dim() == 3) {
+    p.lse_in = lse.data_ptr<float>();
+    p.S = lse.size(2);
+  }
   p.dq = bfp(dq); p.dk = bfp(dk); p.dv = bfp(dv); p.dq_stride = dq.stride(0); p.dkv_stride = dk.stride(0);
   p.cu = cu.data_ptr<int32_t>(); p.T = T; p.Hq = (int)Hq; p.Hkv = (int)Hkv; p.scale = (float)scale;
   nga::launch_varlen_attention_backward(p, (int)B, (int)max_len, (int)D, cur_stream(q));

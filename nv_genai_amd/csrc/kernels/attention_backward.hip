@@ -124,7 +124,8 @@ __device__ __forceinline__ void ab_add_halves(f32x16 (&acc)[DT], float* red, int
 }
 }  // namespace
 
-// delta[hq][t] = sum_d dO O; 8 dims a lane
+// delta[hq][t] = sum_d dO O; 8 dims a lane. Log-sums as torch's attention leaves them, natural and by sequence, become lse beside
+// it (single operations: 9.6 us a call at 2 x 512 tokens, 32 heads)
 template <int D>
 __global__ void __launch_bounds__(256) attn_delta_kernel(AttnBwdParams P) {
   constexpr int LPR = D / 8;
@@ -139,7 +140,10 @@ __global__ void __launch_bounds__(256) attn_delta_kernel(AttnBwdParams P) {
   for (int j = 0; j < 8; ++j) s += bf2f(a[j]) * bf2f(b[j]);
 #pragma unroll
   for (int o = LPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  if (c == 0) P.delta[(int64_t)hq * P.T + t] = s;
+  if (c == 0) {
+    P.delta[(int64_t)hq * P.T + t] = s;
+    if (P.lse_in) P.lse[(int64_t)hq * P.T + t] = P.lse_in[(t / P.S * P.Hq + hq) * P.S + t % P.S] * AB_LOG2E;
+  }
 }
 
 // dk, dv [T, Hkv D] = the sums over the head parts of part [parts, 2, T, Hkv D]

@@ -138,7 +138,9 @@ __device__ __forceinline__ int xcd_item(const PrefillParams& P) {
 struct AttnBwdParams {
   const uint16_t *q, *k, *v, *out, *dout;
   int64_t q_stride, kv_stride, out_stride, dout_stride;
-  const float* lse;    // [Hq, T], log2 of each row's sum of exponentials
+  float* lse;          // [Hq, T], log2 of each row's sum of exponentials; set from lse_in, if given
+  const float* lse_in; // [T / S, Hq, S], their natural logarithms, for sequences of S tokens each
+  int64_t S;
   float* delta;        // [Hq, T] scratch
   uint16_t *dq, *dk, *dv;
   int64_t dq_stride, dkv_stride;

@@ -11,7 +11,6 @@ stands for, has a first derivative only.
 """
 from __future__ import annotations
 
-import math
 from typing import Optional, Sequence, Tuple
 
 import torch
@@ -282,9 +281,8 @@ class _Attention(Function):
         C = ops.kernels()
         d = torch.empty_like(r)
         w = [hq * D, hkv * D, hkv * D]
-        l2 = (lse.transpose(0, 1) * math.log2(math.e)).reshape(hq, -1).contiguous()
-        C.train_attention_backward(*d.split(w, 1), _rows(dout.reshape(-1, hq * D)), *r.split(w, 1), out, l2, cu, hq, hkv, D, lse.shape[2],
-                                   scale)
+        C.train_attention_backward(*d.split(w, 1), _rows(dout.reshape(-1, hq * D)), *r.split(w, 1), out, lse.contiguous(), cu, hq, hkv, D,
+                                   lse.shape[2], scale)
         C.rope_rows(d, cs, hq + hkv, hq + 2 * hkv, D, True, True)
         return (d.view(shape),) + (None,) * 7
 

@@ -50,3 +50,21 @@ def test_edges(gpu, D, hq, hkv, lens):
     ops.kernels().train_attention_backward(*got[:T].split(w, 1), do, *qkv.split(w, 1), out.to(BF), lse, cu, hq, hkv, D, max(lens), scale)
     assert ((got[:T].double() - ref).abs() <= bound + 2.0 ** -8 * (ref.abs() + bound)).all()
     assert (got[T] == 7).all()   # nothing is written past the last row
+
+
+@pytest.mark.parametrize("B,S,D,hq,hkv", [(1, 1, 128, 2, 1), (3, 65, 128, 4, 2), (2, 33, 64, 3, 3)])
+def test_log_sums_by_sequence(gpu, B, S, D, hq, hkv):
+    """Natural logarithms [B, Hq, S] give the bits of what they are turned into."""
+    from nv_genai_amd import ops
+
+    g = torch.Generator("cuda").manual_seed(S)
+    w = [hq * D, hkv * D, hkv * D]
+    rn = lambda *s: torch.randn(*s, device=gpu, generator=g)  # noqa: E731
+    qkv, do, out, lse = rn(B * S, sum(w)).to(BF), rn(B * S, hq * D).to(BF), rn(B * S, hq * D).to(BF), 30 + rn(B, hq, S)
+    cu = torch.arange(B + 1, dtype=torch.int32, device=gpu) * S
+    got = []
+    for how in (lse, (lse.transpose(0, 1) * math.log2(math.e)).reshape(hq, -1).contiguous()):
+        d = torch.empty_like(qkv)
+        ops.kernels().train_attention_backward(*d.split(w, 1), do, *qkv.split(w, 1), out, how, cu, hq, hkv, D, S, D ** -0.5)
+        got.append(d)
+    assert torch.equal(*got)
