@@ -807,19 +807,28 @@ void prefill_attention(Tensor out, Tensor q, c10::optional<Tensor> k, c10::optio
     TORCH_CHECK(k->dim() == 2 && k->stride(1) == 1 && k->stride(0) == v->stride(0) && k->size(0) == q.size(0));
     TORCH_CHECK(k->stride(0) % 8 == 0 && k->size(1) >= Hkv * D && v->size(1) >= Hkv * D);
     if (B == 0 || max_q_len == 0) return;
-    // the kernel's LDS-DMA moves aligned 16-byte pieces: rows of other origins are copied once
-    auto rows = [&](const Tensor& t) {
-      return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.narrow(1, 0, Hkv * D).clone(at::MemoryFormat::Contiguous);
+    // the kernel's LDS-DMA moves aligned 16-byte pieces, a tile's rows within 32 bits: rows of other origins are copied once
+    auto rows = [&](const Tensor& t, int64_t heads) {
+      return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && t.stride(0) < (1 << 25)
+                 ? t : t.narrow(1, 0, heads * D).clone(at::MemoryFormat::Contiguous);
     };
-    Tensor kr = rows(*k), vr = rows(*v);
+    Tensor kr = rows(*k, Hkv), vr = rows(*v, Hkv), qr = rows(q, Hq);
     if (kr.stride(0) != vr.stride(0)) {
       kr = k->narrow(1, 0, Hkv * D).clone(at::MemoryFormat::Contiguous);
       vr = v->narrow(1, 0, Hkv * D).clone(at::MemoryFormat::Contiguous);
     }
+    p.q = bfp(qr);
+    p.q_stride = qr.stride(0);
     p.k = bfp(kr);
     p.v = bfp(vr);
     p.kv_stride = kr.stride(0);
+    const bool straight = reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0 && out.stride(0) % 8 == 0;   // its stores too
+    Tensor o = straight ? out : at::empty({out.size(0), Hq * D}, out.options());
+    if (!straight) o.copy_(out.narrow(1, 0, Hq * D));   // rows of no sequence stay
+    p.out = bfp(o);
+    p.out_stride = o.stride(0);
     nga::launch_varlen_attention(p, (int)B, (int)max_q_len, (int)D, causal, cur_stream(q));
+    if (!straight) out.narrow(1, 0, Hq * D).copy_(o);
     return;
   }
   p.impl = (int)impl;

@@ -14,8 +14,11 @@
 // Bound by the softmax: 32 exponentials and about 100 other vector operations per lane and tile against 16 MFMAs of 32
 // cycles at head_dim 64, and by rounding up short sequences: 670 to 770 TFLOP/s at 512 and 2,048 tokens, 390 for 90 to 512
 // tokens. The 16x16 form before it wrote V transposed into LDS two bytes at a time. Layers as measured: 64 sequences of 90
-// to 512 tokens, 16 heads of 64: 170 -> 96 us, with deal_xcds 77; 20 sequences, 32 / 8 heads of 128: 298 -> 124 us. (The transpose read as
-// an asm block that waits for its own reads alone, where the compiler waits for the next tile's DMA too: equal.)
+// to 512 tokens, 16 heads of 64: 170 -> 96 us, with deal_xcds 71; 20 sequences, 32 / 8 heads of 128: 298 -> 81 us. With queries and
+// results in whole rows through LDS, where a lane's own pieces of 16 and 8 bytes lie a row's stride apart, and tile addresses from a
+// scalar and a lane's fixed offset: 67 and 74 us (64 of 512 tokens, 32 / 8 heads: 382 -> 359). (The transpose read as an asm block that
+// waits for its own reads alone, where the compiler waits for the next tile's DMA too: equal; the maximum over both halves by
+// permlane32_swap: 1 % either way.)
 #include "common.h"
 #include "kernels.h"
 
@@ -69,12 +72,6 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) varlen_attn_kernel(Pref
   const int qr = min(row0 + r32, qlen - 1);
   const int W = CAUSAL ? P.window : 0;
 
-  bf16x8 qf[DS];
-  {
-    const uint16_t* qp = P.q + (int64_t)(q0 + qr) * P.q_stride + (int64_t)hq * D + 8 * h;
-#pragma unroll
-    for (int s = 0; s < DS; ++s) qf[s] = as_bf16x8(load8(qp + 16 * s));
-  }
   // tiles of the workgroup; a wave computes those that its own rows see
   const int hi_wg = min(qlen - 1, qb * RW + RW - 1), hi_w = min(qlen - 1, row0 + 31);
   const int n_tiles = (CAUSAL ? hi_wg : qlen - 1) / KT + 1;
@@ -83,24 +80,47 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) varlen_attn_kernel(Pref
 
   // DMA: wave instruction i fills chunk positions [64 (NI w + i), +64) of a tile, position p holding chunk
   // (p % NC) ^ swizzle of row p / NC
-  int krow[NI], kcol[NI], vcol[NI];
+  const uint32_t step = (uint32_t)P.kv_stride;
+  uint32_t krow[NI], kcol[NI], vcol[NI], koff[NI], vplace[NI];   // a lane's place, to be added to the tile's address (scalar)
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int p = (NI * w + i) * 64 + lane;
     krow[i] = p / NC;
     kcol[i] = ((p % NC) ^ vl_kswz<D>(krow[i])) * 8;
     vcol[i] = ((p % NC) ^ vl_vswz<D>(krow[i])) * 8;
+    koff[i] = krow[i] * step + kcol[i];
+    vplace[i] = krow[i] * step + vcol[i];
   }
   const uint16_t* const kp = P.k + (int64_t)q0 * P.kv_stride + (int64_t)kvh * D;
   const uint16_t* const vp = P.v + (int64_t)q0 * P.kv_stride + (int64_t)kvh * D;
   auto issue = [&](int t, int buf) {
+    const uint32_t left = qlen - 1 - t * KT;
+    const uint16_t *const kt = kp + (int64_t)t * KT * P.kv_stride, *const vt = vp + (int64_t)t * KT * P.kv_stride;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int64_t row = (int64_t)min(t * KT + krow[i], qlen - 1) * P.kv_stride;   // keys past the end are masked
-      glds16(kp + row + kcol[i], kbuf + buf * TILE + (NI * w + i) * 512);
-      glds16(vp + row + vcol[i], vbuf + buf * TILE + (NI * w + i) * 512);
+      uint32_t a = koff[i], c = vplace[i];
+      if (left < KT - 1) {   // keys past the end are masked
+        a = min(krow[i], left) * step + kcol[i];
+        c = min(krow[i], left) * step + vcol[i];
+      }
+      glds16(kt + a, kbuf + buf * TILE + (NI * w + i) * 512);
+      glds16(vt + c, vbuf + buf * TILE + (NI * w + i) * 512);
     }
   };
+  // A wave's 32 rows pass through its quarter of a tile buffer, that of K or V, in whole pieces: the queries through the second
+  // one before its first tile comes, the results through the one whose tile everyone has read. Chunk c of row r lies at c ^ r (mod NC).
+  auto rows_at = [&](int buf) { return smem + ((w >> 1) * 2 + buf) * TILE + (w & 1) * (TILE / 2); };
+  constexpr int NR = D / 16;   // instructions for 32 rows
+  bf16x8 qf[DS];
+  {
+    const uint16_t* qp = P.q + (int64_t)(q0 + row0) * P.q_stride + (int64_t)hq * D;
+    if (active)
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        const int p = i * 64 + lane, r = p / NC;
+        glds16(qp + min(r, qlen - 1 - row0) * P.q_stride + ((p % NC) ^ (r % NC)) * 8, rows_at(1) + i * 512);
+      }
+  }
 
   const int prow = (r32 & ~12) | ((r32 & 4) << 1) | ((r32 & 8) >> 1);   // perm(r32)
   const int ksw = vl_kswz<D>(prow);                                     // of prow + 32 too
@@ -120,6 +140,11 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) varlen_attn_kernel(Pref
   for (int dt = 0; dt < DT; ++dt) o[dt] = (f32x16)(0.f);
 
   issue(t_first, 0);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NI) : "memory");
+#pragma unroll
+  for (int s = 0; s < DS; ++s) qf[s] = as_bf16x8(*reinterpret_cast<const u16x8*>(rows_at(1) + r32 * D + (((2 * s + h) ^ (r32 % NC)) << 3)));
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
   for (int t = t_first; t < n_tiles; ++t) {
     const int buf = (t - t_first) & 1;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's part of tile t is there
@@ -190,19 +215,25 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) varlen_attn_kernel(Pref
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may outlive the workgroup
   l += __shfl_xor(l, 32, 64);
-  if (active && row0 + r32 < qlen) {
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-    uint16_t* op = P.out + (int64_t)(q0 + qr) * P.out_stride + (int64_t)hq * D + 4 * h;
-    // o[dt][j]: dim 32 dt + (j & 3) + 8 (j >> 2) + 4 h
+  if (!active) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  uint16_t* const rows = rows_at((n_tiles - t_first) & 1);
+  // o[dt][j]: dim 32 dt + (j & 3) + 8 (j >> 2) + 4 h
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        u16x4 v;
+    for (int g = 0; g < 4; ++g) {
+      u16x4 v;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = f2bf(o[dt][4 * g + j] * inv);
-        *reinterpret_cast<u16x4*>(op + 32 * dt + 8 * g) = v;
-      }
+      for (int j = 0; j < 4; ++j) v[j] = f2bf(o[dt][4 * g + j] * inv);
+      *reinterpret_cast<u16x4*>(rows + r32 * D + (((4 * dt + g) ^ (r32 % NC)) << 3) + 4 * h) = v;
+    }
+  uint16_t* const op = P.out + (int64_t)(q0 + row0) * P.out_stride + (int64_t)hq * D;
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int p = i * 64 + lane, r = p / NC;
+    const u16x8 v = *reinterpret_cast<const u16x8*>(rows + r * D + (((p % NC) ^ (r % NC)) << 3));
+    if (row0 + r < qlen) *reinterpret_cast<u16x8*>(op + r * P.out_stride + (p % NC) * 8) = v;
   }
 }
 

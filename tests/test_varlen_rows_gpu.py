@@ -1,0 +1,43 @@
+"""Packed attention: rows in and out in whole pieces (attention_varlen.hip). Each row's result is the same bits wherever its tensors
+lie, against 64 bits it is within the kernel's roundings, and nothing else is written."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+# ends within a wave's 32 rows, a workgroup's 128 (32 of four heads with four query heads a KV head), a key tile of 64; one tile and two
+@pytest.mark.parametrize("D,hq,hkv", [(32, 3, 3), (64, 2, 1), (64, 4, 1), (128, 8, 2), (128, 2, 2)])
+@pytest.mark.parametrize("lens", [[1], [31, 33, 64], [65, 127, 2], [129, 200, 63]])
+@pytest.mark.parametrize("causal", [False, True])
+def test_rows(gpu, D, hq, hkv, lens, causal):
+    from nv_genai_amd import ops
+
+    g = torch.Generator("cuda").manual_seed(D + hq + lens[0])
+    T, w, scale = sum(lens), hq * D, D ** -0.5
+    q, k, v = (torch.randn(T, h * D, device=gpu, generator=g).to(BF) for h in (hq, hkv, hkv))
+    cu = torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()], dtype=torch.int32, device=gpu)
+    got = ops.varlen_attention(q, k, v, cu, hq, hkv, D, max(lens), scale, causal)
+    at = 0
+    for n in lens:
+        Q, K, V = (t[at:at + n].view(n, -1, D).transpose(0, 1).double() for t in (q, k, v))
+        K, V = K.repeat_interleave(hq // hkv, 0), V.repeat_interleave(hq // hkv, 0)
+        S = Q @ K.transpose(1, 2).contiguous() * scale
+        P = (S.masked_fill(torch.ones(n, n, device=gpu).triu(1).bool(), float("-inf")) if causal else S).softmax(-1)
+        ref = (P @ V).transpose(0, 1).reshape(n, w)
+        size = (P @ V.abs()).transpose(0, 1).reshape(n, w)
+        # probabilities as bf16 and the result as bf16, 2^-9 each, doubled for the fp32 steps between
+        assert ((got[at:at + n].double() - ref).abs() <= 2.0 ** -8 * (size + ref.abs())).all()
+        at += n
+
+    def odd(t, by):   # the same rows elsewhere: by values off a 16-byte address, 8 more a row
+        s = torch.zeros(T, t.shape[1] + 16, dtype=BF, device=gpu)[:, by:by + t.shape[1]]
+        return s.copy_(t)
+
+    for by in (0, 8, 3):
+        room = torch.full((T + 1, w + 16), 7.0, dtype=BF, device=gpu)
+        ops.varlen_attention(odd(q, by), odd(k, by), odd(v, by), cu, hq, hkv, D, max(lens), scale, causal, out=room[:T, by:by + w])
+        assert torch.equal(room[:T, by:by + w], got)
+        room[:T, by:by + w] = 7.0
+        assert (room == 7.0).all()
