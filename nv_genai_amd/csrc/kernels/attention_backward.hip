@@ -10,10 +10,10 @@
 //          dQ^T[d][q] = K^T[d][key] dS^T[key][q], K^T by the transpose read.
 // A wave alone on its SIMD waits for its own products, exponentials and LDS reads in turn (heads of 128, whose sums and operands
 // fill 440 registers), so there two waves share each 32 keys or queries and take the halves of every tile (HW 2): their sums meet
-// in LDS at the end, and V (dk/dv) stays in LDS. Three buffers instead of two were 15 % slower: it is not the tiles' latency.
-// 8 x 2,048 tokens, 32 / 8 heads of 128: 1.23 ms (558 TFLOP/s; one wave 1.80; torch's flash attention 4.00), 2 x 512 57 us (74), 32 x 32
-// 33 (34); 4 x 1,024, 12 heads of 64: 71 us (84). Of these, rows brought in and out in whole pieces through LDS gave 8 % and 5 %, masks in
-// a branch and tile addresses from a scalar 7 % (12 % with heads of 64).
+// in LDS at the end, and V (dk/dv) stays in LDS. Three buffers instead of two were 8 to 16 % slower: it is not the tiles' latency.
+// 8 x 2,048 tokens, 32 / 8 heads of 128: 1.20 ms (574 TFLOP/s; one wave 1.80; torch's flash attention 4.00), 2 x 512 54 us (74),
+// 32 x 16 30 (32); 4 x 1,024, 12 heads of 64: 71 us (84). Of these, rows brought in and out in whole pieces through LDS gave 8 % and 5 %,
+// masks in a branch and tile addresses from a scalar 7 % (12 % with heads of 64), delta from the dq kernel's rows instead of a launch 4 %.
 // Tiles by LDS-DMA as they lie in memory, two buffers, as in the forward. Chunk swizzle: 16 rows of one chunk and 64 bytes of
 // 4 consecutive rows both fall into distinct banks.
 #include "common.h"
@@ -124,7 +124,13 @@ __device__ __forceinline__ void ab_add_halves(f32x16 (&acc)[DT], float* red, int
 }
 }  // namespace
 
-// delta[hq][t] = sum_d dO O; 8 dims a lane. Log-sums as torch's attention leaves them, natural and by sequence, become lse beside
+// a row's log-sum from lse_in
+__device__ __forceinline__ float ab_lse(const AttnBwdParams& P, uint32_t t, int hq) {
+  const uint32_t S = (uint32_t)P.S;
+  return P.lse_in[((int64_t)(t / S) * P.Hq + hq) * S + t % S] * AB_LOG2E;
+}
+
+// delta[hq][t] = sum_d dO O; 8 dims a lane; with two waves for 32 rows the dq kernel works them out. Log-sums as torch's attention leaves them, natural and by sequence, become lse beside
 // it (single operations: 9.6 us a call at 2 x 512 tokens, 32 heads)
 template <int D>
 __global__ void __launch_bounds__(256) attn_delta_kernel(AttnBwdParams P) {
@@ -142,7 +148,7 @@ __global__ void __launch_bounds__(256) attn_delta_kernel(AttnBwdParams P) {
   for (int o = LPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
   if (c == 0) {
     P.delta[(int64_t)hq * P.T + t] = s;
-    if (P.lse_in) P.lse[(int64_t)hq * P.T + t] = P.lse_in[(t / P.S * P.Hq + hq) * P.S + t % P.S] * AB_LOG2E;
+    if (P.lse_in) P.lse[(int64_t)hq * P.T + t] = ab_lse(P, (uint32_t)t, hq);
   }
 }
 
@@ -344,6 +350,9 @@ __global__ void __launch_bounds__(256 * HW, D == 128 ? HW : 2) attn_bwd_dq_kerne
     if constexpr (HW == 2) {
       ab_rows_in<D>(qp, P.q_stride, len - qb * RW, qt, w, lane);
       ab_rows_in<D>(op, P.dout_stride, len - qb * RW, ot, w, lane);
+      // O, for delta, in the second tile's buffers, which lie a tile apart
+      ab_rows_in<D>(P.out + (int64_t)(q0 + qb * RW) * P.out_stride + (int64_t)hq * D, P.out_stride, len - qb * RW,
+                    smem + (w < 4 ? 1 : 2) * TILE, w, lane);
     } else if (active) {
 #pragma unroll
       for (int s = 0; s < DS; ++s) {
@@ -352,7 +361,8 @@ __global__ void __launch_bounds__(256 * HW, D == 128 ? HW : 2) attn_bwd_dq_kerne
       }
     }
   }
-  const float lse = P.lse[(int64_t)hq * P.T + q0 + qr], delta = P.delta[(int64_t)hq * P.T + q0 + qr];
+  const int64_t stat = (int64_t)hq * P.T + q0 + qr;
+  float lse = P.lse_in ? ab_lse(P, q0 + qr, hq) : P.lse[stat], delta = HW == 2 ? 0.f : P.delta[stat];
   const int hi_w = min(len - 1, row0 + 31);
   const int n_tiles = min(len - 1, qb * RW + RW - 1) / KT + 1;
   const int w_last = hi_w / KT;
@@ -395,6 +405,15 @@ __global__ void __launch_bounds__(256 * HW, D == 128 ? HW : 2) attn_bwd_dq_kerne
     for (int s = 0; s < DS; ++s) {
       qf[s] = ab_frag<D>(qt, 32 * (w % 4) + r32, 2 * s + h);
       of[s] = ab_frag<D>(ot, 32 * (w % 4) + r32, 2 * s + h);
+      const bf16x8 o = ab_frag<D>(smem + (w % 4 < 2 ? 1 : 2) * TILE, 32 * (w % 4) + r32, 2 * s + h);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) delta = __builtin_fmaf((float)of[s][j], (float)o[j], delta);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the second tile comes behind the next barrier
+    delta += __shfl_xor(delta, 32, 64);
+    if (w < 4 && h == 0 && row0 + r32 < len) {
+      P.delta[stat] = delta;
+      if (P.lse_in) P.lse[stat] = lse;
     }
   }
   for (int t = 0; t < n_tiles; ++t) {
@@ -440,16 +459,23 @@ __global__ void __launch_bounds__(256 * HW, D == 128 ? HW : 2) attn_bwd_dq_kerne
 
 template <int D, int HW>
 static void attn_bwd(AttnBwdParams p, int num_seqs, int max_len, hipStream_t stream) {
-  const int64_t dl = p.T * p.Hq * (D / 8);
-  attn_delta_kernel<D><<<(unsigned)((dl + 255) / 256), 256, 0, stream>>>(p);
   p.ntiles = (max_len + 127) / 128;
+  const auto dq = [&](AttnBwdParams p) {
+    p.total = p.ntiles * p.Hq * num_seqs;
+    p.per_xcd = (p.total + 7) / 8;
+    attn_bwd_dq_kernel<D, HW><<<8 * p.per_xcd, 256 * HW, 0, stream>>>(p);
+  };
+  if (HW == 1) {
+    const int64_t dl = p.T * p.Hq * (D / 8);
+    attn_delta_kernel<D><<<(unsigned)((dl + 255) / 256), 256, 0, stream>>>(p);
+  } else {
+    dq(p);
+  }
   p.total = p.ntiles * p.parts * p.Hkv * num_seqs;
   p.per_xcd = (p.total + 7) / 8;
   attn_bwd_dkdv_kernel<D, HW><<<8 * p.per_xcd, 256 * HW, 0, stream>>>(p);
   if (p.parts > 1) attn_sum_parts_kernel<<<(unsigned)((p.T * p.Hkv * D / 4 + 255) / 256), 256, 0, stream>>>(p, p.Hkv * D);
-  p.total = p.ntiles * p.Hq * num_seqs;
-  p.per_xcd = (p.total + 7) / 8;
-  attn_bwd_dq_kernel<D, HW><<<8 * p.per_xcd, 256 * HW, 0, stream>>>(p);
+  if (HW == 1) dq(p);
 }
 
 // The query heads of a KV head one workgroup each, their sums added up after, while key tiles alone leave most CUs idle
