@@ -105,17 +105,9 @@ __device__ __forceinline__ void v2_row_block(const PrefillParams& P, uint16_t* s
   // workgroup's whole tile range (uniform control flow for the software pipeline below); with
   // several row blocks per workgroup the earlier blocks' extra tiles are fully masked.
   int qr = qb * RW + rb * 32 + r32;
-  const bool row_ok = qr < qlen;
-  if (!row_ok) qr = qlen - 1;
+  if (qr >= qlen) qr = qlen - 1;
   const int qpos = ctx - qlen + qr;
   const int W = CAUSAL ? P.window : 0;
-
-  bf16x8 qf[8];
-  {
-    const uint16_t* qp = P.q + (int64_t)(q0 + qr) * P.q_stride + (int64_t)hq * D + 8 * h;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) qf[s] = as_bf16x8(load8(qp + 16 * s));
-  }
 
   // tile range of the workgroup; tiles needing a mask: at / past the first query's diagonal,
   // and (window) before the last query's window start
@@ -181,6 +173,7 @@ __device__ __forceinline__ void v2_row_block(const PrefillParams& P, uint16_t* s
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] = (f32x16)(0.f);
 
+  bf16x8 qf[8];
   // The loop works in 32-key halves of the 64-key DMA tiles. Half h2 of tile t:
   //   S^T = K . Q^T  (8 MFMAs; K rows 32 h2 + perm(r) of the K tile)
   //   softmax        (16 scores per lane; keys (j & 7) + 8h + 16 (j >> 3) of the half)
@@ -316,8 +309,23 @@ __device__ __forceinline__ void v2_row_block(const PrefillParams& P, uint16_t* s
     if constexpr (ABL != 2) stage(Sa, vbuf + par * TILE, 0, Sb, kc_, 1, t, KS > 1 && t >= n_tiles);
   };
 
+  // A wave's 32 rows go in and out in whole pieces, through LDS: a lane's own pieces lie a row's stride apart. The queries come
+  // through the second tile's buffers, a half of one a wave; chunk c of row r lies at c ^ r (mod 16). 32 / 8 heads, us, before and
+  // now: 16 prompts of 600 to 950 tokens 160 and 146, one of 203 11.5 and 10.3, of 1,200 33.0 and 31.0, 4 of 4,096 586 and 586.
+  const int row0 = qb * RW + rb * 32;
+  uint16_t* const qrows = (w < 2 ? kbuf : vbuf) + TILE + (w & 1) * (TILE / 2);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int r = 4 * i + (lane >> 4);
+    glds16(P.q + (int64_t)(q0 + min(row0 + r, qlen - 1)) * P.q_stride + (int64_t)hq * D + (((lane & 15) ^ (r & 15)) << 3), qrows + i * 512);
+  }
   issue_k(tile_of(0), kbuf);
   issue_v(tile_of(0), vbuf);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int s = 0; s < 8; ++s) qf[s] = as_bf16x8(*reinterpret_cast<const u16x8*>(qrows + r32 * D + (((2 * s + h) ^ (r32 & 15)) << 3)));
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
   iter(0, 0, true);
   for (int i = 1; i < nt; i += 2) {
     iter(i, 1, false);
@@ -333,11 +341,13 @@ __device__ __forceinline__ void v2_row_block(const PrefillParams& P, uint16_t* s
 
   // epilogue: o[dt][j] = O^T[d = 32 dt + (j & 3) + 8 (j >> 2) + 4h][q = r32]
   l += __shfl_xor(l, 32, 64);
+  __syncthreads();   // every wave is done with the tiles
+  uint16_t* rows = smem + w * (TILE / 2);
   if constexpr (KS > 1) {
     // group 1 -> LDS (the tile buffers are free: every wave waited for its own DMA above and
     // the barrier below orders the hand-off); group 0 merges: O = 2^(m0-M) O0 + 2^(m1-M) O1
-    __syncthreads();
     float* xo = reinterpret_cast<float*>(smem) + (w * 64 + lane) * 66;
+    rows = smem + w * 64 * 66 * 2;   // where the wave's own part lay
     if (grp == 1) {
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt)
@@ -358,18 +368,21 @@ __device__ __forceinline__ void v2_row_block(const PrefillParams& P, uint16_t* s
       for (int j = 0; j < 16; ++j) o[dt][j] = o[dt][j] * f0 + xo[16 * dt + j] * f1;
     l = l * f0 + l1 * f1;
   }
-  if (row_ok) {
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-    uint16_t* op = P.out + (int64_t)(q0 + qr) * P.out_stride + (int64_t)hq * D + 4 * h;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+  for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        u16x4 v;
+    for (int g = 0; g < 4; ++g) {
+      u16x4 v;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = f2bf(o[dt][4 * g + j] * inv);
-        *reinterpret_cast<u16x4*>(op + 32 * dt + 8 * g) = v;
-      }
+      for (int j = 0; j < 4; ++j) v[j] = f2bf(o[dt][4 * g + j] * inv);
+      *reinterpret_cast<u16x4*>(rows + r32 * D + (((4 * dt + g) ^ (r32 & 15)) << 3) + 4 * h) = v;
+    }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int r = 4 * i + (lane >> 4);
+    const u16x8 v = *reinterpret_cast<const u16x8*>(rows + r * D + (((lane & 15) ^ (r & 15)) << 3));
+    if (row0 + r < qlen) *reinterpret_cast<u16x8*>(P.out + (int64_t)(q0 + row0 + r) * P.out_stride + (int64_t)hq * D + (lane & 15) * 8) = v;
   }
 }
 

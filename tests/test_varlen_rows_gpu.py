@@ -1,4 +1,4 @@
-"""Packed attention: rows in and out in whole pieces (attention_varlen.hip). Each row's result is the same bits wherever its tensors
+"""Packed and paged attention: rows in and out in whole pieces (attention_varlen.hip, attention_prefill_v2.hip). Each row's result is the same bits wherever its tensors
 lie, against 64 bits it is within the kernel's roundings, and nothing else is written."""
 import pytest
 import torch
@@ -40,4 +40,45 @@ def test_rows(gpu, D, hq, hkv, lens, causal):
         ops.varlen_attention(odd(q, by), odd(k, by), odd(v, by), cu, hq, hkv, D, max(lens), scale, causal, out=room[:T, by:by + w])
         assert torch.equal(room[:T, by:by + w], got)
         room[:T, by:by + w] = 7.0
+        assert (room == 7.0).all()
+
+
+# one group of waves and two (few row blocks), one to four heads a workgroup; chunks of prompts, whose keys lie before them
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (4, 2), (2, 2)])
+@pytest.mark.parametrize("lens,ctxs", [([1], [1]), ([31, 64, 33], [31, 70, 200]), ([200, 129], [200, 400]), ([700] * 12, [700] * 12)])
+def test_paged_rows(gpu, hq, hkv, lens, ctxs):
+    from nv_genai_amd import ops
+
+    D, T, B = 128, sum(lens), len(lens)
+    g = torch.Generator("cuda").manual_seed(T + hq)
+    rn = lambda *s: torch.randn(*s, device=gpu, generator=g).to(BF)  # noqa: E731
+    pages = [(c + 63) // 64 for c in ctxs]
+    q, kc, vc = rn(T, hq * D), rn(sum(pages), hkv, 64, D), rn(sum(pages), hkv, D, 64)
+    bt = torch.zeros(B, max(pages), dtype=torch.int32)
+    for i, n in enumerate(pages):
+        bt[i, :n] = torch.arange(n) + sum(pages[:i])
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=gpu)  # noqa: E731
+    cu, cl, bt = i32([0, *torch.tensor(lens).cumsum(0).tolist()]), i32(ctxs), bt.to(gpu)
+
+    def run(q, out):
+        ops.kernels().prefill_attention(out, q, None, None, kc, vc, bt, cu, cl, hq, hkv, D, max(lens), D ** -0.5, True, 0, 0, 1.0, 1.0)
+        return out
+
+    got = run(q, torch.empty(T, hq * D, dtype=BF, device=gpu))
+    at = 0
+    for n, c, p in zip(lens, ctxs, [sum(pages[:i]) for i in range(B)]):
+        m = (c + 63) // 64
+        K = kc[p:p + m].transpose(1, 2).reshape(-1, hkv, D)[:c].transpose(0, 1).double().repeat_interleave(hq // hkv, 0)
+        V = vc[p:p + m].permute(0, 3, 1, 2).reshape(-1, hkv, D)[:c].transpose(0, 1).double().repeat_interleave(hq // hkv, 0)
+        S = q[at:at + n].view(n, -1, D).transpose(0, 1).double() @ K.transpose(1, 2).contiguous() * D ** -0.5
+        P = S.masked_fill(torch.ones(n, c, device=gpu).triu(c - n + 1).bool(), float("-inf")).softmax(-1)
+        flat = lambda x: x.transpose(0, 1).reshape(n, -1)  # noqa: E731
+        ref = flat(P @ V)
+        assert ((got[at:at + n].double() - ref).abs() <= 2.0 ** -8 * (flat(P @ V.abs()) + ref.abs())).all()
+        at += n
+    for by in (0, 8, 3):
+        wide = torch.zeros(T, hq * D + 16, dtype=BF, device=gpu)[:, by:by + hq * D].copy_(q)
+        room = torch.full((T + 1, hq * D + 16 + by), 7.0, dtype=BF, device=gpu)
+        assert torch.equal(run(wide, room[:T, by:by + hq * D]), got)
+        room[:T, by:by + hq * D] = 7.0
         assert (room == 7.0).all()
