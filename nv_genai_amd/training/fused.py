@@ -408,6 +408,6 @@ class _LoraLinear(Function):
 
 
 def lora_linear(x: torch.Tensor, w: torch.Tensor, a: torch.Tensor, b: torch.Tensor, scale: float) -> torch.Tensor:
-    """x w^T + scale (x a^T) b^T with a frozen bf16 w (w.shape[0] % 8 == 0); the adapter's part of x's gradient joins in the
-    accumulator of its second product."""
+    """x w^T + scale (x a^T) b^T with a frozen bf16 w (w.shape[0] % 8 == 0); the adapter's gradients come from lora.hip, which adds
+    its part of x's to that through w, and of ranks that it does not take from single operations."""
     return _LoraLinear.apply(x, w, a, b, a.to(BF16), b.to(BF16), scale)
