@@ -355,7 +355,7 @@ __global__ void __launch_bounds__(256) sample_slices_kernel(const float* __restr
                                                             SampleSlice* __restrict__ slices, SampleEntry* __restrict__ list) {
   __shared__ ArgMax ared[4];
   __shared__ float red[4];
-  __shared__ int counts[4], count;
+  __shared__ int counts[4][4];
   const int row = blockIdx.y, t = threadIdx.x;
   if (penalty && penalty[row] != 1.f) return;   // sample_kernel changes the row first
   const float* x = logits + (int64_t)row * V;
@@ -387,8 +387,6 @@ __global__ void __launch_bounds__(256) sample_slices_kernel(const float* __restr
   }
   am = wave_argmax(am);
   if ((t & 63) == 0) ared[t >> 6] = am;
-  if (t < 4) counts[t] = 0;
-  if (t == 0) count = 0;
   __syncthreads();
   am = am_max(am_max(ared[0], ared[1]), am_max(ared[2], ared[3]));
   SampleEntry* const own = list + ((int64_t)row * gridDim.x + blockIdx.x) * LISTED;
@@ -398,22 +396,35 @@ __global__ void __launch_bounds__(256) sample_slices_kernel(const float* __restr
     const float v = raw[j] * inv_t;
     if (v > -INFINITY) z += v == am.v ? 1.f : __expf(v - am.v);
   }
+  int count = 0;
   if (!greedy) {
+    const int w = t >> 6, lane = t & 63;
     int n[4] = {0, 0, 0, 0};
 #pragma unroll
     for (int j = 0; j < 8; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) n[r] += __popcll(__ballot(am.v - raw[j] * inv_t < DRANGE / (1 << r)));
-    if ((t & 63) < 4) atomicAdd(&counts[t & 63], (t & 63) == 0 ? n[0] : (t & 63) == 1 ? n[1] : (t & 63) == 2 ? n[2] : n[3]);
+    if (lane < 4) counts[w][lane] = lane == 0 ? n[0] : lane == 1 ? n[1] : lane == 2 ? n[2] : n[3];
     __syncthreads();
+    // places by wave, then j, then lane: the passes over the lists add up in their order, so it is the same at every call
+    int place = 0;
 #pragma unroll
-    for (int r = 3; r >= 0; --r)
-      if (counts[r] <= LISTED) range = DRANGE / (1 << r);
+    for (int r = 3; r >= 0; --r) {
+      const int all = counts[0][r] + counts[1][r] + counts[2][r] + counts[3][r];
+      if (all > LISTED) continue;
+      range = DRANGE / (1 << r);
+      count = all;
+      place = (w > 0 ? counts[0][r] : 0) + (w > 1 ? counts[1][r] : 0) + (w > 2 ? counts[2][r] : 0);
+    }
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (am.v - raw[j] * inv_t < range) own[atomicAdd(&count, 1)] = SampleEntry{raw[j], at(j)};   // at most LISTED
+    for (int j = 0; j < 8; ++j) {
+      const bool in = am.v - raw[j] * inv_t < range;
+      const uint64_t m = __ballot(in);
+      if (in) own[place + __popcll(m & ((1ull << lane) - 1ull))] = SampleEntry{raw[j], at(j)};
+      place += __popcll(m);
+    }
   }
-  z = block_sum(z, red);   // with barriers: the count is complete
+  z = block_sum(z, red);
   if (t == 0) slices[(int64_t)row * gridDim.x + blockIdx.x] = SampleSlice{am.v, z, am.i, count, range};
 }
 

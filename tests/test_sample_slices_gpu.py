@@ -66,3 +66,23 @@ def test_a_penalty_changes_the_row_first(gpu):
     tok, lp = ops.sample(x.clone(), *arg, pen, hist)
     assert torch.equal(tok.long(), want.argmax(1))
     assert torch.allclose(lp, torch.log_softmax(want.double(), 1).max(1).values.float(), atol=1e-5)
+
+
+def test_the_same_draw_again(gpu):
+    """top-k and top-p together: the target of top-p comes of a sum of what top-k keeps, so that must add up in one order. Rows whose
+    target lies at the boundary between two values, give or take an ulp, draw again what they drew."""
+    V, K, B = 128_256, 1000, 64
+    g = torch.Generator().manual_seed(5)
+    near = torch.randperm(V, generator=g)[:K + 200]
+    x = torch.full((V,), -30.0)
+    x[near] = -6 * torch.rand(K + 200, generator=g)
+    w = x[near].double().sort(descending=True).values[:K].exp()
+    at = torch.randint(50, K - 200, (B,), generator=g)
+    p = (w.cumsum(0) / w.sum())[at].float() + (torch.arange(B) % 9 - 4) * 2.0 ** -25
+    x = x.expand(B, V).contiguous().to(gpu)
+    arg = (torch.ones(B, device=gpu), torch.full((B,), K, dtype=torch.int32, device=gpu), p.to(gpu))
+    row = torch.arange(B, device=gpu)
+    for s in range(300):
+        first = ops.sample(x, *arg, 1000 * s + row, row)[0]
+        for _ in range(6):
+            assert torch.equal(ops.sample(x, *arg, 1000 * s + row, row)[0], first)
