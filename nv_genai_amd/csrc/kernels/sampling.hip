@@ -472,7 +472,7 @@ __global__ void __launch_bounds__(NT) sample_kernel(
   near.x = x;
   near.V = V;
   near.listed = false;
-  float reach = -INFINITY;   // of this thread's slice all values above it are listed
+  float range = DRANGE;   // of this thread's slice values less than this below its largest one are listed
   if (nslices > 0 && !changed) {
     const SampleSlice* const own = slices + (int64_t)row * nslices;
 #pragma unroll
@@ -487,7 +487,7 @@ __global__ void __launch_bounds__(NT) sample_kernel(
     if (t < nslices) {
       am = ArgMax{own[t].m, own[t].i};
       z = own[t].z;
-      reach = am.v - own[t].range;
+      range = own[t].range;
     }
   } else {
     for_row(x, V, [&](int i, float raw) {
@@ -504,7 +504,9 @@ __global__ void __launch_bounds__(NT) sample_kernel(
   const float m_thr = am.v;
   am = block_argmax(am, sm.ared);
   const float M = am.v;
-  near.listed = __syncthreads_and(nslices > 0 && !changed && reach <= M - DRANGE);
+  // Every value less than DRANGE below M is listed, as the passes work that distance out: a slice's own list that goes so far does (no value
+  // is nearer to M than to the slice's largest), a shorter one by a margin for the roundings. (M - DRANGE is M itself from 2^28 up.)
+  near.listed = __syncthreads_and(nslices > 0 && !changed && (range == DRANGE || M - m_thr + range >= DRANGE * 1.00001f));
   const float Z = block_sum(m_thr == -INFINITY ? 0.f : m_thr == M ? z : z * __expf(m_thr - M), sm.red);
   const float logZ = __logf(Z);
 

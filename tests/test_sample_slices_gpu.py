@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from nv_genai_amd import ops
+from nv_genai_amd.ops import reference as ref
 
 pytestmark = pytest.mark.gpu
 # temperature, top_k, top_p
@@ -86,3 +87,17 @@ def test_the_same_draw_again(gpu):
         first = ops.sample(x, *arg, 1000 * s + row, row)[0]
         for _ in range(6):
             assert torch.equal(ops.sample(x, *arg, 1000 * s + row, row)[0], first)
+
+
+def test_many_equal_largest_values(gpu):
+    """A slice of more largest values than it can list, where the largest value less the lists' distance of 16 rounds to itself. The two
+    seeds' noise is 16.6 for one of these values, which rounds up there, and so decides."""
+    V, temp = 32_000, torch.tensor(1e-6)
+    M = 400.0 * (1.0 / temp)
+    assert M - 16.0 == M and M + 16.6 > M
+    x = torch.randn(V)
+    x[4096:4296] = 400.0
+    x = x.expand(2, V).contiguous()
+    arg = (temp.expand(2).contiguous(), torch.zeros(2, dtype=torch.int32), torch.full((2,), 0.9), torch.tensor([33_800, 77_349]), torch.zeros(2, dtype=torch.long))
+    assert ref.sample(x, *arg)[0].tolist() == [4165, 4167]
+    assert ops.sample(x.to(gpu), *(a.to(gpu) for a in arg))[0].tolist() == [4165, 4167]
