@@ -24,8 +24,6 @@
 #include "common.h"
 #include "kernels.h"
 
-#include <algorithm>
-
 namespace nga {
 
 namespace {
@@ -562,30 +560,27 @@ __global__ void __launch_bounds__(NT) sample_kernel(
   }
 }
 
-// Slices of a row, 0: none: by its length alone, since the partition function adds up in another order with them, and a row's draw is not to
-// depend on the rows beside it. Their launch costs 3 us and up: short rows are through as soon. Both, us, without / with: at the temperature
-// 0.2 and top-p 0.7 that the servers use by default, and greedy, 1 row of 8,000 values (4 slices) 15.3 16.9, 5.4 8.0; 1 of 32,000 24.8 17.3,
-// 8.7 8.0; 1 of 128,256 53 19, 20.4 8.2; 64 of 128,256 60 29, 22.4 14.9; 256 of 128,256 87 58, 27.3 34.6. Lists that are of no use (normal
-// logits of deviation 3 at temperature 1, top-p 0.9): 1 of 32,000 38.4 39.6, 1 of 128,256 113 103, 64 of 128,256 120 120, 256 128 153.
-int sample_slices(int V) {
+// Slices of a row, 0: none. Their launch costs 3 us and up: short rows are through as soon, and many rows fill the chip by themselves. Both,
+// us, without / with: at the temperature 0.2 and top-p 0.7 that the servers use by default, and greedy, 1 row of 8,000 values (4 slices)
+// 15.3 16.9, 5.4 8.0; 1 of 32,000 24.8 17.3, 8.7 8.0; 1 of 128,256 53 19, 20.4 8.2; 64 of 128,256 60 29, 22.4 14.9; 256 of 128,256 87 58,
+// 27.3 34.6. Lists that are of no use (normal logits of deviation 3 at temperature 1, top-p 0.9): 1 of 32,000 38.4 39.6, 1 of 128,256 113
+// 103, 64 of 128,256 120 120, 256 128 153.
+int sample_slices(int B, int V) {
   const int n = (V + SLICE - 1) / SLICE;
-  return n < 12 || n > MAX_SLICES ? 0 : n;
+  return n < 12 || n > MAX_SLICES || (int64_t)B * n > 4096 ? 0 : n;
 }
-int64_t sample_scratch(int B, int V) { return (int64_t)B * sample_slices(V) * (sizeof(SampleSlice) + LISTED * sizeof(SampleEntry)); }
+int64_t sample_scratch(int B, int V) { return (int64_t)B * sample_slices(B, V) * (sizeof(SampleSlice) + LISTED * sizeof(SampleEntry)); }
 
 void launch_sample(float* logits, int B, int V, const float* temperature, const int32_t* top_k,
                    const float* top_p, const float* rep_penalty, const int32_t* history,
                    int hist_len, const int64_t* seeds, const int64_t* steps, void* scratch, int32_t* out_tok,
                    float* out_logprob, hipStream_t stream) {
   if (B == 0) return;
-  const int n = scratch ? sample_slices(V) : 0;
+  const int n = scratch ? sample_slices(B, V) : 0;
   SampleEntry* const list = static_cast<SampleEntry*>(scratch);
   SampleSlice* const slices = reinterpret_cast<SampleSlice*>(list + (int64_t)B * n * LISTED);
-  constexpr int ROWS = 65535;   // of a launch: rows are its second dimension
-  for (int b = 0; n > 0 && b < B; b += ROWS)
-    sample_slices_kernel<<<dim3(n, std::min(ROWS, B - b)), 256, 0, stream>>>(logits + (int64_t)b * V, V, temperature + b, top_k ? top_k + b : nullptr,
-                                                                            history && rep_penalty ? rep_penalty + b : nullptr,
-                                                                            slices + (int64_t)b * n, list + (int64_t)b * n * LISTED);
+  if (n > 0)
+    sample_slices_kernel<<<dim3(n, B), 256, 0, stream>>>(logits, V, temperature, top_k, history ? rep_penalty : nullptr, slices, list);
   sample_kernel<<<B, NT, 0, stream>>>(logits, V, temperature, top_k, top_p, rep_penalty, history,
                                       hist_len, seeds, steps, slices, list, n, out_tok, out_logprob);
 }
