@@ -15,7 +15,7 @@
 // Every pass over the row keeps eight 16-byte loads in flight per thread. Histogram weights are
 // 64-bit fixed point (2^-40 units of exp(v - M)) so the LDS atomics are ds_add_u64: LDS
 // ds_add_f32 measured ~8x slower on gfx950 (scripts/dev/lds_atomic_bench.hip).
-//   * rows of some thousand values first go through sample_slices_kernel, some 2,000 values a workgroup, which finds the largest value and
+//   * rows of 30,000 values and more, up to some dozens of them, first go through sample_slices_kernel, some 2,000 values a workgroup, which finds the largest value and
 //     the partition function's part of each slice and lists its values close to that maximum. One workgroup a row is bound by its
 //     own arithmetic: a pass over 128,256 values takes it 14 to 20 us. Where the lists reach far enough below the row's maximum (at the
 //     temperature of 0.2 that the servers use by default they do, with some 20 of 2,000 values) all passes of the fast path go over
@@ -560,14 +560,24 @@ __global__ void __launch_bounds__(NT) sample_kernel(
   }
 }
 
-// Slices of a row, 0: none. Their launch costs 3 us and up: short rows are through as soon, and many rows fill the chip by themselves. Both,
-// us, without / with: at the temperature 0.2 and top-p 0.7 that the servers use by default, and greedy, 1 row of 8,000 values (4 slices)
-// 15.3 16.9, 5.4 8.0; 1 of 32,000 24.8 17.3, 8.7 8.0; 1 of 128,256 53 19, 20.4 8.2; 64 of 128,256 60 29, 22.4 14.9; 256 of 128,256 87 58,
-// 27.3 34.6. Lists that are of no use (normal logits of deviation 3 at temperature 1, top-p 0.9): 1 of 32,000 38.4 39.6, 1 of 128,256 113
-// 103, 64 of 128,256 120 120, 256 128 153.
+// Slices of a row, 0: none. Their launch costs 3 us and up, and where the lists are of no use or too short the passes over the row come
+// besides: short rows are through as soon, and many rows fill the chip by themselves. The line is where that worst case costs nothing, but
+// for up to 4 rows of 16 to 23 slices, where it costs 1 to 4 % and the others gain 40. Both, us, without / with: (a) at temperature 0.2 and
+// top-p 0.7, the servers' defaults, (b) greedy, (c) normal logits of deviation 3 at temperature 1, top-p 0.9, where lists are of no use:
+//   rows x values    (a)          (b)          (c)             rows x values    (a)          (b)          (c)
+//    1 x  24,576  20.5  16.9    7.0   7.9   31.5  34.0          1 x 128,256  53.0  19.0   19.5   7.9    113   104
+//    1 x  32,000  24.1  17.2    8.0   7.9   37.9  39.4         16 x 128,256  54.0  20.4   20.1   9.0    114   107
+//   16 x  32,000  25.2  26.8    8.4   8.4   39.2  40.8         64 x 128,256  60.3  29.0   21.4  14.1    119   119
+//    8 x  49,152  30.3  17.7   10.5   8.4   52.7  52.3        128 x 128,256  66.9  39.0   22.7  21.0    123   131
+//   48 x  49,152  31.8  33.0   10.6   9.3   53.6  54.9         32 x 256,000  92.0  31.2   35.2  13.9    213   200
+//   32 x  65,536  34.6  19.3   12.2   8.9   64.3  63.5        128 x 256,000   107  59.8   37.6  32.3    219   232
+//   48 x 100,352  45.6  45.0   16.4  11.3   90.5  90.8
+// The partition function adds up in another order with slices than without: a row's log-probability, and with it the target of its top-p, can
+// differ in the last bit between a batch that is sliced and one that is not.
 int sample_slices(int B, int V) {
   const int n = (V + SLICE - 1) / SLICE;
-  return n < 12 || n > MAX_SLICES || (int64_t)B * n > 4096 ? 0 : n;
+  const int most = n < 16 || n > MAX_SLICES ? 0 : n < 24 ? 4 : n < 60 ? n : 4096 / n;   // rows
+  return B <= most ? n : 0;
 }
 int64_t sample_scratch(int B, int V) { return (int64_t)B * sample_slices(B, V) * (sizeof(SampleSlice) + LISTED * sizeof(SampleEntry)); }
 
