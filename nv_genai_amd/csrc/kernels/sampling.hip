@@ -15,9 +15,9 @@
 // Every pass over the row keeps eight 16-byte loads in flight per thread. Histogram weights are
 // 64-bit fixed point (2^-40 units of exp(v - M)) so the LDS atomics are ds_add_u64: LDS
 // ds_add_f32 measured ~8x slower on gfx950 (scripts/dev/lds_atomic_bench.hip).
-//   * rows of 30,000 values and more, up to some dozens of them, first go through sample_slices_kernel, some 2,000 values a workgroup, which finds the largest value and
-//     the partition function's part of each slice and lists its values close to that maximum. One workgroup a row is bound by its
-//     own arithmetic: a pass over 128,256 values takes it 14 to 20 us. Where the lists reach far enough below the row's maximum (at the
+//   * rows of 30,000 values and more, up to some dozens of them, first go through sample_slices_kernel, some 2,000 values a workgroup,
+//     which finds the largest value and the partition function's part of each slice and lists its values close to that maximum. One
+//     workgroup a row is bound by its own arithmetic: a pass over 128,256 values takes it 14 to 20 us. Where the lists reach far enough below the row's maximum (at the
 //     temperature of 0.2 that the servers use by default they do, with some 20 of 2,000 values) all passes of the fast path go over
 //     them, in registers, instead of the row. More in sample_slices.
 // Also returns the chosen token's log-probability under the temperature-scaled distribution.
@@ -503,6 +503,7 @@ __global__ void __launch_bounds__(NT) sample_kernel(
   }
   const float m_thr = am.v;
   am = block_argmax(am, sm.ared);
+  if (am.i == 0x7fffffff) am.i = 0;   // a row of NaN or -inf alone
   const float M = am.v;
   // Every value less than DRANGE below M is listed, as the passes work that distance out: a slice's own list that goes so far does (no value
   // is nearer to M than to the slice's largest), a shorter one by a margin for the roundings. (M - DRANGE is M itself from 2^28 up.)

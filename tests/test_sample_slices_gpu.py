@@ -104,3 +104,15 @@ def test_many_equal_largest_values(gpu):
     arg = (temp.expand(2).contiguous(), torch.zeros(2, dtype=torch.int32), torch.full((2,), 0.9), torch.tensor([33_800, 77_349]), torch.zeros(2, dtype=torch.long))
     assert ref.sample(x, *arg)[0].tolist() == [4165, 4167]
     assert ops.sample(x.to(gpu), *(a.to(gpu) for a in arg))[0].tolist() == [4165, 4167]
+
+
+@pytest.mark.parametrize("V", [1000, 128_256])
+@pytest.mark.parametrize("temp,k,p", [(0.0, 0, 1.0), (1.0, 0, 1.0), (0.2, 40, 0.9)])
+def test_rows_without_a_value(gpu, V, temp, k, p):
+    """A row of NaN or of -inf gives the first token: there is none that it could draw."""
+    x = torch.full((3, V), float("nan"), device=gpu)
+    x[1] = float("-inf")
+    x[2] = torch.arange(V, device=gpu) / V
+    arg = (torch.full((3,), temp, device=gpu), torch.full((3,), k, dtype=torch.int32, device=gpu), torch.full((3,), p, device=gpu))
+    tok, _ = ops.sample(x, *arg, torch.arange(3, device=gpu), torch.arange(3, device=gpu))
+    assert tok[:2].tolist() == [0, 0] and 0 <= int(tok[2]) < V
