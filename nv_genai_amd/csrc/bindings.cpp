@@ -694,25 +694,20 @@ void decode_step(Tensor out, Tensor qkv, Tensor pos, Tensor cos_sin, Tensor slot
                           nparts > 1 ? part_o.data_ptr<float>() : nullptr, (int)window, cur_stream(qkv));
 }
 
-// Work-list prefill (32x32 kernel): q / out rows are absolute token rows of the step (the
-// cu_q offsets of ALL its sequences); items [n, 2] int32 (sequence, row block) pairs, n_items
-// a 1-element device int32 (read by the kernel, so a captured graph replays any step's list)
 // rows that LDS-DMA can read, 16 bytes at 16-byte addresses (strides are checked): others are copied once
 Tensor dma_rows(const Tensor& t, int64_t cols) {
   return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.narrow(1, 0, cols).clone(at::MemoryFormat::Contiguous);
 }
 
-// rows that 16-byte stores can write: others through a copy, in which rows that the kernel does not write are theirs
-struct RowsOut {
-  Tensor out, rows;
-  RowsOut(const Tensor& t, int64_t cols) : out(t.narrow(1, 0, cols)), rows(t) {
-    if (reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 || t.stride(0) % 8) rows = out.clone(at::MemoryFormat::Contiguous);
-  }
-  void done() const {
-    if (rows.data_ptr() != out.data_ptr()) out.copy_(rows);
-  }
-};
+void prefill_out(nga::PrefillParams& p, const Tensor& out) {
+  p.out = bfp(out);
+  p.out_stride = out.stride(0);
+  p.out_wide = reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0 && out.stride(0) % 8 == 0;
+}
 
+// Work-list prefill (32x32 kernel): q / out rows are absolute token rows of the step (the
+// cu_q offsets of ALL its sequences); items [n, 2] int32 (sequence, row block) pairs, n_items
+// a 1-element device int32 (read by the kernel, so a captured graph replays any step's list)
 void prefill_attention_worklist(Tensor out, Tensor q, Tensor kc, Tensor vc, Tensor block_tables,
                                 Tensor cu_q, Tensor ctx_lens, int64_t Hq, int64_t Hkv, double scale,
                                 bool causal, int64_t window, Tensor items, Tensor n_items, int64_t grid,
@@ -744,8 +739,7 @@ void prefill_attention_worklist(Tensor out, Tensor q, Tensor kc, Tensor vc, Tens
   TORCH_CHECK(window >= 0 && (window == 0 || causal));
   TORCH_CHECK(grid >= 1 && grid <= 65535 && (ks == 1 || ks == 2), "prefill_attention_worklist: grid / ks");
   nga::PrefillParams p{};
-  p.out = bfp(out);
-  p.out_stride = out.stride(0);
+  prefill_out(p, out);
   p.q = bfp(q);
   p.q_stride = q.stride(0);
   p.cu_q = cu_q.data_ptr<int32_t>();
@@ -766,15 +760,11 @@ void prefill_attention_worklist(Tensor out, Tensor q, Tensor kc, Tensor vc, Tens
   }
   p.items = items.data_ptr<int32_t>();
   p.n_items = n_items.data_ptr<int32_t>();
-  const Tensor qr = dma_rows(q, Hq * D);
-  const RowsOut o(out, Hq * D);
+  const Tensor qr = impl == 2 ? dma_rows(q, Hq * D) : q;
   p.q = bfp(qr);
   p.q_stride = qr.stride(0);
-  p.out = bfp(o.rows);
-  p.out_stride = o.rows.stride(0);
   if (impl == 2) nga::launch_prefill_attention_v2_worklist(p, (int)grid, (int)ks, causal, cur_stream(q));
   else nga::launch_prefill_attention_v1_worklist(p, (int)grid, (int)D, causal, cur_stream(q));
-  o.done();
 }
 
 void prefill_attention(Tensor out, Tensor q, c10::optional<Tensor> k, c10::optional<Tensor> v,
@@ -796,8 +786,7 @@ void prefill_attention(Tensor out, Tensor q, c10::optional<Tensor> k, c10::optio
   TORCH_CHECK(out.dim() == 2 && out.stride(1) == 1 && out.size(1) >= Hq * D && out.size(0) == q.size(0));
   const int64_t B = cu_q.numel() - 1;
   nga::PrefillParams p{};
-  p.out = bfp(out);
-  p.out_stride = out.stride(0);
+  prefill_out(p, out);
   p.q = bfp(q);
   p.q_stride = q.stride(0);
   p.cu_q = cu_q.data_ptr<int32_t>();
@@ -845,22 +834,14 @@ void prefill_attention(Tensor out, Tensor q, c10::optional<Tensor> k, c10::optio
     p.k = bfp(kr);
     p.v = bfp(vr);
     p.kv_stride = kr.stride(0);
-    const RowsOut o(out, Hq * D);
-    p.out = bfp(o.rows);
-    p.out_stride = o.rows.stride(0);
     nga::launch_varlen_attention(p, (int)B, (int)max_q_len, (int)D, causal, cur_stream(q));
-    o.done();
     return;
   }
   p.impl = (int)impl;
-  const Tensor qr = dma_rows(q, Hq * D);
-  const RowsOut o(out, Hq * D);
+  const Tensor qr = D == 128 && impl != 1 && !p.kv_fp8 ? dma_rows(q, Hq * D) : q;   // what the 32x32 kernel can take
   p.q = bfp(qr);
   p.q_stride = qr.stride(0);
-  p.out = bfp(o.rows);
-  p.out_stride = o.rows.stride(0);
   nga::launch_prefill_attention(p, (int)B, (int)max_q_len, (int)D, causal, cur_stream(q));
-  o.done();
 }
 
 // ------------------------------------------------------------------ attention with gradients (packed rows)

@@ -82,3 +82,32 @@ def test_paged_rows(gpu, hq, hkv, lens, ctxs):
         assert torch.equal(run(wide, room[:T, by:by + hq * D]), got)
         room[:T, by:by + hq * D] = 7.0
         assert (room == 7.0).all()
+
+
+@pytest.mark.parametrize("by", [0, 8, 3])
+def test_out_is_written_in_place(gpu, by):
+    """Rows that no item covers are another kernel's, which may write them at the same time: no copy of the output is made, wherever it lies."""
+    from nv_genai_amd import ops
+
+    D, hq, hkv, lens = 128, 4, 2, [70, 33]
+    T, w = sum(lens), hq * D
+    g = torch.Generator("cuda").manual_seed(by)
+    rn = lambda *s: torch.randn(*s, device=gpu, generator=g).to(BF)  # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=gpu)  # noqa: E731
+    q, k, v, kc, vc = rn(T, w), rn(T, hkv * D), rn(T, hkv * D), rn(3, hkv, 64, D), rn(3, hkv, D, 64)
+    cu, cl, bt = i32([0, 70, T]), i32(lens), i32([[0, 1], [2, 0]])
+    items, n = i32([[0, 0], [0, 1]]), i32([2])   # the first sequence alone
+    room = torch.full((T, w + 16 + by), 7.0, dtype=BF, device=gpu)
+    out, C = room[:, by:by + w], ops.kernels()
+    calls = {2: lambda: C.prefill_attention_worklist(out, q, kc, vc, bt, cu, cl, hq, hkv, D ** -0.5, True, 0, items, n, 3, 1, 2, 1.0, 1.0),
+             1: lambda: C.prefill_attention_worklist(out, q, kc, vc, bt, cu, cl, hq, hkv, D ** -0.5, True, 0, items, n, 3, 1, 1, 1.0, 1.0),
+             "pages": lambda: C.prefill_attention(out, q, None, None, kc, vc, bt, cu, cl, hq, hkv, D, 70, D ** -0.5, True, 0, 2, 1.0, 1.0),
+             "packed": lambda: C.prefill_attention(out, q, k, v, None, None, None, cu, None, hq, hkv, D, 70, D ** -0.5, True, 0, 0, 1.0, 1.0)}
+    for name, call in calls.items():
+        room.fill_(7.0)
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        call()
+        assert torch.cuda.memory_stats()["allocation.all.allocated"] == before, name
+        if name in (1, 2):
+            assert bool((out[70:] == 7).all()) and not bool((out[:70] == 7).all())
+        assert bool((room[:, :by] == 7).all()) and bool((room[:, by + w:] == 7).all())
