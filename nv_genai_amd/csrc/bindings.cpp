@@ -861,12 +861,14 @@ void train_attention_backward(Tensor dq, Tensor dk, Tensor dv, Tensor dout, Tens
   for (const Tensor& t : {q, out, dout, dq}) train_attn_check(t, T, Hq * D);
   for (const Tensor& t : {k, v, dk, dv}) train_attn_check(t, T, Hkv * D);
   TORCH_CHECK(k.stride(0) == v.stride(0) && dk.stride(0) == dv.stride(0), "attention: k and v rows at one stride");
-  for (const Tensor& t : {q, k, dout}) TORCH_CHECK(t.stride(0) < (1 << 25), "attention: a tile's rows within 32 bits");
   CHECK_F32(lse);
   TORCH_CHECK(lse.numel() == Hq * T && scale > 0 && (lse.dim() != 3 || (lse.size(0) == B && lse.size(1) == Hq)),
               "attention: lse [Hq, T] or [B, Hq, S]");
   CHECK_I32(cu);
   if (B < 1 || T == 0 || max_len <= 0) return;
+  // the kernels address a tile's rows within 32 bits: rows further apart are copied once
+  const auto near = [](const Tensor& t) { return t.stride(0) < (1 << 25) ? t : t.clone(at::MemoryFormat::Contiguous); };
+  q = near(q); k = near(k); v = near(v); dout = near(dout);
   Tensor delta = at::empty({Hq, T}, lse.options()), l2 = lse.dim() == 3 ? at::empty_like(delta) : lse, part;
   nga::AttnBwdParams p{};
   p.parts = nga::attn_bwd_parts((int)B, (int)max_len, (int)Hq, (int)Hkv);

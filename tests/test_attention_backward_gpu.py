@@ -68,3 +68,25 @@ def test_log_sums_by_sequence(gpu, B, S, D, hq, hkv):
         ops.kernels().train_attention_backward(*d.split(w, 1), do, *qkv.split(w, 1), out, how, cu, hq, hkv, D, S, D ** -0.5)
         got.append(d)
     assert torch.equal(*got)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_rows_far_apart(gpu, D):
+    """Rows 2^25 values apart, beyond a tile's 32-bit addresses, give the bits of rows one behind the other."""
+    from nv_genai_amd import ops
+
+    T, step = 3, 1 << 25
+    g = torch.Generator("cuda").manual_seed(D)
+    rn = lambda *s: torch.randn(*s, device=gpu, generator=g)  # noqa: E731
+    near = [rn(T, D).to(BF) for _ in range(4)]   # q, k, v, dout
+    out, lse = rn(T, D).to(BF), 30 + rn(1, T)
+    cu = torch.tensor([0, T], dtype=torch.int32, device=gpu)
+    room = torch.empty((T - 1) * step + 4 * D, dtype=BF, device=gpu)
+    far = [torch.as_strided(room, (T, D), (step, 1), i * D).copy_(t) for i, t in enumerate(near)]
+    got = []
+    for max_len in (64, 65):
+        for q, k, v, do in (near, far):
+            d = torch.empty(T, 3 * D, dtype=BF, device=gpu)
+            ops.kernels().train_attention_backward(*d.split(D, 1), do, q, k, v, out, lse, cu, 1, 1, D, max_len, D ** -0.5)
+            got.append(d)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[2], got[3])
