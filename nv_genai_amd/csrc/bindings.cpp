@@ -853,7 +853,8 @@ void train_attn_check(const Tensor& t, int64_t T, int64_t cols) {
 }
 
 // gradients of causal attention of q [T, Hq D], k and v [T, Hkv D] over the sequences of cu, the longest of max_len; out [T, Hq D];
-// lse [Hq, T]: log2 of each row's sum of exponentials, or [B, Hq, S]: their natural logarithms, for B sequences of S tokens each
+// lse [Hq, T]: log2 of each row's sum of exponentials, or [B, Hq, S]: their natural logarithms, for B sequences of S tokens each (none is
+// longer than max_len = S, and they have B S tokens)
 void train_attention_backward(Tensor dq, Tensor dk, Tensor dv, Tensor dout, Tensor q, Tensor k, Tensor v, Tensor out, Tensor lse,
                               Tensor cu, int64_t Hq, int64_t Hkv, int64_t D, int64_t max_len, double scale) {
   const int64_t T = q.size(0), B = cu.numel() - 1;
@@ -862,8 +863,8 @@ void train_attention_backward(Tensor dq, Tensor dk, Tensor dv, Tensor dout, Tens
   for (const Tensor& t : {k, v, dk, dv}) train_attn_check(t, T, Hkv * D);
   TORCH_CHECK(k.stride(0) == v.stride(0) && dk.stride(0) == dv.stride(0), "attention: k and v rows at one stride");
   CHECK_F32(lse);
-  TORCH_CHECK(lse.numel() == Hq * T && scale > 0 && (lse.dim() != 3 || (lse.size(0) == B && lse.size(1) == Hq)),
-              "attention: lse [Hq, T] or [B, Hq, S]");
+  TORCH_CHECK(lse.numel() == Hq * T && scale > 0 && (lse.dim() != 3 || (lse.size(0) == B && lse.size(1) == Hq && lse.size(2) == max_len)),
+              "attention: lse [Hq, T], or [B, Hq, S] of sequences of S tokens each");
   CHECK_I32(cu);
   if (B < 1 || T == 0 || max_len <= 0) return;
   // the kernels address a tile's rows within 32 bits: rows further apart are copied once

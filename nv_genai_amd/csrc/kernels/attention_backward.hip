@@ -130,8 +130,8 @@ __device__ __forceinline__ float ab_lse(const AttnBwdParams& P, uint32_t t, int 
   return P.lse_in[((int64_t)(t / S) * P.Hq + hq) * S + t % S] * AB_LOG2E;
 }
 
-// delta[hq][t] = sum_d dO O; 8 dims a lane; with two waves for 32 rows the dq kernel works them out. Log-sums as torch's attention leaves them, natural and by sequence, become lse beside
-// it (single operations: 9.6 us a call at 2 x 512 tokens, 32 heads)
+// delta[hq][t] = sum_d dO O; 8 dims a lane. Where two waves share 32 rows the dq kernel works it out instead. Log-sums as torch's attention
+// leaves them, natural and by sequence, become lse beside it (single operations: 9.6 us a call at 2 x 512 tokens, 32 heads).
 template <int D>
 __global__ void __launch_bounds__(256) attn_delta_kernel(AttnBwdParams P) {
   constexpr int LPR = D / 8;

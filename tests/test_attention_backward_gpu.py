@@ -90,3 +90,14 @@ def test_rows_far_apart(gpu, D):
             ops.kernels().train_attention_backward(*d.split(D, 1), do, q, k, v, out, lse, cu, 1, 1, D, max_len, D ** -0.5)
             got.append(d)
     assert torch.equal(got[0], got[1]) and torch.equal(got[2], got[3])
+
+
+def test_log_sums_by_sequence_are_of_one_length(gpu):
+    from nv_genai_amd import ops
+
+    T, D = 8, 64
+    t = [torch.zeros(T, D, dtype=BF, device=gpu) for _ in range(8)]
+    lse = torch.zeros(2, 1, 4, device=gpu)   # two sequences of 4 tokens; these are of 3 and 5
+    cu = torch.tensor([0, 3, 8], dtype=torch.int32, device=gpu)
+    with pytest.raises(RuntimeError, match="S tokens each"):
+        ops.kernels().train_attention_backward(*t, lse, cu, 1, 1, D, 5, D ** -0.5)
