@@ -252,6 +252,13 @@ def gemm_kn_covers(M: int, N: int, K: int) -> bool:
             and (K >= 16384 and M <= 2048 and N <= 8192 or M <= 128 and N <= 4096 and K >= 4096))
 
 
+def lora_grads_covers(T: int, N: int, K: int, r: int) -> bool:
+    """Whether lora.hip takes the gradients of an adapter of rank r beside a [N, K] weight, of T rows: what its 16-byte loads, its
+    fragments and its 32-bit counts of tiles take. All such sizes measured are faster than single operations, as lora.hip says."""
+    return (8 <= r <= 64 and r % 8 == 0 and N >= 8 and N % 8 == 0 and K >= 8 and K % 8 == 0
+            and T >= 1 and max(T, N, K) < 1 << 24)
+
+
 def weight_grad_covers(T: int, N: int, K: int) -> bool:
     """Whether dy [T, N]^T . x [T, K], the gradient of a weight, is faster through gemm_kn.hip than the library's product, whose tiles do
     not fill the chip and which does not split T enough. us, library / here, T 4,096 / 5,000 / 10,240: 3,072 x 1,024 45 56 96, 43 48 69;

@@ -392,7 +392,7 @@ class _LoraLinear(Function):
             return dx, None, None, None, da, db, None
         dy2 = dy.reshape(-1, dy.shape[-1])
         need = ctx.needs_input_grad
-        if (bb.shape[1] <= 64 and all(n % 8 == 0 for n in (*bb.shape, x.shape[-1]))   # lora.hip; single operations under vmap too
+        if (ops.lora_grads_covers(dy2.shape[0], bb.shape[0], x.shape[-1], bb.shape[1])   # lora.hip; single operations under vmap too
                 and _takes(dy) and not torch._C._functorch.is_legacy_batchedtensor(dy)):
             dy2 = _rows(dy2)
             dx = _input_grad(dy2, w) if need[0] else None

@@ -50,3 +50,21 @@ def test_batched_gradients_take_single_operations(gpu):
     for i in range(3):
         for p, q in zip(many, torch.autograd.grad(y, (x, a, b), dy[i], retain_graph=True)):
             assert torch.allclose(p[i].float(), q.float(), rtol=2.0 ** -6, atol=2.0 ** -6 * q.float().abs().max().item())
+
+
+@pytest.mark.parametrize("T,N,K,r", [(2, 16, 24, 0), (1 << 24, 8, 8, 8)])
+def test_sizes_that_it_leaves_to_single_operations(gpu, T, N, K, r):
+    """No rank at all, and more rows than its kernels count."""
+    from nv_genai_amd import ops
+    from nv_genai_amd.training import fused
+
+    assert not ops.lora_grads_covers(T, N, K, r)
+    rn = lambda *s: torch.randn(*s, device=gpu, dtype=BF)  # noqa: E731
+    x, w, a, b = rn(T, K).requires_grad_(), rn(N, K), rn(r, K).float().requires_grad_(), rn(N, r).float().requires_grad_()
+    y = fused.lora_linear(x, w, a, b, 0.5)
+    y.backward(torch.ones_like(y))
+    assert a.grad.shape == a.shape and b.grad.shape == b.shape
+    want = w.double().sum(0) + 0.5 * (b.detach().to(BF).double().sum(0) @ a.detach().to(BF).double())
+    # every row's is the same: sums of N and r terms, rounded to bf16 once or twice of magnitudes up to their own sums
+    size = w.double().abs().sum(0) + 0.5 * (b.detach().double().abs().sum(0) @ a.detach().double().abs())
+    assert ((x.grad[::max(1, T // 100)].double() - want).abs() <= 2.0 ** -6 * size).all()
