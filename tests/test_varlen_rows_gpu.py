@@ -43,14 +43,9 @@ def test_rows(gpu, D, hq, hkv, lens, causal):
         assert (room == 7.0).all()
 
 
-# one group of waves and two (few row blocks), one to four heads a workgroup; chunks of prompts, whose keys lie before them
-@pytest.mark.parametrize("hq,hkv", [(8, 2), (4, 2), (2, 2)])
-@pytest.mark.parametrize("lens,ctxs", [([1], [1]), ([31, 64, 33], [31, 70, 200]), ([200, 129], [200, 400]), ([700] * 12, [700] * 12)])
-def test_paged_rows(gpu, hq, hkv, lens, ctxs):
-    from nv_genai_amd import ops
-
+def _pages(gpu, lens, ctxs, hq, hkv, seed):
     D, T, B = 128, sum(lens), len(lens)
-    g = torch.Generator("cuda").manual_seed(T + hq)
+    g = torch.Generator("cuda").manual_seed(seed)
     rn = lambda *s: torch.randn(*s, device=gpu, generator=g).to(BF)  # noqa: E731
     pages = [(c + 63) // 64 for c in ctxs]
     q, kc, vc = rn(T, hq * D), rn(sum(pages), hkv, 64, D), rn(sum(pages), hkv, D, 64)
@@ -58,10 +53,28 @@ def test_paged_rows(gpu, hq, hkv, lens, ctxs):
     for i, n in enumerate(pages):
         bt[i, :n] = torch.arange(n) + sum(pages[:i])
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=gpu)  # noqa: E731
-    cu, cl, bt = i32([0, *torch.tensor(lens).cumsum(0).tolist()]), i32(ctxs), bt.to(gpu)
+    return pages, q, kc, vc, bt.to(gpu), i32([0, *torch.tensor(lens).cumsum(0).tolist()]), i32(ctxs)
+
+
+# one group of waves and two by size, the old kernel among them (impl 0), and each by name (2 and 3); the same by a list of items, more
+# than there are workgroups, so that one takes several in turn; one to four heads a workgroup; chunks of prompts, whose keys lie before them
+@pytest.mark.parametrize("how", [0, 2, 3, "items 1", "items 2"])
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (4, 2), (2, 2)])
+@pytest.mark.parametrize("lens,ctxs", [([1], [1]), ([31, 64, 33], [31, 70, 200]), ([200, 129], [200, 400]), ([700] * 12, [700] * 12)])
+def test_paged_rows(gpu, hq, hkv, lens, ctxs, how):
+    from nv_genai_amd import ops
+
+    D, T, B = 128, sum(lens), len(lens)
+    pages, q, kc, vc, bt, cu, cl = _pages(gpu, lens, ctxs, hq, hkv, T + hq)
+    items = torch.from_numpy(ops.plan_prefill_items(cu.tolist(), ctxs, 0, B, hq, hkv)).to(gpu)
+    n_items = torch.tensor([len(items)], dtype=torch.int32, device=gpu)
 
     def run(q, out):
-        ops.kernels().prefill_attention(out, q, None, None, kc, vc, bt, cu, cl, hq, hkv, D, max(lens), D ** -0.5, True, 0, 0, 1.0, 1.0)
+        if isinstance(how, int):
+            ops.kernels().prefill_attention(out, q, None, None, kc, vc, bt, cu, cl, hq, hkv, D, max(lens), D ** -0.5, True, 0, how, 1.0, 1.0)
+        else:
+            ops.kernels().prefill_attention_worklist(out, q, kc, vc, bt, cu, cl, hq, hkv, D ** -0.5, True, 0, items, n_items, 3, int(how[-1]), 2,
+                                                     1.0, 1.0)
         return out
 
     got = run(q, torch.empty(T, hq * D, dtype=BF, device=gpu))
@@ -91,11 +104,9 @@ def test_out_is_written_in_place(gpu, by):
 
     D, hq, hkv, lens = 128, 4, 2, [70, 33]
     T, w = sum(lens), hq * D
-    g = torch.Generator("cuda").manual_seed(by)
-    rn = lambda *s: torch.randn(*s, device=gpu, generator=g).to(BF)  # noqa: E731
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=gpu)  # noqa: E731
-    q, k, v, kc, vc = rn(T, w), rn(T, hkv * D), rn(T, hkv * D), rn(3, hkv, 64, D), rn(3, hkv, D, 64)
-    cu, cl, bt = i32([0, 70, T]), i32(lens), i32([[0, 1], [2, 0]])
+    _, q, kc, vc, bt, cu, cl = _pages(gpu, lens, lens, hq, hkv, by)
+    k, v = (torch.randn(T, hkv * D, device=gpu).to(BF) for _ in range(2))
     items, n = i32([[0, 0], [0, 1]]), i32([2])   # the first sequence alone
     room = torch.full((T, w + 16 + by), 7.0, dtype=BF, device=gpu)
     out, C = room[:, by:by + w], ops.kernels()
