@@ -699,12 +699,6 @@ Tensor dma_rows(const Tensor& t, int64_t cols) {
   return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.narrow(1, 0, cols).clone(at::MemoryFormat::Contiguous);
 }
 
-void prefill_out(nga::PrefillParams& p, const Tensor& out) {
-  p.out = bfp(out);
-  p.out_stride = out.stride(0);
-  p.out_wide = reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0 && out.stride(0) % 8 == 0;
-}
-
 // Work-list prefill (32x32 kernel): q / out rows are absolute token rows of the step (the
 // cu_q offsets of ALL its sequences); items [n, 2] int32 (sequence, row block) pairs, n_items
 // a 1-element device int32 (read by the kernel, so a captured graph replays any step's list)
@@ -739,7 +733,8 @@ void prefill_attention_worklist(Tensor out, Tensor q, Tensor kc, Tensor vc, Tens
   TORCH_CHECK(window >= 0 && (window == 0 || causal));
   TORCH_CHECK(grid >= 1 && grid <= 65535 && (ks == 1 || ks == 2), "prefill_attention_worklist: grid / ks");
   nga::PrefillParams p{};
-  prefill_out(p, out);
+  p.out = bfp(out);
+  p.out_stride = out.stride(0);
   p.q = bfp(q);
   p.q_stride = q.stride(0);
   p.cu_q = cu_q.data_ptr<int32_t>();
@@ -786,7 +781,8 @@ void prefill_attention(Tensor out, Tensor q, c10::optional<Tensor> k, c10::optio
   TORCH_CHECK(out.dim() == 2 && out.stride(1) == 1 && out.size(1) >= Hq * D && out.size(0) == q.size(0));
   const int64_t B = cu_q.numel() - 1;
   nga::PrefillParams p{};
-  prefill_out(p, out);
+  p.out = bfp(out);
+  p.out_stride = out.stride(0);
   p.q = bfp(q);
   p.q_stride = q.stride(0);
   p.cu_q = cu_q.data_ptr<int32_t>();

@@ -382,7 +382,7 @@ __device__ __forceinline__ void v2_row_block(const PrefillParams& P, uint16_t* s
   for (int i = 0; i < 8; ++i) {
     const int r = 4 * i + (lane >> 4);
     const u16x8 v = *reinterpret_cast<const u16x8*>(rows + r * D + (((lane & 15) ^ (r & 15)) << 3));
-    if (row0 + r < qlen) store8_any(P.out + (int64_t)(q0 + row0 + r) * P.out_stride + (int64_t)hq * D + (lane & 15) * 8, v, P.out_wide);
+    if (row0 + r < qlen) store8_any(P.out + (int64_t)(q0 + row0 + r) * P.out_stride + (int64_t)hq * D + (lane & 15) * 8, v);
   }
 }
 

@@ -233,7 +233,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) varlen_attn_kernel(Pref
   for (int i = 0; i < NR; ++i) {
     const int p = i * 64 + lane, r = p / NC;
     const u16x8 v = *reinterpret_cast<const u16x8*>(rows + r * D + (((p % NC) ^ (r % NC)) << 3));
-    if (row0 + r < qlen) store8_any(op + r * P.out_stride + (p % NC) * 8, v, P.out_wide);
+    if (row0 + r < qlen) store8_any(op + r * P.out_stride + (p % NC) * 8, v);
   }
 }
 

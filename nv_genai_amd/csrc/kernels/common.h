@@ -40,15 +40,8 @@ __device__ __forceinline__ void store8(uint16_t* p, u16x8 v) {
   *reinterpret_cast<u16x8*>(p) = v;
 }
 
-// the same at any address (wide: at one of 16 bytes)
-__device__ __forceinline__ void store8_any(uint16_t* p, u16x8 v, bool wide) {
-  if (wide) {
-    store8(p, v);
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) p[i] = v[i];
-}
+// the same at any address, also in one instruction: the target's code runs with unaligned access
+__device__ __forceinline__ void store8_any(uint16_t* p, u16x8 v) { __builtin_memcpy(p, &v, 16); }
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u16x8 v) {
   return __builtin_bit_cast(bf16x8, v);

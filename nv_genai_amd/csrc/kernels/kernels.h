@@ -87,7 +87,6 @@ void launch_decode_step(uint16_t* out, int64_t out_stride, const uint16_t* qkv, 
 struct PrefillParams {
   uint16_t* out;
   int64_t out_stride;
-  bool out_wide;    // every row of out is at a 16-byte address (read by the 32x32 kernels)
   const uint16_t* q;
   int64_t q_stride;
   const uint16_t* k;  // non-paged K rows (packed like q)
