@@ -1394,11 +1394,17 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
   const auto opt = word.options();
   Tensor x = at::empty({T, H}, opt);
   if (T == 0) return x;
+  const bool rows = T <= 32, tiles = !rows && T <= encoder_tile_rows(H);
+  // up to 32 rows lie a second time as the products read them; those between up and down, and a single query's q/k/v, in that form alone
+  const int64_t tiles16 = (T + 15) / 16 * 16;
+  Tensor xp;
+  if (rows) xp = at::empty({tiles16, H}, opt);
+  uint16_t* const packed = rows ? bfp(xp) : nullptr;
   nga::launch_embed_layernorm(ids.data_ptr<int32_t>(), pos.data_ptr<int32_t>(), types.has_value() ? types->data_ptr<int32_t>() : nullptr,
                               bfp(word), (int)word.size(0), bfp(ptab), (int)ptab.size(0), bfp(ttab), (int)ttab.size(0),
-                              bfp(emb_g), bfp(emb_b), (float)eps, T, (int)H, bfp(x), st);
-  Tensor qkv = at::empty({T, 3 * H}, opt), a = at::empty({T, H}, opt), y = at::empty({T, H}, opt), h = at::empty({T, F}, opt);
-  const bool rows = T <= 32, tiles = !rows && T <= encoder_tile_rows(H);
+                              bfp(emb_g), bfp(emb_b), (float)eps, T, (int)H, bfp(x), packed, st);
+  Tensor qkv = at::empty({rows ? tiles16 : T, 3 * H}, opt), a = at::empty({T, H}, opt), y = at::empty({T, H}, opt);
+  Tensor h = at::empty({rows ? tiles16 : T, F}, opt);
   Tensor slabs;
   const bool one = rows && B == 1 && max_len >= T;   // a single query; where several lie is known on the GPU alone
   const int att_split = one ? nga::row_attn_split((int)heads) : 0;
@@ -1407,7 +1413,7 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
   auto project = [&](const Tensor& in, const Tensor& w, const Tensor& bias, Tensor& out, bool gelu) {
     const int64_t N = w.size(0), K = w.size(1);
     if (rows) {
-      nga::launch_row_gemm({bfp(in), K, bfp(w), bfp(bias), out.data_ptr(), N, (int)T, (int)N, (int)K, 1}, gelu ? 2 : 0, st);
+      nga::launch_row_gemm({packed, 0, bfp(w), bfp(bias), out.data_ptr(), N, (int)T, (int)N, (int)K, 1, nullptr, 0.f, one}, gelu ? 2 : 0, st);
     } else if (tiles) {
       nga::SkinnyGemmParams p{};
       p.x = bfp(in); p.ldx = K; p.w = bfp(w); p.M = (int)T; p.N = (int)N; p.K = (int)K;
@@ -1422,13 +1428,13 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
       at::addmm_out(out, bias, in, w.t());
     }
   };
-  // out = LN(in w^T + bias + resid)
-  auto project_norm = [&](const Tensor& in, const Tensor& w, const Tensor& bias, const Tensor& resid, const Tensor& g,
+  // out = LN(in w^T + bias + resid); in_stride: 0 where up to 32 rows of it are packed
+  auto project_norm = [&](const Tensor& in, int64_t in_stride, const Tensor& w, const Tensor& bias, const Tensor& resid, const Tensor& g,
                           const Tensor& b, Tensor& out) {
     const int64_t K = w.size(1);
     const int split = encoder_split(T, H, K);
     if (rows) {
-      nga::launch_row_gemm({bfp(in), K, bfp(w), nullptr, slabs.data_ptr(), H, (int)T, (int)H, (int)K, split}, 1, st);
+      nga::launch_row_gemm({bfp(in), in_stride, bfp(w), nullptr, slabs.data_ptr(), H, (int)T, (int)H, (int)K, split}, 1, st);
     } else if (tiles) {
       nga::SkinnyGemmParams p{};
       p.x = bfp(in); p.ldx = K; p.w = bfp(w); p.M = (int)T; p.N = (int)H; p.K = (int)K; p.split = split;
@@ -1440,7 +1446,7 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
       return;
     }
     nga::launch_splitk_layernorm(slabs.data_ptr<float>(), split, (int)T, bfp(bias), bfp(resid), bfp(g), bfp(b), (float)eps, (int)H,
-                                 bfp(out), st);
+                                 bfp(out), packed, st);
   };
   nga::PrefillParams p{};
   p.out = bfp(a);
@@ -1455,16 +1461,16 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
   for (size_t i = 0; i < L.size(); i += 12) {
     project(x, L[i], L[i + 1], qkv, false);
     if (one) {
-      nga::launch_row_attn_gemm({bfp(qkv), 3 * H, bfp(L[i + 2]), nullptr, slabs.data_ptr(), H, (int)T, (int)H, (int)H, att_split,
+      nga::launch_row_attn_gemm({bfp(qkv), 0, bfp(L[i + 2]), nullptr, slabs.data_ptr(), H, (int)T, (int)H, (int)H, att_split,
                                  p.cu_q, p.scale}, (int)D, st);
       nga::launch_splitk_layernorm(slabs.data_ptr<float>(), att_split, (int)T, bfp(L[i + 3]), bfp(x), bfp(L[i + 4]), bfp(L[i + 5]),
-                                   (float)eps, (int)H, bfp(x), st);
+                                   (float)eps, (int)H, bfp(x), packed, st);
     } else {
       if (B > 0 && max_len > 0) nga::launch_varlen_attention(p, (int)B, (int)max_len, (int)D, false, st);
-      project_norm(a, L[i + 2], L[i + 3], x, L[i + 4], L[i + 5], x);
+      project_norm(a, H, L[i + 2], L[i + 3], x, L[i + 4], L[i + 5], x);
     }
     project(x, L[i + 6], L[i + 7], h, true);
-    project_norm(h, L[i + 8], L[i + 9], x, L[i + 10], L[i + 11], x);
+    project_norm(h, 0, L[i + 8], L[i + 9], x, L[i + 10], L[i + 11], x);
   }
   post_launch("encoder_forward");
   return x;

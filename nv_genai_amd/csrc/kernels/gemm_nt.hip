@@ -10,6 +10,7 @@
 // with other features or K); the launch of bias and GELU that it saves is what it gains. Both, us, library / here, at 2,048 / 3,072 /
 // 4,096 / 8,192 / 19,264 rows: K 1,024, 4,096 features 34.6 45.0 50.0 94.0 238, 37.9 40.0 43.5 80.0 190; K 768, 3,072 features 27.8 39.6
 // 40.1 74.7 145, 30.7 31.5 33.6 63.0 125.
+#include "gelu.h"
 #include "gemm_tile.h"
 #include "kernels.h"
 
@@ -17,27 +18,6 @@ namespace nga {
 
 namespace {
 constexpr int NT_T = 256, NT_K = 32, NT_STAGE = 2 * NT_T * NT_K, NT_NST = 4, NT_GM = 8;
-
-// x Phi(x). Phi(-|x|) = 2^(-x^2 / (2 ln 2) + R(|x|)): R, the logarithm of a scaled erfc, is smooth, here its minimax polynomial on
-// [0, 7.5], weighted by what an error of it does to the result (beyond, its value at 7.5). No branches, as erff's would take the kernel
-// from 190 to 274 us at 19,264 x 4,096 of K 1,024. By itself in fp32, largest error against 64 bits, with erff / so: x in [-6, -5] 8.3e-8
-// / 1.8e-10, [-4, -3] 6.0e-8 / 5.9e-9, [-2, -1] 4.7e-8 / 5.5e-8, [-1, 0] 3.5e-8 / 4.9e-8, [0, 1] 8.4e-8 / 9.3e-8, [1, 3] 2.5e-7 / 2.1e-7;
-// relative 1.3e-4 at most down to -7.5, where 1 + erf has no digit left from -5.5 on. The rounding to bf16 behind it is up to 2^-8.
-__device__ __forceinline__ float nt_gelu(float x) {
-  const float a = fabsf(x), c = __builtin_amdgcn_fmed3f(a, 0.f, 7.5f);
-  float p = __builtin_fmaf(-1.84474267e-8f, c, 6.14227645e-7f);
-  p = __builtin_fmaf(p, c, -8.58164822e-6f);
-  p = __builtin_fmaf(p, c, 6.38452766e-5f);
-  p = __builtin_fmaf(p, c, -2.39952234e-4f);
-  p = __builtin_fmaf(p, c, -7.65839359e-5f);
-  p = __builtin_fmaf(p, c, 7.03580119e-3f);
-  p = __builtin_fmaf(p, c, -5.24996445e-2f);
-  p = __builtin_fmaf(p, c, 2.62145728e-1f);
-  p = __builtin_fmaf(p, c, -1.15110648f);
-  p = __builtin_fmaf(p, c, -0.99999994f);
-  const float q = __builtin_amdgcn_exp2f(__builtin_fmaf(-0.721347511f * a, a, p));
-  return x * (x < 0.f ? q : 1.f - q);
-}
 }  // namespace
 
 __global__ void __launch_bounds__(256, 1) gemm_nt_gelu_kernel(GemmNtParams p) {
@@ -172,7 +152,7 @@ __global__ void __launch_bounds__(256, 1) gemm_nt_gelu_kernel(GemmNtParams p) {
       for (int t = 0; t < 8; ++t) {
         u16x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = f2bf(nt_gelu(acc[t][j][e]));
+        for (int e = 0; e < 4; ++e) v[e] = f2bf(gelu_f(acc[t][j][e]));
         *reinterpret_cast<u16x4*>(p.out + (int64_t)m * p.N + at + 16 * t) = v;
       }
     }

@@ -2,13 +2,17 @@
 // bias, GELU or a K split for the norm that follows; that norm; and the embedding sum with its norm.
 //
 // With tens of rows a projection is its weight stream, 2 to 8 MB of a BERT-large layer: about a microsecond of HBM time,
-// so latency decides. Every wave loads the MFMA fragments of its whole share of K straight into registers, all in flight
-// at once (W rows are the A operand, token rows the B operand, 16 bytes a lane each), multiplies, and the eight waves of a
-// workgroup, which share 16 features and split K, meet once in LDS. No staging, no loop of barriers. BERT-large at 19
-// rows, weights from HBM (us, library / here): q/k/v 11.1 / 5.1, output 5.8 / 3.0, up 11.3 / 5.4 and its GELU launch
-// saved, down 14.1 / 4.9. Token rows come from L2 again for each workgroup: from 33 rows on the LDS tiles of
-// gemm_skinny.hip are faster (64 rows: q/k/v 8.2 here, 7.6 there).
+// so latency decides, and the cycles of a CU's load path: every workgroup reads all token rows beside its 16 rows of weights. Every wave
+// loads its whole share of K straight into registers, all in flight at once, multiplies (W rows are the A operand, token rows the B
+// operand), and the eight waves of a workgroup, which share 16 features and split K, meet once in LDS. No staging, no loop of barriers.
+// What bounds it is how the lanes of a load lie: as an MFMA operand wants them, 16 rows to neighbouring lanes, a load takes a cycle a
+// lane (37 bytes a nanosecond and CU from L2); with four lanes to 64 bytes of a row 107. So weights come in that order and change
+// lanes (gr_fragment), and token rows lie packed, a step of 16 rows in one piece, written so by what makes them. BERT-large at 19 rows,
+// weights from HBM, us, library / as fragments / so: q/k/v 11.1 / 5.1 / 3.7, output behind its attention - / 5.3 / 4.5, up 11.3 / 5.9 /
+// 3.9 and its GELU launch saved, down 14.1 / 5.3 / 3.9. Token rows come from L2 again for each workgroup: from 33 rows on the LDS tiles
+// of gemm_skinny.hip are faster (64 rows, as fragments: q/k/v 8.2 here, 7.6 there).
 #include "common.h"
+#include "gelu.h"
 #include "kernels.h"
 
 namespace nga {
@@ -17,27 +21,44 @@ namespace {
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4* ltr_t;
 
-// 0.5 x (1 + erf(x / sqrt 2))
-__device__ __forceinline__ float gr_gelu(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
+// 16 rows x 32 values as an instruction brings them fastest, four lanes for 64 bytes of a row (lane 4 r + c: row r, values 8 c ..),
+// as the MFMA operand: lane r + 16 c
+__device__ __forceinline__ bf16x8 gr_fragment(u16x8 v, int lane) {
+  typedef int i32x4 __attribute__((ext_vector_type(4)));
+  const int from = ((lane & 15) * 4 + (lane >> 4)) * 4;
+  i32x4 a = __builtin_bit_cast(i32x4, v);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) a[i] = __builtin_amdgcn_ds_bpermute(from, a[i]);
+  return __builtin_bit_cast(bf16x8, a);
+}
+
+// Where value c of row r of packed rows lies: [rows / 16][values / 32] pieces of 64 x 8 values, each the B operand of one MFMA
+__device__ __forceinline__ int row_packed(int r, int c, int cols) {
+  return (((r >> 4) * (cols >> 5) + (c >> 5)) * 64 + ((c >> 3) & 3) * 16 + (r & 15)) * 8 + (c & 7);
+}
+
 }  // namespace
 
 // MT x 16 token rows and 16 features per workgroup; PD k-steps of 32 in flight per wave, twice.
 // EPI 0: bf16 out, + bias; 1: fp32 slab [split, M, N]; 2: bf16 out, GELU(. + bias)
-template <int MT, int EPI>
+template <int MT, int EPI, bool XP>
 __global__ void __launch_bounds__(512) row_gemm_kernel(RowGemmParams P) {
   constexpr int PD = 4, NW = 8;
   __shared__ __attribute__((aligned(16))) float part[NW * MT * 256];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, h = lane >> 4;
-  const int f0 = blockIdx.x * 16, t0 = blockIdx.y * 16 * MT, ks = blockIdx.z;
+  const int f0 = blockIdx.x * 16, ks = blockIdx.y;
   const int steps = P.K / 32, slices = NW * P.split, sl = ks * NW + w;
   const int s0 = steps * sl / slices, s1 = steps * (sl + 1) / slices;
-  const uint16_t *wp = P.w + (int64_t)(f0 + col) * P.K + 8 * h, *xp[MT];
+  const int lr = lane >> 2, lc = 8 * (lane & 3);   // a lane's row and values of the loads
+  const uint16_t* wp = P.w + (int64_t)(f0 + lr) * P.K + lc;
+  const uint16_t* xp[MT];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) xp[i] = P.x + (int64_t)min(t0 + 16 * i + col, P.M - 1) * P.ldx + 8 * h;
+  for (int i = 0; i < MT; ++i) xp[i] = XP ? P.x + ((int64_t)i * steps * 64 + lane) * 8 : P.x + (int64_t)min(16 * i + lr, P.M - 1) * P.ldx + lc;
   u16x4 bias = (u16x4)(0);   // asked for with the rest: at the end it would be a latency of its own
-  if (EPI != 1 && w < MT) bias = *reinterpret_cast<const u16x4*>(P.bias + f0 + 4 * h);
+  if (EPI == 2) bias[0] = P.bias[f0 + ((tid >> 7) & 1) * 8 + (tid & 7)];
+  if (EPI == 0 && w < MT) bias = *reinterpret_cast<const u16x4*>(P.bias + f0 + 4 * h);
   f32x4 acc[MT];
 #pragma unroll
   for (int j = 0; j < MT; ++j) acc[j] = (f32x4)(0.f);
@@ -48,8 +69,15 @@ __global__ void __launch_bounds__(512) row_gemm_kernel(RowGemmParams P) {
       if (s + d < s1) {
         av[d] = load8(wp + 32 * (s + d));
 #pragma unroll
-        for (int i = 0; i < MT; ++i) bv[d][i] = load8(xp[i] + 32 * (s + d));
+        for (int i = 0; i < MT - 1; ++i) bv[d][i] = load8(xp[i] + (XP ? 512 : 32) * (s + d));
       }
+#pragma unroll
+    for (int d = 0; d < PD; ++d) bv[d][MT - 1] = (u16x8)(0);
+    if ((XP ? col : lr) < P.M - 16 * (MT - 1)) {   // lanes of rows that are not there bring nothing
+#pragma unroll
+      for (int d = 0; d < PD; ++d)
+        if (s + d < s1) bv[d][MT - 1] = load8(xp[MT - 1] + (XP ? 512 : 32) * (s + d));
+    }
   };
   load(s0, a, b);
   for (int s = s0; s < s1; s += PD) {
@@ -57,8 +85,9 @@ __global__ void __launch_bounds__(512) row_gemm_kernel(RowGemmParams P) {
 #pragma unroll
     for (int d = 0; d < PD; ++d)
       if (s + d < s1) {
+        const bf16x8 af = gr_fragment(a[d], lane);
 #pragma unroll
-        for (int j = 0; j < MT; ++j) acc[j] = mfma16(as_bf16x8(a[d]), as_bf16x8(b[d][j]), acc[j]);
+        for (int j = 0; j < MT; ++j) acc[j] = mfma16(af, XP ? as_bf16x8(b[d][j]) : gr_fragment(b[d][j], lane), acc[j]);
       }
     if (s + PD < s1) {
 #pragma unroll
@@ -72,25 +101,30 @@ __global__ void __launch_bounds__(512) row_gemm_kernel(RowGemmParams P) {
 #pragma unroll
   for (int j = 0; j < MT; ++j) *reinterpret_cast<f32x4*>(&part[((w * MT + j) * 64 + lane) * 4]) = acc[j];
   __syncthreads();
-  // tile j: features f0 + 4 h + 0..3 of token t0 + 16 j + col; one wave each
+  if constexpr (EPI == 2) {
+    // a value each thread, eight of a row side by side: with four to a lane of MT waves the four GELUs were half a microsecond
+    if (tid >= MT * 256) return;
+    const int t = (tid >> 8) * 16 + ((tid >> 3) & 15), f = ((tid >> 7) & 1) * 8 + (tid & 7);
+    if (t >= P.M) return;
+    const float* const at = part + ((t >> 4) * 64 + (f >> 2) * 16 + (t & 15)) * 4 + (f & 3);
+    float v = at[0];
 #pragma unroll
-  for (int j = 0; j < MT; ++j) {
-    if (j != w) continue;
+    for (int u = 1; u < NW; ++u) v += at[u * MT * 256];
+    reinterpret_cast<uint16_t*>(P.out)[row_packed(t, f0 + f, P.N)] = f2bf(gelu_f(v + bf2f(bias[0])));
+  } else {
+    // tile w: features f0 + 4 h + 0..3 of token 16 w + col
+    const int t = 16 * w + col, n = f0 + 4 * h;
+    if (w >= MT || t >= P.M) return;
     f32x4 v = (f32x4)(0.f);
 #pragma unroll
-    for (int u = 0; u < NW; ++u) v += *reinterpret_cast<const f32x4*>(&part[((u * MT + j) * 64 + lane) * 4]);
-    const int t = t0 + 16 * j + col, n = f0 + 4 * h;
-    if (t >= P.M) continue;
+    for (int u = 0; u < NW; ++u) v += *reinterpret_cast<const f32x4*>(&part[((u * MT + w) * 64 + lane) * 4]);
     if constexpr (EPI == 1) {
       *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(P.out) + ((int64_t)ks * P.M + t) * P.N + n) = v;
     } else {
       u16x4 o;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float y = v[r] + bf2f(bias[r]);
-        o[r] = f2bf(EPI == 2 ? gr_gelu(y) : y);
-      }
-      *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + (int64_t)t * P.ldo + n) = o;
+      for (int r = 0; r < 4; ++r) o[r] = f2bf(v[r] + bf2f(bias[r]));
+      *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + (P.packed ? row_packed(t, n, P.N) : t * P.ldo + n)) = o;
     }
   }
 }
@@ -106,45 +140,42 @@ __global__ void __launch_bounds__(512) row_attn_gemm_kernel(RowGemmParams P) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, h = lane >> 4;
-  const int f0 = blockIdx.x * 16, ks = blockIdx.z, heads = P.K / D;
+  const int f0 = blockIdx.x * 16, ks = blockIdx.y, heads = P.K / D;
   const int h0 = heads * ks / P.split, h1 = heads * (ks + 1) / P.split, cols = (h1 - h0) * D, ld = cols + 8;
   const int steps = cols / 32, s0 = steps * w / NW, s1 = steps * (w + 1) / NW;
-  const uint16_t* wp = P.w + (int64_t)(f0 + col) * P.K + h0 * D + 8 * h;
+  const uint16_t* wp = P.w + (int64_t)(f0 + (lane >> 2)) * P.K + h0 * D + 8 * (lane & 3);
   u16x8 a[PD];
 #pragma unroll
   for (int d = 0; d < PD; ++d) a[d] = s0 + d < s1 ? load8(wp + 32 * (s0 + d)) : (u16x8)(0);
   // rows beside the sequence are clamped into it: whatever those hold, it would be multiplied by 0
   const int lo = max(0, P.cu[0]), hi = min(P.M, P.cu[1]);
-  auto row = [&](int r) { return (int64_t)max(lo, min(r, hi - 1)) * P.ldx; };
+  auto row = [&](int r) { return min(max(lo, min(r, hi - 1)), P.M - 1); };
   uint16_t* const vh = sm + 16 * MT * ld + w * (16 * MT * VL);
   for (int u = w; u < (h1 - h0) * MT; u += NW) {
     const int hd = u / MT, i = u % MT;   // queries 16 i .. of head h0 + hd
-    const uint16_t* base = P.x + (h0 + hd) * D;
-    u16x8 vr[MT * D / 32], kf[MT][DS], qf[DS];
+    bf16x8 kf[MT][DS], qf[DS];
+    u16x8 vr[MT * D / 32];
+    const int at = (h0 + hd) * D;
 #pragma unroll
     for (int s = 0; s < DS; ++s) {
-      qf[s] = load8(base + row(16 * i + col) + 32 * s + 8 * h);
+      qf[s] = as_bf16x8(load8(P.x + row_packed(row(16 * i + col), at + 32 * s + 8 * h, 3 * P.K)));
 #pragma unroll
       for (int t = 0; t < MT; ++t)   // row `col` of key tile t: key 8 (col / 4) + 4 t + col % 4 (of 16 keys: their order)
-        kf[t][s] = load8(base + P.K + row(MT == 2 ? 8 * (col >> 2) + 4 * t + (col & 3) : col) + 32 * s + 8 * h);
+        kf[t][s] = as_bf16x8(load8(P.x + row_packed(row(MT == 2 ? 8 * (col >> 2) + 4 * t + (col & 3) : col), P.K + at + 32 * s + 8 * h, 3 * P.K)));
     }
+    auto vrow = [&](int j) { return (64 * j + lane) % (16 * MT); };
+    auto vcol = [&](int j) { return (64 * j + lane) / (16 * MT) * 8; };
 #pragma unroll
-    for (int j = 0; j < MT * D / 32; ++j) {
-      const int c = 64 * j + lane;
-      vr[j] = load8(base + 2 * P.K + row(c / (D / 8)) + 8 * (c % (D / 8)));
-    }
+    for (int j = 0; j < MT * D / 32; ++j) vr[j] = load8(P.x + row_packed(row(vrow(j)), 2 * P.K + at + vcol(j), 3 * P.K));
 #pragma unroll
-    for (int j = 0; j < MT * D / 32; ++j) {
-      const int c = 64 * j + lane;
-      store8(vh + c / (D / 8) * VL + 8 * (c % (D / 8)), vr[j]);
-    }
+    for (int j = 0; j < MT * D / 32; ++j) store8(vh + vrow(j) * VL + vcol(j), vr[j]);
     f32x4 S[MT];
     float mx = -INFINITY;
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       S[t] = (f32x4)(0.f);
 #pragma unroll
-      for (int s = 0; s < DS; ++s) S[t] = mfma16(as_bf16x8(kf[t][s]), as_bf16x8(qf[s]), S[t]);
+      for (int s = 0; s < DS; ++s) S[t] = mfma16(kf[t][s], qf[s], S[t]);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int key = MT == 2 ? 8 * h + 4 * t + r : 4 * h + r;
@@ -191,10 +222,12 @@ __global__ void __launch_bounds__(512) row_attn_gemm_kernel(RowGemmParams P) {
       for (int d = 0; d < PD; ++d)
         if (s + d < s1) a[d] = load8(wp + 32 * (s + d));
 #pragma unroll
-    for (int d = 0; d < PD; ++d)
-      if (s + d < s1)
+    for (int d = 0; d < PD; ++d) {
+      if (s + d >= s1) continue;
+      const bf16x8 af = gr_fragment(a[d], lane);
 #pragma unroll
-        for (int j = 0; j < MT; ++j) acc[j] = mfma16(as_bf16x8(a[d]), as_bf16x8(load8(sm + (16 * j + col) * ld + 32 * (s + d) + 8 * h)), acc[j]);
+      for (int j = 0; j < MT; ++j) acc[j] = mfma16(af, as_bf16x8(load8(sm + (16 * j + col) * ld + 32 * (s + d) + 8 * h)), acc[j]);
+    }
   }
   float* const part = reinterpret_cast<float*>(sm + 16 * MT * ld);   // V is read
 #pragma unroll
@@ -219,7 +252,7 @@ __global__ void __launch_bounds__(1024) splitk_layernorm_kernel(const float* __r
                                                                 const uint16_t* __restrict__ bias,
                                                                 const uint16_t* __restrict__ resid,
                                                                 const uint16_t* __restrict__ g, const uint16_t* __restrict__ b,
-                                                                float eps, int H, uint16_t* __restrict__ out) {
+                                                                float eps, int H, uint16_t* __restrict__ out, uint16_t* __restrict__ packed) {
   __shared__ float red[16];
   const int64_t row = blockIdx.x;
   const int c = threadIdx.x * 8;
@@ -273,6 +306,7 @@ __global__ void __launch_bounds__(1024) splitk_layernorm_kernel(const float* __r
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = f2bf((x[i] - mean) * rstd * bf2f(gv[i]) + bf2f(bv[i]));
     store8(out + row * H + c, o);
+    if (packed != nullptr) store8(packed + row_packed((int)row, c, H), o);
   }
 }
 
@@ -284,7 +318,7 @@ __global__ void __launch_bounds__(1024) embed_layernorm_kernel(const int32_t* __
                                                                const uint16_t* __restrict__ ptab, int n_pos,
                                                                const uint16_t* __restrict__ ttab, int n_type,
                                                                const uint16_t* __restrict__ g, const uint16_t* __restrict__ b,
-                                                               float eps, int H, uint16_t* __restrict__ out) {
+                                                               float eps, int H, uint16_t* __restrict__ out, uint16_t* __restrict__ packed) {
   __shared__ float red[16];
   const int64_t row = blockIdx.x;
   const int c = threadIdx.x * 8;
@@ -314,19 +348,21 @@ __global__ void __launch_bounds__(1024) embed_layernorm_kernel(const int32_t* __
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = f2bf((x[i] - mean) * rstd * bf2f(gv[i]) + bf2f(bv[i]));
     store8(out + row * H + c, o);
+    if (packed != nullptr) store8(packed + row_packed((int)row, c, H), o);
   }
 }
 
 void launch_row_gemm(const RowGemmParams& p, int epi, hipStream_t stream) {
   if (p.M == 0 || p.N == 0) return;
   const int mt = p.M <= 16 ? 1 : 2;
-  const dim3 grid(p.N / 16, (p.M + 16 * mt - 1) / (16 * mt), p.split);
-#define NGA_RG(MT_)                                                               \
-  if (mt == MT_) {                                                                \
-    if (epi == 0) row_gemm_kernel<MT_, 0><<<grid, 512, 0, stream>>>(p);           \
-    else if (epi == 1) row_gemm_kernel<MT_, 1><<<grid, 512, 0, stream>>>(p);      \
-    else row_gemm_kernel<MT_, 2><<<grid, 512, 0, stream>>>(p);                    \
-    return;                                                                       \
+  const dim3 grid(p.N / 16, p.split);
+#define NGA_RG(MT_)                                                                                \
+  if (mt == MT_) {                                                                                 \
+    if (epi == 0) row_gemm_kernel<MT_, 0, true><<<grid, 512, 0, stream>>>(p);                      \
+    else if (epi == 2) row_gemm_kernel<MT_, 2, true><<<grid, 512, 0, stream>>>(p);                 \
+    else if (p.ldx == 0) row_gemm_kernel<MT_, 1, true><<<grid, 512, 0, stream>>>(p);               \
+    else row_gemm_kernel<MT_, 1, false><<<grid, 512, 0, stream>>>(p);                              \
+    return;                                                                                        \
   }
   NGA_RG(1) NGA_RG(2)
 #undef NGA_RG
@@ -345,7 +381,7 @@ void launch_row_attn_gemm(const RowGemmParams& p, int D, hipStream_t stream) {
     static const hipError_t attr = hipFuncSetAttribute((const void*)row_attn_gemm_kernel<MT_, DD>,         \
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
     (void)attr;                                                                                            \
-    row_attn_gemm_kernel<MT_, DD><<<dim3(p.N / 16, 1, p.split), 512, lds, stream>>>(p);                    \
+    row_attn_gemm_kernel<MT_, DD><<<dim3(p.N / 16, p.split), 512, lds, stream>>>(p);                    \
   }
 #define NGA_RD(MT_) if (D == 32) NGA_RA(MT_, 32) else if (D == 64) NGA_RA(MT_, 64) else NGA_RA(MT_, 128)
   if (mt == 1) { NGA_RD(1) } else { NGA_RD(2) }
@@ -356,9 +392,9 @@ void launch_row_attn_gemm(const RowGemmParams& p, int D, hipStream_t stream) {
 static int rows_threads(int H) { return (H / 8 + 63) / 64 * 64; }
 
 void launch_splitk_layernorm(const float* P, int S, int M, const uint16_t* bias, const uint16_t* resid, const uint16_t* g,
-                             const uint16_t* b, float eps, int H, uint16_t* out, hipStream_t stream) {
+                             const uint16_t* b, float eps, int H, uint16_t* out, uint16_t* packed, hipStream_t stream) {
   if (M == 0) return;
-#define NGA_SL(NS) splitk_layernorm_kernel<NS><<<M, rows_threads(H), 0, stream>>>(P, S, M, bias, resid, g, b, eps, H, out)
+#define NGA_SL(NS) splitk_layernorm_kernel<NS><<<M, rows_threads(H), 0, stream>>>(P, S, M, bias, resid, g, b, eps, H, out, packed)
   if (S == 1) NGA_SL(1);
   else if (S == 2) NGA_SL(2);
   else if (S == 3) NGA_SL(3);
@@ -370,10 +406,10 @@ void launch_splitk_layernorm(const float* P, int S, int M, const uint16_t* bias,
 
 void launch_embed_layernorm(const int32_t* ids, const int32_t* pos, const int32_t* types, const uint16_t* word, int n_word,
                             const uint16_t* ptab, int n_pos, const uint16_t* ttab, int n_type, const uint16_t* g,
-                            const uint16_t* b, float eps, int64_t rows, int H, uint16_t* out, hipStream_t stream) {
+                            const uint16_t* b, float eps, int64_t rows, int H, uint16_t* out, uint16_t* packed, hipStream_t stream) {
   if (rows == 0) return;
   embed_layernorm_kernel<<<(unsigned)rows, rows_threads(H), 0, stream>>>(ids, pos, types, word, n_word, ptab, n_pos, ttab, n_type,
-                                                                         g, b, eps, H, out);
+                                                                         g, b, eps, H, out, packed);
 }
 
 }  // namespace nga

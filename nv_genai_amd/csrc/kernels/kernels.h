@@ -261,7 +261,7 @@ void launch_search_finish(const float* cand_v, const int32_t* cand_r, const int3
 
 // gemm_rows.hip: projections of few rows with the steps around them
 struct RowGemmParams {
-  const uint16_t* x;   // [M, K], row stride ldx
+  const uint16_t* x;   // [M, K]: packed (row_packed), or for epi 1 rows of stride ldx where that is not 0
   int64_t ldx;
   const uint16_t* w;   // [N, K]; N % 16 == 0, K % 32 == 0; M <= 32
   const uint16_t* bias;
@@ -270,15 +270,16 @@ struct RowGemmParams {
   int M, N, K, split;
   const int32_t* cu;   // row_attn_gemm: the rows' one sequence, cu[0] .. cu[1]; x = q | k | v, K the values of one of them
   float scale;
+  int packed;          // epi 0: out is packed as that of epi 2 is
 };
 void launch_row_gemm(const RowGemmParams& p, int epi, hipStream_t stream);
 int row_attn_split(int heads);
 void launch_row_attn_gemm(const RowGemmParams& p, int D, hipStream_t stream);
 void launch_splitk_layernorm(const float* P, int S, int M, const uint16_t* bias, const uint16_t* resid, const uint16_t* g,
-                             const uint16_t* b, float eps, int H, uint16_t* out, hipStream_t stream);
+                             const uint16_t* b, float eps, int H, uint16_t* out, uint16_t* packed, hipStream_t stream);
 void launch_embed_layernorm(const int32_t* ids, const int32_t* pos, const int32_t* types, const uint16_t* word, int n_word,
                             const uint16_t* ptab, int n_pos, const uint16_t* ttab, int n_type, const uint16_t* g,
-                            const uint16_t* b, float eps, int64_t rows, int H, uint16_t* out, hipStream_t stream);
+                            const uint16_t* b, float eps, int64_t rows, int H, uint16_t* out, uint16_t* packed, hipStream_t stream);
 
 // gemm_kn.hip: out[M, N] = x[M, K] . w[K, N], bf16, or fp32 slabs [split, M, N]; K % 32 == 0, N % 256 == 0, K >= 256 a slice. xt: x lies as
 // [K, M], M % 256 == 0, any K
