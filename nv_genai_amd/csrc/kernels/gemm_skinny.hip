@@ -38,6 +38,7 @@
 
 #include <cstdint>
 #include "common.h"
+#include "gelu.h"
 #include "kernels.h"
 
 namespace nga {
@@ -63,8 +64,6 @@ __device__ __forceinline__ void sk_wait_vm() {
   static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
-
-__device__ __forceinline__ float sk_gelu(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
 
 __device__ __forceinline__ float sk_silu(float x) { return x / (1.f + __expf(-x)); }
 
@@ -260,46 +259,57 @@ __global__ void __launch_bounds__(64 * WN * WM * KG) skinny_gemm_kernel(SkinnyGe
     }
   }
 
-  // epilogue: acc[nt][mt][r] = out[token (16-tile mt, col)][feature (16-tile nt, 4h + r)]
+  // acc[nt][mt][r] = out[token (16-tile mt, col)][feature (16-tile nt, 4h + r)]. Sixteen tokens of a wave at a time pass through LDS
+  // and go out in whole rows, 16 bytes a lane: as they lie in the accumulators neighbouring lanes belong to different rows, and such
+  // a store takes a cycle a lane. 3,072 features of K 1,024 at 208 / 512 / 1,024 rows, us: 7.2 10.1 14.0, so 7.0 9.4 12.8; slabs of
+  // 1,024 features of K 4,096 7.6 11.0 16.9, so 7.5 10.8 16.2
+  constexpr int VB = EPI == 1 ? 4 : 2, OW = EPI == 2 ? RW / 2 : RW, MO = MTW / KG;   // bytes of a value; a wave's features and token tiles
+  constexpr int PITCH = OW * VB + 16, CPO = OW * VB / 16, ROWS = 16 * PITCH;
+  constexpr int BASE = KG > 1 ? KG * MTW * NTW * NW * 64 * 16 : 0;   // behind the groups' sums
+  static_assert(BASE + KG * NW * ROWS <= (int)sizeof(smem), "a row tile of each wave fits the stages");
+  if constexpr (KG == 1) __builtin_amdgcn_s_barrier();   // every stage is read, no DMA is under way
+  char* const rows = reinterpret_cast<char*>(smem) + BASE + (kg * NW + wv) * ROWS;
   const int t_base = mi * BM + wm * CW;
-  const int n_base = nb * BN + wn * RW;
+  const int n_base = EPI == 2 ? nb * (BN / 2) + wn * (RW / 2) : nb * BN + wn * RW;
 #pragma unroll
   for (int mt = 0; mt < MTW; ++mt) {
-    const int t = t_base + mt * 16 + col;
-    if (t >= P.M || (KG > 1 && mt / (MTW / KG) != kg)) continue;
-    if constexpr (EPI == 0 || EPI == 3 || EPI == 4) {
-      uint16_t* op = reinterpret_cast<uint16_t*>(P.out) + (int64_t)t * P.ldo;
+    if (KG > 1 && mt / MO != kg) continue;
+    if (t_base + mt * 16 >= P.M) continue;
+    char* const to = rows + col * PITCH + 4 * h * VB;
+    if constexpr (EPI == 1) {
+#pragma unroll
+      for (int nt = 0; nt < NTW; ++nt) *reinterpret_cast<f32x4*>(to + nt * 64) = acc[nt][mt];
+    } else if constexpr (EPI == 2) {
+#pragma unroll
+      for (int g = 0; g < NTW / 2; ++g) {
+        u16x4 v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = f2bf(sk_silu(acc[2 * g][mt][r]) * acc[2 * g + 1][mt][r]);
+        *reinterpret_cast<u16x4*>(to + g * 32) = v;
+      }
+    } else {
 #pragma unroll
       for (int nt = 0; nt < NTW; ++nt) {
-        const int n = n_base + nt * 16 + 4 * h;
-        if (n >= P.N) continue;
         u16x4 v;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           float y = acc[nt][mt][r];
           if constexpr (EPI >= 3) y += bf2f(bias[nt][r]);
-          if constexpr (EPI == 4) y = sk_gelu(y);
+          if constexpr (EPI == 4) y = gelu_f(y);
           v[r] = f2bf(y);
         }
-        *reinterpret_cast<u16x4*>(op + n) = v;
+        *reinterpret_cast<u16x4*>(to + nt * 32) = v;
       }
-    } else if constexpr (EPI == 1) {
-      float* op = reinterpret_cast<float*>(P.out) + ((int64_t)ks * P.M + t) * P.N;
+    }
 #pragma unroll
-      for (int nt = 0; nt < NTW; ++nt) {
-        const int n = n_base + nt * 16 + 4 * h;
-        if (n >= P.N) continue;
-        *reinterpret_cast<f32x4*>(op + n) = acc[nt][mt];
-      }
-    } else {
-      uint16_t* op = reinterpret_cast<uint16_t*>(P.out) + (int64_t)t * P.ldo;
-#pragma unroll
-      for (int g = 0; g < NTW / 2; ++g) {
-        const int f = nb * (BN / 2) + wn * (RW / 2) + g * 16 + 4 * h;
-        u16x4 v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = f2bf(sk_silu(acc[2 * g][mt][r]) * acc[2 * g + 1][mt][r]);
-        *reinterpret_cast<u16x4*>(op + f) = v;
+    for (int i = 0; i < (16 * CPO + 63) / 64; ++i) {
+      const int p = i * 64 + lane, r = p / CPO, c = p % CPO, t = t_base + mt * 16 + r, n = n_base + c * (16 / VB);
+      if ((16 * CPO % 64 && r >= 16) || t >= P.M || n >= P.N) continue;
+      const u16x8 v = *reinterpret_cast<const u16x8*>(rows + r * PITCH + c * 16);
+      if constexpr (EPI == 1) {
+        *reinterpret_cast<u16x8*>(reinterpret_cast<float*>(P.out) + ((int64_t)ks * P.M + t) * P.N + n) = v;
+      } else {
+        store8_any(reinterpret_cast<uint16_t*>(P.out) + (int64_t)t * P.ldo + n, v);
       }
     }
   }
