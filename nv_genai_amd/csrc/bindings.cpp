@@ -1430,7 +1430,7 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
   };
   // out = LN(in w^T + bias + resid); in_stride: 0 where up to 32 rows of it are packed
   auto project_norm = [&](const Tensor& in, int64_t in_stride, const Tensor& w, const Tensor& bias, const Tensor& resid, const Tensor& g,
-                          const Tensor& b, Tensor& out) {
+                          const Tensor& b, Tensor& out, const nga::ReadAhead& next) {
     const int64_t K = w.size(1);
     const int split = encoder_split(T, H, K);
     if (rows) {
@@ -1446,7 +1446,7 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
       return;
     }
     nga::launch_splitk_layernorm(slabs.data_ptr<float>(), split, (int)T, bfp(bias), bfp(resid), bfp(g), bfp(b), (float)eps, (int)H,
-                                 bfp(out), packed, st);
+                                 bfp(out), packed, next, st);
   };
   nga::PrefillParams p{};
   p.out = bfp(a);
@@ -1458,19 +1458,24 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
   p.cu_q = cu.data_ptr<int32_t>();
   p.Hq = p.Hkv = (int)heads;
   p.scale = (float)scale;
+  // the weights behind a norm
+  auto ahead = [&](size_t i) -> nga::ReadAhead {
+    if (i >= L.size()) return {};
+    return {bfp(L[i]), (int)L[i].size(0), (int)L[i].size(1), tiles};
+  };
   for (size_t i = 0; i < L.size(); i += 12) {
     project(x, L[i], L[i + 1], qkv, false);
     if (one) {
       nga::launch_row_attn_gemm({bfp(qkv), 0, bfp(L[i + 2]), nullptr, slabs.data_ptr(), H, (int)T, (int)H, (int)H, att_split,
                                  p.cu_q, p.scale}, (int)D, st);
       nga::launch_splitk_layernorm(slabs.data_ptr<float>(), att_split, (int)T, bfp(L[i + 3]), bfp(x), bfp(L[i + 4]), bfp(L[i + 5]),
-                                   (float)eps, (int)H, bfp(x), packed, st);
+                                   (float)eps, (int)H, bfp(x), packed, ahead(i + 6), st);
     } else {
       if (B > 0 && max_len > 0) nga::launch_varlen_attention(p, (int)B, (int)max_len, (int)D, false, st);
-      project_norm(a, H, L[i + 2], L[i + 3], x, L[i + 4], L[i + 5], x);
+      project_norm(a, H, L[i + 2], L[i + 3], x, L[i + 4], L[i + 5], x, ahead(i + 6));
     }
     project(x, L[i + 6], L[i + 7], h, true);
-    project_norm(h, 0, L[i + 8], L[i + 9], x, L[i + 10], L[i + 11], x);
+    project_norm(h, 0, L[i + 8], L[i + 9], x, L[i + 10], L[i + 11], x, ahead(i + 12));
   }
   post_launch("encoder_forward");
   return x;

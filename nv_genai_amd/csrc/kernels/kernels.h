@@ -259,6 +259,13 @@ void launch_search_finish(const float* cand_v, const int32_t* cand_r, const int3
                           int k, const float* qf, int64_t q_stride, int D, const int64_t* ids, float* out_v, int64_t* out_id,
                           hipStream_t stream);
 
+// Weights of the launch behind a norm, read into L2 by workgroups beside the norm's: rows [16 p, 16 p + 16) by the die p % 8, where
+// workgroup p of gemm_rows.hip runs, or (tiled) the x-th eighth of them by die x, as gemm_skinny.hip deals its tiles. w null: none
+struct ReadAhead {
+  const uint16_t* w;
+  int N, K, tiled;
+};
+
 // gemm_rows.hip: projections of few rows with the steps around them
 struct RowGemmParams {
   const uint16_t* x;   // [M, K]: packed (row_packed), or for epi 1 rows of stride ldx where that is not 0
@@ -276,7 +283,7 @@ void launch_row_gemm(const RowGemmParams& p, int epi, hipStream_t stream);
 int row_attn_split(int heads);
 void launch_row_attn_gemm(const RowGemmParams& p, int D, hipStream_t stream);
 void launch_splitk_layernorm(const float* P, int S, int M, const uint16_t* bias, const uint16_t* resid, const uint16_t* g,
-                             const uint16_t* b, float eps, int H, uint16_t* out, uint16_t* packed, hipStream_t stream);
+                             const uint16_t* b, float eps, int H, uint16_t* out, uint16_t* packed, const ReadAhead& next, hipStream_t stream);
 void launch_embed_layernorm(const int32_t* ids, const int32_t* pos, const int32_t* types, const uint16_t* word, int n_word,
                             const uint16_t* ptab, int n_pos, const uint16_t* ttab, int n_type, const uint16_t* g,
                             const uint16_t* b, float eps, int64_t rows, int H, uint16_t* out, uint16_t* packed, hipStream_t stream);
