@@ -3015,6 +3015,12 @@ PYBIND11_MODULE(_C, m) {
   m.def("topk", checked("topk", &topk));
   m.def("encoder_tile_rows", &encoder_tile_rows);
   m.def("encoder_forward", &encoder_forward, py::call_guard<py::gil_scoped_release>());   // some 200 launches
+  m.def("encoder_forward_covered", [](Tensor ids, Tensor pos, c10::optional<Tensor> types, Tensor cu, int64_t max_len, Tensor word, Tensor ptab,
+                                      Tensor ttab, Tensor emb_g, Tensor emb_b, std::vector<Tensor> L, int64_t heads, double eps,
+                                      double scale) -> c10::optional<Tensor> {   // weights are looked at once for both questions
+    if (encoder_refuses(word, {ptab, ttab, emb_g, emb_b}, L, heads) != nullptr) return c10::nullopt;
+    return encoder_forward(ids, pos, types, cu, max_len, word, ptab, ttab, emb_g, emb_b, std::move(L), heads, eps, scale);
+  }, py::call_guard<py::gil_scoped_release>());
   m.def("encoder_covers", [](const Tensor& word, const std::vector<Tensor>& tables, const std::vector<Tensor>& L, int64_t heads) {
     return encoder_refuses(word, tables, L, heads) == nullptr;
   });

@@ -144,11 +144,11 @@ class EncoderModel:
         for a reranker (num_labels > 0) returns [B, num_labels] fp32 logits."""
         cfg = self.cfg
         H, nh, hd = cfg.hidden, cfg.heads, cfg.head_dim
-        if (ids.is_cuda and ids.dim() == 1 and pos.shape == ids.shape and (type_ids is None or type_ids.shape == ids.shape)
-                and ops.encoder_covers(self.word, self.layers, nh, (self.pos, self.type, *self.emb_ln))):
+        if ids.is_cuda and ids.dim() == 1 and pos.shape == ids.shape and (type_ids is None or type_ids.shape == ids.shape):
             x = ops.encoder_forward(ids, pos, type_ids, cu, max_len, self.word, self.pos, self.type, self.emb_ln, self.layers,
-                                    nh, cfg.eps, self.scale)
-            return self._pool(x, cu)
+                                    nh, cfg.eps, self.scale, covered_only=True)
+            if x is not None:
+                return self._pool(x, cu)
         tt = self.type[0] if type_ids is None else None
         e = torch.nn.functional.embedding(ids.long(), self.word)
         e = e + torch.nn.functional.embedding(pos.long(), self.pos)

@@ -1387,13 +1387,18 @@ def encoder_covers(word: torch.Tensor, layers, heads: int, tables=()) -> bool:
 
 
 def encoder_forward(ids, pos, types, cu, max_len: int, word, ptab, ttab, emb_ln, layers, heads: int, eps: float,
-                    scale: float) -> torch.Tensor:
+                    scale: float, covered_only: bool = False) -> Optional[torch.Tensor]:
     """Hidden rows [T, H] of packed tokens through a post-norm encoder stack (models/encoder.py), every launch from one
     native call: up to 32 rows the projections of gemm_rows.hip, up to 1,024 the LDS tiles of gemm_skinny.hip, both with
-    bias, GELU and the K split of the norm fused, above that the library's GEMM."""
+    bias, GELU and the K split of the norm fused, above that the library's GEMM. Weights that ``encoder_covers`` refuses raise, or
+    with ``covered_only`` give None."""
+    if covered_only and not _gpu(word):
+        return None
+
     def i32(t):
         return None if t is None else t.to(torch.int32).contiguous()
-    return kernels().encoder_forward(i32(ids), i32(pos), i32(types), i32(cu), int(max_len), word, ptab, ttab, emb_ln[0], emb_ln[1],
+    f = kernels().encoder_forward_covered if covered_only else kernels().encoder_forward
+    return f(i32(ids), i32(pos), i32(types), i32(cu), int(max_len), word, ptab, ttab, emb_ln[0], emb_ln[1],
                                      _encoder_weights(layers), int(heads), float(eps), float(scale))
 
 
