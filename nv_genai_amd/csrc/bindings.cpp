@@ -1647,9 +1647,9 @@ std::vector<Tensor> flat_search(Tensor q, Tensor X, Tensor bias, Tensor ids, dou
   if (ng == 1) {   // up to 16 queries are prepared by every workgroup, while its first vectors come in
     s.a.qf = q.data_ptr<float>();
   } else {
-    qb = at::empty({nq, D}, X.options());
+    qb = at::empty({wide ? (int64_t)items * 16 * ng : nq, D}, X.options());
     s.a.Q = bfp(qb);
-    nga::launch_search_prep(q.data_ptr<float>(), q.stride(0), (int)nq, D, (int)metric, bfp(qb), s.st);
+    nga::launch_search_prep(q.data_ptr<float>(), q.stride(0), (int)nq, D, (int)metric, bfp(qb), wide, s.st);
   }
   if (K == 0) {
     s.a.s_stride = (N + 3) / 4 * 4;

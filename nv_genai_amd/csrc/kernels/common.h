@@ -51,6 +51,13 @@ __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// Where value c of row r of packed rows lies: [rows / 16][values / 32] pieces of 64 x 8 values, each an operand of one MFMA in the order
+// of its lanes. A load whose neighbouring lanes belong to 16 rows, as the operand wants them from rows as they lie, takes a cycle a
+// lane: 37 bytes a nanosecond and CU from L2, a whole piece 107 and more
+__device__ __forceinline__ int packed_at(int r, int c, int cols) {
+  return (((r >> 4) * (cols >> 5) + (c >> 5)) * 64 + ((c >> 3) & 3) * 16 + (r & 15)) * 8 + (c & 7);
+}
+
 // FP8 (OCP e4m3fn) KV cache helpers. 8 cache bytes <-> 8 bf16 values; every e4m3 value is
 // exact in bf16, so reads are lossless. Writes saturate to +-448 (the format has no inf).
 // (fp8 -> f32 pairs, then bf16: exact. The one-step v_cvt_scalef32_pk_bf16_fp8 gave the even

@@ -32,11 +32,6 @@ __device__ __forceinline__ bf16x8 gr_fragment(u16x8 v, int lane) {
   return __builtin_bit_cast(bf16x8, a);
 }
 
-// Where value c of row r of packed rows lies: [rows / 16][values / 32] pieces of 64 x 8 values, each the B operand of one MFMA
-__device__ __forceinline__ int row_packed(int r, int c, int cols) {
-  return (((r >> 4) * (cols >> 5) + (c >> 5)) * 64 + ((c >> 3) & 3) * 16 + (r & 15)) * 8 + (c & 7);
-}
-
 }  // namespace
 
 // MT x 16 token rows and 16 features per workgroup; PD k-steps of 32 in flight per wave, twice.
@@ -110,7 +105,7 @@ __global__ void __launch_bounds__(512) row_gemm_kernel(RowGemmParams P) {
     float v = at[0];
 #pragma unroll
     for (int u = 1; u < NW; ++u) v += at[u * MT * 256];
-    reinterpret_cast<uint16_t*>(P.out)[row_packed(t, f0 + f, P.N)] = f2bf(gelu_f(v + bf2f(bias[0])));
+    reinterpret_cast<uint16_t*>(P.out)[packed_at(t, f0 + f, P.N)] = f2bf(gelu_f(v + bf2f(bias[0])));
   } else {
     // tile w: features f0 + 4 h + 0..3 of token 16 w + col
     const int t = 16 * w + col, n = f0 + 4 * h;
@@ -124,7 +119,7 @@ __global__ void __launch_bounds__(512) row_gemm_kernel(RowGemmParams P) {
       u16x4 o;
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = f2bf(v[r] + bf2f(bias[r]));
-      *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + (P.packed ? row_packed(t, n, P.N) : t * P.ldo + n)) = o;
+      *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + (P.packed ? packed_at(t, n, P.N) : t * P.ldo + n)) = o;
     }
   }
 }
@@ -158,15 +153,15 @@ __global__ void __launch_bounds__(512) row_attn_gemm_kernel(RowGemmParams P) {
     const int at = (h0 + hd) * D;
 #pragma unroll
     for (int s = 0; s < DS; ++s) {
-      qf[s] = as_bf16x8(load8(P.x + row_packed(row(16 * i + col), at + 32 * s + 8 * h, 3 * P.K)));
+      qf[s] = as_bf16x8(load8(P.x + packed_at(row(16 * i + col), at + 32 * s + 8 * h, 3 * P.K)));
 #pragma unroll
       for (int t = 0; t < MT; ++t)   // row `col` of key tile t: key 8 (col / 4) + 4 t + col % 4 (of 16 keys: their order)
-        kf[t][s] = as_bf16x8(load8(P.x + row_packed(row(MT == 2 ? 8 * (col >> 2) + 4 * t + (col & 3) : col), P.K + at + 32 * s + 8 * h, 3 * P.K)));
+        kf[t][s] = as_bf16x8(load8(P.x + packed_at(row(MT == 2 ? 8 * (col >> 2) + 4 * t + (col & 3) : col), P.K + at + 32 * s + 8 * h, 3 * P.K)));
     }
     auto vrow = [&](int j) { return (64 * j + lane) % (16 * MT); };
     auto vcol = [&](int j) { return (64 * j + lane) / (16 * MT) * 8; };
 #pragma unroll
-    for (int j = 0; j < MT * D / 32; ++j) vr[j] = load8(P.x + row_packed(row(vrow(j)), 2 * P.K + at + vcol(j), 3 * P.K));
+    for (int j = 0; j < MT * D / 32; ++j) vr[j] = load8(P.x + packed_at(row(vrow(j)), 2 * P.K + at + vcol(j), 3 * P.K));
 #pragma unroll
     for (int j = 0; j < MT * D / 32; ++j) store8(vh + vrow(j) * VL + vcol(j), vr[j]);
     f32x4 S[MT];
@@ -334,7 +329,7 @@ __global__ void __launch_bounds__(1024) splitk_layernorm_kernel(const float* __r
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = f2bf((x[i] - mean) * rstd * bf2f(gv[i]) + bf2f(bv[i]));
     store8(out + row * H + c, o);
-    if (packed != nullptr) store8(packed + row_packed((int)row, c, H), o);
+    if (packed != nullptr) store8(packed + packed_at((int)row, c, H), o);
   }
 }
 
@@ -376,7 +371,7 @@ __global__ void __launch_bounds__(1024) embed_layernorm_kernel(const int32_t* __
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = f2bf((x[i] - mean) * rstd * bf2f(gv[i]) + bf2f(bv[i]));
     store8(out + row * H + c, o);
-    if (packed != nullptr) store8(packed + row_packed((int)row, c, H), o);
+    if (packed != nullptr) store8(packed + packed_at((int)row, c, H), o);
   }
 }
 

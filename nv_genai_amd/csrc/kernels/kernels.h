@@ -232,7 +232,7 @@ int scan_list(int k, int ng, bool ivf);         // length of the register lists,
 void launch_scan(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream);
 bool scan_wide_covers(int D, int ng);           // flat scans of more than 16 queries
 void launch_scan_wide(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream);
-void launch_search_prep(const float* q, int64_t q_stride, int nq, int D, int metric, uint16_t* qb, hipStream_t stream);
+void launch_search_prep(const float* q, int64_t q_stride, int nq, int D, int metric, uint16_t* qb, bool packed, hipStream_t stream);
 // the whole search of one query but the merge: candidates of workgroup b in the k places from b k on; qf is the query
 constexpr int IVF_ONE_MAX_LISTS = 256;
 struct IvfLists {
@@ -268,7 +268,7 @@ struct ReadAhead {
 
 // gemm_rows.hip: projections of few rows with the steps around them
 struct RowGemmParams {
-  const uint16_t* x;   // [M, K]: packed (row_packed), or for epi 1 rows of stride ldx where that is not 0
+  const uint16_t* x;   // [M, K]: packed (packed_at), or for epi 1 rows of stride ldx where that is not 0
   int64_t ldx;
   const uint16_t* w;   // [N, K]; N % 16 == 0, K % 32 == 0; M <= 32
   const uint16_t* bias;

@@ -112,7 +112,7 @@ struct WaveQuery {
 
 // One wave per query: its bf16 form. Replaces four elementwise and reduction launches of 4 to 5 us each.
 __global__ void __launch_bounds__(256) search_prep_kernel(const float* __restrict__ q, int64_t q_stride, int nq, int D, int metric,
-                                                          uint16_t* __restrict__ qb) {
+                                                          uint16_t* __restrict__ qb, int packed) {
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= nq) return;
@@ -120,7 +120,7 @@ __global__ void __launch_bounds__(256) search_prep_kernel(const float* __restric
   wq.load(q + row * q_stride, D, metric, lane);
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    if (4 * lane + 256 * j < D) *reinterpret_cast<u16x4*>(qb + row * D + 4 * lane + 256 * j) = wq.bf(j);
+    if (4 * lane + 256 * j < D) *reinterpret_cast<u16x4*>(qb + (packed ? packed_at((int)row, 4 * lane + 256 * j, D) : row * D + 4 * lane + 256 * j)) = wq.bf(j);
 }
 
 // Plans of the scan by one workgroup of 1,024 threads, thread t for list t with `mine` probing queries: items of sl query slots
@@ -591,7 +591,7 @@ __global__ void __launch_bounds__(256, 1) scan_wide_kernel(ScanArgs p) {
   for (int g = 0; g < NG; ++g)
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      u16x8 v = load8(p.Q + (int64_t)(item * SL + min(16 * g + col, nql - 1)) * D + w * (D / 4) + 32 * s + 8 * h);
+      u16x8 v = load8(p.Q + packed_at(item * SL + 16 * g + col, w * (D / 4) + 32 * s + 8 * h, D));
       bq[g][s] = as_bf16x8(16 * g + col < nql ? v : (u16x8)(0));
     }
   int off[KS], row[KS];   // of this lane's 16 bytes of instruction i: chunk c of row r lies at c ^ (r & SW)
@@ -1320,8 +1320,9 @@ void launch_scan_wide(const ScanArgs& a, int ng, int K, int blocks, hipStream_t 
 #undef NGA_WIDE
 }
 
-void launch_search_prep(const float* q, int64_t q_stride, int nq, int D, int metric, uint16_t* qb, hipStream_t stream) {
-  search_prep_kernel<<<(nq + 3) / 4, 256, 0, stream>>>(q, q_stride, nq, D, metric, qb);
+void launch_search_prep(const float* q, int64_t q_stride, int nq, int D, int metric, uint16_t* qb, bool packed,
+                        hipStream_t stream) {
+  search_prep_kernel<<<(nq + 3) / 4, 256, 0, stream>>>(q, q_stride, nq, D, metric, qb, packed);
 }
 
 void launch_ivf_probe(const float* q, int64_t q_stride, int nq, int D, int metric, const float* cent, int nlist, int nprobe,
