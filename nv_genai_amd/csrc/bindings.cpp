@@ -1634,7 +1634,8 @@ std::vector<Tensor> flat_search(Tensor q, Tensor X, Tensor bias, Tensor ids, dou
   TORCH_CHECK(cus >= 1 && cus <= 4096, "flat_search: compute units");
   const int64_t nq = q.size(0), N = X.size(0);
   const int D = (int)X.size(1), ng = nq <= 16 ? 1 : nq <= 32 ? 2 : nq <= 48 ? 3 : 4;
-  const int items = (int)((nq + 16 * ng - 1) / (16 * ng)), K = nga::scan_list((int)k, ng, false);
+  const int items = (int)((nq + 16 * ng - 1) / (16 * ng)), held = nga::scan_list((int)k, ng, false);
+  const int K = nga::scan_scores_flat(nq, N, D, (int)k) ? 0 : held;
   const bool wide = nga::scan_wide_covers(D, ng);
   const int blocks = wide ? (int)cus : nga::scan_blocks(D, ng, (int)cus);
   const int64_t tiles = wide ? (N + 31) / 32 : (N + 127) / 128;
@@ -1655,6 +1656,7 @@ std::vector<Tensor> flat_search(Tensor q, Tensor X, Tensor bias, Tensor ids, dou
     s.a.s_stride = (N + 3) / 4 * 4;
     S = at::empty({nq, s.a.s_stride}, X.options().dtype(at::kFloat));
     s.a.S = S.data_ptr<float>();
+    s.a.drop_nan = held > 0;
   }
   if (wide) nga::launch_scan_wide(s.a, ng, K, items * parts, s.st);
   else nga::launch_scan(s.a, ng, K, items * parts, s.st);
@@ -1678,7 +1680,8 @@ std::vector<Tensor> ivf_search(Tensor q, Tensor X, Tensor bias, Tensor ids, Tens
   TORCH_CHECK(list_beg.numel() == nlist && list_end.numel() == nlist, "ivf_search: one row range per list");
   TORCH_CHECK(nprobe >= 1 && nprobe <= nlist, "ivf_search: nprobe must be in [1, lists]");
   TORCH_CHECK(k <= 32 && cus >= 1 && cus <= 4096, "ivf_search: k must be at most 32");
-  if (nga::ivf_one_covers(nq, nlist, D, (int)k)) {
+  const bool scores = nga::scan_scores_lists(nq, X.size(0), D, (int)k, nlist, nprobe);
+  if (nga::ivf_one_covers(nq, nlist, D, (int)k) && !(scores && k > 16)) {
     const int blocks = nga::scan_blocks(D, 1, (int)cus);
     Search s = search_begin(q, X, bias, dot_scale, metric, k, blocks * k);
     s.a.qf = q.data_ptr<float>();
@@ -1688,12 +1691,12 @@ std::vector<Tensor> ivf_search(Tensor q, Tensor X, Tensor bias, Tensor ids, Tens
   }
   int ng = nq <= 16 ? 1 : nq <= 32 ? 2 : nq <= 48 ? 3 : 4;
   if (ng > 2 && k > 8) ng = 2;   // longer register lists leave room for 32 queries
-  const int sl = 16 * ng, K = nga::scan_list((int)k, ng, true), blocks = nga::scan_blocks(D, ng, (int)cus);
+  const int sl = 16 * ng, K = scores ? 0 : nga::scan_list((int)k, ng, true), blocks = nga::scan_blocks(D, ng, (int)cus);
   const int64_t npairs = nq * nprobe, chunks = (nq + sl - 1) / sl;
   const int64_t max_items = std::min(npairs, nlist * chunks);
   TORCH_CHECK(chunks * ((X.size(0) + 127) / 128 + nlist) < (int64_t(1) << 31), "ivf_search: too many queries for one call");
   // the lists of a query lie in at most blocks + 2 nprobe runs
-  Search s = search_begin(q, X, bias, dot_scale, metric, k, (blocks + 2 * nprobe) * k);
+  Search s = search_begin(q, X, bias, dot_scale, metric, k, (K ? blocks + 2 * nprobe : nprobe) * k);
   const auto i32 = X.options().dtype(at::kInt);
   static_assert(sizeof(nga::ScanItem) == 32, "ScanItem");
   Tensor qb = at::empty({nq, D}, X.options());
@@ -1713,8 +1716,18 @@ std::vector<Tensor> ivf_search(Tensor q, Tensor X, Tensor bias, Tensor ids, Tens
   s.a.items = items;
   s.a.run_item = run_item;
   s.a.qtab = qtab;
+  Tensor S;
+  if (K == 0) {
+    s.a.s_stride = X.size(0);
+    S = at::empty({nq, s.a.s_stride}, X.options().dtype(at::kFloat));
+    s.a.S = S.data_ptr<float>();
+    s.a.drop_nan = 1;
+  }
   nga::launch_scan(s.a, ng, K, blocks, s.st);
-  return search_end(s, q, ids, -1, "ivf_search");
+  if (K == 0)
+    nga::launch_select_lists(s.a.S, s.a.s_stride, (int)nq, probes, (int)nprobe, list_beg.data_ptr<int64_t>(), list_end.data_ptr<int64_t>(), (int)k,
+                             s.a.cand_v, s.a.cand_r, s.st);
+  return search_end(s, q, ids, K ? -1 : (int32_t)(nprobe * k), "ivf_search");
 }
 
 void topk(Tensor in, c10::optional<Tensor> in_idx, int64_t seg_len, int64_t k, Tensor out_v,
@@ -3051,6 +3064,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("flat_search", &flat_search);
   m.def("ivf_search", &ivf_search);
   m.def("ivf_one_covers", &nga::ivf_one_covers);
+  m.def("scan_scores_flat", &nga::scan_scores_flat);
+  m.def("scan_scores_lists", &nga::scan_scores_lists);
   m.def("search_covers", [](int64_t d) { return d <= 1024 && nga::scan_chunk((int)d, 1) > 0; });
   m.def("score_topk", checked("score_topk", &score_topk));
   m.def("ivf_plan", checked("ivf_plan", &ivf_plan));

@@ -225,10 +225,13 @@ struct ScanArgs {
   int32_t* cand_r;
   float* S;                     // [nq, s_stride] where no list is kept
   int64_t s_stride;
+  int drop_nan;                 // scores that are no numbers are written as -inf, as register lists leave them out
 };
 int scan_chunk(int D, int ng);                  // dims of a unit of work, 0: not covered
 int scan_blocks(int D, int ng, int cus);        // workgroups that fill the chip
 int scan_list(int k, int ng, bool ivf);         // length of the register lists, 0: scores to S
+bool scan_scores_flat(int64_t nq, int64_t N, int D, int k);   // scores where lists could hold the results
+bool scan_scores_lists(int64_t nq, int64_t N, int D, int k, int64_t nlist, int64_t nprobe);
 void launch_scan(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream);
 bool scan_wide_covers(int D, int ng);           // flat scans of more than 16 queries
 void launch_scan_wide(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream);
@@ -255,6 +258,8 @@ void launch_ivf_items(const int32_t* probes, int npairs, int nprobe, int nlist, 
                       hipStream_t stream);
 void launch_select_segments(const float* S, int64_t s_stride, int nq, int64_t N, int64_t seg, int k, int32_t cap, float* cand_v,
                             int32_t* cand_r, hipStream_t stream);
+void launch_select_lists(const float* S, int64_t s_stride, int nq, const int32_t* probes, int nprobe, const int64_t* lbeg, const int64_t* lend,
+                         int k, float* cand_v, int32_t* cand_r, hipStream_t stream);
 void launch_search_finish(const float* cand_v, const int32_t* cand_r, const int32_t* cnt, int32_t n_fixed, int32_t cap, int nq,
                           int k, const float* qf, int64_t q_stride, int D, const int64_t* ids, float* out_v, int64_t* out_id,
                           hipStream_t stream);

@@ -23,6 +23,13 @@ __device__ __forceinline__ uint32_t ss_key(float f) {
 }
 constexpr uint32_t KEY_NEG_INF = 0x007fffffu;
 
+// a score that is no number, which no register list takes in, as the selection leaves it out
+__device__ __forceinline__ f32x4 ss_drop_nan(f32x4 v) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = v[i] == v[i] ? v[i] : -INFINITY;
+  return v;
+}
+
 // order of results: the higher value, of equal ones the lower row
 __device__ __forceinline__ bool ss_first(float av, int ar, float bv, int br) { return (av > bv) | ((av == bv) & (ar < br)); }
 
@@ -285,8 +292,8 @@ __global__ void __launch_bounds__(1024) ivf_items_kernel(const int32_t* __restri
 // vectors that scan_wide_kernel below does not take, halve what is left of LDS for the stream (33 of them, 250k x 1,024: 4.5 TB/s);
 // reading MFMA fragments from HBM directly, 16 rows x 64 B an instruction, took 187 us.
 // K > 0: a register list of K per lane and group, merged over lanes and waves at the end of a run, and appended to the
-// query's candidates. K = 0 (more than 16 results of up to 32 queries, or 8 of up to 64): scores to S, since inserting
-// into longer lists costs more than the 4 bytes a score.
+// query's candidates. K = 0 (more results than the lists hold, or where scan_scores_flat or scan_scores_lists finds it faster): scores
+// to S, of lists too, at their rows' places.
 template <int NG, int K, int CH>
 __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
   constexpr int SL = 16 * NG;
@@ -359,6 +366,11 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
       }
     };
     if (t0 < t1) issue(t0, 0);
+    int64_t qs[K > 0 ? 1 : NG];   // the queries whose scores this lane has
+    if constexpr (K == 0) {
+#pragma unroll
+      for (int g = 0; g < NG; ++g) qs[g] = 16 * g + col < nql ? slot_q(16 * g + col) : -1;
+    }
     if (NG == 1 && p.qf) {   // unprepared queries: a wave makes the bf16 form of four of them
       for (int r = w; r < SL; r += SS_W) {
         WaveQuery wq;
@@ -448,14 +460,14 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
                 }
               }
             } else {
-              const int q = item * SL + 16 * g + col;   // flat only
-              if (q < p.nq) {
-                float* dst = p.S + (int64_t)q * p.s_stride + rb;   // s_stride % 4 == 0
+              if (qs[g] >= 0) {
+                float* dst = p.S + qs[g] * p.s_stride + rb;
                 f32x4 v;
 #pragma unroll
                 for (int rr = 0; rr < 4; ++rr) v[rr] = acc[i][g][rr] * p.dot_scale + bcur[i][rr];
+                if (p.drop_nan) v = ss_drop_nan(v);
                 if (rb + 3 < end) {
-                  *reinterpret_cast<f32x4*>(dst) = v;
+                  __builtin_memcpy(dst, &v, 16);   // lists begin at any row
                 } else {
 #pragma unroll
                   for (int rr = 0; rr < 4; ++rr)
@@ -669,6 +681,7 @@ __global__ void __launch_bounds__(256, 1) scan_wide_kernel(ScanArgs p) {
         for (int rr = 0; rr < 4; ++rr)
           if (rb + rr < p.N && v[rr] > tv[gg][K - 1]) ss_insert<KR>(tv[gg], tr[gg], v[rr], (int)(rb + rr));
       } else if (16 * g + col < nql) {
+        if (p.drop_nan) v = ss_drop_nan(v);
         float* dst = p.S + (int64_t)(item * SL + 16 * g + col) * p.s_stride + rb;   // s_stride % 4 == 0
         if (rb + 3 < p.N) {
           *reinterpret_cast<f32x4*>(dst) = v;
@@ -1164,6 +1177,24 @@ __global__ void __launch_bounds__(256) select_segments_kernel(const float* __res
   }
 }
 
+// the same of each list that a query probes
+__global__ void __launch_bounds__(256) select_lists_kernel(const float* __restrict__ S, int64_t s_stride, const int32_t* __restrict__ probes,
+                                                           const int64_t* __restrict__ lbeg, const int64_t* __restrict__ lend, int k,
+                                                           float* __restrict__ cand_v, int32_t* __restrict__ cand_r) {
+  __shared__ SelShared s;
+  const int64_t q = blockIdx.y, nprobe = gridDim.x, at = (q * nprobe + blockIdx.x) * k;
+  const int list = probes[q * nprobe + blockIdx.x];
+  const int64_t beg = lbeg[list], n = lend[list] > beg ? lend[list] - beg : 0;
+  const int got = sel_topk<32>(S + q * s_stride + beg, (const int32_t*)nullptr, beg, n, k, s, [&](int place, float v, int32_t r) {
+    cand_v[at + place] = v;
+    cand_r[at + place] = r;
+  });
+  for (int i = got + threadIdx.x; i < k; i += 256) {
+    cand_v[at + i] = -INFINITY;
+    cand_r[at + i] = -1;
+  }
+}
+
 // a query's result from its candidates: the k best, less |q|^2 (l2), with the external ids of finite scores
 __global__ void __launch_bounds__(256) search_finish_kernel(const float* __restrict__ cand_v, const int32_t* __restrict__ cand_r,
                                                             const int32_t* __restrict__ cnt, int32_t n_fixed, int32_t cap,
@@ -1237,6 +1268,34 @@ static void scan_ch(const ScanArgs& a, int blocks, hipStream_t stream) {
 int scan_list(int k, int ng, bool ivf) {
   const int most = ng <= 2 ? (ivf ? 32 : 16) : 8;
   return k > most ? 0 : k <= 4 ? 4 : k <= 8 ? 8 : k <= 16 ? 16 : 32;
+}
+
+// Whether scores go to memory and are selected from there where register lists could hold the results: a list of 16 or 32 costs every
+// lane some 100 or 200 operations whenever one of a wave's takes a value in, and on merging, whatever the rows' length, a score 4 bytes
+// twice and the selection a launch. Up to 128 MiB of scores. Whole searches, us, lists / scores:
+// flat, k 12, at 1 / 12 / 28 queries: 100k x 128 44 49 59, 24 32 33; 130k x 384 52 53 57, 38 44 47; 500k x 512 130 144 160, 103 122 124; 300k x 640
+// 105 109 105, 80 97 104; 600k x 768 174 192 236, 160 200 207; 300k x 896 107 108 136, 97 116 124; 400k x 1,024 164 164 176, 144 171 180;
+// 1M x 1,024, k 14, at 1 / 4 / 12: 323 333 339, 326 358 393; 60k 47 48 50, 41 41 43. k 8, at 34 / 64: 130k x 384 62 68, 48 55; 900k x 384 264 331,
+// 197 232; 300k x 640 118 141, 104 119; 600k x 768 212 277, 212 236; 400k x 1,024 164 196, 184 200; 50k x
+// 768 39 44, 36 42; at 48 20k x 768 29, 31
+bool scan_scores_flat(int64_t nq, int64_t N, int D, int k) {
+  const int64_t n = nq * N;
+  if (nq > 64 || n > (int64_t(1) << 25)) return false;
+  if (nq > 32) return k > 4 && k <= 8 && D >= 256 && D <= 768 && n >= 1500000;
+  if (k <= 8 || k > 16) return false;
+  return D <= 640 || n <= 2000000 || (D <= 768 && n <= 5000000) || (nq > 16 && D <= 896);
+}
+// 64 lists, k 25, 16 probed, at 1 / 5 / 12 / 32 queries: 1M x 1,024 165 386 470 453, 133 299 376 418; 200k x 768 69 130 137 144, 47 80 88 94; 60k x 384
+// 49 75 76 79, 35 41 42 45; k 14, 8 probed, 2 / 5 / 12 / 20 / 32: 1M x 1,024 135 210 299 357 376, 123 196 297 361 392; 200k x 768 60 80 93 102 111, 47 63
+// 73 81 89; k 8: 200k x 768 49 67 77 87 94, 46 63 72 80 88; 60k x 384 32 34 43 44 44, 34 35 40 41 41; 1M x 1,024 117 190 278 325 341, 122 195 298 360
+// 391; k 6, 600k x 384, 16 probed, at 2 / 4 / 8 / 24: 80 98 120 131, 76 93 114 133; 300k x 640, 8 probed, at 8 / 24: 82 91, 78 93. One query of k 12 is
+// the one launch's, where that takes it (1M x 1,024 128 / 131).
+bool scan_scores_lists(int64_t nq, int64_t N, int D, int k, int64_t nlist, int64_t nprobe) {
+  if (k <= 4 || nq * N > (int64_t(1) << 25)) return false;
+  const int64_t n = nq * N / nlist * nprobe;   // scores, with lists of one length
+  if (k > 16) return true;
+  if (k > 8) return D <= 768 || n <= 2000000;
+  return nq * nprobe >= 32 && n <= 3000000 && (D <= 512 || (D <= 768 && nq <= 16));
 }
 
 void launch_scan(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream) {
@@ -1341,6 +1400,11 @@ void launch_select_segments(const float* S, int64_t s_stride, int nq, int64_t N,
                             int32_t* cand_r, hipStream_t stream) {
   dim3 grid((unsigned)((N + seg - 1) / seg), (unsigned)nq);
   select_segments_kernel<<<grid, 256, 0, stream>>>(S, s_stride, N, seg, k, cap, cand_v, cand_r);
+}
+
+void launch_select_lists(const float* S, int64_t s_stride, int nq, const int32_t* probes, int nprobe, const int64_t* lbeg, const int64_t* lend,
+                         int k, float* cand_v, int32_t* cand_r, hipStream_t stream) {
+  select_lists_kernel<<<dim3(nprobe, nq), 256, 0, stream>>>(S, s_stride, probes, lbeg, lend, k, cand_v, cand_r);
 }
 
 void launch_search_finish(const float* cand_v, const int32_t* cand_r, const int32_t* cnt, int32_t n_fixed, int32_t cap, int nq,

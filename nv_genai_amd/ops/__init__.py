@@ -1892,8 +1892,8 @@ def search_many_lists(nq: int, rows: int, D: int, k: int, nlist: int, nprobe: in
 def flat_search(q: torch.Tensor, X: torch.Tensor, row_bias: torch.Tensor, ids: torch.Tensor, metric: str,
                 k: int) -> Tuple[torch.Tensor, torch.Tensor]:
     """Top-k of every row of X [N, D] for fp32 queries q [nq, D]: query preparation (normalised for cosine), scan, merge
-    and id lookup in two launches up to 16 queries and three above, one more where scores are written out (k above the register
-    lists: 16, with more than 32 queries 8). Returns (scores [nq, k], external ids [nq, k]; -1 where the
+    and id lookup in two launches up to 16 queries and three above, one more where scores are written out (``scan_scores_flat``, and k
+    above the register lists: 16, with more than 32 queries 8). Returns (scores [nq, k], external ids [nq, k]; -1 where the
     score is not finite)."""
     return tuple(kernels().flat_search(q, X, row_bias, ids, 2.0 if metric == "l2" else 1.0, _METRIC[metric], int(k),
                                        _cu_count(X.device)))
@@ -1903,7 +1903,7 @@ def ivf_search(q: torch.Tensor, X: torch.Tensor, row_bias: torch.Tensor, ids: to
                list_beg: torch.Tensor, list_end: torch.Tensor, metric: str, nprobe: int,
                k: int) -> Tuple[torch.Tensor, torch.Tensor]:
     """``flat_search`` over the rows of the nprobe lists (X in list order) whose centroids have the largest products with
-    the query: two to four launches, no host synchronisation."""
+    the query: two to five launches, no host synchronisation."""
     return tuple(kernels().ivf_search(q, X, row_bias, ids, centroids, list_beg, list_end, 2.0 if metric == "l2" else 1.0,
                                       _METRIC[metric], int(nprobe), int(k), _cu_count(X.device)))
 

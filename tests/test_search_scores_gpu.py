@@ -1,0 +1,79 @@
+"""Searches whose scores go through memory although register lists could hold the results: against 64 bits, with removed rows, vectors that
+are no numbers and lists that begin at any row or are empty."""
+import pytest
+import torch
+
+from nv_genai_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _vectors(rows, D, nq, metric, gpu):
+    g = torch.Generator().manual_seed(rows + D + nq)
+    X = (torch.randn(rows, D, generator=g) / D ** 0.5).to(torch.bfloat16)
+    X[::97] = float("nan")
+    bias = -X.float().pow(2).sum(1).nan_to_num() if metric == "l2" else torch.zeros(rows)
+    bias[torch.rand(rows, generator=g) < 0.1] = float("-inf")   # removed
+    q = torch.randn(nq, D + 8, generator=g)[:, :D] / D ** 0.5
+    return (t.to(gpu) for t in (X, bias, torch.randperm(rows, generator=g), q))
+
+
+def _exact(X, bias, q, metric):
+    qb = (q / q.norm(dim=1, keepdim=True) if metric == "cosine" else q).to(torch.bfloat16).double()
+    S = qb @ X.double().t().contiguous()
+    if metric == "l2":
+        S = 2 * S + bias.double() - q.double().pow(2).sum(1, keepdim=True)
+    return S.masked_fill(S.isnan() | (bias == float("-inf"))[None], float("-inf"))
+
+
+def _check(v, i, S, ids, k):
+    """S: what a query may find. Sums of up to 1,024 products of bf16 in fp32: 1,024 x 2^-24 of the summed magnitudes, at most 4 here."""
+    want = torch.topk(S, k, 1).values
+    live = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(v), live) and torch.equal(i >= 0, live)
+    assert bool(((v.double() - want)[live].abs() <= 2.5e-4).all())
+    back = torch.empty_like(ids).scatter_(0, ids, torch.arange(ids.numel(), device=ids.device))
+    found = S.gather(1, back[i.clamp_min(0)])
+    assert bool(((found - want)[live].abs() <= 5e-4).all())
+    for row, n in zip(i, live.sum(1).tolist()):
+        assert row[:n].unique().numel() == n
+
+
+# groups of 1 to 4 in the scan with queries in LDS and in that with queries in registers; one segment of 8,192 rows, several, a last one of one row
+@pytest.mark.parametrize("D,rows,nq,k,metric", [
+    (128, 8193, 1, 9, "ip"), (384, 24_577, 5, 16, "cosine"), (1024, 2_000, 16, 12, "l2"), (256, 9_000, 17, 10, "cosine"), (896, 8_192, 32, 16, "l2"),
+    (640, 300, 20, 13, "ip"), (768, 49_153, 33, 8, "cosine"), (256, 31_000, 49, 5, "l2"), (384, 24_575, 64, 7, "cosine"),
+    (384, 31, 32, 16, "cosine")])
+def test_flat(gpu, D, rows, nq, k, metric):
+    assert ops.kernels().scan_scores_flat(nq, rows, D, k)
+    X, bias, ids, q = _vectors(rows, D, nq, metric, gpu)
+    v, i = ops.flat_search(q, X, bias, ids, metric, k)
+    _check(v, i, _exact(X, bias, q, metric), ids, k)
+
+
+# lists longer than the selection keeps in registers, short and empty ones; one query of dimensions that the one launch leaves, and of more results
+@pytest.mark.parametrize("D,rows,nlist,nprobe,nq,k,metric", [
+    (640, 20_001, 9, 4, 1, 12, "cosine"), (1024, 30_000, 3, 2, 1, 32, "l2"), (384, 9_001, 40, 17, 2, 5, "ip"), (1024, 7_003, 64, 16, 3, 9, "cosine"),
+    (768, 5_000, 64, 64, 16, 8, "l2"), (128, 50_001, 5, 3, 33, 17, "cosine"), (256, 333, 50, 25, 70, 32, "ip")])
+def test_lists(gpu, D, rows, nlist, nprobe, nq, k, metric):
+    assert ops.kernels().scan_scores_lists(nq, rows, D, k, nlist, nprobe)
+    X, bias, ids, q = _vectors(rows, D, nq, metric, gpu)
+    g = torch.Generator().manual_seed(D)
+    off = torch.cat([torch.tensor([0]), torch.randint(0, rows + 1, (nlist - 1,), generator=g).sort().values, torch.tensor([rows])])
+    order = torch.randperm(nlist, generator=g)
+    beg, end, cent = (t.to(gpu) for t in (off[:-1][order], off[1:][order], torch.randn(nlist, D, generator=g)))
+    v, i = ops.ivf_search(q, X, bias, ids, cent, beg, end, metric, nprobe, k)
+    qb = (q / q.norm(dim=1, keepdim=True) if metric == "cosine" else q).to(torch.bfloat16).double()
+    probes = torch.topk(qb @ cent.to(torch.bfloat16).double().t().contiguous(), nprobe, dim=1).indices
+    at = torch.arange(rows, device=gpu)
+    seen = torch.stack([((at >= beg[p, None]) & (at < end[p, None])).any(0) for p in probes])
+    _check(v, i, _exact(X, bias, q, metric).masked_fill(~seen, float("-inf")), ids, k)
+
+
+def test_lines():
+    """Up to 128 MiB of scores, and what the register lists are faster for."""
+    f, l = ops.kernels().scan_scores_flat, ops.kernels().scan_scores_lists
+    assert f(32, 1 << 20, 384, 16) and not f(33, 1 << 20, 384, 8) and not f(65, 1000, 384, 8) and not f(1, 1000, 384, 8)
+    assert not f(12, 1_000_000, 1024, 14) and f(4, 400_000, 1024, 12) and not f(34, 400_000, 1024, 8) and not f(40, 100_000, 384, 4) and not f(48, 20_000, 768, 8)
+    assert l(32, 1 << 20, 1024, 25, 64, 16) and not l(33, 1 << 20, 1024, 25, 64, 16) and not l(32, 1_000_000, 1024, 8, 64, 16)
+    assert not l(20, 1000, 384, 4, 64, 16) and not l(2, 60_000, 384, 8, 64, 8) and l(12, 60_000, 384, 8, 64, 8)
