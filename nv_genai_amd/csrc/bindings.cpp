@@ -1638,12 +1638,16 @@ std::vector<Tensor> flat_search(Tensor q, Tensor X, Tensor bias, Tensor ids, dou
   const int K = nga::scan_scores_flat(nq, N, D, (int)k) ? 0 : held;
   const bool wide = nga::scan_wide_covers(D, ng);
   const int blocks = wide ? (int)cus : nga::scan_blocks(D, ng, (int)cus);
-  const int64_t tiles = wide ? (N + 31) / 32 : (N + 127) / 128;
+  // one workgroup a CU with up to two tiles: shared out by waves, where that makes no more candidates of 8 or 16 (20k x 768, 4 queries, k 8:
+  // 24.1 us, shared out 24.4)
+  const bool fine = !wide && blocks == cus && (N + 127) / 128 <= 2 * cus && (K == 0 || k <= 4);
+  const int64_t tiles = wide || fine ? (N + 31) / 32 : (N + 127) / 128;
   const int parts = (int)std::min<int64_t>(std::max(1, blocks / items), tiles);
   constexpr int64_t SEG = 8192;
   const int64_t nseg = (N + SEG - 1) / SEG, cap = (K ? parts : nseg) * k;
   Search s = search_begin(q, X, bias, dot_scale, metric, k, cap);
   s.a.parts = parts;
+  s.a.fine = fine;
   Tensor qb, S;
   if (ng == 1) {   // up to 16 queries are prepared by every workgroup, while its first vectors come in
     s.a.qf = q.data_ptr<float>();

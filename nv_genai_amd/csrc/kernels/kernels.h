@@ -218,6 +218,7 @@ struct ScanArgs {
   const ScanItem* items;
   const int32_t *run_item, *qtab;
   int parts;                    // flat (items null): workgroups of a query group
+  int fine;                     // flat: rows are dealt out to waves, 32 at a time
   int k;
   int32_t cap;                  // candidates of a query
   int32_t* cnt;                 // lists: [nq]

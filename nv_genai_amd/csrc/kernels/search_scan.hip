@@ -311,13 +311,15 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
   uint16_t* const slot = smem + w * SLOT;
   // flat: workgroup b takes tiles part, part + parts, ... of query group `item` (neighbouring workgroups read
   // neighbouring tiles: 309 us for 1M x 1024 with the preparation of the query, 311 with one stretch of rows each and
-  // without it). Lists: tiles [g0, g1) of the sequence of all items' tiles
+  // without it). p.fine: its wave w takes the 32-row tiles w parts + part, so many times 4 parts behind it, since with up to two tiles a
+  // CU whole ones leave CUs idle (us, whole / 32 rows: 13k x 1,024, 2 queries, 22.2 19.8; 40k 35.0 32.9; 20k, one query, 22.8 22.3; 40k x 384
+  // 35.8 27.5 with scores; but 250k x 1,024 95.1 96.3). Lists: tiles [g0, g1) of the sequence of all items' tiles
   int item = 0, part = 0;
   int64_t g0 = 0, g1 = 1, stride = 1;
   if (flat) {
     item = blockIdx.x / p.parts;
     part = blockIdx.x % p.parts;
-    stride = p.parts;
+    stride = p.fine ? SS_W * p.parts : p.parts;
   } else {
     const int64_t total = p.run_item[gridDim.x];
     g0 = total * blockIdx.x / gridDim.x;
@@ -326,7 +328,7 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
     item = p.run_item[blockIdx.x];
   }
   for (; g0 < g1; ++item) {
-    int64_t beg = 0, end = p.N, t0 = part, t1 = (p.N + SS_ROWS - 1) / SS_ROWS;
+    int64_t beg = 0, end = p.N, t0 = p.fine ? w * p.parts + part : part, t1 = p.fine ? (p.N + 31) / 32 : (p.N + SS_ROWS - 1) / SS_ROWS;
     int nql;
     if (flat) {
       nql = p.nq - item * SL < SL ? p.nq - item * SL : SL;
@@ -341,12 +343,13 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
       t1 = (g1 < it.tile1 ? g1 : it.tile1) - it.tile0;
       g0 = it.tile0 + t1;
     }
+    auto row_of = [&](int64_t tile) -> int64_t { return p.fine ? tile * 32 : beg + tile * SS_ROWS + w * 32; };
     auto slot_q = [&](int s) -> int { return flat ? item * SL + s : p.qtab[(int64_t)item * SL + s]; };
     const int ngrp = (nql + 15) / 16;
 
     float bnext[2][4], bcur[2][4];
     auto issue = [&](int64_t tile, int c) {
-      const int64_t rbase = beg + tile * SS_ROWS + w * 32;
+      const int64_t rbase = row_of(tile);
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
         const unsigned li = i * 64 + lane, row = li / NC, pos = li % NC;
@@ -445,7 +448,7 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
       }
       if (c == nchx - 1) {
         // acc[i][g][rr]: row tile + 16 i + 4 h + rr, query slot 16 g + col
-        const int64_t rbase = beg + t * SS_ROWS + w * 32;
+        const int64_t rbase = row_of(t);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           const int64_t rb = rbase + 16 * i + 4 * h;

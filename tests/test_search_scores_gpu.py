@@ -77,3 +77,13 @@ def test_lines():
     assert not f(12, 1_000_000, 1024, 14) and f(4, 400_000, 1024, 12) and not f(34, 400_000, 1024, 8) and not f(40, 100_000, 384, 4) and not f(48, 20_000, 768, 8)
     assert l(32, 1 << 20, 1024, 25, 64, 16) and not l(33, 1 << 20, 1024, 25, 64, 16) and not l(32, 1_000_000, 1024, 8, 64, 16)
     assert not l(20, 1000, 384, 4, 64, 16) and not l(2, 60_000, 384, 8, 64, 8) and l(12, 60_000, 384, 8, 64, 8)
+
+
+# rows that are dealt out to waves: fewer 32-row tiles than workgroups, one for some waves, two for some; and from 65,537 rows on to workgroups
+@pytest.mark.parametrize("D,rows,nq,k,metric", [(1024, 1, 1, 1, "ip"), (384, 33, 3, 4, "cosine"), (768, 8_193, 2, 3, "l2"), (1024, 16_384, 16, 4, "cosine"),
+                                                (512, 32_769, 5, 2, "ip"), (384, 65_536, 1, 4, "l2"), (384, 65_537, 1, 4, "l2"), (1024, 20_000, 9, 25, "cosine")])
+def test_flat_of_few_rows(gpu, D, rows, nq, k, metric):
+    X, bias, ids, q = _vectors(rows, D, nq, metric, gpu)
+    X = X.nan_to_num()
+    v, i = ops.flat_search(q, X, bias, ids, metric, k)
+    _check(v, i, _exact(X, bias, q, metric), ids, k)
