@@ -523,6 +523,74 @@ void stream_gemm(Tensor out, Tensor x, Tensor w, int64_t epi, c10::optional<Tens
                            norm_weight(norm_w, x, epi, "stream_gemm"), (float)eps}, (int)epi, cur_stream(x));
 }
 
+// A decode step of 2 to 16 rows without launches for its norms (gemm_stream.hip, XP). Packed rows are [16 H] bf16, squares' sums
+// [tiles / 4][16][4] fp32 in which only the first M of 16 are defined.
+// xw = x norm_w packed and the squares' sums of x's rows
+std::vector<Tensor> stream_open(Tensor x, Tensor norm_w) {
+  CHECK_BF16(x); CHECK_BF16(norm_w); CHECK_CONTIG(norm_w);
+  TORCH_CHECK(x.dim() == 2 && x.size(0) >= 1 && x.size(0) <= 16 && x.size(1) % 256 == 0 && x.size(1) <= 8192 && x.stride(1) == 1 && x.stride(0) % 8 == 0 &&
+                  norm_w.numel() == x.size(1) && norm_w.device() == x.device() &&
+                  (reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(norm_w.data_ptr())) % 16 == 0, "stream_open: up to 16 rows of 256 n values");
+  Tensor xw = at::empty({16 * x.size(1)}, x.options()), sq = at::empty({64}, x.options().dtype(at::kFloat));
+  nga::launch_stream_open(bfp(x), x.stride(0), bfp(norm_w), (int)x.size(0), (int)x.size(1), bfp(xw), sq.data_ptr<float>(), cur_stream(x));
+  return {xw, sq};
+}
+
+void stream_packed_check(const Tensor& xw, const Tensor& w, int64_t M, int64_t N) {
+  CHECK_DEV(xw); CHECK_BF16(xw); CHECK_CONTIG(xw); CHECK_BF16(w); CHECK_CONTIG(w);
+  TORCH_CHECK(w.dim() == 2 && M >= 1 && M <= 16 && w.size(1) % 256 == 0 && w.size(1) >= 256 && N % 64 == 0 && N >= 64 && N < (int64_t(1) << 24) &&
+                  xw.numel() == 16 * w.size(1) && xw.device() == w.device() &&
+                  (reinterpret_cast<uintptr_t>(xw.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) % 16 == 0, "stream: packed rows and w [N, K]");
+}
+
+// the normed rows' product with w: fp32 [M, N] (epi 1), or SwiGLU of [gate | up], packed (epi 2)
+Tensor stream_normed(Tensor xw, Tensor sq, int64_t M, Tensor w, int64_t epi, double eps) {
+  TORCH_CHECK(epi == 1 || (epi == 2 && w.size(0) % 2 == 0), "stream_normed: epi 1 or 2");
+  const int64_t N = epi == 2 ? w.size(0) / 2 : w.size(0);
+  stream_packed_check(xw, w, M, N);
+  CHECK_DEV(sq); CHECK_DT(sq, at::kFloat); CHECK_CONTIG(sq);
+  TORCH_CHECK(sq.numel() % 64 == 0 && sq.numel() >= 64 && sq.device() == xw.device(), "stream_normed: squares' sums");
+  Tensor out = epi == 2 ? at::empty({16 * N}, xw.options()) : at::empty({M, N}, sq.options());
+  nga::StreamGemmParams p{bfp(xw), 0, bfp(w), (int)M, (int)N, (int)w.size(1), out.data_ptr(), N, nullptr, (float)eps};
+  p.packed = 1;
+  p.sq = sq.data_ptr<float>();
+  p.n_sq = (int)(sq.numel() / 16);
+  nga::launch_stream_gemm(p, (int)epi, cur_stream(xw));
+  return out;
+}
+
+// resid += x w^T of rows [M, K] or packed ones; with next_w the packed rows times it and their squares' sums
+std::vector<Tensor> stream_add(Tensor resid, Tensor x, Tensor w, c10::optional<Tensor> next_w) {
+  CHECK_DEV(resid); CHECK_BF16(resid); CHECK_BF16(x);
+  TORCH_CHECK(resid.dim() == 2 && w.dim() == 2 && resid.size(1) == w.size(0) && resid.stride(1) == 1 && resid.stride(0) % 4 == 0 &&
+                  reinterpret_cast<uintptr_t>(resid.data_ptr()) % 16 == 0 && resid.device() == x.device(), "stream_add: resid [M, N]");
+  const int64_t M = resid.size(0), N = w.size(0), K = w.size(1);
+  const bool packed = x.dim() == 1;
+  if (packed) {
+    stream_packed_check(x, w, M, N);
+  } else {
+    CHECK_DEV(x); CHECK_BF16(w); CHECK_CONTIG(w);
+    TORCH_CHECK(x.dim() == 2 && x.size(0) == M && x.size(1) == K && M >= 1 && M <= 16 && K % 256 == 0 && N % 64 == 0 && x.stride(1) == 1 &&
+                    x.stride(0) % 8 == 0 && x.device() == w.device() &&
+                    (reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) % 16 == 0, "stream_add: rows at 16-byte addresses");
+  }
+  nga::StreamGemmParams p{bfp(x), packed ? 0 : x.stride(0), bfp(w), (int)M, (int)N, (int)K, resid.data_ptr(), resid.stride(0), nullptr, 0.f};
+  p.packed = packed;
+  Tensor xw, sq;
+  if (next_w.has_value()) {
+    CHECK_BF16(*next_w); CHECK_CONTIG(*next_w);
+    TORCH_CHECK(next_w->numel() == N && next_w->device() == x.device() && reinterpret_cast<uintptr_t>(next_w->data_ptr()) % 8 == 0, "stream_add: the next norm's weights [N]");
+    xw = at::empty({16 * N}, x.options());
+    sq = at::empty({N}, x.options().dtype(at::kFloat));   // N / 16 tiles of 16 rows
+    p.xw = bfp(xw);
+    p.sq_out = sq.data_ptr<float>();
+    p.next_w = bfp(*next_w);
+  }
+  nga::launch_stream_gemm(p, 3, cur_stream(x));
+  if (!next_w.has_value()) return {};
+  return {xw, sq};
+}
+
 // x [M, K] . w [K, N], rows of x at any multiple of 8 values; xt: x^T . w of x [K, M], both operands' rows so, any K
 Tensor gemm_kn(Tensor x, Tensor w, bool xt) {
   CHECK_DEV(x); CHECK_BF16(x); CHECK_BF16(w);
@@ -3022,6 +3090,9 @@ PYBIND11_MODULE(_C, m) {
   m.def("splitk_reduce", checked("splitk_reduce", &splitk_reduce));
   m.def("splitk_swiglu", checked("splitk_swiglu", &splitk_swiglu));
   m.def("stream_gemm", checked("stream_gemm", &stream_gemm));
+  m.def("stream_open", on_device(&stream_open));
+  m.def("stream_normed", on_device(&stream_normed));
+  m.def("stream_add", on_device(&stream_add));
   m.def("stream_gemm_reads_ahead", &nga::stream_gemm_reads_ahead);
   m.def("stream_gemm_covers", &nga::stream_gemm_covers);
   m.def("gemv", checked("gemv", &gemv));

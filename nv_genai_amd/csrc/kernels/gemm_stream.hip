@@ -30,11 +30,16 @@ __device__ __forceinline__ float st_silu(float x) { return x / (1.f + __expf(-x)
 }  // namespace
 
 // EPI 0: bf16 out; 1: fp32 out; 2: bf16 silu(gate) up of W = [gate | up] rows, N = F (8 NT features a tile); 3: bf16 out += product
+// XP: a layer of 2 to 16 rows without launches for its norms. What adds to the residual (epi 3) leaves the rows times the next norm's
+// weights, packed as the next projection's operand wants them, and the squares' sum of each row over its features; that projection's sums
+// are multiplied by the rows' 1 / rms at the end. A bf16 rounding of x w for one of x w / rms, the squares in fp32 as before. 8B, us at 2 /
+// 8 / 16 rows, with rows as they lie and without norms / so: q/k/v 10.5 10.9 11.8 / 11.3 11.3 11.8, output 7.0 7.2 8.1 / 7.5 7.6 8.8, SwiGLU
+// 38.5 39.7 44.3 / 38.5 38.6 41.9, down 21.3 22.5 26.7 (and 22.4 in slabs) / 21.8 21.8 23.5; each of the two norms was a launch of 4.6 to 4.8.
 // NJ > 0: the one row is normed first (RMSNorm, K <= 512 NJ), while the first two stages are under way. Each wave sums the row's
 // squares by itself and lays the K range that it multiplies in its own part of LDS, so that none waits for another. It takes the
 // place of a launch of 4.6 us (6,144 x 4,096: 10.0 us, with the norm 12.1); for two rows it costs what it saves (SwiGLU 2 x 14,336 x
 // 4,096: 38.3, with the norm 43.0), since every workgroup reads them whole.
-template <int NT, int EPI, int NJ>
+template <int NT, int EPI, int NJ, bool XP>
 __global__ void __launch_bounds__(256) stream_gemm_kernel(StreamGemmParams P) {
   constexpr int NW = 4;
   constexpr int KS = 256 / NT, CPR = KS / 8, KSTEPS = KS / 32;   // k of a stage, its 16-byte chunks a row, its MFMA steps
@@ -54,7 +59,7 @@ __global__ void __launch_bounds__(256) stream_gemm_kernel(StreamGemmParams P) {
     const int64_t row = EPI == 2 ? (r < hr ? (int64_t)tile * hr + r : (int64_t)P.N + tile * hr + r - hr) : (int64_t)tile * 16 * NT + r;
     wsrc[i] = P.w + row * P.K + ((lane % CPR ^ (r & 15)) << 3);
   }
-  const uint16_t* xp = P.x + (int64_t)min(col, P.M - 1) * P.ldx + 8 * h;
+  const uint16_t* xp = XP ? P.x + (16 * h + min(col, P.M - 1)) * 8 : P.x + (int64_t)min(col, P.M - 1) * P.ldx + 8 * h;
   uint16_t* buf = ring + wv * (2 * 4096);
 
   auto issue = [&](int s) {
@@ -65,7 +70,7 @@ __global__ void __launch_bounds__(256) stream_gemm_kernel(StreamGemmParams P) {
   const uint16_t* xl = ring + XS + 8 * h;
   auto load_x = [&](int s, u16x8 (&x)[KSTEPS]) {
 #pragma unroll
-    for (int k = 0; k < KSTEPS; ++k) x[k] = NJ ? *reinterpret_cast<const u16x8*>(xl + s * KS + 32 * k) : load8(xp + (int64_t)s * KS + 32 * k);
+    for (int k = 0; k < KSTEPS; ++k) x[k] = NJ ? *reinterpret_cast<const u16x8*>(xl + s * KS + 32 * k) : load8(xp + (XP ? (s * KSTEPS + k) * 512 : s * KS + 32 * k));
   };
   constexpr int XV = NJ ? 0 : KSTEPS;   // loads of token rows in flight
   f32x4 acc[NT];
@@ -96,6 +101,44 @@ __global__ void __launch_bounds__(256) stream_gemm_kernel(StreamGemmParams P) {
     st_wait_vm<8 + XV>();
     multiply(s, x);
   };
+  // what the end needs, asked for first by the wave that adds up: the rows' squares (shared out over the waves the launch was 0.4 us
+  // longer), the residual that the product is added to, the next norm's weights
+  constexpr int SQ = 16;
+  f32x4 sv[SQ];
+  u16x4 res[NT], nw_next[NT];
+  const int groups = XP ? P.n_sq >> 2 : 0;
+  if (wv == 0) {
+    if constexpr (XP) {
+      if (P.sq != nullptr)
+#pragma unroll
+        for (int i = 0; i < SQ; ++i) {
+          const int g = h + 4 * i;
+          sv[i] = g < groups ? *reinterpret_cast<const f32x4*>(P.sq + (g * 16 + col) * 4) : (f32x4)(0.f);
+        }
+    }
+    if constexpr (EPI == 3) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        const int n = 16 * (NT * tile + i) + 4 * h;
+        res[i] = *reinterpret_cast<const u16x4*>(reinterpret_cast<const uint16_t*>(P.out) + (int64_t)min(col, P.M - 1) * P.ldo + n);
+        nw_next[i] = P.xw != nullptr ? *reinterpret_cast<const u16x4*>(P.next_w + n) : (u16x4)(0);
+      }
+    }
+  }
+  auto squares = [&]() {   // 1 / rms of row `col`
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < SQ; ++i) ss += (sv[i][0] + sv[i][1]) + (sv[i][2] + sv[i][3]);
+    for (int g = h + 4 * SQ; g < groups; g += 4) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(P.sq + (g * 16 + col) * 4);
+      ss += (v[0] + v[1]) + (v[2] + v[3]);
+    }
+    ss += __shfl_xor(ss, 16, 64);
+    ss += __shfl_xor(ss, 32, 64);
+    return rsqrtf(ss / (float)P.K + P.eps);
+  };
+  float scale = 1.f;
+  if (XP && s0 >= s1 && wv == 0 && P.sq != nullptr) scale = squares();   // a K of fewer stages than waves
   u16x8 xa[KSTEPS], xb[KSTEPS];
   if (s0 < s1) {
     int s = s0;
@@ -133,6 +176,7 @@ __global__ void __launch_bounds__(256) stream_gemm_kernel(StreamGemmParams P) {
       __builtin_amdgcn_sched_barrier(0);
       issue(s0);
       __builtin_amdgcn_sched_barrier(0);
+      if (XP && wv == 0 && P.sq != nullptr) scale = squares();
     }
     // the last steps apart: a branch around the loads would make the compiler wait for all of them
     for (; s + 2 < s1; s += 2) {
@@ -161,7 +205,7 @@ __global__ void __launch_bounds__(256) stream_gemm_kernel(StreamGemmParams P) {
     f32x4 v = (f32x4)(0.f);
 #pragma unroll
     for (int u = 0; u < NW; ++u) v += *reinterpret_cast<const f32x4*>(part + ((u * NT + i) * 64 + lane) * 4);
-    acc[i] = v;
+    acc[i] = XP ? v * scale : v;
   }
   if constexpr (EPI == 2) {
     float up[4];
@@ -171,7 +215,28 @@ __global__ void __launch_bounds__(256) stream_gemm_kernel(StreamGemmParams P) {
     u16x4 o;
 #pragma unroll
     for (int r = 0; r < 4; ++r) o[r] = f2bf(st_silu(acc[0][r]) * up[r]);
-    *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + (int64_t)col * P.ldo + 8 * NT * tile + 4 * h) = o;
+    const int n = 8 * NT * tile + 4 * h;
+    *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + (XP ? packed_at(col, n, P.N) : (int64_t)col * P.ldo + n)) = o;
+  } else if constexpr (EPI == 3) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int t = NT * tile + i, n = 16 * t + 4 * h;
+      u16x4 o, y;
+      float ss = 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        o[r] = f2bf(bf2f(res[i][r]) + acc[i][r]);
+        const float x = bf2f(o[r]);
+        y[r] = f2bf(x * bf2f(nw_next[i][r]));
+        ss = __builtin_fmaf(x, x, ss);
+      }
+      if (col < P.M) *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + (int64_t)col * P.ldo + n) = o;
+      if (P.xw == nullptr) continue;
+      ss += __shfl_xor(ss, 16, 64);
+      ss += __shfl_xor(ss, 32, 64);
+      if (col < P.M) *reinterpret_cast<u16x4*>(P.xw + packed_at(col, n, P.N)) = y;
+      if (h == 0) P.sq_out[((t >> 2) * 16 + col) * 4 + (t & 3)] = ss;
+    }
   } else {
     if (col >= P.M) return;
 #pragma unroll
@@ -180,12 +245,10 @@ __global__ void __launch_bounds__(256) stream_gemm_kernel(StreamGemmParams P) {
       if constexpr (EPI == 1) {
         *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(P.out) + at) = acc[i];
       } else {
-        u16x4* to = reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + at);
         u16x4 o;
-        if constexpr (EPI == 3) o = *to;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = f2bf(EPI == 3 ? bf2f(o[r]) + acc[i][r] : acc[i][r]);
-        *to = o;
+        for (int r = 0; r < 4; ++r) o[r] = f2bf(acc[i][r]);
+        *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(P.out) + at) = o;
       }
     }
   }
@@ -229,10 +292,19 @@ bool stream_gemm_reads_ahead(int64_t M, int64_t N, int64_t K) {
 void launch_stream_gemm(const StreamGemmParams& p, int epi, hipStream_t stream) {
   const int t = (int)st_tiles(p.N, epi == 2);
   if (p.M == 0 || t == 0) return;
-  const bool two = st_two(p.M, p.N, t);
+  const bool two = st_two(p.packed ? 1 : p.M, p.N, t);   // packed rows cost no more at 16 than at 8
 #define NGA_ST(EPI, NJ)                                                                  \
-  if (two) stream_gemm_kernel<2, EPI, NJ><<<t / 2, 256, 0, stream>>>(p);                 \
-  else stream_gemm_kernel<1, EPI, NJ><<<t, 256, 0, stream>>>(p)
+  if (two) stream_gemm_kernel<2, EPI, NJ, false><<<t / 2, 256, 0, stream>>>(p);          \
+  else stream_gemm_kernel<1, EPI, NJ, false><<<t, 256, 0, stream>>>(p)
+#define NGA_SP(EPI)                                                                      \
+  if (two) stream_gemm_kernel<2, EPI, 0, true><<<t / 2, 256, 0, stream>>>(p);            \
+  else stream_gemm_kernel<1, EPI, 0, true><<<t, 256, 0, stream>>>(p)
+  if (p.packed) {
+    if (epi == 1) { NGA_SP(1); }
+    else if (epi == 2) { NGA_SP(2); }
+    else { NGA_SP(3); }
+    return;
+  }
   if (p.norm_w != nullptr && p.K <= 4096) {
     if (epi == 1) { NGA_ST(1, 8); }
     else { NGA_ST(2, 8); }
@@ -243,7 +315,34 @@ void launch_stream_gemm(const StreamGemmParams& p, int epi, hipStream_t stream) 
   else if (epi == 1) { NGA_ST(1, 0); }
   else if (epi == 2) { NGA_ST(2, 0); }
   else { NGA_ST(3, 0); }
+#undef NGA_SP
 #undef NGA_ST
+}
+
+// xw = x norm_w in bf16, packed, and the squares' sum of each row, as the epilogue above leaves them, in one group of four
+__global__ void __launch_bounds__(1024) stream_open_kernel(const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ norm_w, int H,
+                                                           uint16_t* __restrict__ xw, float* __restrict__ sq) {
+  __shared__ float red[16];
+  const int row = blockIdx.x, c = threadIdx.x * 8;
+  float ss = 0.f;
+  if (c < H) {
+    const u16x8 v = load8(x + row * ldx + c), w = load8(norm_w + c);
+    u16x8 o;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float a = bf2f(v[i]);
+      o[i] = f2bf(a * bf2f(w[i]));
+      ss = __builtin_fmaf(a, a, ss);
+    }
+    store8(xw + packed_at(row, c, H), o);
+  }
+  ss = block_sum(ss, red);
+  if (threadIdx.x < 4) sq[row * 4 + threadIdx.x] = threadIdx.x ? 0.f : ss;
+}
+
+void launch_stream_open(const uint16_t* x, int64_t ldx, const uint16_t* norm_w, int M, int H, uint16_t* xw, float* sq, hipStream_t stream) {
+  if (M == 0) return;
+  stream_open_kernel<<<M, (H / 8 + 63) / 64 * 64, 0, stream>>>(x, ldx, norm_w, H, xw, sq);
 }
 
 }  // namespace nga

@@ -301,6 +301,40 @@ def linear_add_(resid: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> torch.
     return resid
 
 
+def stream_layer_covers(resid: torch.Tensor, attn_norm, wqkv, wo, mlp_norm, wgu, wd) -> bool:
+    """Whether a decode layer of 2 to 16 rows runs as ``stream_open`` / ``stream_normed`` / ``stream_add_``, without launches for its norms:
+    where the stream kernel is each projection's, and down's of up to 256 tiles at 9 to 16 rows too, which packed rows make level with the
+    K-split one (4,096 x 14,336 at 16 rows: 22.4 us and a sum of slabs, packed 23.5)."""
+    M = resid.shape[0]
+    if not (2 <= M <= 16 and _gpu(resid) and resid.dtype == torch.bfloat16 and resid.stride(1) == 1 and resid.stride(0) % 8 == 0
+            and resid.data_ptr() % 16 == 0 and resid.shape[1] % 256 == 0 and resid.shape[1] <= 8192):
+        return False
+    ws = (attn_norm, wqkv, wo, mlp_norm, wgu, wd)
+    if not all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0 and t.device == resid.device for t in ws):
+        return False
+    covers, F = kernels().stream_gemm_covers, wd.shape[1]
+    return (wgu.shape[0] == 2 * F and all(n % 64 == 0 for n in (wqkv.shape[0], wo.shape[0], F)) and wo.shape[1] % 256 == 0
+            and covers(M, wqkv.shape[0], wqkv.shape[1], False) and covers(M, wo.shape[0], wo.shape[1], False)
+            and covers(M, F, wgu.shape[1], True) and covers(min(M, 8) if F > 4096 else M, wd.shape[0], F, False))
+
+
+def stream_open(x: torch.Tensor, norm_w: torch.Tensor):
+    """What ``stream_normed`` takes of rows x [M <= 16, H]: x norm_w packed, and the rows' squares."""
+    return tuple(kernels().stream_open(x, norm_w))
+
+
+def stream_normed(rows, M: int, w: torch.Tensor, eps: float, epi: int) -> torch.Tensor:
+    """rmsnorm(rows) @ w^T: fp32 [M, N] (``epi`` 1), or SwiGLU, packed (2)."""
+    return kernels().stream_normed(*rows, M, w, int(epi), float(eps))
+
+
+def stream_add_(resid: torch.Tensor, x: torch.Tensor, w: torch.Tensor, next_w: Optional[torch.Tensor] = None):
+    """resid += x @ w^T of rows [M, K] or packed ones (fp32 sums, one bf16 rounding of the residual); what ``stream_normed`` takes of the new
+    rows under the norm ``next_w``, None without one."""
+    got = kernels().stream_add(resid, x, w, next_w)
+    return tuple(got) if got else None
+
+
 def splitk_reduce(P: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """bf16 sum of the K-split partial slabs P [S, M, N]."""
     S, M, N = P.shape
