@@ -1702,9 +1702,9 @@ std::vector<Tensor> flat_search(Tensor q, Tensor X, Tensor bias, Tensor ids, dou
   TORCH_CHECK(cus >= 1 && cus <= 4096, "flat_search: compute units");
   const int64_t nq = q.size(0), N = X.size(0);
   const int D = (int)X.size(1), ng = nq <= 16 ? 1 : nq <= 32 ? 2 : nq <= 48 ? 3 : 4;
-  const int items = (int)((nq + 16 * ng - 1) / (16 * ng)), held = nga::scan_list((int)k, ng, false);
-  const int K = nga::scan_scores_flat(nq, N, D, (int)k) ? 0 : held;
-  const bool wide = nga::scan_wide_covers(D, ng);
+  const int items = (int)((nq + 16 * ng - 1) / (16 * ng));
+  const bool wide = ng > 1 && nga::scan_wide_covers(D, ng);
+  const int held = nga::scan_list((int)k, ng, false), K = nga::scan_scores_flat(nq, N, D, (int)k) ? 0 : held;
   const int blocks = wide ? (int)cus : nga::scan_blocks(D, ng, (int)cus);
   // one workgroup a CU with up to two tiles: shared out by waves, where that makes no more candidates of 8 or 16 (20k x 768, 4 queries, k 8:
   // 24.1 us, shared out 24.4)

@@ -559,16 +559,25 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
 // k 4: 200 240 315, 183 218 272; x 640, 33 / 64: 287 371, 232 285; x 896, 17 / 33 / 64: 316 358 451, 267 283 343; x 256, 17 / 64: 153 245, 140 228.
 // Of 128 dimensions two barriers for 8 KB cost more than the smaller queries in LDS (1M, 17 / 33 / 64: 77 111 103, here 126 175 215); left there
 // too are 33 to 48 queries of 256 (1M 178, 189; 100k 41, 36) and 17 to 32 of 640 (1M 207, 214; 100k 39, 36). Each dimension takes its own registers.
+// Where results are kept in lists, four more waves (wide_apart) take the sums in: inserting, some 10 operations a place of the list whenever one of
+// 64 lanes takes a value in, then no longer holds up the DMA and the products of the next tile. Us, whole search, in the stream's waves / apart:
+// k 4, 64 queries: 1M x 1,024 341 318, 600k x 896 224 174, 900k x 512 246 180, 130k x 384 52 45, 10k x 768 22.9 22.4; 33 queries: 900k x 512
+// 197 156; 20 queries: 130k x 384 36.6 33.2; k 8: 250k x 1,024, 64 queries, 146 105, 600k x 896, 40 queries, 235 187, 900k x 512, 20 queries, 195 160;
+// k 12, 20 queries: 600k x 768 226 162, 60k x 1,024 47 44. Writing scores so gains nothing (it is the memory's time: 33 x 250k x 1,024 124 126, 64 x 1M 479
+// 502); lists of 32, or of 16 for more than 32 queries, remain slower than scores (33 x 900k x 512, k 12, 223 372).
 namespace {
-constexpr int WIDE_BIAS = 8;   // tiles whose biases have a place, more than are under way
+constexpr int WIDE_BIAS = 8;   // where the stream's waves take the sums in: tiles whose biases have a place, more than are under way
 // which numbers of groups (NG) it takes of 128 KS dimensions
 constexpr bool wide_takes(int KS, int NG) { return NG >= 2 && NG <= 4 && KS >= 2 && KS <= 8 && !(KS == 2 && NG == 3) && !(KS == 5 && NG == 2); }
 // units of 4 KS KiB for all waves that fill the LDS beside the sums and the biases, ten at most (384 dimensions, 33 queries: 205 us with ten and
 // 213 with eleven)
-constexpr int wide_slots(int KS, int NG) {
-  const int n = (160 - 8 * NG - WIDE_BIAS / 4) / (4 * KS);
+constexpr int wide_slots(int KS, int NG, bool apart) {
+  const int n = (160 - 8 * NG - (apart ? 0 : WIDE_BIAS / 4)) / (4 * KS);
   return n < 10 ? n : 10;
 }
+// whether waves of their own take the sums in: lists do not hold up the stream then. Not where it is what bounds: 1M x 1,024, k 4, 20 / 33 queries, in
+// the stream's waves / apart, 315 311 / 323 323; 64 queries 345 / 318, k 8, 20 queries 250k 97 / 98
+constexpr bool wide_apart(int NG, int K, int KS) { return K > 0 && !(KS == 8 && K == 4 && NG < 4); }
 constexpr int wide_swizzle(int KS) { return KS % 4 == 0 ? 15 : KS % 2 == 0 ? 7 : 3; }
 template <int N>
 __device__ __forceinline__ void wide_wait() {
@@ -584,58 +593,23 @@ __device__ __forceinline__ void wide_store(float* p, f32x4 v) {
 __device__ __forceinline__ void wide_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 }  // namespace
 
-static size_t wide_lds(int NG, int KS) { return (size_t)SS_W * wide_slots(KS, NG) * KS * 1024 + 8192 * NG + WIDE_BIAS * SS_W * 64; }
+static size_t wide_lds(int NG, int KS, bool apart) {
+  return (size_t)SS_W * wide_slots(KS, NG, apart) * KS * 1024 + 8192 * NG + (apart ? 0 : WIDE_BIAS * SS_W * 64);
+}
 
 template <int NG, int K, int KS>
-__global__ void __launch_bounds__(256, 1) scan_wide_kernel(ScanArgs p) {
-  constexpr int SL = 16 * NG, NSL = wide_slots(KS, NG), UNIT = 512 * KS, NC = 4 * KS, SW = wide_swizzle(KS), GW = (NG + 1) / 2;
+__global__ void __launch_bounds__(wide_apart(NG, K, KS) ? 512 : 256, 1) scan_wide_kernel(ScanArgs p) {
+  constexpr bool APART = wide_apart(NG, K, KS);
+  constexpr int SL = 16 * NG, NSL = wide_slots(KS, NG, APART), UNIT = 512 * KS, NC = 4 * KS, SW = wide_swizzle(KS), GW = (NG + 1) / 2;
   constexpr int KR = K > 0 ? K : 1;
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   float* const xch = reinterpret_cast<float*>(smem + SS_W * NSL * UNIT);
-  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave % SS_W;
   const int col = lane & 15, h = lane >> 4;
   const int D = 128 * KS;
-  uint16_t* const ring = smem + w * NSL * UNIT;
-  float* const bias_s = xch + 2048 * NG + w * 16;   // [WIDE_BIAS][SS_W][16]
   const int item = blockIdx.x / p.parts, part = blockIdx.x % p.parts;
   const int nql = p.nq - item * SL < SL ? p.nq - item * SL : SL, ngrp = (nql + 15) / 16;
   const int tiles = (int)((p.N + 31) / 32), nt = part < tiles ? (tiles - 1 - part) / p.parts + 1 : 0, units = 2 * nt;
-
-  bf16x8 bq[NG][KS];
-#pragma unroll
-  for (int g = 0; g < NG; ++g)
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      u16x8 v = load8(p.Q + packed_at(item * SL + 16 * g + col, w * (D / 4) + 32 * s + 8 * h, D));
-      bq[g][s] = as_bf16x8(16 * g + col < nql ? v : (u16x8)(0));
-    }
-  int off[KS], row[KS];   // of this lane's 16 bytes of instruction i: chunk c of row r lies at c ^ (r & SW)
-#pragma unroll
-  for (int i = 0; i < KS; ++i) {
-    const int li = 64 * i + lane;
-    row[i] = li / NC;
-    off[i] = w * (D / 4) + (((li % NC) ^ (row[i] & SW)) << 3);
-  }
-  auto issue = [&](int u, bool first) {   // first: of a tile, whose biases come before it
-    const int64_t rbase = (part + (int64_t)(u >> 1) * p.parts) * 32 + (u & 1) * 16;
-    if (first && lane < 16) {
-      const int64_t r = rbase + 16 * (w & 1) + lane;
-      __builtin_amdgcn_global_load_lds((gptr_t)(p.bias + (r < p.N ? r : p.N - 1)), (lptr_t)(bias_s + ((u >> 1) % WIDE_BIAS) * (SS_W * 16)), 4, 0, 0);
-    }
-    uint16_t* to = ring + (u % NSL) * UNIT;
-#pragma unroll
-    for (int i = 0; i < KS; ++i) {
-      const int64_t r = rbase + row[i];
-      __builtin_amdgcn_global_load_lds((gptr_t)(p.X + (r < p.N ? r : p.N - 1) * D + off[i]), (lptr_t)(to + i * 512), 16, 0, 2);
-    }
-  };
-#pragma unroll
-  for (int u = 0; u < NSL; ++u) issue(u, u % 2 == 0);
-  // the queries are used here, so that the compiler's wait for them lies before the loop
-#pragma unroll
-  for (int g = 0; g < NG; ++g)
-#pragma unroll
-    for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(bq[g][s]));
 
   float tv[GW][KR];
   int tr[GW][KR];
@@ -646,30 +620,9 @@ __global__ void __launch_bounds__(256, 1) scan_wide_kernel(ScanArgs p) {
       tv[g][j] = -INFINITY;
       tr[g][j] = -1;
     }
-  f32x4 acc[2][NG];
-  auto multiply = [&](int u, int i) {
-    const uint16_t* from = ring + (u % NSL) * UNIT + col * (NC * 8);
-    u16x8 a[KS];
-#pragma unroll
-    for (int s = 0; s < KS; ++s) a[s] = *reinterpret_cast<const u16x8*>(from + (((4 * s + h) ^ (col & SW)) << 3));
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the unit's place is free
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int g = 0; g < NG; ++g) acc[i][g] = (f32x4)(0.f);
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int g = 0; g < NG; ++g) acc[i][g] = mfma16(as_bf16x8(a[s]), bq[g][s], acc[i][g]);
-  };
-  auto finish = [&](int n) {   // tile n of this workgroup
-    wide_barrier();   // the sums of the tile before have been read
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int g = 0; g < NG; ++g) wide_store(xch + (((w * 2 + i) * NG + g) * 64 + lane) * 4, acc[i][g]);
-    wide_barrier();
+  // the sums of tile n: rows 16 (w & 1) .. of it and every second group, with the biases b of this lane's four rows
+  auto take = [&](int n, const f32x4 b) {
     const int64_t rb = (part + (int64_t)n * p.parts) * 32 + 16 * (w & 1) + 4 * h;
-    const f32x4 b = *reinterpret_cast<const f32x4*>(bias_s + (n % WIDE_BIAS) * (SS_W * 16) + 4 * h);
 #pragma unroll
     for (int gg = 0; gg < GW; ++gg) {
       const int g = 2 * gg + (w >> 1);
@@ -696,26 +649,103 @@ __global__ void __launch_bounds__(256, 1) scan_wide_kernel(ScanArgs p) {
       }
     }
   };
-  // younger than unit u when its turn comes: the NSL - 1 units behind it, a bias before each even one. Stores of scores are not
-  // counted: they may be done before older loads
-  static_assert(NSL / 2 + 2 <= WIDE_BIAS, "biases under way and of the tile in hand lie apart");
-  constexpr int Y0 = (NSL - 1) * KS + (NSL - 1) / 2, Y1 = (NSL - 1) * KS + NSL / 2;
-  int n = 0;
-  for (; 2 * n + 1 + NSL < units; ++n) {
-    wide_wait<Y0>();
-    multiply(2 * n, 0);
-    issue(2 * n + NSL, NSL % 2 == 0);
-    wide_wait<Y1>();
-    multiply(2 * n + 1, 1);
-    issue(2 * n + 1 + NSL, NSL % 2 == 1);
-    finish(n);
-  }
-  for (; n < nt; ++n) {   // the last units: nothing more to ask for, but one unit if it is the ring's first place that is missing
-    wide_wait<0>();
-    multiply(2 * n, 0);
-    if (2 * n + NSL < units) issue(2 * n + NSL, NSL % 2 == 0);
-    multiply(2 * n + 1, 1);
-    finish(n);
+  if (!APART || wave < SS_W) {
+    float* const bias_s = xch + 2048 * NG + w * 16;   // unless APART: [WIDE_BIAS][SS_W][16]
+    uint16_t* const ring = smem + w * NSL * UNIT;
+    bf16x8 bq[NG][KS];
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        u16x8 v = load8(p.Q + packed_at(item * SL + 16 * g + col, w * (D / 4) + 32 * s + 8 * h, D));
+        bq[g][s] = as_bf16x8(16 * g + col < nql ? v : (u16x8)(0));
+      }
+    int off[KS], row[KS];   // of this lane's 16 bytes of instruction i: chunk c of row r lies at c ^ (r & SW)
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+      const int li = 64 * i + lane;
+      row[i] = li / NC;
+      off[i] = w * (D / 4) + (((li % NC) ^ (row[i] & SW)) << 3);
+    }
+    auto issue = [&](int u, bool first) {   // first: of a tile, whose biases come before it
+      const int64_t rbase = (part + (int64_t)(u >> 1) * p.parts) * 32 + (u & 1) * 16;
+      if (!APART && first && lane < 16) {
+        const int64_t r = rbase + 16 * (w & 1) + lane;
+        __builtin_amdgcn_global_load_lds((gptr_t)(p.bias + (r < p.N ? r : p.N - 1)), (lptr_t)(bias_s + ((u >> 1) % WIDE_BIAS) * (SS_W * 16)), 4, 0, 0);
+      }
+      uint16_t* to = ring + (u % NSL) * UNIT;
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+        const int64_t r = rbase + row[i];
+        __builtin_amdgcn_global_load_lds((gptr_t)(p.X + (r < p.N ? r : p.N - 1) * D + off[i]), (lptr_t)(to + i * 512), 16, 0, 2);
+      }
+    };
+#pragma unroll
+    for (int u = 0; u < NSL; ++u) issue(u, u % 2 == 0);
+    // the queries are used here, so that the compiler's wait for them lies before the loop
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(bq[g][s]));
+
+    f32x4 acc[2][NG];
+    auto multiply = [&](int u, int i) {
+      const uint16_t* from = ring + (u % NSL) * UNIT + col * (NC * 8);
+      u16x8 a[KS];
+#pragma unroll
+      for (int s = 0; s < KS; ++s) a[s] = *reinterpret_cast<const u16x8*>(from + (((4 * s + h) ^ (col & SW)) << 3));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the unit's place is free
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int g = 0; g < NG; ++g) acc[i][g] = (f32x4)(0.f);
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int g = 0; g < NG; ++g) acc[i][g] = mfma16(as_bf16x8(a[s]), bq[g][s], acc[i][g]);
+    };
+    auto finish = [&](int n) {   // tile n of this workgroup
+      wide_barrier();   // the sums of the tile before have been read
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int g = 0; g < NG; ++g) wide_store(xch + (((w * 2 + i) * NG + g) * 64 + lane) * 4, acc[i][g]);
+      wide_barrier();
+      if constexpr (!APART) take(n, *reinterpret_cast<const f32x4*>(bias_s + (n % WIDE_BIAS) * (SS_W * 16) + 4 * h));
+    };
+    // younger than unit u when its turn comes: the NSL - 1 units behind it, a bias before each even one. Stores of scores are not
+    // counted: they may be done before older loads
+    static_assert(APART || NSL / 2 + 2 <= WIDE_BIAS, "biases under way and of the tile in hand lie apart");
+    constexpr int Y0 = (NSL - 1) * KS + (APART ? 0 : (NSL - 1) / 2), Y1 = (NSL - 1) * KS + (APART ? 0 : NSL / 2);
+    int n = 0;
+    for (; 2 * n + 1 + NSL < units; ++n) {
+      wide_wait<Y0>();
+      multiply(2 * n, 0);
+      issue(2 * n + NSL, NSL % 2 == 0);
+      wide_wait<Y1>();
+      multiply(2 * n + 1, 1);
+      issue(2 * n + 1 + NSL, NSL % 2 == 1);
+      finish(n);
+    }
+    for (; n < nt; ++n) {   // the last units: nothing more to ask for, but one unit if it is the ring's first place that is missing
+      wide_wait<0>();
+      multiply(2 * n, 0);
+      if (2 * n + NSL < units) issue(2 * n + NSL, NSL % 2 == 0);
+      multiply(2 * n + 1, 1);
+      finish(n);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the ring is free
+  } else {
+    for (int n = 0; n < nt; ++n) {   // as many barriers as the other waves pass
+      f32x4 b;
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        const int64_t r = (part + (int64_t)n * p.parts) * 32 + 16 * (w & 1) + 4 * h + rr;
+        b[rr] = p.bias[r < p.N ? r : p.N - 1];
+      }
+      wide_barrier();
+      wide_barrier();
+      take(n, b);
+    }
   }
 
   if constexpr (K > 0) {
@@ -724,11 +754,10 @@ __global__ void __launch_bounds__(256, 1) scan_wide_kernel(ScanArgs p) {
       ss_merge_xor<KR>(tv[g], tr[g], 16);
       ss_merge_xor<KR>(tv[g], tr[g], 32);
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     float* mv = reinterpret_cast<float*>(smem);   // [SL][2][K]
     int* mr = reinterpret_cast<int*>(mv + SL * 2 * K);
-    if (h == 0) {
+    if ((!APART || wave >= SS_W) && h == 0) {
 #pragma unroll
       for (int gg = 0; gg < GW; ++gg) {
         const int g = 2 * gg + (w >> 1);
@@ -1278,12 +1307,16 @@ int scan_list(int k, int ng, bool ivf) {
 // twice and the selection a launch. Up to 128 MiB of scores. Whole searches, us, lists / scores:
 // flat, k 12, at 1 / 12 / 28 queries: 100k x 128 44 49 59, 24 32 33; 130k x 384 52 53 57, 38 44 47; 500k x 512 130 144 160, 103 122 124; 300k x 640
 // 105 109 105, 80 97 104; 600k x 768 174 192 236, 160 200 207; 300k x 896 107 108 136, 97 116 124; 400k x 1,024 164 164 176, 144 171 180;
-// 1M x 1,024, k 14, at 1 / 4 / 12: 323 333 339, 326 358 393; 60k 47 48 50, 41 41 43. k 8, at 34 / 64: 130k x 384 62 68, 48 55; 900k x 384 264 331,
-// 197 232; 300k x 640 118 141, 104 119; 600k x 768 212 277, 212 236; 400k x 1,024 164 196, 184 200; 50k x
-// 768 39 44, 36 42; at 48 20k x 768 29, 31
+// 1M x 1,024, k 14, at 1 / 4 / 12: 323 333 339, 326 358 393; 60k 47 48 50, 41 41 43 (more than 16 queries of most dimensions: in scan_wide_kernel's
+// lists by now). k 6, 40 queries, 900k x 256: 266 in scores
+bool scan_wide_covers(int D, int ng) { return D % 128 == 0 && wide_takes(D / 128, ng); }   // flat scans of 17 to 64 queries, prepared
+
 bool scan_scores_flat(int64_t nq, int64_t N, int D, int k) {
   const int64_t n = nq * N;
   if (nq > 64 || n > (int64_t(1) << 25)) return false;
+  // scan_wide_kernel's lists, in waves of their own, cost its stream little: in lists / scores 600k x 768, 20 queries, k 12, 161 208, 33, k 8, 161
+  // 230; 900k x 512, 33, k 8, 222 247; closest 130k x 384, 20, k 12, 51 48
+  if (nq > 16 && scan_wide_covers(D, nq <= 32 ? 2 : nq <= 48 ? 3 : 4)) return false;
   if (nq > 32) return k > 4 && k <= 8 && D >= 256 && D <= 768 && n >= 1500000;
   if (k <= 8 || k > 16) return false;
   return D <= 640 || n <= 2000000 || (D <= 768 && n <= 5000000) || (nq > 16 && D <= 896);
@@ -1347,9 +1380,6 @@ void launch_ivf_one(const ScanArgs& a, const IvfLists& l, int blocks, hipStream_
   }
 }
 
-// 17 to 64 queries of all rows, prepared
-bool scan_wide_covers(int D, int ng) { return D % 128 == 0 && wide_takes(D / 128, ng); }
-
 template <int NG, int K, int KS>
 static void wide_go(const ScanArgs& a, int blocks, hipStream_t stream) {
   if constexpr (wide_takes(KS, NG)) {
@@ -1359,7 +1389,7 @@ static void wide_go(const ScanArgs& a, int blocks, hipStream_t stream) {
       return true;
     }();
     (void)attr;
-    scan_wide_kernel<NG, K, KS><<<blocks, 256, wide_lds(NG, KS), stream>>>(a);
+    scan_wide_kernel<NG, K, KS><<<blocks, wide_apart(NG, K, KS) ? 512 : 256, wide_lds(NG, KS, wide_apart(NG, K, KS)), stream>>>(a);
   }
 }
 

@@ -45,7 +45,8 @@ def _check(v, i, S, ids, k):
     (640, 300, 20, 13, "ip"), (768, 49_153, 33, 8, "cosine"), (256, 31_000, 49, 5, "l2"), (384, 24_575, 64, 7, "cosine"),
     (384, 31, 32, 16, "cosine")])
 def test_flat(gpu, D, rows, nq, k, metric):
-    assert ops.kernels().scan_scores_flat(nq, rows, D, k)
+    # 17 to 64 queries of the dimensions whose lists waves of their own keep need no scores
+    assert ops.kernels().scan_scores_flat(nq, rows, D, k) == (nq <= 16 or D == 640)
     X, bias, ids, q = _vectors(rows, D, nq, metric, gpu)
     v, i = ops.flat_search(q, X, bias, ids, metric, k)
     _check(v, i, _exact(X, bias, q, metric), ids, k)
@@ -73,7 +74,8 @@ def test_lists(gpu, D, rows, nlist, nprobe, nq, k, metric):
 def test_lines():
     """Up to 128 MiB of scores, and what the register lists are faster for."""
     f, l = ops.kernels().scan_scores_flat, ops.kernels().scan_scores_lists
-    assert f(32, 1 << 20, 384, 16) and not f(33, 1 << 20, 384, 8) and not f(65, 1000, 384, 8) and not f(1, 1000, 384, 8)
+    assert f(16, 1 << 20, 384, 16) and not f(33, 1 << 20, 384, 8) and not f(65, 1000, 384, 8) and not f(1, 1000, 384, 8)
+    assert not f(20, 600_000, 768, 12) and not f(33, 600_000, 768, 8) and f(48, 100_000, 256, 8) and f(32, 100_000, 640, 16)
     assert not f(12, 1_000_000, 1024, 14) and f(4, 400_000, 1024, 12) and not f(34, 400_000, 1024, 8) and not f(40, 100_000, 384, 4) and not f(48, 20_000, 768, 8)
     assert l(32, 1 << 20, 1024, 25, 64, 16) and not l(33, 1 << 20, 1024, 25, 64, 16) and not l(32, 1_000_000, 1024, 8, 64, 16)
     assert not l(20, 1000, 384, 4, 64, 16) and not l(2, 60_000, 384, 8, 64, 8) and l(12, 60_000, 384, 8, 64, 8)
@@ -85,5 +87,16 @@ def test_lines():
 def test_flat_of_few_rows(gpu, D, rows, nq, k, metric):
     X, bias, ids, q = _vectors(rows, D, nq, metric, gpu)
     X = X.nan_to_num()
+    v, i = ops.flat_search(q, X, bias, ids, metric, k)
+    _check(v, i, _exact(X, bias, q, metric), ids, k)
+
+
+# lists that waves of their own keep: one row, one more than a tile, workgroups with one tile more than others, every length of the ring's tail
+@pytest.mark.parametrize("D,nq,k,metric", [(256, 64, 8, "l2"), (384, 17, 4, "cosine"), (512, 33, 8, "ip"), (640, 49, 4, "cosine"), (768, 32, 16, "l2"),
+                                           (896, 48, 8, "ip"), (1024, 64, 4, "cosine"), (1024, 20, 12, "l2"), (1024, 33, 3, "ip")])
+@pytest.mark.parametrize("rows", [17, 33, 8_193, 24_576, 57_345])
+def test_flat_lists_apart(gpu, D, nq, k, metric, rows):
+    assert not ops.kernels().scan_scores_flat(nq, rows, D, k)
+    X, bias, ids, q = _vectors(rows, D, nq, metric, gpu)
     v, i = ops.flat_search(q, X, bias, ids, metric, k)
     _check(v, i, _exact(X, bias, q, metric), ids, k)
