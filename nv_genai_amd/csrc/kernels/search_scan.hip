@@ -1060,7 +1060,8 @@ __global__ void __launch_bounds__(256, 1) ivf_one_kernel(ScanArgs p, IvfLists l)
 // 1,024 values reach the bound (equal scores), the k-th key is found bit by bit, and the last row that is taken of those with
 // that key in the same way. Three passes over 2,048 LDS counters,
 // most of them on the same few exponents, took 82 us for both levels of 33 x 250k scores, k 25; two reads of the scores, and ranks
-// from one LDS read after another, 30; these take 23.
+// from one LDS read after another, 30; these took 23, and 21 with loads of 16 bytes, one operation a value and pass, and 64 registers (of 64 x 1M
+// scores the whole search 476, 465; with 115 registers 480).
 // Order: value, then row (the lower first).
 namespace {
 struct SelShared {
@@ -1078,28 +1079,39 @@ __device__ __forceinline__ int sel_block_count(int c, int* red) {
   return red[0] + red[1] + red[2] + red[3];
 }
 
-// returns how many of the first k places are filled; emit(place, value, row) is called for each of them. More than 256 RV values are
-// read twice.
-template <int RV, typename Emit>
+// returns how many of the first k places are filled; emit(place, value, row, fetch(row)) is called for each of them, where fetch comes before
+// the places are counted. mid() is called once while the first values are on their way. More than 256 RV values are read twice.
+template <int RV, typename Mid, typename Fetch, typename Emit>
 __device__ __forceinline__ int sel_topk(const float* __restrict__ v, const int32_t* __restrict__ r, int64_t row0, int64_t n, int k,
-                                        SelShared& s, Emit emit) {
+                                        SelShared& s, Mid mid, Fetch fetch, Emit emit) {
   const int t = threadIdx.x;
   const bool kept = n <= 256 * RV;
-  uint32_t mx = 0;
+  float mxf = -INFINITY;
   float x[RV];
   int32_t xr[RV];
-  for (int64_t i0 = t; i0 < (kept ? t + 1 : n); i0 += RV * 256) {
+  // values c0 .. of a turn: a thread's are 256 apart, or where all are there four in a row, in loads of 16 bytes
+  auto whole = [&](int64_t c0) -> bool { return !r && n - c0 >= 256 * RV; };
+  auto load = [&](int64_t c0) {
+    if (whole(c0)) {
 #pragma unroll
-    for (int u = 0; u < RV; ++u) x[u] = i0 + 256 * u < n ? v[i0 + 256 * u] : -INFINITY;
+      for (int u = 0; u < RV; u += 4) __builtin_memcpy(&x[u], v + c0 + 4 * t + 256 * u, 16);   // lists begin at any row
+      return;
+    }
+    const int left = (int)(n - c0 < 256 * RV ? n - c0 : 256 * RV) - t;
+#pragma unroll
+    for (int u = 0; u < RV; ++u) x[u] = 256 * u < left ? v[c0 + t + 256 * u] : -INFINITY;
     if (r && kept)
 #pragma unroll
-      for (int u = 0; u < RV; ++u) xr[u] = i0 + 256 * u < n ? r[i0 + 256 * u] : -1;
+      for (int u = 0; u < RV; ++u) xr[u] = 256 * u < left ? r[c0 + t + 256 * u] : -1;
+  };
+  for (int64_t c0 = 0; c0 < (kept ? 1 : n); c0 += RV * 256) {
+    load(c0);
+    if (kept) mid();
 #pragma unroll
-    for (int u = 0; u < RV; ++u) {
-      const uint32_t key = ss_key(x[u]);
-      mx = key > mx ? key : mx;
-    }
+    for (int u = 0; u < RV; ++u) mxf = fmaxf(mxf, x[u]);
   }
+  if (!kept) mid();
+  uint32_t mx = ss_key(mxf);
   const int ngr = k <= 32 ? 64 : 256;   // groups of four threads, or threads
   if (ngr == 64) {
     uint32_t o = __shfl_xor(mx, 1, 64);
@@ -1124,17 +1136,18 @@ __device__ __forceinline__ int sel_topk(const float* __restrict__ v, const int32
   }
   __syncthreads();
   const uint32_t bound = s.bound;
-  for (int64_t i0 = t; i0 < (kept ? t + 1 : n); i0 += RV * 256) {
-    if (!kept)
-#pragma unroll
-      for (int u = 0; u < RV; ++u) x[u] = i0 + 256 * u < n ? v[i0 + 256 * u] : -INFINITY;
+  const float least = __uint_as_float((bound & 0x80000000u) ? (bound & 0x7fffffffu) : ~bound);
+  for (int64_t c0 = 0; c0 < (kept ? 1 : n); c0 += RV * 256) {
+    if (!kept) load(c0);
+    const bool four = whole(c0);
 #pragma unroll
     for (int u = 0; u < RV; ++u) {
-      const uint32_t key = ss_key(x[u]);
-      if (key >= bound) {
+      if (!(x[u] < least)) {   // one operation a value; the key orders what is left
+        const uint32_t key = ss_key(x[u]);
+        if (key < bound) continue;
         const uint32_t pos = atomicAdd(&s.n_got, 1u);
         if (pos < SEL_CAP) {
-          const int64_t i = i0 + 256 * u;
+          const int64_t i = c0 + (four ? 4 * t + 256 * (u & ~3) + (u & 3) : t + 256 * u);
           const int32_t row = r ? (kept ? xr[u] : r[i]) : (int32_t)(row0 + i);
           s.kr[pos] = (uint64_t)key << 32 | (uint32_t)~row;
         }
@@ -1177,6 +1190,8 @@ __device__ __forceinline__ int sel_topk(const float* __restrict__ v, const int32
   }
   for (int i = t; i < got; i += 256) {
     const uint64_t own = s.kr[i];
+    const int32_t row = (int32_t)~(uint32_t)own;
+    const auto with = fetch(row);
     int place = 0;
 #pragma unroll 16
     for (int o = 0; o < got; ++o) {
@@ -1184,14 +1199,14 @@ __device__ __forceinline__ int sel_topk(const float* __restrict__ v, const int32
       place += x > own || (x == own && o < i);
     }
     const uint32_t key = (uint32_t)(own >> 32);
-    if (place < k) emit(place, __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key), (int32_t)~(uint32_t)own);
+    if (place < k) emit(place, __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key), row, with);
   }
   return got < k ? got : k;
 }
 }  // namespace
 
 // the k best of each segment of a row of scores, as candidates
-__global__ void __launch_bounds__(256) select_segments_kernel(const float* __restrict__ S, int64_t s_stride, int64_t N,
+__global__ void __launch_bounds__(256, 8) select_segments_kernel(const float* __restrict__ S, int64_t s_stride, int64_t N,
                                                               int64_t seg, int k, int32_t cap, float* __restrict__ cand_v,
                                                               int32_t* __restrict__ cand_r) {
   __shared__ SelShared s;
@@ -1199,7 +1214,7 @@ __global__ void __launch_bounds__(256) select_segments_kernel(const float* __res
   const int64_t n = N - beg < seg ? N - beg : seg;
   float* ov = cand_v + q * cap + (int64_t)blockIdx.x * k;
   int32_t* orow = cand_r + q * cap + (int64_t)blockIdx.x * k;
-  const int got = sel_topk<32>(S + q * s_stride + beg, (const int32_t*)nullptr, beg, n, k, s, [&](int place, float v, int32_t r) {
+  const int got = sel_topk<32>(S + q * s_stride + beg, (const int32_t*)nullptr, beg, n, k, s, [] {}, [](int32_t) { return 0; }, [&](int place, float v, int32_t r, int) {
     ov[place] = v;
     orow[place] = r;
   });
@@ -1210,14 +1225,14 @@ __global__ void __launch_bounds__(256) select_segments_kernel(const float* __res
 }
 
 // the same of each list that a query probes
-__global__ void __launch_bounds__(256) select_lists_kernel(const float* __restrict__ S, int64_t s_stride, const int32_t* __restrict__ probes,
+__global__ void __launch_bounds__(256, 8) select_lists_kernel(const float* __restrict__ S, int64_t s_stride, const int32_t* __restrict__ probes,
                                                            const int64_t* __restrict__ lbeg, const int64_t* __restrict__ lend, int k,
                                                            float* __restrict__ cand_v, int32_t* __restrict__ cand_r) {
   __shared__ SelShared s;
   const int64_t q = blockIdx.y, nprobe = gridDim.x, at = (q * nprobe + blockIdx.x) * k;
   const int list = probes[q * nprobe + blockIdx.x];
   const int64_t beg = lbeg[list], n = lend[list] > beg ? lend[list] - beg : 0;
-  const int got = sel_topk<32>(S + q * s_stride + beg, (const int32_t*)nullptr, beg, n, k, s, [&](int place, float v, int32_t r) {
+  const int got = sel_topk<32>(S + q * s_stride + beg, (const int32_t*)nullptr, beg, n, k, s, [] {}, [](int32_t) { return 0; }, [&](int place, float v, int32_t r, int) {
     cand_v[at + place] = v;
     cand_r[at + place] = r;
   });
@@ -1227,7 +1242,8 @@ __global__ void __launch_bounds__(256) select_lists_kernel(const float* __restri
   }
 }
 
-// a query's result from its candidates: the k best, less |q|^2 (l2), with the external ids of finite scores
+// a query's result from its candidates: the k best, less |q|^2 (l2), with the external ids of finite scores. A chain of latencies: the
+// query's squares are added up while the candidates are on their way, the ids come while the places are counted
 __global__ void __launch_bounds__(256) search_finish_kernel(const float* __restrict__ cand_v, const int32_t* __restrict__ cand_r,
                                                             const int32_t* __restrict__ cnt, int32_t n_fixed, int32_t cap,
                                                             int k, const float* __restrict__ qf, int64_t q_stride, int D,
@@ -1238,15 +1254,25 @@ __global__ void __launch_bounds__(256) search_finish_kernel(const float* __restr
   const int64_t q = blockIdx.x;
   int n = n_fixed >= 0 ? n_fixed : cnt[q];
   n = n < cap ? n : cap;
-  float less = 0.f;
-  if (qf) {   // l2
-    for (int i = threadIdx.x; i < D; i += 256) less += qf[q * q_stride + i] * qf[q * q_stride + i];
-    less = block_sum(less, red);
-  }
-  const int got = sel_topk<16>(cand_v + q * cap, cand_r + q * cap, 0, n, k, s, [&](int place, float v, int32_t r) {
-    const float x = v - less;
+  const int t = threadIdx.x;
+  float qv[4] = {0.f, 0.f, 0.f, 0.f};
+  if (qf)   // l2; D <= 1,024
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (t + 256 * j < D) qv[j] = qf[q * q_stride + t + 256 * j];
+  auto squares = [&]() {
+    if (!qf) return;
+    float less = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) less = __builtin_fmaf(qv[j], qv[j], less);
+    less = wave_sum(less);
+    if ((t & 63) == 0) red[t >> 6] = less;   // read behind the selection's barriers
+  };
+  const int got = sel_topk<16>(cand_v + q * cap, cand_r + q * cap, 0, n, k, s, squares, [&](int32_t r) { return r >= 0 ? ids[r] : (int64_t)-1; },
+                               [&](int place, float v, int32_t, int64_t id) {
+    const float x = qf ? v - (((red[0] + red[1]) + red[2]) + red[3]) : v;
     out_v[q * k + place] = x;
-    out_id[q * k + place] = r >= 0 && isfinite(x) ? ids[r] : -1;
+    out_id[q * k + place] = isfinite(x) ? id : -1;
   });
   for (int i = got + threadIdx.x; i < k; i += 256) {
     out_v[q * k + i] = -INFINITY;
