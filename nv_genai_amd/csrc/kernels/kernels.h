@@ -472,17 +472,7 @@ struct GemvParams {
   int64_t ldo;
   const uint16_t* norm_w;   // epi 1 / 2: x goes through an RMSNorm of this weight first (M 1, K <= 8,192), or null
   float eps;
-  // Steps of a decode layer without norms of their own: x packed (packed_at; epi 2: and out), where sq is given times a norm's weights, the
-  // row's 1 / rms still to come, from the squares' sums of n_sq 16-feature tiles [n_sq / 4][16][4]
-  int packed;
-  const float* sq;
-  int n_sq;
-  // epi 3: the rows times the next norm's weights, packed, and their squares' sums, or null
-  uint16_t* xw;
-  float* sq_out;
-  const uint16_t* next_w;
 };
-void launch_stream_open(const uint16_t* x, int64_t ldx, const uint16_t* norm_w, int M, int H, uint16_t* xw, float* sq, hipStream_t stream);
 // out = x . W^T for M <= 4 rows (gemv.hip); false if the shape is out of range
 bool launch_gemv(const GemvParams& p, int epi, hipStream_t stream);
 
@@ -504,6 +494,8 @@ struct StreamGemmParams {
   uint16_t* xw;
   float* sq_out;
   const uint16_t* next_w;
+  const uint16_t* ahead;
+  int ahead_tiles, ahead_nt, ahead_K, ahead_F;
 };
 void launch_stream_open(const uint16_t* x, int64_t ldx, const uint16_t* norm_w, int M, int H, uint16_t* xw, float* sq, hipStream_t stream);
 bool stream_gemm_covers(int64_t M, int64_t N, int64_t K, bool swiglu);
