@@ -1728,7 +1728,6 @@ std::vector<Tensor> flat_search(Tensor q, Tensor X, Tensor bias, Tensor ids, dou
     s.a.s_stride = (N + 3) / 4 * 4;
     S = at::empty({nq, s.a.s_stride}, X.options().dtype(at::kFloat));
     s.a.S = S.data_ptr<float>();
-    s.a.drop_nan = held > 0;
   }
   if (wide) nga::launch_scan_wide(s.a, ng, K, items * parts, s.st);
   else nga::launch_scan(s.a, ng, K, items * parts, s.st);
@@ -1793,7 +1792,6 @@ std::vector<Tensor> ivf_search(Tensor q, Tensor X, Tensor bias, Tensor ids, Tens
     s.a.s_stride = X.size(0);
     S = at::empty({nq, s.a.s_stride}, X.options().dtype(at::kFloat));
     s.a.S = S.data_ptr<float>();
-    s.a.drop_nan = 1;
   }
   nga::launch_scan(s.a, ng, K, blocks, s.st);
   if (K == 0)

@@ -224,9 +224,8 @@ struct ScanArgs {
   int32_t* cnt;                 // lists: [nq]
   float* cand_v;                // [nq, cap]
   int32_t* cand_r;
-  float* S;                     // [nq, s_stride] where no list is kept
+  float* S;                     // [nq, s_stride] where no list is kept; -inf for scores that are no numbers
   int64_t s_stride;
-  int drop_nan;                 // scores that are no numbers are written as -inf, as register lists leave them out
 };
 int scan_chunk(int D, int ng);                  // dims of a unit of work, 0: not covered
 int scan_blocks(int D, int ng, int cus);        // workgroups that fill the chip

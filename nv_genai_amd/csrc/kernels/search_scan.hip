@@ -23,7 +23,8 @@ __device__ __forceinline__ uint32_t ss_key(float f) {
 }
 constexpr uint32_t KEY_NEG_INF = 0x007fffffu;
 
-// a score that is no number, which no register list takes in, as the selection leaves it out
+// Scores that are no numbers as the selection leaves them out; no register list takes them in. As keys those without a sign would come first
+// (the matrix unit's have one, a bias may have none)
 __device__ __forceinline__ f32x4 ss_drop_nan(f32x4 v) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) v[i] = v[i] == v[i] ? v[i] : -INFINITY;
@@ -468,7 +469,7 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
                 f32x4 v;
 #pragma unroll
                 for (int rr = 0; rr < 4; ++rr) v[rr] = acc[i][g][rr] * p.dot_scale + bcur[i][rr];
-                if (p.drop_nan) v = ss_drop_nan(v);
+                v = ss_drop_nan(v);
                 if (rb + 3 < end) {
                   __builtin_memcpy(dst, &v, 16);   // lists begin at any row
                 } else {
@@ -637,7 +638,7 @@ __global__ void __launch_bounds__(wide_apart(NG, K, KS) ? 512 : 256, 1) scan_wid
         for (int rr = 0; rr < 4; ++rr)
           if (rb + rr < p.N && v[rr] > tv[gg][K - 1]) ss_insert<KR>(tv[gg], tr[gg], v[rr], (int)(rb + rr));
       } else if (16 * g + col < nql) {
-        if (p.drop_nan) v = ss_drop_nan(v);
+        v = ss_drop_nan(v);
         float* dst = p.S + (int64_t)(item * SL + 16 * g + col) * p.s_stride + rb;   // s_stride % 4 == 0
         if (rb + 3 < p.N) {
           *reinterpret_cast<f32x4*>(dst) = v;

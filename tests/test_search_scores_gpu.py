@@ -86,7 +86,6 @@ def test_lines():
                                                 (512, 32_769, 5, 2, "ip"), (384, 65_536, 1, 4, "l2"), (384, 65_537, 1, 4, "l2"), (1024, 20_000, 9, 25, "cosine")])
 def test_flat_of_few_rows(gpu, D, rows, nq, k, metric):
     X, bias, ids, q = _vectors(rows, D, nq, metric, gpu)
-    X = X.nan_to_num()
     v, i = ops.flat_search(q, X, bias, ids, metric, k)
     _check(v, i, _exact(X, bias, q, metric), ids, k)
 
@@ -100,3 +99,15 @@ def test_flat_lists_apart(gpu, D, nq, k, metric, rows):
     X, bias, ids, q = _vectors(rows, D, nq, metric, gpu)
     v, i = ops.flat_search(q, X, bias, ids, metric, k)
     _check(v, i, _exact(X, bias, q, metric), ids, k)
+
+
+# more results than lists hold: scores of one group and of several, queries in LDS and in registers, up to the most results. A NaN without a sign is
+# the highest of sortable keys
+@pytest.mark.parametrize("D,rows,nq,k,metric", [(1024, 20_000, 9, 25, "cosine"), (384, 5_000, 3, 200, "ip"), (640, 9_000, 20, 17, "l2"), (128, 8_193, 40, 9, "cosine"),
+                                                (1024, 30_001, 33, 25, "l2"), (512, 8_192, 64, 100, "cosine"), (768, 300, 70, 256, "ip"),
+                                                (384, 5_000, 3, 12, "ip"), (384, 5_000, 3, 4, "ip"), (1024, 9_000, 33, 4, "l2")])
+def test_scores_that_are_no_numbers(gpu, D, rows, nq, k, metric):
+    X, bias, ids, q = _vectors(rows, D, nq, metric, gpu)
+    bias[7::89] = float("nan")
+    v, i = ops.flat_search(q, X, bias, ids, metric, k)
+    _check(v, i, _exact(X, bias.nan_to_num(nan=float("-inf"), neginf=float("-inf")), q, metric), ids, k)
