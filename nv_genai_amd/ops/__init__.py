@@ -1859,16 +1859,16 @@ def search_topk(Q: torch.Tensor, X: torch.Tensor, row_bias=None, dot_scale: floa
     row_bias, without materialising S: the fused MFMA score + per-block top-k kernel writes
     [nq, blocks, k] candidates and one ``topk`` pass merges them (K13: per-tile top-k fused
     into scoring, then the k-merge). Returns (scores [nq, k], rows [nq, k]; -inf / -1 where X
-    has fewer than k live rows). Falls back to the score matrix + ``topk`` when k exceeds the
+    has fewer than k live rows; scores that are no numbers count as -inf). Falls back to the score matrix + ``topk`` when k exceeds the
     kernel's register lists."""
     k = int(min(k, X.shape[0]))
     nq = Q.shape[0]
     if not _gpu(X):
-        return ref.topk(ref.score(Q, X, row_bias, dot_scale), k)
+        return ref.topk(ref.drop_nan_(ref.score(Q, X, row_bias, dot_scale)), k)
     C = kernels()
     qpi = min(nq, 64)
     if k > C.score_topk_kmax(qpi) or nq == 0:
-        return topk(score(Q, X, row_bias, dot_scale), k)
+        return topk(ref.drop_nan_(score(Q, X, row_bias, dot_scale)), k)
     items = -(-nq // 64)
     dma = bool(C.score_topk_dma_ok(X.shape[1], qpi))
     nblk = score_topk_blocks(X.shape[0], X.shape[0], items, qpi, dma, _cu_count(X.device) if dma else 256)

@@ -336,6 +336,11 @@ def topk(S: torch.Tensor, k: int) -> Tuple[torch.Tensor, torch.Tensor]:
     return v, i
 
 
+def drop_nan_(S: torch.Tensor) -> torch.Tensor:
+    """Scores that are no numbers as -inf, in place: a search leaves them out, where ``torch.topk`` would put them first."""
+    return torch.nan_to_num_(S, nan=float("-inf"), posinf=float("inf"), neginf=float("-inf"))
+
+
 def ivf_search_topk(Q, X, row_bias, dot_scale, probes, list_beg, list_end, k):
     """Per query: exact top-k over the rows of its probed lists (slab rows; -inf / -1 pads)."""
     nq = Q.shape[0]
@@ -350,7 +355,7 @@ def ivf_search_topk(Q, X, row_bias, dot_scale, probes, list_beg, list_end, k):
         s = score(Q[i:i + 1], X.index_select(0, r), None if row_bias is None else row_bias.index_select(0, r),
                   dot_scale)[0]
         kk = min(k, r.numel())
-        v, j = torch.topk(s, kk)
+        v, j = torch.topk(drop_nan_(s), kk)
         vals[i, :kk] = v
         rows[i, :kk] = r[j]
     return vals, rows
