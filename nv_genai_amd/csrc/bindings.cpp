@@ -1672,6 +1672,17 @@ Search search_begin(const Tensor& q, const Tensor& X, const Tensor& bias, double
   return s;
 }
 
+// room for the scores of a search, or nothing where its results can also be held in lists (`held`) and there is no memory: lists take kilobytes,
+// scores up to 128 MiB, and a process may have filled the GPU with its cache
+Tensor score_room(int64_t nq, int64_t stride, const Tensor& X, bool held) {
+  try {
+    return at::empty({nq, stride}, X.options().dtype(at::kFloat));
+  } catch (const c10::OutOfMemoryError&) {
+    if (!held) throw;
+  }
+  return {};
+}
+
 std::vector<Tensor> search_end(Search& s, const Tensor& q, const Tensor& ids, int32_t n_fixed, const char* name) {
   nga::launch_search_finish(s.a.cand_v, s.a.cand_r, s.a.cnt, n_fixed, s.a.cap, s.a.nq, s.a.k,
                             s.a.metric == nga::SEARCH_L2 ? q.data_ptr<float>() : nullptr, s.a.q_stride, s.a.D,
@@ -1704,7 +1715,11 @@ std::vector<Tensor> flat_search(Tensor q, Tensor X, Tensor bias, Tensor ids, dou
   const int D = (int)X.size(1), ng = nq <= 16 ? 1 : nq <= 32 ? 2 : nq <= 48 ? 3 : 4;
   const int items = (int)((nq + 16 * ng - 1) / (16 * ng));
   const bool wide = ng > 1 && nga::scan_wide_covers(D, ng);
-  const int held = nga::scan_list((int)k, ng, false), K = nga::scan_scores_flat(nq, N, D, (int)k) ? 0 : held;
+  const int held = nga::scan_list((int)k, ng, false);
+  const int64_t s_stride = (N + 3) / 4 * 4;
+  Tensor S;
+  if (held == 0 || nga::scan_scores_flat(nq, N, D, (int)k)) S = score_room(nq, s_stride, X, held > 0);
+  const int K = S.defined() ? 0 : held;
   const int blocks = wide ? (int)cus : nga::scan_blocks(D, ng, (int)cus);
   // one workgroup a CU with up to two tiles: shared out by waves, where that makes no more candidates of 8 or 16 (20k x 768, 4 queries, k 8:
   // 24.1 us, shared out 24.4)
@@ -1716,7 +1731,7 @@ std::vector<Tensor> flat_search(Tensor q, Tensor X, Tensor bias, Tensor ids, dou
   Search s = search_begin(q, X, bias, dot_scale, metric, k, cap);
   s.a.parts = parts;
   s.a.fine = fine;
-  Tensor qb, S;
+  Tensor qb;
   if (ng == 1) {   // up to 16 queries are prepared by every workgroup, while its first vectors come in
     s.a.qf = q.data_ptr<float>();
   } else {
@@ -1725,8 +1740,7 @@ std::vector<Tensor> flat_search(Tensor q, Tensor X, Tensor bias, Tensor ids, dou
     nga::launch_search_prep(q.data_ptr<float>(), q.stride(0), (int)nq, D, (int)metric, bfp(qb), wide, s.st);
   }
   if (K == 0) {
-    s.a.s_stride = (N + 3) / 4 * 4;
-    S = at::empty({nq, s.a.s_stride}, X.options().dtype(at::kFloat));
+    s.a.s_stride = s_stride;
     s.a.S = S.data_ptr<float>();
   }
   if (wide) nga::launch_scan_wide(s.a, ng, K, items * parts, s.st);
@@ -1751,8 +1765,11 @@ std::vector<Tensor> ivf_search(Tensor q, Tensor X, Tensor bias, Tensor ids, Tens
   TORCH_CHECK(list_beg.numel() == nlist && list_end.numel() == nlist, "ivf_search: one row range per list");
   TORCH_CHECK(nprobe >= 1 && nprobe <= nlist, "ivf_search: nprobe must be in [1, lists]");
   TORCH_CHECK(k <= 32 && cus >= 1 && cus <= 4096, "ivf_search: k must be at most 32");
-  const bool scores = nga::scan_scores_lists(nq, X.size(0), D, (int)k, nlist, nprobe);
-  if (nga::ivf_one_covers(nq, nlist, D, (int)k) && !(scores && k > 16)) {
+  const bool one = nga::ivf_one_covers(nq, nlist, D, (int)k);
+  Tensor S;
+  if (nga::scan_scores_lists(nq, X.size(0), D, (int)k, nlist, nprobe) && !(one && k <= 16)) S = score_room(nq, X.size(0), X, true);
+  const bool scores = S.defined();
+  if (one && !scores) {
     const int blocks = nga::scan_blocks(D, 1, (int)cus);
     Search s = search_begin(q, X, bias, dot_scale, metric, k, blocks * k);
     s.a.qf = q.data_ptr<float>();
@@ -1775,10 +1792,10 @@ std::vector<Tensor> ivf_search(Tensor q, Tensor X, Tensor bias, Tensor ids, Tens
   auto* items = reinterpret_cast<nga::ScanItem*>(tab.data_ptr<int32_t>());
   int32_t *cnt = tab.data_ptr<int32_t>() + 8 * max_items, *probes = cnt + nq, *run_item = probes + npairs,
           *qtab = run_item + blocks + 1;
-  nga::IvfOne one{};
-  if (nq == 1) one = {sl, blocks, list_beg.data_ptr<int64_t>(), list_end.data_ptr<int64_t>(), items, run_item, qtab};
+  nga::IvfOne plan{};
+  if (nq == 1) plan = {sl, blocks, list_beg.data_ptr<int64_t>(), list_end.data_ptr<int64_t>(), items, run_item, qtab};
   nga::launch_ivf_probe(q.data_ptr<float>(), q.stride(0), (int)nq, D, (int)metric, centroids.data_ptr<float>(), (int)nlist,
-                        (int)nprobe, bfp(qb), cnt, probes, one, s.st);
+                        (int)nprobe, bfp(qb), cnt, probes, plan, s.st);
   if (nq > 1)
     nga::launch_ivf_items(probes, (int)npairs, (int)nprobe, (int)nlist, sl, (int)max_items, blocks, list_beg.data_ptr<int64_t>(),
                         list_end.data_ptr<int64_t>(), items, run_item, qtab, s.st);
@@ -1787,10 +1804,8 @@ std::vector<Tensor> ivf_search(Tensor q, Tensor X, Tensor bias, Tensor ids, Tens
   s.a.items = items;
   s.a.run_item = run_item;
   s.a.qtab = qtab;
-  Tensor S;
   if (K == 0) {
     s.a.s_stride = X.size(0);
-    S = at::empty({nq, s.a.s_stride}, X.options().dtype(at::kFloat));
     s.a.S = S.data_ptr<float>();
   }
   nga::launch_scan(s.a, ng, K, blocks, s.st);

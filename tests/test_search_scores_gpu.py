@@ -1,5 +1,7 @@
 """Searches whose scores go through memory although register lists could hold the results: against 64 bits, with removed rows, vectors that
 are no numbers and lists that begin at any row or are empty."""
+import contextlib
+
 import pytest
 import torch
 
@@ -111,3 +113,37 @@ def test_scores_that_are_no_numbers(gpu, D, rows, nq, k, metric):
     bias[7::89] = float("nan")
     v, i = ops.flat_search(q, X, bias, ids, metric, k)
     _check(v, i, _exact(X, bias.nan_to_num(nan=float("-inf"), neginf=float("-inf")), q, metric), ids, k)
+
+
+@contextlib.contextmanager
+def _no_room(size):
+    """No block of `size` bytes of device memory for this process, but some 24 MB in new ones."""
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.mem_get_info()[1]
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (24 << 20)) / total)
+    held = []
+    try:
+        with pytest.raises(torch.cuda.OutOfMemoryError):   # what other work has left free in its blocks
+            while True:
+                held.append(torch.empty(size, dtype=torch.uint8, device="cuda"))
+        yield
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+# 64 MB of scores, where lists take less than 2 (the allocator asks for 2 or 20 at once)
+@pytest.mark.parametrize("nq,k", [(16, 12), (16, 9)])
+def test_no_memory_for_scores(gpu, nq, k):
+    """A search whose results lists hold needs no memory for scores: with neither it gives the same."""
+    rows, D, nlist, nprobe = 1_000_000, 128, 64, 4
+    X, bias, ids, q = _vectors(rows, D, nq, "l2", gpu)
+    g = torch.Generator().manual_seed(k)
+    off = torch.linspace(0, rows, nlist + 1).long().to(gpu)
+    cent = torch.randn(nlist, D, generator=g).to(gpu)
+    assert ops.kernels().scan_scores_flat(nq, rows, D, k) and ops.kernels().scan_scores_lists(nq, rows, D, k, nlist, nprobe)
+    for f in (lambda: ops.flat_search(q, X, bias, ids, "l2", k), lambda: ops.ivf_search(q, X, bias, ids, cent, off[:-1], off[1:], "l2", nprobe, k)):
+        v, i = f()
+        with _no_room(60 << 20):
+            w, j = f()
+        assert torch.equal(v, w) and torch.equal(i, j)
