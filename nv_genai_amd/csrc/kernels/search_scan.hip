@@ -1329,24 +1329,26 @@ int scan_list(int k, int ng, bool ivf) {
   return k > most ? 0 : k <= 4 ? 4 : k <= 8 ? 8 : k <= 16 ? 16 : 32;
 }
 
-// Whether scores go to memory and are selected from there where register lists could hold the results: a list of 16 or 32 costs every
-// lane some 100 or 200 operations whenever one of a wave's takes a value in, and on merging, whatever the rows' length, a score 4 bytes
-// twice and the selection a launch. Up to 128 MiB of scores. Whole searches, us, lists / scores:
-// flat, k 12, at 1 / 12 / 28 queries: 100k x 128 44 49 59, 24 32 33; 130k x 384 52 53 57, 38 44 47; 500k x 512 130 144 160, 103 122 124; 300k x 640
-// 105 109 105, 80 97 104; 600k x 768 174 192 236, 160 200 207; 300k x 896 107 108 136, 97 116 124; 400k x 1,024 164 164 176, 144 171 180;
-// 1M x 1,024, k 14, at 1 / 4 / 12: 323 333 339, 326 358 393; 60k 47 48 50, 41 41 43 (more than 16 queries of most dimensions: in scan_wide_kernel's
-// lists by now). k 6, 40 queries, 900k x 256: 266 in scores
 bool scan_wide_covers(int D, int ng) { return D % 128 == 0 && wide_takes(D / 128, ng); }   // flat scans of 17 to 64 queries, prepared
 
+// Whether scores go to memory and are selected from there where register lists could hold the results: a list of 16 or 32 costs every
+// lane some 100 or 200 operations whenever one of a wave's takes a value in, and on merging, whatever the rows' length: some 5 to 20 us, more
+// with fewer dimensions. A score costs 4 bytes twice, and the writes hold up the stream the more, the more of its time is the vectors' own:
+// the line is one of rows x (queries + 2). Up to 128 MiB of scores. Whole searches, us, lists / scores, on either side of the lines:
+// 512 dimensions, k 9, at 1 / 16 queries: 60k 37 39, 29 33; 2M 350 452, 325 424 (fewer gain more: 128, 2M 168 204, 111 154).
+// 640, k 9, at 1 / 8 / 16: 250k 85 89 91, 67 77 86; 1M 244 254 257, 221 268 286; 2M 441 463 468, 432 518 551; at 17 / 32: 250k 88 90, 80 86; 700k 187 194,
+// 191 208. 768, at 1 / 8 / 16: 250k 96 100 100, 79 88 97; 1M 257 287 290, 249 302 324; one of 2M 470, 480. 896: 250k 88 90 92, 81 91 100; 1M 276 282 285, 283
+// 329 350. 1,024: 250k 110 113 114, 96 106 116; 1M 321 335 338, 324 378 402. k 16 moves the lines out a little: 896, 8 of 250k 102 / 93.
+// 17 to 64 queries of the dimensions of scan_wide_kernel stay in its lists, which waves of their own keep: 600k x 768, 20 queries, k 12, 161 208, 33, k
+// 8, 161 230; 900k x 512, 33, k 8, 222 247; closest 130k x 384, 20, k 12, 51 48. 33 to 48 of 256 dimensions, k 5 / 8, at 34 / 48: 12k 27 27, 23 24; 100k 52 51,
+// 42 45; 600k 178 193, 122 127
 bool scan_scores_flat(int64_t nq, int64_t N, int D, int k) {
-  const int64_t n = nq * N;
-  if (nq > 64 || n > (int64_t(1) << 25)) return false;
-  // scan_wide_kernel's lists, in waves of their own, cost its stream little: in lists / scores 600k x 768, 20 queries, k 12, 161 208, 33, k 8, 161
-  // 230; 900k x 512, 33, k 8, 222 247; closest 130k x 384, 20, k 12, 51 48
+  if (nq > 64 || nq * N > (int64_t(1) << 25)) return false;
   if (nq > 16 && scan_wide_covers(D, nq <= 32 ? 2 : nq <= 48 ? 3 : 4)) return false;
-  if (nq > 32) return k > 4 && k <= 8 && D >= 256 && D <= 768 && n >= 1500000;
+  if (nq > 32) return D == 256 && k > 4 && k <= 8;   // what is left of 128 dimensions keeps its lists
   if (k <= 8 || k > 16) return false;
-  return D <= 640 || n <= 2000000 || (D <= 768 && n <= 5000000) || (nq > 16 && D <= 896);
+  const int64_t cost = N * (nq + 2);
+  return D <= 512 || cost <= (nq > 16 ? 12000000 : D <= 768 ? 5000000 : D == 896 ? 2000000 : 2500000);   // above 16 queries: 640 dimensions
 }
 // 64 lists, k 25, 16 probed, at 1 / 5 / 12 / 32 queries: 1M x 1,024 165 386 470 453, 133 299 376 418; 200k x 768 69 130 137 144, 47 80 88 94; 60k x 384
 // 49 75 76 79, 35 41 42 45; k 14, 8 probed, 2 / 5 / 12 / 20 / 32: 1M x 1,024 135 210 299 357 376, 123 196 297 361 392; 200k x 768 60 80 93 102 111, 47 63

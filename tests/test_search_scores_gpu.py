@@ -45,10 +45,10 @@ def _check(v, i, S, ids, k):
 @pytest.mark.parametrize("D,rows,nq,k,metric", [
     (128, 8193, 1, 9, "ip"), (384, 24_577, 5, 16, "cosine"), (1024, 2_000, 16, 12, "l2"), (256, 9_000, 17, 10, "cosine"), (896, 8_192, 32, 16, "l2"),
     (640, 300, 20, 13, "ip"), (768, 49_153, 33, 8, "cosine"), (256, 31_000, 49, 5, "l2"), (384, 24_575, 64, 7, "cosine"),
-    (384, 31, 32, 16, "cosine")])
+    (384, 31, 32, 16, "cosine"), (256, 40_001, 40, 8, "l2"), (256, 700, 33, 5, "cosine")])
 def test_flat(gpu, D, rows, nq, k, metric):
     # 17 to 64 queries of the dimensions whose lists waves of their own keep need no scores
-    assert ops.kernels().scan_scores_flat(nq, rows, D, k) == (nq <= 16 or D == 640)
+    assert ops.kernels().scan_scores_flat(nq, rows, D, k) == (nq <= 16 or D == 640 or (D == 256 and 32 < nq <= 48))
     X, bias, ids, q = _vectors(rows, D, nq, metric, gpu)
     v, i = ops.flat_search(q, X, bias, ids, metric, k)
     _check(v, i, _exact(X, bias, q, metric), ids, k)
@@ -81,6 +81,16 @@ def test_lines():
     assert not f(12, 1_000_000, 1024, 14) and f(4, 400_000, 1024, 12) and not f(34, 400_000, 1024, 8) and not f(40, 100_000, 384, 4) and not f(48, 20_000, 768, 8)
     assert l(32, 1 << 20, 1024, 25, 64, 16) and not l(33, 1 << 20, 1024, 25, 64, 16) and not l(32, 1_000_000, 1024, 8, 64, 16)
     assert not l(20, 1000, 384, 4, 64, 16) and not l(2, 60_000, 384, 8, 64, 8) and l(12, 60_000, 384, 8, 64, 8)
+
+
+def test_lines_of_many_scores():
+    """Where writing the scores holds up the stream of the vectors by more than lists cost, by rows and queries."""
+    f = ops.kernels().scan_scores_flat
+    for D, few, many in ((640, (1_600_000, 1), (1_700_000, 1)), (640, (500_000, 8), (501_000, 8)), (640, (352_000, 32), (354_000, 32)), (768, (1_000_000, 3), (1_000_000, 4)),
+                         (768, (277_000, 16), (278_000, 16)), (896, (666_000, 1), (667_000, 1)), (1024, (250_000, 8), (251_000, 8)), (512, (2_000_000, 16), (2_200_000, 16))):
+        for k in (9, 16):
+            assert f(few[1], few[0], D, k) and not f(many[1], many[0], D, k), (D, k)
+    assert f(33, 1000, 256, 5) and f(48, 500_000, 256, 8) and not f(33, 1000, 256, 4) and not f(49, 1000, 256, 8) and not f(33, 1000, 256, 9) and not f(33, 1000, 128, 8)
 
 
 # rows that are dealt out to waves: fewer 32-row tiles than workgroups, one for some waves, two for some; and from 65,537 rows on to workgroups
