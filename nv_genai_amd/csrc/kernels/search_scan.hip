@@ -6,6 +6,7 @@
 // of any sizes load the chip evenly: with a fixed count of workgroups per list the longest list decided (1M x 1024
 // in 64 lists of unequal size, 16 probed, one query: scan 143 us, so 102; the whole search 189 us, so 113; in one launch with its
 // probing, further below, 103).
+#include <algorithm>
 #include "common.h"
 #include "kernels.h"
 
@@ -1350,17 +1351,27 @@ bool scan_scores_flat(int64_t nq, int64_t N, int D, int k) {
   const int64_t cost = N * (nq + 2);
   return D <= 512 || cost <= (nq > 16 ? 12000000 : D <= 768 ? 5000000 : D == 896 ? 2000000 : 2500000);   // above 16 queries: 640 dimensions
 }
-// 64 lists, k 25, 16 probed, at 1 / 5 / 12 / 32 queries: 1M x 1,024 165 386 470 453, 133 299 376 418; 200k x 768 69 130 137 144, 47 80 88 94; 60k x 384
-// 49 75 76 79, 35 41 42 45; k 14, 8 probed, 2 / 5 / 12 / 20 / 32: 1M x 1,024 135 210 299 357 376, 123 196 297 361 392; 200k x 768 60 80 93 102 111, 47 63
-// 73 81 89; k 8: 200k x 768 49 67 77 87 94, 46 63 72 80 88; 60k x 384 32 34 43 44 44, 34 35 40 41 41; 1M x 1,024 117 190 278 325 341, 122 195 298 360
-// 391; k 6, 600k x 384, 16 probed, at 2 / 4 / 8 / 24: 80 98 120 131, 76 93 114 133; 300k x 640, 8 probed, at 8 / 24: 82 91, 78 93. One query of k 12 is
-// the one launch's, where that takes it (1M x 1,024 128 / 131).
+// The same of lists. What register lists cost here is a merge for every run of a query's rows; what scores cost, beside the writes, is a selection by one
+// workgroup a query and list (which reads more than 8,192 scores twice): a few long lists leave the chip waiting for it, and of many short ones, or few rows
+// in all, it is a launch too much. Measured on 4,000 searches of any sizes; us, register lists / scores:
+// k 25, 16 of 64 lists, at 1 / 5 / 12 / 32 queries: 1M x 1,024 165 386 470 453, 133 299 376 418; 200k x 768 69 130 137 144, 47 80 88 94; 60k x 384 49 75 76 79, 35 41
+// 42 45. No search of 17 to 32 results was faster in lists.
+// k 9 to 16: 8 of 64, k 14, 2 / 5 / 12 / 20 / 32 queries: 1M x 1,024 135 210 299 357 376, 123 196 297 361 392; 200k x 768 60 80 93 102 111, 47 63 73 81 89. On either side of the
+// lists' length, 6 x 1.3M x 128, 8 of 8, 163 138, 3 x 885k x 384, 2 of 2, 196 232; 6 x 317k x 768, 8 of 8, 139 131, 3 x 1.1M x 768, 1 of 16, 154 191; of the scores
+// (and the rows read), 8 x 1.5M x 768, 8 of 64, 307 284, 8 x 1.5M x 640, 32 of 32, 365 417, 8 x 1.3M x 1,024, 16 of 64, 444 452; more than 16 queries write whole lines: 32 x 490k x 768, 64 of 64, 235 212.
+// k 5 to 8: 20 x 109k x 256, 16 of 64, 26 % less, 12 x 93k x 128 15, 4 x 95k x 384 10, 6 x 220k x 640 9; beyond the lines 6 x 416k x 512, 8 of 8, 112 141; 12 x 817k x 640, 4 of
+// 16, 203 242; 64 x 16k x 128, 64 of 256, 50 58; 8 x 15k x 256, 4 of 4, 28 31; 12 x 927k x 768, 16 of 64, 260 277. Of the 290 of 1,500 that these lines take 16 are slower, by
+// 1.5 to 5 %. One query of k 12 is the one launch's, where that takes it (1M x 1,024 128 / 131).
 bool scan_scores_lists(int64_t nq, int64_t N, int D, int k, int64_t nlist, int64_t nprobe) {
   if (k <= 4 || nq * N > (int64_t(1) << 25)) return false;
-  const int64_t n = nq * N / nlist * nprobe;   // scores, with lists of one length
+  const int64_t rows = N / nlist, pairs = nq * nprobe, n = pairs * rows;   // a list's rows and all scores, with lists of one length
   if (k > 16) return true;
-  if (k > 8) return D <= 768 || n <= 2000000;
-  return nq * nprobe >= 32 && n <= 3000000 && (D <= 512 || (D <= 768 && nq <= 16));
+  if (k > 8) {
+    if (D <= 512) return rows <= 262144;
+    return rows <= (D <= 768 ? 49152 : 32768) && (nq > 16 || n + 2 * std::min(pairs, nlist) * rows <= (D <= 768 ? 6000000 : 3000000));
+  }
+  return rows <= (D <= 256 ? 24576 : 8192) && pairs >= 32 && pairs <= 2048 && N >= 30000 && n >= 30000 && n <= 3000000 &&
+         (D <= 512 || (D <= 768 && nq <= 16));
 }
 
 void launch_scan(const ScanArgs& a, int ng, int K, int blocks, hipStream_t stream) {

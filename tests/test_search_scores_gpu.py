@@ -57,9 +57,10 @@ def test_flat(gpu, D, rows, nq, k, metric):
 # lists longer than the selection keeps in registers, short and empty ones; one query of dimensions that the one launch leaves, and of more results
 @pytest.mark.parametrize("D,rows,nlist,nprobe,nq,k,metric", [
     (640, 20_001, 9, 4, 1, 12, "cosine"), (1024, 30_000, 3, 2, 1, 32, "l2"), (384, 9_001, 40, 17, 2, 5, "ip"), (1024, 7_003, 64, 16, 3, 9, "cosine"),
-    (768, 5_000, 64, 64, 16, 8, "l2"), (128, 50_001, 5, 3, 33, 17, "cosine"), (256, 333, 50, 25, 70, 32, "ip")])
+    (768, 5_000, 64, 64, 16, 8, "l2"), (128, 50_001, 5, 3, 33, 17, "cosine"), (256, 333, 50, 25, 70, 32, "ip"),
+    (384, 30_001, 16, 8, 60, 8, "cosine"), (256, 40_003, 40, 17, 2, 5, "ip"), (768, 31_000, 64, 64, 16, 8, "l2"), (512, 33_333, 30, 20, 40, 6, "cosine")])
 def test_lists(gpu, D, rows, nlist, nprobe, nq, k, metric):
-    assert ops.kernels().scan_scores_lists(nq, rows, D, k, nlist, nprobe)
+    assert ops.kernels().scan_scores_lists(nq, rows, D, k, nlist, nprobe) == (k > 8 or rows >= 30_000)   # fewer rows keep lists of up to 8
     X, bias, ids, q = _vectors(rows, D, nq, metric, gpu)
     g = torch.Generator().manual_seed(D)
     off = torch.cat([torch.tensor([0]), torch.randint(0, rows + 1, (nlist - 1,), generator=g).sort().values, torch.tensor([rows])])
@@ -91,6 +92,22 @@ def test_lines_of_many_scores():
         for k in (9, 16):
             assert f(few[1], few[0], D, k) and not f(many[1], many[0], D, k), (D, k)
     assert f(33, 1000, 256, 5) and f(48, 500_000, 256, 8) and not f(33, 1000, 256, 4) and not f(49, 1000, 256, 8) and not f(33, 1000, 256, 9) and not f(33, 1000, 128, 8)
+
+
+def test_lines_of_long_and_short_lists():
+    """Where one workgroup a query and list is too few, or its launch too much."""
+    f = ops.kernels().scan_scores_lists
+    for k in (9, 16):
+        assert f(3, 1_000_000, 128, k, 4, 4) and not f(3, 1_100_000, 128, k, 4, 4) and not f(3, 885_098, 384, k, 2, 2)
+        assert f(2, 49_152 * 16, 768, k, 16, 1) and not f(2, 49_153 * 16, 768, k, 16, 1) and not f(4, 443_621, 896, k, 2, 1) and not f(2, 32_769 * 16, 1024, k, 16, 1)
+        assert f(16, 1_000_000, 640, k, 64, 16) and not f(16, 1_001_000, 768, k, 64, 16) and not f(8, 1_468_481, 640, k, 32, 32)
+        assert f(16, 500_000, 896, k, 64, 16) and not f(16, 501_000, 896, k, 64, 16) and f(17, 1_500_000, 1024, k, 64, 16) and not f(16, 1_500_000, 1024, k, 64, 16)
+    for k in (5, 8):
+        assert f(4, 64 * 8192, 512, k, 64, 16) and not f(4, 64 * 8193, 512, k, 64, 16) and not f(6, 415_530, 512, k, 8, 8)
+        assert f(4, 64 * 24_576, 256, k, 64, 16) and not f(4, 64 * 24_577, 256, k, 64, 16) and not f(16, 247_773, 128, k, 8, 4)
+        assert f(128, 90_000, 512, k, 64, 16) and not f(129, 90_000, 512, k, 64, 16) and not f(64, 15_650, 128, k, 256, 64)
+        assert f(4, 30_000, 256, k, 8, 8) and not f(4, 29_999, 256, k, 8, 8) and not f(8, 200_000, 256, k, 1024, 4)
+    assert f(1, 2_000_000, 1024, 25, 2, 2) and not f(1, 2_000_000, 1024, 4, 64, 16)
 
 
 # rows that are dealt out to waves: fewer 32-row tiles than workgroups, one for some waves, two for some; and from 65,537 rows on to workgroups
