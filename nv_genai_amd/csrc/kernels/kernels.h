@@ -493,8 +493,6 @@ struct StreamGemmParams {
   uint16_t* xw;
   float* sq_out;
   const uint16_t* next_w;
-  const uint16_t* ahead;
-  int ahead_tiles, ahead_nt, ahead_K, ahead_F;
 };
 void launch_stream_open(const uint16_t* x, int64_t ldx, const uint16_t* norm_w, int M, int H, uint16_t* xw, float* sq, hipStream_t stream);
 bool stream_gemm_covers(int64_t M, int64_t N, int64_t K, bool swiglu);
