@@ -1443,9 +1443,13 @@ const char* encoder_refuses(const Tensor& word, const std::vector<Tensor>& table
 // Post-norm encoder stack (BERT): embedding sum + norm, then per layer q/k/v, packed attention, output + norm, up + GELU,
 // down + norm. Layer tensors: wqkv, bqkv, wo, bo, ln1_g, ln1_b, wi, bi, wo2, bo2, ln2_g, ln2_b. All launches go out from
 // here: from Python the 200 of a BERT-large forward took longer than they ran (2.3 ms for one query).
-Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tensor cu, int64_t max_len, Tensor word,
-                       Tensor ptab, Tensor ttab, Tensor emb_g, Tensor emb_b, std::vector<Tensor> L, int64_t heads, double eps,
-                       double scale) {
+// Weights that it does not take raise, or with covered_only give nothing.
+c10::optional<Tensor> encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tensor cu, int64_t max_len, Tensor word,
+                                      Tensor ptab, Tensor ttab, Tensor emb_g, Tensor emb_b, std::vector<Tensor> L, int64_t heads,
+                                      double eps, double scale, bool covered_only) {
+  const char* why = encoder_refuses(word, {ptab, ttab, emb_g, emb_b}, L, heads);
+  if (why != nullptr && covered_only) return c10::nullopt;
+  TORCH_CHECK(why == nullptr, why);
   at::NoGradGuard no_grad;
   CHECK_DEV(ids); CHECK_DT(ids, at::kInt); CHECK_CONTIG(ids);
   CHECK_DEV(pos); CHECK_DT(pos, at::kInt); CHECK_CONTIG(pos);
@@ -1453,8 +1457,6 @@ Tensor encoder_forward(Tensor ids, Tensor pos, c10::optional<Tensor> types, Tens
   const int64_t T = ids.numel(), H = word.size(-1), D = heads > 0 ? H / heads : 0;
   TORCH_CHECK(pos.numel() == T && (!types.has_value() || types->numel() == T), "encoder: one position and type per token");
   if (types.has_value()) { CHECK_DEV(*types); CHECK_DT(*types, at::kInt); CHECK_CONTIG(*types); }
-  const char* why = encoder_refuses(word, {ptab, ttab, emb_g, emb_b}, L, heads);
-  TORCH_CHECK(why == nullptr, why);
   TORCH_CHECK(ids.device() == word.device() && T < (int64_t(1) << 31) && cu.numel() >= 1 && max_len >= 0, "encoder: tokens");
   const int64_t F = L.empty() ? H : L[6].size(0);
   const int64_t B = cu.numel() - 1;
@@ -3115,13 +3117,9 @@ PYBIND11_MODULE(_C, m) {
   m.def("score", checked("score", &score));
   m.def("topk", checked("topk", &topk));
   m.def("encoder_tile_rows", &encoder_tile_rows);
-  m.def("encoder_forward", &encoder_forward, py::call_guard<py::gil_scoped_release>());   // some 200 launches
-  m.def("encoder_forward_covered", [](Tensor ids, Tensor pos, c10::optional<Tensor> types, Tensor cu, int64_t max_len, Tensor word, Tensor ptab,
-                                      Tensor ttab, Tensor emb_g, Tensor emb_b, std::vector<Tensor> L, int64_t heads, double eps,
-                                      double scale) -> c10::optional<Tensor> {   // weights are looked at once for both questions
-    if (encoder_refuses(word, {ptab, ttab, emb_g, emb_b}, L, heads) != nullptr) return c10::nullopt;
-    return encoder_forward(ids, pos, types, cu, max_len, word, ptab, ttab, emb_g, emb_b, std::move(L), heads, eps, scale);
-  }, py::call_guard<py::gil_scoped_release>());
+  m.def("encoder_forward", &encoder_forward, py::arg("ids"), py::arg("pos"), py::arg("types"), py::arg("cu"), py::arg("max_len"),
+        py::arg("word"), py::arg("ptab"), py::arg("ttab"), py::arg("emb_g"), py::arg("emb_b"), py::arg("layers"), py::arg("heads"),
+        py::arg("eps"), py::arg("scale"), py::arg("covered_only") = false, py::call_guard<py::gil_scoped_release>());   // some 200 launches
   m.def("encoder_covers", [](const Tensor& word, const std::vector<Tensor>& tables, const std::vector<Tensor>& L, int64_t heads) {
     return encoder_refuses(word, tables, L, heads) == nullptr;
   });

@@ -1431,9 +1431,8 @@ def encoder_forward(ids, pos, types, cu, max_len: int, word, ptab, ttab, emb_ln,
 
     def i32(t):
         return None if t is None else t.to(torch.int32).contiguous()
-    f = kernels().encoder_forward_covered if covered_only else kernels().encoder_forward
-    return f(i32(ids), i32(pos), i32(types), i32(cu), int(max_len), word, ptab, ttab, emb_ln[0], emb_ln[1],
-                                     _encoder_weights(layers), int(heads), float(eps), float(scale))
+    return kernels().encoder_forward(i32(ids), i32(pos), i32(types), i32(cu), int(max_len), word, ptab, ttab, emb_ln[0], emb_ln[1],
+                                     _encoder_weights(layers), int(heads), float(eps), float(scale), bool(covered_only))
 
 
 # ------------------------------------------------------------------------- MoE

@@ -27,6 +27,11 @@ def _close(a, b):
     assert a.shape == b.shape and ((a - b).norm() / b.norm()).item() < 2e-2
 
 
+def _native(m, t):
+    """What the model's forward asks first: the hidden rows, or None for weights that the native call leaves."""
+    return ops.encoder_forward(t[0], t[1], None, t[2], t[3], m.word, m.pos, m.type, m.emb_ln, m.layers, m.cfg.heads, m.cfg.eps, m.scale, covered_only=True)
+
+
 def _odd(t):
     return torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape).copy_(t)
 
@@ -42,11 +47,12 @@ def test_weights_of_any_layout(gpu, n, what, how):
     """Views that do not begin at 16 bytes, and tables and projections whose elements lie apart."""
     m, t = _model(gpu), _tokens(gpu, n)
     want = m.forward(*t)
+    assert torch.equal(m._pool(_native(m, t), t[2]), want)
     if what in m.layers[0]:
         m.layers[0][what] = how(m.layers[0][what])
     else:
         setattr(m, what, tuple(how(w) for w in m.emb_ln) if what == "emb_ln" else how(getattr(m, what)))
-    assert not ops.encoder_covers(m.word, m.layers, m.cfg.heads, (m.pos, m.type, *m.emb_ln))
+    assert not ops.encoder_covers(m.word, m.layers, m.cfg.heads, (m.pos, m.type, *m.emb_ln)) and _native(m, t) is None
     _close(m.forward(*t), want)
 
 
@@ -56,7 +62,9 @@ def test_weights_of_other_shapes_are_not_covered(gpu, name, size):
     tables = (m.pos, m.type, *m.emb_ln)
     assert ops.encoder_covers(m.word, m.layers, m.cfg.heads, tables)
     m.layers[1][name] = torch.zeros(size, dtype=torch.bfloat16, device=gpu)
-    assert not ops.encoder_covers(m.word, m.layers, m.cfg.heads, tables)
+    assert not ops.encoder_covers(m.word, m.layers, m.cfg.heads, tables) and _native(m, _tokens(gpu, 30)) is None
+    with pytest.raises(RuntimeError):   # asked for by name it raises
+        ops.encoder_forward(*_tokens(gpu, 30)[:2], None, *_tokens(gpu, 30)[2:], m.word, m.pos, m.type, m.emb_ln, m.layers, m.cfg.heads, m.cfg.eps, m.scale)
     with pytest.raises(RuntimeError):
         m.forward(*_tokens(gpu, 30))
 
