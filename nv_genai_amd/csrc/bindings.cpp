@@ -3120,6 +3120,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("encoder_forward", &encoder_forward, py::arg("ids"), py::arg("pos"), py::arg("types"), py::arg("cu"), py::arg("max_len"),
         py::arg("word"), py::arg("ptab"), py::arg("ttab"), py::arg("emb_g"), py::arg("emb_b"), py::arg("layers"), py::arg("heads"),
         py::arg("eps"), py::arg("scale"), py::arg("covered_only") = false, py::call_guard<py::gil_scoped_release>());   // some 200 launches
+  m.def("norm_reads_ahead", &nga::norm_reads_ahead);
   m.def("encoder_covers", [](const Tensor& word, const std::vector<Tensor>& tables, const std::vector<Tensor>& L, int64_t heads) {
     return encoder_refuses(word, tables, L, heads) == nullptr;
   });

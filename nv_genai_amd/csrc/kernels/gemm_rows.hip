@@ -414,11 +414,21 @@ void launch_row_attn_gemm(const RowGemmParams& p, int D, hipStream_t stream) {
 
 static int rows_threads(int H) { return (H / 8 + 63) / 64 * 64; }
 
+// Up to how many weights reading ahead gains: what a die's 4 MB of L2 do not hold until the product comes is read twice, and the norm takes as long as
+// the whole stream. A layer, us, without / q/k/v's / up's too, at 19 rows: hidden 1,024 27.6 26.5 25.8, 1,536 44.2 42.1 41.4, 2,048 51.9 51.1 50.7,
+// 2,304 66.2 66.2 66.3, 2,560 74.2 74.1 76.0, 4,096 137 143 153. Tiles come with token rows beside their weights, so their line lies lower, and lower
+// still with many: at 64 / 208 / 512 / 768 rows 1,024 38.2 43.4 56.6 69.2, 37.9 42.7 55.9 69.2, 37.6 42.5 54.7 68.4; 1,280 43.4 56.8 74.6 81.9, 42.8 56.6
+// 73.1 82.2, 42.4 54.9 72.8 83.2; 1,536 46.1 64.2 85.5 126, 45.8 63.6 85.7 127, 46.3 63.4 86.2 129; 2,048 54.7 74.5 107 181, 55.7 76.7 109 184, 57.2 78.5
+// 112 186. Other numbers of weights than multiples of 128 are not dealt out
+bool norm_reads_ahead(int64_t M, int64_t N, int64_t K, bool tiled) {
+  return N % 128 == 0 && K % 128 == 0 && N * K <= (!tiled ? 1 << 24 : M <= 512 ? 6600000 : 1 << 22);
+}
+
 void launch_splitk_layernorm(const float* P, int S, int M, const uint16_t* bias, const uint16_t* resid, const uint16_t* g,
                              const uint16_t* b, float eps, int H, uint16_t* out, uint16_t* packed, const ReadAhead& next, hipStream_t stream) {
   if (M == 0) return;
-  // 32 workgroups a die have 8 MB under way at once; 16 and 64 a die were 1 % slower. Rows of fewer weights have no pieces
-  const int beside = next.w != nullptr && next.N % 128 == 0 && next.K % 128 == 0 ? 256 : 0;
+  // 32 workgroups a die have 8 MB under way at once; 16 and 64 a die were 1 % slower
+  const int beside = next.w != nullptr && norm_reads_ahead(M, next.N, next.K, next.tiled) ? 256 : 0;
 #define NGA_SL(NS) splitk_layernorm_kernel<NS><<<M + beside, rows_threads(H), 0, stream>>>(P, S, M, bias, resid, g, b, eps, H, out, packed, next)
   if (S == 1) NGA_SL(1);
   else if (S == 2) NGA_SL(2);

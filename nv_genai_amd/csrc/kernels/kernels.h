@@ -270,6 +270,7 @@ struct ReadAhead {
   const uint16_t* w;
   int N, K, tiled;
 };
+bool norm_reads_ahead(int64_t M, int64_t N, int64_t K, bool tiled);   // whether a norm of M rows does well to read weights [N, K]
 
 // gemm_rows.hip: projections of few rows with the steps around them
 struct RowGemmParams {

@@ -88,6 +88,16 @@ def test_tiles_end_where_the_library_is_faster(gpu, H, tiles, library):
     assert tiles <= ops.kernels().encoder_tile_rows(H) < library
 
 
+def test_norms_read_ahead_what_the_caches_hold(gpu):
+    """The next product's weights, of the sizes that gain from it: what lies beyond them would be read twice."""
+    f = ops.kernels().norm_reads_ahead
+    for M in (1, 32):
+        assert f(M, 4096, 1024, False) and f(M, 8192, 2048, False) and not f(M, 10240, 2560, False) and not f(M, 16384, 4096, False)
+    for M, most, beyond in ((33, 1280, 1408), (512, 1280, 1408), (513, 1024, 1152), (1024, 1024, 1152)):
+        assert f(M, 4 * most, most, True) and not f(M, 4 * beyond, beyond, True) and not f(M, 32768, 8192, True)
+    assert not f(19, 1536, 448, False) and not f(19, 448, 1536, False) and f(19, 1152, 384, False)
+
+
 def test_no_hidden_size_jumps(gpu):
     """Neighbouring sizes (64 apart) take the tiles up to neighbouring row counts: neither product nor quotient of rows and size jumps."""
     rows = {H: ops.kernels().encoder_tile_rows(H) for H in range(64, 4097, 64)}
