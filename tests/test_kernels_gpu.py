@@ -754,6 +754,27 @@ def test_skinny_gemm_every_cfg(gpu, M):
                     rel=1e-4)
 
 
+@pytest.mark.parametrize("M", [1, 16, 33, 130, 300])
+@pytest.mark.parametrize("at,gap", [(4, 0), (0, 4), (4, 12)])
+def test_skinny_gemm_rows_at_8_bytes(gpu, M, at, gap):
+    """Results of bf16 go out 16 bytes a lane, to rows that begin at 8: the same values, and nothing beside them, also of a ragged last
+    weight block and token tile."""
+    C = ops.kernels()
+    torch.manual_seed(M)
+    x, w = _bf(M, 256, dev=gpu), _bf(2 * 448, 256, dev=gpu, scale=0.05)
+    for cfg in range(C.skinny_cfg_count()):
+        for epi, N in ((0, 2 * 448 - 8), (2, 448 if 448 % (C.skinny_cfg(cfg)[0] // 2) == 0 else 256)):
+            wc = w[:N].contiguous() if epi == 0 else w[:2 * N].contiguous()
+            want = ops.skinny_gemm(x, wc, cfg, 1, epi)
+            buf = torch.full((at + M * (N + gap) + 8,), 7.0, dtype=torch.bfloat16, device=gpu)
+            out = buf[at:at + M * (N + gap)].view(M, N + gap)[:, :N]
+            assert (out.data_ptr() % 16, out.stride(0) % 8) == (2 * at, gap % 8)
+            ops.skinny_gemm(x, wc, cfg, 1, epi, out=out)
+            assert torch.equal(out, want), (cfg, epi)
+            out.fill_(7.0)
+            assert bool((buf == 7.0).all()), (cfg, epi)
+
+
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
 @pytest.mark.parametrize("N,K", [(37, 1000), (4096, 4096), (300, 14336)])
 def test_gemv(gpu, M, N, K):
