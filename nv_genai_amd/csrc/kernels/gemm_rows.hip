@@ -9,8 +9,10 @@
 // lane (37 bytes a nanosecond and CU from L2); with four lanes to 64 bytes of a row 107. So weights come in that order and change
 // lanes (gr_fragment), and token rows lie packed, a step of 16 rows in one piece, written so by what makes them. BERT-large at 19 rows,
 // weights from HBM, us, library / as fragments / so: q/k/v 11.1 / 5.1 / 3.7, output behind its attention - / 5.3 / 4.5, up 11.3 / 5.9 /
-// 3.9 and its GELU launch saved, down 14.1 / 5.3 / 3.9. Token rows come from L2 again for each workgroup: from 33 rows on the LDS tiles
-// of gemm_skinny.hip are faster (64 rows, as fragments: q/k/v 8.2 here, 7.6 there).
+// 3.9 and its GELU launch saved, down 14.1 / 5.3 / 3.9. Token rows come from L2 again for each workgroup, up
+// to two tiles of 16. A layer of an encoder at 16 / 20 / 32 rows, us, here / in the LDS tiles of gemm_skinny.hip: hidden size 384 22.1 23.2 23.7 / 26.7 27.3
+// 27.4, 768 23.5 24.9 25.2 / 29.6 30.1 30.4, 1,024 26.9 28.2 28.7 / 34.6 34.8 35.4 (at 36 rows 25.5, 31.0, 36.8 there). Three tiles and more were slower than LDS
+// tiles while every load came as fragments (64 rows: q/k/v 8.2, 7.6 there), and have not been tried with these loads.
 #include "common.h"
 #include "gelu.h"
 #include "kernels.h"
