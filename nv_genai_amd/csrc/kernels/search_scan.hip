@@ -565,8 +565,8 @@ __global__ void __launch_bounds__(256, 1) scan_kernel(ScanArgs p) {
 // 64 lanes takes a value in, then no longer holds up the DMA and the products of the next tile. Us, whole search, in the stream's waves / apart:
 // k 4, 64 queries: 1M x 1,024 341 318, 600k x 896 224 174, 900k x 512 246 180, 130k x 384 52 45, 10k x 768 22.9 22.4; 33 queries: 900k x 512
 // 197 156; 20 queries: 130k x 384 36.6 33.2; k 8: 250k x 1,024, 64 queries, 146 105, 600k x 896, 40 queries, 235 187, 900k x 512, 20 queries, 195 160;
-// k 12, 20 queries: 600k x 768 226 162, 60k x 1,024 47 44. Writing scores so gains nothing (it is the memory's time: 33 x 250k x 1,024 124 126, 64 x 1M 479
-// 502); lists of 32, or of 16 for more than 32 queries, remain slower than scores (33 x 900k x 512, k 12, 223 372).
+// k 12, 20 queries: 600k x 768 226 162, 60k x 1,024 47 44. Writing scores so gains nothing (33 x 250k x 1,024 124 126, 64 x 1M 479
+// 502; their 33 MB cost some 18 us there, where a copy writes as much in 7); lists of 32, or of 16 for more than 32 queries, remain slower than scores (33 x 900k x 512, k 12, 223 372).
 namespace {
 constexpr int WIDE_BIAS = 8;   // where the stream's waves take the sums in: tiles whose biases have a place, more than are under way
 // which numbers of groups (NG) it takes of 128 KS dimensions
