@@ -1423,7 +1423,7 @@ def encoder_covers(word: torch.Tensor, layers, heads: int, tables=()) -> bool:
 def encoder_forward(ids, pos, types, cu, max_len: int, word, ptab, ttab, emb_ln, layers, heads: int, eps: float,
                     scale: float, covered_only: bool = False) -> Optional[torch.Tensor]:
     """Hidden rows [T, H] of packed tokens through a post-norm encoder stack (models/encoder.py), every launch from one
-    native call: up to 32 rows the projections of gemm_rows.hip, up to 1,024 the LDS tiles of gemm_skinny.hip, both with
+    native call: up to 32 rows the projections of gemm_rows.hip, up to 1,024 (smaller models more, ``encoder_tile_rows``) the LDS tiles of gemm_skinny.hip, both with
     bias, GELU and the K split of the norm fused, above that the library's GEMM. Weights that ``encoder_covers`` refuses raise, or
     with ``covered_only`` give None."""
     if covered_only and not _gpu(word):
